@@ -350,9 +350,9 @@ struct Plan {
     int nbq, nbk, es;
     int sel_width;        // columns of the index lists: k_sel, or the cap of the CDF rule
     bool cdf;
-    bool direct_qo, direct_kv;
+    bool f32, direct_kv;
     bool frag;            // k and v are rewritten in fragment order for fwd_frag_kernel (bsa_fwd_frag.hip)
-    size_t off_qp, off_kp, off_vp, off_op, off_qc, off_kc, off_score, off_idx, off_idx_sorted, off_lens, off_valid, off_qrows, off_ktiles, off_order, off_queue, off_knorm, off_fallback, total;
+    size_t off_kp, off_vp, off_qc, off_kc, off_score, off_idx, off_idx_sorted, off_lens, off_valid, off_qrows, off_krows, off_ktiles, off_order, off_queue, off_knorm, off_fallback, total;
 };
 inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -383,18 +383,19 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     const size_t bh = (size_t)p->B * p->Hn;
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += up256(bytes); return o; };
-    // The MFMA kernel reads q and writes o in THW order itself, and gathers k and v tiles from THW
-    // order when the kv grid allows it; blocked copies are only made for the fp32 kernel and for
-    // kv grids that do not qualify.
-    pl->direct_qo = p->dtype != BSA_F32;
-    pl->frag = pl->direct_qo && !compact;
-    pl->direct_kv = pl->direct_qo && !pl->frag && kv_direct_ok(pl->gk, (int64_t)p->D * pl->es);
-    pl->off_qp = take(pl->direct_qo ? 0 : bh * pl->Sqp * p->D * pl->es);
+    // The attention kernels read q and write o where they lie.  k and v: the fp32 kernel reads them where they lie too,
+    // the fragment-order kernel from rewritten copies, the gathering route where the grid allows it and from blocked
+    // copies where it does not.
+    pl->f32 = p->dtype == BSA_F32;
+    pl->frag = !pl->f32 && !compact;
+    pl->direct_kv = !pl->f32 && !pl->frag && kv_direct_ok(pl->gk, (int64_t)p->D * pl->es);
     // fragment order is a permutation of the padded blocked order: the same size
-    const size_t kv_rows = pl->direct_kv ? (size_t)edge_count(pl->gk) * pl->gk.chunk() : (size_t)pl->Skp;
+    const size_t kv_rows = pl->f32 ? 0 : pl->direct_kv ? (size_t)edge_count(pl->gk) * pl->gk.chunk() : (size_t)pl->Skp;
     pl->off_kp = take(bh * kv_rows * p->D * pl->es);
     pl->off_vp = take(bh * kv_rows * p->D * pl->es);
-    pl->off_op = take(pl->direct_qo ? 0 : bh * pl->Sqp * p->D * pl->es);
+    // Callers size their fp32 workspaces for blocked copies of the four tensors (bsa_workspace_bytes is part of the
+    // interface): the size stays, the kernels no longer need that part of it.
+    if (pl->f32) take(2 * bh * (pl->Sqp + pl->Skp) * p->D * pl->es);
     pl->off_qc = take(bh * pl->nbq * p->D * pl->es);
     pl->off_kc = take(bh * pl->nbk * p->D * pl->es);
     pl->off_score = take(bh * pl->nbq * (size_t)pl->nbk * pl->es);
@@ -402,11 +403,12 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->off_idx_sorted = take(bh * pl->nbq * (size_t)(pl->sel_width > 0 ? pl->sel_width : 1) * sizeof(int32_t));
     pl->off_lens = take(bh * pl->nbq * sizeof(int32_t));
     pl->off_valid = take((size_t)(pl->Skp / 64) * sizeof(uint64_t));
-    pl->off_qrows = take(pl->direct_qo ? (size_t)pl->Sqp * sizeof(int32_t) : 0);
+    pl->off_qrows = take((size_t)pl->Sqp * sizeof(int32_t));
+    pl->off_krows = take(pl->f32 ? (size_t)pl->Skp * sizeof(int32_t) : 0);
     pl->off_ktiles = take(pl->direct_kv ? (size_t)(pl->Skp / 64) * sizeof(uint32_t) : 0);
     // lists of unequal length (the CDF rule): work items by descending length, and the counter they are drawn with
-    pl->off_order = take(pl->cdf && pl->direct_qo ? bh * (size_t)(pl->Sqp / 64) * sizeof(int32_t) : 0);
-    pl->off_queue = take(pl->cdf && pl->direct_qo ? 2 * sizeof(uint32_t) : 0);    // the counter and the choice of schedule
+    pl->off_order = take(pl->cdf && !pl->f32 ? bh * (size_t)(pl->Sqp / 64) * sizeof(int32_t) : 0);
+    pl->off_queue = take(pl->cdf && !pl->f32 ? 2 * sizeof(uint32_t) : 0);    // the counter and the choice of schedule
     pl->off_knorm = take(pl->frag ? frag_key_norm_floats(p->B, p->Hn, pl->Skp / 64) * sizeof(float) : 0);   // key norms per head and tile
     pl->off_fallback = take(pl->frag ? frag_fallback_ints((int64_t)bh * (pl->Sqp / 64)) * sizeof(int32_t) : 0);
     pl->total = off;
@@ -422,8 +424,8 @@ size_t bsa_workspace_bytes(const bsa_3d_params* p) {
 
 namespace {
 struct Ws {
-    void *qp, *kp, *vp, *op, *qc, *kc, *score;
-    int32_t *idx, *idx_sorted, *lens, *qrows, *order;
+    void *kp, *vp, *qc, *kc, *score;
+    int32_t *idx, *idx_sorted, *lens, *qrows, *krows, *order;
     uint32_t *ktiles, *queue;
     uint64_t* valid;
     float* knorm;
@@ -435,16 +437,17 @@ int carve(const Plan& pl, void* workspace, size_t workspace_bytes, const char* w
         return set_error(BSA_ERR_WORKSPACE, "%s: workspace of %zu bytes is smaller than the %zu required", who, workspace_bytes, pl.total);
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return set_error(BSA_ERR_BAD_ARG, "%s: workspace must be 256-byte aligned", who);
     char* ws = static_cast<char*>(workspace);
-    w->qp = ws + pl.off_qp; w->kp = ws + pl.off_kp; w->vp = ws + pl.off_vp; w->op = ws + pl.off_op;
+    w->kp = ws + pl.off_kp; w->vp = ws + pl.off_vp;
     w->qc = ws + pl.off_qc; w->kc = ws + pl.off_kc; w->score = ws + pl.off_score;
     w->idx = reinterpret_cast<int32_t*>(ws + pl.off_idx);
     w->idx_sorted = reinterpret_cast<int32_t*>(ws + pl.off_idx_sorted);
     w->lens = reinterpret_cast<int32_t*>(ws + pl.off_lens);
     w->valid = reinterpret_cast<uint64_t*>(ws + pl.off_valid);
-    w->qrows = pl.direct_qo ? reinterpret_cast<int32_t*>(ws + pl.off_qrows) : nullptr;
+    w->qrows = reinterpret_cast<int32_t*>(ws + pl.off_qrows);
+    w->krows = reinterpret_cast<int32_t*>(ws + pl.off_krows);
     w->ktiles = pl.direct_kv ? reinterpret_cast<uint32_t*>(ws + pl.off_ktiles) : nullptr;
-    w->order = pl.cdf && pl.direct_qo ? reinterpret_cast<int32_t*>(ws + pl.off_order) : nullptr;
-    w->queue = pl.cdf && pl.direct_qo ? reinterpret_cast<uint32_t*>(ws + pl.off_queue) : nullptr;
+    w->order = pl.cdf && !pl.f32 ? reinterpret_cast<int32_t*>(ws + pl.off_order) : nullptr;
+    w->queue = pl.cdf && !pl.f32 ? reinterpret_cast<uint32_t*>(ws + pl.off_queue) : nullptr;
     w->knorm = pl.frag ? reinterpret_cast<float*>(ws + pl.off_knorm) : nullptr;
     w->fallback = pl.frag ? reinterpret_cast<int32_t*>(ws + pl.off_fallback) : nullptr;
     return BSA_OK;
@@ -551,7 +554,7 @@ int bsa_thw_prepare(const bsa_3d_params* p, const void* k, const int64_t k_strid
     Plan pl;
     Ws w;
     BSA_TRY(make_plan(p, &pl));
-    if (!pl.direct_qo) return set_error(BSA_ERR_UNSUPPORTED, "thw_prepare: bf16 and fp16 only (fp32 runs through bsa_fwd_3d)");
+    if (pl.f32) return set_error(BSA_ERR_UNSUPPORTED, "thw_prepare: bf16 and fp16 only (fp32 runs through bsa_fwd_3d)");
     BSA_TRY(carve(pl, workspace, workspace_bytes, "thw_prepare", &w));
     BSA_TRY(check_tensor(k, k_strides, p, "k"));
     BSA_TRY(check_tensor(v, v_strides, p, "v"));
@@ -568,7 +571,7 @@ int bsa_fwd_thw(const bsa_3d_params* p, const void* q, const int64_t q_strides[3
     Plan pl;
     Ws w;
     BSA_TRY(make_plan(p, &pl));
-    if (!pl.direct_qo) return set_error(BSA_ERR_UNSUPPORTED, "fwd_thw: bf16 and fp16 only (fp32 runs through bsa_fwd_3d)");
+    if (pl.f32) return set_error(BSA_ERR_UNSUPPORTED, "fwd_thw: bf16 and fp16 only (fp32 runs through bsa_fwd_3d)");
     BSA_TRY(carve(pl, workspace, workspace_bytes, "fwd_thw", &w));
     BSA_TRY(check_tensor(q, q_strides, p, "q"));
     BSA_TRY(check_tensor(k, k_strides, p, "k"));
@@ -603,7 +606,6 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     BSA_TRY(check_tensor(o, o_strides, p, "o"));
     BSA_TRY(check_kv_views(pl, k_strides, v_strides, "fwd_3d"));
 
-    const bool padded_k = kv_padded(p);
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
 #define BSA_HIP(call, what) do { e = (call); if (e != hipSuccess) return hip_fail(e, what); } while (0)
@@ -616,37 +618,43 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, &trq, &trk), "pool, norm, rotate and prepare");
         q = q_normed;
         q_strides = qn_strides;
-    } else if (pl.direct_qo) {
+    } else if (!pl.f32) {
         BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st), "pool and prepare");
     } else {
-        BSA_HIP(launch_permute(q, q_strides, w.qp, w.qc, nullptr, p->B, p->Hn, pl.gq, p->D, p->dtype, st), "permute q");
-        BSA_HIP(launch_permute(k, k_strides, w.kp, w.kc, padded_k ? w.valid : nullptr, p->B, p->Hn, pl.gk, p->D, p->dtype, st), "permute k");
-        BSA_HIP(launch_permute(v, v_strides, w.vp, nullptr, nullptr, p->B, p->Hn, pl.gk, p->D, p->dtype, st), "permute v");
+        BSA_HIP(launch_pool_f32(q, q_strides, pl.gq, (float*)w.qc, w.qrows, k, k_strides, pl.gk, (float*)w.kc, w.krows, p->B, p->Hn, st),
+                "pool q and k");
     }
-    BSA_HIP(launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st), "score");
     // the lists the attention kernel walks come out in ascending block order and, for the fragment-order
     // kernel, are then put in its visiting order (L2 locality); the score order is only produced when the
     // caller asks for the selection
     const int64_t sel_rows = (int64_t)p->B * p->Hn * pl.nbq;
-    if (pl.cdf) {
-        BSA_HIP(launch_cdf_count(w.score, w.lens, sel_rows, pl.nbk, p->cdf_threshold, p->sm_scale, p->k_sel < pl.sel_width ? p->k_sel : pl.sel_width,
-                                 pl.sel_width, p->dtype, st), "cdf count");
-        BSA_HIP(launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, 0, p->dtype, st, w.lens, pl.sel_width), "top-k");
+    if (!pl.cdf && idx_out == nullptr && score_out == nullptr && gate_fits(p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, p->dtype)) {
+        BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st), "gate");
     } else {
-        BSA_HIP(launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, p->k_sel, p->dtype, st), "top-k");
+        BSA_HIP(launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st), "score");
+        if (pl.cdf) {
+            BSA_HIP(launch_cdf_count(w.score, w.lens, sel_rows, pl.nbk, p->cdf_threshold, p->sm_scale, p->k_sel < pl.sel_width ? p->k_sel : pl.sel_width,
+                                     pl.sel_width, p->dtype, st), "cdf count");
+            BSA_HIP(launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, 0, p->dtype, st, w.lens, pl.sel_width), "top-k");
+        } else {
+            BSA_HIP(launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, p->k_sel, p->dtype, st), "top-k");
+        }
+        if (pl.frag && pl.sel_width > 0)
+            BSA_HIP(launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st), "visit order");
     }
-    if (pl.frag && pl.sel_width > 0)
-        BSA_HIP(launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st), "visit order");
-    if (pl.direct_qo) {
+    if (!pl.f32) {
         // lists of unequal length: one launch whose workgroups draw the items, longest lists first
         if (pl.cdf)
             BSA_HIP(launch_order_by_length(w.lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, pl.sel_width, st), "order by length");
         BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, w.idx_sorted, w.lens, pl.sel_width,
                               lse_out, st, pl.cdf), "attention");
     } else {
-        BSA_HIP(launch_fwd(w.qp, w.kp, w.vp, w.idx_sorted, w.lens, padded_k ? w.valid : nullptr, w.op, nullptr, p->B, p->Hn, pl.Sqp, pl.Skp,
-                           pl.gq.chunk(), pl.gk.chunk(), pl.sel_width, p->sm_scale, p->dtype, st), "attention");
-        BSA_HIP(launch_unpermute(w.op, o, o_strides, p->B, p->Hn, pl.gq, p->D, p->dtype, st), "unpermute");
+        F32Layout L;
+        L.q_rows = w.qrows; L.k_rows = w.krows;
+        L.lse_rows = (int64_t)p->Tq * p->Hq * p->Wq;
+        for (int i = 0; i < 3; ++i) { L.q_st[i] = q_strides[i]; L.k_st[i] = k_strides[i]; L.v_st[i] = v_strides[i]; L.o_st[i] = o_strides[i]; }
+        BSA_HIP(launch_fwd_f32(q, k, v, w.idx_sorted, w.lens, nullptr, o, nullptr, p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(),
+                               pl.sel_width, p->sm_scale, st, &L), "attention");
     }
     const size_t bh = (size_t)p->B * p->Hn;
     if (idx_out && pl.sel_width > 0)
@@ -719,7 +727,7 @@ int bsa_fwd_3d_lse(const bsa_3d_params* p, const void* q, const int64_t q_stride
                    size_t workspace_bytes, void* stream) {
     Plan pl;
     BSA_TRY(make_plan(p, &pl));
-    if (!pl.direct_qo) return set_error(BSA_ERR_UNSUPPORTED, "fwd_3d_lse: bf16 and fp16 only (the backward is built for them)");
+    if (pl.f32) return set_error(BSA_ERR_UNSUPPORTED, "fwd_3d_lse: bf16 and fp16 only (the backward is built for them)");
     if (!lse_out || !walk_out || !lens_out) return set_error(BSA_ERR_BAD_ARG, "fwd_3d_lse: lse_out, walk_out and lens_out are required");
     return fwd_3d_impl(pl, p, q, q_strides, k, k_strides, v, v_strides, o, o_strides, workspace, workspace_bytes, nullptr,
                        lens_out, nullptr, stream, nullptr, nullptr, nullptr, lse_out, walk_out);
@@ -733,7 +741,7 @@ int bsa_fwd_3d_qknorm(const bsa_3d_params* p, const bsa_qk_norm* n, const void* 
     BSA_TRY(make_plan(p, &pl));
     if (!n || !n->rope_table || !n->q_weight || !n->k_weight || !q_normed || !qn_strides)
         return set_error(BSA_ERR_BAD_ARG, "fwd_3d_qknorm: null pointer");
-    if (!(pl.direct_qo && pl.frag && pl.gq.chunk() == 64 && pl.gk.chunk() == 64) || p->tq > 8 || p->hq > 8 || p->wq > 8 ||
+    if (!(pl.frag && pl.gq.chunk() == 64 && pl.gk.chunk() == 64) || p->tq > 8 || p->hq > 8 || p->wq > 8 ||
         p->tk > 8 || p->hk > 8 || p->wk > 8)
         return set_error(BSA_ERR_UNSUPPORTED, "fwd_3d_qknorm: bf16 / fp16 with 64-token chunks of at most 8 positions per axis only "
                          "(use bsa_qk_norm_rope and bsa_fwd_3d)");

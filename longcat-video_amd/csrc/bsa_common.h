@@ -120,6 +120,12 @@ hipError_t launch_score(const void* q_cmp, const void* k_cmp, void* score, int B
 hipError_t launch_topk(const void* score, int32_t* idx, int32_t* idx_sorted, int32_t* lens, int64_t rows,
                        int nbk, int k_sel, int dtype, hipStream_t st, const int32_t* k_rows = nullptr,
                        int stride = 0);
+// Scores, top-k and (with `paced`) visiting order of a small call in one launch: lists [BH][nbq][k_sel], ascending or in
+// visiting order, lens = k_sel.  The same lists as launch_score, launch_topk and launch_pace_order; gate_fits says for
+// which sizes it is built and the better choice.
+bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype);
+hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
+                       bool paced, int dtype, hipStream_t st);
 // lens[row] = number of columns the CDF rule keeps, clamped to [k_min, cap]
 hipError_t launch_cdf_count(const void* score, int32_t* lens, int64_t rows, int nbk, float threshold,
                             float scale, int k_min, int cap, int dtype, hipStream_t st);
@@ -129,6 +135,19 @@ hipError_t launch_fwd(const void* q, const void* k, const void* v, const int32_t
                       float sm_scale, int dtype, hipStream_t st, const FwdLayout* layout = nullptr,
                       int64_t layout_lse_rows = 0, int64_t layout_edge_bytes = 0, const int32_t* order = nullptr,
                       uint32_t* queue = nullptr);
+// fp32 (bsa_f32.hip).  Chunk means and row tables (token of every blocked-order slot of one (batch, head), -1 = padding) of
+// q and k in one launch, and the attention kernel; layout null: q, k, v, o in blocked order.
+struct F32Layout {
+    const int32_t *q_rows, *k_rows;
+    int64_t q_st[3], k_st[3], v_st[3], o_st[3];      // element strides {batch, head, token}
+    int64_t lse_rows;
+};
+hipError_t launch_pool_f32(const void* q, const int64_t q_st[3], const Grid3& gq, float* q_pooled, int32_t* q_rows, const void* k,
+                           const int64_t k_st[3], const Grid3& gk, float* k_pooled, int32_t* k_rows, int B, int Hn, hipStream_t st);
+hipError_t launch_fwd_f32(const void* q, const void* k, const void* v, const int32_t* idx, const int32_t* lens,
+                          const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k,
+                          int idx_stride, float sm_scale, hipStream_t st, const F32Layout* layout = nullptr);
+
 // Rewrites every row's ascending list of KV blocks into the order the attention kernel visits them in (see
 // pace_order_kernel).  rows of `stride` entries, lens[row] of them in use; in == out allowed; stride <= 5000.
 hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* lens, int64_t rows, int nbk, int stride,

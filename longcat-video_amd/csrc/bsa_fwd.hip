@@ -1,5 +1,4 @@
-// Block-sparse flash-attention forward for gfx950 (bf16 / fp16 MFMA), plus a
-// plain fp32 kernel for fp32 inputs.
+// Block-sparse flash-attention forward for gfx950 (bf16 / fp16 MFMA).
 //
 // Work decomposition (MFMA kernel).  One workgroup = 256 threads = 4
 // wavefronts processes one work item at a time: 64 query rows against the
@@ -466,80 +465,6 @@ __global__ __launch_bounds__(256, 2) void fwd_mfma_kernel(
     }   // work items
 }
 
-// ------------------------------------------------------------------ fp32
-// 4 lanes per query row, each owning the d values 4*p + 16*j .. +4 (j = 0..7);
-// K and V tiles staged in LDS as fp32; one online-softmax step per key.
-__global__ __launch_bounds__(256) void fwd_f32_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
-    const int32_t* __restrict__ idx, const int32_t* __restrict__ lens,
-    const uint64_t* __restrict__ tile_valid, float* __restrict__ o, float* __restrict__ lse,
-    int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float qk_scale) {
-    __shared__ __attribute__((aligned(16))) float ks[kTile * kD];
-    __shared__ __attribute__((aligned(16))) float vs[kTile * kD];
-    const int tid = threadIdx.x;
-    const int r = tid >> 2, p = tid & 3;
-    const int bh = blockIdx.y;
-    const int64_t qrow0 = (int64_t)blockIdx.x * kTile;
-    const int nbq = (int)(Sq / bs_q);
-    const int qblock = (int)(qrow0 / bs_q);
-    const int nsub = bs_k / kTile;
-    const int32_t* list = idx + ((int64_t)bh * nbq + qblock) * idx_stride;
-    const int ntiles = min(max(lens[(int64_t)bh * nbq + qblock], 0), idx_stride) * nsub;   // never past the list row
-    const float* kbase = k + (int64_t)bh * Sk * kD;
-    const float* vbase = v + (int64_t)bh * Sk * kD;
-
-    float4 qv[8], acc[8];
-    const float* qp = q + ((int64_t)bh * Sq + qrow0 + r) * kD + 4 * p;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        qv[j] = *reinterpret_cast<const float4*>(qp + 16 * j);
-        acc[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-    float m_i = -INFINITY, l_i = 0.f;
-    for (int it = 0; it < ntiles; ++it) {
-        const int64_t row0 = (int64_t)min(max(list[it / nsub], 0), (int)(Sk / bs_k) - 1) * bs_k + (int64_t)(it % nsub) * kTile;
-        const uint64_t vmask = tile_valid ? tile_valid[row0 / kTile] : ~0ull;
-        __syncthreads();
-        for (int i = tid; i < kTile * kD / 4; i += 256) {
-            reinterpret_cast<float4*>(ks)[i] = reinterpret_cast<const float4*>(kbase + row0 * kD)[i];
-            reinterpret_cast<float4*>(vs)[i] = reinterpret_cast<const float4*>(vbase + row0 * kD)[i];
-        }
-        __syncthreads();
-        for (int key = 0; key < kTile; ++key) {
-            float s = 0.f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float4 kk = *reinterpret_cast<const float4*>(ks + key * kD + 16 * j + 4 * p);
-                s = fmaf(qv[j].x, kk.x, s); s = fmaf(qv[j].y, kk.y, s);
-                s = fmaf(qv[j].z, kk.z, s); s = fmaf(qv[j].w, kk.w, s);
-            }
-            s += __shfl_xor(s, 1);
-            s += __shfl_xor(s, 2);
-            if (!((vmask >> key) & 1ull)) continue;
-            s *= qk_scale;
-            const float m_new = fmaxf(m_i, s);
-            const float alpha = exp2f(m_i - m_new);
-            const float pe = exp2f(s - m_new);
-            l_i = l_i * alpha + pe;
-            m_i = m_new;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float4 vv = *reinterpret_cast<const float4*>(vs + key * kD + 16 * j + 4 * p);
-                acc[j].x = fmaf(pe, vv.x, acc[j].x * alpha); acc[j].y = fmaf(pe, vv.y, acc[j].y * alpha);
-                acc[j].z = fmaf(pe, vv.z, acc[j].z * alpha); acc[j].w = fmaf(pe, vv.w, acc[j].w * alpha);
-            }
-        }
-    }
-    const float inv = l_i > 0.f ? 1.0f / l_i : 0.f;
-    float* op = o + ((int64_t)bh * Sq + qrow0 + r) * kD + 4 * p;
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-        *reinterpret_cast<float4*>(op + 16 * j) =
-            make_float4(acc[j].x * inv, acc[j].y * inv, acc[j].z * inv, acc[j].w * inv);
-    if (lse != nullptr && p == 0)
-        lse[(int64_t)bh * Sq + qrow0 + r] = l_i > 0.f ? (m_i + log2f(l_i)) * kLn2 : -INFINITY;
-}
-
 }  // namespace
 
 __global__ void zero_words_kernel(uint32_t* p, int n) {
@@ -640,6 +565,8 @@ hipError_t launch_fwd(const void* q, const void* k, const void* v, const int32_t
                       int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride,
                       float sm_scale, int dtype, hipStream_t st, const FwdLayout* layout, int64_t layout_lse_rows,
                       int64_t layout_edge_bytes, const int32_t* order, uint32_t* queue) {
+    if (dtype == BSA_F32)
+        return launch_fwd_f32(q, k, v, idx, lens, tile_valid, o, lse, B, Hn, Sq, Sk, bs_q, bs_k, idx_stride, sm_scale, st);
     const float qk_scale = sm_scale * kLog2e;
     FwdLayout L;
     int64_t lse_S = Sq, edge_bh_bytes = 0;
@@ -659,13 +586,6 @@ hipError_t launch_fwd(const void* q, const void* k, const void* v, const int32_t
         L.kw = 4; L.kh = 16; L.kH = 16; L.kW = 4;     // 16 runs of 4 rows, one after the other
     }
     const dim3 block(256);
-    if (dtype == BSA_F32) {
-        const dim3 grid((unsigned)(Sq / kTile), (unsigned)(B * Hn));
-        hipLaunchKernelGGL(fwd_f32_kernel, grid, block, 0, st, (const float*)q, (const float*)k,
-                           (const float*)v, idx, lens, tile_valid, (float*)o, lse, Sq, Sk, bs_q,
-                           bs_k, idx_stride, qk_scale);
-        return hipGetLastError();
-    }
     // One launch per round of as many work items as the device runs at once: the workgroups of a
     // launch start together and walk their (ascending) KV lists in step, so that a tile fetched
     // by one of them is still in L2 when its neighbours ask for it.  When the query tiles of a head

@@ -102,20 +102,34 @@ __global__ __launch_bounds__(256) void score_mfma_kernel(const T* __restrict__ q
     }
 }
 
-// fp32 storage type: plain fp32 dot products (used by the fp32 plumbing case).
-__global__ __launch_bounds__(256) void score_f32_kernel(const float* __restrict__ qc,
-                                                        const float* __restrict__ kc,
-                                                        float* __restrict__ score, int nbq,
-                                                        int nbk, int D) {
-    const int bh = blockIdx.z;
-    const int n = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int m = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (m >= nbq || n >= nbk) return;
-    const float* a = qc + ((int64_t)bh * nbq + m) * D;
-    const float* b = kc + ((int64_t)bh * nbk + n) * D;
-    float s = 0.f;
-    for (int d = 0; d < D; ++d) s = fmaf(a[d], b[d], s);
-    score[((int64_t)bh * nbq + m) * nbk + n] = s;
+// fp32 storage type: v_mfma_f32_16x16x4, a wavefront per 16 x 16 scores.  Step (j, e) contracts d = 16 j + 4 (lane / 16) + e,
+// so that a lane reads its row in 16-byte pieces.  score_tile_f32 is also what the one-launch gating runs: the same bits.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void score_row_f32(const float* row, f32x4 (&x)[8]) {       // row + 4 (lane / 16)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = *reinterpret_cast<const f32x4*>(row + 16 * j);
+}
+__device__ __forceinline__ f32x4 score_tile_f32(const f32x4 (&a)[8], const f32x4 (&b)[8]) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][e], b[j][e], acc, 0, 0, 0);
+    return acc;                              // accumulator i of lane l: row 4 (l / 16) + i, column l % 16
+}
+__global__ __launch_bounds__(256) void score_f32_kernel(const float* __restrict__ qc, const float* __restrict__ kc,
+                                                        float* __restrict__ score, int nbq, int nbk) {
+    constexpr int D = 128;
+    const int bh = blockIdx.z, lane = threadIdx.x & 63, n16 = lane & 15, g = lane >> 4;
+    const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 64 + (threadIdx.x >> 6) * 16;
+    if (n0 >= nbk) return;
+    f32x4 a[8], b[8];
+    score_row_f32(qc + ((int64_t)bh * nbq + min(m0 + n16, nbq - 1)) * D + 4 * g, a);
+    score_row_f32(kc + ((int64_t)bh * nbk + min(n0 + n16, nbk - 1)) * D + 4 * g, b);
+    const f32x4 acc = score_tile_f32(a, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (m0 + 4 * g + i < nbq && n0 + n16 < nbk) score[((int64_t)bh * nbq + m0 + 4 * g + i) * nbk + n0 + n16] = acc[i];
 }
 
 // ---------------------------------------------------------------- top-k
@@ -421,39 +435,32 @@ __global__ __launch_bounds__(256) void topk_blocked_kernel(const uint16_t* __res
 // block order.  in == out is allowed.  A malformed list (unsorted, repeated or out-of-range blocks) still
 // gives a permutation of the blocks clamped to the valid range.
 constexpr int kPaceWidth = 8;
-__global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32_t* out, const int32_t* __restrict__ lens, int nbk, int stride) {
-    extern __shared__ int32_t pace_lds[];
-    int32_t* const lst = pace_lds;               // [stride] the row, ascending
-    int32_t* const slots = lst + stride;         // [stride] block per visit slot, -1 = empty
-    int32_t* const spare = slots + stride;       // [stride] blocks over their group's room, ascending
-    int32_t* const first = spare + stride;       // [groups] position of a group's first block in lst
-    const int lane = threadIdx.x;
-    const int64_t row = blockIdx.x;
-    const int32_t* src = in + row * stride;
-    int32_t* dst = out + row * stride;
-    const int n = min(max(lens[row], 0), stride);
-    if (src != dst)
-        for (int e = n + lane; e < stride; e += 64) dst[e] = src[e];
-    if (n <= kPaceWidth) {
-        if (src != dst)
-            for (int e = lane; e < n; e += 64) dst[e] = src[e];
-        return;
-    }
+// Orders this wavefront's LDS accesses on both sides of it, for the compiler and the hardware; no other wavefront waits.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// 32-bit words of LDS that pace_row needs for lists of n entries
+__host__ __device__ inline int pace_words(int n) { return 3 * n + (n + kPaceWidth - 1) / kPaceWidth; }
+// work[0 .. n): the ascending list, clamped to the valid range; dst: where its visiting order goes
+__device__ inline void pace_row(int32_t* work, int n, int cap, int nbk, int lane, int32_t* __restrict__ dst) {
+    int32_t* const lst = work;                   // [cap] the row, ascending
+    int32_t* const slots = lst + cap;            // [cap] block per visit slot, -1 = empty
+    int32_t* const spare = slots + cap;          // [cap] blocks over their group's room, ascending
+    int32_t* const first = spare + cap;          // [groups] position of a group's first block in lst
     const int groups = (n + kPaceWidth - 1) / kPaceWidth;
-    // n <= stride < 2^13 (the LDS that launch_pace_order asks for bounds it) and b < nbk: 32-bit products and quotients
+    // n < 2^13 (the LDS that the callers ask for bounds it) and b < nbk: 32-bit products and quotients
     const uint32_t span = (uint32_t)nbk * kPaceWidth;
     auto group_of = [&](int32_t b) { return (int)min((uint32_t)b * (uint32_t)n / span, (uint32_t)groups - 1u); };
-    for (int e = lane; e < n; e += 64) {
-        lst[e] = min(max(src[e], 0), nbk - 1);
-        slots[e] = -1;
-    }
+    for (int e = lane; e < n; e += 64) slots[e] = -1;
     for (int g = lane; g < groups; g += 64) first[g] = 0;
-    __syncthreads();
+    wave_sync();
     for (int e = lane; e < n; e += 64) {
         const int g = group_of(lst[e]);
         if (e == 0 || group_of(lst[e - 1]) != g) first[g] = e;
     }
-    __syncthreads();
+    wave_sync();
     const uint64_t below = ((uint64_t)1 << lane) - 1;
     int taken = 0;
     for (int base = 0; base < n; base += 64) {
@@ -469,7 +476,7 @@ __global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32
         if (over) spare[taken + __popcll(m & below)] = lst[e];
         taken += __popcll(m);
     }
-    __syncthreads();
+    wave_sync();
     taken = 0;
     for (int base = 0; base < n; base += 64) {
         const int s = base + lane;
@@ -478,7 +485,7 @@ __global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32
         if (empty) slots[s] = spare[taken + __popcll(m & below)];
         taken += __popcll(m);
     }
-    __syncthreads();
+    wave_sync();
     for (int s = lane; s < n; s += 64) {
         const int lo = s / kPaceWidth * kPaceWidth, hi = min(lo + kPaceWidth, n);
         const int32_t b = slots[s];
@@ -486,6 +493,142 @@ __global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32
         for (int t = lo; t < hi; ++t) rank += (slots[t] < b || (slots[t] == b && t < s)) ? 1 : 0;
         dst[lo + rank] = b;
     }
+}
+__global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32_t* out, const int32_t* __restrict__ lens, int nbk, int stride) {
+    extern __shared__ int32_t pace_lds[];
+    const int lane = threadIdx.x;
+    const int64_t row = blockIdx.x;
+    const int32_t* src = in + row * stride;
+    int32_t* dst = out + row * stride;
+    const int n = min(max(lens[row], 0), stride);
+    if (src != dst)
+        for (int e = n + lane; e < stride; e += 64) dst[e] = src[e];
+    if (n <= kPaceWidth) {
+        if (src != dst)
+            for (int e = lane; e < n; e += 64) dst[e] = src[e];
+        return;
+    }
+    for (int e = lane; e < n; e += 64) pace_lds[e] = min(max(src[e], 0), nbk - 1);
+    wave_sync();
+    pace_row(pace_lds, n, stride, nbk, lane, dst);
+}
+
+// ---------------------------------------------------------------- the whole gating of a small call in one launch
+// Scores, top-k and visiting order of kRows score rows per workgroup of 16 wavefronts: the scores go to LDS instead of
+// memory (the same MFMA chain as score_mfma_kernel and the same rounding, so the same bits), a wavefront selects
+// kRows / 16 of the rows from there and writes their lists in visiting order.  One launch instead of three: a launch of
+// a few microseconds' work costs 4.4 us in a stream of dependent ones.  A workgroup takes most of a CU's LDS, so a call
+// of many rows overlaps nothing and is better served by the separate kernels (gate_fits has the line).
+template <typename T> struct GateRows { static constexpr int kRows = 32; typedef uint16_t bits; };
+template <> struct GateRows<float> { static constexpr int kRows = 16; typedef uint32_t bits; };
+constexpr int kGateThreads = 1024;
+constexpr int kGateMaxBlocks = 512;
+constexpr int kGateMaxGroups = 256;
+__host__ __device__ inline int gate_pitch(int nbk) { return (nbk + 31) / 32 * 32 + 8; }
+// words of LDS a wavefront selects and orders in: its histogram, later the row's list
+__host__ __device__ inline int gate_wave_words(int k_sel) { const int w = pace_words(k_sel); return ((w > 256 ? w : 256) + 3) / 4 * 4; }
+
+template <typename T, int NPL>
+__global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict__ qc, const T* __restrict__ kc, int32_t* __restrict__ lists,
+                                                            int32_t* __restrict__ lens, int nbq, int nbk, int k_sel, int paced) {
+    typedef typename GateRows<T>::bits S;
+    constexpr int D = 128, R = GateRows<T>::kRows;
+    extern __shared__ __attribute__((aligned(16))) unsigned char gate_lds[];
+    const int pitch = gate_pitch(nbk), words = gate_wave_words(k_sel);
+    T* const scores = reinterpret_cast<T*>(gate_lds);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    uint32_t* const mine = reinterpret_cast<uint32_t*>(gate_lds + (size_t)R * pitch * sizeof(T)) + wave * words;
+    const int bh = blockIdx.y, m0 = blockIdx.x * R;
+    const T* qb = qc + (int64_t)bh * nbq * D;
+    const T* kb = kc + (int64_t)bh * nbk * D;
+    if constexpr (sizeof(T) == 2) {
+        typedef typename Vec8<T>::type V8;
+        const int lr = lane & 31, lh = lane >> 5;
+        if (wave * 32 < nbk) {
+            V8 a[8];
+            const T* qa = qb + (int64_t)min(m0 + lr, nbq - 1) * D + lh * 8;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) a[s] = *reinterpret_cast<const V8*>(qa + s * 16);
+            for (int n0 = wave * 32; n0 < nbk; n0 += 32 * (kGateThreads / 64)) {
+                const T* kt = kb + (int64_t)min(n0 + lr, nbk - 1) * D + lh * 8;
+                V8 b[8];
+#pragma unroll
+                for (int s = 0; s < 8; ++s) b[s] = *reinterpret_cast<const V8*>(kt + s * 16);
+                f32x16 acc;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+                for (int s = 0; s < 8; ++s) acc = mfma32(a[s], b[s], acc);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) scores[(8 * (i / 4) + 4 * lh + (i % 4)) * pitch + n0 + lr] = (T)acc[i];
+            }
+        }
+    } else {
+        const int n16 = lane & 15, g = lane >> 4;
+        if (wave * 16 < nbk) {
+            f32x4 a[8], b[8];
+            score_row_f32(qb + (int64_t)min(m0 + n16, nbq - 1) * D + 4 * g, a);
+            for (int n0 = wave * 16; n0 < nbk; n0 += 16 * (kGateThreads / 64)) {
+                score_row_f32(kb + (int64_t)min(n0 + n16, nbk - 1) * D + 4 * g, b);
+                const f32x4 acc = score_tile_f32(a, b);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) scores[(4 * g + i) * pitch + n0 + n16] = acc[i];
+            }
+        }
+    }
+    __syncthreads();
+    // with gridDim.z == 2 two workgroups compute the same scores and select half of the rows each
+    for (int r = wave + (kGateThreads / 64) * blockIdx.z; r < R; r += (kGateThreads / 64) * gridDim.z) {
+        const int m = m0 + r;
+        if (m >= nbq) break;
+        const int64_t row = (int64_t)bh * nbq + m;
+        if (lane == 0) lens[row] = k_sel;
+        if (k_sel == 0) continue;
+        const S* srow = reinterpret_cast<const S*>(scores + r * pitch);
+        uint32_t val[NPL];
+#pragma unroll
+        for (int j = 0; j < NPL; ++j) {
+            const int i = j * 64 + lane;
+            const S raw = srow[min(i, nbk - 1)];
+            val[j] = i < nbk ? ord_of(raw) : 0u;
+        }
+        int32_t* const list = reinterpret_cast<int32_t*>(mine);
+        select_row<S, NPL, false>(val, [&](int i) { return srow[i]; }, lane, nbk, k_sel, nullptr, list, nullptr, mine);
+        wave_sync();
+        int32_t* const dst = lists + row * k_sel;
+        if (paced && k_sel > kPaceWidth) pace_row(list, k_sel, k_sel, nbk, lane, dst);
+        else
+            for (int e = lane; e < k_sel; e += 64) dst[e] = list[e];
+        wave_sync();
+    }
+}
+
+template <typename T>
+size_t gate_lds_bytes(int nbk, int k_sel) {
+    return (size_t)GateRows<T>::kRows * gate_pitch(nbk) * sizeof(T) + (size_t)(kGateThreads / 64) * gate_wave_words(k_sel) * 4;
+}
+
+template <typename T>
+hipError_t launch_gate_t(const T* qc, const T* kc, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel, bool paced,
+                         hipStream_t st) {
+    const size_t lds = gate_lds_bytes<T>(nbk, k_sel);
+    const int blocks = (nbq + GateRows<T>::kRows - 1) / GateRows<T>::kRows;
+    const int halves = GateRows<T>::kRows > kGateThreads / 64 && blocks * BH <= kGateMaxGroups / 2 ? 2 : 1;
+    const dim3 grid(blocks, BH, halves), block(kGateThreads);
+#define BSA_GATE(N)                                                                                                          \
+    do {                                                                                                                     \
+        if (lds > 64 * 1024) {                                                                                               \
+            const hipError_t ea = hipFuncSetAttribute((const void*)gate_kernel<T, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+            if (ea != hipSuccess) return ea;                                                                                 \
+        }                                                                                                                    \
+        hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0);  \
+    } while (0)
+    if (nbk <= 64) BSA_GATE(1);
+    else if (nbk <= 128) BSA_GATE(2);
+    else if (nbk <= 256) BSA_GATE(4);
+    else BSA_GATE(8);
+#undef BSA_GATE
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- CDF rule
@@ -636,9 +779,9 @@ hipError_t launch_topk_t(const S* score, int32_t* idx, int32_t* idx_sorted, int3
 hipError_t launch_score(const void* q_cmp, const void* k_cmp, void* score, int BH, int nbq, int nbk,
                         int D, int dtype, hipStream_t st) {
     if (dtype == BSA_F32) {
-        dim3 grid((nbk + 63) / 64, (nbq + 3) / 4, BH);
+        dim3 grid((nbk + 63) / 64, (nbq + 15) / 16, BH);
         hipLaunchKernelGGL(score_f32_kernel, grid, dim3(256), 0, st, (const float*)q_cmp,
-                           (const float*)k_cmp, (float*)score, nbq, nbk, D);
+                           (const float*)k_cmp, (float*)score, nbq, nbk);
     } else {
         dim3 grid((nbk + kScoreCols - 1) / kScoreCols, (nbq + 127) / 128, BH);
         if (dtype == BSA_BF16)
@@ -657,6 +800,20 @@ hipError_t launch_topk(const void* score, int32_t* idx, int32_t* idx_sorted, int
     if (dtype == BSA_F32)
         return launch_topk_t<uint32_t>((const uint32_t*)score, idx, idx_sorted, lens, rows, nbk, k_sel, k_rows, stride, st);
     return launch_topk_t<uint16_t>((const uint16_t*)score, idx, idx_sorted, lens, rows, nbk, k_sel, k_rows, stride, st);
+}
+
+bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype) {
+    if (nbk > kGateMaxBlocks) return false;
+    const int rows = dtype == BSA_F32 ? GateRows<float>::kRows : GateRows<__bf16>::kRows;
+    const size_t lds = dtype == BSA_F32 ? gate_lds_bytes<float>(nbk, k_sel) : gate_lds_bytes<__bf16>(nbk, k_sel);
+    return lds <= 160 * 1024 && (int64_t)BH * ((nbq + rows - 1) / rows) <= kGateMaxGroups;
+}
+
+hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
+                       bool paced, int dtype, hipStream_t st) {
+    if (dtype == BSA_F32) return launch_gate_t<float>((const float*)q_cmp, (const float*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st);
+    if (dtype == BSA_BF16) return launch_gate_t<__bf16>((const __bf16*)q_cmp, (const __bf16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st);
+    return launch_gate_t<_Float16>((const _Float16*)q_cmp, (const _Float16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st);
 }
 
 hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* lens, int64_t rows, int nbk, int stride,

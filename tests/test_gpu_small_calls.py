@@ -1,0 +1,58 @@
+"""Kernels that small calls run: the fp32 attention kernel in both of its splits, and the gating in one launch."""
+import math
+
+import pytest
+import torch
+
+from oracle import bsa_oracle as O
+from conftest import seeded_qkv
+
+pytestmark = pytest.mark.gpu
+
+
+def I():
+    from longcat_video_amd.block_sparse_attention import bsa_interface
+    return bsa_interface
+
+
+@pytest.mark.parametrize("latent,chunk,heads,sparsity", [
+    ((4, 8, 8), (4, 4, 4), 1, 0.75),        # one key block per row
+    ((5, 9, 13), (4, 4, 4), 2, 0.5),        # ragged in every axis: whole key groups of padding
+    ((3, 6, 12), (4, 4, 8), 3, 0.5),        # 128-slot chunks
+    ((8, 32, 32), (4, 4, 4), 8, 0.875),     # 4 096 units of 16 rows: the last size of the split walk
+    ((8, 32, 36), (4, 4, 4), 8, 0.9375),    # beyond it
+])
+def test_fp32_operator_against_the_oracle(latent, chunk, heads, sparsity):
+    """fp32 products and sums in another order than the oracle's: 2e-5, the bound of the other fp32 tests."""
+    S = math.prod(latent)
+    q, k, v = seeded_qkv(71, 1, heads, S, S, 128, torch.float32)
+    dev = [x.cuda() for x in (q, k, v)]
+    o, idx, lens, score = I()._bsa_3d(*dev, latent, latent, sparsity, chunk, chunk, True)
+    assert torch.equal(I().flash_attn_bsa_3d(*dev, latent, latent, sparsity=sparsity, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk), o)
+    bs = math.prod(chunk)
+    kvalid = torch.from_numpy(O.slot_validity(latent, chunk))
+    heads_checked = [0, heads - 1] if heads > 3 else list(range(heads))
+    sub = lambda x: x[:, heads_checked]      # noqa: E731
+    qp, kp, vp = (O.rearrange_thw_to_3d_block(sub(x), latent, chunk) for x in (q, k, v))
+    mask = O.block_mask_from_indices(sub(idx).cpu().long(), sub(lens).cpu(), score.shape[-1])
+    want, _ = O.masked_dense_attention(qp, kp, vp, mask, bs, bs, 1 / math.sqrt(128), key_valid=kvalid)
+    want = O.rearrange_3d_block_to_thw(want, latent, chunk)
+    assert (sub(o).cpu() - want).abs().max() <= 2e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("latent,heads,sparsity", [
+    ((4, 4, 8), 1, 0.5),           # two blocks, one kept
+    ((4, 12, 44), 3, 0.5),         # 33 blocks: a second row group and a second column tile of one
+    ((8, 32, 32), 2, 0.875),       # 128
+    ((8, 34, 60), 2, 0.9),         # 270: not a multiple of 8
+    ((16, 32, 64), 1, 0.75),       # 512: the widest, lists of 128
+    ((16, 32, 68), 1, 0.75),       # 544: the separate kernels
+])
+def test_one_launch_gating_equals_the_separate_kernels(dtype, latent, heads, sparsity):
+    """A call that asks for the selection runs score, top-k and visiting order one by one; the others gate in one launch
+    where it is built.  The same lists in the same order give the same bits."""
+    chunk, S = (4, 4, 4), math.prod(latent)
+    q, k, v = (x.cuda() for x in seeded_qkv(72, 1, heads, S, S, 128, dtype))
+    o = I()._bsa_3d(q, k, v, latent, latent, sparsity, chunk, chunk, True)[0]
+    assert torch.equal(I().flash_attn_bsa_3d(q, k, v, latent, latent, sparsity=sparsity, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk), o)
