@@ -22,7 +22,9 @@ Differences from the reference, all supersets:
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes as C
+import functools
 import math
 import threading
 from typing import Optional, Sequence, Tuple
@@ -47,18 +49,38 @@ def _need_gpu(*tensors: torch.Tensor) -> None:
             raise RuntimeError("the block-sparse attention engine runs on the GPU only; got a %s tensor" % t.device)
 
 
-def _stream(t: torch.Tensor) -> C.c_void_p:
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+# Handles and pointers go to ctypes as plain integers (None = null): the declared argument types convert them.
+def _stream(t: torch.Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
-def _ptr(t: Optional[torch.Tensor]) -> C.c_void_p:
-    return C.c_void_p(None if t is None else t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def _on_device(t: torch.Tensor):
+    """torch.cuda.device(t.device), without the switch (a few microseconds) when that device is current already."""
+    return _NO_SWITCH if t.device.index == torch._C._cuda_getDevice() else torch.cuda.device(t.device)
+
+
+@functools.lru_cache(maxsize=1024)
+def _strides_of(s0: int, s1: int, s2: int) -> C.Array:
+    return _capi.strides3((s0, s1, s2))
+
+
+def _st(t: torch.Tensor) -> C.Array:
+    """Batch, head and token strides of a [B,H,S,D] tensor for the C ABI (read-only there)."""
+    s = t.stride()
+    return _strides_of(s[0], s[1], s[2])
 
 
 def _rows_ok(t: torch.Tensor) -> torch.Tensor:
     """[B,H,S,D] with a contiguous, 16-byte aligned D axis; anything else is copied."""
-    es = t.element_size()
-    ok = t.stride(3) == 1 and t.data_ptr() % 16 == 0 and all((t.stride(i) * es) % 16 == 0 for i in range(3))
+    s = t.stride()
+    ok = s[3] == 1 and (t.data_ptr() | (s[0] | s[1] | s[2]) * t.element_size()) % 16 == 0
     return t if ok else t.contiguous()
 
 
@@ -73,8 +95,8 @@ def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     (it then lives as long as the graph does, and a later regrowth here cannot pull it from under a replay)."""
     if torch.cuda.is_current_stream_capturing():
         return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
-    key = (device.index if device.index is not None else torch.cuda.current_device(),
-           torch.cuda.current_stream(device).cuda_stream, threading.get_ident())
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    key = (index, torch._C._cuda_getCurrentRawStream(index), threading.get_ident())
     buf = _WORKSPACES.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
@@ -108,9 +130,9 @@ def _permute(x, latent_shape, chunk, want_pooled=False, want_valid=False):
     out = torch.empty(B, H, Sp, D, dtype=x.dtype, device=x.device)
     pooled = torch.empty(B, H, nb, D, dtype=x.dtype, device=x.device) if want_pooled else None
     valid = torch.empty(Sp // 64, dtype=torch.int64, device=x.device) if want_valid else None
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(lib.bsa_permute_thw_to_blocks(
-            _ptr(x), _capi.strides3(x.stride()[:3]), _ptr(out), _ptr(pooled), _ptr(valid),
+            _ptr(x), _st(x), _ptr(out), _ptr(pooled), _ptr(valid),
             B, H, T, Hh, W, t, h, w, D, _code(x), _stream(x)), "permute")
     return out, pooled, valid
 
@@ -134,9 +156,9 @@ def rearrange_3d_block_to_THW(x, Nt, Nh, Nw, t, h, w, D=None, latent_shape=None)
     x = x.contiguous()
     out = torch.empty(B, H, T * Hh * W, Dd, dtype=x.dtype, device=x.device)
     lib = _capi.load()
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(lib.bsa_unpermute_blocks_to_thw(
-            _ptr(x), _ptr(out), _capi.strides3(out.stride()[:3]), B, H, T, Hh, W, t, h, w, Dd, _code(x),
+            _ptr(x), _ptr(out), _st(out), B, H, T, Hh, W, t, h, w, Dd, _code(x),
             _stream(x)), "unpermute")
     return out
 
@@ -152,7 +174,7 @@ def mean_pooling_compression(x: torch.Tensor, block_size: int) -> torch.Tensor:
     nb = math.ceil(S / block_size)
     out = torch.empty(B, H, nb, D, dtype=x.dtype, device=x.device)
     lib = _capi.load()
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(lib.bsa_mean_pool(_ptr(x), _ptr(out), B, H, S, int(block_size), D, _code(x), _stream(x)), "mean_pool")
     return out
 
@@ -169,7 +191,7 @@ def _score_topk(q_cmp, k_cmp, k_sel, order="score"):
     idx = buf[: B * H * nbq * k_sel].view(B, H, nbq, k_sel)
     lens = torch.empty(B, H, nbq, dtype=torch.int32, device=q_cmp.device)
     lib = _capi.load()
-    with torch.cuda.device(q_cmp.device):
+    with _on_device(q_cmp):
         by_score = order == "score"
         _capi.check(lib.bsa_score_topk(_ptr(q_cmp), _ptr(k_cmp), _ptr(buf) if by_score else None,
                                        None if by_score else _ptr(buf), _ptr(lens), _ptr(score),
@@ -188,7 +210,7 @@ def visit_order(idx_sorted: torch.Tensor, lens: torch.Tensor, n_kv_blocks: int) 
     if idx_sorted.numel() == 0:
         return out
     lib = _capi.load()
-    with torch.cuda.device(idx_sorted.device):
+    with _on_device(idx_sorted):
         _capi.check(lib.bsa_visit_order(_ptr(idx_sorted), _ptr(lens), _ptr(out), lens.numel(), int(n_kv_blocks),
                                         idx_sorted.shape[-1], _stream(idx_sorted)), "visit_order")
     return out
@@ -210,7 +232,7 @@ def get_select_indices_topk_from_score(score: torch.Tensor, sparsity: float):
     idx = buf[: B * H * nbq * k_sel].view(B, H, nbq, k_sel)
     lens = torch.empty(B, H, nbq, dtype=torch.int32, device=score.device)
     lib = _capi.load()
-    with torch.cuda.device(score.device):
+    with _on_device(score):
         _capi.check(lib.bsa_topk_from_score(_ptr(score), _ptr(buf), None, _ptr(lens), B, H, nbq, nbk, k_sel,
                                             _code(score), _stream(score)), "topk")
     return idx.long(), lens
@@ -245,7 +267,7 @@ def _select_cdf(score, q_cmp, k_cmp, cdf_threshold, sm_scale, k_min, order="scor
     idx = torch.empty(B, H, nbq, width, dtype=torch.int32, device=dev)
     lens = torch.empty(B, H, nbq, dtype=torch.int32, device=dev)
     a, b = (_ptr(idx), None) if order == "score" else (None, _ptr(idx))
-    with torch.cuda.device(dev):
+    with _on_device(dt):
         if q_cmp is None:
             _capi.check(lib.bsa_cdf_from_score(_ptr(score), a, b, _ptr(lens), B, H, nbq, nbk, float(cdf_threshold),
                                                float(sm_scale), int(k_min), width, _code(dt), _stream(dt)), "cdf")
@@ -331,7 +353,7 @@ def attn_fwd_bsa_varlen(q, k, v, sm_scale, block_indices, block_indices_lens, ch
     o = torch.empty_like(q)
     lse = torch.empty(B, H, Sq, dtype=torch.float32, device=q.device)
     lib = _capi.load()
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         if kernel == "fragment":
             need = lib.bsa_fwd_fragment_workspace_bytes(B, H, Sq, Sk, D, _code(q))
             if need == 0:
@@ -373,7 +395,7 @@ def attn_bwd_bsa_varlen(do, q, k, v, o, dq, dk, dv, sm_scale, M, block_indices, 
     if need == 0:
         raise RuntimeError("bsa_bwd: " + lib.bsa_last_error().decode())
     ws = _workspace(need, q.device)
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         _capi.check(lib.bsa_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(idx), _ptr(lens),
                                 _ptr(tile_valid), _ptr(dq), _ptr(dk), _ptr(dv), B, H, Sq, Sk, D, int(chunk_size_q),
                                 int(chunk_size_k), idx.shape[3], float(sm_scale), _code(q), _ptr(ws), need, _stream(q)),
@@ -454,29 +476,14 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
     (o, lists in the kernel's visiting order, lens, lse in token order) for the backward."""
     _need_gpu(q, k, v)
     B, H, Sq, D = q.shape
-    Tq, Hq, Wq = (int(x) for x in latent_shape_q)
-    Tk, Hk, Wk = (int(x) for x in latent_shape_k)
-    tq, hq, wq = (int(x) for x in chunk_q)
-    tk, hk, wk = (int(x) for x in chunk_k)
-    lib = _capi.load()
     q, k, v = _rows_ok(q), _rows_ok(k), _rows_ok(v)
-    if k.stride(2) != v.stride(2) or max(1, 64 // (wk * hk)) * Hk * Wk * k.stride(2) * k.element_size() >= 2 ** 32:
+    lib = _capi.load()
+    plan = _plan_3d(B, H, D, _code(q), *latent_shape_q, *latent_shape_k, *chunk_q, *chunk_k, sparsity, cdf_threshold)
+    prm, need, nbq, nbk, width = plan.prm, plan.need, plan.nbq, plan.nbk, plan.width
+    if k.stride(2) != v.stride(2) or plan.tile_tokens * k.stride(2) * k.element_size() >= 2 ** 32:
         # the engine gathers k and v tiles with one set of in-tile offsets (32 bits); views that
         # do not fit are copied once
         k, v = k.contiguous(), v.contiguous()
-    nbk = lib.bsa_padded_tokens(Tk, Hk, Wk, tk, hk, wk) // (tk * hk * wk)
-    nbq = lib.bsa_padded_tokens(Tq, Hq, Wq, tq, hq, wq) // (tq * hq * wq)
-    k_sel = 0 if sparsity is None else num_selected(sparsity, nbk)
-    width = k_sel
-    if cdf_threshold is not None:
-        width = _cdf_width(nbk)
-        k_sel = min(k_sel, width)
-    prm = _capi.Bsa3dParams(B, H, D, _code(q), Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, k_sel,
-                            1.0 / D ** 0.5, 0.0 if cdf_threshold is None else float(cdf_threshold))
-    need = lib.bsa_workspace_bytes(C.byref(prm))
-    if need == 0:
-        _capi.check(lib.bsa_fwd_3d(C.byref(prm), None, None, None, None, None, None, None, None, None, 0,
-                                   None, None, None, None), "flash_attn_bsa_3d")
     ws = None if static_scratch else _workspace(need, q.device)
     o = torch.empty(B, H, Sq, D, dtype=q.dtype, device=q.device) if out is None else out
     assert o.shape == (B, H, Sq, D) and o.dtype == q.dtype and o.stride(3) == 1
@@ -489,34 +496,63 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
         walk = torch.empty(B, H, nbq, max(width, 1), dtype=torch.int32, device=q.device)[..., :width]
         lens = torch.empty(B, H, nbq, dtype=torch.int32, device=q.device)
         lse = torch.empty(B, H, Sq, dtype=torch.float32, device=q.device)
-        with torch.cuda.device(q.device):
+        with _on_device(q):
             _capi.check(lib.bsa_fwd_3d_lse(
-                C.byref(prm), _ptr(q), _capi.strides3(q.stride()[:3]), _ptr(k), _capi.strides3(k.stride()[:3]),
-                _ptr(v), _capi.strides3(v.stride()[:3]), _ptr(o), _capi.strides3(o.stride()[:3]),
+                prm, _ptr(q), _st(q), _ptr(k), _st(k),
+                _ptr(v), _st(v), _ptr(o), _st(o),
                 _ptr(lse), _ptr(walk), _ptr(lens), _ptr(ws), need, _stream(q)), "flash_attn_bsa_3d (with lse)")
         return o, walk, lens, lse
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         if qk_norm is not None:
             qw, kw, tab, table_T, t_off_q, t_off_k, eps = qk_norm
             qw, kw = qw.to(q.dtype).contiguous(), kw.to(q.dtype).contiguous()
             q_normed = torch.empty(B, H, Sq, D, dtype=q.dtype, device=q.device)
             n = _capi.BsaQkNorm(_ptr(qw), _ptr(kw), _ptr(tab), int(table_T), int(t_off_q), int(t_off_k), float(eps))
             _capi.check(lib.bsa_fwd_3d_qknorm(
-                C.byref(prm), C.byref(n), _ptr(q), _capi.strides3(q.stride()[:3]), _ptr(q_normed),
-                _capi.strides3(q_normed.stride()[:3]), _ptr(k), _capi.strides3(k.stride()[:3]),
-                _ptr(v), _capi.strides3(v.stride()[:3]), _ptr(o), _capi.strides3(o.stride()[:3]),
+                prm, C.byref(n), _ptr(q), _st(q), _ptr(q_normed),
+                _st(q_normed), _ptr(k), _st(k),
+                _ptr(v), _st(v), _ptr(o), _st(o),
                 _ptr(ws), need, _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d (q/k norm inside)")
         elif static_scratch:
             _capi.check(lib.bsa_fwd_3d_static(
-                C.byref(prm), _ptr(q), _capi.strides3(q.stride()[:3]), _ptr(k), _capi.strides3(k.stride()[:3]),
-                _ptr(v), _capi.strides3(v.stride()[:3]), _ptr(o), _capi.strides3(o.stride()[:3]),
+                prm, _ptr(q), _st(q), _ptr(k), _st(k),
+                _ptr(v), _st(v), _ptr(o), _st(o),
                 _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d (static scratch)")
         else:
             _capi.check(lib.bsa_fwd_3d(
-                C.byref(prm), _ptr(q), _capi.strides3(q.stride()[:3]), _ptr(k), _capi.strides3(k.stride()[:3]),
-                _ptr(v), _capi.strides3(v.stride()[:3]), _ptr(o), _capi.strides3(o.stride()[:3]),
+                prm, _ptr(q), _st(q), _ptr(k), _st(k),
+                _ptr(v), _st(v), _ptr(o), _st(o),
                 _ptr(ws), need, _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d")
     return (o, idx, lens, score) if want_selection else o
+
+
+class _Plan3d:
+    """What a call's geometry alone decides: the C-ABI parameters, the workspace size, the numbers of query and KV
+    blocks, the width of the index lists, and the tokens a 64-slot KV tile spans."""
+    __slots__ = ("prm", "need", "nbq", "nbk", "width", "tile_tokens")
+
+
+@functools.lru_cache(maxsize=256)
+def _plan_3d(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, sparsity, cdf_threshold) -> _Plan3d:
+    lib = _capi.load()
+    Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk = (int(x) for x in (Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk))
+    p = _Plan3d()
+    p.nbk = lib.bsa_padded_tokens(Tk, Hk, Wk, tk, hk, wk) // (tk * hk * wk)
+    p.nbq = lib.bsa_padded_tokens(Tq, Hq, Wq, tq, hq, wq) // (tq * hq * wq)
+    k_sel = 0 if sparsity is None else num_selected(sparsity, p.nbk)
+    p.width = k_sel
+    if cdf_threshold is not None:
+        p.width = _cdf_width(p.nbk)
+        k_sel = min(k_sel, p.width)
+    prm = _capi.Bsa3dParams(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, k_sel,
+                            1.0 / D ** 0.5, 0.0 if cdf_threshold is None else float(cdf_threshold))
+    p.prm = C.byref(prm)
+    p.need = lib.bsa_workspace_bytes(p.prm)
+    p.tile_tokens = max(1, 64 // (wk * hk)) * Hk * Wk
+    if p.need == 0:      # the call itself names what is wrong with the problem
+        _capi.check(lib.bsa_fwd_3d(p.prm, None, None, None, None, None, None, None, None, None, 0,
+                                   None, None, None, None), "flash_attn_bsa_3d")
+    return p
 
 
 class ThwAttention:
@@ -545,8 +581,8 @@ class ThwAttention:
                                      1.0 if unequal_lengths else 0.0)
         self.need = lib.bsa_workspace_bytes(C.byref(self.prm))
         self.ws = torch.empty(max(self.need, 1), dtype=torch.uint8, device=k.device)
-        self.ks, self.vs = _capi.strides3(k.stride()[:3]), _capi.strides3(v.stride()[:3])
-        with torch.cuda.device(k.device):
+        self.ks, self.vs = _st(k), _st(v)
+        with _on_device(k):
             _capi.check(lib.bsa_thw_prepare(C.byref(self.prm), _ptr(k), self.ks, _ptr(v), self.vs, _ptr(self.ws),
                                             self.need, _stream(k)), "bsa_thw_prepare")
 
@@ -562,10 +598,10 @@ class ThwAttention:
         o = torch.empty(B, H, Sq, D, dtype=q.dtype, device=q.device) if out is None else out
         assert o.shape == (B, H, Sq, D) and o.dtype == q.dtype and o.stride(3) == 1
         lse = torch.empty(B, H, Sq, dtype=torch.float32, device=q.device) if return_lse else None
-        with torch.cuda.device(q.device):
+        with _on_device(q):
             _capi.check(self.lib.bsa_fwd_thw(
-                C.byref(self.prm), _ptr(q), _capi.strides3(q.stride()[:3]), _ptr(self.k), self.ks, _ptr(self.v), self.vs,
-                _ptr(o), _capi.strides3(o.stride()[:3]), _ptr(idx), _ptr(lens), idx.shape[3], _ptr(lse),
+                C.byref(self.prm), _ptr(q), _st(q), _ptr(self.k), self.ks, _ptr(self.v), self.vs,
+                _ptr(o), _st(o), _ptr(idx), _ptr(lens), idx.shape[3], _ptr(lse),
                 _ptr(self.ws), self.need, _stream(q)), "bsa_fwd_thw")
         return (o, lse) if return_lse else o
 
@@ -621,6 +657,18 @@ class _Bsa3dWithGrad(torch.autograd.Function):
         return _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_q, chunk_k, sm_scale) + (None,) * 6
 
 
+@functools.lru_cache(maxsize=256)
+def _plan_3d_backward(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, sm_scale, width):
+    """C-ABI parameters and workspace size of a backward call."""
+    lib = _capi.load()
+    prm = C.byref(_capi.Bsa3dParams(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, 0, sm_scale, 0.0))
+    need = lib.bsa_bwd_3d_workspace_bytes(prm, width)
+    if need == 0:        # the call itself names what is wrong with the shape
+        _capi.check(lib.bsa_bwd_3d(prm, *([None] * 10), None, None, None, width, *([None] * 6), None, 0, None), "bsa_bwd_3d")
+        raise RuntimeError("bsa_bwd_3d: no workspace size for this problem")
+    return prm, need
+
+
 def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_q, chunk_k, sm_scale):
     """bsa_bwd_3d: dq, dk, dv in token order from token-order tensors (bsa_interface.py:570-596 between the
     rearrangements of :650-652 and :659, of which only those of q and v are made, inside the call)."""
@@ -628,18 +676,14 @@ def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_
     B, H, Sq, D = q.shape
     lib = _capi.load()
     q, k, v, o, do = (_rows_ok(t) for t in (q, k, v, o, do))
-    prm = _capi.Bsa3dParams(B, H, D, _code(q), *latent_q, *latent_k, *chunk_q, *chunk_k, 0, float(sm_scale), 0.0)
     width = walk.shape[3]
-    need = lib.bsa_bwd_3d_workspace_bytes(C.byref(prm), width)
-    if need == 0:        # the call itself names what is wrong with the shape
-        _capi.check(lib.bsa_bwd_3d(C.byref(prm), *([None] * 10), None, None, None, width, *([None] * 6), None, 0, None), "bsa_bwd_3d")
-        raise RuntimeError("bsa_bwd_3d: no workspace size for this problem")
+    prm, need = _plan_3d_backward(B, H, D, _code(q), *latent_q, *latent_k, *chunk_q, *chunk_k, float(sm_scale), width)
     ws = _workspace(need, q.device)
     dq, dk, dv = (torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in (q, k, v))
     lse, walk, lens = lse.contiguous(), walk.contiguous(), lens.contiguous()
-    st = lambda t: _capi.strides3(t.stride()[:3])
-    with torch.cuda.device(q.device):
-        _capi.check(lib.bsa_bwd_3d(C.byref(prm), _ptr(q), st(q), _ptr(k), st(k), _ptr(v), st(v), _ptr(o), st(o), _ptr(do), st(do),
+    st = _st
+    with _on_device(q):
+        _capi.check(lib.bsa_bwd_3d(prm, _ptr(q), st(q), _ptr(k), st(k), _ptr(v), st(v), _ptr(o), st(o), _ptr(do), st(do),
                                    _ptr(lse), _ptr(walk), _ptr(lens), width, _ptr(dq), st(dq), _ptr(dk), st(dk), _ptr(dv), st(dv),
                                    _ptr(ws), need, _stream(q)), "bsa_bwd_3d")
     return dq, dk, dv
@@ -677,6 +721,13 @@ def _bsa_3d_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, latent_shape_q
     # a negative sparsity / cdf_threshold stands for None (operator schemas have no optional floats here)
     return _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, None if sparsity < 0 else sparsity, chunk_3d_shape_q,
                    chunk_3d_shape_k, cdf_threshold=None if cdf_threshold < 0 else cdf_threshold)
+
+
+def _calls_directly(*tensors: torch.Tensor) -> bool:
+    """Plain tensors and nothing that wants to see the operator go by (tracing, a dispatch mode, functorch): the custom
+    op's dispatch, 20 us of a call, is then left out."""
+    return (all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors) and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None)
 
 
 @_bsa_3d_op.register_fake
@@ -721,6 +772,8 @@ def flash_attn_bsa_3d(
             raise NotImplementedError("the backward is built for bf16 and fp16")
         return _Bsa3dWithGrad.apply(q, k, v, [int(x) for x in latent_shape_q], [int(x) for x in latent_shape_k], sparsity,
                                     cdf_threshold, [int(x) for x in chunk_3d_shape_q], [int(x) for x in chunk_3d_shape_k])
+    if not torch.compiler.is_compiling() and _calls_directly(q, k, v):
+        return _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_3d_shape_q, chunk_3d_shape_k, cdf_threshold=cdf_threshold)
     return _bsa_3d_op(q, k, v, [int(x) for x in latent_shape_q], [int(x) for x in latent_shape_k],
                       -1.0 if sparsity is None else float(sparsity), -1.0 if cdf_threshold is None else float(cdf_threshold),
                       [int(x) for x in chunk_3d_shape_q], [int(x) for x in chunk_3d_shape_k])

@@ -30,7 +30,7 @@ import torch
 import torch.nn as nn
 
 from .. import _capi
-from ..block_sparse_attention.bsa_interface import _bsa_3d, _ptr, _stream
+from ..block_sparse_attention.bsa_interface import _bsa_3d, _on_device, _ptr, _st, _stream
 
 
 class RMSNorm_FP32(nn.Module):
@@ -56,7 +56,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     code = {torch.bfloat16: _capi.BSA_BF16, torch.float16: _capi.BSA_F16}.get(x.dtype)
     if code is None:
         raise NotImplementedError("rms_norm: dtype %s is not built (bf16, fp16)" % x.dtype)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(_capi.load().bsa_rmsnorm(_ptr(x), _ptr(w), _ptr(out), x.numel() // dim, dim, float(eps), code,
                                              _stream(x)), "rmsnorm")
     return out
@@ -81,7 +81,7 @@ _GEMM_WORKSPACES = _Bounded(16)          # 64 MiB each
 
 def _gemm_workspace(device) -> torch.Tensor:
     """64 MiB per device and stream, kept: calls on one stream run one after the other."""
-    key = (str(device), torch.cuda.current_stream(device).cuda_stream)
+    key = (str(device), torch._C._cuda_getCurrentRawStream(device.index))
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None:
         ws = _GEMM_WORKSPACES[key] = torch.empty(64 << 20, dtype=torch.uint8, device=device)
@@ -111,7 +111,7 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
         assert r.shape == out.shape and r.dtype == torch.bfloat16
     if workspace is None:
         workspace = _gemm_workspace(x.device)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(_capi.load().bsa_linear_bf16(_ptr(x2), _ptr(w), _ptr(b), _ptr(r), _ptr(out), x2.shape[0], N, K,
                                                  _ptr(workspace), workspace.numel(), _stream(x)), "linear")
     return out.view(*x.shape[:-1], N)
@@ -133,7 +133,7 @@ def tune_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     if workspace is None:
         workspace = _gemm_workspace(x.device)
     d, best = C.c_float(0), C.c_float(0)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         n = _capi.load().bsa_linear_bf16_tune(_ptr(x2), K, _ptr(w), K, _ptr(b), _ptr(r), _ptr(out), N, x2.shape[0], N, K,
                                               _ptr(workspace), workspace.numel(), _stream(x), C.byref(d), C.byref(best))
     if n <= 0:
@@ -166,7 +166,7 @@ def gemm_bf16(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
         r = residual.reshape(-1, N)
         assert r.shape == out.shape and r.dtype == torch.bfloat16 and r.stride(1) == 1
         ldr = r.stride(0)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(_capi.load().bsa_gemm_bf16(_ptr(x2), x2.stride(0), _ptr(w), w.stride(0), _ptr(b), _ptr(r), ldr, _ptr(out),
                                                out.stride(0), x2.shape[0], N, K, _stream(x)), "gemm")
     return out.view(*x.shape[:-1], N)
@@ -196,7 +196,7 @@ def qkv_projection(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     b = None if bias is None else bias.to(torch.bfloat16).contiguous()
     qw, kw = q_weight.to(torch.bfloat16).contiguous(), k_weight.to(torch.bfloat16).contiguous()
     qkv = torch.empty(3, B, num_heads, S, 128, dtype=torch.bfloat16, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(_capi.load().bsa_qkv_projection(
             _ptr(x2), x2.stride(0), _ptr(w), w.stride(0), _ptr(b), _ptr(qw), _ptr(kw), _ptr(tab), _ptr(qkv[0]), _ptr(qkv[1]),
             _ptr(qkv[2]), _capi.strides3(qkv[0].stride()[:3]), B, num_heads, T, Hg, Wg, int(t_offset), table_grid[0], 128, K,
@@ -237,9 +237,9 @@ def qk_norm_rope_(q: torch.Tensor, k: torch.Tensor, q_weight, k_weight, grid_siz
         raise NotImplementedError("qk_norm_rope: dtype %s is not built (bf16, fp16)" % q.dtype)
     tab = rope_table(grid_size, D, q.device)
     qw, kw = q_weight.to(q.dtype).contiguous(), k_weight.to(q.dtype).contiguous()
-    with torch.cuda.device(q.device):
+    with _on_device(q):
         _capi.check(_capi.load().bsa_qk_norm_rope(
-            _ptr(q), _capi.strides3(q.stride()[:3]), _ptr(k), _capi.strides3(k.stride()[:3]), _ptr(qw), _ptr(kw),
+            _ptr(q), _st(q), _ptr(k), _st(k), _ptr(qw), _ptr(kw),
             _ptr(tab), B, H, T, Hg, Wg, D, float(eps), code, _stream(q)), "qk_norm_rope")
 
 
@@ -261,9 +261,9 @@ def norm_rope(src: torch.Tensor, dst: torch.Tensor, weight=None, grid_size=None,
         assert table_grid[1:] == (Hg, Wg)
         tab, table_T = rope_table(table_grid, D, src.device), table_grid[0]
     w = None if weight is None else weight.to(src.dtype).contiguous()
-    with torch.cuda.device(src.device):
+    with _on_device(src):
         _capi.check(_capi.load().bsa_norm_rope(
-            _ptr(src), _capi.strides3(src.stride()[:3]), _ptr(dst), _capi.strides3(dst.stride()[:3]), _ptr(w), _ptr(tab),
+            _ptr(src), _st(src), _ptr(dst), _st(dst), _ptr(w), _ptr(tab),
             B, H, T, Hg, Wg, int(t_offset), table_T, D, float(eps), code, _stream(src)), "norm_rope")
     return dst
 
@@ -479,7 +479,7 @@ def layernorm_modulate(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor
     scale, _ = _frames(x, scale, "scale")
     x = x.contiguous()
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(_capi.load().bsa_layernorm_modulate(_ptr(x), _ptr(shift), _ptr(scale), _ptr(out), x.shape[0] * x.shape[1],
                                                         per, x.shape[2], float(eps), code, _stream(x)), "layernorm_modulate")
     return out
@@ -496,7 +496,7 @@ def gated_residual(x: torch.Tensor, gate: torch.Tensor, y: torch.Tensor) -> torc
     assert y.shape == x.shape and y.dtype == x.dtype
     x, y = x.contiguous(), y.contiguous()
     out = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(_capi.load().bsa_gated_residual(_ptr(x), _ptr(y), _ptr(gate), _ptr(out), x.shape[0] * x.shape[1], per,
                                                     x.shape[2], code, _stream(x)), "gated_residual")
     return out

@@ -12,7 +12,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from .. import _capi
-from .attention import _gemm_workspace, _ptr, _stream, linear_bf16
+from .attention import _gemm_workspace, _on_device, _ptr, _stream, linear_bf16
 
 MAX_BRANCHES = 4
 
@@ -55,7 +55,7 @@ def _up_projection(lx: torch.Tensor, branch: LoRABranch, workspace: torch.Tensor
     per = branch.lora_up[0].shape[0]
     out = torch.empty(M, n * per, dtype=torch.bfloat16, device=lx.device)
     lib = _capi.load()
-    with torch.cuda.device(lx.device):
+    with _on_device(lx):
         for i, w in enumerate(branch.lora_up):
             w = w.contiguous()
             _capi.check(lib.bsa_linear_bf16_ld(lx.data_ptr() + 2 * i * r, n * r, _ptr(w), r, None, None,
@@ -92,7 +92,7 @@ def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     # alpha_scale lives in a bf16 buffer in the reference
     alpha = (C.c_float * n)(*[float(torch.tensor(b.alpha_scale, dtype=torch.bfloat16)) for b in active])
     out2 = org.view(-1, N)
-    with torch.cuda.device(x.device):
+    with _on_device(x):
         _capi.check(_capi.load().bsa_lora_add(_ptr(out2), up_ptrs, mult, alpha, n, _ptr(out2), out2.numel(),
                                               _capi.BSA_BF16, _stream(x)), "lora_add")
     return org
