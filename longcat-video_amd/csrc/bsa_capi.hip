@@ -250,12 +250,18 @@ static int check_fwd_fragment(const void* q, const void* k, const void* v, const
 }
 
 namespace {
+PrepRows prep_rows(const void* p, const int64_t st[3]) {
+    PrepRows x = {};
+    x.p = static_cast<const uint16_t*>(p);
+    x.sB = st[0]; x.sH = st[1]; x.sS = st[2];
+    return x;
+}
 struct FragmentWs { size_t kv, norms, fallback, total; };
 FragmentWs fragment_ws(int B, int Hn, int64_t Sq, int64_t Sk, int D) {
     auto up = [](size_t x) { return (x + 255) & ~(size_t)255; };
     FragmentWs w;
     w.kv = up((size_t)B * Hn * (size_t)Sk * D * 2);
-    w.norms = up(frag_key_norm_floats(B, Hn, Sk / 64) * sizeof(float));
+    w.norms = up(key_norm_floats(B, Hn, Sk / 64) * sizeof(float));
     w.fallback = up(frag_fallback_ints((int64_t)B * Hn * (Sq / 64)) * sizeof(int32_t));
     w.total = 2 * w.kv + w.norms + w.fallback;       // K, V, key norms, the list of items left to the second kernel
     return w;
@@ -291,11 +297,20 @@ int bsa_fwd_fragment(const void* q, const void* k, const void* v, const int32_t*
     float* knorm = reinterpret_cast<float*>(vf + fw.kv);
     int32_t* fallback = reinterpret_cast<int32_t*>(vf + fw.kv + fw.norms);
     hipStream_t st = (hipStream_t)stream;
-    hipError_t e = launch_frag(k, kv_st, kf, B, Hn, g, dtype, false, st, nullptr, nullptr, nullptr, knorm);
-    if (e == hipSuccess) e = launch_frag(v, kv_st, vf, B, Hn, g, dtype, true, st);
+    PrepArgs a = {};
+    a.Hn = Hn;
+    a.gk = g;
+    a.k = prep_rows(k, kv_st);
+    a.k.frag = kf;
+    a.k.tile_norm = knorm + tile_norm_offset(B, Hn);
+    a.v = prep_rows(v, kv_st);
+    a.v.frag = vf;
+    a.zero = reinterpret_cast<uint32_t*>(fallback);
+    hipError_t e = launch_prepare(a, B, dtype, st);
+    if (e == hipSuccess) e = launch_head_norm(a.k.tile_norm, knorm, B * Hn, (int)(Sk / 64), st);
     if (e == hipSuccess)
         e = launch_fwd_frag(q, kf, vf, idx, lens, tile_valid, o, lse, B, Hn, Sq, Sk, bs_q, bs_k, idx_stride, sm_scale, dtype, st,
-                            nullptr, q_st, q_st, Sq, nullptr, nullptr, knorm, fallback);
+                            nullptr, q_st, q_st, Sq, nullptr, nullptr, knorm, fallback, true);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "fwd_fragment");
 }
 
@@ -409,7 +424,7 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     // lists of unequal length (the CDF rule): work items by descending length, and the counter they are drawn with
     pl->off_order = take(pl->cdf && !pl->f32 ? bh * (size_t)(pl->Sqp / 64) * sizeof(int32_t) : 0);
     pl->off_queue = take(pl->cdf && !pl->f32 ? 2 * sizeof(uint32_t) : 0);    // the counter and the choice of schedule
-    pl->off_knorm = take(pl->frag ? frag_key_norm_floats(p->B, p->Hn, pl->Skp / 64) * sizeof(float) : 0);   // key norms per head and tile
+    pl->off_knorm = take(pl->frag ? key_norm_floats(p->B, p->Hn, pl->Skp / 64) * sizeof(float) : 0);   // key norms per head and tile
     pl->off_fallback = take(pl->frag ? frag_fallback_ints((int64_t)bh * (pl->Sqp / 64)) * sizeof(int32_t) : 0);
     pl->total = off;
     return BSA_OK;
@@ -463,46 +478,55 @@ int check_kv_views(const Plan& pl, const int64_t k_strides[3], const int64_t v_s
 }
 
 // Everything the attention kernel needs besides the selection, for the 16-bit types: the row table
-// of q, and for k and v the tile table, the validity words and the copies of the edge chunks (or
-// of all chunks when the kv grid does not allow gathering).  With `pool`, q and k are also read in
-// full and their chunk means stored (one pass over each).
+// of q, and k and v in fragment order with the key norms and validity words, or (gathering) the tile table, the
+// validity words and the copies of the edge chunks (or of all chunks when the kv grid does not allow gathering).
+// With `pool`, the chunk means of q and k come from the same passes.  qkn: q and k are as the projection left them; their
+// rows are normalised and rotated on the way, q's into q_normed.
 hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, const void* q, const int64_t q_strides[3],
                        const void* k, const int64_t k_strides[3], const void* v, const int64_t v_strides[3], bool pool,
-                       hipStream_t st, const RowTransform* trq = nullptr, const RowTransform* trk = nullptr) {
+                       hipStream_t st, const bsa_qk_norm* qkn = nullptr, void* q_normed = nullptr, const int64_t* qn_strides = nullptr) {
     hipError_t e;
     const bool padded_k = kv_padded(p);
-    if (pool && !(pl.frag && pl.gq.chunk() == 64))
+    if (pl.frag) {
+        PrepArgs a = {};
+        a.Hn = p->Hn;
+        a.gq = pl.gq;
+        a.gk = pl.gk;
+        a.k = prep_rows(k, k_strides);
+        a.k.frag = static_cast<char*>(w.kp);
+        a.k.tile_norm = w.knorm + tile_norm_offset(p->B, p->Hn);
+        a.k.valid = padded_k ? w.valid : nullptr;
+        a.v = prep_rows(v, v_strides);
+        a.v.frag = static_cast<char*>(w.vp);
+        if (pool) {
+            a.k.pooled = static_cast<uint16_t*>(w.kc);
+            a.q = prep_rows(q, q_strides);
+            a.q.pooled = static_cast<uint16_t*>(w.qc);
+            a.q.rows = w.qrows;
+            a.zero = reinterpret_cast<uint32_t*>(w.fallback);
+        }
+        if (qkn != nullptr) {
+            a.tab = qkn->rope_table;
+            a.tab_T = qkn->table_T;
+            a.eps = qkn->eps;
+            a.q.norm_w = static_cast<const uint16_t*>(qkn->q_weight);
+            a.k.norm_w = static_cast<const uint16_t*>(qkn->k_weight);
+            a.q.t0 = qkn->t_offset_q;
+            a.k.t0 = qkn->t_offset_k;
+            a.q.rows_out = static_cast<uint16_t*>(q_normed);
+            a.q.rB = qn_strides[0]; a.q.rH = qn_strides[1]; a.q.rS = qn_strides[2];
+        }
+        e = launch_prepare(a, p->B, p->dtype, st);
+        if (e != hipSuccess || pool) return e;                 // scoring takes the largest norm per head on its way
+        e = launch_row_table(pl.gq, w.qrows, st);
+        if (e != hipSuccess) return e;
+        return launch_head_norm(a.k.tile_norm, w.knorm, p->B * p->Hn, (int)(pl.Skp / 64), st);
+    }
+    if (pool)
         e = launch_permute(q, q_strides, nullptr, w.qc, nullptr, p->B, p->Hn, pl.gq, p->D, p->dtype, st, false, w.qrows, nullptr);
     else    // tables only: one (batch, head) slice of workgroups, no row is read
         e = launch_permute(q, q_strides, nullptr, nullptr, nullptr, 1, 1, pl.gq, p->D, p->dtype, st, false, w.qrows, nullptr);
     if (e != hipSuccess) return e;
-    if (pool && pl.frag && pl.gq.chunk() == 64) {
-        // chunk means of q from a read-only pass (the same sums); with a row transform, from the fragment pass run
-        // without a destination, which applies it
-        if (trq == nullptr && p->D == 128) e = launch_pool_tiles(q, q_strides, w.qrows, w.qc, p->B, p->Hn, pl.gq, p->dtype, st);
-        else e = launch_frag(q, q_strides, nullptr, p->B, p->Hn, pl.gq, p->dtype, false, st, w.qc, nullptr, trq);
-        if (e != hipSuccess) return e;
-    }
-    if (pl.frag) {
-        // 64-slot chunks: one pass over k gives its fragment order, its chunk means and the validity words
-        if (pl.gk.chunk() == 64) {
-            e = launch_frag(k, k_strides, w.kp, p->B, p->Hn, pl.gk, p->dtype, false, st, pool ? w.kc : nullptr,
-                            padded_k ? w.valid : nullptr, trk, w.knorm);
-            if (e != hipSuccess) return e;
-            return launch_frag(v, v_strides, w.vp, p->B, p->Hn, pl.gk, p->dtype, true, st);
-        }
-        // larger chunks: pooled means and validity words of k by the pooling pass, then k and v in fragment order
-        if (pool || padded_k) {
-            if (pool)
-                e = launch_permute(k, k_strides, nullptr, w.kc, padded_k ? w.valid : nullptr, p->B, p->Hn, pl.gk, p->D, p->dtype, st);
-            else
-                e = launch_permute(k, k_strides, nullptr, nullptr, w.valid, 1, 1, pl.gk, p->D, p->dtype, st);
-            if (e != hipSuccess) return e;
-        }
-        e = launch_frag(k, k_strides, w.kp, p->B, p->Hn, pl.gk, p->dtype, false, st, nullptr, nullptr, nullptr, w.knorm);
-        if (e != hipSuccess) return e;
-        return launch_frag(v, v_strides, w.vp, p->B, p->Hn, pl.gk, p->dtype, true, st);
-    }
     // gathering: the pass over k copies the edge chunks of v along with those of k
     e = launch_permute(k, k_strides, w.kp, pool ? w.kc : nullptr, padded_k ? w.valid : nullptr, p->B, p->Hn, pl.gk, p->D,
                        p->dtype, st, pl.direct_kv, nullptr, w.ktiles, pl.direct_kv && padded_k ? v : nullptr, v_strides, w.vp);
@@ -515,11 +539,11 @@ hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, cons
 hipError_t attention_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, const void* q, const int64_t q_strides[3],
                          const void* k, const int64_t k_strides[3], const void* v, const int64_t v_strides[3], void* o,
                          const int64_t o_strides[3], const int32_t* idx, const int32_t* lens, int idx_stride, float* lse,
-                         hipStream_t st, bool by_length = false) {
+                         hipStream_t st, bool by_length = false, bool fallback_cleared = false) {
     if (pl.frag)
         return launch_fwd_frag(q, w.kp, w.vp, idx, lens, kv_padded(p) ? w.valid : nullptr, o, lse, p->B, p->Hn, pl.Sqp, pl.Skp,
                                pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype, st, w.qrows, q_strides, o_strides,
-                               (int64_t)p->Tq * p->Hq * p->Wq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback);
+                               (int64_t)p->Tq * p->Hq * p->Wq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared);
     FwdLayout L;
     L.q_rows = w.qrows;
     L.k_tiles = w.ktiles;
@@ -613,9 +637,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         // q and k as the projection left them: the pass that takes q's chunk means also normalises and rotates its
         // rows into q_normed (what the attention kernel then reads), the pass that rewrites k in fragment order
         // normalises and rotates on the way
-        RowTransform trq = {qkn->q_weight, qkn->rope_table, qkn->t_offset_q, qkn->table_T, qkn->eps, q_normed, qn_strides[0], qn_strides[1], qn_strides[2]};
-        RowTransform trk = {qkn->k_weight, qkn->rope_table, qkn->t_offset_k, qkn->table_T, qkn->eps, nullptr, 0, 0, 0};
-        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, &trq, &trk), "pool, norm, rotate and prepare");
+        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, qkn, q_normed, qn_strides), "pool, norm, rotate and prepare");
         q = q_normed;
         q_strides = qn_strides;
     } else if (!pl.f32) {
@@ -628,10 +650,11 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     // kernel, are then put in its visiting order (L2 locality); the score order is only produced when the
     // caller asks for the selection
     const int64_t sel_rows = (int64_t)p->B * p->Hn * pl.nbq;
+    const HeadNorms norms = {pl.frag ? w.knorm + tile_norm_offset(p->B, p->Hn) : nullptr, w.knorm, (int)(pl.Skp / 64)};
     if (!pl.cdf && idx_out == nullptr && score_out == nullptr && gate_fits(p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, p->dtype)) {
-        BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st), "gate");
+        BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st, norms), "gate");
     } else {
-        BSA_HIP(launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st), "score");
+        BSA_HIP(launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st, norms), "score");
         if (pl.cdf) {
             BSA_HIP(launch_cdf_count(w.score, w.lens, sel_rows, pl.nbk, p->cdf_threshold, p->sm_scale, p->k_sel < pl.sel_width ? p->k_sel : pl.sel_width,
                                      pl.sel_width, p->dtype, st), "cdf count");
@@ -647,7 +670,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         if (pl.cdf)
             BSA_HIP(launch_order_by_length(w.lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, pl.sel_width, st), "order by length");
         BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, w.idx_sorted, w.lens, pl.sel_width,
-                              lse_out, st, pl.cdf), "attention");
+                              lse_out, st, pl.cdf, pl.frag), "attention");
     } else {
         F32Layout L;
         L.q_rows = w.qrows; L.k_rows = w.krows;

@@ -103,17 +103,18 @@ hipError_t launch_permute(const void* src, const int64_t strides[3], void* dst, 
                           hipStream_t st, bool edge_only = false, int32_t* row_table = nullptr,
                           uint32_t* tile_table = nullptr, const void* src2 = nullptr,
                           const int64_t* strides2 = nullptr, void* dst2 = nullptr);
-// Chunk means of a 16-bit tensor with 64-slot chunks and D = 128, nothing else: the bits of launch_permute's pooling
-// from a read-only pass.  row_table: the token of every slot of one (batch, head), -1 for padding, as launch_permute
-// writes it.
-hipError_t launch_pool_tiles(const void* src, const int64_t strides[3], const int32_t* row_table, void* pooled, int B, int Hn,
-                             const Grid3& g, int dtype, hipStream_t st);
 hipError_t launch_unpermute(const void* src, void* dst, const int64_t strides[3], int B, int Hn,
                             const Grid3& g, int D, int dtype, hipStream_t st);
 hipError_t launch_mean_pool(const void* x, void* out, int B, int Hn, int64_t S, int block, int D,
                             int dtype, hipStream_t st);
+// The kernels that score can also take the largest key norm of every (batch, head) from those of its tiles on the way
+struct HeadNorms {
+    const float* tile_norm;      // [BH][tiles]; null: not wanted
+    float* key_norm;             // [BH]
+    int tiles;
+};
 hipError_t launch_score(const void* q_cmp, const void* k_cmp, void* score, int BH, int nbq, int nbk,
-                        int D, int dtype, hipStream_t st);
+                        int D, int dtype, hipStream_t st, HeadNorms norms = {nullptr, nullptr, 0});
 // idx: descending score order; idx_sorted: ascending block index; either may be null
 // k_rows: one count per row instead of k_sel (may alias lens); stride: row pitch of idx / idx_sorted
 // (default k_sel), entries past a row's count are set to -1
@@ -125,7 +126,7 @@ hipError_t launch_topk(const void* score, int32_t* idx, int32_t* idx_sorted, int
 // which sizes it is built and the better choice.
 bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype);
 hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
-                       bool paced, int dtype, hipStream_t st);
+                       bool paced, int dtype, hipStream_t st, HeadNorms norms = {nullptr, nullptr, 0});
 // lens[row] = number of columns the CDF rule keeps, clamped to [k_min, cap]
 hipError_t launch_cdf_count(const void* score, int32_t* lens, int64_t rows, int nbk, float threshold,
                             float scale, int k_min, int cap, int dtype, hipStream_t st);
@@ -164,28 +165,37 @@ hipError_t launch_order_by_length(const int32_t* lens, int32_t* order, int BH, i
 void launch_schedule_choice(const int32_t* lens, int nbq, int tiles_per_block, int total, int round, int resident,
                             int max_len, uint32_t* queue, hipStream_t st);
 
-// K or V of a (T, H, W)-ordered tensor in fragment order (bsa_fwd_frag.hip): dst [B*Hn][padded slots / 64][16 KB],
-// padded slots zero; transpose = false for K, true for V.  bf16 / fp16.
-// For K (transpose = false) of 64-slot chunks the pass can also write the chunk means (pooled, [B*Hn][blocks][128],
-// the bits launch_permute's pooling gives) and the tile validity words; both optional.  dst may be null: the pass
-// then only reads (chunk means of q).
-// tr (optional, transpose = false only): per-head RMSNorm and / or 3-D RoPE of every row on its way through the pass.
-// key_norm (optional, transpose = false only, frag_key_norm_floats() floats): its first B*Hn entries receive the largest
-// Euclidean norm of a row of every (batch, head) as the pass writes it (a part in a thousand above), the rest is
-// the per-tile norms they are reduced from; launch_fwd_frag takes the first part to bound q . k.
-size_t frag_key_norm_floats(int B, int Hn, int64_t tiles);
-struct RowTransform {
-    const void* norm_w;      // 128 norm weights in the storage type; null: no norm
-    const float* tab;        // rotation table (the layout bsa_norm_rope reads); null: no rotation
-    int t0, Ttab;            // frame offset of the grid inside the table, frames of the table
-    float eps;
-    void* rows_out;          // optional: the transformed rows at their token positions
-    int64_t rB, rH, rS;      // ... element strides {batch, head, token}
-    int head_fastest;        // set by launch_frag: the order in which workgroups take (tile, head)
+// One tensor on its way through launch_prepare (bsa_prepare.hip).  16-bit types as raw bits; strides in elements.
+struct PrepRows {
+    const uint16_t* p;               // null: this part is left out
+    int64_t sB, sH, sS;              // batch, head, token
+    char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, padded slots zero
+    uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
+    int32_t* rows;                   // q: token row of every blocked-order slot of one (batch, head), -1 = padding
+    uint64_t* valid;                 // k, optional: bit s of word i = slot 64 i + s holds a real token
+    float* tile_norm;                // k, optional: largest Euclidean norm of a row of every tile, a part in a thousand above
+    const uint16_t* norm_w;          // q, k, optional: 128 weights of a per-head RMSNorm that the rows go through first
+    int t0;                          // q, k: frame offset of the grid inside the rotation table
+    uint16_t* rows_out;              // q, k, optional: the transformed rows at their token positions
+    int64_t rB, rH, rS;              // ... element strides
+    int head_fastest;                // set by launch_prepare: the order in which workgroups take (chunk, head)
+    int offsets_32;                  // set by launch_prepare: the rows of a (batch, head) lie within 4 GB
 };
-hipError_t launch_frag(const void* src, const int64_t strides[3], void* dst, int B, int Hn, const Grid3& g, int dtype,
-                       bool transpose, hipStream_t st, void* pooled = nullptr, uint64_t* tile_valid = nullptr,
-                       const RowTransform* tr = nullptr, float* key_norm = nullptr);
+struct PrepArgs {
+    PrepRows q, k, v;
+    Grid3 gq, gk;
+    int Hn;
+    const float* tab;                // rotation table (the layout bsa_norm_rope reads) for q and k; null: no rotation
+    int tab_T;                       // ... its frames
+    float eps;
+    uint32_t* zero;                  // optional: a word to clear
+};
+hipError_t launch_prepare(const PrepArgs& a, int B, int dtype, hipStream_t st);
+hipError_t launch_row_table(const Grid3& g, int32_t* rows, hipStream_t st);
+// Key norms: one per (batch, head), the largest of its tiles', then (from a 256-byte boundary) one per tile.
+inline size_t tile_norm_offset(int B, int Hn) { return ((size_t)B * Hn + 63) & ~(size_t)63; }
+size_t key_norm_floats(int B, int Hn, int64_t tiles);
+hipError_t launch_head_norm(const float* tile_norm, float* key_norm, int BH, int tiles, hipStream_t st);
 // The attention kernel on fragment-order K and V.  q_rows (optional): token row of every blocked-order query
 // slot, -1 for padding; q_st / o_st: element strides {batch, head, row}; lse_rows: rows per (batch, head) of lse.
 hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const int32_t* idx, const int32_t* lens,
@@ -193,9 +203,10 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
-                           int32_t* fallback = nullptr);
+                           int32_t* fallback = nullptr, bool fallback_cleared = false);
 // fallback (optional, frag_fallback_ints(B * Hn * Sq / 64) int32): with it and key_norm the rounds run the kernel that
-// takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.
+// takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.  Its first word
+// counts them: fallback_cleared says that it is zero already.
 size_t frag_fallback_ints(int64_t items);
 
 

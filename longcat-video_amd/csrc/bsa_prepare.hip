@@ -1,0 +1,440 @@
+// What the fragment-order attention kernel needs besides the selection, in one launch (HBM-bound): k and v in fragment
+// order (the layout is described in bsa_fwd_frag.hip), the chunk means of q and k, the row table of q, the validity
+// words of the KV tiles, the largest key norm per tile; with a row transform also the per-head RMSNorm and the 3-D RoPE of
+// q and k on their way through.
+//
+// A small call runs the three parts (workgroups 0 .. wg_k - 1 take chunks of k, the next wg_v tiles of v, the rest chunks of
+// q) in one launch instead of six: its parts take a few microseconds each, and a launch in a stream of dependent ones
+// costs 4.4.  A large call runs one launch per part: together, the part that needs most registers (q, sixteen loads in
+// flight per lane) sets the occupancy of all three, 0.65 instead of 0.56 ms for 32 heads of 720p (launch_prepare has the
+// line).
+#include "bsa_mfma.h"
+#include "bsa_rope.h"
+
+namespace bsa {
+namespace {
+
+using namespace mfma;
+
+template <int kCtrl>
+__device__ __forceinline__ float dpp_f32(float x) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(x), kCtrl, 0xf, 0xf, true));
+}
+
+template <bool kBf16>
+__device__ __forceinline__ void widen(uint32_t w, float& lo, float& hi) {
+    if (kBf16) { lo = __uint_as_float(w << 16); hi = __uint_as_float(w & 0xffff0000u); }
+    else { lo = (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu)); hi = (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)); }
+}
+template <bool kBf16>
+__device__ __forceinline__ uint16_t narrow(float x) {
+    return kBf16 ? __builtin_bit_cast(uint16_t, (__bf16)x) : __builtin_bit_cast(uint16_t, (_Float16)x);
+}
+template <bool kBf16>
+__device__ __forceinline__ void add_row(float (&acc)[8], const uint4& x) {
+    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float lo, hi;
+        widen<kBf16>(w[e], lo, hi);
+        acc[2 * e] += lo;
+        acc[2 * e + 1] += hi;
+    }
+}
+
+// key_norm[batch * heads + head] = the largest entry of the head's tile norms
+__global__ __launch_bounds__(256) void head_norm_kernel(const float* __restrict__ tile_norm, float* __restrict__ key_norm, int tiles) {
+    __shared__ float part[4];
+    float best = 0.f;
+    for (int i = threadIdx.x; i < tiles; i += 256) {
+        const float x = tile_norm[(int64_t)blockIdx.x * tiles + i];
+        best = x != x ? INFINITY : fmaxf(best, x);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) best = fmaxf(best, __shfl_xor(best, off));
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) key_norm[blockIdx.x] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+}
+
+__device__ __forceinline__ void keep_if(uint4& x, bool keep) {
+    const uint32_t m = keep ? ~0u : 0u;
+    x.x &= m; x.y &= m; x.z &= m; x.w &= m;
+}
+
+// The 64 slots of a tile as a wavefront sees them, one per lane: grid position, token row (-1: padding), and the word of
+// the real ones.
+struct Slots {
+    int token, loc;        // loc: position inside the chunk, ti | hi << 8 | wi << 16
+    uint64_t word;
+};
+__device__ __forceinline__ Slots slots_of(const Grid3& g, int blk, int sub, int lane) {
+    const int nw = blk % g.Nw, nh = (blk / g.Nw) % g.Nh, nt = blk / (g.Nw * g.Nh);
+    const int r = sub * kTile + lane;
+    int wi, hi, ti;
+    if (((g.w & (g.w - 1)) | (g.h & (g.h - 1))) == 0) {           // the usual chunks: shifts instead of three divisions
+        const int ws = __builtin_ctz(g.w), hs = __builtin_ctz(g.h);
+        wi = r & (g.w - 1); hi = (r >> ws) & (g.h - 1); ti = r >> (ws + hs);
+    } else {
+        wi = r % g.w; hi = (r / g.w) % g.h; ti = r / (g.w * g.h);
+    }
+    const int tt = nt * g.t + ti, hh = nh * g.h + hi, ww = nw * g.w + wi;
+    const bool ok = tt < g.T && hh < g.H && ww < g.W;
+    Slots s;
+    s.token = ok ? (tt * g.H + hh) * g.W + ww : -1;
+    s.loc = ti | (hi << 8) | (wi << 16);
+    s.word = __ballot(ok);
+    return s;
+}
+
+// workgroup -> (tile or chunk, batch * head).  For a token-major source (the heads of a token next to each other, as a QKV
+// projection leaves them) the heads of one chunk run side by side, so that the 256-byte rows they fetch share DRAM pages
+// and cache lines' neighbourhoods; otherwise the chunks of one head do.
+__device__ __forceinline__ void place(int id, int per_head, int Hn, int head_fastest, int& chunk, int& bh) {
+    if (head_fastest) {
+        const int per_batch = per_head * Hn, b = id / per_batch, rest = id - b * per_batch;
+        chunk = rest / Hn;
+        bh = b * Hn + (rest - chunk * Hn);
+    } else {
+        bh = id / per_head;
+        chunk = id - bh * per_head;
+    }
+}
+
+constexpr int kPitchK = kD + 4;      // elements: 264-byte rows for 16-byte pieces read row by row
+constexpr int kPitchV = kD + 16;     // 288-byte rows: the transposing reads fetch 4 keys x 16 d per 16 lanes, and with rows 72 banks apart the four keys fall on different banks
+
+// k (or q, when it has a row transform): a workgroup per chunk, tile by tile.  The chunk mean keeps permute_kernel's order
+// of summation - a thread adds its rows rg, rg + 16, ... of the chunk, then the 16 partial sums of a column are added in
+// ascending rg, one rounding at the end - so every route gives the same bits.
+template <bool kBf16, bool kTransform>
+__device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int Hn, int id, const float* tab, int tab_T, float eps,
+                                         uint16_t* tile, float2* cs) {
+    typedef typename std::conditional<kBf16, __bf16, _Float16>::type T;
+    const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
+    int blk, bh;
+    place(id, g.blocks(), Hn, x.head_fastest, blk, bh);
+    const int lane = threadIdx.x & 63;
+    const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;      // 16 pieces of 16 B per row, 16 rows at a time
+    const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
+    // Rotation: a chunk spans at most 8 positions per axis, and a rotation pair turns with one axis only, so the
+    // (cos, sin) the rows of the chunk need are 8 x 64 table entries, fetched once per workgroup instead of per row and head.
+    if (kTransform && tab != nullptr) {
+        const int nw = blk % g.Nw, nh = (blk / g.Nw) % g.Nh, nt = blk / (g.Nw * g.Nh);
+        for (int e = threadIdx.x; e < 8 * 64; e += 256) {
+            const int a = e >> 6, pr = e & 63;
+            int at, dsin;
+            if (pr < kRopePairsT) {
+                at = min(x.t0 + nt * g.t + a, tab_T - 1) * kRopePairsT + pr;
+                dsin = tab_T * kRopePairsT;
+            } else if (pr < kRopePairsT + kRopePairsH) {
+                at = 2 * tab_T * kRopePairsT + min(nh * g.h + a, g.H - 1) * kRopePairsH + pr - kRopePairsT;
+                dsin = g.H * kRopePairsH;
+            } else {
+                at = 2 * tab_T * kRopePairsT + 2 * g.H * kRopePairsH + min(nw * g.w + a, g.W - 1) * kRopePairsW + pr - kRopePairsT - kRopePairsH;
+                dsin = g.W * kRopePairsW;
+            }
+            cs[e] = make_float2(tab[at], tab[at + dsin]);
+        }
+        __syncthreads();
+    }
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    for (int sub = 0; sub < per_chunk; ++sub) {
+        const int tile_id = blk * per_chunk + sub;
+        const Slots s = slots_of(g, blk, sub, lane);
+        uint4 xs[4];
+        int token[4], loc[4];
+        // all four loads first, then the arithmetic: a row transformed right behind its own load would wait for it
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            token[i] = __shfl(s.token, rg + 16 * i);
+            if (kTransform) loc[i] = __shfl(s.loc, rg + 16 * i);
+            xs[i] = *reinterpret_cast<const uint4*>(src + (int64_t)max(token[i], 0) * x.sS);
+        }
+        if (s.word != ~0ull) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) keep_if(xs[i], token[i] >= 0);
+        }
+        if (bh == 0 && threadIdx.x < 64) {
+            if (x.valid != nullptr && lane == 0) x.valid[tile_id] = s.word;
+            if (x.rows != nullptr) x.rows[(int64_t)tile_id * kTile + lane] = s.token;
+        }
+        if (kTransform) {
+            uint4 wraw = make_uint4(0, 0, 0, 0);
+            if (x.norm_w != nullptr) wraw = *reinterpret_cast<const uint4*>(x.norm_w + c16 * 8);
+            uint16_t* rows = x.rows_out == nullptr ? nullptr : x.rows_out + (int64_t)(bh / Hn) * x.rB + (int64_t)(bh % Hn) * x.rH + c16 * 8;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (token[i] < 0) continue;                         // the 16 lanes of a row go together
+                float c[4] = {1.f, 1.f, 1.f, 1.f}, sn[4] = {0.f, 0.f, 0.f, 0.f};
+                if (tab != nullptr) {
+                    const int ti = loc[i] & 255, hi = (loc[i] >> 8) & 255, wi = loc[i] >> 16;
+#pragma unroll
+                    for (int jj = 0; jj < 4; ++jj) {
+                        const int pr = c16 * 4 + jj;
+                        const float2 a = cs[(pr < kRopePairsT ? ti : pr < kRopePairsT + kRopePairsH ? hi : wi) * 64 + pr];
+                        c[jj] = a.x;
+                        sn[jj] = a.y;
+                    }
+                }
+                xs[i] = norm_rope_piece<T>(xs[i], wraw, x.norm_w != nullptr, tab != nullptr, c, sn, eps);
+                if (rows != nullptr) *reinterpret_cast<uint4*>(rows + (int64_t)token[i] * x.rS) = xs[i];
+            }
+        }
+        if (x.pooled != nullptr) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) add_row<kBf16>(acc, xs[i]);
+        }
+        if (x.tile_norm != nullptr) {
+            // the largest Euclidean norm of a row of this tile as it is stored (after the transform), a little above the
+            // exact value: the attention kernel bounds q . k by |q| |k| with the largest of a head.  The sixteen lanes of
+            // a row add their squares (butterfly over the row's lanes with DPP moves), then the maximum over the rows.
+            float best = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t w[4] = {xs[i].x, xs[i].y, xs[i].z, xs[i].w};
+                float sq = 0.f;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float lo, hi;
+                    widen<kBf16>(w[e], lo, hi);
+                    sq = fmaf(lo, lo, fmaf(hi, hi, sq));
+                }
+                sq += dpp_f32<0xB1>(sq);         // quad_perm [1, 0, 3, 2]
+                sq += dpp_f32<0x4E>(sq);         // quad_perm [2, 3, 0, 1]
+                sq += dpp_f32<0x141>(sq);        // row_half_mirror
+                sq += dpp_f32<0x140>(sq);        // row_mirror
+                best = fmaxf(best, sq);          // NaN squares drop out here; such a row has no bound (below)
+                if (sq != sq) best = INFINITY;
+            }
+#pragma unroll
+            for (int off = 32; off >= 16; off >>= 1) best = fmaxf(best, __shfl_xor(best, off));
+            __shared__ float wave_best[4];
+            if (lane == 0) wave_best[threadIdx.x >> 6] = best;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                best = fmaxf(fmaxf(wave_best[0], wave_best[1]), fmaxf(wave_best[2], wave_best[3]));
+                x.tile_norm[(int64_t)bh * tiles + tile_id] = __builtin_sqrtf(best) * 1.001f;
+            }
+        }
+        if (x.frag != nullptr) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                uint16_t* row = tile + (rg + 16 * i) * kPitchK + c16 * 8;          // 8-byte aligned (pitch 264 B)
+                *reinterpret_cast<uint2*>(row) = make_uint2(xs[i].x, xs[i].y);
+                *reinterpret_cast<uint2*>(row + 4) = make_uint2(xs[i].z, xs[i].w);
+            }
+            __syncthreads();
+            char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int e = threadIdx.x + 256 * i;                       // 16-byte piece of the output, 0..1023
+                const int l = e & 63, f = e >> 6;                          // lane and fragment: key half f / 8, d chunk f % 8
+                const uint16_t* p = tile + (32 * (f >> 3) + (l & 31)) * kPitchK + 16 * (f & 7) + 8 * (l >> 5);
+                const uint2 lo = *reinterpret_cast<const uint2*>(p), hi = *reinterpret_cast<const uint2*>(p + 4);
+                *reinterpret_cast<uint4*>(out + (int64_t)e * 16) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+            }
+            __syncthreads();                      // the next tile, or the sums below, may have the memory
+        }
+    }
+    if (x.pooled != nullptr) {
+        float* red = reinterpret_cast<float*>(tile);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) red[rg * kD + c16 * 8 + e] = acc[e];
+        __syncthreads();
+        if (threadIdx.x < kD) {
+            float sum = 0.f;
+            for (int i = 0; i < 16; ++i) sum += red[i * kD + threadIdx.x];
+            x.pooled[((int64_t)bh * g.blocks() + blk) * kD + threadIdx.x] = narrow<kBf16>(sum * (1.0f / g.chunk()));
+        }
+    }
+}
+
+// v: a workgroup per tile, gathered into LDS and read transposed: a piece holds 8 keys of one d
+__device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, int Hn, int id, uint16_t* tile) {
+    const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
+    int tile_id, bh;
+    place(id, tiles, Hn, x.head_fastest, tile_id, bh);
+    const int lane = threadIdx.x & 63;
+    const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
+    const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
+    const Slots s = slots_of(g, tile_id / per_chunk, tile_id % per_chunk, lane);
+    uint4 xs[4];
+    int token[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        token[i] = __shfl(s.token, rg + 16 * i);
+        xs[i] = *reinterpret_cast<const uint4*>(src + (int64_t)max(token[i], 0) * x.sS);
+    }
+    if (s.word != ~0ull) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) keep_if(xs[i], token[i] >= 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(tile + (rg + 16 * i) * kPitchV + c16 * 8) = xs[i];
+    __syncthreads();
+    char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int e = threadIdx.x + 256 * i;
+        const int l = e & 63, f = e >> 6;
+        // ds_read_b64_tr_b16: the 16 lanes of a group point at a 4-key x 16-d patch (lane s at key s / 4,
+        // d 4 (s % 4) .. + 4) and each receives the 4 keys of one d
+        const int kh = f >> 3, s2 = (f >> 2) & 1, t = f & 3, lh = l >> 5;
+        const int s16 = l & 15, g1 = (l >> 4) & 1;
+        const uint16_t* from = tile + (32 * kh + 16 * s2 + 4 * lh + (s16 >> 2)) * kPitchV + 32 * t + 16 * g1 + 4 * (s16 & 3);
+        const s16x4 lo = lds_read_tr16(from), hi = lds_read_tr16(from + 8 * kPitchV);
+        typedef short s16x8_ __attribute__((ext_vector_type(8)));
+        *reinterpret_cast<s16x8_*>(out + (int64_t)e * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+}
+
+// Chunk means and row table of q, nothing else of it: a wavefront per chunk, no LDS, all of a lane's sixteen 16-byte loads
+// of a tile in flight at once.  Lane = (c16, r4): 16-byte piece c16 of the rows rg = 4 r4 .. 4 r4 + 3 and their likes 16, 32,
+// 48, ... slots on, summed in permute_kernel's order.
+template <bool kBf16>
+__device__ __forceinline__ void query_part(const PrepRows& x, const Grid3& g, int Hn, int64_t id, int64_t total) {
+    if (id >= total) return;
+    int blk, bh;
+    place((int)id, g.blocks(), Hn, x.head_fastest, blk, bh);
+    const int lane = threadIdx.x & 63, c16 = lane & 15, r4 = lane >> 4;
+    const char* src = reinterpret_cast<const char*>(x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH);
+    const int per_chunk = g.chunk() / kTile;
+    float part[4][8];                       // this lane's rows rg = 4 r4 + u
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part[u][e] = 0.f;
+    for (int sub = 0; sub < per_chunk; ++sub) {
+        const Slots s = slots_of(g, blk, sub, lane);
+        if (bh == 0 && x.rows != nullptr) x.rows[((int64_t)blk * per_chunk + sub) * kTile + lane] = s.token;
+        // every row unconditionally (a padded slot reads token 0 and is cleared afterwards): sixteen independent loads
+        // per lane, no branch between them
+        uint4 xs[4][4];
+        const int slot0 = 4 * r4;
+        if (x.offsets_32) {                 // one register per address instead of two
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t at = (uint32_t)max(__shfl(s.token, slot0 + u + 16 * i), 0) * (uint32_t)(x.sS * 2) + (uint32_t)c16 * 16u;
+                    xs[u][i] = *reinterpret_cast<const uint4*>(src + at);
+                }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    xs[u][i] = *reinterpret_cast<const uint4*>(src + (int64_t)max(__shfl(s.token, slot0 + u + 16 * i), 0) * (x.sS * 2) + c16 * 16);
+        }
+        if (s.word != ~0ull) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) keep_if(xs[u][i], (s.word >> (slot0 + u + 16 * i)) & 1ull);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) add_row<kBf16>(part[u], xs[u][i]);
+    }
+    // the sixteen partial sums of a column in ascending rg: four per lane, handed from r4 to r4 + 1
+    float sum[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+#pragma unroll
+    for (int stage = 0; stage < 4; ++stage) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float below = stage == 0 ? 0.f : __shfl_up(sum[e], 16);
+            if (r4 == stage) sum[e] = (((below + part[0][e]) + part[1][e]) + part[2][e]) + part[3][e];
+        }
+    }
+    if (r4 == 3) {
+        const float inv = 1.0f / g.chunk();
+        uint32_t out[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[e] = narrow<kBf16>(sum[2 * e] * inv) | ((uint32_t)narrow<kBf16>(sum[2 * e + 1] * inv) << 16);
+        *reinterpret_cast<uint4*>(x.pooled + ((int64_t)bh * g.blocks() + blk) * kD + c16 * 8) = make_uint4(out[0], out[1], out[2], out[3]);
+    }
+}
+
+constexpr int64_t kOneLaunchGroups = 8192;
+
+enum { kAllParts, kKeys, kValues, kQueries };
+template <bool kBf16, bool kTransform, int kPart>
+__global__ __launch_bounds__(256) void prepare_kernel(PrepArgs a, int wg_k, int wg_v, int64_t chunks_q) {
+    __shared__ __attribute__((aligned(16))) uint16_t tile[kPart == kQueries && !kTransform ? 8 : kTile * kPitchV];
+    __shared__ float2 cs[kTransform && kPart != kValues ? 8 * 64 : 1];
+    const int w = blockIdx.x;
+    if (kPart <= kKeys && w == 0 && threadIdx.x == 0 && a.zero != nullptr) *a.zero = 0u;
+    if (kPart == kKeys || (kPart == kAllParts && w < wg_k)) {
+        row_part<kBf16, kTransform>(a.k, a.gk, a.Hn, w, a.tab, a.tab_T, a.eps, tile, cs);
+        return;
+    }
+    if (kPart == kValues || (kPart == kAllParts && w < wg_k + wg_v)) {
+        value_part(a.v, a.gk, a.Hn, kPart == kValues ? w : w - wg_k, tile);
+        return;
+    }
+    const int wq = kPart == kQueries ? w : w - wg_k - wg_v;
+    if (kTransform) row_part<kBf16, true>(a.q, a.gq, a.Hn, wq, a.tab, a.tab_T, a.eps, tile, cs);
+    else query_part<kBf16>(a.q, a.gq, a.Hn, (int64_t)wq * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), chunks_q);
+}
+
+// the row table of q alone (the selection is the caller's): one workgroup per four tiles
+__global__ __launch_bounds__(256) void row_table_kernel(Grid3 g, int32_t* __restrict__ rows, int tiles) {
+    const int tile = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, per_chunk = g.chunk() / kTile;
+    if (tile < tiles) rows[(int64_t)tile * kTile + lane] = slots_of(g, tile / per_chunk, tile % per_chunk, lane).token;
+}
+
+}  // namespace
+
+hipError_t launch_prepare(const PrepArgs& args, int B, int dtype, hipStream_t st) {
+    PrepArgs a = args;
+    for (PrepRows* x : {&a.q, &a.k, &a.v}) x->head_fastest = x->sH < x->sS ? 1 : 0;
+    a.q.offsets_32 = ((int64_t)a.gq.T * a.gq.H * a.gq.W + 1) * a.q.sS * 2 < ((int64_t)1 << 32) ? 1 : 0;
+    const int64_t bh = (int64_t)B * a.Hn;
+    const bool transform = a.q.norm_w != nullptr || a.k.norm_w != nullptr || a.tab != nullptr;
+    const int64_t wg_k = a.k.p != nullptr ? bh * a.gk.blocks() : 0;
+    const int64_t wg_v = a.v.p != nullptr ? bh * a.gk.blocks() * (a.gk.chunk() / kTile) : 0;
+    const int64_t chunks_q = a.q.p != nullptr ? bh * a.gq.blocks() : 0;
+    const int64_t wg_q = transform ? chunks_q : (chunks_q + 3) / 4;
+    const int64_t total = wg_k + wg_v + wg_q;
+    if (total <= 0 || total > 0x7fffffff) return hipErrorInvalidValue;
+    const dim3 block(256);
+#define BSA_PREPARE(PART, N)                                                                                                        \
+    do {                                                                                                                            \
+        const dim3 grid((unsigned)(N));                                                                                             \
+        if (dtype == BSA_BF16 && transform) hipLaunchKernelGGL((prepare_kernel<true, true, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q); \
+        else if (dtype == BSA_BF16) hipLaunchKernelGGL((prepare_kernel<true, false, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);       \
+        else if (transform) hipLaunchKernelGGL((prepare_kernel<false, true, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);               \
+        else hipLaunchKernelGGL((prepare_kernel<false, false, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);       \
+    } while (0)
+    if (total <= kOneLaunchGroups) {
+        BSA_PREPARE(kAllParts, total);
+    } else {
+        if (wg_q > 0) BSA_PREPARE(kQueries, wg_q);
+        if (wg_k > 0) BSA_PREPARE(kKeys, wg_k);
+        if (wg_v > 0) BSA_PREPARE(kValues, wg_v);
+    }
+#undef BSA_PREPARE
+    return hipGetLastError();
+}
+
+hipError_t launch_row_table(const Grid3& g, int32_t* rows, hipStream_t st) {
+    const int tiles = g.blocks() * (g.chunk() / kTile);
+    hipLaunchKernelGGL(row_table_kernel, dim3((tiles + 3) / 4), dim3(256), 0, st, g, rows, tiles);
+    return hipGetLastError();
+}
+
+hipError_t launch_head_norm(const float* tile_norm, float* key_norm, int BH, int tiles, hipStream_t st) {
+    hipLaunchKernelGGL(head_norm_kernel, dim3((unsigned)BH), dim3(256), 0, st, tile_norm, key_norm, tiles);
+    return hipGetLastError();
+}
+
+// floats of the key norms: one per (batch, head), then (from a 256-byte boundary) one per tile
+size_t key_norm_floats(int B, int Hn, int64_t tiles) { return tile_norm_offset(B, Hn) + (size_t)B * Hn * (size_t)tiles; }
+
+}  // namespace bsa

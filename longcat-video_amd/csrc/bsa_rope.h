@@ -1,6 +1,6 @@
 // Per-head RMSNorm and 3-D RoPE of one (token, head) row of 128 elements held by 16 consecutive lanes, 8
 // elements (4 interleaved rotation pairs) per lane.  Shared by the stand-alone pass (bsa_glue.hip) and by the
-// passes that apply the same steps while they move q and k (bsa_fwd_frag.hip), so that every route rounds at the
+// passes that apply the same steps while they move q and k (bsa_prepare.hip), so that every route rounds at the
 // same points:
 //   x -> T(x * rsqrt(mean(x^2) + eps)) -> T(. * w) -> fp32 x*cos + rot(x)*sin -> T
 // with rot(x)[2i] = -x[2i+1], rot(x)[2i+1] = x[2i] (blocks.py:42-53, rope_3d.py:34-38, 112-120).  Every product

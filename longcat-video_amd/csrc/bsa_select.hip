@@ -33,10 +33,21 @@ using mfma::Vec8;
 // as 16-byte stores (half a row per lane) instead of 2-byte ones.
 constexpr int kScoreCols = 256;
 constexpr int kScorePitch = 128 + 8;     // elements: 272-byte rows keep 16-byte alignment and spread the banks
+// key_norm[bh] = the largest entry of the head's tile norms (a NaN row has no bound), by one wavefront
+__device__ inline void head_norm(const HeadNorms& n, int bh, int lane) {
+    float best = 0.f;
+    for (int i = lane; i < n.tiles; i += 64) {
+        const float x = n.tile_norm[(int64_t)bh * n.tiles + i];
+        best = x != x ? INFINITY : fmaxf(best, x);
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) best = fmaxf(best, __shfl_xor(best, off));
+    if (lane == 0) n.key_norm[bh] = best;
+}
 template <typename T>
 __global__ __launch_bounds__(256) void score_mfma_kernel(const T* __restrict__ qc,
                                                          const T* __restrict__ kc,
-                                                         T* __restrict__ score, int nbq, int nbk) {
+                                                         T* __restrict__ score, int nbq, int nbk, HeadNorms norms) {
     typedef typename Vec8<T>::type V8;
     constexpr int D = 128;
     __shared__ __attribute__((aligned(16))) T keys[kScoreCols * kScorePitch];
@@ -68,6 +79,7 @@ __global__ __launch_bounds__(256) void score_mfma_kernel(const T* __restrict__ q
 #pragma unroll
     for (int s = 0; s < 8; ++s) a[s] = *reinterpret_cast<const V8*>(qa + s * 16);
     __syncthreads();
+    if (norms.tile_norm != nullptr && blockIdx.x == 0 && blockIdx.y == gridDim.y - 1 && wave == 3) head_norm(norms, bh, lane);
     if (m0 >= nbq) return;                    // whole wavefront out of range (no workgroup barrier below)
     T (*mine)[40] = patch[wave];
     const bool vec_ok = (nbk % 8) == 0;       // rows of the score matrix stay 16-byte aligned
@@ -530,7 +542,7 @@ __host__ __device__ inline int gate_wave_words(int k_sel) { const int w = pace_w
 
 template <typename T, int NPL>
 __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict__ qc, const T* __restrict__ kc, int32_t* __restrict__ lists,
-                                                            int32_t* __restrict__ lens, int nbq, int nbk, int k_sel, int paced) {
+                                                            int32_t* __restrict__ lens, int nbq, int nbk, int k_sel, int paced, HeadNorms norms) {
     typedef typename GateRows<T>::bits S;
     constexpr int D = 128, R = GateRows<T>::kRows;
     extern __shared__ __attribute__((aligned(16))) unsigned char gate_lds[];
@@ -539,6 +551,7 @@ __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict_
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t* const mine = reinterpret_cast<uint32_t*>(gate_lds + (size_t)R * pitch * sizeof(T)) + wave * words;
     const int bh = blockIdx.y, m0 = blockIdx.x * R;
+    if (norms.tile_norm != nullptr && wave == kGateThreads / 64 - 1 && blockIdx.x == 0 && blockIdx.z == 0) head_norm(norms, bh, lane);
     const T* qb = qc + (int64_t)bh * nbq * D;
     const T* kb = kc + (int64_t)bh * nbk * D;
     if constexpr (sizeof(T) == 2) {
@@ -610,7 +623,7 @@ size_t gate_lds_bytes(int nbk, int k_sel) {
 
 template <typename T>
 hipError_t launch_gate_t(const T* qc, const T* kc, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel, bool paced,
-                         hipStream_t st) {
+                         hipStream_t st, HeadNorms norms) {
     const size_t lds = gate_lds_bytes<T>(nbk, k_sel);
     const int blocks = (nbq + GateRows<T>::kRows - 1) / GateRows<T>::kRows;
     const int halves = GateRows<T>::kRows > kGateThreads / 64 && blocks * BH <= kGateMaxGroups / 2 ? 2 : 1;
@@ -621,7 +634,7 @@ hipError_t launch_gate_t(const T* qc, const T* kc, int32_t* lists, int32_t* lens
             const hipError_t ea = hipFuncSetAttribute((const void*)gate_kernel<T, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
             if (ea != hipSuccess) return ea;                                                                                 \
         }                                                                                                                    \
-        hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0);  \
+        hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0, norms);  \
     } while (0)
     if (nbk <= 64) BSA_GATE(1);
     else if (nbk <= 128) BSA_GATE(2);
@@ -777,7 +790,7 @@ hipError_t launch_topk_t(const S* score, int32_t* idx, int32_t* idx_sorted, int3
 }  // namespace
 
 hipError_t launch_score(const void* q_cmp, const void* k_cmp, void* score, int BH, int nbq, int nbk,
-                        int D, int dtype, hipStream_t st) {
+                        int D, int dtype, hipStream_t st, HeadNorms norms) {
     if (dtype == BSA_F32) {
         dim3 grid((nbk + 63) / 64, (nbq + 15) / 16, BH);
         hipLaunchKernelGGL(score_f32_kernel, grid, dim3(256), 0, st, (const float*)q_cmp,
@@ -786,10 +799,10 @@ hipError_t launch_score(const void* q_cmp, const void* k_cmp, void* score, int B
         dim3 grid((nbk + kScoreCols - 1) / kScoreCols, (nbq + 127) / 128, BH);
         if (dtype == BSA_BF16)
             hipLaunchKernelGGL((score_mfma_kernel<__bf16>), grid, dim3(256), 0, st,
-                               (const __bf16*)q_cmp, (const __bf16*)k_cmp, (__bf16*)score, nbq, nbk);
+                               (const __bf16*)q_cmp, (const __bf16*)k_cmp, (__bf16*)score, nbq, nbk, norms);
         else
             hipLaunchKernelGGL((score_mfma_kernel<_Float16>), grid, dim3(256), 0, st,
-                               (const _Float16*)q_cmp, (const _Float16*)k_cmp, (_Float16*)score, nbq, nbk);
+                               (const _Float16*)q_cmp, (const _Float16*)k_cmp, (_Float16*)score, nbq, nbk, norms);
     }
     return hipGetLastError();
 }
@@ -810,10 +823,10 @@ bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype) {
 }
 
 hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
-                       bool paced, int dtype, hipStream_t st) {
-    if (dtype == BSA_F32) return launch_gate_t<float>((const float*)q_cmp, (const float*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st);
-    if (dtype == BSA_BF16) return launch_gate_t<__bf16>((const __bf16*)q_cmp, (const __bf16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st);
-    return launch_gate_t<_Float16>((const _Float16*)q_cmp, (const _Float16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st);
+                       bool paced, int dtype, hipStream_t st, HeadNorms norms) {
+    if (dtype == BSA_F32) return launch_gate_t<float>((const float*)q_cmp, (const float*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms);
+    if (dtype == BSA_BF16) return launch_gate_t<__bf16>((const __bf16*)q_cmp, (const __bf16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms);
+    return launch_gate_t<_Float16>((const _Float16*)q_cmp, (const _Float16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms);
 }
 
 hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* lens, int64_t rows, int nbk, int stride,
