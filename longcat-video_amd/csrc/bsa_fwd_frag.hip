@@ -106,8 +106,12 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     int32_t* __restrict__ fallback, uint32_t* __restrict__ fallback_count) {
     typedef typename Vec8<T>::type V8;
     // log2 headroom before the running maximum is raised: probabilities reach 2^kTau, which the storage type of P
-    // must hold (fp16 ends at 65 504) and the fp32 sums must hold times the number of keys
-    constexpr float kTau = std::is_same<T, _Float16>::value ? 14.0f : 30.0f;
+    // must hold (fp16 ends at 65 504 = 2^15.99) and the fp32 sums must hold times the number of keys
+    constexpr float kTau = std::is_same<T, _Float16>::value ? 15.5f : 30.0f;
+    // How far the fixed reference of an item without row maxima may lie above the largest logit of its first keys (see
+    // where the bound is tested): the largest probability of a row is then at least 2^-kSlack.  bf16 has fp32's exponents;
+    // fp16 loses relative precision below 2^-14, 2^-10 of that largest probability.
+    constexpr float kSlack = std::is_same<T, _Float16>::value ? 4.0f : 60.0f;
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     if (gate != nullptr && *gate != gate_want) return;
     // output staging: 64 rows of 256 B, 272 B apart.  The same memory stages a list that is too long for the small
@@ -575,18 +579,27 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             rescale_pending = false;                                     // nothing accumulated yet
 
             // Cauchy-Schwarz: no logit of this item exceeds |q| times the largest key norm of the head.  If that bound
-            // lies below the level at which the running maximum would be raised - for every query of the item, with
-            // the maximum the first 32 keys have set - no later step can raise it, and the steps of this kernel, which
-            // do not look at the row maxima (a fifth of the softmax instructions), give the same result.  An item
-            // without such a bound (a first half tile of padding, norms far above the logits) is left to the kernel
-            // that does look: it is put on the fallback list, nothing of it is stored, and the item after it
-            // starts from scratch.
+            // lies below the level at which the running maximum would be raised, no later step can raise it, and the steps
+            // of this kernel, which do not look at the row maxima (a fifth of the softmax instructions), give the same
+            // result.  A bound above that level moves the reference up to where it holds, unless the probabilities would
+            // then start too low (kSlack): such an item (a first half tile of padding, norms far above the logits) is left
+            // to the kernel that does look: it is put on the fallback list, nothing of it is stored, and the item
+            // after it starts from scratch.
             if constexpr (kBounded) {
-                float qn[2];
-#pragma unroll
-                for (int qq = 0; qq < 2; ++qq) qn[qq] = __builtin_sqrtf(q_sq[qq] + __shfl_xor(q_sq[qq], 32)) * 1.001f;   // both halves of the row's d
                 const float kn = __uint_as_float((uint32_t)uni((int)__float_as_uint(cur.kn)));
-                run = __all(qn[0] * kn <= raise_at[0] && qn[1] * kn <= raise_at[1]);
+                bool fits[2];
+#pragma unroll
+                for (int qq = 0; qq < 2; ++qq) {
+                    const float bound = __builtin_sqrtf(q_sq[qq] + __shfl_xor(q_sq[qq], 32)) * 1.001f * kn * qk_scale;   // both halves of the row's d
+                    const float lowest = m_i[qq] == -INFINITY ? -bound : m_i[qq];       // the row's largest logit is no smaller
+                    const float ref = bound - kTau;
+                    fits[qq] = ref <= lowest + kSlack;                                  // false for a NaN
+                    if (ref > m_i[qq]) {
+                        m_i[qq] = ref;
+                        neg_m[qq] = -ref;
+                    }
+                }
+                run = __all(fits[0] && fits[1]);
                 if (!run && lane == 0) fallback[atomicAdd(fallback_count, 1u)] = cur.item;
             }
             if (run) {
@@ -800,13 +813,14 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
             else BSA_FRAG_LAUNCH_T(_Float16, false, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);        \
         }                                                                                                              \
     } while (0)
+    if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
     if (queue != nullptr && one_span) {
         launch_schedule_choice(lens, (int)(Sq / bs_q), bs_q / kTile, total, resident, resident, idx_stride, queue, st);
         gate = queue + 1;
         const dim3 grid((unsigned)(total < resident ? total : resident));
-        BSA_FRAG_LAUNCH(false, grid, 0, total, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
+        if (bounded) BSA_FRAG_LAUNCH(true, grid, 0, total, order, queue, 1u, 0, whole_span, fb_list, fb_count);
+        else BSA_FRAG_LAUNCH(false, grid, 0, total, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
     }
-    if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
     // kRoundsPerLaunch rounds per launch, every workgroup running one item of each: the items of a round start
     // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
     const int span = (idx_stride * (bs_k / kTile) <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
