@@ -305,6 +305,7 @@ int bsa_fwd_fragment(const void* q, const void* k, const void* v, const int32_t*
     a.k.tile_norm = knorm + tile_norm_offset(B, Hn);
     a.v = prep_rows(v, kv_st);
     a.v.frag = vf;
+    a.k.valid_in = a.v.valid_in = tile_valid;
     a.zero = reinterpret_cast<uint32_t*>(fallback);
     hipError_t e = launch_prepare(a, B, dtype, st);
     if (e == hipSuccess) e = launch_head_norm(a.k.tile_norm, knorm, B * Hn, (int)(Sk / 64), st);
@@ -364,10 +365,11 @@ struct Plan {
     int64_t Sqp, Skp;
     int nbq, nbk, es;
     int sel_width;        // columns of the index lists: k_sel, or the cap of the CDF rule
+    int half_width;       // ... of the lists of 32-key halves that a padded grid is walked with; 0: block lists
     bool cdf;
     bool f32, direct_kv;
     bool frag;            // k and v are rewritten in fragment order for fwd_frag_kernel (bsa_fwd_frag.hip)
-    size_t off_kp, off_vp, off_qc, off_kc, off_score, off_idx, off_idx_sorted, off_lens, off_valid, off_qrows, off_krows, off_ktiles, off_order, off_queue, off_knorm, off_fallback, total;
+    size_t off_kp, off_vp, off_qc, off_kc, off_score, off_idx, off_idx_sorted, off_lens, off_valid, off_qrows, off_krows, off_ktiles, off_order, off_queue, off_knorm, off_fallback, off_halves, off_half_lens, total;
 };
 inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -426,6 +428,13 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->off_queue = take(pl->cdf && !pl->f32 ? 2 * sizeof(uint32_t) : 0);    // the counter and the choice of schedule
     pl->off_knorm = take(pl->frag ? key_norm_floats(p->B, p->Hn, pl->Skp / 64) * sizeof(float) : 0);   // key norms per head and tile
     pl->off_fallback = take(pl->frag ? frag_fallback_ints((int64_t)bh * (pl->Sqp / 64)) * sizeof(int32_t) : 0);
+    // On a padded grid the attention kernel walks lists of the halves that hold keys (a list of 4 096 halves still fits its
+    // LDS; longer ones, CDF rows over huge grids, keep the blocks and walk the padding).
+    const bool padded = (p->Tk % p->tk) || (p->Hk % p->hk) || (p->Wk % p->wk);
+    const int64_t halves = 2 * (int64_t)pl->sel_width * (pl->gk.chunk() / 64);
+    pl->half_width = pl->frag && padded && halves <= 4096 ? (int)halves : 0;
+    pl->off_halves = take(bh * pl->nbq * (size_t)pl->half_width * sizeof(int32_t));
+    pl->off_half_lens = take(pl->half_width > 0 ? bh * pl->nbq * sizeof(int32_t) : 0);
     pl->total = off;
     return BSA_OK;
 }
@@ -445,6 +454,7 @@ struct Ws {
     uint64_t* valid;
     float* knorm;
     int32_t* fallback;
+    int32_t *halves, *half_lens;
 };
 int carve(const Plan& pl, void* workspace, size_t workspace_bytes, const char* who, Ws* w) {
     if (!workspace) return set_error(BSA_ERR_BAD_ARG, "%s: workspace is null", who);
@@ -464,6 +474,8 @@ int carve(const Plan& pl, void* workspace, size_t workspace_bytes, const char* w
     w->order = pl.cdf && !pl.f32 ? reinterpret_cast<int32_t*>(ws + pl.off_order) : nullptr;
     w->queue = pl.cdf && !pl.f32 ? reinterpret_cast<uint32_t*>(ws + pl.off_queue) : nullptr;
     w->knorm = pl.frag ? reinterpret_cast<float*>(ws + pl.off_knorm) : nullptr;
+    w->halves = pl.half_width > 0 ? reinterpret_cast<int32_t*>(ws + pl.off_halves) : nullptr;
+    w->half_lens = pl.half_width > 0 ? reinterpret_cast<int32_t*>(ws + pl.off_half_lens) : nullptr;
     w->fallback = pl.frag ? reinterpret_cast<int32_t*>(ws + pl.off_fallback) : nullptr;
     return BSA_OK;
 }
@@ -539,11 +551,11 @@ hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, cons
 hipError_t attention_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, const void* q, const int64_t q_strides[3],
                          const void* k, const int64_t k_strides[3], const void* v, const int64_t v_strides[3], void* o,
                          const int64_t o_strides[3], const int32_t* idx, const int32_t* lens, int idx_stride, float* lse,
-                         hipStream_t st, bool by_length = false, bool fallback_cleared = false) {
+                         hipStream_t st, bool by_length = false, bool fallback_cleared = false, bool halves = false) {
     if (pl.frag)
         return launch_fwd_frag(q, w.kp, w.vp, idx, lens, kv_padded(p) ? w.valid : nullptr, o, lse, p->B, p->Hn, pl.Sqp, pl.Skp,
                                pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype, st, w.qrows, q_strides, o_strides,
-                               (int64_t)p->Tq * p->Hq * p->Wq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared);
+                               (int64_t)p->Tq * p->Hq * p->Wq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves);
     FwdLayout L;
     L.q_rows = w.qrows;
     L.k_tiles = w.ktiles;
@@ -651,8 +663,9 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     // caller asks for the selection
     const int64_t sel_rows = (int64_t)p->B * p->Hn * pl.nbq;
     const HeadNorms norms = {pl.frag ? w.knorm + tile_norm_offset(p->B, p->Hn) : nullptr, w.knorm, (int)(pl.Skp / 64)};
+    const HalfLists halves = {w.valid, pl.gk.chunk() / 64, w.halves, w.half_lens, pl.half_width};
     if (!pl.cdf && idx_out == nullptr && score_out == nullptr && gate_fits(p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, p->dtype)) {
-        BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st, norms), "gate");
+        BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st, norms, halves), "gate");
     } else {
         BSA_HIP(launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st, norms), "score");
         if (pl.cdf) {
@@ -663,14 +676,17 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
             BSA_HIP(launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, p->k_sel, p->dtype, st), "top-k");
         }
         if (pl.frag && pl.sel_width > 0)
-            BSA_HIP(launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st), "visit order");
+            BSA_HIP(launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st, halves), "visit order");
     }
     if (!pl.f32) {
         // lists of unequal length: one launch whose workgroups draw the items, longest lists first
+        const bool by_half = w.halves != nullptr;
+        const int32_t *walk = by_half ? w.halves : w.idx_sorted, *walk_lens = by_half ? w.half_lens : w.lens;
+        const int walk_width = by_half ? pl.half_width : pl.sel_width;
         if (pl.cdf)
-            BSA_HIP(launch_order_by_length(w.lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, pl.sel_width, st), "order by length");
-        BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, w.idx_sorted, w.lens, pl.sel_width,
-                              lse_out, st, pl.cdf, pl.frag), "attention");
+            BSA_HIP(launch_order_by_length(walk_lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, walk_width, st), "order by length");
+        BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, walk, walk_lens, walk_width,
+                              lse_out, st, pl.cdf, pl.frag, by_half), "attention");
     } else {
         F32Layout L;
         L.q_rows = w.qrows; L.k_rows = w.krows;

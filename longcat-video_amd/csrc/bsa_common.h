@@ -121,12 +121,21 @@ hipError_t launch_score(const void* q_cmp, const void* k_cmp, void* score, int B
 hipError_t launch_topk(const void* score, int32_t* idx, int32_t* idx_sorted, int32_t* lens, int64_t rows,
                        int nbk, int k_sel, int dtype, hipStream_t st, const int32_t* k_rows = nullptr,
                        int stride = 0);
+// Lists of 32-key halves for the attention kernel's walk over a padded grid (launch_fwd_frag, halves), written next to the
+// visiting order: rows of `stride` entries (even, at least twice the tiles of a list), lens = entries in use.
+struct HalfLists {
+    const uint64_t* valid;       // validity words of the KV tiles
+    int nsub;                    // tiles per KV block
+    int32_t* lists;              // null: not wanted
+    int32_t* lens;
+    int stride;
+};
 // Scores, top-k and (with `paced`) visiting order of a small call in one launch: lists [BH][nbq][k_sel], ascending or in
 // visiting order, lens = k_sel.  The same lists as launch_score, launch_topk and launch_pace_order; gate_fits says for
 // which sizes it is built and the better choice.
 bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype);
 hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
-                       bool paced, int dtype, hipStream_t st, HeadNorms norms = {nullptr, nullptr, 0});
+                       bool paced, int dtype, hipStream_t st, HeadNorms norms = {nullptr, nullptr, 0}, HalfLists halves = {});
 // lens[row] = number of columns the CDF rule keeps, clamped to [k_min, cap]
 hipError_t launch_cdf_count(const void* score, int32_t* lens, int64_t rows, int nbk, float threshold,
                             float scale, int k_min, int cap, int dtype, hipStream_t st);
@@ -152,7 +161,7 @@ hipError_t launch_fwd_f32(const void* q, const void* k, const void* v, const int
 // Rewrites every row's ascending list of KV blocks into the order the attention kernel visits them in (see
 // pace_order_kernel).  rows of `stride` entries, lens[row] of them in use; in == out allowed; stride <= 5000.
 hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* lens, int64_t rows, int nbk, int stride,
-                             hipStream_t st);
+                             hipStream_t st, HalfLists halves = {});
 // order: for every (batch, head) its 64-row query tiles by descending list length (lens is per query
 // block of tiles_per_block tiles, clamped to [0, max_len]); with `order` and a two-word `queue`
 // launch_fwd enqueues the 16-bit kernel both as rounds and as one launch whose workgroups draw items
@@ -169,10 +178,11 @@ void launch_schedule_choice(const int32_t* lens, int nbq, int tiles_per_block, i
 struct PrepRows {
     const uint16_t* p;               // null: this part is left out
     int64_t sB, sH, sS;              // batch, head, token
-    char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, padded slots zero
+    char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, the real slots of a tile first, zeros behind
     uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
-    int32_t* rows;                   // q: token row of every blocked-order slot of one (batch, head), -1 = padding
+    int32_t* rows;                   // q: token row of every slot of one (batch, head), -1 = padding; the real ones of a tile first
     uint64_t* valid;                 // k, optional: bit s of word i = slot 64 i + s holds a real token
+    const uint64_t* valid_in;        // k, v, optional: the real slots of every tile as the caller has them (instead of the grid's)
     float* tile_norm;                // k, optional: largest Euclidean norm of a row of every tile, a part in a thousand above
     const uint16_t* norm_w;          // q, k, optional: 128 weights of a per-head RMSNorm that the rows go through first
     int t0;                          // q, k: frame offset of the grid inside the rotation table
@@ -203,10 +213,11 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
-                           int32_t* fallback = nullptr, bool fallback_cleared = false);
+                           int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false);
 // fallback (optional, frag_fallback_ints(B * Hn * Sq / 64) int32): with it and key_norm the rounds run the kernel that
 // takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.  Its first word
 // counts them: fallback_cleared says that it is zero already.
+// halves: idx and lens are HalfLists, idx_stride their row pitch (at most 4 096).
 size_t frag_fallback_ints(int64_t items);
 
 

@@ -44,6 +44,7 @@ using namespace mfma;
 
 constexpr int kHalfBytes = 8192;      // 32 keys of a fragment-order K (or V) tile
 constexpr int kListEntries = 4096;    // longest list a work item can walk (its staging area in LDS: 17 KB)
+constexpr int kHalfEntries = 4096;    // ... of halves
 
 // ------------------------------------------------------------------ attention
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant expression
@@ -77,7 +78,13 @@ struct FragLayout {
 // Lists of at most this many entries are staged in LDS for the next work item while the current one runs.
 constexpr int kPipeList = 256;
 
-// kNsub1: KV blocks of one 64-key tile (bs_k == 64): no division in the walk.
+// How an item's keys are listed (kWalk).  The walk goes in pairs of 32-key halves:
+//   kTiles:  idx holds KV blocks of one 64-key tile (bs_k == 64; no division in the walk), a pair is a tile;
+//   kBlocks: KV blocks of several tiles;
+//   kHalves: idx holds the halves themselves, empty ones left out: half of the (batch, head) | real keys << 20, an even
+//            number of entries (the last may repeat a half with no key), lens counts them without such a repeat.
+// The real keys of a tile come first (prepare_kernel), so its validity is a count.  Leaving out a half whose
+// probabilities would all be 0 changes no bit of the result: the sums run over the same numbers in the same order.
 //
 // A workgroup (one wavefront) runs the work items b, b + round, b + 2 round, ... of its launch one after the other
 // (or draws them from `queue`).  What an item needs before its first MFMA - its list, its Q rows, its first K and
@@ -95,7 +102,11 @@ constexpr int kPipeList = 256;
 // (see where the bound is tested): its steps take no row maxima.  An item that fails the test is not computed but
 // appended to `fallback` (its count in fallback_count), and the other instantiation, which takes its items from that
 // list, runs behind it.
-template <typename T, bool kNsub1, bool kBounded>
+enum { kTiles, kBlocks, kHalves };
+constexpr uint32_t kHalfId = 0xfffff;     // of a kHalves entry: the half; above it: its number of real keys
+constexpr int kHalfCountShift = 20;
+
+template <typename T, int kWalk, bool kBounded>
 __global__ __launch_bounds__(64) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
     const int32_t* __restrict__ idx, const int32_t* __restrict__ lens, const uint64_t* __restrict__ tile_valid,
@@ -118,7 +129,8 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // buffers (kListEntries words at most) during the tile loop of an item that was not prepared ahead of time.
     constexpr int kOutPitch = kD + 8;
     __shared__ __attribute__((aligned(16))) T ost[kTile * kOutPitch];
-    __shared__ uint32_t lists[2][kPipeList];
+    constexpr int kWords = kWalk == kHalves ? 2 : 1;              // list words of a pair
+    __shared__ __attribute__((aligned(8))) uint32_t lists[2][kPipeList * kWords];
     __shared__ int32_t out_rows[2][kTile];       // token rows of this and the next item's 64 query slots (row table given)
     __shared__ __attribute__((aligned(16))) char qstage[kTileBytes];      // Q of the next item, in register order
     uint32_t* const big = reinterpret_cast<uint32_t*>(ost);
@@ -127,7 +139,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     const int lr = lane & 31, lh = lane >> 5;
     const int nbq = (int)(Sq / bs_q);
     const int nqt = (int)(Sq / kTile);
-    const int nsub = kNsub1 ? 1 : bs_k / kTile;
+    const int nsub = kWalk == kBlocks ? bs_k / kTile : 1;
     const int nbk = (int)(Sk / bs_k);
     const int tiles_bh = (int)(Sk / kTile);
     const uint32_t lane_off = (uint32_t)lane * 16u;
@@ -141,13 +153,13 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kf) + bh_first * kv_bh_bytes, 0, (int)kv_span_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t vrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vf) + bh_first * kv_bh_bytes, 0, (int)kv_span_bytes, 0x00020000);
-    // tile: index of the 64-key tile counted from (batch, head) bh_first; h: its half; c / f: fragment of the half
-    auto k_frag = [&](uint32_t tile, int h, int c) -> V8 {
-        const uint32_t so = tile * (uint32_t)kTileBytes + (uint32_t)(h * kHalfBytes + (c >> 2) * 4096);
+    // half: index of the 32-key half counted from (batch, head) bh_first; c / f: fragment of the half
+    auto k_frag = [&](uint32_t half, int c) -> V8 {
+        const uint32_t so = half * (uint32_t)kHalfBytes + (uint32_t)((c >> 2) * 4096);
         return __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(krs, lane_off + (uint32_t)((c & 3) * 1024), so, 0));
     };
-    auto v_frag = [&](uint32_t tile, int h, int f) -> V8 {          // f = 4 * key step + d tile
-        const uint32_t so = tile * (uint32_t)kTileBytes + (uint32_t)(h * kHalfBytes + (f >> 2) * 4096);
+    auto v_frag = [&](uint32_t half, int f) -> V8 {          // f = 4 * key step + d tile
+        const uint32_t so = half * (uint32_t)kHalfBytes + (uint32_t)((f >> 2) * 4096);
         return __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(vrs, lane_off + (uint32_t)((f & 3) * 1024), so, 0));
     };
 
@@ -171,15 +183,18 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     auto next_local = [&]() -> int { return queue != nullptr ? draw() : round_local(rounds_taken++); };
     // what is known of an item ahead of time: its number, the length of its list and its first entry (both as
     // they lie in memory; they are clamped where they are used)
-    struct Desc { int item, nent, blk0; float kn; };
+    struct Desc { int item, nent, ent[2]; float kn; };              // ent: the first list entry (kHalves: the first two)
     auto fetch = [&](int local) -> Desc {
-        Desc d = {-1, 0, 0, INFINITY};
+        Desc d = {-1, 0, {0, 0}, INFINITY};
         if (local < 0) return d;
         d.item = item_begin + (order != nullptr ? order[local] : local);
         const int bh = d.item / nqt, qblock = (int)((int64_t)(d.item % nqt) * kTile / bs_q);
         const int64_t row = (int64_t)bh * nbq + qblock;
         d.nent = lens[row];
-        if (idx_stride > 0) d.blk0 = idx[row * idx_stride];
+        if (idx_stride > 0) {
+            d.ent[0] = idx[row * idx_stride];
+            if (kWalk == kHalves) d.ent[1] = idx[row * idx_stride + 1];
+        }
         if (key_norm != nullptr) d.kn = key_norm[bh];
         return d;
     };
@@ -187,10 +202,22 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // does not use the scalar cache): the values are the same in every lane and are made scalars where they are used,
     // not where they are loaded, so that the wait for them stands there.
     auto uni = [](int x) -> int { return __builtin_amdgcn_readfirstlane(x); };
-    auto list_length = [&](const Desc& d) -> int { return d.item < 0 ? 0 : min(min(max(uni(d.nent), 0), idx_stride), kListEntries); };
-    auto first_tile = [&](const Desc& d) -> uint32_t {              // the tile position 0 of d's walk names
-        const int bh = d.item / nqt;
-        return (uint32_t)((bh - bh_first) * tiles_bh + min(max(uni(d.blk0), 0), nbk - 1) * nsub);
+    // list words in use
+    auto list_length = [&](const Desc& d) -> int {
+        if (d.item < 0) return 0;
+        const int n = min(max(uni(d.nent), 0), idx_stride);
+        return kWalk == kHalves ? (n + 1) & ~1 : min(n, kListEntries);
+    };
+    // the pair of halves that position 0 of d's walk names
+    auto first_pair = [&](const Desc& d, uint32_t (&h)[2]) {
+        const uint32_t base = (uint32_t)((d.item / nqt - bh_first) * tiles_bh) * 2u;
+        if (kWalk == kHalves) {
+            h[0] = base + ((uint32_t)uni(d.ent[0]) & kHalfId);
+            h[1] = base + ((uint32_t)uni(d.ent[1]) & kHalfId);
+        } else {
+            h[0] = base + (uint32_t)(min(max(uni(d.ent[0]), 0), nbk - 1) * nsub) * 2u;
+            h[1] = h[0] + 1u;
+        }
     };
 
     // ---- registers that live across items
@@ -234,42 +261,60 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     };
 
     // ---- per item
-    int ntiles = 0;
-    uint32_t tile_base = 0;          // first tile of the item's (batch, head)
-    uint32_t beyond_tile = 0;        // what the positions behind the end of the list name
+    int npairs = 0;
+    uint32_t half_base = 0;          // first half of the item's (batch, head)
+    uint32_t beyond[2] = {0, 0};     // what the positions behind the end of the list name
     const uint32_t* ents = big;      // the item's list in LDS
-    // window of the walk: positions g, g + 1, g + 2 of loop iteration g (one tile per iteration)
-    uint32_t w_tile[3];
-    uint64_t w_mask[3];
+    // window of the walk: the halves 2 g + 1 .. 2 g + 5 of loop iteration g (one pair per iteration) and the keys to keep
+    uint32_t w_half[5], w_mask[5];
 
-    // Position tp of the tile walk -> tile and validity word of its 64 keys.  Positions behind the list name
-    // `beyond_tile` with every key masked out.  The entry is read from LDS (entry_raw, to be issued early) and
-    // decoded later (entry_tile / entry_mask).
-    auto entry_raw = [&](int tp) -> uint32_t {
-        const int tc = min(tp, ntiles - 1);
-        return ents[kNsub1 ? tc : tc / nsub];                   // the same address in every lane
+    // Pair tp of the walk -> its halves and the keys of theirs that count (bit i: key i).  Positions behind the list name
+    // `beyond` with every key masked out.  The entry is read from LDS (pair_raw, to be issued early) and decoded later.
+    struct Raw { uint32_t e[kWords]; };
+    auto pair_raw = [&](int tp) -> Raw {
+        const int tc = min(tp, npairs - 1);
+        Raw r;
+        if constexpr (kWalk == kHalves) {
+            const uint2 x = *reinterpret_cast<const uint2*>(ents + 2 * tc);               // the same address in every lane
+            r.e[0] = x.x; r.e[1] = x.y;
+        } else {
+            r.e[0] = ents[kWalk == kTiles ? tc : tc / nsub];
+        }
+        return r;
     };
-    auto entry_tile = [&](int tp, uint32_t raw) -> uint32_t {
-        if (tp >= ntiles) return beyond_tile;
-        const int blk = min(max(__builtin_amdgcn_readfirstlane((int)raw), 0), nbk - 1);   // a malformed list: wrong numbers, never a fault
-        if (kNsub1) return tile_base + (uint32_t)blk;
-        return tile_base + (uint32_t)(blk * nsub + tp % nsub);
+    auto count_mask = [&](int n) -> uint64_t { return n >= 64 ? ~0ull : ((uint64_t)1 << n) - 1; };
+    auto pair_halves = [&](int tp, const Raw& raw, uint32_t (&h)[2]) {
+        if (kWalk == kHalves) {
+#pragma unroll
+            for (int x = 0; x < kWords; ++x)
+                h[x] = tp >= npairs ? beyond[x] : half_base + ((uint32_t)uni((int)raw.e[x]) & kHalfId);
+            return;
+        }
+        if (tp >= npairs) { h[0] = beyond[0]; h[1] = beyond[1]; return; }
+        const int blk = min(max(uni((int)raw.e[0]), 0), nbk - 1);                          // a malformed list: wrong numbers, never a fault
+        h[0] = half_base + 2u * (uint32_t)(kWalk == kTiles ? blk : blk * nsub + tp % nsub);
+        h[1] = h[0] + 1u;
     };
-    // the validity word of a tile (all keys valid without padding), in two steps so that a caller can ask for several
-    // words before it waits for the first
-    auto entry_word = [&](int tp, uint32_t tile) -> uint64_t {
-        if (tile_valid == nullptr) return ~0ull;
-        return tile_valid[tp >= ntiles ? 0u : tile - tile_base];                        // behind the list: another head's tile
+    // the validity word of a pair's tile (all keys valid without padding; kHalves: the entries say it), in two steps so that
+    // a caller can ask for several words before it waits for the first
+    auto pair_word = [&](int tp, const uint32_t (&h)[2]) -> uint64_t {
+        if (kWalk == kHalves || tile_valid == nullptr) return ~0ull;
+        return tile_valid[tp >= npairs ? 0u : (h[0] - half_base) >> 1];                    // behind the list: another head's tile
     };
-    auto mask_of = [&](int tp, uint64_t word) -> uint64_t {
+    auto pair_masks = [&](int tp, const Raw& raw, uint64_t word, uint32_t (&m)[2]) {
+        const uint32_t keep = tp >= npairs ? 0u : ~0u;
+        if (kWalk == kHalves) {
+#pragma unroll
+            for (int x = 0; x < kWords; ++x) m[x] = (uint32_t)count_mask(uni((int)raw.e[x]) >> kHalfCountShift) & keep;
+            return;
+        }
         // the same word in every lane; made a scalar by hand (behind the stores of an earlier item's output the
         // compiler reads it with a vector load)
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)word);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(word >> 32));
-        const uint32_t keep = tp >= ntiles ? 0u : ~0u;
-        return (uint64_t)(lo & keep) | ((uint64_t)(hi & keep) << 32);
+        const uint32_t lo = (uint32_t)uni((int)(uint32_t)word), hi = (uint32_t)uni((int)(uint32_t)(word >> 32));
+        const uint64_t front = count_mask(__builtin_popcountll((uint64_t)lo | ((uint64_t)hi << 32)));
+        m[0] = (uint32_t)front & keep;
+        m[1] = (uint32_t)(front >> 32) & keep;
     };
-    auto entry_mask = [&](int tp, uint32_t tile) -> uint64_t { return mask_of(tp, entry_word(tp, tile)); };
     // accumulator i <-> key 8 (i / 4) + 4 lh + i % 4 of the step's 32 keys, query lr (+32)
     auto mask_pair = [&](f32x16 (&sv)[2], uint32_t half) {
         if (__builtin_expect(half != ~0u, 0)) {
@@ -389,15 +434,15 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             // arithmetic cost more issue time than they take): V_B(u+1), K(u+3), V_A(u+2)
             if constexpr (slot == 7) {
 #pragma unroll
-                for (int tt = 1; tt <= 4; ++tt) vb[vprev][4 + (tt & 3)] = v_frag(w_tile[(j + 1) >> 1], (j + 1) & 1, 4 + (tt & 3));
+                for (int tt = 1; tt <= 4; ++tt) vb[vprev][4 + (tt & 3)] = v_frag(w_half[j], 4 + (tt & 3));
             }
             if constexpr (slot == 23) {
 #pragma unroll
-                for (int cc = 1; cc <= 8; ++cc) kb[kslot][cc & 7] = k_frag(w_tile[(j + 3) >> 1], (j + 1) & 1, cc & 7);
+                for (int cc = 1; cc <= 8; ++cc) kb[kslot][cc & 7] = k_frag(w_half[j + 2], cc & 7);
             }
             if constexpr (slot == 31) {
 #pragma unroll
-                for (int tt = 1; tt <= 4; ++tt) vb[vcur][tt & 3] = v_frag(w_tile[(j + 2) >> 1], j & 1, tt & 3);
+                for (int tt = 1; tt <= 4; ++tt) vb[vcur][tt & 3] = v_frag(w_half[j + 1], tt & 3);
             }
             if constexpr (slot == 7) {
                 if (__builtin_expect(rescale_pending, 0)) rescale_out();
@@ -416,8 +461,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 if constexpr (r == 1) {
                     mfma_chain_end(s[sn][0]);
                     mfma_chain_end(s[sn][1]);
-                    // validity of the keys of step u + 1: tile window slot (j + 1) / 2, half (j + 1) & 1
-                    mask_pair(s[sn], (uint32_t)(w_mask[(j + 1) >> 1] >> (32 * ((j + 1) & 1))));
+                    mask_pair(s[sn], w_mask[j]);               // the keys of step u + 1
                     if constexpr (!kBounded) {
                         mx[0] = fmaxf(fmaxf(s[sn][0][0], s[sn][0][1]), s[sn][0][2]);
                         mx[1] = fmaxf(fmaxf(s[sn][1][0], s[sn][1][1]), s[sn][1][2]);
@@ -457,13 +501,19 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         const int qblock = (int)(qrow0 / bs_q);
         const int64_t o_bh = (int64_t)(bh / Hn) * L.o_st[0] + (int64_t)(bh % Hn) * L.o_st[1];
         const int nent = list_length(cur);
-        ntiles = uni(nent * nsub);
-        tile_base = (uint32_t)uni((bh - bh_first) * tiles_bh);
+        npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
+        half_base = (uint32_t)uni((bh - bh_first) * tiles_bh) * 2u;
         // the next item can be prepared while this one runs if this one has a loop to hide it behind, the next one
         // has a first tile to point the walk at, a list that fits a small buffer, and Q rows the LDS DMA can address
         const int next_nent = list_length(nxt);
-        const bool prepare_next = nxt.item >= 0 && ntiles > 0 && next_nent > 0 && next_nent <= kPipeList && q_offsets_32 != 0;
-        beyond_tile = (uint32_t)uni((int)(prepare_next ? first_tile(nxt) : tile_base));
+        const bool prepare_next = nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
+        if (prepare_next) {
+            first_pair(nxt, beyond);
+            beyond[0] = (uint32_t)uni((int)beyond[0]);
+            beyond[1] = (uint32_t)uni((int)beyond[1]);
+        } else {
+            beyond[0] = beyond[1] = half_base;
+        }
         const int nbh = prepare_next ? nxt.item / nqt : 0;
         const int64_t nqrow0 = prepare_next ? (int64_t)(nxt.item % nqt) * kTile : 0;
         const int32_t* nlist = idx + ((int64_t)nbh * nbq + nqrow0 / bs_q) * idx_stride;
@@ -509,32 +559,37 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 for (int i = 0; i < 16; ++i) oacc[t][qq][i] = 0.f;
 
         bool run = true;                     // this kernel computes the item (see the bound on q . k below)
-        if (ntiles > 0) {
+        if (npairs > 0) {
+            uint32_t half0, mask0;           // position 0 of the walk
             {
                 // the three entries, then the three words, each kind in one sweep: one wait per kind instead of three
-                uint32_t raw3[3];
+                Raw raw3[3];
+                uint32_t h[3][2], m[3][2];
                 uint64_t word3[3];
 #pragma unroll
-                for (int r = 0; r < 3; ++r) raw3[r] = entry_raw(r);
+                for (int r = 0; r < 3; ++r) raw3[r] = pair_raw(r);
 #pragma unroll
-                for (int r = 0; r < 3; ++r) w_tile[r] = entry_tile(r, raw3[r]);
+                for (int r = 0; r < 3; ++r) pair_halves(r, raw3[r], h[r]);
 #pragma unroll
-                for (int r = 0; r < 3; ++r) word3[r] = entry_word(r, w_tile[r]);
+                for (int r = 0; r < 3; ++r) word3[r] = pair_word(r, h[r]);
 #pragma unroll
-                for (int r = 0; r < 3; ++r) w_mask[r] = mask_of(r, word3[r]);
+                for (int r = 0; r < 3; ++r) pair_masks(r, raw3[r], word3[r], m[r]);
+                half0 = h[0][0]; mask0 = m[0][0];
+                w_half[0] = h[0][1]; w_half[1] = h[1][0]; w_half[2] = h[1][1]; w_half[3] = h[2][0]; w_half[4] = h[2][1];
+                w_mask[0] = m[0][1]; w_mask[1] = m[1][0]; w_mask[2] = m[1][1]; w_mask[3] = m[2][0]; w_mask[4] = m[2][1];
             }
             // ---- prologue.  In flight when the loop starts: K(1), K(2), V_A(0), V_B(0), V_A(1); the ring slot of
             // V_B(1) holds zeros, which the first step multiplies with P = 0 (there is no step -1).  A prepared item
             // finds all of them but K(2) requested already (K(0) sits where K(2) belongs until S(0) has been issued).
             if (!prepared) {
 #pragma unroll
-                for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(w_tile[0], 0, c);             // K(0)
+                for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(half0, c);                    // K(0)
 #pragma unroll
-                for (int c = 0; c < 8; ++c) kb[1][c] = k_frag(w_tile[0], 1, c);             // K(1)
+                for (int c = 0; c < 8; ++c) kb[1][c] = k_frag(w_half[0], c);                // K(1)
 #pragma unroll
-                for (int f = 0; f < 8; ++f) vb[0][f] = v_frag(w_tile[0], 0, f);             // V_A(0), V_B(0)
+                for (int f = 0; f < 8; ++f) vb[0][f] = v_frag(half0, f);                    // V_A(0), V_B(0)
 #pragma unroll
-                for (int f = 0; f < 4; ++f) vb[1][f] = v_frag(w_tile[0], 1, f);             // V_A(1)
+                for (int f = 0; f < 4; ++f) vb[1][f] = v_frag(w_half[0], f);                // V_A(1)
             }
 #pragma unroll
             for (int f = 4; f < 8; ++f)
@@ -563,11 +618,11 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 else { mfma_s<false, false>(s[0][0], kb[0][c], qreg[0][c]); mfma_s<false, true>(s[0][1], kb[0][c], qreg[1][c]); }
             }
 #pragma unroll
-            for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(w_tile[1], 0, c);                 // K(2), behind the last reader of K(0)
+            for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(w_half[1], c);                    // K(2), behind the last reader of K(0)
             asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");           // MFMA results before the VALU reads them
             mfma_chain_end(s[0][0]);
             mfma_chain_end(s[0][1]);
-            mask_pair(s[0], (uint32_t)w_mask[0]);
+            mask_pair(s[0], mask0);
             float mx[2];
 #pragma unroll
             for (int qq = 0; qq < 2; ++qq) {
@@ -611,7 +666,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 // outstanding loads, which can only make its waits for the fragment loads stricter than they need
                 // be while the DMA is under way.
 #pragma unroll
-                for (int e = 0; e < kPipeList / 64; ++e)
+                for (int e = 0; e < kPipeList * kWords / 64; ++e)
                     if (64 * e < next_nent)
                         load_to_lds_4(nlist, (uint32_t)min(lane + 64 * e, next_nent - 1) * 4u, (uint32_t)uni((int)lds_address(&lists[list_buf ^ 1][64 * e])));
                 // and the token rows of its 64 query slots, which its epilogue stores through
@@ -628,22 +683,27 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             }
             // The entry that comes into the window is decoded one iteration before it enters (its validity word may
             // be a load) and read from LDS one iteration before that.
-            uint32_t p_tile = entry_tile(3, entry_raw(3));
-            uint64_t p_mask = entry_mask(3, p_tile);
-            uint32_t raw = entry_raw(4);
-            for (int g = 0; g < ntiles; ++g) {
+            uint32_t p_half[2], p_mask[2];
+            {
+                const Raw raw3 = pair_raw(3);
+                pair_halves(3, raw3, p_half);
+                pair_masks(3, raw3, pair_word(3, p_half), p_mask);
+            }
+            Raw raw = pair_raw(4);
+            for (int g = 0; g < npairs; ++g) {
                 step(std::integral_constant<int, 0>{});
                 step(std::integral_constant<int, 1>{});
-                w_tile[0] = w_tile[1]; w_mask[0] = w_mask[1];
-                w_tile[1] = w_tile[2]; w_mask[1] = w_mask[2];
-                w_tile[2] = p_tile;
-                w_mask[2] = p_mask;
-                asm volatile("" : "+s"(w_tile[0]), "+s"(w_tile[1]), "+s"(w_tile[2]));
-                asm volatile("" : "+s"(w_mask[0]), "+s"(w_mask[1]), "+s"(w_mask[2]));
-                p_tile = entry_tile(g + 4, raw);
-                p_mask = entry_mask(g + 4, p_tile);
+                w_half[0] = w_half[2]; w_mask[0] = w_mask[2];
+                w_half[1] = w_half[3]; w_mask[1] = w_mask[3];
+                w_half[2] = w_half[4]; w_mask[2] = w_mask[4];
+#pragma unroll
+                for (int x = 0; x < 2; ++x) { w_half[3 + x] = p_half[x]; w_mask[3 + x] = p_mask[x]; }
+#pragma unroll
+                for (int x = 0; x < 5; ++x) asm volatile("" : "+s"(w_half[x]), "+s"(w_mask[x]));
+                pair_halves(g + 4, raw, p_half);
+                pair_masks(g + 4, raw, pair_word(g + 4, p_half), p_mask);
                 __builtin_amdgcn_sched_barrier(0);
-                raw = entry_raw(g + 5);
+                raw = pair_raw(g + 5);
                 __builtin_amdgcn_sched_barrier(0);
             }
             __syncthreads();                          // the list in LDS has been read: the memory may become the staging tile
@@ -662,7 +722,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 for (int qq = 0; qq < 2; ++qq) oacc[t][qq] = mfma32(vb[1][4 + t], pb[qq][1], oacc[t][qq]);
             if (rescale_pending) rescale_out();
             }   // run
-        }   // ntiles > 0
+        }   // npairs > 0
 
         if (run) {
         // ---- epilogue: combine the two key groups of every query, normalise, store through LDS ----
@@ -770,8 +830,10 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk,
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
-                           const int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared) {
-    if (idx_stride > kListEntries) return hipErrorInvalidValue;   // the C-ABI layer keeps lists within this limit
+                           const int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
+                           bool halves) {
+    // the C-ABI layer keeps lists within these limits (a list that is too long for the small buffers is staged in `ost`)
+    if (idx_stride > (halves ? kHalfEntries : kListEntries)) return hipErrorInvalidValue;
     const float qk_scale = sm_scale * kLog2e;
     FragLayout L;
     L.q_rows = q_rows;
@@ -799,18 +861,20 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const bool bounded = key_norm != nullptr && fallback != nullptr && one_span && total > resident;
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
-#define BSA_FRAG_LAUNCH_T(T, N1, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
-    hipLaunchKernelGGL((fwd_frag_kernel<T, N1, BD>), grid, block, 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
+#define BSA_FRAG_LAUNCH_T(T, WALK, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
+    hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD>), grid, block, 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
                        lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, resident, Hn, lse_rows, \
                        L, ord, que, gate, want, bh0, span, q_offsets_32, key_norm, fbl, fbc)
 #define BSA_FRAG_LAUNCH(BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                                     \
     do {                                                                                                               \
         if (dtype == BSA_BF16) {                                                                                       \
-            if (bs_k == kTile) BSA_FRAG_LAUNCH_T(__bf16, true, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);   \
-            else BSA_FRAG_LAUNCH_T(__bf16, false, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);          \
+            if (halves) BSA_FRAG_LAUNCH_T(__bf16, kHalves, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
+            else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(__bf16, kTiles, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
+            else BSA_FRAG_LAUNCH_T(__bf16, kBlocks, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);        \
         } else {                                                                                                       \
-            if (bs_k == kTile) BSA_FRAG_LAUNCH_T(_Float16, true, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
-            else BSA_FRAG_LAUNCH_T(_Float16, false, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);        \
+            if (halves) BSA_FRAG_LAUNCH_T(_Float16, kHalves, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
+            else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(_Float16, kTiles, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
+            else BSA_FRAG_LAUNCH_T(_Float16, kBlocks, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);      \
         }                                                                                                              \
     } while (0)
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
@@ -823,7 +887,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     }
     // kRoundsPerLaunch rounds per launch, every workgroup running one item of each: the items of a round start
     // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
-    const int span = (idx_stride * (bs_k / kTile) <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
+    const int list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
+    const int span = (list_tiles <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
     for (int first = 0; first < total;) {
         int end = first + span < total ? first + span : total;
         const int bh0 = first / per_head;

@@ -87,6 +87,14 @@ __device__ __forceinline__ Slots slots_of(const Grid3& g, int blk, int sub, int 
     return s;
 }
 
+// Where a slot of a tile goes: the real ones (bits of `word`) to the front, both groups in slot order.  The keys of a tile
+// may come in any order, so a tile with n real keys costs the attention kernel ceil(n / 32) steps instead of two.
+__device__ __forceinline__ int front_place(uint64_t word, int slot) {
+    if (word == ~0ull) return slot;
+    const int before = __popcll(word & (((uint64_t)1 << slot) - 1));
+    return (word >> slot) & 1ull ? before : __popcll(word) + slot - before;
+}
+
 // workgroup -> (tile or chunk, batch * head).  For a token-major source (the heads of a token next to each other, as a QKV
 // projection leaves them) the heads of one chunk run side by side, so that the 256-byte rows they fetch share DRAM pages
 // and cache lines' neighbourhoods; otherwise the chunks of one head do.
@@ -143,7 +151,8 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
     for (int e = 0; e < 8; ++e) acc[e] = 0.f;
     for (int sub = 0; sub < per_chunk; ++sub) {
         const int tile_id = blk * per_chunk + sub;
-        const Slots s = slots_of(g, blk, sub, lane);
+        Slots s = slots_of(g, blk, sub, lane);
+        if (x.valid_in != nullptr) s.word = x.valid_in[tile_id];
         uint4 xs[4];
         int token[4], loc[4];
         // all four loads first, then the arithmetic: a row transformed right behind its own load would wait for it
@@ -155,11 +164,11 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         }
         if (s.word != ~0ull) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) keep_if(xs[i], token[i] >= 0);
+            for (int i = 0; i < 4; ++i) keep_if(xs[i], (s.word >> (rg + 16 * i)) & 1ull);
         }
         if (bh == 0 && threadIdx.x < 64) {
             if (x.valid != nullptr && lane == 0) x.valid[tile_id] = s.word;
-            if (x.rows != nullptr) x.rows[(int64_t)tile_id * kTile + lane] = s.token;
+            if (x.rows != nullptr) x.rows[(int64_t)tile_id * kTile + front_place(s.word, lane)] = s.token;
         }
         if (kTransform) {
             uint4 wraw = make_uint4(0, 0, 0, 0);
@@ -222,7 +231,7 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         if (x.frag != nullptr) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                uint16_t* row = tile + (rg + 16 * i) * kPitchK + c16 * 8;          // 8-byte aligned (pitch 264 B)
+                uint16_t* row = tile + front_place(s.word, rg + 16 * i) * kPitchK + c16 * 8;          // 8-byte aligned (pitch 264 B)
                 *reinterpret_cast<uint2*>(row) = make_uint2(xs[i].x, xs[i].y);
                 *reinterpret_cast<uint2*>(row + 4) = make_uint2(xs[i].z, xs[i].w);
             }
@@ -260,7 +269,8 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
     const int lane = threadIdx.x & 63;
     const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
     const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
-    const Slots s = slots_of(g, tile_id / per_chunk, tile_id % per_chunk, lane);
+    Slots s = slots_of(g, tile_id / per_chunk, tile_id % per_chunk, lane);
+    if (x.valid_in != nullptr) s.word = x.valid_in[tile_id];
     uint4 xs[4];
     int token[4];
 #pragma unroll
@@ -270,10 +280,10 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
     }
     if (s.word != ~0ull) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) keep_if(xs[i], token[i] >= 0);
+        for (int i = 0; i < 4; ++i) keep_if(xs[i], (s.word >> (rg + 16 * i)) & 1ull);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(tile + (rg + 16 * i) * kPitchV + c16 * 8) = xs[i];
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(tile + front_place(s.word, rg + 16 * i) * kPitchV + c16 * 8) = xs[i];
     __syncthreads();
     char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
 #pragma unroll
@@ -309,7 +319,7 @@ __device__ __forceinline__ void query_part(const PrepRows& x, const Grid3& g, in
         for (int e = 0; e < 8; ++e) part[u][e] = 0.f;
     for (int sub = 0; sub < per_chunk; ++sub) {
         const Slots s = slots_of(g, blk, sub, lane);
-        if (bh == 0 && x.rows != nullptr) x.rows[((int64_t)blk * per_chunk + sub) * kTile + lane] = s.token;
+        if (bh == 0 && x.rows != nullptr) x.rows[((int64_t)blk * per_chunk + sub) * kTile + front_place(s.word, lane)] = s.token;
         // every row unconditionally (a padded slot reads token 0 and is cleared afterwards): sixteen independent loads
         // per lane, no branch between them
         uint4 xs[4][4];
@@ -386,7 +396,9 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepArgs a, int wg_k, int 
 // the row table of q alone (the selection is the caller's): one workgroup per four tiles
 __global__ __launch_bounds__(256) void row_table_kernel(Grid3 g, int32_t* __restrict__ rows, int tiles) {
     const int tile = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, per_chunk = g.chunk() / kTile;
-    if (tile < tiles) rows[(int64_t)tile * kTile + lane] = slots_of(g, tile / per_chunk, tile % per_chunk, lane).token;
+    if (tile >= tiles) return;
+    const Slots s = slots_of(g, tile / per_chunk, tile % per_chunk, lane);
+    rows[(int64_t)tile * kTile + front_place(s.word, lane)] = s.token;
 }
 
 }  // namespace

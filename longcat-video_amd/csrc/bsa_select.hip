@@ -453,10 +453,42 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
+// A visiting list of n blocks (LDS, visible to the wavefront) as the halves that hold keys, for the attention kernel's
+// kHalves walk: half of the (batch, head) | real keys << 20.  An odd number is made even with a repeat that holds no key.
+__device__ inline void expand_row(const int32_t* list, int n, const HalfLists& h, int64_t row, int lane) {
+    int32_t* const out = h.lists + row * h.stride;
+    const uint64_t below = ((uint64_t)1 << lane) - 1;
+    const int tiles = n * h.nsub;
+    int total = 0, last_at = -1, last = 0;
+    for (int base = 0; base < tiles; base += 64) {
+        const int e = base + lane;
+        int keys = 0, tile = 0;
+        if (e < tiles) {
+            const int j = h.nsub == 1 ? e : e / h.nsub;
+            tile = list[j] * h.nsub + (e - j * h.nsub);
+            keys = __popcll(h.valid[tile]);
+        }
+        const uint64_t one = __ballot(keys > 0), two = __ballot(keys > 32);
+        const int at = total + __popcll(one & below) + __popcll(two & below);
+        if (keys > 0) {
+            last = 2 * tile; last_at = at;
+            out[at] = last | (min(keys, 32) << 20);
+        }
+        if (keys > 32) {
+            last = 2 * tile + 1; last_at = at + 1;
+            out[at + 1] = last | ((keys - 32) << 20);
+        }
+        total += __popcll(one) + __popcll(two);
+    }
+    if ((total & 1) && last_at == total - 1) out[total] = last;
+    if (lane == 0) h.lens[row] = total;
+}
+
 // 32-bit words of LDS that pace_row needs for lists of n entries
 __host__ __device__ inline int pace_words(int n) { return 3 * n + (n + kPaceWidth - 1) / kPaceWidth; }
-// work[0 .. n): the ascending list, clamped to the valid range; dst: where its visiting order goes
-__device__ inline void pace_row(int32_t* work, int n, int cap, int nbk, int lane, int32_t* __restrict__ dst) {
+// work[0 .. n): the ascending list, clamped to the valid range; dst: where its visiting order goes.  Returns the visiting
+// order in LDS.
+__device__ inline const int32_t* pace_row(int32_t* work, int n, int cap, int nbk, int lane, int32_t* __restrict__ dst) {
     int32_t* const lst = work;                   // [cap] the row, ascending
     int32_t* const slots = lst + cap;            // [cap] block per visit slot, -1 = empty
     int32_t* const spare = slots + cap;          // [cap] blocks over their group's room, ascending
@@ -504,9 +536,12 @@ __device__ inline void pace_row(int32_t* work, int n, int cap, int nbk, int lane
         int rank = 0;
         for (int t = lo; t < hi; ++t) rank += (slots[t] < b || (slots[t] == b && t < s)) ? 1 : 0;
         dst[lo + rank] = b;
+        spare[lo + rank] = b;
     }
+    wave_sync();
+    return spare;
 }
-__global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32_t* out, const int32_t* __restrict__ lens, int nbk, int stride) {
+__global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32_t* out, const int32_t* __restrict__ lens, int nbk, int stride, HalfLists halves) {
     extern __shared__ int32_t pace_lds[];
     const int lane = threadIdx.x;
     const int64_t row = blockIdx.x;
@@ -515,14 +550,18 @@ __global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32
     const int n = min(max(lens[row], 0), stride);
     if (src != dst)
         for (int e = n + lane; e < stride; e += 64) dst[e] = src[e];
-    if (n <= kPaceWidth) {
+    if (n <= kPaceWidth && halves.lists == nullptr) {
         if (src != dst)
             for (int e = lane; e < n; e += 64) dst[e] = src[e];
         return;
     }
     for (int e = lane; e < n; e += 64) pace_lds[e] = min(max(src[e], 0), nbk - 1);
     wave_sync();
-    pace_row(pace_lds, n, stride, nbk, lane, dst);
+    const int32_t* order = pace_lds;
+    if (n > kPaceWidth) order = pace_row(pace_lds, n, stride, nbk, lane, dst);
+    else if (src != dst)
+        for (int e = lane; e < n; e += 64) dst[e] = src[e];
+    if (halves.lists != nullptr) expand_row(order, n, halves, row, lane);
 }
 
 // ---------------------------------------------------------------- the whole gating of a small call in one launch
@@ -542,7 +581,7 @@ __host__ __device__ inline int gate_wave_words(int k_sel) { const int w = pace_w
 
 template <typename T, int NPL>
 __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict__ qc, const T* __restrict__ kc, int32_t* __restrict__ lists,
-                                                            int32_t* __restrict__ lens, int nbq, int nbk, int k_sel, int paced, HeadNorms norms) {
+                                                            int32_t* __restrict__ lens, int nbq, int nbk, int k_sel, int paced, HeadNorms norms, HalfLists halves) {
     typedef typename GateRows<T>::bits S;
     constexpr int D = 128, R = GateRows<T>::kRows;
     extern __shared__ __attribute__((aligned(16))) unsigned char gate_lds[];
@@ -596,7 +635,10 @@ __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict_
         if (m >= nbq) break;
         const int64_t row = (int64_t)bh * nbq + m;
         if (lane == 0) lens[row] = k_sel;
-        if (k_sel == 0) continue;
+        if (k_sel == 0) {
+            if (halves.lists != nullptr && lane == 0) halves.lens[row] = 0;
+            continue;
+        }
         const S* srow = reinterpret_cast<const S*>(scores + r * pitch);
         uint32_t val[NPL];
 #pragma unroll
@@ -609,9 +651,11 @@ __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict_
         select_row<S, NPL, false>(val, [&](int i) { return srow[i]; }, lane, nbk, k_sel, nullptr, list, nullptr, mine);
         wave_sync();
         int32_t* const dst = lists + row * k_sel;
-        if (paced && k_sel > kPaceWidth) pace_row(list, k_sel, k_sel, nbk, lane, dst);
+        const int32_t* order = list;
+        if (paced && k_sel > kPaceWidth) order = pace_row(list, k_sel, k_sel, nbk, lane, dst);
         else
             for (int e = lane; e < k_sel; e += 64) dst[e] = list[e];
+        if (halves.lists != nullptr) expand_row(order, k_sel, halves, row, lane);
         wave_sync();
     }
 }
@@ -623,18 +667,18 @@ size_t gate_lds_bytes(int nbk, int k_sel) {
 
 template <typename T>
 hipError_t launch_gate_t(const T* qc, const T* kc, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel, bool paced,
-                         hipStream_t st, HeadNorms norms) {
+                         hipStream_t st, HeadNorms norms, HalfLists halves) {
     const size_t lds = gate_lds_bytes<T>(nbk, k_sel);
     const int blocks = (nbq + GateRows<T>::kRows - 1) / GateRows<T>::kRows;
-    const int halves = GateRows<T>::kRows > kGateThreads / 64 && blocks * BH <= kGateMaxGroups / 2 ? 2 : 1;
-    const dim3 grid(blocks, BH, halves), block(kGateThreads);
+    const int parts = GateRows<T>::kRows > kGateThreads / 64 && blocks * BH <= kGateMaxGroups / 2 ? 2 : 1;
+    const dim3 grid(blocks, BH, parts), block(kGateThreads);
 #define BSA_GATE(N)                                                                                                          \
     do {                                                                                                                     \
         if (lds > 64 * 1024) {                                                                                               \
             const hipError_t ea = hipFuncSetAttribute((const void*)gate_kernel<T, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
             if (ea != hipSuccess) return ea;                                                                                 \
         }                                                                                                                    \
-        hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0, norms);  \
+        hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0, norms, halves);  \
     } while (0)
     if (nbk <= 64) BSA_GATE(1);
     else if (nbk <= 128) BSA_GATE(2);
@@ -823,19 +867,19 @@ bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype) {
 }
 
 hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
-                       bool paced, int dtype, hipStream_t st, HeadNorms norms) {
-    if (dtype == BSA_F32) return launch_gate_t<float>((const float*)q_cmp, (const float*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms);
-    if (dtype == BSA_BF16) return launch_gate_t<__bf16>((const __bf16*)q_cmp, (const __bf16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms);
-    return launch_gate_t<_Float16>((const _Float16*)q_cmp, (const _Float16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms);
+                       bool paced, int dtype, hipStream_t st, HeadNorms norms, HalfLists halves) {
+    if (dtype == BSA_F32) return launch_gate_t<float>((const float*)q_cmp, (const float*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms, halves);
+    if (dtype == BSA_BF16) return launch_gate_t<__bf16>((const __bf16*)q_cmp, (const __bf16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms, halves);
+    return launch_gate_t<_Float16>((const _Float16*)q_cmp, (const _Float16*)k_cmp, lists, lens, BH, nbq, nbk, k_sel, paced, st, norms, halves);
 }
 
 hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* lens, int64_t rows, int nbk, int stride,
-                             hipStream_t st) {
+                             hipStream_t st, HalfLists halves) {
     if (rows <= 0 || stride <= 0) return hipSuccess;
     const int groups = (stride + kPaceWidth - 1) / kPaceWidth;
     const size_t lds = ((size_t)3 * stride + groups) * sizeof(int32_t);
     if (lds > 64 * 1024 || rows > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pace_order_kernel, dim3((unsigned)rows), dim3(64), lds, st, in, out, lens, nbk, stride);
+    hipLaunchKernelGGL(pace_order_kernel, dim3((unsigned)rows), dim3(64), lds, st, in, out, lens, nbk, stride, halves);
     return hipGetLastError();
 }
 
