@@ -369,7 +369,7 @@ struct Plan {
     bool cdf;
     bool f32, direct_kv;
     bool frag;            // k and v are rewritten in fragment order for fwd_frag_kernel (bsa_fwd_frag.hip)
-    size_t off_kp, off_vp, off_qc, off_kc, off_score, off_idx, off_idx_sorted, off_lens, off_valid, off_qrows, off_krows, off_ktiles, off_order, off_queue, off_knorm, off_fallback, off_halves, off_half_lens, total;
+    size_t off_kp, off_vp, off_qc, off_kc, off_score, off_idx, off_idx_sorted, off_lens, off_valid, off_qrows, off_krows, off_ktiles, off_order, off_queue, off_knorm, off_fallback, off_halves, off_half_lens, off_parts, total;
 };
 inline size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -435,6 +435,8 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->half_width = pl->frag && padded && halves <= 4096 ? (int)halves : 0;
     pl->off_halves = take(bh * pl->nbq * (size_t)pl->half_width * sizeof(int32_t));
     pl->off_half_lens = take(pl->half_width > 0 ? bh * pl->nbq * sizeof(int32_t) : 0);
+    // the top-k rule's lists are of one length: the last round of the attention kernel may be cut into parts
+    pl->off_parts = take(pl->frag && !pl->cdf ? frag_part_floats((int64_t)bh * (pl->Sqp / 64)) * sizeof(float) : 0);
     pl->total = off;
     return BSA_OK;
 }
@@ -455,6 +457,7 @@ struct Ws {
     float* knorm;
     int32_t* fallback;
     int32_t *halves, *half_lens;
+    float* parts;
 };
 int carve(const Plan& pl, void* workspace, size_t workspace_bytes, const char* who, Ws* w) {
     if (!workspace) return set_error(BSA_ERR_BAD_ARG, "%s: workspace is null", who);
@@ -474,6 +477,7 @@ int carve(const Plan& pl, void* workspace, size_t workspace_bytes, const char* w
     w->order = pl.cdf && !pl.f32 ? reinterpret_cast<int32_t*>(ws + pl.off_order) : nullptr;
     w->queue = pl.cdf && !pl.f32 ? reinterpret_cast<uint32_t*>(ws + pl.off_queue) : nullptr;
     w->knorm = pl.frag ? reinterpret_cast<float*>(ws + pl.off_knorm) : nullptr;
+    w->parts = pl.frag && !pl.cdf ? reinterpret_cast<float*>(ws + pl.off_parts) : nullptr;
     w->halves = pl.half_width > 0 ? reinterpret_cast<int32_t*>(ws + pl.off_halves) : nullptr;
     w->half_lens = pl.half_width > 0 ? reinterpret_cast<int32_t*>(ws + pl.off_half_lens) : nullptr;
     w->fallback = pl.frag ? reinterpret_cast<int32_t*>(ws + pl.off_fallback) : nullptr;
@@ -551,11 +555,11 @@ hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, cons
 hipError_t attention_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, const void* q, const int64_t q_strides[3],
                          const void* k, const int64_t k_strides[3], const void* v, const int64_t v_strides[3], void* o,
                          const int64_t o_strides[3], const int32_t* idx, const int32_t* lens, int idx_stride, float* lse,
-                         hipStream_t st, bool by_length = false, bool fallback_cleared = false, bool halves = false) {
+                         hipStream_t st, bool by_length = false, bool fallback_cleared = false, bool halves = false, float* parts = nullptr) {
     if (pl.frag)
         return launch_fwd_frag(q, w.kp, w.vp, idx, lens, kv_padded(p) ? w.valid : nullptr, o, lse, p->B, p->Hn, pl.Sqp, pl.Skp,
                                pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype, st, w.qrows, q_strides, o_strides,
-                               (int64_t)p->Tq * p->Hq * p->Wq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves);
+                               (int64_t)p->Tq * p->Hq * p->Wq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves, parts);
     FwdLayout L;
     L.q_rows = w.qrows;
     L.k_tiles = w.ktiles;
@@ -686,7 +690,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         if (pl.cdf)
             BSA_HIP(launch_order_by_length(walk_lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, walk_width, st), "order by length");
         BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, walk, walk_lens, walk_width,
-                              lse_out, st, pl.cdf, pl.frag, by_half), "attention");
+                              lse_out, st, pl.cdf, pl.frag, by_half, pl.cdf ? nullptr : w.parts), "attention");
     } else {
         F32Layout L;
         L.q_rows = w.qrows; L.k_rows = w.krows;

@@ -213,10 +213,12 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
-                           int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false);
+                           int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false, float* part_buf = nullptr);
 // fallback (optional, frag_fallback_ints(B * Hn * Sq / 64) int32): with it and key_norm the rounds run the kernel that
 // takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.  Its first word
 // counts them: fallback_cleared says that it is zero already.
+// part_buf (optional, frag_part_floats(B * Hn * Sq / 64) floats): the last, partial round may be cut into parts, merged at the end.
+size_t frag_part_floats(int64_t items);
 // halves: idx and lens are HalfLists, idx_stride their row pitch (at most 4 096).
 size_t frag_fallback_ints(int64_t items);
 

@@ -106,6 +106,15 @@ enum { kTiles, kBlocks, kHalves };
 constexpr uint32_t kHalfId = 0xfffff;     // of a kHalves entry: the half; above it: its number of real keys
 constexpr int kHalfCountShift = 20;
 
+// An item in parts: `count` wavefronts walk a share of its pairs each and leave the sums of their share (unnormalised
+// accumulators in register order, running maximum and row sum per query) in `buf`, kPartFloats per part; merge_parts_kernel
+// puts them together.  Part p of the launch's item i is its work item p * items + i.  count 1: whole items.
+constexpr int kPartFloats = kTile * kD + 2 * kTile;
+struct Parts {
+    float* buf;
+    int count, items;
+};
+
 template <typename T, int kWalk, bool kBounded>
 __global__ __launch_bounds__(64) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
@@ -114,7 +123,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     float qk_scale, int item_begin, int item_end, int round, int Hn, int64_t lse_S, FragLayout L,
     const int32_t* __restrict__ order, uint32_t* __restrict__ queue, const uint32_t* __restrict__ gate, uint32_t gate_want,
     int bh_first, uint32_t kv_span_bytes, int q_offsets_32, const float* __restrict__ key_norm,
-    int32_t* __restrict__ fallback, uint32_t* __restrict__ fallback_count) {
+    int32_t* __restrict__ fallback, uint32_t* __restrict__ fallback_count, Parts parts) {
     typedef typename Vec8<T>::type V8;
     // log2 headroom before the running maximum is raised: probabilities reach 2^kTau, which the storage type of P
     // must hold (fp16 ends at 65 504 = 2^15.99) and the fp32 sums must hold times the number of keys
@@ -144,7 +153,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     const int tiles_bh = (int)(Sk / kTile);
     const uint32_t lane_off = (uint32_t)lane * 16u;
     // the kernel that runs the fallback list takes as many items as the list holds
-    const int n_launch = kBounded ? item_end - item_begin
+    const int n_launch = kBounded ? item_end - item_begin : parts.count > 1 ? parts.count * parts.items
                                   : (fallback_count != nullptr ? __builtin_amdgcn_readfirstlane((int)min(*fallback_count, (uint32_t)(item_end - item_begin)))
                                                                : item_end - item_begin);
 
@@ -183,10 +192,11 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     auto next_local = [&]() -> int { return queue != nullptr ? draw() : round_local(rounds_taken++); };
     // what is known of an item ahead of time: its number, the length of its list and its first entry (both as
     // they lie in memory; they are clamped where they are used)
-    struct Desc { int item, nent, ent[2]; float kn; };              // ent: the first list entry (kHalves: the first two)
+    struct Desc { int item, nent, ent[2], local; float kn; };       // ent: the first list entry (kHalves: the first two)
     auto fetch = [&](int local) -> Desc {
-        Desc d = {-1, 0, {0, 0}, INFINITY};
+        Desc d = {-1, 0, {0, 0}, local, INFINITY};
         if (local < 0) return d;
+        if (!kBounded && parts.count > 1) local %= parts.items;
         d.item = item_begin + (order != nullptr ? order[local] : local);
         const int bh = d.item / nqt, qblock = (int)((int64_t)(d.item % nqt) * kTile / bs_q);
         const int64_t row = (int64_t)bh * nbq + qblock;
@@ -261,7 +271,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     };
 
     // ---- per item
-    int npairs = 0;
+    int npairs = 0, pair0 = 0;       // the walk covers the pairs pair0 .. pair0 + npairs - 1 of the list
     uint32_t half_base = 0;          // first half of the item's (batch, head)
     uint32_t beyond[2] = {0, 0};     // what the positions behind the end of the list name
     const uint32_t* ents = big;      // the item's list in LDS
@@ -272,7 +282,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // `beyond` with every key masked out.  The entry is read from LDS (pair_raw, to be issued early) and decoded later.
     struct Raw { uint32_t e[kWords]; };
     auto pair_raw = [&](int tp) -> Raw {
-        const int tc = min(tp, npairs - 1);
+        const int tc = min(tp, npairs - 1) + pair0;
         Raw r;
         if constexpr (kWalk == kHalves) {
             const uint2 x = *reinterpret_cast<const uint2*>(ents + 2 * tc);               // the same address in every lane
@@ -292,7 +302,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         }
         if (tp >= npairs) { h[0] = beyond[0]; h[1] = beyond[1]; return; }
         const int blk = min(max(uni((int)raw.e[0]), 0), nbk - 1);                          // a malformed list: wrong numbers, never a fault
-        h[0] = half_base + 2u * (uint32_t)(kWalk == kTiles ? blk : blk * nsub + tp % nsub);
+        h[0] = half_base + 2u * (uint32_t)(kWalk == kTiles ? blk : blk * nsub + (tp + pair0) % nsub);
         h[1] = h[0] + 1u;
     };
     // the validity word of a pair's tile (all keys valid without padding; kHalves: the entries say it), in two steps so that
@@ -502,11 +512,17 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         const int64_t o_bh = (int64_t)(bh / Hn) * L.o_st[0] + (int64_t)(bh % Hn) * L.o_st[1];
         const int nent = list_length(cur);
         npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
+        if (!kBounded && parts.count > 1) {
+            const int part = cur.local / parts.items;
+            pair0 = (int)((int64_t)npairs * part / parts.count);
+            npairs = (int)((int64_t)npairs * (part + 1) / parts.count) - pair0;
+        }
         half_base = (uint32_t)uni((bh - bh_first) * tiles_bh) * 2u;
         // the next item can be prepared while this one runs if this one has a loop to hide it behind, the next one
         // has a first tile to point the walk at, a list that fits a small buffer, and Q rows the LDS DMA can address
         const int next_nent = list_length(nxt);
-        const bool prepare_next = nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
+        // (an item in parts has no first pair that is known ahead)
+        const bool prepare_next = (kBounded || parts.count == 1) && nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
         if (prepare_next) {
             first_pair(nxt, beyond);
             beyond[0] = (uint32_t)uni((int)beyond[0]);
@@ -724,7 +740,25 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             }   // run
         }   // npairs > 0
 
-        if (run) {
+        if (!kBounded && parts.count > 1) {
+            float* const out = parts.buf + (int64_t)cur.local * kPartFloats;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+                    for (int gq = 0; gq < 4; ++gq)
+                        *reinterpret_cast<float4*>(out + (((t * 2 + qq) * 4 + gq) * 64 + lane) * 4) =
+                            make_float4(oacc[t][qq][4 * gq], oacc[t][qq][4 * gq + 1], oacc[t][qq][4 * gq + 2], oacc[t][qq][4 * gq + 3]);
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq) {
+                const float l = l_i[qq] + __shfl_xor(l_i[qq], 32);
+                if (lh == 0) {
+                    out[kTile * kD + 32 * qq + lr] = m_i[qq];
+                    out[kTile * kD + kTile + 32 * qq + lr] = l;
+                }
+            }
+        } else if (run) {
         // ---- epilogue: combine the two key groups of every query, normalise, store through LDS ----
         float inv[2];
 #pragma unroll
@@ -791,6 +825,50 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     }   // work items
 }
 
+// Puts the parts of an item together: rescale to the largest of the running maxima, add, normalise, round, store.  One
+// workgroup per item; bound by the parts' bytes (33 KB each).
+template <typename T>
+__global__ __launch_bounds__(256) void merge_parts_kernel(Parts parts, T* __restrict__ o, float* __restrict__ lse, int item_begin,
+                                                          int nqt, int Hn, int64_t lse_S, FragLayout L) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 31, lh = lane >> 5;
+    const int item = item_begin + blockIdx.x, bh = item / nqt;
+    const int64_t qrow0 = (int64_t)(item % nqt) * kTile;
+    const float* first = parts.buf + (int64_t)blockIdx.x * kPartFloats;
+    const int64_t stride = (int64_t)parts.items * kPartFloats;
+    float M[2] = {-INFINITY, -INFINITY}, inv[2] = {0.f, 0.f};
+    int64_t row[2];
+#pragma unroll
+    for (int qq = 0; qq < 2; ++qq) {
+        const int slot = 32 * qq + lr;
+        row[qq] = L.q_rows != nullptr ? (int64_t)L.q_rows[qrow0 + slot] : qrow0 + slot;
+        for (int p = 0; p < parts.count; ++p) M[qq] = fmaxf(M[qq], first[p * stride + kTile * kD + slot]);
+        float l = 0.f;
+        for (int p = 0; p < parts.count; ++p) {
+            const float m = first[p * stride + kTile * kD + slot];
+            if (m > -INFINITY) l += first[p * stride + kTile * kD + kTile + slot] * __builtin_amdgcn_exp2f(m - M[qq]);
+        }
+        inv[qq] = l > 0.f ? 1.0f / l : 0.f;
+        if (lse != nullptr && wave == 0 && lh == 0 && row[qq] >= 0)
+            lse[(int64_t)bh * lse_S + row[qq]] = l > 0.f ? (M[qq] + __builtin_log2f(l)) * kLn2 : -INFINITY;
+    }
+    T* const out = o + (int64_t)(bh / Hn) * L.o_st[0] + (int64_t)(bh % Hn) * L.o_st[1];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        const int chunk = wave * 8 + c, t = chunk >> 3, qq = (chunk >> 2) & 1, gq = chunk & 3;      // qq is c >> 2
+        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        for (int p = 0; p < parts.count; ++p) {
+            const float m = first[p * stride + kTile * kD + 32 * qq + lr];
+            const float f = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M[c >> 2]) : 0.f;
+            const float4 x = *reinterpret_cast<const float4*>(first + p * stride + (chunk * 64 + lane) * 4);
+            sum.x = fmaf(x.x, f, sum.x); sum.y = fmaf(x.y, f, sum.y); sum.z = fmaf(x.z, f, sum.z); sum.w = fmaf(x.w, f, sum.w);
+        }
+        if (row[c >> 2] < 0) continue;
+        const float n = inv[c >> 2];
+        T x4[4] = {(T)(sum.x * n), (T)(sum.y * n), (T)(sum.z * n), (T)(sum.w * n)};
+        *reinterpret_cast<uint2*>(out + row[c >> 2] * L.o_st[2] + 32 * t + 8 * gq + 4 * lh) = *reinterpret_cast<const uint2*>(x4);
+    }
+}
+
 }  // namespace
 
 // Rounds per launch: five (four to six measure the same at 90 tiles per list and 1.5 % better than two, now that an
@@ -823,6 +901,31 @@ __global__ void frag_zero_kernel(uint32_t* p, int n) {
     if (i < n) p[i] = 0u;
 }
 
+// How many parts the last, partial round of `items` work items with lists of list_tiles tiles is cut into, so that the
+// wavefronts it leaves idle share its walk: the count with the least estimated time.  A 64-key tile of a list takes 1.72 us of a
+// wavefront when the chip is full, 1.15 us when it is half empty (its power then allows the full clock: with one price for
+// both, rounds of 512 and 640 items were cut and a 480p layer took 1 838 us instead of 1 826, four heads of 720p 1 113 instead
+// of 1 095), a part 6 us to start and end, the merge a launch and the parts' bytes (33 KB written and read).  Shares of
+// fewer than 10 tiles are not worth it.
+constexpr int kMaxParts = 16, kMaxPartRounds = 2, kMinPartTiles = 10;
+static int choose_parts(int items, int list_tiles, int resident) {
+    int best = 1;
+    float best_us = 0.f;
+    for (int p = 1; p == 1 || (p <= kMaxParts && p * kMinPartTiles <= list_tiles && (int64_t)items * p <= kMaxPartRounds * resident); ++p) {
+        const int rounds = (int)(((int64_t)items * p + resident - 1) / resident);
+        const float full = (float)items * p / ((float)rounds * resident), tile_us = 1.15f + 1.14f * (full > 0.5f ? full - 0.5f : 0.f);
+        const float us = rounds * (tile_us * list_tiles / p + 6.f) + (p > 1 ? 5.f + 0.0125f * items * p : 0.f);
+        if (p == 1 || us < best_us) { best = p; best_us = us; }
+    }
+    return best;
+}
+// floats of the parts' buffer for `total` items, whatever the length of their lists
+size_t frag_part_floats(int64_t total) {
+    const int resident = resident_wavefronts();
+    const int64_t tail = total % resident, most = (int64_t)kMaxPartRounds * resident;
+    return (size_t)(tail * kMaxParts < most ? tail * kMaxParts : most) * kPartFloats;
+}
+
 // int32 entries launch_fwd_frag's `fallback` argument must hold for `items` work items (64-row query tiles)
 size_t frag_fallback_ints(int64_t items) { return 64 + (size_t)items; }
 
@@ -831,7 +934,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
-                           bool halves) {
+                           bool halves, float* part_buf) {
     // the C-ABI layer keeps lists within these limits (a list that is too long for the small buffers is staged in `ost`)
     if (idx_stride > (halves ? kHalfEntries : kListEntries)) return hipErrorInvalidValue;
     const float qk_scale = sm_scale * kLog2e;
@@ -858,13 +961,14 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     // the items it has to leave to the other kernel is given, and that kernel can reach every head from one buffer.
     // A call of one round runs the exact kernel alone: its steps are 3 % longer, but a last launch that finds nothing to do
     // costs 3.6 us, a fifth of a small call's attention.
-    const bool bounded = key_norm != nullptr && fallback != nullptr && one_span && total > resident;
+    Parts parts = {nullptr, 1, 0};
+    const bool bounded = key_norm != nullptr && fallback != nullptr && one_span && total > resident;      // (see `whole` below)
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
 #define BSA_FRAG_LAUNCH_T(T, WALK, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
     hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD>), grid, block, 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
                        lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, resident, Hn, lse_rows, \
-                       L, ord, que, gate, want, bh0, span, q_offsets_32, key_norm, fbl, fbc)
+                       L, ord, que, gate, want, bh0, span, q_offsets_32, key_norm, fbl, fbc, parts)
 #define BSA_FRAG_LAUNCH(BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                                     \
     do {                                                                                                               \
         if (dtype == BSA_BF16) {                                                                                       \
@@ -889,8 +993,13 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
     const int list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
     const int span = (list_tiles <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
-    for (int first = 0; first < total;) {
-        int end = first + span < total ? first + span : total;
+    // The last, partial round in parts when its wavefronts would leave too much of the chip idle (and the exact kernel
+    // reaches every head from one buffer; the caller gives a buffer for lists of one length only).
+    const int tail = total % resident;
+    const int n_parts = part_buf != nullptr && one_span && queue == nullptr && tail > 0 ? choose_parts(tail, list_tiles, resident) : 1;
+    const int whole = n_parts > 1 ? total - tail : total;
+    for (int first = 0; first < whole;) {
+        int end = first + span < whole ? first + span : whole;
         const int bh0 = first / per_head;
         if ((end - 1) / per_head - bh0 + 1 > heads_per_span) end = (bh0 + heads_per_span) * per_head;
         const int heads = (end - 1) / per_head - bh0 + 1;
@@ -902,6 +1011,17 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
             BSA_FRAG_LAUNCH(false, grid, first, end, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, bh0, (uint32_t)(heads * kv_bh_bytes),
                             (int32_t*)nullptr, (uint32_t*)nullptr);
         first = end;
+    }
+    if (n_parts > 1) {
+        parts = {part_buf, n_parts, tail};
+        const int n = tail * n_parts;
+        const dim3 grid((unsigned)(n < resident ? n : resident));
+        BSA_FRAG_LAUNCH(false, grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
+        if (dtype == BSA_BF16)
+            hipLaunchKernelGGL((merge_parts_kernel<__bf16>), dim3(tail), dim3(256), 0, st, parts, (__bf16*)o, lse, whole, per_head, Hn, lse_rows, L);
+        else
+            hipLaunchKernelGGL((merge_parts_kernel<_Float16>), dim3(tail), dim3(256), 0, st, parts, (_Float16*)o, lse, whole, per_head, Hn, lse_rows, L);
+        parts = {nullptr, 1, 0};
     }
     if (bounded) {
         // what the rounds left over: as many items as the list holds, found out on the device
