@@ -460,6 +460,27 @@ int bsa_fwd_3d_qknorm(const bsa_3d_params* p, const bsa_qk_norm* n, const void* 
                       const int64_t v_strides[3], void* o, const int64_t o_strides[3], void* workspace, size_t workspace_bytes,
                       int32_t* idx_out, int32_t* lens_out, void* score_out, void* stream);
 
+/* bsa_fwd_3d_qknorm with the key / value cache of the attention module (attention.py:118-119, 149-181) inside the same
+ * passes.  cached_frames > 0: the first cached_frames of the Tk frames of k and v are read from k_cache (after the norm,
+ * before the rotation, as the module keeps it) and v_cache; the arguments k and v then hold the other frames.
+ * k_out / v_out (optional): receive k after the norm and before the rotation, and v, of the frames that the arguments k and
+ * v hold, at their token positions.  Strides in elements {batch, head, token}; a batch stride of 0 shares a cache. */
+typedef struct bsa_kv_cache {
+    int cached_frames;
+    const void* k_cache;
+    int64_t k_cache_strides[3];
+    const void* v_cache;
+    int64_t v_cache_strides[3];
+    void* k_out;
+    int64_t k_out_strides[3];
+    void* v_out;
+    int64_t v_out_strides[3];
+} bsa_kv_cache;
+int bsa_fwd_3d_qknorm_kv(const bsa_3d_params* p, const bsa_qk_norm* n, const bsa_kv_cache* c, const void* q, const int64_t q_strides[3],
+                         void* q_normed, const int64_t qn_strides[3], const void* k, const int64_t k_strides[3], const void* v,
+                         const int64_t v_strides[3], void* o, const int64_t o_strides[3], void* workspace, size_t workspace_bytes,
+                         int32_t* idx_out, int32_t* lens_out, void* score_out, void* stream);
+
 /* The engine's own GEMM for the two projections of the attention module (attention.py:111 and :142):
  * out[M,N] = x[M,K] . w[N,K]^T (+ bias[N]) (+ residual[M,N]), bf16 in/out, fp32 accumulation on MFMA, one
  * rounding at the end.  Row strides in elements (ldx, ldw >= K; ldo, ldr >= N; multiples of 8).  N must be a

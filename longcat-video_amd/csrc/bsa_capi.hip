@@ -500,7 +500,8 @@ int check_kv_views(const Plan& pl, const int64_t k_strides[3], const int64_t v_s
 // rows are normalised and rotated on the way, q's into q_normed.
 hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, const void* q, const int64_t q_strides[3],
                        const void* k, const int64_t k_strides[3], const void* v, const int64_t v_strides[3], bool pool,
-                       hipStream_t st, const bsa_qk_norm* qkn = nullptr, void* q_normed = nullptr, const int64_t* qn_strides = nullptr) {
+                       hipStream_t st, const bsa_qk_norm* qkn = nullptr, void* q_normed = nullptr, const int64_t* qn_strides = nullptr,
+                       const bsa_kv_cache* c = nullptr) {
     hipError_t e;
     const bool padded_k = kv_padded(p);
     if (pl.frag) {
@@ -531,6 +532,20 @@ hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, cons
             a.k.t0 = qkn->t_offset_k;
             a.q.rows_out = static_cast<uint16_t*>(q_normed);
             a.q.rB = qn_strides[0]; a.q.rH = qn_strides[1]; a.q.rS = qn_strides[2];
+            if (c != nullptr) {
+                auto out = [](PrepRows& x, void* to, const int64_t st3[3]) {
+                    x.rows_out = static_cast<uint16_t*>(to);
+                    x.rB = st3[0]; x.rH = st3[1]; x.rS = st3[2];
+                };
+                auto cached = [&](PrepRows& x, const void* from, const int64_t st3[3]) {
+                    x.cached = static_cast<const uint16_t*>(from);
+                    x.cB = st3[0]; x.cH = st3[1]; x.cS = st3[2];
+                    x.split = c->cached_frames * p->Hk * p->Wk;
+                };
+                if (c->cached_frames > 0) { cached(a.k, c->k_cache, c->k_cache_strides); cached(a.v, c->v_cache, c->v_cache_strides); }
+                if (c->k_out) out(a.k, c->k_out, c->k_out_strides);
+                if (c->v_out) out(a.v, c->v_out, c->v_out_strides);
+            }
         }
         e = launch_prepare(a, p->B, p->dtype, st);
         if (e != hipSuccess || pool) return e;                 // scoring takes the largest norm per head on its way
@@ -636,7 +651,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
                 const int64_t k_strides[3], const void* v, const int64_t v_strides[3], void* o,
                 const int64_t o_strides[3], void* workspace, size_t workspace_bytes, int32_t* idx_out,
                 int32_t* lens_out, void* score_out, void* stream, const bsa_qk_norm* qkn = nullptr, void* q_normed = nullptr,
-                const int64_t* qn_strides = nullptr, float* lse_out = nullptr, int32_t* walk_out = nullptr) {
+                const int64_t* qn_strides = nullptr, float* lse_out = nullptr, int32_t* walk_out = nullptr, const bsa_kv_cache* kvc = nullptr) {
     Ws w;
     if (!q || !k || !v || !o || !workspace) return set_error(BSA_ERR_BAD_ARG, "fwd_3d: null pointer");
     BSA_TRY(carve(pl, workspace, workspace_bytes, "fwd_3d", &w));
@@ -653,7 +668,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         // q and k as the projection left them: the pass that takes q's chunk means also normalises and rotates its
         // rows into q_normed (what the attention kernel then reads), the pass that rewrites k in fragment order
         // normalises and rotates on the way
-        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, qkn, q_normed, qn_strides), "pool, norm, rotate and prepare");
+        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, qkn, q_normed, qn_strides, kvc), "pool, norm, rotate and prepare");
         q = q_normed;
         q_strides = qn_strides;
     } else if (!pl.f32) {
@@ -780,6 +795,14 @@ int bsa_fwd_3d_qknorm(const bsa_3d_params* p, const bsa_qk_norm* n, const void* 
                       void* q_normed, const int64_t qn_strides[3], const void* k, const int64_t k_strides[3], const void* v,
                       const int64_t v_strides[3], void* o, const int64_t o_strides[3], void* workspace, size_t workspace_bytes,
                       int32_t* idx_out, int32_t* lens_out, void* score_out, void* stream) {
+    return bsa_fwd_3d_qknorm_kv(p, n, nullptr, q, q_strides, q_normed, qn_strides, k, k_strides, v, v_strides, o, o_strides, workspace,
+                                workspace_bytes, idx_out, lens_out, score_out, stream);
+}
+
+int bsa_fwd_3d_qknorm_kv(const bsa_3d_params* p, const bsa_qk_norm* n, const bsa_kv_cache* c, const void* q, const int64_t q_strides[3],
+                         void* q_normed, const int64_t qn_strides[3], const void* k, const int64_t k_strides[3], const void* v,
+                         const int64_t v_strides[3], void* o, const int64_t o_strides[3], void* workspace, size_t workspace_bytes,
+                         int32_t* idx_out, int32_t* lens_out, void* score_out, void* stream) {
     Plan pl;
     BSA_TRY(make_plan(p, &pl));
     if (!n || !n->rope_table || !n->q_weight || !n->k_weight || !q_normed || !qn_strides)
@@ -797,8 +820,18 @@ int bsa_fwd_3d_qknorm(const bsa_3d_params* p, const bsa_qk_norm* n, const void* 
     if ((reinterpret_cast<uintptr_t>(n->q_weight) | reinterpret_cast<uintptr_t>(n->k_weight)) & 15u)
         return set_error(BSA_ERR_BAD_ARG, "fwd_3d_qknorm: norm weights must be 16-byte aligned");
     BSA_TRY(check_tensor(q_normed, qn_strides, p, "q_normed"));
+    if (c != nullptr) {
+        if (c->cached_frames < 0 || c->cached_frames >= p->Tk)
+            return set_error(BSA_ERR_SHAPE, "fwd_3d_qknorm_kv: %d cached frames of %d", c->cached_frames, p->Tk);
+        if (c->cached_frames > 0) {
+            BSA_TRY(check_tensor(c->k_cache, c->k_cache_strides, p, "k_cache"));
+            BSA_TRY(check_tensor(c->v_cache, c->v_cache_strides, p, "v_cache"));
+        }
+        if (c->k_out) BSA_TRY(check_tensor(c->k_out, c->k_out_strides, p, "k_out"));
+        if (c->v_out) BSA_TRY(check_tensor(c->v_out, c->v_out_strides, p, "v_out"));
+    }
     return fwd_3d_impl(pl, p, q, q_strides, k, k_strides, v, v_strides, o, o_strides, workspace, workspace_bytes, idx_out,
-                       lens_out, score_out, stream, n, q_normed, qn_strides);
+                       lens_out, score_out, stream, n, q_normed, qn_strides, nullptr, nullptr, c);
 }
 
 int bsa_fwd_3d_static(const bsa_3d_params* p, const void* q, const int64_t q_strides[3], const void* k,

@@ -178,6 +178,9 @@ void launch_schedule_choice(const int32_t* lens, int nbq, int tiles_per_block, i
 struct PrepRows {
     const uint16_t* p;               // null: this part is left out
     int64_t sB, sH, sS;              // batch, head, token
+    const uint16_t* cached;          // k, v, optional: the tokens before `split` come from here, already normalised, and p holds the rest
+    int64_t cB, cH, cS;
+    int split;
     char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, the real slots of a tile first, zeros behind
     uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
     int32_t* rows;                   // q: token row of every slot of one (batch, head), -1 = padding; the real ones of a tile first
@@ -186,7 +189,7 @@ struct PrepRows {
     float* tile_norm;                // k, optional: largest Euclidean norm of a row of every tile, a part in a thousand above
     const uint16_t* norm_w;          // q, k, optional: 128 weights of a per-head RMSNorm that the rows go through first
     int t0;                          // q, k: frame offset of the grid inside the rotation table
-    uint16_t* rows_out;              // q, k, optional: the transformed rows at their token positions
+    uint16_t* rows_out;              // optional: the rows of p at their token positions; q after the transform, k before the rotation
     int64_t rB, rH, rS;              // ... element strides
     int head_fastest;                // set by launch_prepare: the order in which workgroups take (chunk, head)
     int offsets_32;                  // set by launch_prepare: the rows of a (batch, head) lie within 4 GB

@@ -95,6 +95,12 @@ __device__ __forceinline__ int front_place(uint64_t word, int slot) {
     return (word >> slot) & 1ull ? before : __popcll(word) + slot - before;
 }
 
+// the row of token t: before `split` from the cache, from there on from src
+__device__ __forceinline__ const uint16_t* row_at(const uint16_t* src, int64_t sS, const uint16_t* old, int64_t cS, int split, int t) {
+    if (old == nullptr) return src + (int64_t)t * sS;
+    return t < split ? old + (int64_t)t * cS : src + (int64_t)(t - split) * sS;
+}
+
 // workgroup -> (tile or chunk, batch * head).  For a token-major source (the heads of a token next to each other, as a QKV
 // projection leaves them) the heads of one chunk run side by side, so that the 256-byte rows they fetch share DRAM pages
 // and cache lines' neighbourhoods; otherwise the chunks of one head do.
@@ -115,7 +121,7 @@ constexpr int kPitchV = kD + 16;     // 288-byte rows: the transposing reads fet
 // k (or q, when it has a row transform): a workgroup per chunk, tile by tile.  The chunk mean keeps permute_kernel's order
 // of summation - a thread adds its rows rg, rg + 16, ... of the chunk, then the 16 partial sums of a column are added in
 // ascending rg, one rounding at the end - so every route gives the same bits.
-template <bool kBf16, bool kTransform>
+template <bool kBf16, bool kTransform, bool kIsK>
 __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int Hn, int id, const float* tab, int tab_T, float eps,
                                          uint16_t* tile, float2* cs) {
     typedef typename std::conditional<kBf16, __bf16, _Float16>::type T;
@@ -125,6 +131,7 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
     const int lane = threadIdx.x & 63;
     const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;      // 16 pieces of 16 B per row, 16 rows at a time
     const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
+    const uint16_t* old = kTransform && x.cached != nullptr ? x.cached + (int64_t)(bh / Hn) * x.cB + (int64_t)(bh % Hn) * x.cH + c16 * 8 : nullptr;
     // Rotation: a chunk spans at most 8 positions per axis, and a rotation pair turns with one axis only, so the
     // (cos, sin) the rows of the chunk need are 8 x 64 table entries, fetched once per workgroup instead of per row and head.
     if (kTransform && tab != nullptr) {
@@ -160,7 +167,7 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         for (int i = 0; i < 4; ++i) {
             token[i] = __shfl(s.token, rg + 16 * i);
             if (kTransform) loc[i] = __shfl(s.loc, rg + 16 * i);
-            xs[i] = *reinterpret_cast<const uint4*>(src + (int64_t)max(token[i], 0) * x.sS);
+            xs[i] = *reinterpret_cast<const uint4*>(kTransform ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
         }
         if (s.word != ~0ull) {
 #pragma unroll
@@ -188,8 +195,15 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
                         sn[jj] = a.y;
                     }
                 }
-                xs[i] = norm_rope_piece<T>(xs[i], wraw, x.norm_w != nullptr, tab != nullptr, c, sn, eps);
-                if (rows != nullptr) *reinterpret_cast<uint4*>(rows + (int64_t)token[i] * x.rS) = xs[i];
+                const bool fresh = old == nullptr || token[i] >= x.split;      // the cache holds normalised rows
+                if (kIsK && rows != nullptr) {
+                    xs[i] = norm_rope_piece<T>(xs[i], wraw, x.norm_w != nullptr && fresh, false, c, sn, eps);
+                    if (fresh) *reinterpret_cast<uint4*>(rows + (int64_t)(old == nullptr ? token[i] : token[i] - x.split) * x.rS) = xs[i];
+                    xs[i] = norm_rope_piece<T>(xs[i], wraw, false, tab != nullptr, c, sn, eps);
+                } else {
+                    xs[i] = norm_rope_piece<T>(xs[i], wraw, x.norm_w != nullptr && fresh, tab != nullptr, c, sn, eps);
+                    if (!kIsK && rows != nullptr) *reinterpret_cast<uint4*>(rows + (int64_t)token[i] * x.rS) = xs[i];
+                }
             }
         }
         if (x.pooled != nullptr) {
@@ -262,6 +276,7 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
 }
 
 // v: a workgroup per tile, gathered into LDS and read transposed: a piece holds 8 keys of one d
+template <bool kTransform>
 __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, int Hn, int id, uint16_t* tile) {
     const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
     int tile_id, bh;
@@ -269,6 +284,7 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
     const int lane = threadIdx.x & 63;
     const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
     const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
+    const uint16_t* old = kTransform && x.cached != nullptr ? x.cached + (int64_t)(bh / Hn) * x.cB + (int64_t)(bh % Hn) * x.cH + c16 * 8 : nullptr;
     Slots s = slots_of(g, tile_id / per_chunk, tile_id % per_chunk, lane);
     if (x.valid_in != nullptr) s.word = x.valid_in[tile_id];
     uint4 xs[4];
@@ -276,11 +292,19 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         token[i] = __shfl(s.token, rg + 16 * i);
-        xs[i] = *reinterpret_cast<const uint4*>(src + (int64_t)max(token[i], 0) * x.sS);
+        xs[i] = *reinterpret_cast<const uint4*>(kTransform ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
     }
     if (s.word != ~0ull) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) keep_if(xs[i], (s.word >> (rg + 16 * i)) & 1ull);
+    }
+    if (kTransform && x.rows_out != nullptr) {
+        uint16_t* rows = x.rows_out + (int64_t)(bh / Hn) * x.rB + (int64_t)(bh % Hn) * x.rH + c16 * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int at = old == nullptr ? token[i] : token[i] - x.split;
+            if (at >= 0) *reinterpret_cast<uint4*>(rows + (int64_t)at * x.rS) = xs[i];
+        }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(tile + front_place(s.word, rg + 16 * i) * kPitchV + c16 * 8) = xs[i];
@@ -381,15 +405,15 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepArgs a, int wg_k, int 
     const int w = blockIdx.x;
     if (kPart <= kKeys && w == 0 && threadIdx.x == 0 && a.zero != nullptr) *a.zero = 0u;
     if (kPart == kKeys || (kPart == kAllParts && w < wg_k)) {
-        row_part<kBf16, kTransform>(a.k, a.gk, a.Hn, w, a.tab, a.tab_T, a.eps, tile, cs);
+        row_part<kBf16, kTransform, true>(a.k, a.gk, a.Hn, w, a.tab, a.tab_T, a.eps, tile, cs);
         return;
     }
     if (kPart == kValues || (kPart == kAllParts && w < wg_k + wg_v)) {
-        value_part(a.v, a.gk, a.Hn, kPart == kValues ? w : w - wg_k, tile);
+        value_part<kTransform>(a.v, a.gk, a.Hn, kPart == kValues ? w : w - wg_k, tile);
         return;
     }
     const int wq = kPart == kQueries ? w : w - wg_k - wg_v;
-    if (kTransform) row_part<kBf16, true>(a.q, a.gq, a.Hn, wq, a.tab, a.tab_T, a.eps, tile, cs);
+    if (kTransform) row_part<kBf16, true, false>(a.q, a.gq, a.Hn, wq, a.tab, a.tab_T, a.eps, tile, cs);
     else query_part<kBf16>(a.q, a.gq, a.Hn, (int64_t)wq * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), chunks_q);
 }
 

@@ -33,6 +33,11 @@ class BsaQkNorm(C.Structure):
                 ("t_offset_q", C.c_int), ("t_offset_k", C.c_int), ("eps", C.c_float)]
 
 
+class BsaKvCache(C.Structure):
+    _fields_ = [("cached_frames", C.c_int)] + [f for n in ("k_cache", "v_cache", "k_out", "v_out")
+                                               for f in ((n, C.c_void_p), (n + "_strides", C.c_int64 * 3))]
+
+
 _i, _i64, _p, _f = C.c_int, C.c_int64, C.c_void_p, C.c_float
 _strides = C.POINTER(C.c_int64)
 
@@ -64,6 +69,8 @@ SIGNATURES = {
                             _p, _p, _p, _p, C.c_size_t, _p]),
     "bsa_fwd_3d_qknorm": (_i, [C.POINTER(Bsa3dParams), C.POINTER(BsaQkNorm), _p, _strides, _p, _strides, _p, _strides, _p, _strides,
                                _p, _strides, _p, C.c_size_t, _p, _p, _p, _p]),
+    "bsa_fwd_3d_qknorm_kv": (_i, [C.POINTER(Bsa3dParams), C.POINTER(BsaQkNorm), C.POINTER(BsaKvCache), _p, _strides, _p, _strides,
+                                  _p, _strides, _p, _strides, _p, _strides, _p, C.c_size_t, _p, _p, _p, _p]),
     "bsa_fwd_3d_static": (_i, [C.POINTER(Bsa3dParams), _p, _strides, _p, _strides, _p, _strides, _p, _strides,
                                _p, _p, _p, _p]),
     "bsa_thw_prepare": (_i, [C.POINTER(Bsa3dParams), _p, _strides, _p, _strides, _p, C.c_size_t, _p]),

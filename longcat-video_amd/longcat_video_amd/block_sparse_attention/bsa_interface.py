@@ -465,14 +465,16 @@ def flash_attn_bsa(q, k, v, chunk_size_q, chunk_size_k, sparsity, cdf_threshold,
 # R9: the operator
 # ---------------------------------------------------------------------------
 def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k, want_selection=False, out=None,
-            cdf_threshold=None, static_scratch=False, qk_norm=None, for_backward=False):
+            cdf_threshold=None, static_scratch=False, qk_norm=None, for_backward=False, kv_cache=None, kv_out=None):
     """`out`: optional [B,H,Sq,D] view (any B/H/S strides, contiguous D) to write into.  `sparsity` may be
     None when `cdf_threshold` is given (bsa_interface.py:268-277).  `static_scratch`: run through
     bsa_fwd_3d_static, which keeps its scratch memory in a buffer built into the library instead of a
     workspace tensor (problems beyond that buffer raise; calls on one GPU must not overlap).
     `qk_norm` = (q_weight, k_weight, rope_table, table_T, t_offset_q, t_offset_k, eps): q and k are the raw
     projections and are normalised per head and rotated inside the operator's own passes (bsa_fwd_3d_qknorm;
-    bf16 / fp16 and 64-token chunks only).  `for_backward`: the same kernels through bsa_fwd_3d_lse; returns
+    bf16 / fp16 and 64-token chunks only); then `kv_cache` = (k_cache, v_cache, frames): the first frames of the keys and
+    values, k and v hold the rest; `kv_out` = (k_out, v_out): receive the normalised, unrotated k and v of the frames that k
+    and v hold.  `for_backward`: the same kernels through bsa_fwd_3d_lse; returns
     (o, lists in the kernel's visiting order, lens, lse in token order) for the backward."""
     _need_gpu(q, k, v)
     B, H, Sq, D = q.shape
@@ -480,8 +482,8 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
     lib = _capi.load()
     plan = _plan_3d(B, H, D, _code(q), *latent_shape_q, *latent_shape_k, *chunk_q, *chunk_k, sparsity, cdf_threshold)
     prm, need, nbq, nbk, width = plan.prm, plan.need, plan.nbq, plan.nbk, plan.width
-    if k.stride(2) != v.stride(2) or plan.tile_tokens * k.stride(2) * k.element_size() >= 2 ** 32:
-        # the engine gathers k and v tiles with one set of in-tile offsets (32 bits); views that
+    if static_scratch and (k.stride(2) != v.stride(2) or plan.tile_tokens * k.stride(2) * k.element_size() >= 2 ** 32):
+        # this route gathers k and v tiles with one set of in-tile offsets (32 bits); views that
         # do not fit are copied once
         k, v = k.contiguous(), v.contiguous()
     ws = None if static_scratch else _workspace(need, q.device)
@@ -508,8 +510,22 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
             qw, kw = qw.to(q.dtype).contiguous(), kw.to(q.dtype).contiguous()
             q_normed = torch.empty(B, H, Sq, D, dtype=q.dtype, device=q.device)
             n = _capi.BsaQkNorm(_ptr(qw), _ptr(kw), _ptr(tab), int(table_T), int(t_off_q), int(t_off_k), float(eps))
-            _capi.check(lib.bsa_fwd_3d_qknorm(
-                prm, C.byref(n), _ptr(q), _st(q), _ptr(q_normed),
+            c = None
+            if kv_cache is not None or kv_out is not None:
+                c = _capi.BsaKvCache()
+                named = []
+                if kv_cache is not None:
+                    c.cached_frames = int(kv_cache[2])
+                    named += [("k_cache", kv_cache[0]), ("v_cache", kv_cache[1])]
+                if kv_out is not None:
+                    named += [("k_out", kv_out[0]), ("v_out", kv_out[1])]
+                for name, t in named:
+                    assert t.dtype == q.dtype and t.stride(3) == 1
+                    setattr(c, name, _ptr(t))
+                    setattr(c, name + "_strides", _st(t))
+                c = C.byref(c)
+            _capi.check(lib.bsa_fwd_3d_qknorm_kv(
+                prm, C.byref(n), c, _ptr(q), _st(q), _ptr(q_normed),
                 _st(q_normed), _ptr(k), _st(k),
                 _ptr(v), _st(v), _ptr(o), _st(o),
                 _ptr(ws), need, _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d (q/k norm inside)")

@@ -328,9 +328,9 @@ class Attention(nn.Module):
         b = tune_linear(x, self.proj.weight, self.proj.bias, residual=residual)
         return a, b
 
-    def _process_attn(self, q, k, v, shape, out=None, qk_norm=None):
+    def _process_attn(self, q, k, v, shape, out=None, qk_norm=None, kv_cache=None, kv_out=None):
         """attention.py:50-105, block-sparse branch; writes into `out` ([B,H,SQ,D] view) if given.  `qk_norm`: q and
-        k are the raw projections, normalised and rotated inside the operator (see _bsa_3d)."""
+        k are the raw projections, normalised and rotated inside the operator; `kv_cache`, `kv_out`: see _bsa_3d."""
         B, H, SQ, D = q.shape
         SKV = k.shape[2]
         if not (self.enable_bsa and shape[0] > 1):
@@ -339,19 +339,20 @@ class Attention(nn.Module):
         _, Hh, W = shape
         if self.cp_split_hw[0] * self.cp_split_hw[1] != 1:
             raise NotImplementedError("context parallelism is not built: one GPU holds every head and token")
-        Tq, Tk = SQ // (Hh * W), SKV // (Hh * W)
+        Tq, Tk = SQ // (Hh * W), SKV // (Hh * W) + (0 if kv_cache is None else kv_cache[2])
         prm = dict(sparsity=0.875, cdf_threshold=None, chunk_3d_shape_q=[4, 4, 8], chunk_3d_shape_k=[4, 4, 8])
         prm.update(self.bsa_params)
         if prm["sparsity"] is None and prm["cdf_threshold"] is None:
             raise ValueError
         return _bsa_3d(q, k, v, (Tq, Hh, W), (Tk, Hh, W), prm["sparsity"], prm["chunk_3d_shape_q"],
-                       prm["chunk_3d_shape_k"], out=out, cdf_threshold=prm["cdf_threshold"], qk_norm=qk_norm)
+                       prm["chunk_3d_shape_k"], out=out, cdf_threshold=prm["cdf_threshold"], qk_norm=qk_norm,
+                       kv_cache=kv_cache, kv_out=kv_out)
 
-    def _norm_inside_operator(self, x, shape, num_cond_latents, return_kv):
+    def _norm_inside_operator(self, x, shape):
         """True when q and k can go to the operator as projected: its passes over them (chunk means of q, k into
-        the attention kernel's operand order) then apply the norm and the rotation, and the two stand-alone passes
-        drop out.  One operator call over the whole grid, 64-token chunks, no k cache wanted."""
-        if return_kv or (num_cond_latents is not None and num_cond_latents > 0) or self.head_dim != 128:
+        the attention kernel's operand order) then apply the norm and the rotation, read the cached keys and values
+        where they lie and write the new ones, and the stand-alone passes drop out.  64-token chunks."""
+        if self.head_dim != 128:
             return False
         if not (self.enable_bsa and shape[0] > 1) or x.dtype not in (torch.bfloat16, torch.float16):
             return False
@@ -376,15 +377,24 @@ class Attention(nn.Module):
         if self._fused_projection(x, shape, return_kv):
             q, k, v = qkv_projection(x, self.qkv.weight, self.qkv.bias, self.q_norm.weight, self.k_norm.weight, shape,
                                      Hn, eps=eps)
-        elif self._norm_inside_operator(x, shape, num_cond_latents, return_kv):
+        elif self._norm_inside_operator(x, shape):
             # q, k, v stay where the projection left them: the operator's pass over q (chunk means) normalises and
             # rotates it into a per-head tensor of its own, its pass over k (fragment order) does the same on the way
-            qs, ks, v = self._project_qkv(x)
+            # and leaves the normalised rows for the cache
+            qs, ks, vs = self._project_qkv(x)
             o = torch.empty(B, N, Hn, D, dtype=x.dtype, device=x.device)
-            tab = rope_table(shape, D, x.device)
-            self._process_attn(qs, ks, v, shape, out=o.permute(0, 2, 1, 3),
-                               qk_norm=(self.q_norm.weight, self.k_norm.weight, tab, int(shape[0]), 0, 0, eps))
-            return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual=residual)
+            ov = o.permute(0, 2, 1, 3)
+            T = int(shape[0])
+            kv_out = (new(), new()) if return_kv else None
+            norm = lambda t_q: (self.q_norm.weight, self.k_norm.weight, rope_table(shape, D, x.device), T, t_q, 0, eps)
+            if num_cond_latents is not None and num_cond_latents > 0:
+                n = num_cond_latents * (N // T)
+                self._process_attn(qs[:, :, :n], ks[:, :, :n], vs[:, :, :n], shape, out=ov[:, :, :n], qk_norm=norm(0))      # attention.py:127-130
+                self._process_attn(qs[:, :, n:], ks, vs, shape, out=ov[:, :, n:], qk_norm=norm(num_cond_latents), kv_out=kv_out)   # attention.py:132-133
+            else:
+                self._process_attn(qs, ks, vs, shape, out=ov, qk_norm=norm(0), kv_out=kv_out)
+            y = self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual=residual)
+            return (y, kv_out) if return_kv else y
         else:
             # q moves into a per-head tensor on the way (the attention kernel fetches its rows tile by tile); k is
             # normed and rotated where it lies and v stays where it is: the operator reads both once, to rewrite
@@ -429,6 +439,14 @@ class Attention(nn.Module):
         qs, ks, vs = self._project_qkv(x)
         eps = self.q_norm.eps
         grid_full = (T + num_cond_latents, Hg, Wg)
+        if self._norm_inside_operator(x, grid_full):
+            # the operator reads the cached frames where they lie (rotation only) and the new ones from the projection
+            kc, vc = (t.to(x.device).expand(B, -1, -1, -1) for t in (k_cache, v_cache))                # attention.py:162-164
+            o = torch.empty(B, N, Hn, D, dtype=x.dtype, device=x.device)
+            tab = rope_table(grid_full, D, x.device)
+            self._process_attn(qs, ks, vs, shape, out=o.permute(0, 2, 1, 3), kv_cache=(kc, vc, int(num_cond_latents)),
+                               qk_norm=(self.q_norm.weight, self.k_norm.weight, tab, T + num_cond_latents, num_cond_latents, 0, eps))
+            return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual=residual)
         k_full = torch.empty(B, Hn, n_c + N, D, dtype=x.dtype, device=x.device)
         v_full = torch.empty_like(k_full)
         kc = k_cache.to(x.device).expand(B, -1, -1, -1)                            # attention.py:162-164

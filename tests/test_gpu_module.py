@@ -425,3 +425,28 @@ def test_operator_with_the_norm_inside_equals_the_separate_passes(grid, dtype):
     # 128-token chunks are not built for this entry point
     with pytest.raises(NotImplementedError):
         bi._bsa_3d(qs, ks, vs, grid, grid, 0.5, (4, 4, 8), (4, 4, 8), qk_norm=(qw, kw, tab, grid[0], 0, 0, 1e-6))
+
+
+@pytest.mark.parametrize("T,cond,Hh,W", [(8, 4, 8, 8), (5, 3, 6, 10), (2, 1, 9, 7)])
+def test_cache_inside_the_operator_equals_the_separate_passes(T, cond, Hh, W):
+    """Cached keys and values read by the operator's own passes, and the new ones written by them, against norm_rope moves
+    into full tensors followed by the operator: whole and ragged frames on both sides of the seam, one cache for two batches."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    att, dt, Hn, ch = M(), torch.bfloat16, 3, (4, 4, 4)
+    full, new, S, Sc = (T + cond, Hh, W), (T, Hh, W), T * Hh * W, cond * Hh * W
+    g = torch.Generator().manual_seed(7)
+    qkv = torch.randn(2, S, 3, Hn, 128, generator=g).to(dt).cuda()
+    kc, vc = (torch.randn(1, Hn, Sc, 128, generator=g).to(dt).cuda().expand(2, -1, -1, -1) for _ in range(2))
+    qw, kw = ((1 + 0.1 * torch.randn(128, generator=g)).to(dt).cuda() for _ in range(2))
+    qs, ks, vs = qkv.permute(2, 0, 3, 1, 4).unbind(0)
+    tab = att.rope_table(full, 128, qkv.device)
+    k_out, v_out = (torch.full((2, Hn, S, 128), float("nan"), dtype=dt, device="cuda") for _ in range(2))
+    got = bi._bsa_3d(qs, ks, vs, new, full, 0.5, ch, ch, qk_norm=(qw, kw, tab, T + cond, cond, 0, 1e-6), kv_cache=(kc, vc, cond),
+                     kv_out=(k_out, v_out))
+    empty = lambda s: torch.empty(2, Hn, s, 128, dtype=dt, device="cuda")      # noqa: E731
+    k, v = empty(S + Sc), torch.cat([vc, vs], 2)
+    att.norm_rope(kc, k[:, :, :Sc], None, (cond, Hh, W), table_grid=full)
+    att.norm_rope(ks, k[:, :, Sc:], kw, new, t_offset=cond, table_grid=full)
+    q = att.norm_rope(qs, empty(S), qw, new, t_offset=cond, table_grid=full)
+    assert torch.equal(got, bi.flash_attn_bsa_3d(q, k, v, new, full, sparsity=0.5, chunk_3d_shape_q=ch, chunk_3d_shape_k=ch))
+    assert torch.equal(k_out, att.norm_rope(ks, empty(S), kw)) and torch.equal(v_out, vs)
