@@ -187,7 +187,7 @@ struct PrepRows {
     uint64_t* valid;                 // k, optional: bit s of word i = slot 64 i + s holds a real token
     const uint64_t* valid_in;        // k, v, optional: the real slots of every tile as the caller has them (instead of the grid's)
     float* tile_norm;                // k, optional: largest Euclidean norm of a row of every tile, a part in a thousand above
-    const uint16_t* norm_w;          // q, k, optional: 128 weights of a per-head RMSNorm that the rows go through first
+    const uint16_t* norm_w;          // q, k, with a rotation table: 128 weights of the per-head RMSNorm in front of the rotation
     int t0;                          // q, k: frame offset of the grid inside the rotation table
     uint16_t* rows_out;              // optional: the rows of p at their token positions; q after the transform, k before the rotation
     int64_t rB, rH, rS;              // ... element strides
@@ -198,7 +198,7 @@ struct PrepArgs {
     PrepRows q, k, v;
     Grid3 gq, gk;
     int Hn;
-    const float* tab;                // rotation table (the layout bsa_norm_rope reads) for q and k; null: no rotation
+    const float* tab;                // rotation table (the layout bsa_norm_rope reads) for q and k; null: rows as they are
     int tab_T;                       // ... its frames
     float eps;
     uint32_t* zero;                  // optional: a word to clear

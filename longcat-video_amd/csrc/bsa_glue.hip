@@ -51,58 +51,83 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
 // out = T(((x - mean) * rsqrt(var + eps)) * (scale + 1) + shift), everything in fp32 with one rounding at
 // the end; mean and the biased variance over the row (two passes over registers).  shift / scale are fp32
 // rows shared by `rows_per_group` consecutive rows (one latent frame).  One wavefront per row, dim <= 8192.
-template <typename T>
-__global__ __launch_bounds__(256) void layernorm_modulate_kernel(const T* __restrict__ x, const float* __restrict__ shift,
+// HBM-bound if shift and scale stay on the CU: read from L2 for every row they are four times the row's own bytes (205 us
+// for 32 760 rows of 4 096, 2.6 TB/s of x and out).  A workgroup therefore holds them in LDS for kLnRows rows of a group
+// (in two planes of four, so that the lanes' 16-byte reads fall on different banks).
+constexpr int kLnRows = 32;
+template <typename T, int kPieces>        // 16-byte pieces of a row per lane: dim <= 512 kPieces
+__global__ __launch_bounds__(256, kPieces <= 8 ? 4 : 2) void layernorm_modulate_kernel(const T* __restrict__ x, const float* __restrict__ shift,
                                                                  const float* __restrict__ scale, T* __restrict__ out,
-                                                                 int64_t rows, int rows_per_group, int dim, float eps) {
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const T* xr = x + row * dim;
-    const float* sh = shift + (row / rows_per_group) * dim;
-    const float* sc = scale + (row / rows_per_group) * dim;
-    uint4 raw[16];                     // the row stays in registers in its storage type
-    float sum = 0.f;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int d = j * 512 + lane * 8;
-        if (d < dim) {
-            raw[j] = *reinterpret_cast<const uint4*>(xr + d);
-            const T* e = reinterpret_cast<const T*>(&raw[j]);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) sum += (float)e[i];
-        }
+                                                                 int rows_per_group, int per_group, int dim, float eps) {
+    extern __shared__ __attribute__((aligned(16))) float ln_lds[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int group = blockIdx.x / per_group, row0 = (blockIdx.x - group * per_group) * kLnRows;
+    const int n = min(kLnRows, rows_per_group - row0), plane = dim / 2;
+    float* const sc = ln_lds;                    // scale + 1
+    float* const sh = ln_lds + dim;
+    for (int d = threadIdx.x * 4; d < dim; d += 1024) {
+        const int at = (d >> 3) * 4 + ((d >> 2) & 1) * plane;
+        float4 a = *reinterpret_cast<const float4*>(scale + (int64_t)group * dim + d);
+        a.x = __fadd_rn(a.x, 1.0f); a.y = __fadd_rn(a.y, 1.0f); a.z = __fadd_rn(a.z, 1.0f); a.w = __fadd_rn(a.w, 1.0f);
+        *reinterpret_cast<float4*>(sc + at) = a;
+        *reinterpret_cast<float4*>(sh + at) = *reinterpret_cast<const float4*>(shift + (int64_t)group * dim + d);
     }
+    __syncthreads();
+    for (int r = wave; r < n; r += 4) {
+        const int64_t row = (int64_t)group * rows_per_group + row0 + r;
+        const T* xr = x + row * dim;
+        uint4 raw[kPieces];                     // the row stays in registers in its storage type
+        float sum = 0.f;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-    const float mean = sum / (float)dim;
-    float sq = 0.f;
+        for (int j = 0; j < kPieces; ++j)
+            if (j * 512 + lane * 8 < dim) raw[j] = *reinterpret_cast<const uint4*>(xr + j * 512 + lane * 8);
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-        if (j * 512 + lane * 8 < dim) {
-            const T* e = reinterpret_cast<const T*>(&raw[j]);
+        for (int j = 0; j < kPieces; ++j)
+            if (j * 512 + lane * 8 < dim) {
+                const T* e = reinterpret_cast<const T*>(&raw[j]);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) { const float c = (float)e[i] - mean; sq = fmaf(c, c, sq); }
-        }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
-    const float rstd = rsqrtf(sq / (float)dim + eps);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const int d = j * 512 + lane * 8;
-        if (d < dim) {
-            const float4 s0 = *reinterpret_cast<const float4*>(sc + d), s1 = *reinterpret_cast<const float4*>(sc + d + 4);
-            const float4 h0 = *reinterpret_cast<const float4*>(sh + d), h1 = *reinterpret_cast<const float4*>(sh + d + 4);
-            const float scl[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-            const float sft[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
-            const T* e = reinterpret_cast<const T*>(&raw[j]);
-            T res[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const float n = __fmul_rn((float)e[i] - mean, rstd);
-                res[i] = (T)__fadd_rn(__fmul_rn(n, __fadd_rn(scl[i], 1.0f)), sft[i]);     // x * (scale + 1) + shift
+                for (int i = 0; i < 8; ++i) sum += (float)e[i];
             }
-            *reinterpret_cast<uint4*>(out + row * dim + d) = *reinterpret_cast<const uint4*>(res);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+        const float mean = sum / (float)dim;
+        // widened again in every pass: kept in fp32 between them, a row of 4 096 would take 64 registers more and spill
+        auto forget = [&]() {
+#pragma unroll
+            for (int j = 0; j < kPieces; ++j) asm volatile("" : "+v"(raw[j].x), "+v"(raw[j].y), "+v"(raw[j].z), "+v"(raw[j].w));
+        };
+        forget();
+        float sq = 0.f;
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            if (j * 512 + lane * 8 < dim) {
+                const T* e = reinterpret_cast<const T*>(&raw[j]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) { const float c = (float)e[i] - mean; sq = fmaf(c, c, sq); }
+            }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o);
+        forget();
+        const float rstd = rsqrtf(sq / (float)dim + eps);
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j) {
+            const int d = j * 512 + lane * 8;
+            if (d < dim) {
+                const float* a = sc + (d >> 3) * 4;
+                const float* b = sh + (d >> 3) * 4;
+                const float4 s0 = *reinterpret_cast<const float4*>(a), s1 = *reinterpret_cast<const float4*>(a + plane);
+                const float4 h0 = *reinterpret_cast<const float4*>(b), h1 = *reinterpret_cast<const float4*>(b + plane);
+                const float scl[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+                const float sft[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+                const T* e = reinterpret_cast<const T*>(&raw[j]);
+                T res[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float nrm = __fmul_rn((float)e[i] - mean, rstd);
+                    res[i] = (T)__fadd_rn(__fmul_rn(nrm, scl[i]), sft[i]);     // x * (scale + 1) + shift
+                }
+                *reinterpret_cast<uint4*>(out + row * dim + d) = *reinterpret_cast<const uint4*>(res);
+            }
         }
     }
 }
@@ -324,12 +349,18 @@ int bsa_layernorm_modulate(const void* x, const float* shift, const float* scale
     if (!(eps >= 0.f)) return set_error(BSA_ERR_BAD_ARG, "layernorm_modulate: eps must be non-negative");
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(shift) | reinterpret_cast<uintptr_t>(scale) | reinterpret_cast<uintptr_t>(out)) & 15u)
         return set_error(BSA_ERR_BAD_ARG, "layernorm_modulate: pointers must be 16-byte aligned");
-    const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-    if (dtype == BSA_BF16)
-        hipLaunchKernelGGL((layernorm_modulate_kernel<__bf16>), grid, block, 0, (hipStream_t)stream, (const __bf16*)x, shift, scale, (__bf16*)out, rows, rows_per_group, dim, eps);
-    else if (dtype == BSA_F16)
-        hipLaunchKernelGGL((layernorm_modulate_kernel<_Float16>), grid, block, 0, (hipStream_t)stream, (const _Float16*)x, shift, scale, (_Float16*)out, rows, rows_per_group, dim, eps);
-    else
+    const int per_group = (rows_per_group + kLnRows - 1) / kLnRows;
+    const int64_t wgs = rows / rows_per_group * per_group;
+    if (wgs > 0x7fffffffLL) return set_error(BSA_ERR_UNSUPPORTED, "layernorm_modulate: too many rows");
+    const dim3 grid((unsigned)wgs), block(256);
+    const size_t lds = (size_t)2 * dim * sizeof(float);            // at most 64 KB
+#define BSA_LN(T, N) hipLaunchKernelGGL((layernorm_modulate_kernel<T, N>), grid, block, lds, (hipStream_t)stream, (const T*)x, shift, scale, (T*)out, rows_per_group, per_group, dim, eps)
+    if (dtype == BSA_BF16) {
+        if (dim <= 2048) BSA_LN(__bf16, 4); else if (dim <= 4096) BSA_LN(__bf16, 8); else BSA_LN(__bf16, 16);
+    } else if (dtype == BSA_F16) {
+        if (dim <= 2048) BSA_LN(_Float16, 4); else if (dim <= 4096) BSA_LN(_Float16, 8); else BSA_LN(_Float16, 16);
+    } else
+#undef BSA_LN
         return set_error(BSA_ERR_UNSUPPORTED, "layernorm_modulate: dtype %d is not built (bf16, fp16)", dtype);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? BSA_OK : set_error(BSA_ERR_HIP, "layernorm_modulate launch: %s", hipGetErrorString(e));

@@ -118,12 +118,16 @@ __device__ __forceinline__ void place(int id, int per_head, int Hn, int head_fas
 constexpr int kPitchK = kD + 4;      // elements: 264-byte rows for 16-byte pieces read row by row
 constexpr int kPitchV = kD + 16;     // 288-byte rows: the transposing reads fetch 4 keys x 16 d per 16 lanes, and with rows 72 banks apart the four keys fall on different banks
 
+// kMode: rows as they are; with norm and rotation; and with a cache in front of k and v, or their rows written out.
+enum { kPlain, kNorm, kCached };
+
 // k (or q, when it has a row transform): a workgroup per chunk, tile by tile.  The chunk mean keeps permute_kernel's order
 // of summation - a thread adds its rows rg, rg + 16, ... of the chunk, then the 16 partial sums of a column are added in
 // ascending rg, one rounding at the end - so every route gives the same bits.
-template <bool kBf16, bool kTransform, bool kIsK>
+template <bool kBf16, int kMode, bool kIsK>
 __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int Hn, int id, const float* tab, int tab_T, float eps,
                                          uint16_t* tile, float2* cs) {
+    constexpr bool kTransform = kMode != kPlain, kCache = kMode == kCached;
     typedef typename std::conditional<kBf16, __bf16, _Float16>::type T;
     const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
     int blk, bh;
@@ -131,10 +135,16 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
     const int lane = threadIdx.x & 63;
     const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;      // 16 pieces of 16 B per row, 16 rows at a time
     const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
-    const uint16_t* old = kTransform && x.cached != nullptr ? x.cached + (int64_t)(bh / Hn) * x.cB + (int64_t)(bh % Hn) * x.cH + c16 * 8 : nullptr;
+    const uint16_t* old = kCache && x.cached != nullptr ? x.cached + (int64_t)(bh / Hn) * x.cB + (int64_t)(bh % Hn) * x.cH + c16 * 8 : nullptr;
     // Rotation: a chunk spans at most 8 positions per axis, and a rotation pair turns with one axis only, so the
     // (cos, sin) the rows of the chunk need are 8 x 64 table entries, fetched once per workgroup instead of per row and head.
-    if (kTransform && tab != nullptr) {
+    int turn[4];                          // where the position that turns this lane's pair jj stands in Slots::loc
+    if (kTransform) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) {
+            const int pr = c16 * 4 + jj;
+            turn[jj] = pr < kRopePairsT ? 0 : pr < kRopePairsT + kRopePairsH ? 8 : 16;
+        }
         const int nw = blk % g.Nw, nh = (blk / g.Nw) % g.Nh, nt = blk / (g.Nw * g.Nh);
         for (int e = threadIdx.x; e < 8 * 64; e += 256) {
             const int a = e >> 6, pr = e & 63;
@@ -167,7 +177,7 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         for (int i = 0; i < 4; ++i) {
             token[i] = __shfl(s.token, rg + 16 * i);
             if (kTransform) loc[i] = __shfl(s.loc, rg + 16 * i);
-            xs[i] = *reinterpret_cast<const uint4*>(kTransform ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
+            xs[i] = *reinterpret_cast<const uint4*>(kCache ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
         }
         if (s.word != ~0ull) {
 #pragma unroll
@@ -178,31 +188,28 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
             if (x.rows != nullptr) x.rows[(int64_t)tile_id * kTile + front_place(s.word, lane)] = s.token;
         }
         if (kTransform) {
-            uint4 wraw = make_uint4(0, 0, 0, 0);
-            if (x.norm_w != nullptr) wraw = *reinterpret_cast<const uint4*>(x.norm_w + c16 * 8);
+            const uint4 wraw = *reinterpret_cast<const uint4*>(x.norm_w + c16 * 8);
             uint16_t* rows = x.rows_out == nullptr ? nullptr : x.rows_out + (int64_t)(bh / Hn) * x.rB + (int64_t)(bh % Hn) * x.rH + c16 * 8;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (token[i] < 0) continue;                         // the 16 lanes of a row go together
-                float c[4] = {1.f, 1.f, 1.f, 1.f}, sn[4] = {0.f, 0.f, 0.f, 0.f};
-                if (tab != nullptr) {
-                    const int ti = loc[i] & 255, hi = (loc[i] >> 8) & 255, wi = loc[i] >> 16;
+                float c[4], sn[4];
 #pragma unroll
-                    for (int jj = 0; jj < 4; ++jj) {
-                        const int pr = c16 * 4 + jj;
-                        const float2 a = cs[(pr < kRopePairsT ? ti : pr < kRopePairsT + kRopePairsH ? hi : wi) * 64 + pr];
-                        c[jj] = a.x;
-                        sn[jj] = a.y;
-                    }
+                for (int jj = 0; jj < 4; ++jj) {
+                    const float2 a = cs[((loc[i] >> turn[jj]) & 255) * 64 + c16 * 4 + jj];
+                    c[jj] = a.x;
+                    sn[jj] = a.y;
                 }
-                const bool fresh = old == nullptr || token[i] >= x.split;      // the cache holds normalised rows
-                if (kIsK && rows != nullptr) {
-                    xs[i] = norm_rope_piece<T>(xs[i], wraw, x.norm_w != nullptr && fresh, false, c, sn, eps);
-                    if (fresh) *reinterpret_cast<uint4*>(rows + (int64_t)(old == nullptr ? token[i] : token[i] - x.split) * x.rS) = xs[i];
-                    xs[i] = norm_rope_piece<T>(xs[i], wraw, false, tab != nullptr, c, sn, eps);
+                if (!kCache) {
+                    xs[i] = norm_rope_piece<T>(xs[i], wraw, true, true, c, sn, eps);
+                    if (!kIsK) *reinterpret_cast<uint4*>(rows + (int64_t)token[i] * x.rS) = xs[i];
                 } else {
-                    xs[i] = norm_rope_piece<T>(xs[i], wraw, x.norm_w != nullptr && fresh, tab != nullptr, c, sn, eps);
-                    if (!kIsK && rows != nullptr) *reinterpret_cast<uint4*>(rows + (int64_t)token[i] * x.rS) = xs[i];
+                    const int at = old == nullptr ? token[i] : token[i] - x.split;       // of p; below 0: cached (the cache holds normalised rows)
+                    if (at >= 0) {
+                        xs[i] = norm_rope_piece<T>(xs[i], wraw, true, false, c, sn, eps);
+                        if (rows != nullptr) *reinterpret_cast<uint4*>(rows + (int64_t)at * x.rS) = xs[i];
+                    }
+                    xs[i] = norm_rope_piece<T>(xs[i], wraw, false, true, c, sn, eps);
                 }
             }
         }
@@ -276,7 +283,7 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
 }
 
 // v: a workgroup per tile, gathered into LDS and read transposed: a piece holds 8 keys of one d
-template <bool kTransform>
+template <bool kCache>
 __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, int Hn, int id, uint16_t* tile) {
     const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
     int tile_id, bh;
@@ -284,7 +291,7 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
     const int lane = threadIdx.x & 63;
     const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
     const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
-    const uint16_t* old = kTransform && x.cached != nullptr ? x.cached + (int64_t)(bh / Hn) * x.cB + (int64_t)(bh % Hn) * x.cH + c16 * 8 : nullptr;
+    const uint16_t* old = kCache && x.cached != nullptr ? x.cached + (int64_t)(bh / Hn) * x.cB + (int64_t)(bh % Hn) * x.cH + c16 * 8 : nullptr;
     Slots s = slots_of(g, tile_id / per_chunk, tile_id % per_chunk, lane);
     if (x.valid_in != nullptr) s.word = x.valid_in[tile_id];
     uint4 xs[4];
@@ -292,13 +299,13 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         token[i] = __shfl(s.token, rg + 16 * i);
-        xs[i] = *reinterpret_cast<const uint4*>(kTransform ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
+        xs[i] = *reinterpret_cast<const uint4*>(kCache ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
     }
     if (s.word != ~0ull) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) keep_if(xs[i], (s.word >> (rg + 16 * i)) & 1ull);
     }
-    if (kTransform && x.rows_out != nullptr) {
+    if (kCache && x.rows_out != nullptr) {
         uint16_t* rows = x.rows_out + (int64_t)(bh / Hn) * x.rB + (int64_t)(bh % Hn) * x.rH + c16 * 8;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -398,22 +405,23 @@ __device__ __forceinline__ void query_part(const PrepRows& x, const Grid3& g, in
 constexpr int64_t kOneLaunchGroups = 8192;
 
 enum { kAllParts, kKeys, kValues, kQueries };
-template <bool kBf16, bool kTransform, int kPart>
+template <bool kBf16, int kMode, int kPart>
 __global__ __launch_bounds__(256) void prepare_kernel(PrepArgs a, int wg_k, int wg_v, int64_t chunks_q) {
+    constexpr bool kTransform = kMode != kPlain;
     __shared__ __attribute__((aligned(16))) uint16_t tile[kPart == kQueries && !kTransform ? 8 : kTile * kPitchV];
     __shared__ float2 cs[kTransform && kPart != kValues ? 8 * 64 : 1];
     const int w = blockIdx.x;
     if (kPart <= kKeys && w == 0 && threadIdx.x == 0 && a.zero != nullptr) *a.zero = 0u;
     if (kPart == kKeys || (kPart == kAllParts && w < wg_k)) {
-        row_part<kBf16, kTransform, true>(a.k, a.gk, a.Hn, w, a.tab, a.tab_T, a.eps, tile, cs);
+        row_part<kBf16, kMode, true>(a.k, a.gk, a.Hn, w, a.tab, a.tab_T, a.eps, tile, cs);
         return;
     }
     if (kPart == kValues || (kPart == kAllParts && w < wg_k + wg_v)) {
-        value_part<kTransform>(a.v, a.gk, a.Hn, kPart == kValues ? w : w - wg_k, tile);
+        value_part<kMode == kCached>(a.v, a.gk, a.Hn, kPart == kValues ? w : w - wg_k, tile);
         return;
     }
     const int wq = kPart == kQueries ? w : w - wg_k - wg_v;
-    if (kTransform) row_part<kBf16, true, false>(a.q, a.gq, a.Hn, wq, a.tab, a.tab_T, a.eps, tile, cs);
+    if (kTransform) row_part<kBf16, kTransform ? kNorm : kPlain, false>(a.q, a.gq, a.Hn, wq, a.tab, a.tab_T, a.eps, tile, cs);
     else query_part<kBf16>(a.q, a.gq, a.Hn, (int64_t)wq * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), chunks_q);
 }
 
@@ -432,7 +440,9 @@ hipError_t launch_prepare(const PrepArgs& args, int B, int dtype, hipStream_t st
     for (PrepRows* x : {&a.q, &a.k, &a.v}) x->head_fastest = x->sH < x->sS ? 1 : 0;
     a.q.offsets_32 = ((int64_t)a.gq.T * a.gq.H * a.gq.W + 1) * a.q.sS * 2 < ((int64_t)1 << 32) ? 1 : 0;
     const int64_t bh = (int64_t)B * a.Hn;
-    const bool transform = a.q.norm_w != nullptr || a.k.norm_w != nullptr || a.tab != nullptr;
+    const bool transform = a.tab != nullptr;                    // norm and rotation come together, q's rows are always wanted
+    if (transform && (a.q.norm_w == nullptr || a.k.norm_w == nullptr || a.q.rows_out == nullptr)) return hipErrorInvalidValue;
+    const bool cached = a.k.cached != nullptr || a.k.rows_out != nullptr || a.v.rows_out != nullptr;      // comes with a transform
     const int64_t wg_k = a.k.p != nullptr ? bh * a.gk.blocks() : 0;
     const int64_t wg_v = a.v.p != nullptr ? bh * a.gk.blocks() * (a.gk.chunk() / kTile) : 0;
     const int64_t chunks_q = a.q.p != nullptr ? bh * a.gq.blocks() : 0;
@@ -443,10 +453,15 @@ hipError_t launch_prepare(const PrepArgs& args, int B, int dtype, hipStream_t st
 #define BSA_PREPARE(PART, N)                                                                                                        \
     do {                                                                                                                            \
         const dim3 grid((unsigned)(N));                                                                                             \
-        if (dtype == BSA_BF16 && transform) hipLaunchKernelGGL((prepare_kernel<true, true, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q); \
-        else if (dtype == BSA_BF16) hipLaunchKernelGGL((prepare_kernel<true, false, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);       \
-        else if (transform) hipLaunchKernelGGL((prepare_kernel<false, true, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);               \
-        else hipLaunchKernelGGL((prepare_kernel<false, false, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);       \
+        if (dtype == BSA_BF16) {                                                                                                    \
+            if (cached) hipLaunchKernelGGL((prepare_kernel<true, kCached, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);         \
+            else if (transform) hipLaunchKernelGGL((prepare_kernel<true, kNorm, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);   \
+            else hipLaunchKernelGGL((prepare_kernel<true, kPlain, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);   \
+        } else {                                                                                                                    \
+            if (cached) hipLaunchKernelGGL((prepare_kernel<false, kCached, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);        \
+            else if (transform) hipLaunchKernelGGL((prepare_kernel<false, kNorm, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);  \
+            else hipLaunchKernelGGL((prepare_kernel<false, kPlain, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);  \
+        }                                                                                                                           \
     } while (0)
     if (total <= kOneLaunchGroups) {
         BSA_PREPARE(kAllParts, total);

@@ -39,6 +39,16 @@ __device__ inline float row_ror(float x) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + N, 0xf, 0xf, false));
 }
 
+// both values rounded to T and widened again
+template <typename T>
+__device__ __forceinline__ void round_pair(float& lo, float& hi) {
+    typedef float f32x2_ __attribute__((ext_vector_type(2)));
+    typedef T t2_ __attribute__((ext_vector_type(2)));
+    const t2_ r = __builtin_convertvector((f32x2_{lo, hi}), t2_);
+    lo = (float)r[0];
+    hi = (float)r[1];
+}
+
 // The row piece of this lane through the norm (wraw: the lane's 8 weights; skipped when !do_norm) and the rotation
 // (skipped when !do_rope).  The 16 lanes of the row must all be active: the sum of squares crosses them.
 template <typename T>
@@ -63,8 +73,17 @@ __device__ inline uint4 norm_rope_piece(uint4 raw, uint4 wraw, bool do_norm, boo
         // the hardware's reciprocal square root (1 ulp) named directly: rsqrtf() expands differently under different
         // floating-point flags, and the files that share this function are compiled with different ones
         const float rs = __builtin_amdgcn_rsqf(ss * (1.0f / (float)kRopeD) + eps);
+        // two values per conversion: one by one they cost an instruction each
 #pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = (float)(T)((float)(T)(f[i] * rs) * (float)we[i]);
+        for (int i = 0; i < 8; i += 2) {
+            float lo = f[i] * rs, hi = f[i + 1] * rs;
+            round_pair<T>(lo, hi);
+            lo = lo * (float)we[i];
+            hi = hi * (float)we[i + 1];
+            round_pair<T>(lo, hi);
+            f[i] = lo;
+            f[i + 1] = hi;
+        }
     }
     T res[8];
     if (do_rope) {

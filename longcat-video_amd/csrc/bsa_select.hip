@@ -36,9 +36,12 @@ constexpr int kScorePitch = 128 + 8;     // elements: 272-byte rows keep 16-byte
 // key_norm[bh] = the largest entry of the head's tile norms (a NaN row has no bound), by one wavefront
 __device__ inline void head_norm(const HeadNorms& n, int bh, int lane) {
     float best = 0.f;
-    for (int i = lane; i < n.tiles; i += 64) {
-        const float x = n.tile_norm[(int64_t)bh * n.tiles + i];
-        best = x != x ? INFINITY : fmaxf(best, x);
+    for (int i0 = lane; i0 < n.tiles; i0 += 8 * 64) {          // eight requests in flight: the workgroup waits for this wavefront
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = n.tile_norm[(int64_t)bh * n.tiles + min(i0 + 64 * j, n.tiles - 1)];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) best = x[j] != x[j] ? INFINITY : fmaxf(best, x[j]);
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) best = fmaxf(best, __shfl_xor(best, off));

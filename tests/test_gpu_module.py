@@ -450,3 +450,19 @@ def test_cache_inside_the_operator_equals_the_separate_passes(T, cond, Hh, W):
     q = att.norm_rope(qs, empty(S), qw, new, t_offset=cond, table_grid=full)
     assert torch.equal(got, bi.flash_attn_bsa_3d(q, k, v, new, full, sparsity=0.5, chunk_3d_shape_q=ch, chunk_3d_shape_k=ch))
     assert torch.equal(k_out, att.norm_rope(ks, empty(S), kw)) and torch.equal(v_out, vs)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("frames,per,dim", [(3, 1, 8), (2, 33, 2048), (2, 32, 2056), (1, 31, 4096), (3, 70, 4104), (2, 5, 8192)])
+def test_layernorm_modulate_sizes(dtype, frames, per, dim):
+    """Rows per frame around a workgroup's 32, rows around the 2 048 and 4 096 that change the instantiation: within one
+    ulp of the fp32 expression (one rounding at the end)."""
+    g = torch.Generator().manual_seed(dim)
+    x = torch.randn(2, frames * per, dim, generator=g).to(dtype)
+    shift, scale = (torch.randn(2, frames, 1, dim, generator=g) for _ in range(2))
+    got = M().layernorm_modulate(x.cuda(), shift.cuda(), scale.cuda()).cpu().float()
+    xf = x.float().view(2, frames, per, dim)
+    n = (xf - xf.mean(-1, keepdim=True)) * torch.rsqrt(xf.var(-1, unbiased=False, keepdim=True) + 1e-6)
+    want = (n * (scale + 1) + shift).view_as(x)
+    ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
+    assert torch.all((got - want).abs() <= want.abs() * ulp + 1e-5)
