@@ -311,7 +311,7 @@ int bsa_fwd_fragment(const void* q, const void* k, const void* v, const int32_t*
     if (e == hipSuccess) e = launch_head_norm(a.k.tile_norm, knorm, B * Hn, (int)(Sk / 64), st);
     if (e == hipSuccess)
         e = launch_fwd_frag(q, kf, vf, idx, lens, tile_valid, o, lse, B, Hn, Sq, Sk, bs_q, bs_k, idx_stride, sm_scale, dtype, st,
-                            nullptr, q_st, q_st, Sq, nullptr, nullptr, knorm, fallback, true);
+                            nullptr, q_st, q_st, Sq, nullptr, nullptr, nullptr, knorm, fallback, true);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "fwd_fragment");
 }
 
@@ -420,7 +420,7 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->off_idx_sorted = take(bh * pl->nbq * (size_t)(pl->sel_width > 0 ? pl->sel_width : 1) * sizeof(int32_t));
     pl->off_lens = take(bh * pl->nbq * sizeof(int32_t));
     pl->off_valid = take((size_t)(pl->Skp / 64) * sizeof(uint64_t));
-    pl->off_qrows = take((size_t)pl->Sqp * sizeof(int32_t));
+    pl->off_qrows = take(row_table_ints(pl->Sqp) * sizeof(int32_t));
     pl->off_krows = take(pl->f32 ? (size_t)pl->Skp * sizeof(int32_t) : 0);
     pl->off_ktiles = take(pl->direct_kv ? (size_t)(pl->Skp / 64) * sizeof(uint32_t) : 0);
     // lists of unequal length (the CDF rule): work items by descending length, and the counter they are drawn with
@@ -436,7 +436,7 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->off_halves = take(bh * pl->nbq * (size_t)pl->half_width * sizeof(int32_t));
     pl->off_half_lens = take(pl->half_width > 0 ? bh * pl->nbq * sizeof(int32_t) : 0);
     // the top-k rule's lists are of one length: the last round of the attention kernel may be cut into parts
-    pl->off_parts = take(pl->frag && !pl->cdf ? frag_part_floats((int64_t)bh * (pl->Sqp / 64)) * sizeof(float) : 0);
+    pl->off_parts = take(pl->frag && !pl->cdf ? frag_part_floats(pl->gq, (int64_t)bh) * sizeof(float) : 0);
     pl->total = off;
     return BSA_OK;
 }
@@ -574,7 +574,7 @@ hipError_t attention_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, co
     if (pl.frag)
         return launch_fwd_frag(q, w.kp, w.vp, idx, lens, kv_padded(p) ? w.valid : nullptr, o, lse, p->B, p->Hn, pl.Sqp, pl.Skp,
                                pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype, st, w.qrows, q_strides, o_strides,
-                               (int64_t)p->Tq * p->Hq * p->Wq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves, parts);
+                               (int64_t)p->Tq * p->Hq * p->Wq, &pl.gq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves, parts);
     FwdLayout L;
     L.q_rows = w.qrows;
     L.k_tiles = w.ktiles;

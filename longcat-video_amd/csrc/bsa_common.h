@@ -23,6 +23,26 @@ inline Grid3 make_grid(int T, int H, int W, int t, int h, int w) {
     return g;
 }
 
+// A chunk's real rows come first in the row table of q, so that its 64-slot tiles behind the first ceil(rows / 64) hold none
+// and drop out of the attention kernel's work.  Real rows of chunk (nt, nh, nw):
+__host__ __device__ inline int chunk_rows(const Grid3& g, int nt, int nh, int nw) {
+    auto extent = [](int n, int N, int size, int all) { return n < N - 1 ? size : all - (N - 1) * size; };
+    return extent(nt, g.Nt, g.t, g.T) * extent(nh, g.Nh, g.h, g.H) * extent(nw, g.Nw, g.w, g.W);
+}
+// Tiles with real rows in the chunks in front of (nt, nh, nw); all of them for (Nt, 0, 0).  Chunks differ only in whether they
+// are the last of an axis: 8 kinds.
+__host__ __device__ inline int live_tiles_before(const Grid3& g, int nt, int nh, int nw) {
+    auto chunk = [&](int t, int h, int w) { return (chunk_rows(g, t, h, w) + 63) / 64; };
+    auto row = [&](int t, int h) { return (g.Nw - 1) * chunk(t, h, 0) + chunk(t, h, g.Nw - 1); };
+    auto plane = [&](int t) { return (g.Nh - 1) * row(t, 0) + row(t, g.Nh - 1); };
+    if (nt >= g.Nt) return (g.Nt - 1) * plane(0) + plane(g.Nt - 1);
+    return nt * plane(0) + nh * row(nt, 0) + nw * chunk(nt, nh, 0);      // (.., 0) stands for every one but the last
+}
+__host__ __device__ inline int live_query_tiles(const Grid3& g) { return live_tiles_before(g, g.Nt, 0, 0); }
+// int32 entries of the row table of q for `slots` padded slots: token row of every slot (-1: padding), then the numbers of the
+// tiles that hold real rows, ascending.
+inline size_t row_table_ints(int64_t slots) { return (size_t)(slots + slots / 64); }
+
 // Where the rows of the attention operands live.  Blocked order: tile i of a (batch, head) is rows
 // 64*i .. 64*i+63 of a contiguous [B, Hn, S, D] tensor.  THW order: tile i is (a 64-slot part of)
 // chunk i of the grid and its slots are gathered from / scattered to token positions, so the
@@ -183,7 +203,7 @@ struct PrepRows {
     int split;
     char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, the real slots of a tile first, zeros behind
     uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
-    int32_t* rows;                   // q: token row of every slot of one (batch, head), -1 = padding; the real ones of a tile first
+    int32_t* rows;                   // q: row_table_ints() entries; the real slots of a chunk come first
     uint64_t* valid;                 // k, optional: bit s of word i = slot 64 i + s holds a real token
     const uint64_t* valid_in;        // k, v, optional: the real slots of every tile as the caller has them (instead of the grid's)
     float* tile_norm;                // k, optional: largest Euclidean norm of a row of every tile, a part in a thousand above
@@ -215,13 +235,14 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk,
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
-                           const int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
+                           const Grid3* q_grid = nullptr, const int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
                            int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false, float* part_buf = nullptr);
 // fallback (optional, frag_fallback_ints(B * Hn * Sq / 64) int32): with it and key_norm the rounds run the kernel that
 // takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.  Its first word
 // counts them: fallback_cleared says that it is zero already.
-// part_buf (optional, frag_part_floats(B * Hn * Sq / 64) floats): the last, partial round may be cut into parts, merged at the end.
-size_t frag_part_floats(int64_t items);
+// q_grid (optional, with q_rows): the grid whose row table (row_table_ints) q_rows is; tiles without real rows are then left out.
+// part_buf (optional, frag_part_floats() floats): the last, partial round may be cut into parts, merged at the end.
+size_t frag_part_floats(const Grid3& q_grid, int64_t heads);
 // halves: idx and lens are HalfLists, idx_stride their row pitch (at most 4 096).
 size_t frag_fallback_ints(int64_t items);
 

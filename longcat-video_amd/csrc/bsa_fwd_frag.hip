@@ -73,7 +73,18 @@ __device__ __forceinline__ float dot2_self(f16x8 x, int e, float acc) {
 struct FragLayout {
     const int32_t* q_rows;        // token row of every blocked-order query slot, -1 = padding; null: q, o in blocked order
     int64_t q_st[3], o_st[3];     // element strides: batch, head, row
+    // The query tiles of one (batch, head) that hold real rows, n_live numbers (null: every tile): work item u is then tile
+    // tiles[u % n_live] of (batch, head) u / n_live.
+    const int32_t* tiles;
+    int n_live;
 };
+// work item u as base + *entry (entry null: base alone)
+struct ItemAt { int base; const int32_t* entry; };
+__device__ __forceinline__ ItemAt item_at(const FragLayout& L, int u, int nqt) {
+    if (L.tiles == nullptr) return {u, nullptr};
+    const int bh = u / L.n_live;
+    return {bh * nqt, L.tiles + (u - bh * L.n_live)};
+}
 
 // Lists of at most this many entries are staged in LDS for the next work item while the current one runs.
 constexpr int kPipeList = 256;
@@ -188,16 +199,30 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)drawn);
         return l < (uint32_t)n_launch ? (int)l : -1;
     };
+    // Where an item's number comes from a table, the entry is asked for one item before the item's own descriptor is.
+    struct Turn { int local, base, entry; };
+    auto look_up = [&](int local) -> Turn {
+        if (local < 0) return {-1, 0, 0};
+        const int u = !kBounded && parts.count > 1 ? local % parts.items : local;
+        if (order != nullptr) return {local, item_begin, order[u]};
+        const ItemAt at = item_at(L, item_begin + u, nqt);
+        return {local, at.base, at.entry != nullptr ? *at.entry : 0};
+    };
     int rounds_taken = 0;
-    auto next_local = [&]() -> int { return queue != nullptr ? draw() : round_local(rounds_taken++); };
+    Turn ahead = {-1, 0, 0};
+    auto next_turn = [&]() -> Turn {
+        if (queue != nullptr) return look_up(draw());
+        const Turn t = ahead;
+        ahead = look_up(round_local(rounds_taken++));
+        return t;
+    };
     // what is known of an item ahead of time: its number, the length of its list and its first entry (both as
     // they lie in memory; they are clamped where they are used)
     struct Desc { int item, nent, ent[2], local; float kn; };       // ent: the first list entry (kHalves: the first two)
-    auto fetch = [&](int local) -> Desc {
-        Desc d = {-1, 0, {0, 0}, local, INFINITY};
-        if (local < 0) return d;
-        if (!kBounded && parts.count > 1) local %= parts.items;
-        d.item = item_begin + (order != nullptr ? order[local] : local);
+    auto fetch = [&](const Turn& t) -> Desc {
+        Desc d = {-1, 0, {0, 0}, t.local, INFINITY};
+        if (t.local < 0) return d;
+        d.item = t.base + __builtin_amdgcn_readfirstlane(t.entry);
         const int bh = d.item / nqt, qblock = (int)((int64_t)(d.item % nqt) * kTile / bs_q);
         const int64_t row = (int64_t)bh * nbq + qblock;
         d.nent = lens[row];
@@ -498,13 +523,14 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     };
 
     // ---- the workgroup's items
-    Desc cur = fetch(next_local());
-    Desc nxt = fetch(next_local());
+    if (queue == nullptr) next_turn();
+    Desc cur = fetch(next_turn());
+    Desc nxt = fetch(next_turn());
     bool prepared = false;           // the current item's list, Q rows and first fragments were requested by the item before it
     int list_buf = 0;                // which of the small list buffers holds the current item's list, if prepared
     while (uni(cur.item) >= 0) {
         cur.item = uni(cur.item);
-        const Desc nx2 = fetch(next_local());                    // in flight while this item runs
+        const Desc nx2 = fetch(next_turn());                     // in flight while this item runs
         const int bh = cur.item / nqt;
         const int qtile = cur.item % nqt;
         const int64_t qrow0 = (int64_t)qtile * kTile;
@@ -530,8 +556,8 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         } else {
             beyond[0] = beyond[1] = half_base;
         }
-        const int nbh = prepare_next ? nxt.item / nqt : 0;
-        const int64_t nqrow0 = prepare_next ? (int64_t)(nxt.item % nqt) * kTile : 0;
+        const int nbh = prepare_next ? uni(nxt.item / nqt) : 0;
+        const int64_t nqrow0 = prepare_next ? (int64_t)uni(nxt.item - nbh * nqt) * kTile : 0;
         const int32_t* nlist = idx + ((int64_t)nbh * nbq + nqrow0 / bs_q) * idx_stride;
 
         if (!prepared) {
@@ -831,7 +857,8 @@ template <typename T>
 __global__ __launch_bounds__(256) void merge_parts_kernel(Parts parts, T* __restrict__ o, float* __restrict__ lse, int item_begin,
                                                           int nqt, int Hn, int64_t lse_S, FragLayout L) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 31, lh = lane >> 5;
-    const int item = item_begin + blockIdx.x, bh = item / nqt;
+    const ItemAt at = item_at(L, item_begin + blockIdx.x, nqt);
+    const int item = at.base + (at.entry != nullptr ? *at.entry : 0), bh = item / nqt;
     const int64_t qrow0 = (int64_t)(item % nqt) * kTile;
     const float* first = parts.buf + (int64_t)blockIdx.x * kPartFloats;
     const int64_t stride = (int64_t)parts.items * kPartFloats;
@@ -919,10 +946,10 @@ static int choose_parts(int items, int list_tiles, int resident) {
     }
     return best;
 }
-// floats of the parts' buffer for `total` items, whatever the length of their lists
-size_t frag_part_floats(int64_t total) {
+// floats of the parts' buffer, whatever the length of the lists
+size_t frag_part_floats(const Grid3& g, int64_t heads) {
     const int resident = resident_wavefronts();
-    const int64_t tail = total % resident, most = (int64_t)kMaxPartRounds * resident;
+    const int64_t tail = heads * live_query_tiles(g) % resident, most = (int64_t)kMaxPartRounds * resident;
     return (size_t)(tail * kMaxParts < most ? tail * kMaxParts : most) * kPartFloats;
 }
 
@@ -933,7 +960,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk,
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
-                           const int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
+                           const Grid3* q_grid, const int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
                            bool halves, float* part_buf) {
     // the C-ABI layer keeps lists within these limits (a list that is too long for the small buffers is staged in `ost`)
     if (idx_stride > (halves ? kHalfEntries : kListEntries)) return hipErrorInvalidValue;
@@ -942,7 +969,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     L.q_rows = q_rows;
     for (int i = 0; i < 3; ++i) { L.q_st[i] = q_st[i]; L.o_st[i] = o_st[i]; }
     const int per_head = (int)(Sq / kTile);
-    const int total = B * Hn * per_head;
+    const int all_tiles = B * Hn * per_head;
     const int resident = resident_wavefronts();
     const dim3 block(64);
     const uint32_t* gate = nullptr;
@@ -953,6 +980,14 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     if (kv_bh_bytes > span_limit) return hipErrorInvalidValue;
     const int heads_per_span = (int)(span_limit / kv_bh_bytes);
     const bool one_span = (int64_t)B * Hn <= heads_per_span;
+    // Query tiles without real rows drop out; they would walk their lists for nothing.  A 13x30x53 grid in 4x4x8 chunks has
+    // 448 tiles, 371 of them with rows: 820 -> 727 us for 16 heads in fp16.  (Tiles with at most 32 rows, an eighth of a 30-row
+    // grid's, stay whole: a walk with half of the MFMAs and the same loads took longer per tile, 206 against 179 us a round at
+    // 720p, and a third longer overall where such tiles ran between full ones and put the items of an XCD out of step.)
+    const int n_live = q_grid != nullptr && one_span ? live_query_tiles(*q_grid) : per_head;
+    const int total = B * Hn * n_live;
+    L.tiles = n_live < per_head ? q_rows + Sq : nullptr;
+    L.n_live = n_live;
     const uint32_t whole_span = one_span ? (uint32_t)((int64_t)B * Hn * kv_bh_bytes) : 0u;
     // the LDS DMA that brings the next item's Q rows forms its addresses from 32-bit row offsets
     const int64_t q_rows_max = q_rows != nullptr ? lse_rows : Sq;
@@ -983,11 +1018,11 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     } while (0)
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
     if (queue != nullptr && one_span) {
-        launch_schedule_choice(lens, (int)(Sq / bs_q), bs_q / kTile, total, resident, resident, idx_stride, queue, st);
+        launch_schedule_choice(lens, (int)(Sq / bs_q), bs_q / kTile, all_tiles, resident, resident, idx_stride, queue, st);
         gate = queue + 1;
-        const dim3 grid((unsigned)(total < resident ? total : resident));
-        if (bounded) BSA_FRAG_LAUNCH(true, grid, 0, total, order, queue, 1u, 0, whole_span, fb_list, fb_count);
-        else BSA_FRAG_LAUNCH(false, grid, 0, total, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
+        const dim3 grid((unsigned)(all_tiles < resident ? all_tiles : resident));
+        if (bounded) BSA_FRAG_LAUNCH(true, grid, 0, all_tiles, order, queue, 1u, 0, whole_span, fb_list, fb_count);
+        else BSA_FRAG_LAUNCH(false, grid, 0, all_tiles, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
     }
     // kRoundsPerLaunch rounds per launch, every workgroup running one item of each: the items of a round start
     // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
@@ -1000,9 +1035,9 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const int whole = n_parts > 1 ? total - tail : total;
     for (int first = 0; first < whole;) {
         int end = first + span < whole ? first + span : whole;
-        const int bh0 = first / per_head;
-        if ((end - 1) / per_head - bh0 + 1 > heads_per_span) end = (bh0 + heads_per_span) * per_head;
-        const int heads = (end - 1) / per_head - bh0 + 1;
+        const int bh0 = one_span ? 0 : first / per_head;
+        if (!one_span && (end - 1) / per_head - bh0 + 1 > heads_per_span) end = (bh0 + heads_per_span) * per_head;
+        const int heads = one_span ? B * Hn : (end - 1) / per_head - bh0 + 1;
         const int n = end - first;
         const dim3 grid((unsigned)(n < resident ? n : resident));
         if (bounded)
@@ -1025,8 +1060,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     }
     if (bounded) {
         // what the rounds left over: as many items as the list holds, found out on the device
-        const dim3 grid((unsigned)(total < resident ? total : resident));
-        BSA_FRAG_LAUNCH(false, grid, 0, total, (const int32_t*)fb_list, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, fb_count);
+        const dim3 grid((unsigned)(all_tiles < resident ? all_tiles : resident));
+        BSA_FRAG_LAUNCH(false, grid, 0, all_tiles, (const int32_t*)fb_list, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, fb_count);
     }
 #undef BSA_FRAG_LAUNCH
 #undef BSA_FRAG_LAUNCH_T

@@ -95,6 +95,18 @@ __device__ __forceinline__ int front_place(uint64_t word, int slot) {
     return (word >> slot) & 1ull ? before : __popcll(word) + slot - before;
 }
 
+// The row table of one tile of q (row_table_ints): the real slots of a chunk to its front, and the numbers of the tiles that
+// hold any.  before: real slots in the chunk's earlier tiles.
+__device__ __forceinline__ void write_row_table(const Grid3& g, int32_t* rows, int blk, int sub, int lane, const Slots& s, int before) {
+    const int nw = blk % g.Nw, nh = (blk / g.Nw) % g.Nh, nt = blk / (g.Nw * g.Nh);
+    const int real = chunk_rows(g, nt, nh, nw);
+    const int ahead = __popcll(s.word & (((uint64_t)1 << lane) - 1));
+    const int place = (s.word >> lane) & 1ull ? before + ahead : real + (sub * kTile - before) + lane - ahead;
+    rows[(int64_t)blk * g.chunk() + place] = s.token;
+    if (lane == 0 && sub * kTile < real)
+        rows[(int64_t)g.blocks() * g.chunk() + live_tiles_before(g, nt, nh, nw) + sub] = blk * (g.chunk() / kTile) + sub;
+}
+
 // the row of token t: before `split` from the cache, from there on from src
 __device__ __forceinline__ const uint16_t* row_at(const uint16_t* src, int64_t sS, const uint16_t* old, int64_t cS, int split, int t) {
     if (old == nullptr) return src + (int64_t)t * sS;
@@ -166,6 +178,7 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    int rows_before = 0;
     for (int sub = 0; sub < per_chunk; ++sub) {
         const int tile_id = blk * per_chunk + sub;
         Slots s = slots_of(g, blk, sub, lane);
@@ -185,7 +198,10 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         }
         if (bh == 0 && threadIdx.x < 64) {
             if (x.valid != nullptr && lane == 0) x.valid[tile_id] = s.word;
-            if (x.rows != nullptr) x.rows[(int64_t)tile_id * kTile + front_place(s.word, lane)] = s.token;
+            if (x.rows != nullptr) {
+                write_row_table(g, x.rows, blk, sub, lane, s, rows_before);
+                rows_before += __popcll(s.word);
+            }
         }
         if (kTransform) {
             const uint4 wraw = *reinterpret_cast<const uint4*>(x.norm_w + c16 * 8);
@@ -348,9 +364,13 @@ __device__ __forceinline__ void query_part(const PrepRows& x, const Grid3& g, in
     for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int e = 0; e < 8; ++e) part[u][e] = 0.f;
+    int rows_before = 0;
     for (int sub = 0; sub < per_chunk; ++sub) {
         const Slots s = slots_of(g, blk, sub, lane);
-        if (bh == 0 && x.rows != nullptr) x.rows[((int64_t)blk * per_chunk + sub) * kTile + front_place(s.word, lane)] = s.token;
+        if (bh == 0 && x.rows != nullptr) {
+            write_row_table(g, x.rows, blk, sub, lane, s, rows_before);
+            rows_before += __popcll(s.word);
+        }
         // every row unconditionally (a padded slot reads token 0 and is cleared afterwards): sixteen independent loads
         // per lane, no branch between them
         uint4 xs[4][4];
@@ -429,8 +449,10 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepArgs a, int wg_k, int 
 __global__ __launch_bounds__(256) void row_table_kernel(Grid3 g, int32_t* __restrict__ rows, int tiles) {
     const int tile = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63, per_chunk = g.chunk() / kTile;
     if (tile >= tiles) return;
-    const Slots s = slots_of(g, tile / per_chunk, tile % per_chunk, lane);
-    rows[(int64_t)tile * kTile + front_place(s.word, lane)] = s.token;
+    const int blk = tile / per_chunk, mine = tile % per_chunk;
+    int before = 0;
+    for (int sub = 0; sub < mine; ++sub) before += __popcll(slots_of(g, blk, sub, lane).word);
+    write_row_table(g, rows, blk, mine, lane, slots_of(g, blk, mine, lane), before);
 }
 
 }  // namespace
