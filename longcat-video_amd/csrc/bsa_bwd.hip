@@ -220,6 +220,11 @@ __device__ inline void mfma_from_v(f32x16& acc, f16x8 a, f16x8 b, const f32x16& 
     asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(init));
 }
 
+// An MFMA reads its C operand for as long as its passes run, and nothing holds back a VALU write to those registers meanwhile
+// (fifteen wait states; the compiler adds them behind its own MFMAs, not behind an assembly statement, where it sees the
+// registers free at once).  The blocks that start a chain stay allocated up to here, at least two MFMAs on.
+__device__ __forceinline__ void keep_start(const f32x16& a, const f32x16& b) { asm volatile("" :: "v"(a), "v"(b)); }
+
 constexpr int kDqStage = 2 * kBwdHalfTileBytes;              // K_s rows and V rows of 32 keys
 constexpr int kDqRingLds = 2 * kDqStage;
 
@@ -631,6 +636,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
             }
             mfma_s<false, false>(s_next, fq[b][1], kreg[c + 1]);
             mfma_s<false, false>(dp_next, fd[b][1], vreg[c + 1]);
+            if (g4 == 0) keep_start(from_m, from_d);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int i = 4 * g4 + j;
@@ -703,6 +709,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
                 mfma_s<false, false>(s0, *reinterpret_cast<const V8*>(qn + roff[c]), kreg[c]);
                 mfma_s<false, false>(dp0, *reinterpret_cast<const V8*>(dn + roff[c]), vreg[c]);
             }
+            keep_start(from_m, from_d);
             asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
             mfma_chain_end(s0); mfma_chain_end(dp0);
         }
