@@ -23,6 +23,8 @@
 // dK, dV: one kernel, a workgroup of two wavefronts per 64 keys.  S = Q K_s^T and dP = dO V^T (K_s and V rows in
 // registers as B operands) put one key per lane; P and dS in the accumulator registers are the B operands of
 // dV^T += dO^T P and dK^T += Q^T dS.  Q and dO are read as they lie in memory, through LDS (see that kernel).
+// Where its dS fits in memory the dK / dV kernel runs first and keeps it, and dQ is one product instead of three
+// (bwd_dq_from_ds_kernel).
 // The query blocks of a KV block come from a bit matrix [KV block][query block] that a small kernel fills from
 // the forward's lists (ascending order for free).  Lists are expected to name a block at most once, as a
 // selection does; for a repeated block dQ follows the list (as the forward does) and dK / dV the bit matrix, like
@@ -173,14 +175,56 @@ __global__ __launch_bounds__(256) void bwd_mask_kernel(const int32_t* __restrict
     }
 }
 
-// counts[bh * nbk + j] = number of query blocks that selected KV block j (bits set in its row of the bit matrix)
+// counts[bh * nbk + j] = number of query blocks that selected KV block j (bits set in its row of the bit matrix); with `base`
+// also the number of tile pairs of the head's blocks in front of j (per_entry pairs for each entry of a list).  One workgroup
+// per head.
 __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restrict__ bits, int32_t* __restrict__ counts,
-                                                        int words, int64_t rows) {
-    const int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x;
+                                                        int32_t* __restrict__ base, int words, int nbk, int per_entry) {
+    __shared__ int part[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t head = (int64_t)blockIdx.x * nbk;
+    int before = 0;
+    for (int j0 = 0; j0 < nbk; j0 += 256) {
+        const int j = j0 + threadIdx.x;
+        int c = 0;
+        if (j < nbk)
+            for (int w = 0; w < words; ++w) c += __popc(bits[(head + j) * words + w]);
+        if (j < nbk) counts[head + j] = c;
+        if (base == nullptr) continue;
+        int upto = c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(upto, off);
+            if (lane >= off) upto += t;
+        }
+        if (lane == 63) part[wave] = upto;
+        __syncthreads();
+        for (int w = 0; w < wave; ++w) upto += part[w];
+        if (j < nbk) base[head + j] = (before + upto - c) * per_entry;
+        before += part[0] + part[1] + part[2] + part[3];
+        __syncthreads();
+    }
+}
+
+// place[row * stride + e] = the first tile pair of list entry e in the order in which the dK / dV kernel walks the pairs of its
+// head: KV blocks ascending, inside a block its query blocks ascending (the rank of this query block among the bits of the
+// block's row).
+__global__ __launch_bounds__(256) void bwd_place_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ lens,
+                                                        const uint32_t* __restrict__ bits, const int32_t* __restrict__ base,
+                                                        int32_t* __restrict__ place, int nbq, int nbk, int stride, int words,
+                                                        int per_entry, int64_t rows) {
+    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
-    int c = 0;
-    for (int w = 0; w < words; ++w) c += __popc(bits[row * words + w]);
-    counts[row] = c;
+    const int64_t bh = row / nbq;
+    const int m = (int)(row - bh * nbq);
+    const int n = min(max(lens[row], 0), stride);
+    for (int e = threadIdx.x & 63; e < n; e += 64) {
+        const int64_t j = bh * nbk + min(max(idx[row * stride + e], 0), nbk - 1);
+        const uint32_t* r = bits + j * words;
+        int rank = __popc(r[m >> 5] & ((1u << (m & 31)) - 1u));
+        for (int w = 0; w < (m >> 5); ++w) rank += __popc(r[w]);
+        place[row * stride + e] = base[j] + rank * per_entry;
+    }
 }
 
 template <typename T, typename V8>
@@ -451,6 +495,192 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
     }
 }
 
+// ------------------------------------------------------------------ dQ from kept dS
+// Where the dK / dV kernel keeps the dS it rounds for its own product (kDsPairBytes per tile pair), dQ^T += K_s^T dS^T is all
+// that is left to do: one product of three and no exponentials.  A wavefront walks the list of its 64 query rows as in
+// bwd_dq_lds_kernel; per half tile (32 keys) the K_s rows (8 KB) and the dS of its 64 queries (4 KB) go into one of three
+// LDS stages, and both operands come out with transposing reads: the next half's while this one's sixteen MFMAs run, so all
+// three stages can be on their way.  Bound by the 24 KB per pair that enter the CU (32 MFMAs take two thirds of the time of
+// their loads at 64 B/clk); dS is read once, from beyond the L2.
+//   dS of a pair: [query half][key half][16-query step st][lane][8 elements], lane = 32 lh + key: the queries 16 st + 4 lh .. + 3
+//   and 8 further (the accumulator order of the dK / dV kernel), 1 KB per store instruction.
+//   In LDS: unit (key, lh, st) at 16-byte slot 4 key + 2 lh + st of its 2 KB block, so that the 32 lanes of a pass of a
+//   transposing read (4 keys x 16 queries, two groups) cover 256 consecutive bytes.
+constexpr int kDsPairBytes = kTile * kTile * 2;
+constexpr int kDsqStage = kBwdHalfTileBytes + kDsPairBytes / 2;
+constexpr int kDsqStages = 3;
+constexpr int kDsqLoads = kDsqStage / 1024;      // LDS DMA instructions per half
+
+template <typename T>
+__global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict__ ks, const char* __restrict__ ds,
+                                                            const int32_t* __restrict__ idx, const int32_t* __restrict__ place,
+                                                            const int32_t* __restrict__ lens, T* __restrict__ dq, int64_t Sq,
+                                                            int64_t Sk, int bs_q, int bs_k, int stride, int item_begin, int item_end,
+                                                            int round, int64_t pairs_per_head, BwdStore dq_to) {
+    typedef typename Vec8<T>::type V8;
+    extern __shared__ __attribute__((aligned(1024))) char dsq_ring[];
+    const int lane = threadIdx.x, lr = lane & 31, lh = lane >> 5;
+    const int64_t groups = Sq / kTile;
+    int64_t item;
+    {
+        const int local = blockIdx.x, r0 = local / round * round;
+        const int n = min(round, item_end - item_begin - r0), w = local - r0, x = w & 7;
+        item = item_begin + r0 + x * (n >> 3) + min(x, n & 7) + (w >> 3);
+    }
+    const int64_t bh = __builtin_amdgcn_readfirstlane((int)(item / groups));
+    const int64_t qrow0 = (int64_t)__builtin_amdgcn_readfirstlane((int)(item - bh * groups)) * kTile;
+    const int nbq = (int)(Sq / bs_q), nbk = (int)(Sk / bs_k), nsub = bs_k / kTile;
+    const int64_t lrow = bh * nbq + qrow0 / bs_q;
+    const int sub_q = (int)(qrow0 % bs_q) / kTile;
+    const int n = __builtin_amdgcn_readfirstlane(min(max(lens[lrow], 0), stride));
+    const char* k_src = reinterpret_cast<const char*>(ks) + bh * Sk * (int64_t)(kD * 2);
+    const char* ds_src = ds + bh * pairs_per_head * kDsPairBytes;
+    f32x16 acc[4][2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[t][qq][i] = 0.f;
+    const int nhalves = 2 * n * nsub;
+
+    // ---- the list, 64 entries at a time in a register each, an entry per lane (no vector load between the counted DMA loads
+    // but one pair every 64 entries)
+    int list_j = 0, list_p = 0;
+    auto take_entries = [&](int e0) {
+        const int e = min(e0 + lane, n - 1);
+        list_j = min(max(idx[lrow * stride + e], 0), nbk - 1);
+        list_p = place[lrow * stride + e];
+        asm volatile("" : "+v"(list_j), "+v"(list_p));
+    };
+    // ---- global -> LDS
+    const uint32_t lds0 = lds_address(dsq_ring);
+    uint32_t voff[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = 4 * i + (lane >> 4);                                     // + 16 j
+        const int f = ((row & 3) << 2) | ((row >> 2) & 3);
+        voff[i] = (uint32_t)(row * 256 + (((lane & 15) ^ f) << 4));
+    }
+    const uint32_t voff_ds = (uint32_t)((lane & 1) * 1024 + ((lane >> 1) & 1) * 512 + (lane >> 2) * 16);
+    int entry = 0, sub = 0, key_half = 0, issued = 0, issue_stage = 0;
+    auto issue = [&]() {                          // the next half of the walk
+        if (issued >= nhalves) return;
+        if (key_half == 0 && sub == 0 && entry > 0 && (entry & 63) == 0) take_entries(entry);
+        const int64_t tile = (int64_t)__builtin_amdgcn_readlane(list_j, entry & 63) * nsub + sub;
+        const int64_t pair = (int64_t)__builtin_amdgcn_readlane(list_p, entry & 63) + sub_q * nsub + sub;
+        auto uniform = [](const char* x) -> const char* {          // the compiler cannot tell
+            const uint64_t a = reinterpret_cast<uint64_t>(x);
+            return reinterpret_cast<const char*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+                                                 ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32));
+        };
+        const char* kp = uniform(k_src + tile * kTileBytes + key_half * kBwdHalfTileBytes);
+        const char* dp = uniform(ds_src + pair * kDsPairBytes + key_half * 2048);
+        const uint32_t dst = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + issue_stage * kDsqStage));
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load_to_lds_16(kp + j * 4096, voff[i], dst + j * 4096 + i * 1024);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) load_to_lds_16_once(dp + h * 4096 + i * 256, voff_ds, dst + kBwdHalfTileBytes + h * 2048 + i * 1024);
+        ++issued;
+        issue_stage = issue_stage == kDsqStages - 1 ? 0 : issue_stage + 1;
+        key_half ^= 1;
+        if (key_half == 0 && ++sub == nsub) { sub = 0; ++entry; }
+    };
+    // ---- LDS -> fragments
+    const int s16 = lane & 15, g1 = (lane >> 4) & 1, tx = s16 >> 2, ty = (s16 & 3) >> 1, tz = s16 & 1;
+    uint32_t toff[4][2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int hi = 0; hi < 2; ++hi)
+            toff[t][hi] = (uint32_t)((4 * lh + tx + 8 * hi) * 256) + ((((uint32_t)(4 * t + 2 * g1 + ty)) ^ (uint32_t)((4 * tx) | (lh + 2 * hi))) << 4) +
+                          (uint32_t)(tz * 8);
+    const uint32_t doff = (uint32_t)((4 * (4 * lh + tx) + 2 * tz + g1) * 16 + 8 * ty);      // chunk s16 & 3: lh' = its bit 0, the unit's half its bit 1
+    int read_stage = 0;
+    auto take = [&](V8 (&kt)[8], V8 (&dst)[2][2]) {
+        const char* part = dsq_ring + read_stage * kDsqStage;
+        auto both = [](s16x4 lo, s16x4 hi) { return __builtin_bit_cast(V8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)); };
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq) {
+                const char* d = part + kBwdHalfTileBytes + qq * 2048 + st * 1024 + doff;
+                dst[qq][st] = both(lds_read_tr16(d), lds_read_tr16(d + 512));
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const char* k = part + st * 4096;
+                kt[4 * st + t] = both(lds_read_tr16(k + toff[t][0]), lds_read_tr16(k + toff[t][1]));
+            }
+        }
+        read_stage = read_stage == kDsqStages - 1 ? 0 : read_stage + 1;
+    };
+    auto multiply = [&](const V8 (&kt)[8], const V8 (&dst)[2][2]) {
+#pragma unroll
+        for (int st = 0; st < 2; ++st)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int qq = 0; qq < 2; ++qq) acc[t][qq] = mfma32(kt[4 * st + t], dst[qq][st], acc[t][qq]);
+    };
+    // lgkmcnt(0) as the builtin: in assembly the compiler would not know of it and wait again in front of the products
+    auto reads_done = [&]() {
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        asm volatile("" ::: "memory");
+    };
+    // half hp in (kt, d); the next half's operands are read, then its stage is free for half hp + 4
+    auto step = [&](int hp, const V8 (&kt)[8], const V8 (&d)[2][2], V8 (&nkt)[8], V8 (&nd)[2][2]) {
+        if (hp + 1 < nhalves) {
+            static_assert(kDsqLoads == 12, "the counts below");
+            if (hp + 3 < nhalves) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");          // halves hp + 2 and hp + 3 may be on their way
+            else if (hp + 2 < nhalves) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            take(nkt, nd);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(kt, d);
+        __builtin_amdgcn_sched_barrier(0);
+        reads_done();
+        issue();
+    };
+    if (nhalves > 0) {
+        V8 kt[2][8], d[2][2][2];
+        take_entries(0);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // from here on the DMA loads are counted by hand
+        issue();
+        issue();
+        issue();
+        if (nhalves > 2) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        take(kt[0], d[0]);
+        reads_done();
+        issue();
+        for (int hp = 0; hp < nhalves; hp += 2) {                                // halves come in pairs
+            step(hp, kt[0], d[0], kt[1], d[1]);
+            step(hp + 1, kt[1], d[1], kt[0], d[0]);
+        }
+    }
+    // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, query lr (+ 32)
+#pragma unroll
+    for (int qq = 0; qq < 2; ++qq) {
+        T* out = store_row(dq, dq_to, bh, Sq, qrow0 + 32 * qq + lr);
+        if (out == nullptr) continue;                            // a padded slot of a token-order destination
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                T x[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) x[j] = (T)(acc[t][qq][4 * g4 + j] * kLn2);
+                *reinterpret_cast<uint2*>(out + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(x);
+            }
+    }
+}
+
 // ------------------------------------------------------------------ dK and dV in one kernel, Q and dO through LDS
 // One workgroup of two wavefronts per 64 keys; wavefront w owns keys 32 w .. 32 w + 31 and both of their gradients
 // (128 accumulator registers).  The Q and dO tiles of a query tile (64 rows x 256 B each, as they lie in memory)
@@ -471,7 +701,8 @@ constexpr int kBwdStage = 2 * kBwdHalfTile + kBwdStats;      // one half tile of
 constexpr int kBwdStages = 4;                                // two in use (this half, the next half's rows), two on their way
 
 // kMasked: as in the dQ kernel - without validity words no key is padding and the test is compiled out.
-template <typename T, bool kMasked>
+// kKeep: dS, rounded as for the product, is also written out for bwd_dq_from_ds_kernel (pair_base: bwd_count_kernel's base).
+template <typename T, bool kMasked, bool kKeep>
 __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, const T* __restrict__ dout,
                                                        const T* __restrict__ ks, const T* __restrict__ v,
                                                        const float* __restrict__ m2, const float* __restrict__ delta,
@@ -479,7 +710,8 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
                                                        const uint64_t* __restrict__ tile_valid, T* __restrict__ dk,
                                                        T* __restrict__ dv, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int words,
                                                        float dk_scale, const int32_t* __restrict__ order, int n_items, int round,
-                                                       BwdStore dk_to, BwdStore dv_to) {
+                                                       BwdStore dk_to, BwdStore dv_to, char* __restrict__ ds_out,
+                                                       const int32_t* __restrict__ pair_base, int64_t pairs_per_head) {
     typedef typename Vec8<T>::type V8;
     extern __shared__ __attribute__((aligned(1024))) char bwd_lds[];
     const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
@@ -647,12 +879,17 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
             }
         }
     };
+    const int nsub = bs_k / kTile;
+    char* const ds_item = !kKeep ? nullptr
+        : ds_out + (bh * pairs_per_head + pair_base[bh * nbk + kblk] + (krow0 / kTile) % nsub) * kDsPairBytes + wave * 2048 + lane * 16;
     auto gradients = [&](int hp, const f32x16& p, const f32x16& ds) {
         const char* qt = bwd_lds + (hp & 3) * kBwdStage;
         const char* dt = qt + kBwdHalfTile;
 #pragma unroll
         for (int st2 = 0; st2 < 2; ++st2) {
             const V8 bp = pack8<T, V8>(p, st2), bds = pack8<T, V8>(ds, st2);
+            if (kKeep)
+                __builtin_nontemporal_store(bds, reinterpret_cast<V8*>(ds_item + (int64_t)(hp >> 1) * nsub * kDsPairBytes + (hp & 1) * 4096 + st2 * 1024));
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 acc_dv[t] = mfma32(frag_tr_lds(dt, st2, t), bp, acc_dv[t]);
@@ -669,11 +906,16 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         gradients(hp, s, dp);
         // the chains into (s_next, dp_next) end here, sixteen MFMAs behind their last one
         mfma_chain_end(s_next); mfma_chain_end(dp_next);
-        if (hp + 3 < nhalves) {
-            if (wave == 0) asm volatile("s_waitcnt vmcnt(9) lgkmcnt(0)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
+        // With kKeep the two stores of this half and those of the one before may be on their way as well: a store is
+        // acknowledged later than a load (waiting for those of the half before cost 0.4 of 4.2 ms at 480p).
+        if (hp + 3 >= nhalves) {
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(kKeep ? 4 : 0) : "memory");
+        } else if (kKeep && hp == 0) {                           // no half before
+            if (wave == 0) asm volatile("s_waitcnt vmcnt(11) lgkmcnt(0)" ::: "memory");
+            else asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
         } else {
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+            if (wave == 0) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(kKeep ? 13 : 9) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(kKeep ? 12 : 8) : "memory");
         }
         __builtin_amdgcn_s_barrier();
     };
@@ -747,14 +989,49 @@ constexpr size_t kBwdLdsLimit = 160 * 1024;
 size_t bwd_dkdv_lds_bytes(int nbq) { return (size_t)kBwdStages * kBwdStage + (size_t)nbq * sizeof(int32_t); }
 int bwd_max_query_blocks() { return (int)((kBwdLdsLimit - (size_t)kBwdStages * kBwdStage) / sizeof(int32_t)); }
 
-// Workspace of the backward, in bytes: k_s in blocked order, delta and M2, the bit matrix, the lists in the dQ kernel's visiting
-// order, per KV block its number of query blocks, the KV tiles of every head by that number.
+// dS is kept between the two kernels where all of it (every list full) fits kDsBytes: 6.4 GB for 32 heads of 480p, where the
+// backward takes 6.28 ms instead of 6.61 (dQ 1.81 instead of 2.58 ms, dK / dV 3.99 instead of 3.59 with the stores).  Beyond
+// that dQ is computed from scratch: in groups of heads that fit, each with the tail of its longest lists, nothing is left of
+// the gain (32 heads of 720p in groups of seven 31.2 ms, of four 32.1, from scratch 31.3).
+constexpr size_t kDsBytes = (size_t)8 << 30;
+struct KeptDs {
+    bool keep;
+    int64_t pairs_per_head;
+};
+static KeptDs plan_ds(int64_t bh, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride) {
+    const int64_t pairs = (Sq / kTile) * idx_stride * (bs_k / kTile);
+    return {pairs <= (int64_t)(kDsBytes / kDsPairBytes) / bh, pairs};
+}
+
+// The pieces of the backward's workspace.
+struct BwdWs {
+    size_t ks, delta, m2, bits, paced, counts, order;      // k_s in blocked order; delta and M2; the bit matrix; the lists in the dQ
+                                                           // kernel's visiting order; per KV block its number of query blocks; the KV
+                                                           // tiles of every head by that number
+    size_t base, place, ds;                                // with kept dS: pairs in front of a KV block, the pair of a list entry, dS
+    size_t total;
+};
+static BwdWs bwd_ws(const KeptDs& kept, int64_t bh, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride) {
+    BwdWs w;
+    size_t off = 0;
+    auto take = [&](size_t n) { const size_t at = off; off += (n + 255) / 256 * 256; return at; };
+    const size_t words = (size_t)((Sq / bs_q + 31) / 32), nbq = (size_t)(Sq / bs_q), nbk = (size_t)(Sk / bs_k);
+    w.ks = take(bh * Sk * kD * 2);
+    w.delta = take(bh * Sq * 4);
+    w.m2 = take(bh * Sq * 4);
+    w.bits = take(bh * nbk * words * 4);
+    w.paced = take(bh * nbq * (size_t)idx_stride * 4);
+    w.counts = take(bh * nbk * 4);
+    w.order = take(bh * (size_t)(Sk / kTile) * 4);
+    w.base = take(kept.keep ? bh * nbk * 4 : 0);
+    w.place = take(kept.keep ? bh * nbq * (size_t)idx_stride * 4 : 0);
+    w.ds = take(kept.keep ? (size_t)bh * (size_t)kept.pairs_per_head * kDsPairBytes : 0);
+    w.total = off;
+    return w;
+}
 size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride) {
-    const size_t bh = (size_t)B * Hn;
-    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-    const size_t words = (size_t)((Sq / bs_q + 31) / 32);
-    return up(bh * Sk * kD * 2) + 2 * up(bh * Sq * 4) + up(bh * (Sk / bs_k) * words * 4) +
-           up(bh * (Sq / bs_q) * (size_t)idx_stride * 4) + up(bh * (Sk / bs_k) * 4) + up(bh * (Sk / kTile) * 4);
+    const int64_t bh = (int64_t)B * Hn;
+    return bwd_ws(plan_ds(bh, Sq, Sk, bs_q, bs_k, idx_stride), bh, Sq, Sk, bs_q, bs_k, idx_stride).total;
 }
 
 hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,
@@ -762,18 +1039,21 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
                       int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
                       void* workspace, hipStream_t st, const BwdThw* thw) {
     const size_t bh = (size_t)B * Hn;
-    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    const KeptDs kept = plan_ds((int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
+    const BwdWs at = bwd_ws(kept, (int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
     char* ws = static_cast<char*>(workspace);
-    auto take = [&](size_t n) { char* p = ws; ws += up(n); return p; };
-    char* ks = take(bh * Sk * kD * 2);
-    float* delta = reinterpret_cast<float*>(take(bh * Sq * 4));
-    float* m2 = reinterpret_cast<float*>(take(bh * Sq * 4));
+    char* ks = ws + at.ks;
+    float* delta = reinterpret_cast<float*>(ws + at.delta);
+    float* m2 = reinterpret_cast<float*>(ws + at.m2);
     const int nbq = (int)(Sq / bs_q), nbk = (int)(Sk / bs_k);
     const int words = (nbq + 31) / 32;
-    uint32_t* bits = reinterpret_cast<uint32_t*>(take(bh * nbk * (size_t)words * 4));
-    int32_t* paced = reinterpret_cast<int32_t*>(take(bh * nbq * (size_t)idx_stride * 4));
-    int32_t* counts = reinterpret_cast<int32_t*>(take(bh * nbk * 4));
-    int32_t* order = reinterpret_cast<int32_t*>(take(bh * (size_t)(Sk / kTile) * 4));
+    uint32_t* bits = reinterpret_cast<uint32_t*>(ws + at.bits);
+    int32_t* paced = reinterpret_cast<int32_t*>(ws + at.paced);
+    int32_t* counts = reinterpret_cast<int32_t*>(ws + at.counts);
+    int32_t* order = reinterpret_cast<int32_t*>(ws + at.order);
+    int32_t* base = reinterpret_cast<int32_t*>(ws + at.base);
+    int32_t* place = reinterpret_cast<int32_t*>(ws + at.place);
+    const int per_entry = (bs_q / kTile) * (bs_k / kTile);
 
     const int64_t qrows = (int64_t)bh * Sq, krows = (int64_t)bh * Sk;
     const float c = sm_scale * kRcpLn2;
@@ -817,7 +1097,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     hipLaunchKernelGGL(bwd_mask_kernel, dim3((unsigned)((lrows + 3) / 4)), dim3(256), 0, st, idx, lens, bits, nbq, nbk, idx_stride,
                        words, lrows);
     hipError_t e;
-    hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)((bh * nbk + 255) / 256)), dim3(256), 0, st, bits, counts, words, (int64_t)(bh * nbk));
+    hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)bh), dim3(256), 0, st, bits, counts, kept.keep ? base : nullptr, words, nbk, per_entry);
     if ((e = launch_order_by_length(counts, order, (int)bh, nbk, bs_k / kTile, nbq, st)) != hipSuccess) return e;
     // dQ walks every list in the forward kernel's visiting order when the list is ascending (a selection in block
     // order); any other order is walked as given.  The order only moves fp32 roundings of the dQ sum.
@@ -828,67 +1108,63 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     const size_t lds = bwd_dkdv_lds_bytes(nbq);
     if (lds > kBwdLdsLimit) return hipErrorInvalidValue;          // the C-ABI layer has rejected such a shape already
     const bool masked = tile_valid != nullptr;
-    // Per device, once: the four dK / dV instantiations may use all of the LDS, and the number of compute units.
+    // Per device, once: the dK / dV instantiations may use all of the LDS, and the number of compute units.
     static std::atomic<int> device_cus[64];
     int dev = 0;
     if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
     if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
     int cus = device_cus[dev].load(std::memory_order_acquire);
     if (cus == 0) {
-        const void* kernels[4] = {reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false>),
-                                  reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false>)};
+        const void* kernels[8] = {
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, false>),
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, true>),
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, false>),
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, true>)};
         for (const void* kf : kernels)
             if ((e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBwdLdsLimit)) != hipSuccess) return e;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
         device_cus[dev].store(cus, std::memory_order_release);   // threads racing here set the same attributes
     }
-    const dim3 grid_k((unsigned)(bh * (Sk / kTile)));
     // dQ: rounds of as many wavefronts as the device runs at once (one per SIMD), two rounds per launch.  The dK / dV
     // kernel runs as one grid, longest list first: its lists (the query blocks of a KV block) differ in length, and
     // rounds that wait for the longest list cost more than they bring.
     const int round = 4 * cus, span = 2 * round;
     const int total_q = (int)(bh * (Sq / kTile)), total_k = (int)(bh * (Sk / kTile));
-    if (dtype == BSA_BF16) {
-        for (int first = 0; first < total_q; first += span) {
-            const int end = first + span < total_q ? first + span : total_q;
-            if (tile_valid != nullptr)
-                hipLaunchKernelGGL((bwd_dq_lds_kernel<__bf16, true>), dim3(end - first), block, kDqRingLds, st, (const __bf16*)q,
-                                   (const __bf16*)dout, (const __bf16*)ks, (const __bf16*)v, m2, delta, paced, lens, tile_valid, (__bf16*)dq, Sq, Sk,
-                                   bs_q, bs_k, idx_stride, first, end, round, dq_to);
-            else
-                hipLaunchKernelGGL((bwd_dq_lds_kernel<__bf16, false>), dim3(end - first), block, kDqRingLds, st, (const __bf16*)q,
-                                   (const __bf16*)dout, (const __bf16*)ks, (const __bf16*)v, m2, delta, paced, lens, tile_valid, (__bf16*)dq, Sq, Sk,
-                                   bs_q, bs_k, idx_stride, first, end, round, dq_to);
-        }
-        if (masked)
-            hipLaunchKernelGGL((bwd_dkdv_kernel<__bf16, true>), grid_k, dim3(128), lds, st, (const __bf16*)q, (const __bf16*)dout,
-                               (const __bf16*)ks, (const __bf16*)v, m2, delta, bits, tile_valid, (__bf16*)dk, (__bf16*)dv, Sq, Sk, bs_q, bs_k, words,
-                               sm_scale, order, total_k, round, dk_to, dv_to);
-        else
-            hipLaunchKernelGGL((bwd_dkdv_kernel<__bf16, false>), grid_k, dim3(128), lds, st, (const __bf16*)q, (const __bf16*)dout,
-                               (const __bf16*)ks, (const __bf16*)v, m2, delta, bits, tile_valid, (__bf16*)dk, (__bf16*)dv, Sq, Sk, bs_q, bs_k, words,
-                               sm_scale, order, total_k, round, dk_to, dv_to);
-    } else {
-        for (int first = 0; first < total_q; first += span) {
-            const int end = first + span < total_q ? first + span : total_q;
-            if (tile_valid != nullptr)
-                hipLaunchKernelGGL((bwd_dq_lds_kernel<_Float16, true>), dim3(end - first), block, kDqRingLds, st, (const _Float16*)q,
-                                   (const _Float16*)dout, (const _Float16*)ks, (const _Float16*)v, m2, delta, paced, lens, tile_valid, (_Float16*)dq,
-                                   Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, dq_to);
-            else
-                hipLaunchKernelGGL((bwd_dq_lds_kernel<_Float16, false>), dim3(end - first), block, kDqRingLds, st, (const _Float16*)q,
-                                   (const _Float16*)dout, (const _Float16*)ks, (const _Float16*)v, m2, delta, paced, lens, tile_valid, (_Float16*)dq,
-                                   Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, dq_to);
-        }
-        if (masked)
-            hipLaunchKernelGGL((bwd_dkdv_kernel<_Float16, true>), grid_k, dim3(128), lds, st, (const _Float16*)q, (const _Float16*)dout,
-                               (const _Float16*)ks, (const _Float16*)v, m2, delta, bits, tile_valid, (_Float16*)dk, (_Float16*)dv, Sq, Sk, bs_q,
-                               bs_k, words, sm_scale, order, total_k, round, dk_to, dv_to);
-        else
-            hipLaunchKernelGGL((bwd_dkdv_kernel<_Float16, false>), grid_k, dim3(128), lds, st, (const _Float16*)q, (const _Float16*)dout,
-                               (const _Float16*)ks, (const _Float16*)v, m2, delta, bits, tile_valid, (_Float16*)dk, (_Float16*)dv, Sq, Sk, bs_q,
-                               bs_k, words, sm_scale, order, total_k, round, dk_to, dv_to);
+#define BSA_DKDV(T, M, K)                                                                                                              \
+    hipLaunchKernelGGL((bwd_dkdv_kernel<T, M, K>), dim3((unsigned)total_k), dim3(128), lds, st, (const T*)q, (const T*)dout, (const T*)ks,  \
+                       (const T*)v, m2, delta, bits, tile_valid, (T*)dk, (T*)dv, Sq, Sk, bs_q, bs_k, words, sm_scale, order, total_k, round,  \
+                       dk_to, dv_to, ws + at.ds, base, kept.pairs_per_head)
+#define BSA_DQ(T, M)                                                                                                                   \
+    hipLaunchKernelGGL((bwd_dq_lds_kernel<T, M>), dim3(end - first), block, kDqRingLds, st, (const T*)q, (const T*)dout, (const T*)ks, (const T*)v,  \
+                       m2, delta, paced, lens, tile_valid, (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, dq_to)
+#define BSA_DQ_DS(T)                                                                                                                   \
+    hipLaunchKernelGGL((bwd_dq_from_ds_kernel<T>), dim3(end - first), block, kDsqStages* kDsqStage, st, (const T*)ks, ws + at.ds, paced, place, lens,  \
+                       (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, kept.pairs_per_head, dq_to)
+#define BSA_BY_TYPE(F, ...)                                     \
+    do {                                                        \
+        if (dtype == BSA_BF16) F(__bf16, ##__VA_ARGS__);        \
+        else F(_Float16, ##__VA_ARGS__);                        \
+    } while (0)
+    if (kept.keep) {
+        hipLaunchKernelGGL(bwd_place_kernel, dim3((unsigned)((lrows + 3) / 4)), dim3(256), 0, st, paced, lens, bits, base, place, nbq, nbk, idx_stride,
+                           words, per_entry, lrows);
+        if (masked) BSA_BY_TYPE(BSA_DKDV, true, true);
+        else BSA_BY_TYPE(BSA_DKDV, false, true);
     }
+    for (int first = 0; first < total_q; first += span) {
+        const int end = first + span < total_q ? first + span : total_q;
+        if (kept.keep) BSA_BY_TYPE(BSA_DQ_DS);
+        else if (masked) BSA_BY_TYPE(BSA_DQ, true);
+        else BSA_BY_TYPE(BSA_DQ, false);
+    }
+    if (!kept.keep) {
+        if (masked) BSA_BY_TYPE(BSA_DKDV, true, false);
+        else BSA_BY_TYPE(BSA_DKDV, false, false);
+    }
+#undef BSA_DKDV
+#undef BSA_DQ
+#undef BSA_DQ_DS
+#undef BSA_BY_TYPE
     return hipGetLastError();
 }
 

@@ -44,6 +44,11 @@ __device__ inline void load_to_lds_16(const void* sbase, uint32_t voff, uint32_t
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
 }
+// The same for data that is read once: it leaves the L2 to what is read again.
+__device__ inline void load_to_lds_16_once(const void* sbase, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 :: "s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
+}
 // The same with 4 bytes per lane: the LDS address is m0 + 4*lane.
 __device__ inline void load_to_lds_4(const void* sbase, uint32_t voff, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"

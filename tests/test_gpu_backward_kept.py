@@ -1,0 +1,44 @@
+"""dQ from the dS that the dK / dV kernel keeps, against dQ from scratch."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def run(q, k, v, do, idx, lens, stride, chunk_q, chunk_k):
+    """The same lists in rows of `stride` entries (the workspace, and with it what is kept, is planned for full rows)."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    wide = torch.zeros(*idx.shape[:-1], stride, dtype=torch.int32, device="cuda")
+    wide[..., :idx.shape[-1]] = idx
+    sm = 1 / math.sqrt(128)
+    o, lse = bi.attn_fwd_bsa_varlen(q, k, v, sm, wide, lens, chunk_q, chunk_k)
+    grads = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+    bi.attn_bwd_bsa_varlen(do, q, k, v, o, *grads, sm, lse, wide, lens, chunk_q, chunk_k)
+    return grads
+
+
+def case(heads, nbq, nbk, width, chunk_q, chunk_k, dtype, seed=41):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    new = lambda n: torch.randn(1, heads, n, 128, generator=g, device="cuda").to(dtype)      # noqa: E731
+    q, do, k, v = new(nbq * chunk_q), new(nbq * chunk_q), new(nbk * chunk_k), new(nbk * chunk_k)
+    idx = torch.rand(1, heads, nbq, nbk, generator=g, device="cuda").argsort(-1)[..., :width].int()
+    lens = torch.randint(0, width + 1, (1, heads, nbq), generator=g, device="cuda").int()
+    return q, k, v, do, idx, lens
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("chunk_q,chunk_k,nbq,nbk,wide", [(64, 64, 600, 900, 900), (128, 64, 300, 900, 900), (64, 128, 600, 450, 450), (192, 128, 200, 450, 450)])
+def test_kept_ds_against_dq_from_scratch(dtype, chunk_q, chunk_k, nbq, nbk, wide):
+    """Rows of full length need more than is kept (8 GB), short ones do not.
+    dK and dV come from the same kernel: the same bits.  The two dQ start dP from 0 or from -delta, an fp32 rounding, so a dS
+    may round the other way: an ulp of dS (2^-8, 2^-11) of one of up to 9 x 64 terms; a row's 2-norm stays within that."""
+    q, k, v, do, idx, lens = case(3, nbq, nbk, 9, chunk_q, chunk_k, dtype)
+    dq0, dk0, dv0 = run(q, k, v, do, idx, lens, 9, chunk_q, chunk_k)
+    dq1, dk1, dv1 = run(q, k, v, do, idx, lens, wide, chunk_q, chunk_k)
+    assert torch.equal(dk0, dk1) and torch.equal(dv0, dv1)
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert torch.isfinite(dq0.float()).all()
+    assert (dq0.float() - dq1.float()).norm() <= ulp * dq1.float().norm()
+
