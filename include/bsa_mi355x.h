@@ -259,8 +259,11 @@ int bsa_fwd_3d_lse(const bsa_3d_params* p,
  *   most once); tile_valid as in bsa_fwd (padded keys get no gradient and give none).
  *   workspace: bsa_bwd_workspace_bytes() bytes, 256-byte aligned (the scaled k, two fp32 vectors per query row, a
  *   bit matrix [kv block][query block], a copy of the lists, two small per-block tables).  Ascending lists are
- *   walked in bsa_visit_order's order by the dQ kernel (fp32 roundings only).
+ *   walked in bsa_visit_order's order by the dQ kernel (fp32 roundings only).  Where it comes to at most 8 GB, the dS
+ *   of every pair of tiles is kept in it too and spares the dQ kernel two of its three products; a workspace of
+ *   bsa_bwd_workspace_least_bytes() has no room for that and is accepted all the same.
  */
+size_t bsa_bwd_workspace_least_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int D, int bs_q, int bs_k, int idx_stride, int dtype);
 size_t bsa_bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int D, int bs_q, int bs_k, int idx_stride, int dtype);
 int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
             const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv, int B,
@@ -280,6 +283,7 @@ int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const vo
  *   and k are read through the row tables by the passes that take delta and the scaled k, and the kernels store the
  *   gradient rows at their tokens: five of the eight rearrangements a caller of bsa_bwd would run are not made.
  */
+size_t bsa_bwd_3d_workspace_least_bytes(const bsa_3d_params* p, int idx_stride);      /* without the kept dS */
 size_t bsa_bwd_3d_workspace_bytes(const bsa_3d_params* p, int idx_stride);
 int bsa_bwd_3d(const bsa_3d_params* p,
                const void* q, const int64_t q_strides[3],

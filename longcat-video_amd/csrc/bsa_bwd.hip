@@ -992,7 +992,8 @@ int bwd_max_query_blocks() { return (int)((kBwdLdsLimit - (size_t)kBwdStages * k
 // dS is kept between the two kernels where all of it (every list full) fits kDsBytes: 6.4 GB for 32 heads of 480p, where the
 // backward takes 6.28 ms instead of 6.61 (dQ 1.81 instead of 2.58 ms, dK / dV 3.99 instead of 3.59 with the stores).  Beyond
 // that dQ is computed from scratch: in groups of heads that fit, each with the tail of its longest lists, nothing is left of
-// the gain (32 heads of 720p in groups of seven 31.2 ms, of four 32.1, from scratch 31.3).
+// the gain (32 heads of 720p in groups of seven 31.2 ms, of four 32.1, from scratch 31.3).  Nor is it kept when the caller's
+// workspace has no room for it: the pieces that it needs are the last ones.
 constexpr size_t kDsBytes = (size_t)8 << 30;
 struct KeptDs {
     bool keep;
@@ -1029,17 +1030,20 @@ static BwdWs bwd_ws(const KeptDs& kept, int64_t bh, int64_t Sq, int64_t Sk, int 
     w.total = off;
     return w;
 }
-size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride) {
+size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, bool least) {
     const int64_t bh = (int64_t)B * Hn;
-    return bwd_ws(plan_ds(bh, Sq, Sk, bs_q, bs_k, idx_stride), bh, Sq, Sk, bs_q, bs_k, idx_stride).total;
+    KeptDs kept = plan_ds(bh, Sq, Sk, bs_q, bs_k, idx_stride);
+    if (least) kept.keep = false;
+    return bwd_ws(kept, bh, Sq, Sk, bs_q, bs_k, idx_stride).total;
 }
 
 hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,
                       const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv,
                       int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
-                      void* workspace, hipStream_t st, const BwdThw* thw) {
+                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw) {
     const size_t bh = (size_t)B * Hn;
-    const KeptDs kept = plan_ds((int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
+    KeptDs kept = plan_ds((int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
+    kept.keep = kept.keep && bwd_ws(kept, (int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride).total <= workspace_bytes;
     const BwdWs at = bwd_ws(kept, (int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
     char* ws = static_cast<char*>(workspace);
     char* ks = ws + at.ks;

@@ -338,6 +338,10 @@ size_t bsa_bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int D, int
     if (idx_stride <= 0 || idx_stride > 4096) { set_error(BSA_ERR_BAD_ARG, "bwd: idx_stride=%d outside [1, 4096]", idx_stride); return 0; }
     return bwd_workspace_bytes(B, Hn, Sq, Sk, bs_q, bs_k, idx_stride);
 }
+size_t bsa_bwd_workspace_least_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int D, int bs_q, int bs_k, int idx_stride, int dtype) {
+    return bsa_bwd_workspace_bytes(B, Hn, Sq, Sk, D, bs_q, bs_k, idx_stride, dtype) == 0
+               ? 0 : bwd_workspace_bytes(B, Hn, Sq, Sk, bs_q, bs_k, idx_stride, true);
+}
 
 int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
             const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv, int B,
@@ -351,10 +355,10 @@ int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const vo
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(d_o) || !aligned16(dq) || !aligned16(dk) ||
         !aligned16(dv) || (reinterpret_cast<uintptr_t>(workspace) & 255u))
         return set_error(BSA_ERR_BAD_ARG, "bwd: tensors must be 16-byte aligned, the workspace 256-byte aligned");
-    const size_t need = bwd_workspace_bytes(B, Hn, Sq, Sk, bs_q, bs_k, idx_stride);
+    const size_t need = bwd_workspace_bytes(B, Hn, Sq, Sk, bs_q, bs_k, idx_stride, true);
     if (workspace_bytes < need) return set_error(BSA_ERR_WORKSPACE, "bwd: workspace of %zu bytes, %zu needed", workspace_bytes, need);
     const hipError_t e = launch_bwd(q, k, v, o, d_o, lse, idx, lens, tile_valid, dq, dk, dv, B, Hn, Sq, Sk, bs_q, bs_k, idx_stride,
-                                    sm_scale, dtype, workspace, (hipStream_t)stream);
+                                    sm_scale, dtype, workspace, workspace_bytes, (hipStream_t)stream);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "bwd launch");
 }
 
@@ -880,7 +884,7 @@ namespace {
 struct Bwd3dPlan {
     Grid3 gq, gk;
     int64_t Sqp, Skp;
-    size_t off_qp, off_vp, off_dop, off_qrows, off_krows, off_valid, off_bwd, total;
+    size_t off_qp, off_vp, off_dop, off_qrows, off_krows, off_valid, off_bwd, least, total;
 };
 int make_bwd3d_plan(const bsa_3d_params* p, int idx_stride, Bwd3dPlan* pl) {
     if (!p) return set_error(BSA_ERR_BAD_ARG, "params are null");
@@ -903,8 +907,9 @@ int make_bwd3d_plan(const bsa_3d_params* p, int idx_stride, Bwd3dPlan* pl) {
     pl->off_qrows = take((size_t)pl->Sqp * sizeof(int32_t));
     pl->off_krows = take((size_t)pl->Skp * sizeof(int32_t));
     pl->off_valid = take((size_t)(pl->Skp / 64) * sizeof(uint64_t));
-    pl->off_bwd = take(bwd_workspace_bytes(p->B, p->Hn, pl->Sqp, pl->Skp, pl->gq.chunk(), pl->gk.chunk(), idx_stride));
-    pl->total = off;
+    pl->off_bwd = off;
+    pl->least = off + up256(bwd_workspace_bytes(p->B, p->Hn, pl->Sqp, pl->Skp, pl->gq.chunk(), pl->gk.chunk(), idx_stride, true));
+    pl->total = off + up256(bwd_workspace_bytes(p->B, p->Hn, pl->Sqp, pl->Skp, pl->gq.chunk(), pl->gk.chunk(), idx_stride));
     return BSA_OK;
 }
 }  // namespace
@@ -913,6 +918,11 @@ size_t bsa_bwd_3d_workspace_bytes(const bsa_3d_params* p, int idx_stride) {
     Bwd3dPlan pl;
     if (make_bwd3d_plan(p, idx_stride, &pl) != BSA_OK) return 0;
     return pl.total;
+}
+size_t bsa_bwd_3d_workspace_least_bytes(const bsa_3d_params* p, int idx_stride) {
+    Bwd3dPlan pl;
+    if (make_bwd3d_plan(p, idx_stride, &pl) != BSA_OK) return 0;
+    return pl.least;
 }
 
 int bsa_bwd_3d(const bsa_3d_params* p, const void* q, const int64_t q_strides[3], const void* k, const int64_t k_strides[3],
@@ -932,7 +942,7 @@ int bsa_bwd_3d(const bsa_3d_params* p, const void* q, const int64_t q_strides[3]
     BSA_TRY(check_tensor(dk, dk_strides, p, "dk"));
     BSA_TRY(check_tensor(dv, dv_strides, p, "dv"));
     if (!workspace) return set_error(BSA_ERR_BAD_ARG, "bwd_3d: workspace is null");
-    if (workspace_bytes < pl.total) return set_error(BSA_ERR_WORKSPACE, "bwd_3d: workspace of %zu bytes, %zu needed", workspace_bytes, pl.total);
+    if (workspace_bytes < pl.least) return set_error(BSA_ERR_WORKSPACE, "bwd_3d: workspace of %zu bytes, %zu needed", workspace_bytes, pl.least);
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return set_error(BSA_ERR_BAD_ARG, "bwd_3d: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = (hipStream_t)stream;
@@ -959,7 +969,7 @@ int bsa_bwd_3d(const bsa_3d_params* p, const void* q, const int64_t q_strides[3]
     }
     e = launch_bwd(ws + pl.off_qp, nullptr, ws + pl.off_vp, nullptr, nullptr, nullptr, idx, lens, kv_padded(p) ? valid : nullptr, nullptr,
                    nullptr, nullptr, p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype,
-                   ws + pl.off_bwd, st, &t);
+                   ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "bwd_3d launch");
 }
 

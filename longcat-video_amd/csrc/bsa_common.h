@@ -247,8 +247,9 @@ size_t frag_part_floats(const Grid3& q_grid, int64_t heads);
 size_t frag_fallback_ints(int64_t items);
 
 
-// Backward of the blocked-order attention (bsa_bwd.hip), bf16 / fp16.  workspace: bwd_workspace_bytes() bytes.
-size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride);
+// Backward of the blocked-order attention (bsa_bwd.hip), bf16 / fp16.  workspace: bwd_workspace_bytes() bytes, or at least
+// those with `least` (then dS is not kept between the kernels and dQ is computed from scratch).
+size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, bool least = false);
 int bwd_max_query_blocks();      // the dK / dV kernel stages a KV block's query blocks in LDS: Sq / bs_q may not exceed this
 // With `thw` the caller's o, dO, lse, k and the three gradients are in token order: the passes that take delta and k_s
 // read them through the row tables (token of every blocked-order slot of one (batch, head), -1 = padding) and the
@@ -270,6 +271,6 @@ struct BwdThw {
 hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,
                       const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv,
                       int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
-                      void* workspace, hipStream_t st, const BwdThw* thw = nullptr);
+                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw = nullptr);
 
 }  // namespace bsa

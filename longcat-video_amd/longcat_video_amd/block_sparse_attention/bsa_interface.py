@@ -104,6 +104,18 @@ def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return buf
 
 
+def _backward_workspace(nbytes: int, least: int, device: torch.device) -> torch.Tensor:
+    """A backward's scratch, of which up to 8 GB are the dS it keeps between two kernels: from torch's allocator for the one
+    call, which the activations may have back afterwards; without room for dS if the card has none (slower, same result but
+    for fp32 roundings)."""
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        if least == nbytes:
+            raise
+    return torch.empty(least, dtype=torch.uint8, device=device)
+
+
 def release_workspaces() -> None:
     """Drops the cached scratch buffers (they are re-created on demand)."""
     _WORKSPACES.clear()
@@ -391,14 +403,15 @@ def attn_bwd_bsa_varlen(do, q, k, v, o, dq, dk, dv, sm_scale, M, block_indices, 
     lens = block_indices_lens.to(torch.int32).contiguous()
     assert idx.shape[:3] == (B, H, Sq // chunk_size_q) and lens.shape == idx.shape[:3] and lse.shape == (B, H, Sq)
     lib = _capi.load()
-    need = lib.bsa_bwd_workspace_bytes(B, H, Sq, Sk, D, int(chunk_size_q), int(chunk_size_k), idx.shape[3], _code(q))
+    sizes = B, H, Sq, Sk, D, int(chunk_size_q), int(chunk_size_k), idx.shape[3], _code(q)
+    need = lib.bsa_bwd_workspace_bytes(*sizes)
     if need == 0:
         raise RuntimeError("bsa_bwd: " + lib.bsa_last_error().decode())
-    ws = _workspace(need, q.device)
+    ws = _backward_workspace(need, lib.bsa_bwd_workspace_least_bytes(*sizes), q.device)
     with _on_device(q):
         _capi.check(lib.bsa_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(idx), _ptr(lens),
                                 _ptr(tile_valid), _ptr(dq), _ptr(dk), _ptr(dv), B, H, Sq, Sk, D, int(chunk_size_q),
-                                int(chunk_size_k), idx.shape[3], float(sm_scale), _code(q), _ptr(ws), need, _stream(q)),
+                                int(chunk_size_k), idx.shape[3], float(sm_scale), _code(q), _ptr(ws), ws.numel(), _stream(q)),
                     "bsa_bwd")
 
 
@@ -675,14 +688,14 @@ class _Bsa3dWithGrad(torch.autograd.Function):
 
 @functools.lru_cache(maxsize=256)
 def _plan_3d_backward(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, sm_scale, width):
-    """C-ABI parameters and workspace size of a backward call."""
+    """C-ABI parameters of a backward call and the most and the least workspace it takes."""
     lib = _capi.load()
     prm = C.byref(_capi.Bsa3dParams(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, 0, sm_scale, 0.0))
     need = lib.bsa_bwd_3d_workspace_bytes(prm, width)
     if need == 0:        # the call itself names what is wrong with the shape
         _capi.check(lib.bsa_bwd_3d(prm, *([None] * 10), None, None, None, width, *([None] * 6), None, 0, None), "bsa_bwd_3d")
         raise RuntimeError("bsa_bwd_3d: no workspace size for this problem")
-    return prm, need
+    return prm, need, lib.bsa_bwd_3d_workspace_least_bytes(prm, width)
 
 
 def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_q, chunk_k, sm_scale):
@@ -693,15 +706,15 @@ def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_
     lib = _capi.load()
     q, k, v, o, do = (_rows_ok(t) for t in (q, k, v, o, do))
     width = walk.shape[3]
-    prm, need = _plan_3d_backward(B, H, D, _code(q), *latent_q, *latent_k, *chunk_q, *chunk_k, float(sm_scale), width)
-    ws = _workspace(need, q.device)
+    prm, need, least = _plan_3d_backward(B, H, D, _code(q), *latent_q, *latent_k, *chunk_q, *chunk_k, float(sm_scale), width)
+    ws = _backward_workspace(need, least, q.device)
     dq, dk, dv = (torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in (q, k, v))
     lse, walk, lens = lse.contiguous(), walk.contiguous(), lens.contiguous()
     st = _st
     with _on_device(q):
         _capi.check(lib.bsa_bwd_3d(prm, _ptr(q), st(q), _ptr(k), st(k), _ptr(v), st(v), _ptr(o), st(o), _ptr(do), st(do),
                                    _ptr(lse), _ptr(walk), _ptr(lens), width, _ptr(dq), st(dq), _ptr(dk), st(dk), _ptr(dv), st(dv),
-                                   _ptr(ws), need, _stream(q)), "bsa_bwd_3d")
+                                   _ptr(ws), ws.numel(), _stream(q)), "bsa_bwd_3d")
     return dq, dk, dv
 
 
@@ -740,9 +753,10 @@ def _bsa_3d_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, latent_shape_q
 
 
 def _calls_directly(*tensors: torch.Tensor) -> bool:
-    """Plain tensors and nothing that wants to see the operator go by (tracing, a dispatch mode, functorch): the custom
-    op's dispatch, 20 us of a call, is then left out."""
-    return (all(type(t) is torch.Tensor or type(t) is torch.nn.Parameter for t in tensors) and torch._C._len_torch_dispatch_stack() == 0
+    """Plain tensors on the GPU and nothing that wants to see the operator go by (tracing, a dispatch or function mode,
+    functorch): the custom op's dispatch, 20 us of a call, is then left out."""
+    return (all((type(t) is torch.Tensor or type(t) is torch.nn.Parameter) and t.is_cuda for t in tensors)
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None)
 
 
@@ -789,7 +803,11 @@ def flash_attn_bsa_3d(
         return _Bsa3dWithGrad.apply(q, k, v, [int(x) for x in latent_shape_q], [int(x) for x in latent_shape_k], sparsity,
                                     cdf_threshold, [int(x) for x in chunk_3d_shape_q], [int(x) for x in chunk_3d_shape_k])
     if not torch.compiler.is_compiling() and _calls_directly(q, k, v):
-        return _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_3d_shape_q, chunk_3d_shape_k, cdf_threshold=cdf_threshold)
+        # as the custom op passes them on: plain integers, plain floats, a rule below 0 is none
+        sparsity = None if sparsity is None or sparsity < 0 else float(sparsity)
+        cdf_threshold = None if cdf_threshold is None or cdf_threshold < 0 else float(cdf_threshold)
+        return _bsa_3d(q, k, v, (int(Tq), int(Hq), int(Wq)), (int(Tk), int(Hk), int(Wk)), sparsity, (int(tq), int(hq), int(wq)),
+                       (int(tk), int(hk), int(wk)), cdf_threshold=cdf_threshold)
     return _bsa_3d_op(q, k, v, [int(x) for x in latent_shape_q], [int(x) for x in latent_shape_k],
                       -1.0 if sparsity is None else float(sparsity), -1.0 if cdf_threshold is None else float(cdf_threshold),
                       [int(x) for x in chunk_3d_shape_q], [int(x) for x in chunk_3d_shape_k])

@@ -56,3 +56,28 @@ def test_one_launch_gating_equals_the_separate_kernels(dtype, latent, heads, spa
     q, k, v = (x.cuda() for x in seeded_qkv(72, 1, heads, S, S, 128, dtype))
     o = I()._bsa_3d(q, k, v, latent, latent, sparsity, chunk, chunk, True)[0]
     assert torch.equal(I().flash_attn_bsa_3d(q, k, v, latent, latent, sparsity=sparsity, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk), o)
+
+
+def test_a_rule_below_zero_is_none():
+    """Called directly or through the custom op (a function mode sees the op go by), the arguments mean the same."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    g = torch.Generator(device="cuda").manual_seed(3)
+    grid, chunk = (4, 8, 16), [4, 4, 4]
+    q, k, v = (torch.randn(1, 2, 512, 128, generator=g, device="cuda").bfloat16() for _ in range(3))
+    kw = dict(chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk)
+    seen = []
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+    for rule in (dict(sparsity=0.5, cdf_threshold=-1.0), dict(sparsity=-0.5, cdf_threshold=0.5), dict(sparsity=0.5, cdf_threshold=0.0)):
+        direct = bi.flash_attn_bsa_3d(q, k, v, grid, grid, **rule, **kw)
+        with Mode():
+            through = bi.flash_attn_bsa_3d(q, k, v, grid, grid, **rule, **kw)
+        assert torch.equal(direct, through)
+    assert any("bsa" in s for s in seen)
+    want = bi.flash_attn_bsa_3d(q, k, v, grid, grid, sparsity=0.5, **kw)
+    assert torch.equal(want, bi.flash_attn_bsa_3d(q, k, v, grid, grid, sparsity=0.5, cdf_threshold=-1.0, **kw))
+    shape = [torch.tensor(x) for x in grid]      # sizes that are changed in place are not remembered
+    assert torch.equal(want, bi.flash_attn_bsa_3d(q, k, v, shape, shape, sparsity=0.5, **kw))
