@@ -78,12 +78,14 @@ struct FragLayout {
     const int32_t* tiles;
     int n_live;
 };
-// work item u as base + *entry (entry null: base alone)
-struct ItemAt { int base; const int32_t* entry; };
-__device__ __forceinline__ ItemAt item_at(const FragLayout& L, int u, int nqt) {
-    if (L.tiles == nullptr) return {u, nullptr};
+// The tile number (over all heads) of work item u.  The table was written by an earlier kernel and is read through the scalar
+// cache: the wait for it is its own, not one for every load of the wavefront, and all that is derived from it stays scalar.
+// (Asked for an item ahead with vector loads, at every turn of every call, it cost grids without such a table 70 of 8 500 us
+// at 32 heads of 720p.)
+__device__ __forceinline__ int item_at(const FragLayout& L, int u, int nqt) {
+    if (L.tiles == nullptr) return u;
     const int bh = u / L.n_live;
-    return {bh * nqt, L.tiles + (u - bh * L.n_live)};
+    return bh * nqt + *(const __attribute__((address_space(4))) int32_t*)(L.tiles + (u - bh * L.n_live));
 }
 
 // Lists of at most this many entries are staged in LDS for the next work item while the current one runs.
@@ -199,30 +201,16 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)drawn);
         return l < (uint32_t)n_launch ? (int)l : -1;
     };
-    // Where an item's number comes from a table, the entry is asked for one item before the item's own descriptor is.
-    struct Turn { int local, base, entry; };
-    auto look_up = [&](int local) -> Turn {
-        if (local < 0) return {-1, 0, 0};
-        const int u = !kBounded && parts.count > 1 ? local % parts.items : local;
-        if (order != nullptr) return {local, item_begin, order[u]};
-        const ItemAt at = item_at(L, item_begin + u, nqt);
-        return {local, at.base, at.entry != nullptr ? *at.entry : 0};
-    };
     int rounds_taken = 0;
-    Turn ahead = {-1, 0, 0};
-    auto next_turn = [&]() -> Turn {
-        if (queue != nullptr) return look_up(draw());
-        const Turn t = ahead;
-        ahead = look_up(round_local(rounds_taken++));
-        return t;
-    };
+    auto next_local = [&]() -> int { return queue != nullptr ? draw() : round_local(rounds_taken++); };
     // what is known of an item ahead of time: its number, the length of its list and its first entry (both as
     // they lie in memory; they are clamped where they are used)
     struct Desc { int item, nent, ent[2], local; float kn; };       // ent: the first list entry (kHalves: the first two)
-    auto fetch = [&](const Turn& t) -> Desc {
-        Desc d = {-1, 0, {0, 0}, t.local, INFINITY};
-        if (t.local < 0) return d;
-        d.item = t.base + __builtin_amdgcn_readfirstlane(t.entry);
+    auto fetch = [&](int local) -> Desc {
+        Desc d = {-1, 0, {0, 0}, local, INFINITY};
+        if (local < 0) return d;
+        if (!kBounded && parts.count > 1) local %= parts.items;
+        d.item = order != nullptr ? item_begin + order[local] : item_at(L, item_begin + local, nqt);
         const int bh = d.item / nqt, qblock = (int)((int64_t)(d.item % nqt) * kTile / bs_q);
         const int64_t row = (int64_t)bh * nbq + qblock;
         d.nent = lens[row];
@@ -523,14 +511,13 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     };
 
     // ---- the workgroup's items
-    if (queue == nullptr) next_turn();
-    Desc cur = fetch(next_turn());
-    Desc nxt = fetch(next_turn());
+    Desc cur = fetch(next_local());
+    Desc nxt = fetch(next_local());
     bool prepared = false;           // the current item's list, Q rows and first fragments were requested by the item before it
     int list_buf = 0;                // which of the small list buffers holds the current item's list, if prepared
     while (uni(cur.item) >= 0) {
         cur.item = uni(cur.item);
-        const Desc nx2 = fetch(next_turn());                     // in flight while this item runs
+        const Desc nx2 = fetch(next_local());                    // in flight while this item runs
         const int bh = cur.item / nqt;
         const int qtile = cur.item % nqt;
         const int64_t qrow0 = (int64_t)qtile * kTile;
@@ -556,8 +543,8 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         } else {
             beyond[0] = beyond[1] = half_base;
         }
-        const int nbh = prepare_next ? uni(nxt.item / nqt) : 0;
-        const int64_t nqrow0 = prepare_next ? (int64_t)uni(nxt.item - nbh * nqt) * kTile : 0;
+        const int nbh = prepare_next ? nxt.item / nqt : 0;
+        const int64_t nqrow0 = prepare_next ? (int64_t)(nxt.item % nqt) * kTile : 0;
         const int32_t* nlist = idx + ((int64_t)nbh * nbq + nqrow0 / bs_q) * idx_stride;
 
         if (!prepared) {
@@ -857,8 +844,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void merge_parts_kernel(Parts parts, T* __restrict__ o, float* __restrict__ lse, int item_begin,
                                                           int nqt, int Hn, int64_t lse_S, FragLayout L) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 31, lh = lane >> 5;
-    const ItemAt at = item_at(L, item_begin + blockIdx.x, nqt);
-    const int item = at.base + (at.entry != nullptr ? *at.entry : 0), bh = item / nqt;
+    const int item = item_at(L, item_begin + blockIdx.x, nqt), bh = item / nqt;
     const int64_t qrow0 = (int64_t)(item % nqt) * kTile;
     const float* first = parts.buf + (int64_t)blockIdx.x * kPartFloats;
     const int64_t stride = (int64_t)parts.items * kPartFloats;
