@@ -577,6 +577,9 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
         const char* kp = uniform(k_src + tile * kTileBytes + key_half * kBwdHalfTileBytes);
         const char* dp = uniform(ds_src + pair * kDsPairBytes + key_half * 2048);
         const uint32_t dst = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + issue_stage * kDsqStage));
+        // an SGPR that a VALU instruction wrote may be a VMEM address five wait states later; the compiler does not count them
+        // in front of an assembly statement (it left two)
+        asm volatile("s_nop 4" : "+s"(kp), "+s"(dp));
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
