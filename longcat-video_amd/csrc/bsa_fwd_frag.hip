@@ -1045,7 +1045,9 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         parts = {nullptr, 1, 0};
     }
     if (bounded) {
-        // what the rounds left over: as many items as the list holds, found out on the device
+        // what the schedule that ran left over, be it the rounds or the longest-first queue: as many items as the list holds,
+        // found out on the device.  Not behind the gate of either: only the one that ran has put items on the list.
+        gate = nullptr;
         const dim3 grid((unsigned)(all_tiles < resident ? all_tiles : resident));
         BSA_FRAG_LAUNCH(false, grid, 0, all_tiles, (const int32_t*)fb_list, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, fb_count);
     }
