@@ -477,6 +477,27 @@ def flash_attn_bsa(q, k, v, chunk_size_q, chunk_size_k, sparsity, cdf_threshold,
 # ---------------------------------------------------------------------------
 # R9: the operator
 # ---------------------------------------------------------------------------
+def _kv_cache_arg(q, k, plane, kv_cache, kv_out):
+    """The C ABI's view of `kv_cache` and `kv_out` (see _bsa_3d), None without either.  The kernels read the cached frames and
+    write the others by pointer and stride alone, so every extent is held against q and k here.  `plane`: tokens of a frame."""
+    if kv_cache is None and kv_out is None:
+        return None
+    c = _capi.BsaKvCache()
+    named = []
+    if kv_cache is not None:
+        c.cached_frames = int(kv_cache[2])
+        cached = (q.shape[0], q.shape[1], c.cached_frames * plane, q.shape[3])
+        named += [("k_cache", kv_cache[0], cached), ("v_cache", kv_cache[1], cached)]
+    if kv_out is not None:
+        named += [("k_out", kv_out[0], tuple(k.shape)), ("v_out", kv_out[1], tuple(k.shape))]
+    for name, t, shape in named:
+        assert tuple(t.shape) == shape, "%s is %s, expected %s" % (name, tuple(t.shape), shape)
+        assert t.dtype == q.dtype and t.device == q.device and t.stride(3) == 1, name
+        setattr(c, name, _ptr(t))
+        setattr(c, name + "_strides", _st(t))
+    return c
+
+
 def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k, want_selection=False, out=None,
             cdf_threshold=None, static_scratch=False, qk_norm=None, for_backward=False, kv_cache=None, kv_out=None):
     """`out`: optional [B,H,Sq,D] view (any B/H/S strides, contiguous D) to write into.  `sparsity` may be
@@ -523,22 +544,9 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
             qw, kw = qw.to(q.dtype).contiguous(), kw.to(q.dtype).contiguous()
             q_normed = torch.empty(B, H, Sq, D, dtype=q.dtype, device=q.device)
             n = _capi.BsaQkNorm(_ptr(qw), _ptr(kw), _ptr(tab), int(table_T), int(t_off_q), int(t_off_k), float(eps))
-            c = None
-            if kv_cache is not None or kv_out is not None:
-                c = _capi.BsaKvCache()
-                named = []
-                if kv_cache is not None:
-                    c.cached_frames = int(kv_cache[2])
-                    named += [("k_cache", kv_cache[0]), ("v_cache", kv_cache[1])]
-                if kv_out is not None:
-                    named += [("k_out", kv_out[0]), ("v_out", kv_out[1])]
-                for name, t in named:
-                    assert t.dtype == q.dtype and t.stride(3) == 1
-                    setattr(c, name, _ptr(t))
-                    setattr(c, name + "_strides", _st(t))
-                c = C.byref(c)
+            c = _kv_cache_arg(q, k, int(latent_shape_k[1]) * int(latent_shape_k[2]), kv_cache, kv_out)
             _capi.check(lib.bsa_fwd_3d_qknorm_kv(
-                prm, C.byref(n), c, _ptr(q), _st(q), _ptr(q_normed),
+                prm, C.byref(n), None if c is None else C.byref(c), _ptr(q), _st(q), _ptr(q_normed),
                 _st(q_normed), _ptr(k), _st(k),
                 _ptr(v), _st(v), _ptr(o), _st(o),
                 _ptr(ws), need, _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d (q/k norm inside)")

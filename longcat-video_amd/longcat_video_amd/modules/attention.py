@@ -436,6 +436,8 @@ class Attention(nn.Module):
             raise ValueError("forward_with_kv_cache needs num_cond_latents > 0")
         n_c = k_cache.shape[2]
         assert n_c == num_cond_latents * Hg * Wg and N == T * Hg * Wg
+        assert tuple(k_cache.shape[1:]) == tuple(v_cache.shape[1:]) == (Hn, n_c, D), \
+            "caches are %s and %s, expected [1 or %d, %d, %d, %d]" % (tuple(k_cache.shape), tuple(v_cache.shape), B, Hn, n_c, D)
         qs, ks, vs = self._project_qkv(x)
         eps = self.q_norm.eps
         grid_full = (T + num_cond_latents, Hg, Wg)

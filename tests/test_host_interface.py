@@ -85,3 +85,46 @@ def test_module_caches_are_bounded():
     d[3] = 30                                    # rewriting a key evicts nothing
     assert list(d) == [2, 3, 4] and d[3] == 30
     assert isinstance(A._GEMM_WORKSPACES, A._Bounded) and isinstance(A._ROPE_TABLES, A._Bounded)
+
+
+def _small_module(monkeypatch):
+    from longcat_video_amd.modules.attention import Attention
+    attn = Attention(256, 2, enable_bsa=True, bsa_params=dict(sparsity=0.5, chunk_3d_shape_q=[4, 4, 4], chunk_3d_shape_k=[4, 4, 4]))
+
+    def launched(x):
+        raise RuntimeError("GPU work was reached")
+
+    monkeypatch.setattr(attn, "_project_qkv", launched)
+    return attn
+
+
+@pytest.mark.parametrize("k_shape,v_shape", [
+    ((1, 2, 128, 128), (1, 2, 64, 128)),       # fewer values than keys
+    ((1, 1, 128, 128), (1, 1, 128, 128)),      # a head share of the cache
+    ((1, 2, 128, 128), (1, 1, 128, 128)),
+    ((1, 2, 128, 64), (1, 2, 128, 64)),        # another head dim
+    ((1, 2, 64, 128), (1, 2, 64, 128)),        # fewer frames than said
+])
+def test_a_cache_of_another_shape_is_refused_before_any_launch(monkeypatch, k_shape, v_shape):
+    attn = _small_module(monkeypatch)
+    x = torch.zeros(1, 256, 256, dtype=torch.bfloat16)
+    caches = [torch.zeros(s, dtype=torch.bfloat16) for s in (k_shape, v_shape)]
+    with pytest.raises(AssertionError):
+        attn.forward_with_kv_cache(x, shape=(4, 8, 8), num_cond_latents=2, kv_cache=caches)
+    good = [torch.zeros(1, 2, 128, 128, dtype=torch.bfloat16) for _ in range(2)]
+    with pytest.raises(RuntimeError, match="was reached"):
+        attn.forward_with_kv_cache(x, shape=(4, 8, 8), num_cond_latents=2, kv_cache=good)
+
+
+def test_the_operators_cache_argument_is_held_against_q_and_k():
+    t = lambda *s, dtype=torch.bfloat16: torch.zeros(*s, dtype=dtype)      # noqa: E731
+    q, k = t(1, 2, 256, 128), t(1, 2, 256, 128)
+    c = I._kv_cache_arg(q, k, 64, (t(1, 2, 128, 128), t(1, 2, 128, 128), 2), (t(1, 2, 256, 128), t(1, 2, 256, 128)))
+    assert c.cached_frames == 2 and list(c.v_cache_strides) == [2 * 128 * 128, 128 * 128, 128]
+    assert I._kv_cache_arg(q, k, 64, None, None) is None
+    for cache in ((t(1, 2, 128, 128), t(1, 2, 64, 128), 2), (t(1, 1, 128, 128), t(1, 2, 128, 128), 2),
+                  (t(1, 2, 128, 128), t(1, 2, 128, 128), 3), (t(1, 2, 128, 128), t(1, 2, 128, 128, dtype=torch.float16), 2)):
+        with pytest.raises(AssertionError):
+            I._kv_cache_arg(q, k, 64, cache, None)
+    with pytest.raises(AssertionError):
+        I._kv_cache_arg(q, k, 64, None, (t(1, 2, 256, 128), t(1, 2, 192, 128)))
