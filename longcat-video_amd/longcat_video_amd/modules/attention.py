@@ -378,6 +378,7 @@ class Attention(nn.Module):
             q, k, v = qkv_projection(x, self.qkv.weight, self.qkv.bias, self.q_norm.weight, self.k_norm.weight, shape,
                                      Hn, eps=eps)
         elif self._norm_inside_operator(x, shape):
+            assert N == int(shape[0]) * int(shape[1]) * int(shape[2]), "%d tokens on a grid of %s" % (N, tuple(shape))
             # q, k, v stay where the projection left them: the operator's pass over q (chunk means) normalises and
             # rotates it into a per-head tensor of its own, its pass over k (fragment order) does the same on the way
             # and leaves the normalised rows for the cache

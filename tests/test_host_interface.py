@@ -128,3 +128,13 @@ def test_the_operators_cache_argument_is_held_against_q_and_k():
             I._kv_cache_arg(q, k, 64, cache, None)
     with pytest.raises(AssertionError):
         I._kv_cache_arg(q, k, 64, None, (t(1, 2, 256, 128), t(1, 2, 192, 128)))
+
+
+@pytest.mark.parametrize("kw", [dict(num_cond_latents=1), dict(return_kv=True), dict()])
+def test_tokens_that_do_not_fill_the_grid_are_refused(monkeypatch, kw):
+    attn = _small_module(monkeypatch)
+    for n in (250, 260):
+        with pytest.raises(AssertionError):
+            attn(torch.zeros(1, n, 256, dtype=torch.bfloat16), shape=(4, 8, 8), **kw)
+    with pytest.raises(RuntimeError, match="was reached"):
+        attn(torch.zeros(1, 256, 256, dtype=torch.bfloat16), shape=(4, 8, 8), **kw)
