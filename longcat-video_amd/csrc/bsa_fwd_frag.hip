@@ -139,12 +139,17 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     int32_t* __restrict__ fallback, uint32_t* __restrict__ fallback_count, Parts parts) {
     typedef typename Vec8<T>::type V8;
     // log2 headroom before the running maximum is raised: probabilities reach 2^kTau, which the storage type of P
-    // must hold (fp16 ends at 65 504 = 2^15.99) and the fp32 sums must hold times the number of keys
-    constexpr float kTau = std::is_same<T, _Float16>::value ? 15.5f : 30.0f;
+    // must hold (fp16 ends at 65 504) and the fp32 sums must hold times the number of keys
+    constexpr float kTau = std::is_same<T, _Float16>::value ? 14.0f : 30.0f;
     // How far the fixed reference of an item without row maxima may lie above the largest logit of its first keys (see
-    // where the bound is tested): the largest probability of a row is then at least 2^-kSlack.  bf16 has fp32's exponents;
-    // fp16 loses relative precision below 2^-14, 2^-10 of that largest probability.
-    constexpr float kSlack = std::is_same<T, _Float16>::value ? 4.0f : 60.0f;
+    // where the bound is tested): the largest probability of a row is then at least 2^-kSlack, which costs bf16 no bit (it
+    // has fp32's exponents).  fp16 has none to spare - a probability below 2^-14 is subnormal - and always looks at the
+    // maxima: RMS-normalised rows bound their logits at 16.3, beyond its headroom, so they would all fail a test without
+    // slack and be computed behind the rounds, one list after another (16 heads of 13x30x53 in 4x4x8 chunks: 743 us
+    // with the maxima, 822 with the test and no slack, 723 with a slack of 4, which left subnormal probabilities four bits
+    // fewer).
+    constexpr float kSlack = 60.0f;
+    static_assert(!kBounded || std::is_same<T, __bf16>::value, "fp16 probabilities need the running maximum");
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     if (gate != nullptr && *gate != gate_want) return;
     // output staging: 64 rows of 256 B, 272 B apart.  The same memory stages a list that is too long for the small
@@ -978,12 +983,12 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     // the LDS DMA that brings the next item's Q rows forms its addresses from 32-bit row offsets
     const int64_t q_rows_max = q_rows != nullptr ? lse_rows : Sq;
     const int q_offsets_32 = q_rows_max * q_st[2] * 2 + 512 < ((int64_t)1 << 32) ? 1 : 0;
-    // The rounds run the kernel whose steps take no row maxima when the key norms are known, a place for the list of
+    // The bf16 rounds run the kernel whose steps take no row maxima when the key norms are known, a place for the list of
     // the items it has to leave to the other kernel is given, and that kernel can reach every head from one buffer.
     // A call of one round runs the exact kernel alone: its steps are 3 % longer, but a last launch that finds nothing to do
     // costs 3.6 us, a fifth of a small call's attention.
     Parts parts = {nullptr, 1, 0};
-    const bool bounded = key_norm != nullptr && fallback != nullptr && one_span && total > resident;      // (see `whole` below)
+    const bool bounded = dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident;      // (see `whole` below)
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
 #define BSA_FRAG_LAUNCH_T(T, WALK, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
@@ -997,9 +1002,9 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
             else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(__bf16, kTiles, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
             else BSA_FRAG_LAUNCH_T(__bf16, kBlocks, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);        \
         } else {                                                                                                       \
-            if (halves) BSA_FRAG_LAUNCH_T(_Float16, kHalves, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
-            else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(_Float16, kTiles, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
-            else BSA_FRAG_LAUNCH_T(_Float16, kBlocks, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);      \
+            if (halves) BSA_FRAG_LAUNCH_T(_Float16, kHalves, false, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
+            else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(_Float16, kTiles, false, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
+            else BSA_FRAG_LAUNCH_T(_Float16, kBlocks, false, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);   \
         }                                                                                                              \
     } while (0)
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);

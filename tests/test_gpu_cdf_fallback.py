@@ -15,8 +15,8 @@ def bi():
 
 def inputs(dtype, size):
     """Nine chunks of ten point in one direction each (peaked pooled scores, short lists), the tenth has independent rows (flat
-    scores, long lists), so the longest-first schedule wins.  Norms of 11 and 11 size: size 3 in fp16 and 8 in bf16 give bounds
-    on the logits beyond what the kernel without row maxima takes; at size 1 fp16 has items on both sides of the line."""
+    scores, long lists), so the longest-first schedule wins.  Norms of 11 and 11 size: 8 in bf16 gives
+    bounds on the logits beyond what the kernel without row maxima takes (fp16 always looks at the maxima)."""
     S = LATENT[0] * LATENT[1] * LATENT[2]
     g = torch.Generator().manual_seed(91)
     q, k, v = (torch.randn(1, HEADS, S, 128, generator=g) for _ in range(3))
