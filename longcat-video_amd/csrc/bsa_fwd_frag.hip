@@ -896,15 +896,17 @@ constexpr int kRoundsPerLaunch = 5;
 constexpr int kRoundsPerLaunchShort = 8;     // lists of at most kShortList tiles
 constexpr int kShortList = 64;
 
-// Workgroups (of one wavefront) the device runs at once with this kernel: one per SIMD.
+// Workgroups (of one wavefront) the device runs at once with this kernel: one per SIMD, at most kMostResident (256 compute
+// units).
+constexpr int kMostResident = 1024;
 static int resident_wavefronts() {
     static int cached[64] = {0};
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 1024;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return kMostResident;
     if (cached[dev] == 0) {
         int cus = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        cached[dev] = 4 * cus;
+        cached[dev] = 4 * cus < kMostResident ? 4 * cus : kMostResident;
     }
     return cached[dev];
 }
@@ -937,11 +939,11 @@ static int choose_parts(int items, int list_tiles, int resident) {
     }
     return best;
 }
-// floats of the parts' buffer, whatever the length of the lists
+// floats of the parts' buffer, whatever the length of the lists and whichever device runs the call (a caller asks for the size
+// of a workspace once, for all of its devices): a partial round has no more items than the call, choose_parts the limits
 size_t frag_part_floats(const Grid3& g, int64_t heads) {
-    const int resident = resident_wavefronts();
-    const int64_t tail = heads * live_query_tiles(g) % resident, most = (int64_t)kMaxPartRounds * resident;
-    return (size_t)(tail * kMaxParts < most ? tail * kMaxParts : most) * kPartFloats;
+    const int64_t all = heads * live_query_tiles(g) * kMaxParts, most = (int64_t)kMaxPartRounds * kMostResident;
+    return (size_t)(all < most ? all : most) * kPartFloats;
 }
 
 // int32 entries launch_fwd_frag's `fallback` argument must hold for `items` work items (64-row query tiles)

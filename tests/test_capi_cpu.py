@@ -235,3 +235,18 @@ def test_header_and_library_from_a_plain_c_program(tmp_path):
     _capi.load()                       # raises with the build hint if the library is missing
     out = subprocess.run([exe, _capi.LIB_PATH], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.startswith("ok"), (out.returncode, out.stdout, out.stderr)
+
+
+@pytest.mark.parametrize("cus", [256, 240, 128, 32])
+def test_workspace_holds_for_devices_of_any_size(cus):
+    """The last, partial round of the attention kernel may be cut into parts, 33 280 bytes each, at most 16 of an item and
+    two rounds of them.  How many items that round has depends on the device; the size that a caller asks for once must not.
+    The lists of the CDF rule are never cut, which leaves the parts as the difference between two calls of the same sizes
+    but for the CDF rule's order and queue."""
+    lib = _capi.load()
+    for heads, frames in ((4, 16), (7, 36), (1, 8)):                     # 256, 576, 128 query tiles a head
+        size = lambda cdf: lib.bsa_workspace_bytes(C.byref(_capi.Bsa3dParams(       # noqa: E731
+            1, heads, 128, _capi.BSA_BF16, frames, 32, 32, frames, 32, 32, 4, 4, 4, 4, 4, 4, 64 * frames // 4, 0.1, cdf)))
+        items, round_ = heads * 64 * frames // 4, 4 * cus
+        parts = size(0.0) - size(0.5) + 4 * items + 256                  # its order, its queue
+        assert parts >= min(items % round_ * 16, 2 * round_) * 33280
