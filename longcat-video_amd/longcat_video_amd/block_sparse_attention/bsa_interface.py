@@ -514,7 +514,7 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
     B, H, Sq, D = q.shape
     q, k, v = _rows_ok(q), _rows_ok(k), _rows_ok(v)
     lib = _capi.load()
-    plan = _plan_3d(B, H, D, _code(q), *latent_shape_q, *latent_shape_k, *chunk_q, *chunk_k, sparsity, cdf_threshold)
+    plan = _plan_of(B, H, D, _code(q), latent_shape_q, latent_shape_k, chunk_q, chunk_k, sparsity, cdf_threshold)
     prm, need, nbq, nbk, width = plan.prm, plan.need, plan.nbq, plan.nbk, plan.width
     if static_scratch and (k.stride(2) != v.stride(2) or plan.tile_tokens * k.stride(2) * k.element_size() >= 2 ** 32):
         # this route gathers k and v tiles with one set of in-tile offsets (32 bits); views that
@@ -590,6 +590,20 @@ def _plan_3d(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, spar
         _capi.check(lib.bsa_fwd_3d(p.prm, None, None, None, None, None, None, None, None, None, 0,
                                    None, None, None, None), "flash_attn_bsa_3d")
     return p
+
+
+def _plan_of(B, H, D, code, latent_q, latent_k, chunk_q, chunk_k, sparsity, cdf_threshold) -> _Plan3d:
+    """_plan_3d by the values alone: a grid given as tensor elements would be kept by their identity, and their values may
+    change.  Rules that are not plain numbers are computed with as they are, and not kept."""
+    sizes = (*latent_q, *latent_k, *chunk_q, *chunk_k)
+    if not _PLAIN.issuperset(map(type, (*sizes, sparsity, cdf_threshold))):
+        sizes = [int(x) for x in sizes]
+        if not (type(sparsity) in _PLAIN and type(cdf_threshold) in _PLAIN):
+            return _plan_3d.__wrapped__(B, H, D, code, *sizes, sparsity, cdf_threshold)
+    return _plan_3d(B, H, D, code, *sizes, sparsity, cdf_threshold)
+
+
+_PLAIN = frozenset((float, int, type(None)))
 
 
 class ThwAttention:

@@ -138,3 +138,17 @@ def test_tokens_that_do_not_fill_the_grid_are_refused(monkeypatch, kw):
             attn(torch.zeros(1, n, 256, dtype=torch.bfloat16), shape=(4, 8, 8), **kw)
     with pytest.raises(RuntimeError, match="was reached"):
         attn(torch.zeros(1, 256, 256, dtype=torch.bfloat16), shape=(4, 8, 8), **kw)
+
+
+def test_plans_are_kept_by_value():
+    """Grids as tensor elements (what an int() of them would have read at each call), rules as tensors."""
+    I._capi.load()
+    grid = [torch.tensor(8), torch.tensor(8), torch.tensor(16)]
+    rule = torch.tensor(0.5)
+    plan = lambda: I._plan_of(1, 2, 128, 0, grid, grid, (4, 4, 4), [4, 4, 4], rule, None)      # noqa: E731
+    assert (plan().nbq, plan().width) == (16, 8)
+    grid[0].fill_(16)
+    assert (plan().nbq, plan().width) == (32, 16)
+    rule.fill_(0.75)
+    assert plan().width == 8
+    assert I._plan_of(1, 2, 128, 0, (16, 8, 16), (16, 8, 16), (4, 4, 4), (4, 4, 4), 0.75, None).width == 8
