@@ -663,6 +663,10 @@ __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict_
     }
 }
 
+// What a kernel that wants more than 64 KB of LDS is allowed: all of it, whatever this call needs, so that host threads with
+// calls of different sizes do not lower each other's limit between its setting and the launch.
+constexpr size_t kLdsLimit = 160 * 1024;
+
 template <typename T>
 size_t gate_lds_bytes(int nbk, int k_sel) {
     return (size_t)GateRows<T>::kRows * gate_pitch(nbk) * sizeof(T) + (size_t)(kGateThreads / 64) * gate_wave_words(k_sel) * 4;
@@ -678,7 +682,7 @@ hipError_t launch_gate_t(const T* qc, const T* kc, int32_t* lists, int32_t* lens
 #define BSA_GATE(N)                                                                                                          \
     do {                                                                                                                     \
         if (lds > 64 * 1024) {                                                                                               \
-            const hipError_t ea = hipFuncSetAttribute((const void*)gate_kernel<T, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+            const hipError_t ea = hipFuncSetAttribute((const void*)gate_kernel<T, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit); \
             if (ea != hipSuccess) return ea;                                                                                 \
         }                                                                                                                    \
         hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0, norms, halves);  \
@@ -812,11 +816,12 @@ hipError_t launch_topk_t(const S* score, int32_t* idx, int32_t* idx_sorted, int3
     }
     // the score-order ranking keeps the winners of the workgroup's four rows in LDS
     const size_t lds = idx != nullptr ? (size_t)4 * stride * sizeof(typename KeyOf<S>::type) : 0;
+    const size_t most = (size_t)4 * kMaxSel * sizeof(typename KeyOf<S>::type);      // allowed for every call alike, as in launch_gate_t
 #define BSA_TOPK(N)                                                                                \
     do {                                                                                           \
         if (idx != nullptr) {                                                                      \
             if (lds > 64 * 1024) {                                                                 \
-                const hipError_t ea = hipFuncSetAttribute((const void*)topk_kernel<S, N, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+                const hipError_t ea = hipFuncSetAttribute((const void*)topk_kernel<S, N, true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most); \
                 if (ea != hipSuccess) return ea;                                                   \
             }                                                                                      \
             hipLaunchKernelGGL((topk_kernel<S, N, true>), grid, block, lds, st, score, idx, idx_sorted, lens, rows, nbk, k_sel, k_rows, stride);  \
@@ -866,7 +871,7 @@ bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype) {
     if (nbk > kGateMaxBlocks) return false;
     const int rows = dtype == BSA_F32 ? GateRows<float>::kRows : GateRows<__bf16>::kRows;
     const size_t lds = dtype == BSA_F32 ? gate_lds_bytes<float>(nbk, k_sel) : gate_lds_bytes<__bf16>(nbk, k_sel);
-    return lds <= 160 * 1024 && (int64_t)BH * ((nbq + rows - 1) / rows) <= kGateMaxGroups;
+    return lds <= kLdsLimit && (int64_t)BH * ((nbq + rows - 1) / rows) <= kGateMaxGroups;
 }
 
 hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,

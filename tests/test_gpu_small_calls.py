@@ -81,3 +81,28 @@ def test_a_rule_below_zero_is_none():
     assert torch.equal(want, bi.flash_attn_bsa_3d(q, k, v, grid, grid, sparsity=0.5, cdf_threshold=-1.0, **kw))
     shape = [torch.tensor(x) for x in grid]      # sizes that are changed in place are not remembered
     assert torch.equal(want, bi.flash_attn_bsa_3d(q, k, v, shape, shape, sparsity=0.5, **kw))
+
+
+def test_threads_with_different_lds_sizes():
+    """Lists of 256 and of 496 blocks (84 and 130 KB of LDS for the one-launch gating), each from a host thread and on a
+    stream of its own, at the same time: what each gives alone."""
+    import threading
+    latent, chunk = (16, 32, 64), (4, 4, 4)
+    S, alone, got = math.prod(latent), {}, {0.5: [], 0.03125: []}
+    q, k, v = (x.cuda() for x in seeded_qkv(73, 1, 1, S, S, 128, torch.bfloat16))
+    call = lambda rule: I().flash_attn_bsa_3d(q, k, v, latent, latent, sparsity=rule, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk)      # noqa: E731
+    for rule in got:
+        alone[rule] = call(rule)
+    torch.cuda.synchronize()
+
+    def work(rule):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            got[rule] += [call(rule) for _ in range(20)]
+            torch.cuda.current_stream().synchronize()
+    threads = [threading.Thread(target=work, args=(rule,)) for rule in got]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for rule in got:
+        assert len(got[rule]) == 20 and all(torch.equal(o, alone[rule]) for o in got[rule])
