@@ -104,10 +104,26 @@ def _workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return buf
 
 
+def _has_room(nbytes: int, device: torch.device) -> bool:
+    """Whether torch's allocator can have `nbytes` from what it holds unused and what the card has free."""
+    try:
+        free = torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+    except RuntimeError:            # an allocator without statistics
+        return True
+    return nbytes <= free
+
+
+_LARGE_SCRATCH = 1 << 30
+
+
 def _backward_workspace(nbytes: int, least: int, device: torch.device) -> torch.Tensor:
     """A backward's scratch, of which up to 8 GB are the dS it keeps between two kernels: from torch's allocator for the one
     call, which the activations may have back afterwards; without room for dS if the card has none (slower, same result but
-    for fp32 roundings)."""
+    for fp32 roundings).  A large request that the card has no room for is not made: before it raises, the allocator gives back
+    everything it holds unused, and a training run at the card's limit would pay for that in every layer's backward.  (Asking
+    costs 95 us of host time, which the kernels of a gigabyte of dS, over a millisecond, hide.)"""
+    if nbytes > least and nbytes >= _LARGE_SCRATCH and not torch.cuda.is_current_stream_capturing() and not _has_room(nbytes, device):
+        nbytes = least
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device=device)
     except torch.OutOfMemoryError:

@@ -152,3 +152,22 @@ def test_plans_are_kept_by_value():
     rule.fill_(0.75)
     assert plan().width == 8
     assert I._plan_of(1, 2, 128, 0, (16, 8, 16), (16, 8, 16), (4, 4, 4), (4, 4, 4), 0.75, None).width == 8
+
+
+@pytest.mark.parametrize("free,unused,asked", [(2 << 30, 1 << 30, [1 << 20]), (2 << 30, 5 << 30, [6 << 30]), (7 << 30, 0, [6 << 30])])
+def test_a_backward_does_not_ask_for_room_that_is_not_there(monkeypatch, free, unused, asked):
+    """A request that fails makes torch's allocator give back all it holds, at every call."""
+    made = []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda d=None: (free, 288 << 30))
+    monkeypatch.setattr(torch.cuda, "memory_reserved", lambda d=None: 20 << 30)
+    monkeypatch.setattr(torch.cuda, "memory_allocated", lambda d=None: (20 << 30) - unused)
+
+    def empty(n, **kw):
+        made.append(n)
+        if n > free + unused:
+            raise torch.OutOfMemoryError("no room")
+        return n
+    monkeypatch.setattr(torch, "empty", empty)
+    assert I._backward_workspace(6 << 30, 1 << 20, torch.device("cuda", 0)) == asked[-1]
+    assert made == asked
