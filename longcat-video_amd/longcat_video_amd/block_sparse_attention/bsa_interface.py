@@ -78,7 +78,9 @@ def _st(t: torch.Tensor) -> C.Array:
 
 
 def _rows_ok(t: torch.Tensor) -> torch.Tensor:
-    """[B,H,S,D] with a contiguous, 16-byte aligned D axis; anything else is copied."""
+    """[B,H,S,D] with a contiguous, 16-byte aligned D axis and its values in memory; anything else is copied."""
+    if t.is_neg() or t._is_zerotensor():          # a sign or zeros that only torch's own operators know of
+        return t.clone(memory_format=torch.contiguous_format)
     s = t.stride()
     ok = s[3] == 1 and (t.data_ptr() | (s[0] | s[1] | s[2]) * t.element_size()) % 16 == 0
     return t if ok else t.contiguous()

@@ -106,3 +106,16 @@ def test_threads_with_different_lds_sizes():
         t.join()
     for rule in got:
         assert len(got[rule]) == 20 and all(torch.equal(o, alone[rule]) for o in got[rule])
+
+
+def test_values_that_are_not_in_memory():
+    """A negated view and a zero tensor carry their sign, or all of their values, as a mark that the dispatcher resolves for
+    operators that do not know of it; the direct call goes by the dispatcher and has to do the same."""
+    g = torch.Generator(device="cuda").manual_seed(4)
+    grid, rule = (4, 8, 16), dict(sparsity=0.5, chunk_3d_shape_q=[4, 4, 4], chunk_3d_shape_k=[4, 4, 4])
+    q, k, v = (torch.randn(1, 2, 512, 128, generator=g, device="cuda").bfloat16() for _ in range(3))
+    want = I().flash_attn_bsa_3d(-q, k, v, grid, grid, **rule)
+    assert not torch.equal(want, I().flash_attn_bsa_3d(q, k, v, grid, grid, **rule))
+    assert torch.equal(want, I().flash_attn_bsa_3d(torch._neg_view(q), k, v, grid, grid, **rule))
+    nothing = torch._efficientzerotensor(v.shape, dtype=v.dtype, device="cuda")
+    assert torch.equal(I().flash_attn_bsa_3d(q, k, nothing, grid, grid, **rule), torch.zeros_like(v))
