@@ -209,7 +209,7 @@ int bsa_fwd_fragment(const void* q, const void* k, const void* v, const int32_t*
  * For bf16 / fp16 no permuted copy of q, k, v or o is made: one pass over q and k
  * produces the pooled means (and the tables of bsa_thw_prepare), and the attention
  * kernel reads and writes THW order directly; k and v must then share one token
- * stride (BSA_ERR_UNSUPPORTED otherwise).  fp32 goes through blocked copies.
+ * stride (BSA_ERR_UNSUPPORTED otherwise).  fp32 tensors are read and written where they lie too.
  */
 typedef struct bsa_3d_params {
     int B, Hn, D, dtype;

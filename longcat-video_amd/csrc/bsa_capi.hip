@@ -414,9 +414,6 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     const size_t kv_rows = pl->f32 ? 0 : pl->direct_kv ? (size_t)edge_count(pl->gk) * pl->gk.chunk() : (size_t)pl->Skp;
     pl->off_kp = take(bh * kv_rows * p->D * pl->es);
     pl->off_vp = take(bh * kv_rows * p->D * pl->es);
-    // Callers size their fp32 workspaces for blocked copies of the four tensors (bsa_workspace_bytes is part of the
-    // interface): the size stays, the kernels no longer need that part of it.
-    if (pl->f32) take(2 * bh * (pl->Sqp + pl->Skp) * p->D * pl->es);
     pl->off_qc = take(bh * pl->nbq * p->D * pl->es);
     pl->off_kc = take(bh * pl->nbk * p->D * pl->es);
     pl->off_score = take(bh * pl->nbq * (size_t)pl->nbk * pl->es);

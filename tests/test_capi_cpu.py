@@ -131,7 +131,8 @@ def test_fwd_3d_plan_and_workspace():
     kv = 2 * 32 * 92160 * 128 * 2
     assert need > kv and need < kv + 300 * 2 ** 20
     prm32 = _capi.Bsa3dParams(1, 32, 128, _capi.BSA_F32, 24, 45, 80, 24, 45, 80, 4, 4, 4, 4, 4, 4, 90, 0.0883883)
-    assert lib.bsa_workspace_bytes(C.byref(prm32)) > 4 * 32 * 92160 * 128 * 4     # fp32: blocked copies of all four
+    # fp32: no tensor is copied; pooled vectors, the score matrix and the lists, in fp32
+    assert 32 * 1440 * 1440 * 4 < lib.bsa_workspace_bytes(C.byref(prm32)) < 32 * 1440 * 1440 * 4 + 200 * 2 ** 20
     st = _capi.strides3([32 * 86400 * 128, 86400 * 128, 128])
     args = (FAKE, st, FAKE, st, FAKE, st, FAKE, st)
     ws = C.c_void_p(0x100000)
