@@ -246,11 +246,14 @@ def measure_c4(torch, steps, warmup, settle, where):
     return ms, ms_attn, pairs, (T, Hh, W, cond, S, n)
 
 
-def same_output(torch, out, want):
+def same_output(torch, out, want, query_tiles=None):
     """The same bits but for query tiles of the operator's last, partial round, whose walk it may cut into parts that are
-    added in fp32 afterwards: a few of their values then round the other way, by a bf16 ulp (2^-7 of the value at most)."""
+    added in fp32 afterwards: a few of their values then round the other way, by a bf16 ulp (2^-7 of the value at most).
+    `query_tiles` of all heads: where they fill whole rounds (four per compute unit) there are no parts, and no bit differs."""
     if torch.equal(out, want):
         return True
+    if query_tiles is not None and query_tiles % (4 * torch.cuda.get_device_properties(out.device).multi_processor_count) == 0:
+        return False
     d = (out.float() - want.float()).abs()
     return float((d > 0).float().mean()) < 0.02 and bool((d <= 2.0 ** -7 * want.float().abs() + 2.0 ** -10).all())
 
@@ -310,7 +313,7 @@ def measure_operator(torch, workload, steps, warmup, settle, where, coherent=Fal
     attend = I.ThwAttention(k, v, latent, latent, CHUNK, CHUNK)
     o_buf = torch.empty_like(q)
     ms_attn = time_events(torch, lambda: attend(q, idx, lens, out=o_buf), max(steps, 20), max(warmup, 5), settle_s=settle)
-    assert same_output(torch, o_buf, o), "the separately timed attention kernel must reproduce the operator's output"
+    assert same_output(torch, o_buf, o, HEADS * idx.shape[2]), "the separately timed attention kernel must reproduce the operator's output"
     if clocks is not None:
         clocks.update(sample_clocks(torch, lambda: attend(q, idx, lens, out=o_buf)))
     del attend, o_buf, o
