@@ -53,28 +53,32 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
 // rows shared by `rows_per_group` consecutive rows (one latent frame).  One wavefront per row, dim <= 8192.
 // HBM-bound if shift and scale stay on the CU: read from L2 for every row they are four times the row's own bytes (205 us
 // for 32 760 rows of 4 096, 2.6 TB/s of x and out).  A workgroup therefore holds them in LDS for kLnRows rows of a group
-// (in two planes of four, so that the lanes' 16-byte reads fall on different banks).
+// (in two planes of four, so that the lanes' 16-byte reads fall on different banks).  With a modulation row for every row
+// (kShared false) there is nothing to hold: 32 760 rows of 4 096 take 313 us from memory and 373 through LDS (from two rows
+// a group on LDS is the faster: 220 against 231).
 constexpr int kLnRows = 32;
-template <typename T, int kPieces>        // 16-byte pieces of a row per lane: dim <= 512 kPieces
+template <typename T, int kPieces, bool kShared>        // 16-byte pieces of a row per lane: dim <= 512 kPieces
 __global__ __launch_bounds__(256, kPieces <= 8 ? 4 : 2) void layernorm_modulate_kernel(const T* __restrict__ x, const float* __restrict__ shift,
                                                                  const float* __restrict__ scale, T* __restrict__ out,
-                                                                 int rows_per_group, int per_group, int dim, float eps) {
+                                                                 int64_t rows, int rows_per_group, int per_group, int dim, float eps) {
     extern __shared__ __attribute__((aligned(16))) float ln_lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int group = blockIdx.x / per_group, row0 = (blockIdx.x - group * per_group) * kLnRows;
-    const int n = min(kLnRows, rows_per_group - row0), plane = dim / 2;
+    const int64_t first = kShared ? (int64_t)group * rows_per_group + row0 : (int64_t)blockIdx.x * 4;
+    const int n = kShared ? min(kLnRows, rows_per_group - row0) : (int)min((int64_t)4, rows - first), plane = dim / 2;
     float* const sc = ln_lds;                    // scale + 1
     float* const sh = ln_lds + dim;
-    for (int d = threadIdx.x * 4; d < dim; d += 1024) {
-        const int at = (d >> 3) * 4 + ((d >> 2) & 1) * plane;
-        float4 a = *reinterpret_cast<const float4*>(scale + (int64_t)group * dim + d);
-        a.x = __fadd_rn(a.x, 1.0f); a.y = __fadd_rn(a.y, 1.0f); a.z = __fadd_rn(a.z, 1.0f); a.w = __fadd_rn(a.w, 1.0f);
-        *reinterpret_cast<float4*>(sc + at) = a;
-        *reinterpret_cast<float4*>(sh + at) = *reinterpret_cast<const float4*>(shift + (int64_t)group * dim + d);
+    auto plus_one = [](float4 a) { return make_float4(__fadd_rn(a.x, 1.0f), __fadd_rn(a.y, 1.0f), __fadd_rn(a.z, 1.0f), __fadd_rn(a.w, 1.0f)); };
+    if (kShared) {
+        for (int d = threadIdx.x * 4; d < dim; d += 1024) {
+            const int at = (d >> 3) * 4 + ((d >> 2) & 1) * plane;
+            *reinterpret_cast<float4*>(sc + at) = plus_one(*reinterpret_cast<const float4*>(scale + (int64_t)group * dim + d));
+            *reinterpret_cast<float4*>(sh + at) = *reinterpret_cast<const float4*>(shift + (int64_t)group * dim + d);
+        }
+        __syncthreads();
     }
-    __syncthreads();
     for (int r = wave; r < n; r += 4) {
-        const int64_t row = (int64_t)group * rows_per_group + row0 + r;
+        const int64_t row = first + r;
         const T* xr = x + row * dim;
         uint4 raw[kPieces];                     // the row stays in registers in its storage type
         float sum = 0.f;
@@ -113,10 +117,12 @@ __global__ __launch_bounds__(256, kPieces <= 8 ? 4 : 2) void layernorm_modulate_
         for (int j = 0; j < kPieces; ++j) {
             const int d = j * 512 + lane * 8;
             if (d < dim) {
-                const float* a = sc + (d >> 3) * 4;
-                const float* b = sh + (d >> 3) * 4;
-                const float4 s0 = *reinterpret_cast<const float4*>(a), s1 = *reinterpret_cast<const float4*>(a + plane);
-                const float4 h0 = *reinterpret_cast<const float4*>(b), h1 = *reinterpret_cast<const float4*>(b + plane);
+                const float* a = kShared ? sc + (d >> 3) * 4 : scale + row * dim + d;
+                const float* b = kShared ? sh + (d >> 3) * 4 : shift + row * dim + d;
+                const int half = kShared ? plane : 4;
+                float4 s0 = *reinterpret_cast<const float4*>(a), s1 = *reinterpret_cast<const float4*>(a + half);
+                const float4 h0 = *reinterpret_cast<const float4*>(b), h1 = *reinterpret_cast<const float4*>(b + half);
+                if (!kShared) { s0 = plus_one(s0); s1 = plus_one(s1); }
                 const float scl[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
                 const float sft[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
                 const T* e = reinterpret_cast<const T*>(&raw[j]);
@@ -349,17 +355,20 @@ int bsa_layernorm_modulate(const void* x, const float* shift, const float* scale
     if (!(eps >= 0.f)) return set_error(BSA_ERR_BAD_ARG, "layernorm_modulate: eps must be non-negative");
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(shift) | reinterpret_cast<uintptr_t>(scale) | reinterpret_cast<uintptr_t>(out)) & 15u)
         return set_error(BSA_ERR_BAD_ARG, "layernorm_modulate: pointers must be 16-byte aligned");
+    const bool shared = rows_per_group > 1;
     const int per_group = (rows_per_group + kLnRows - 1) / kLnRows;
-    const int64_t wgs = rows / rows_per_group * per_group;
+    const int64_t wgs = shared ? rows / rows_per_group * per_group : (rows + 3) / 4;
     if (wgs > 0x7fffffffLL) return set_error(BSA_ERR_UNSUPPORTED, "layernorm_modulate: too many rows");
     const dim3 grid((unsigned)wgs), block(256);
-    const size_t lds = (size_t)2 * dim * sizeof(float);            // at most 64 KB
-#define BSA_LN(T, N) hipLaunchKernelGGL((layernorm_modulate_kernel<T, N>), grid, block, lds, (hipStream_t)stream, (const T*)x, shift, scale, (T*)out, rows_per_group, per_group, dim, eps)
+    const size_t lds = shared ? (size_t)2 * dim * sizeof(float) : 0;            // at most 64 KB
+#define BSA_LN_(T, N, S) hipLaunchKernelGGL((layernorm_modulate_kernel<T, N, S>), grid, block, lds, (hipStream_t)stream, (const T*)x, shift, scale, (T*)out, rows, rows_per_group, per_group, dim, eps)
+#define BSA_LN(T, N) do { if (shared) BSA_LN_(T, N, true); else BSA_LN_(T, N, false); } while (0)
     if (dtype == BSA_BF16) {
         if (dim <= 2048) BSA_LN(__bf16, 4); else if (dim <= 4096) BSA_LN(__bf16, 8); else BSA_LN(__bf16, 16);
     } else if (dtype == BSA_F16) {
         if (dim <= 2048) BSA_LN(_Float16, 4); else if (dim <= 4096) BSA_LN(_Float16, 8); else BSA_LN(_Float16, 16);
     } else
+#undef BSA_LN_
 #undef BSA_LN
         return set_error(BSA_ERR_UNSUPPORTED, "layernorm_modulate: dtype %d is not built (bf16, fp16)", dtype);
     const hipError_t e = hipGetLastError();

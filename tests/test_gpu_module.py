@@ -466,3 +466,14 @@ def test_layernorm_modulate_sizes(dtype, frames, per, dim):
     want = (n * (scale + 1) + shift).view_as(x)
     ulp = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
     assert torch.all((got - want).abs() <= want.abs() * ulp + 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,dim", [(1, 8), (5, 2048), (6, 2056), (7, 4104)])
+def test_layernorm_modulate_with_a_row_per_token(dtype, rows, dim):
+    """A modulation row for every token is read from memory and not held in LDS: the same bits as frames of two equal rows."""
+    g = torch.Generator().manual_seed(dim)
+    x = torch.randn(2, rows, dim, generator=g).to(dtype).cuda()
+    shift, scale = (torch.randn(2, rows, 1, dim, generator=g).cuda() for _ in range(2))
+    twice = M().layernorm_modulate(x.repeat_interleave(2, 1), shift, scale)
+    assert torch.equal(M().layernorm_modulate(x, shift, scale).repeat_interleave(2, 1), twice)
