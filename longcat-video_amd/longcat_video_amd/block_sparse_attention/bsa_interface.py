@@ -79,10 +79,10 @@ def _st(t: torch.Tensor) -> C.Array:
 
 def _rows_ok(t: torch.Tensor) -> torch.Tensor:
     """[B,H,S,D] with a contiguous, 16-byte aligned D axis and its values in memory; anything else is copied."""
-    if t.is_neg() or t._is_zerotensor():          # a sign or zeros that only torch's own operators know of
+    at, s = t.data_ptr(), t.stride()
+    if at == 0 or t.is_neg():          # zeros (a zero tensor has no memory) or a sign that only torch's own operators know of
         return t.clone(memory_format=torch.contiguous_format)
-    s = t.stride()
-    ok = s[3] == 1 and (t.data_ptr() | (s[0] | s[1] | s[2]) * t.element_size()) % 16 == 0
+    ok = s[3] == 1 and (at | (s[0] | s[1] | s[2]) * t.element_size()) % 16 == 0
     return t if ok else t.contiguous()
 
 
@@ -517,7 +517,7 @@ def _kv_cache_arg(q, k, plane, kv_cache, kv_out):
 
 
 def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k, want_selection=False, out=None,
-            cdf_threshold=None, static_scratch=False, qk_norm=None, for_backward=False, kv_cache=None, kv_out=None):
+            cdf_threshold=None, static_scratch=False, qk_norm=None, for_backward=False, kv_cache=None, kv_out=None, plain=False):
     """`out`: optional [B,H,Sq,D] view (any B/H/S strides, contiguous D) to write into.  `sparsity` may be
     None when `cdf_threshold` is given (bsa_interface.py:268-277).  `static_scratch`: run through
     bsa_fwd_3d_static, which keeps its scratch memory in a buffer built into the library instead of a
@@ -527,12 +527,16 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
     bf16 / fp16 and 64-token chunks only); then `kv_cache` = (k_cache, v_cache, frames): the first frames of the keys and
     values, k and v hold the rest; `kv_out` = (k_out, v_out): receive the normalised, unrotated k and v of the frames that k
     and v hold.  `for_backward`: the same kernels through bsa_fwd_3d_lse; returns
-    (o, lists in the kernel's visiting order, lens, lse in token order) for the backward."""
+    (o, lists in the kernel's visiting order, lens, lse in token order) for the backward.  `plain`: the caller
+    knows grids, chunks and rules to be plain numbers (see _plan_of)."""
     _need_gpu(q, k, v)
     B, H, Sq, D = q.shape
     q, k, v = _rows_ok(q), _rows_ok(k), _rows_ok(v)
     lib = _capi.load()
-    plan = _plan_of(B, H, D, _code(q), latent_shape_q, latent_shape_k, chunk_q, chunk_k, sparsity, cdf_threshold)
+    if plain:
+        plan = _plan_3d(B, H, D, _code(q), *latent_shape_q, *latent_shape_k, *chunk_q, *chunk_k, sparsity, cdf_threshold)
+    else:
+        plan = _plan_of(B, H, D, _code(q), latent_shape_q, latent_shape_k, chunk_q, chunk_k, sparsity, cdf_threshold)
     prm, need, nbq, nbk, width = plan.prm, plan.need, plan.nbq, plan.nbk, plan.width
     if static_scratch and (k.stride(2) != v.stride(2) or plan.tile_tokens * k.stride(2) * k.element_size() >= 2 ** 32):
         # this route gathers k and v tiles with one set of in-tile offsets (32 bits); views that
@@ -847,7 +851,7 @@ def flash_attn_bsa_3d(
         sparsity = None if sparsity is None or sparsity < 0 else float(sparsity)
         cdf_threshold = None if cdf_threshold is None or cdf_threshold < 0 else float(cdf_threshold)
         return _bsa_3d(q, k, v, (int(Tq), int(Hq), int(Wq)), (int(Tk), int(Hk), int(Wk)), sparsity, (int(tq), int(hq), int(wq)),
-                       (int(tk), int(hk), int(wk)), cdf_threshold=cdf_threshold)
+                       (int(tk), int(hk), int(wk)), cdf_threshold=cdf_threshold, plain=True)
     return _bsa_3d_op(q, k, v, [int(x) for x in latent_shape_q], [int(x) for x in latent_shape_k],
                       -1.0 if sparsity is None else float(sparsity), -1.0 if cdf_threshold is None else float(cdf_threshold),
                       [int(x) for x in chunk_3d_shape_q], [int(x) for x in chunk_3d_shape_k])
