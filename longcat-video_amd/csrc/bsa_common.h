@@ -237,7 +237,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const Grid3* q_grid = nullptr, const int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
                            int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false, float* part_buf = nullptr);
-// fallback (optional, frag_fallback_ints(B * Hn * Sq / 64) int32): with it and key_norm the rounds run the kernel that
+// fallback (optional, frag_fallback_ints(B * Hn * Sq / 64) int32): with it and key_norm the bf16 rounds run the kernel that
 // takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.  Its first word
 // counts them: fallback_cleared says that it is zero already.
 // q_grid (optional, with q_rows): the grid whose row table (row_table_ints) q_rows is; tiles without real rows are then left out.

@@ -1,5 +1,5 @@
 // Block-sparse flash-attention forward for gfx950 (bf16 / fp16 MFMA) on K and V held in
-// "fragment order", and the pass that produces that order.
+// "fragment order".
 //
 // Why another layout.  The kernel of bsa_fwd.hip stages row-major K/V tiles in LDS, where every
 // byte is written once and read twice (two wavefronts share each 32-key half): 96 KB of LDS
@@ -29,7 +29,8 @@
 // The output accumulators (128 registers) and the rings live in the 512-register file that a
 // single wavefront per SIMD has to itself.
 //
-// Softmax: lazy running maximum as in bsa_fwd.hip (raised only when exceeded by 2^8); numerics
+// Softmax: lazy running maximum as in bsa_fwd.hip, raised only when exceeded by 2^kTau, and for
+// bf16 a form that takes no maxima where the norms bound the logits (kBounded); numerics
 // follow flash_attn_bsa_varlen_mask.py:242-285: fp32 logits, scale * log2(e) applied after the
 // dot, exp2, P rounded to the storage type for the P V product, fp32 row sum, one final rounding.
 #include "bsa_mfma.h"

@@ -6,8 +6,7 @@
 // A small call runs the three parts (workgroups 0 .. wg_k - 1 take chunks of k, the next wg_v tiles of v, the rest chunks of
 // q) in one launch instead of six: its parts take a few microseconds each, and a launch in a stream of dependent ones
 // costs 4.4.  A large call runs one launch per part: together, the part that needs most registers (q, sixteen loads in
-// flight per lane) sets the occupancy of all three, 0.65 instead of 0.56 ms for 32 heads of 720p (launch_prepare has the
-// line).
+// flight per lane) sets the occupancy of all three, 0.65 instead of 0.56 ms for 32 heads of 720p (kOneLaunchGroups).
 #include "bsa_mfma.h"
 #include "bsa_rope.h"
 
@@ -422,6 +421,10 @@ __device__ __forceinline__ void query_part(const PrepRows& x, const Grid3& g, in
     }
 }
 
+// Workgroups up to which the three parts go in one launch.  The whole operator, one launch against three, us (24x32x52, 4x4x4
+// chunks, density 0.01, by heads): rows as they are 84.6 / 89.5 at 2 808 groups, 130.0 / 136.7 at 5 616, 182.0 / 188.1 at 8 424,
+// 350.9 / 351.3 at 16 848, 681 / 670 at 33 696; with norm and rotation 152 / 163 at 7 488, 272 / 286 at 14 976, 756 / 765 at
+// 44 928.  The line stands where all of them gain.
 constexpr int64_t kOneLaunchGroups = 8192;
 
 enum { kAllParts, kKeys, kValues, kQueries };

@@ -572,11 +572,16 @@ __global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32
 // memory (the same MFMA chain as score_mfma_kernel and the same rounding, so the same bits), a wavefront selects
 // kRows / 16 of the rows from there and writes their lists in visiting order.  One launch instead of three: a launch of
 // a few microseconds' work costs 4.4 us in a stream of dependent ones.  A workgroup takes most of a CU's LDS, so a call
-// of many rows overlaps nothing and is better served by the separate kernels (gate_fits has the line).
+// of many rows overlaps nothing and is better served by the separate kernels (kGateMaxGroups).
 template <typename T> struct GateRows { static constexpr int kRows = 32; typedef uint16_t bits; };
 template <> struct GateRows<float> { static constexpr int kRows = 16; typedef uint32_t bits; };
 constexpr int kGateThreads = 1024;
 constexpr int kGateMaxBlocks = 512;
+// Row groups up to which a call gates in one launch: one per CU.  The whole operator, one launch against the separate
+// kernels, us (480 blocks, by heads): bf16, lists of 30: 97.1 / 103.8 at 30 groups, 313 / 325 at 120, 646 / 651 at 255,
+// 790 / 792 at 300, 952 / 952 at 360, 1 217 / 1 214 at 480; lists of 240, whose selection takes longer than a launch:
+// 469 / 479 at 30, 1 733 / 1 729 at 120, 3 441 / 3 419 at 240.  fp32 gains where blocks are few: 15.4 / 17.6 with 4 blocks and
+// 4 heads, 114 / 115 with 64, 386 / 386 with 128, 833 / 831 with 192; one head of 480 blocks loses 414 / 402.
 constexpr int kGateMaxGroups = 256;
 __host__ __device__ inline int gate_pitch(int nbk) { return (nbk + 31) / 32 * 32 + 8; }
 // words of LDS a wavefront selects and orders in: its histogram, later the row's list
