@@ -426,14 +426,15 @@ def test_random_shapes_against_the_oracle(seed):
     assert torch.isfinite(o.float()).all(), c
 
 
+@pytest.mark.parametrize("heads", [5, 9])
 @pytest.mark.parametrize("spread", ["wide", "narrow"])
-def test_cdf_lists_of_unequal_length_schedule(spread):
+def test_cdf_lists_of_unequal_length_schedule(spread, heads):
     """With the CDF rule the operator enqueues two schedules of the attention kernel (rounds of equal work items,
     and one launch whose workgroups draw the items longest list first) and picks one on the device from the list
     lengths.  Whatever it picks, the output must equal, bit for bit, what the kernel gives in plain rounds on the
-    same lists in the same visiting order (ThwAttention), here with more work items (640) than one round holds: 'wide' has lists from a few
-    blocks to most of them, 'narrow' lists of nearly equal length."""
-    latent, heads = (8, 32, 32), 5
+    same lists in the same visiting order (ThwAttention), here with fewer work items (5 heads, 640) than one round holds (1 024) and with
+    more (9 heads, 1 152): 'wide' has lists from a few blocks to most of them, 'narrow' lists of nearly equal length."""
+    latent = (8, 32, 32)
     S = int(np.prod(latent))
     g = torch.Generator().manual_seed(52)
     q = torch.randn(1, heads, S, 128, generator=g)
