@@ -424,9 +424,9 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->off_qrows = take(row_table_ints(pl->Sqp) * sizeof(int32_t));
     pl->off_krows = take(pl->f32 ? (size_t)pl->Skp * sizeof(int32_t) : 0);
     pl->off_ktiles = take(pl->direct_kv ? (size_t)(pl->Skp / 64) * sizeof(uint32_t) : 0);
-    // lists of unequal length (the CDF rule): work items by descending length, and the counter they are drawn with
+    // lists of unequal length (the CDF rule): the order in which work items are drawn, the counters, the choice of schedule
     pl->off_order = take(pl->cdf && !pl->f32 ? bh * (size_t)(pl->Sqp / 64) * sizeof(int32_t) : 0);
-    pl->off_queue = take(pl->cdf && !pl->f32 ? 2 * sizeof(uint32_t) : 0);    // the counter and the choice of schedule
+    pl->off_queue = take(pl->cdf && !pl->f32 ? kFragQueueWords * sizeof(uint32_t) : 0);
     pl->off_knorm = take(pl->frag ? key_norm_floats(p->B, p->Hn, pl->Skp / 64) * sizeof(float) : 0);   // key norms per head and tile
     pl->off_fallback = take(pl->frag ? frag_fallback_ints((int64_t)bh * (pl->Sqp / 64)) * sizeof(int32_t) : 0);
     // On a padded grid the attention kernel walks lists of the halves that hold keys (a list of 4 096 halves still fits its
@@ -637,7 +637,7 @@ int bsa_fwd_thw(const bsa_3d_params* p, const void* q, const int64_t q_strides[3
     if (!lens || idx_stride < 0 || (!idx && idx_stride > 0)) return set_error(BSA_ERR_BAD_ARG, "fwd_thw: selection is missing");
     hipError_t e = hipSuccess;
     // p->cdf_threshold > 0 declares lists of unequal length: work items by length, both schedules enqueued
-    if (pl.cdf && idx_stride > 0)
+    if (pl.cdf && !pl.frag && idx_stride > 0)
         e = launch_order_by_length(lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, idx_stride, (hipStream_t)stream);
     if (e == hipSuccess)
         e = attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, idx, lens, idx_stride, lse,
@@ -703,7 +703,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         const bool by_half = w.halves != nullptr;
         const int32_t *walk = by_half ? w.halves : w.idx_sorted, *walk_lens = by_half ? w.half_lens : w.lens;
         const int walk_width = by_half ? pl.half_width : pl.sel_width;
-        if (pl.cdf)
+        if (pl.cdf && !pl.frag)
             BSA_HIP(launch_order_by_length(walk_lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, walk_width, st), "order by length");
         BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, walk, walk_lens, walk_width,
                               lse_out, st, pl.cdf, pl.frag, by_half, pl.cdf ? nullptr : w.parts), "attention");

@@ -189,7 +189,7 @@ hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* len
 hipError_t launch_order_by_length(const int32_t* lens, int32_t* order, int BH, int nbq, int tiles_per_block, int max_len,
                                   hipStream_t st);
 
-// queue[0] = 0 (the counter work items are drawn with) and queue[1] = the choice between rounds (0) and the
+// For launch_fwd: queue[0] = 0 (the counter work items are drawn with) and queue[1] = the choice between rounds (0) and the
 // longest-first queue (1), made on the device from the list lengths (see choose_schedule_kernel)
 void launch_schedule_choice(const int32_t* lens, int nbq, int tiles_per_block, int total, int round, int resident,
                             int max_len, uint32_t* queue, hipStream_t st);
@@ -235,8 +235,11 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk,
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
-                           const Grid3* q_grid = nullptr, const int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
+                           const Grid3* q_grid = nullptr, int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
                            int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false, float* part_buf = nullptr);
+// order (B * Hn * Sq / 64 int32) and queue (kFragQueueWords), both or none: scratch for the schedule of lists of unequal length,
+// enqueued besides the rounds; which of the two runs is decided on the device.
+constexpr int kFragQueueWords = 16;
 // fallback (optional, frag_fallback_ints(B * Hn * Sq / 64) int32): with it and key_norm the bf16 rounds run the kernel that
 // takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.  Its first word
 // counts them: fallback_cleared says that it is zero already.

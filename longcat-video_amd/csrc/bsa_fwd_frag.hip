@@ -101,7 +101,7 @@ constexpr int kPipeList = 256;
 // probabilities would all be 0 changes no bit of the result: the sums run over the same numbers in the same order.
 //
 // A workgroup (one wavefront) runs the work items b, b + round, b + 2 round, ... of its launch one after the other
-// (or draws them from `queue`).  What an item needs before its first MFMA - its list, its Q rows, its first K and
+// (or draws them from its XCD's queue).  What an item needs before its first MFMA - its list, its Q rows, its first K and
 // V fragments - is requested while the item before it still runs, so that an item costs its tile walk and an
 // epilogue, not a chain of three dependent memory round trips:
 //   * lens and the first list entry of the item after next are scalar loads issued at the start of an item;
@@ -128,6 +128,12 @@ struct Parts {
     float* buf;
     int count, items;
 };
+
+// The schedule for lists of unequal length: a queue per XCD.  Section x holds the items [section_begin(x), section_begin(x + 1))
+// of the call, a contiguous run of query tiles, and workgroup b draws from section b % 8, the XCD it runs on.
+constexpr int kQueues = 8, kQueueChoice = kQueues, kQueueWords = kQueues + 1;      // a counter per section, the choice of schedule
+static_assert(kQueueWords <= kFragQueueWords, "the caller's buffer holds the words");
+__device__ __forceinline__ int section_begin(int n, int x) { return (int)(((int64_t)n * x) >> 3); }
 
 template <typename T, int kWalk, bool kBounded>
 __global__ __launch_bounds__(64) void fwd_frag_kernel(
@@ -201,11 +207,18 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         if (w >= n) return -1;
         return (int)r0 + x * (n >> 3) + min(x, n & 7) + (w >> 3);
     };
+    // From the queues (queue_plan_kernel): the section of this workgroup's XCD first, then what the others have left.
+    int section_turn = 0;
     auto draw = [&]() -> int {
-        uint32_t drawn = 0;
-        if (lane == 0) drawn = atomicAdd(queue, 1u);
-        const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)drawn);
-        return l < (uint32_t)n_launch ? (int)l : -1;
+        for (; section_turn < kQueues; ++section_turn) {
+            const int x = (blockIdx.x + section_turn) & (kQueues - 1);
+            const int begin = section_begin(n_launch, x), n = section_begin(n_launch, x + 1) - begin;
+            uint32_t drawn = 0;
+            if (lane == 0) drawn = atomicAdd(queue + x, 1u);
+            const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)drawn);
+            if (l < (uint32_t)n) return begin + (int)l;
+        }
+        return -1;
     };
     int rounds_taken = 0;
     auto next_local = [&]() -> int { return queue != nullptr ? draw() : round_local(rounds_taken++); };
@@ -890,6 +903,107 @@ __global__ __launch_bounds__(256) void merge_parts_kernel(Parts parts, T* __rest
 
 }  // namespace
 
+// The price of a tile walked out of step, by which the queues' estimate is weighed against the rounds'.  Attention of 16 heads of
+// 20x30x52 by the CDF threshold, queues / rounds, whole operator in us: smooth inputs 0.25 (lists of 32 to 49 blocks) 815 / 775,
+// 0.5 (32 to 157) 1 200 / 1 485, 0.75 (54 to 313) 2 497 / 3 267, 32 heads of 24x45x80 at 0.5 (90 to 635) 8 592 / 10 396; random
+// inputs (lists of one length, give or take three) 0.5 3 800 / 3 928, where rounds leave seven of eight wavefronts idle in
+// the last; equal lists of 32 heads over whole rounds 1 840 / 1 848 smooth, 2 450 / 1 870 and 9 900 / 8 325 random.
+constexpr double kQueuePrice = 1.4;
+// Classes an octave of list length: 0 (query order alone) 1 441 us for the 0.5 case, 1 1 200, 2 1 229, 4 1 250; one counter over
+// every head's tiles by exact length 1 834.
+constexpr float kClassesPerOctave = 1.0f;
+
+// The plan of the queue schedule, one launch.  Workgroup x < kQueues writes section x of `order`: its items in classes of
+// similar list length, longest class first (so that the last items drawn are short), and within a class in the order of
+// the query tiles.  Neighbouring tiles of a layer whose queries vary smoothly select largely the same blocks; drawn one after
+// another by the workgroups of one XCD, with lists of about one length and so at about one pace, they find each other's
+// tiles in its L2.  The last workgroup clears the counters and chooses between rounds and queues: a round lasts as long as
+// its longest list, the queues keep every workgroup busy but walk out of step.
+constexpr int kPlanThreads = 1024, kPlanClasses = 12, kPlanRounds = 8192;
+__global__ __launch_bounds__(kPlanThreads) void queue_plan_kernel(const int32_t* __restrict__ lens, int tiles_per_block, int nqt, FragLayout L,
+                                                                  int total, int resident, int max_len, int32_t* __restrict__ order,
+                                                                  uint32_t* __restrict__ queue) {
+    __shared__ int sm[kPlanClasses * kPlanThreads];
+    __shared__ int wave_sum[kPlanThreads / 64];
+    __shared__ int longest_sm;
+    __shared__ unsigned long long sum_sm;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    auto length_of = [&](int item) { return min(max(lens[item / tiles_per_block], 0), max_len); };
+    auto wave_max = [](int x) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) x = max(x, __shfl_xor(x, off));
+        return x;
+    };
+    if (tid == 0) { longest_sm = 0; sum_sm = 0ull; }
+    if (blockIdx.x == kQueues) {
+        const int rounds = (total + resident - 1) / resident;
+        if (tid < kQueues) queue[tid] = 0u;
+        if (rounds > kPlanRounds) { if (tid == 0) queue[kQueueChoice] = 0u; return; }
+        for (int r = tid; r < rounds; r += kPlanThreads) sm[r] = 0;
+        __syncthreads();
+        unsigned long long sum = 0ull;
+        int longest = 0;
+        for (int u0 = 64 * wave; u0 < total; u0 += kPlanThreads) {          // 64 consecutive items, mostly of one round
+            const int u = min(u0 + lane, total - 1), l = length_of(item_at(L, u, nqt));
+            sum += u0 + lane < total ? (unsigned long long)l : 0ull;
+            longest = max(longest, l);
+            const int most = wave_max(l), r = u0 / resident;
+            if (r == min(u0 + 63, total - 1) / resident) { if (lane == 0) atomicMax(&sm[r], most); }
+            else atomicMax(&sm[u / resident], l);
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+        longest = wave_max(longest);
+        if (lane == 0) {
+            atomicAdd(&sum_sm, sum);
+            atomicMax(&longest_sm, longest);
+        }
+        __syncthreads();
+        if (tid == 0) {
+            unsigned long long rounds_cost = 0ull;
+            for (int r = 0; r < rounds; ++r) rounds_cost += (unsigned long long)sm[r];
+            const double queue_cost = kQueuePrice * (double)sum_sm / (double)resident + (double)longest_sm;
+            queue[kQueueChoice] = queue_cost < (double)rounds_cost ? 1u : 0u;
+        }
+        return;
+    }
+    const int begin = section_begin(total, blockIdx.x), end = section_begin(total, blockIdx.x + 1);
+    const int per = (end - begin + kPlanThreads - 1) / kPlanThreads;
+    const int first = min(begin + tid * per, end), last = min(first + per, end);      // this thread's items
+    for (int c = 0; c < kPlanClasses; ++c) sm[c * kPlanThreads + tid] = 0;
+    __syncthreads();
+    int longest = 0;
+    for (int u = first; u < last; ++u) longest = max(longest, length_of(item_at(L, u, nqt)));
+    longest = wave_max(longest);
+    if (lane == 0) atomicMax(&longest_sm, longest);
+    __syncthreads();
+    const float top = __builtin_log2f((float)max(longest_sm, 1));
+    auto class_of = [&](int l) { return l <= 0 ? kPlanClasses - 1 : min((int)(kClassesPerOctave * (top - __builtin_log2f((float)l)) + 0.001f), kPlanClasses - 1); };
+    for (int u = first; u < last; ++u) ++sm[class_of(length_of(item_at(L, u, nqt))) * kPlanThreads + tid];
+    __syncthreads();
+    // exclusive sums over (class, thread): twelve consecutive entries per thread, the threads' totals over the workgroup
+    int own[kPlanClasses], run = 0;
+#pragma unroll
+    for (int c = 0; c < kPlanClasses; ++c) { own[c] = sm[tid * kPlanClasses + c]; run += own[c]; }
+    int before = run;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int x = __shfl_up(before, off);
+        if (lane >= off) before += x;
+    }
+    if (lane == 63) wave_sum[wave] = before;
+    __syncthreads();
+    before -= run;
+    for (int w = 0; w < wave; ++w) before += wave_sum[w];
+#pragma unroll
+    for (int c = 0; c < kPlanClasses; ++c) { sm[tid * kPlanClasses + c] = before; before += own[c]; }
+    __syncthreads();
+    for (int u = first; u < last; ++u) {
+        const int item = item_at(L, u, nqt);
+        order[begin + sm[class_of(length_of(item)) * kPlanThreads + tid]++] = item;
+    }
+}
+
 // Rounds per launch: five (four to six measure the same at 90 tiles per list and 1.5 % better than two, now that an
 // item that was prepared by the one before it starts 7 us sooner than a launch's first; from eight on the items drift
 // apart and the L2 hit rate falls); eight for short lists (six to ten measure the same, twenty lose 3 %).
@@ -915,7 +1029,7 @@ static int resident_wavefronts() {
 // kf / vf: fragment-order K and V, [B * Hn][Sk / 64][16 KB].  q, o in blocked order (q_rows null) or in
 // (T, H, W) order through the row table.  Scheduling: rounds of as many work items as the device runs at once,
 // across (batch, head) boundaries, kRoundsPerLaunch rounds per launch, every workgroup running one item of each round;
-// with `order` and `queue` also the schedule that draws items longest list first, the choice between the two being
+// with `order` and `queue` also the schedule that draws items from the XCDs' queues, the choice between the two being
 // made on the device.
 __global__ void frag_zero_kernel(uint32_t* p, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -954,7 +1068,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk,
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
-                           const Grid3* q_grid, const int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
+                           const Grid3* q_grid, int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
                            bool halves, float* part_buf) {
     // the C-ABI layer keeps lists within these limits (a list that is too long for the small buffers is staged in `ost`)
     if (idx_stride > (halves ? kHalfEntries : kListEntries)) return hipErrorInvalidValue;
@@ -1012,11 +1126,12 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     } while (0)
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
     if (queue != nullptr && one_span) {
-        launch_schedule_choice(lens, (int)(Sq / bs_q), bs_q / kTile, all_tiles, resident, resident, idx_stride, queue, st);
-        gate = queue + 1;
-        const dim3 grid((unsigned)(all_tiles < resident ? all_tiles : resident));
-        if (bounded) BSA_FRAG_LAUNCH(true, grid, 0, all_tiles, order, queue, 1u, 0, whole_span, fb_list, fb_count);
-        else BSA_FRAG_LAUNCH(false, grid, 0, all_tiles, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
+        hipLaunchKernelGGL(queue_plan_kernel, dim3(kQueues + 1), dim3(kPlanThreads), 0, st, lens, bs_q / kTile, per_head, L, total, resident, idx_stride,
+                           order, queue);
+        gate = queue + kQueueChoice;
+        const dim3 grid((unsigned)(total < resident ? total : resident));
+        if (bounded) BSA_FRAG_LAUNCH(true, grid, 0, total, order, queue, 1u, 0, whole_span, fb_list, fb_count);
+        else BSA_FRAG_LAUNCH(false, grid, 0, total, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
     }
     // kRoundsPerLaunch rounds per launch, every workgroup running one item of each: the items of a round start
     // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
@@ -1053,7 +1168,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         parts = {nullptr, 1, 0};
     }
     if (bounded) {
-        // what the schedule that ran left over, be it the rounds or the longest-first queue: as many items as the list holds,
+        // what the schedule that ran left over, be it the rounds or the queues: as many items as the list holds,
         // found out on the device.  Not behind the gate of either: only the one that ran has put items on the list.
         gate = nullptr;
         const dim3 grid((unsigned)(all_tiles < resident ? all_tiles : resident));

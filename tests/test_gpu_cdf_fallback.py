@@ -78,3 +78,36 @@ def test_an_infinite_key_reaches_the_output(dtype):
     bi()._bsa_3d(q, k, v, LATENT, LATENT, None, CHUNK, CHUNK, out=out, cdf_threshold=0.5)
     assert torch.equal(out.nan_to_num(nan=5.0), rounds.nan_to_num(nan=5.0))
     assert not torch.isfinite(out[0, 4]).all() and torch.isfinite(out[0, 3]).all()
+
+
+@pytest.mark.parametrize("latent,heads,chunk,dtype", [
+    ((13, 30, 53), 9, (4, 4, 8), torch.bfloat16),      # 3 339 of 4 032 query tiles hold rows: sections of 417 and 418 of them
+    ((13, 30, 53), 9, (4, 4, 8), torch.float16),
+    ((8, 33, 32), 15, (4, 4, 4), torch.bfloat16),      # 2 160 tiles: more items than the device runs at once, twice over
+])
+def test_queues_cover_ragged_grids(latent, heads, chunk, dtype):
+    """Every row is computed once, whichever XCD's queue it is drawn from, on grids whose query tiles drop out or hold few rows.
+    Bit for bit the rounds on the same lists."""
+    T, H, W = latent
+    S = T * H * W
+    g = torch.Generator().manual_seed(93)
+    q, k, v = (torch.randn(1, heads, S, 128, generator=g) for _ in range(3))
+    pos = torch.arange(S)
+    nh, nw = -(-H // chunk[1]), -(-W // chunk[2])
+    block = ((pos // (H * W)) // chunk[0]) * nh * nw + (((pos // W) % H) // chunk[1]) * nw + (pos % W) // chunk[2]
+    peaked = block % 10 != 0
+    direction = torch.randn(1, heads, int(block.max()) + 1, 128, generator=g)[:, :, block]
+    for x in (q, k):
+        x[:, :, peaked] = 3 * direction[:, :, peaked] + 0.1 * x[:, :, peaked]
+    q, k, v = (x.to(dtype).cuda() for x in (q, k, v))
+    _, idx, lens, _ = bi()._bsa_3d(q, k, v, latent, latent, None, chunk, chunk, True, cdf_threshold=0.5)
+    # what the choice on the device takes the queues for: long lists in every round of 1 024 items, and few of them
+    tiles = -(-heads * lens.shape[-1] * chunk[2] // 4 // 1024)
+    assert 1.4 * float(lens.float().sum()) * (chunk[2] // 4) / 1024 + int(lens.max()) < 0.9 * tiles * int(lens.max())
+    nbk = int(block.max()) + 1
+    asc = torch.where(idx < 0, torch.full_like(idx, 1 << 20), idx).sort(dim=-1).values
+    walk = bi().visit_order(torch.where(asc == 1 << 20, torch.zeros_like(asc), asc).int(), lens, nbk)
+    rounds = bi().ThwAttention(k, v, latent, latent, chunk, chunk)(q, walk, lens)
+    out = torch.full_like(q, float("nan"))
+    bi()._bsa_3d(q, k, v, latent, latent, None, chunk, chunk, out=out, cdf_threshold=0.5)
+    assert torch.equal(out, rounds)
