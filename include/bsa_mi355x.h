@@ -442,6 +442,14 @@ int bsa_linear_bf16_tune(const void* x, int64_t ldx, const void* w, int64_t ldw,
 int bsa_lora_add(const void* org, const void* const* up, const float* multiplier, const float* alpha_scale, int n_loras,
                  void* out, int64_t n, int dtype, void* stream);
 
+/* One side branch from its down projection on, bf16: the up-projection and the sum of bsa_lora_add in one pass over org.
+ * t: [M, n_sep * rank] with rows ldt elements apart (lora_down(x)); up: a HOST array of n_sep device pointers to
+ * [N / n_sep, rank] weights, slice i taking the rank columns i * rank .. of t; out [M, N], may alias org.  The product is
+ * accumulated in fp32 and rounded once, then scaled and added as bsa_lora_add does.  Built for a rank that is a multiple of 16
+ * up to 128 and at most 8 slices of a multiple of 64 columns (BSA_ERR_UNSUPPORTED otherwise). */
+int bsa_lora_up_add(const void* org, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank, float multiplier,
+                    float alpha_scale, void* out, int64_t M, int N, void* stream);
+
 /* bsa_fwd_3d for the attention module (attention.py:116-137): q and k arrive as the QKV projection left them
  * (strided views into its output are fine) and go through the per-head RMSNorm (RMSNorm_FP32, blocks.py:42-53) and
  * the 3-D RoPE (rope_3d.py:100-120) inside the operator's own passes over them, at the rounding points of

@@ -3,8 +3,10 @@
 The reference patches the forward of every Linear a LoRA file names (longcat_video_dit.py:211-249):
 ``org_forward(x) + sum_i lora_up_i(lora_down_i(x)) * multiplier_i * alpha_scale_i``.  ``lora_up`` is either one
 Linear or, for fused projections such as qkv, one Linear per equal slice of the output features, each fed its own
-slice of the rank axis (lora_utils.py:12-21, 47-53).  Here the three GEMMs go to hipBLASLt through the C ABI (the
-sliced up-projection with row strides, in place) and one elementwise pass applies the scaling and the sums with the
+slice of the rank axis (lora_utils.py:12-21, 47-53).  Here the layer and the down projection go to hipBLASLt through the
+C ABI; the up-projection of a single branch, its scaling and the sum are one pass over the layer's output
+(bsa_lora_up_add).  Several branches, whose scaled terms are summed before the layer's output is added, take their
+up-projections from hipBLASLt too (the sliced one with row strides, in place) and one elementwise pass.  Both with the
 eager expression's roundings.
 """
 from typing import List, Optional, Sequence
@@ -64,6 +66,13 @@ def _up_projection(lx: torch.Tensor, branch: LoRABranch, workspace: torch.Tensor
     return out
 
 
+def _one_pass(b: LoRABranch) -> bool:
+    """What bsa_lora_up_add is built for; other branches, and sums over several, take the up-projection as a tensor."""
+    per = b.lora_up[0].shape[0]
+    return (b.rank % 16 == 0 and b.rank <= 128 and len(b.lora_up) <= 8 and per % 64 == 0
+            and all(u.dtype == torch.bfloat16 and (not u.is_contiguous() or u.data_ptr() % 16 == 0) for u in b.lora_up))
+
+
 @torch.no_grad()
 def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                 loras: Optional[List[LoRABranch]] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -78,19 +87,27 @@ def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
         workspace = _gemm_workspace(x.device)
     N = weight.shape[0]
     x2 = x.reshape(-1, x.shape[-1])
+    import ctypes as C
+    # alpha_scale lives in a bf16 buffer in the reference
+    alphas = [float(torch.tensor(b.alpha_scale, dtype=torch.bfloat16)) for b in active]
     ups = []
-    for b in active:
+    for b, a in zip(active, alphas):
         assert b.out_features == N and b.lora_down.shape[1] == x.shape[-1]
         if b.lora_down.dtype != torch.bfloat16:
             raise NotImplementedError("LoRA weights must be bf16 (the reference moves them to the model dtype)")
         lx = linear_bf16(x2, b.lora_down, None, workspace=workspace)              # [M, n_sep * rank]
+        if len(active) == 1 and _one_pass(b):
+            w = [u.contiguous() for u in b.lora_up]
+            ptrs = (C.c_void_p * len(w))(*[u.data_ptr() for u in w])
+            with _on_device(x):
+                _capi.check(_capi.load().bsa_lora_up_add(_ptr(org), _ptr(lx), lx.shape[1], ptrs, len(w), b.rank, float(b.multiplier), a,
+                                                         _ptr(org), lx.shape[0], N, _stream(x)), "lora_up_add")
+            return org
         ups.append(_up_projection(lx, b, workspace))
-    import ctypes as C
     n = len(ups)
     up_ptrs = (C.c_void_p * n)(*[u.data_ptr() for u in ups])
     mult = (C.c_float * n)(*[float(b.multiplier) for b in active])
-    # alpha_scale lives in a bf16 buffer in the reference
-    alpha = (C.c_float * n)(*[float(torch.tensor(b.alpha_scale, dtype=torch.bfloat16)) for b in active])
+    alpha = (C.c_float * n)(*alphas)
     out2 = org.view(-1, N)
     with _on_device(x):
         _capi.check(_capi.load().bsa_lora_add(_ptr(out2), up_ptrs, mult, alpha, n, _ptr(out2), out2.numel(),

@@ -349,6 +349,27 @@ def test_lora_linear_random_inputs():
     assert (want - plain).abs().mean() > 10 * (got - want).abs().mean()      # the side branch is not lost in the tolerance
 
 
+@pytest.mark.parametrize("M,r,n_sep,per", [
+    (1, 16, 1, 64), (31, 48, 1, 192), (33, 128, 3, 128), (65, 64, 8, 64),       # edges of the 32 tokens of a turn and the 256 columns
+    (700, 112, 1, 320), (40, 96, 5, 64),
+    (24700, 32, 1, 64),                                                        # more turns than workgroups
+    (50, 24, 1, 64), (50, 16, 2, 96), (50, 144, 1, 64),                        # not built in one pass: rank, slice, rank
+])
+def test_lora_up_projection_and_sum(M, r, n_sep, per):
+    """Small integers are exact in every product and sum: the one-pass kernel, and the separate passes where it is not built,
+    give the oracle's bits, whole tokens and columns included.  An up weight that is a transposed view is read as it is."""
+    g = torch.Generator().manual_seed(M + r)
+    K, N = 64, n_sep * per
+    x, w = (torch.randint(-2, 3, s, generator=g).bfloat16() for s in ((M, K), (N, K)))
+    br, term = _branch(g, K, N, r, n_sep, 0.5, r / 2, integers=True)
+    br.lora_down.mul_(0.25)                                                    # products of up to 2^12 quarters: 16 bits at most
+    want = O.lora_linear(x, w, None, [term])
+    br.to("cuda")
+    assert torch.equal(L().lora_linear(x.cuda(), w.cuda(), None, [br]).cpu(), want)
+    br.lora_up = [u.t().contiguous().t() for u in br.lora_up]
+    assert torch.equal(L().lora_linear(x.cuda(), w.cuda(), None, [br]).cpu(), want)
+
+
 def test_module_forward_with_lora_branches():
     """longcat_video_dit.py:211-249: LoRA branches on attn.qkv (up-projection split in three) and attn.proj."""
     shape = (4, 8, 8)
