@@ -201,6 +201,7 @@ struct PrepRows {
     const uint16_t* cached;          // k, v, optional: the tokens before `split` come from here, already normalised, and p holds the rest
     int64_t cB, cH, cS;
     int split;
+    int heads;                       // set by launch_prepare: heads of a chunk that a workgroup takes
     char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, the real slots of a tile first, zeros behind
     uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
     int32_t* rows;                   // q: row_table_ints() entries; the real slots of a chunk come first

@@ -41,6 +41,9 @@ __device__ __forceinline__ void add_row(float (&acc)[8], const uint4& x) {
     }
 }
 
+// what is derived from x is not worked out ahead of this place
+__device__ __forceinline__ void opaque(uint4& x) { asm volatile("" : "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w)); }
+
 // key_norm[batch * heads + head] = the largest entry of the head's tile norms
 __global__ __launch_bounds__(256) void head_norm_kernel(const float* __restrict__ tile_norm, float* __restrict__ key_norm, int tiles) {
     __shared__ float part[4];
@@ -115,11 +118,12 @@ __device__ __forceinline__ const uint16_t* row_at(const uint16_t* src, int64_t s
 // workgroup -> (tile or chunk, batch * head).  For a token-major source (the heads of a token next to each other, as a QKV
 // projection leaves them) the heads of one chunk run side by side, so that the 256-byte rows they fetch share DRAM pages
 // and cache lines' neighbourhoods; otherwise the chunks of one head do.
-__device__ __forceinline__ void place(int id, int per_head, int Hn, int head_fastest, int& chunk, int& bh) {
+// `heads`: heads of a batch, or groups of them.
+__device__ __forceinline__ void place(int id, int per_head, int heads, int head_fastest, int& chunk, int& bh) {
     if (head_fastest) {
-        const int per_batch = per_head * Hn, b = id / per_batch, rest = id - b * per_batch;
-        chunk = rest / Hn;
-        bh = b * Hn + (rest - chunk * Hn);
+        const int per_batch = per_head * heads, b = id / per_batch, rest = id - b * per_batch;
+        chunk = rest / heads;
+        bh = b * heads + (rest - chunk * heads);
     } else {
         bh = id / per_head;
         chunk = id - bh * per_head;
@@ -132,7 +136,7 @@ constexpr int kPitchV = kD + 16;     // 288-byte rows: the transposing reads fet
 // kMode: rows as they are; with norm and rotation; and with a cache in front of k and v, or their rows written out.
 enum { kPlain, kNorm, kCached };
 
-// k (or q, when it has a row transform): a workgroup per chunk, tile by tile.  The chunk mean keeps permute_kernel's order
+// k (or q, when it has a row transform): a workgroup per chunk of x.heads heads, tile by tile.  The chunk mean keeps permute_kernel's order
 // of summation - a thread adds its rows rg, rg + 16, ... of the chunk, then the 16 partial sums of a column are added in
 // ascending rg, one rounding at the end - so every route gives the same bits.
 template <bool kBf16, int kMode, bool kIsK>
@@ -141,12 +145,35 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
     constexpr bool kTransform = kMode != kPlain, kCache = kMode == kCached;
     typedef typename std::conditional<kBf16, __bf16, _Float16>::type T;
     const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
-    int blk, bh;
-    place(id, g.blocks(), Hn, x.head_fastest, blk, bh);
+    const int units = (Hn + x.heads - 1) / x.heads;               // groups of heads of a batch
+    int blk, unit;
+    place(id, g.blocks(), units, x.head_fastest, blk, unit);
+    const int batch = unit / units, head0 = (unit - batch * units) * x.heads, heads = min(x.heads, Hn - head0);
     const int lane = threadIdx.x & 63;
     const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;      // 16 pieces of 16 B per row, 16 rows at a time
-    const uint16_t* src = x.p + (int64_t)(bh / Hn) * x.sB + (int64_t)(bh % Hn) * x.sH + c16 * 8;
-    const uint16_t* old = kCache && x.cached != nullptr ? x.cached + (int64_t)(bh / Hn) * x.cB + (int64_t)(bh % Hn) * x.cH + c16 * 8 : nullptr;
+    const uint16_t* src = x.p + (int64_t)batch * x.sB + (int64_t)head0 * x.sH + c16 * 8;
+    const uint16_t* old = kCache && x.cached != nullptr ? x.cached + (int64_t)batch * x.cB + (int64_t)head0 * x.cH + c16 * 8 : nullptr;
+    // The rows of the first tile are asked for before anything else, those of a later one as soon as the tile before it is in
+    // LDS: the loads of a tile are under way while the workgroup writes out, meets and stages.
+    Slots s;
+    uint4 xs[4];
+    int token[4], loc[4];
+    auto locate = [&](int sub) {
+        s = slots_of(g, blk, sub, lane);
+        if (x.valid_in != nullptr) s.word = x.valid_in[blk * per_chunk + sub];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            token[i] = __shfl(s.token, rg + 16 * i);
+            if (kTransform) loc[i] = __shfl(s.loc, rg + 16 * i);
+        }
+    };
+    auto load = [&]() {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            xs[i] = *reinterpret_cast<const uint4*>(kCache ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
+    };
+    locate(0);
+    load();
     // Rotation: a chunk spans at most 8 positions per axis, and a rotation pair turns with one axis only, so the
     // (cos, sin) the rows of the chunk need are 8 x 64 table entries, fetched once per workgroup instead of per row and head.
     int turn[4];                          // where the position that turns this lane's pair jj stands in Slots::loc
@@ -174,23 +201,19 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         }
         __syncthreads();
     }
+    for (int hi = 0; hi < heads; ++hi) {
+    const int head = head0 + hi, bh = batch * Hn + head;
     float acc[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = 0.f;
     int rows_before = 0;
     for (int sub = 0; sub < per_chunk; ++sub) {
         const int tile_id = blk * per_chunk + sub;
-        Slots s = slots_of(g, blk, sub, lane);
-        if (x.valid_in != nullptr) s.word = x.valid_in[tile_id];
-        uint4 xs[4];
-        int token[4], loc[4];
-        // all four loads first, then the arithmetic: a row transformed right behind its own load would wait for it
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            token[i] = __shfl(s.token, rg + 16 * i);
-            if (kTransform) loc[i] = __shfl(s.loc, rg + 16 * i);
-            xs[i] = *reinterpret_cast<const uint4*>(kCache ? row_at(src, x.sS, old, x.cS, x.split, max(token[i], 0)) : src + (int64_t)max(token[i], 0) * x.sS);
-        }
+        // What follows from the thread's number is worked out in every turn: kept over all of them, the LDS addresses and bit
+        // positions of four rows would cost a wavefront a SIMD.
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int rg = tid >> 4, c16 = tid & 15;
         if (s.word != ~0ull) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) keep_if(xs[i], (s.word >> (rg + 16 * i)) & 1ull);
@@ -204,10 +227,11 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         }
         if (kTransform) {
             const uint4 wraw = *reinterpret_cast<const uint4*>(x.norm_w + c16 * 8);
-            uint16_t* rows = x.rows_out == nullptr ? nullptr : x.rows_out + (int64_t)(bh / Hn) * x.rB + (int64_t)(bh % Hn) * x.rH + c16 * 8;
+            uint16_t* rows = x.rows_out == nullptr ? nullptr : x.rows_out + (int64_t)batch * x.rB + (int64_t)head * x.rH + c16 * 8;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (token[i] < 0) continue;                         // the 16 lanes of a row go together
+                opaque(xs[i]);
                 float c[4], sn[4];
 #pragma unroll
                 for (int jj = 0; jj < 4; ++jj) {
@@ -226,27 +250,28 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
                     }
                     xs[i] = norm_rope_piece<T>(xs[i], wraw, false, true, c, sn, eps);
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (x.pooled != nullptr) {
+        // Of k also the largest Euclidean norm of a row of this tile as it is stored (after the transform), a little above the
+        // exact value: the attention kernel bounds q . k by |q| |k| with the largest of a head.  The sixteen lanes of
+        // a row add their squares (butterfly over the row's lanes with DPP moves), then the maximum over the rows.
+        // Piece by piece: widened all at once, the 32 values of a lane's rows cost a wavefront a SIMD.
+        float best = 0.f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) add_row<kBf16>(acc, xs[i]);
-        }
-        if (x.tile_norm != nullptr) {
-            // the largest Euclidean norm of a row of this tile as it is stored (after the transform), a little above the
-            // exact value: the attention kernel bounds q . k by |q| |k| with the largest of a head.  The sixteen lanes of
-            // a row add their squares (butterfly over the row's lanes with DPP moves), then the maximum over the rows.
-            float best = 0.f;
+        for (int i = 0; i < 4; ++i) {
+            opaque(xs[i]);
+            const uint32_t w[4] = {xs[i].x, xs[i].y, xs[i].z, xs[i].w};
+            float sq = 0.f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t w[4] = {xs[i].x, xs[i].y, xs[i].z, xs[i].w};
-                float sq = 0.f;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float lo, hi;
-                    widen<kBf16>(w[e], lo, hi);
-                    sq = fmaf(lo, lo, fmaf(hi, hi, sq));
-                }
+            for (int e = 0; e < 4; ++e) {
+                float lo, hi;
+                widen<kBf16>(w[e], lo, hi);
+                acc[2 * e] += lo;
+                acc[2 * e + 1] += hi;
+                if (kIsK) sq = fmaf(lo, lo, fmaf(hi, hi, sq));
+            }
+            if (kIsK) {
                 sq += dpp_f32<0xB1>(sq);         // quad_perm [1, 0, 3, 2]
                 sq += dpp_f32<0x4E>(sq);         // quad_perm [2, 3, 0, 1]
                 sq += dpp_f32<0x141>(sq);        // row_half_mirror
@@ -254,6 +279,11 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
                 best = fmaxf(best, sq);          // NaN squares drop out here; such a row has no bound (below)
                 if (sq != sq) best = INFINITY;
             }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(acc[e]));      // added here, not where the sums are used
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (kIsK && x.tile_norm != nullptr) {
 #pragma unroll
             for (int off = 32; off >= 16; off >>= 1) best = fmaxf(best, __shfl_xor(best, off));
             __shared__ float wave_best[4];
@@ -271,11 +301,21 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
                 *reinterpret_cast<uint2*>(row) = make_uint2(xs[i].x, xs[i].y);
                 *reinterpret_cast<uint2*>(row + 4) = make_uint2(xs[i].z, xs[i].w);
             }
+        }
+        if (sub + 1 < per_chunk || hi + 1 < heads) {
+            if (sub + 1 == per_chunk) {
+                src += x.sH;
+                if (kCache && old != nullptr) old += x.cH;
+            }
+            if (per_chunk > 1) locate(sub + 1 < per_chunk ? sub + 1 : 0);
+            load();
+        }
+        if (x.frag != nullptr) {
             __syncthreads();
             char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int e = threadIdx.x + 256 * i;                       // 16-byte piece of the output, 0..1023
+                const int e = tid + 256 * i;                               // 16-byte piece of the output, 0..1023
                 const int l = e & 63, f = e >> 6;                          // lane and fragment: key half f / 8, d chunk f % 8
                 const uint16_t* p = tile + (32 * (f >> 3) + (l & 31)) * kPitchK + 16 * (f & 7) + 8 * (l >> 5);
                 const uint2 lo = *reinterpret_cast<const uint2*>(p), hi = *reinterpret_cast<const uint2*>(p + 4);
@@ -294,7 +334,9 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
             for (int i = 0; i < 16; ++i) sum += red[i * kD + threadIdx.x];
             x.pooled[((int64_t)bh * g.blocks() + blk) * kD + threadIdx.x] = narrow<kBf16>(sum * (1.0f / g.chunk()));
         }
+        __syncthreads();                          // the next head may have the memory
     }
+    }   // heads
 }
 
 // v: a workgroup per tile, gathered into LDS and read transposed: a piece holds 8 keys of one d
@@ -427,9 +469,17 @@ __device__ __forceinline__ void query_part(const PrepRows& x, const Grid3& g, in
 // 44 928.  The line stands where all of them gain.
 constexpr int64_t kOneLaunchGroups = 8192;
 
+// Heads of a chunk that a workgroup with a row transform takes, one after another: where the rows lie and the rotation angles are
+// the same for all of them, and a head's rows are on their way while the one before it is transformed and written.  By heads to a
+// workgroup (32 heads of 24x45x80, k / q, us): 1 445 / 392 (a workgroup's loads behind its look-up of the angles), then with
+// the loads in front and by 2 404 / 337, 4 362 / 307, 8 352 / 295, 16 354 / 297; with fewer registers (row_part) 8 317 / 275 = 4.6 and
+// 5.1 TB/s.  Calls of fewer chunks than a launch of one part keep the workgroups instead, and rows as they are gain nothing (229
+// by one head, 253 by four).
+constexpr int kHeadsPerGroup = 8;
+
 enum { kAllParts, kKeys, kValues, kQueries };
 template <bool kBf16, int kMode, int kPart>
-__global__ __launch_bounds__(256) void prepare_kernel(PrepArgs a, int wg_k, int wg_v, int64_t chunks_q) {
+__global__ __launch_bounds__(256, kPart == kKeys && kMode != kPlain ? 5 : 1) void prepare_kernel(PrepArgs a, int wg_k, int wg_v, int64_t chunks_q) {
     constexpr bool kTransform = kMode != kPlain;
     __shared__ __attribute__((aligned(16))) uint16_t tile[kPart == kQueries && !kTransform ? 8 : kTile * kPitchV];
     __shared__ float2 cs[kTransform && kPart != kValues ? 8 * 64 : 1];
@@ -468,10 +518,16 @@ hipError_t launch_prepare(const PrepArgs& args, int B, int dtype, hipStream_t st
     const bool transform = a.tab != nullptr;                    // norm and rotation come together, q's rows are always wanted
     if (transform && (a.q.norm_w == nullptr || a.k.norm_w == nullptr || a.q.rows_out == nullptr)) return hipErrorInvalidValue;
     const bool cached = a.k.cached != nullptr || a.k.rows_out != nullptr || a.v.rows_out != nullptr;      // comes with a transform
-    const int64_t wg_k = a.k.p != nullptr ? bh * a.gk.blocks() : 0;
+    for (PrepRows* x : {&a.q, &a.k}) {
+        const bool many = transform && bh * (x == &a.q ? a.gq : a.gk).blocks() >= kOneLaunchGroups;
+        const int units = many ? (a.Hn + kHeadsPerGroup - 1) / kHeadsPerGroup : a.Hn;      // evenly: 9 heads are 5 and 4
+        x->heads = (a.Hn + units - 1) / units;
+    }
+    auto groups = [&](const PrepRows& x, const Grid3& g) { return (int64_t)B * ((a.Hn + x.heads - 1) / x.heads) * g.blocks(); };
+    const int64_t wg_k = a.k.p != nullptr ? groups(a.k, a.gk) : 0;
     const int64_t wg_v = a.v.p != nullptr ? bh * a.gk.blocks() * (a.gk.chunk() / kTile) : 0;
     const int64_t chunks_q = a.q.p != nullptr ? bh * a.gq.blocks() : 0;
-    const int64_t wg_q = transform ? chunks_q : (chunks_q + 3) / 4;
+    const int64_t wg_q = transform ? (a.q.p != nullptr ? groups(a.q, a.gq) : 0) : (chunks_q + 3) / 4;
     const int64_t total = wg_k + wg_v + wg_q;
     if (total <= 0 || total > 0x7fffffff) return hipErrorInvalidValue;
     const dim3 block(256);

@@ -473,6 +473,35 @@ def test_cache_inside_the_operator_equals_the_separate_passes(T, cond, Hh, W):
     assert torch.equal(k_out, att.norm_rope(ks, empty(S), kw)) and torch.equal(v_out, vs)
 
 
+@pytest.mark.parametrize("Hn,dtype", [(19, torch.bfloat16), (16, torch.float16)])
+@pytest.mark.parametrize("cond", [0, 3])
+def test_workgroups_of_several_heads(Hn, dtype, cond):
+    """Calls of so many chunks that a workgroup takes several heads of one (19: seven, seven and five): the bits of the separate
+    passes, with and without a cache, over a grid that is ragged in every axis and two batches."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    att, ch = M(), (4, 4, 4)
+    new, full = (5, 62, 61), (5 + cond, 62, 61)
+    S, Sc = 5 * 62 * 61, cond * 62 * 61
+    g = torch.Generator("cuda").manual_seed(8)
+    rnd = lambda *s: torch.randn(*s, generator=g, device="cuda").to(dtype)      # noqa: E731
+    qs, ks, vs = rnd(2, S, 3, Hn, 128).permute(2, 0, 3, 1, 4).unbind(0)
+    kc, vc = rnd(2, Hn, Sc, 128), rnd(2, Hn, Sc, 128)
+    qw, kw = 1 + 0.1 * rnd(128), 1 + 0.1 * rnd(128)
+    tab = att.rope_table(full, 128, qs.device)
+    empty = lambda s: torch.full((2, Hn, s, 128), float("nan"), dtype=dtype, device="cuda")      # noqa: E731
+    k_out, v_out = empty(S), empty(S)
+    more = dict(kv_cache=(kc, vc, cond), kv_out=(k_out, v_out)) if cond else {}
+    got = bi._bsa_3d(qs, ks, vs, new, full, 0.9375, ch, ch, qk_norm=(qw, kw, tab, 5 + cond, cond, 0, 1e-6), **more)
+    k = empty(S + Sc)
+    if cond:
+        att.norm_rope(kc, k[:, :, :Sc], None, (cond, 62, 61), table_grid=full)
+        assert torch.equal(k_out, att.norm_rope(ks, empty(S), kw)) and torch.equal(v_out, vs)
+    att.norm_rope(ks, k[:, :, Sc:], kw, new, t_offset=cond, table_grid=full)
+    q = att.norm_rope(qs, empty(S), qw, new, t_offset=cond, table_grid=full)
+    v = torch.cat([vc, vs], 2)
+    assert torch.equal(got, bi.flash_attn_bsa_3d(q, k, v, new, full, sparsity=0.9375, chunk_3d_shape_q=ch, chunk_3d_shape_k=ch))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("frames,per,dim", [(3, 1, 8), (2, 33, 2048), (2, 32, 2056), (1, 31, 4096), (3, 70, 4104), (2, 5, 8192)])
 def test_layernorm_modulate_sizes(dtype, frames, per, dim):
