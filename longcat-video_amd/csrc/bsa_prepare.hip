@@ -5,8 +5,9 @@
 //
 // A small call runs the three parts (workgroups 0 .. wg_k - 1 take chunks of k, the next wg_v tiles of v, the rest chunks of
 // q) in one launch instead of six: its parts take a few microseconds each, and a launch in a stream of dependent ones
-// costs 4.4.  A large call runs one launch per part: together, the part that needs most registers (q, sixteen loads in
-// flight per lane) sets the occupancy of all three, 0.65 instead of 0.56 ms for 32 heads of 720p (kOneLaunchGroups).
+// costs 4.4.  There q goes the way of k, which needs half of the registers: with query_part's sixteen loads in flight per lane
+// in it the launch had half of the wavefronts (two prompts of 8 heads, 7x15x26: 16.3 -> 13.4 us).  A large call runs one launch per
+// part, each with the form and the registers that suit it (kOneLaunchGroups).
 #include "bsa_mfma.h"
 #include "bsa_rope.h"
 
@@ -463,19 +464,21 @@ __device__ __forceinline__ void query_part(const PrepRows& x, const Grid3& g, in
     }
 }
 
-// Workgroups up to which the three parts go in one launch.  The whole operator, one launch against three, us (24x32x52, 4x4x4
-// chunks, density 0.01, by heads): rows as they are 84.6 / 89.5 at 2 808 groups, 130.0 / 136.7 at 5 616, 182.0 / 188.1 at 8 424,
-// 350.9 / 351.3 at 16 848, 681 / 670 at 33 696; with norm and rotation 152 / 163 at 7 488, 272 / 286 at 14 976, 756 / 765 at
-// 44 928.  The line stands where all of them gain.
-constexpr int64_t kOneLaunchGroups = 8192;
+// Workgroups (counted as the separate launches have them) up to which the three parts go in one launch.  The whole operator, one
+// launch against three, us: rows as they are, 4x4x4 chunks, 8 heads of 24x30x52 (11 232 groups) 471 / 482, 4 heads of 24x45x80
+// (12 960) 1 106 / 1 120, 16 heads of 24x30x52 (22 464) 933 / 931, 32 (44 928) 1 845 / 1 825; 16 heads of 13x30x53 in 4x4x8
+// (11 648) 751 / 765; a block with norm, rotation and a cache, 16 + 5 frames of 30x52, 6 heads (9 984) 504 / 519, 12 (19 968) 986 /
+// 1 005.
+constexpr int64_t kOneLaunchGroups = 20480;
 
 // Heads of a chunk that a workgroup with a row transform takes, one after another: where the rows lie and the rotation angles are
 // the same for all of them, and a head's rows are on their way while the one before it is transformed and written.  By heads to a
 // workgroup (32 heads of 24x45x80, k / q, us): 1 445 / 392 (a workgroup's loads behind its look-up of the angles), then with
 // the loads in front and by 2 404 / 337, 4 362 / 307, 8 352 / 295, 16 354 / 297; with fewer registers (row_part) 8 317 / 275 = 4.6 and
-// 5.1 TB/s.  Calls of fewer chunks than a launch of one part keep the workgroups instead, and rows as they are gain nothing (229
+// 5.1 TB/s.  Calls of fewer chunks than kGroupedChunks keep the workgroups instead, and rows as they are gain nothing (229
 // by one head, 253 by four).
 constexpr int kHeadsPerGroup = 8;
+constexpr int64_t kGroupedChunks = 8192;
 
 enum { kAllParts, kKeys, kValues, kQueries };
 template <bool kBf16, int kMode, int kPart>
@@ -494,7 +497,7 @@ __global__ __launch_bounds__(256, kPart == kKeys && kMode != kPlain ? 5 : 1) voi
         return;
     }
     const int wq = kPart == kQueries ? w : w - wg_k - wg_v;
-    if (kTransform) row_part<kBf16, kTransform ? kNorm : kPlain, false>(a.q, a.gq, a.Hn, wq, a.tab, a.tab_T, a.eps, tile, cs);
+    if (kTransform || kPart == kAllParts) row_part<kBf16, kTransform ? kNorm : kPlain, false>(a.q, a.gq, a.Hn, wq, a.tab, a.tab_T, a.eps, tile, cs);
     else query_part<kBf16>(a.q, a.gq, a.Hn, (int64_t)wq * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), chunks_q);
 }
 
@@ -519,7 +522,7 @@ hipError_t launch_prepare(const PrepArgs& args, int B, int dtype, hipStream_t st
     if (transform && (a.q.norm_w == nullptr || a.k.norm_w == nullptr || a.q.rows_out == nullptr)) return hipErrorInvalidValue;
     const bool cached = a.k.cached != nullptr || a.k.rows_out != nullptr || a.v.rows_out != nullptr;      // comes with a transform
     for (PrepRows* x : {&a.q, &a.k}) {
-        const bool many = transform && bh * (x == &a.q ? a.gq : a.gk).blocks() >= kOneLaunchGroups;
+        const bool many = transform && bh * (x == &a.q ? a.gq : a.gk).blocks() >= kGroupedChunks;
         const int units = many ? (a.Hn + kHeadsPerGroup - 1) / kHeadsPerGroup : a.Hn;      // evenly: 9 heads are 5 and 4
         x->heads = (a.Hn + units - 1) / units;
     }
@@ -544,8 +547,8 @@ hipError_t launch_prepare(const PrepArgs& args, int B, int dtype, hipStream_t st
             else hipLaunchKernelGGL((prepare_kernel<false, kPlain, PART>), grid, block, 0, st, a, (int)wg_k, (int)wg_v, chunks_q);  \
         }                                                                                                                           \
     } while (0)
-    if (total <= kOneLaunchGroups) {
-        BSA_PREPARE(kAllParts, total);
+    if (total <= kOneLaunchGroups) {      // a workgroup per chunk of q here as well
+        BSA_PREPARE(kAllParts, wg_k + wg_v + (transform ? wg_q : chunks_q));
     } else {
         if (wg_q > 0) BSA_PREPARE(kQueries, wg_q);
         if (wg_k > 0) BSA_PREPARE(kKeys, wg_k);
