@@ -30,6 +30,7 @@
 // selection does; for a repeated block dQ follows the list (as the forward does) and dK / dV the bit matrix, like
 // the reference.
 #include "bsa_mfma.h"
+#include "bsa_slots.h"
 
 #include <atomic>
 
@@ -42,6 +43,22 @@ constexpr float kRcpLn2 = 1.4426950408889634f;
 constexpr int kBwdHalfTileBytes = kTileBytes / 2;            // 32 rows of 256 B
 
 // ------------------------------------------------------------------ small passes
+// the sum of products of a lane's eight values, the same instructions in every kernel: fp16 pairs in one (what the compiler makes
+// of the plain loop in one kernel and not in the next), bf16 one by one
+__device__ __forceinline__ float dot8(const f16x8& a, const f16x8& b) {
+    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) s = __builtin_amdgcn_fdot2(f16x2{a[e], a[e + 1]}, f16x2{b[e], b[e + 1]}, s, false);
+    return s;
+}
+__device__ __forceinline__ float dot8(const bf16x8& a, const bf16x8& b) {
+    float s = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = fmaf((float)a[e], (float)b[e], s);
+    return s;
+}
+
 // Per query row, both negated because the kernels below add them (as the start value of an MFMA chain):
 // delta[row] = -sum_d o * do (fp32), m2[row] = -lse * log2(e), -inf for rows without any key (their p is then 0).
 // One 16-lane group per row.
@@ -56,8 +73,7 @@ __global__ __launch_bounds__(256) void bwd_rows_kernel(const T* __restrict__ o, 
     if (row < rows) {
         const V8 a = *reinterpret_cast<const V8*>(o + row * kD + c * 8);
         const V8 b = *reinterpret_cast<const V8*>(dout + row * kD + c * 8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += (float)a[e] * (float)b[e];
+        s = dot8(a, b);
     }
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off);
@@ -96,61 +112,91 @@ __device__ __forceinline__ T* store_row(T* blocked, const BwdStore& w, int64_t b
     return blocked + (bh / w.Hn) * w.sB + (bh % w.Hn) * w.sH + (int64_t)token * w.sS;
 }
 
-// bwd_rows_kernel for o, dO and lse in token order (element strides oS / dS per token, lse [B * Hn][tokens]): the
-// same delta and m2 per blocked-order slot, and dO copied into blocked order on the way (padded slots: a zero row,
-// delta 0, m2 -inf, so that their p is 0).  One 16-lane group per slot.
+// What the kernels below need of tensors in token order, in one launch (HBM-bound): q, dO and v in blocked order, k_s, delta and
+// M2 per slot (padded slots: zero rows, delta -0, M2 -inf, so that their p is 0), the row tables of both grids, the validity
+// words of the keys, and the bit matrix cleared.  A workgroup per 64-slot tile; workgroups 0 .. wg_q - 1 take tiles of the
+// queries, the next wg_k tiles of the keys, the rest words of the matrix.  delta and M2 as bwd_rows_kernel takes them.
+// Five launches less in front of a small backward, at 4 us each; at 32 heads of 24x30x52 it takes what the separate passes took.
+struct BwdPrep {
+    Grid3 gq, gk;
+    int Hn;
+    const uint16_t *q, *o, *dout, *k, *v;
+    int64_t q_st[3], o_st[3], do_st[3], k_st[3], v_st[3];      // element strides {batch, head, token}
+    const float* lse;                                          // [B * Hn][tokens]
+    int64_t q_tokens;
+    uint16_t *q_blocked, *dout_blocked, *ks, *v_blocked;
+    float *delta, *m2;
+    int32_t *q_rows, *k_rows;
+    uint64_t* valid;
+    uint32_t* bits;
+    int64_t n_bits;
+    float c;                                                   // of k_s
+};
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_rows_thw_kernel(const T* __restrict__ o, int64_t oB, int64_t oH, int64_t oS,
-                                                           const T* __restrict__ dout, int64_t dB, int64_t dH, int64_t dS,
-                                                           const float* __restrict__ lse, const int32_t* __restrict__ rows,
-                                                           int64_t tokens, int Hn, int64_t slots, T* __restrict__ dout_blocked,
-                                                           float* __restrict__ delta, float* __restrict__ m2, int64_t total) {
+__global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, int wg_k) {
     typedef typename Vec8<T>::type V8;
-    const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-    const int c = threadIdx.x & 15;
-    if (row >= total) return;                                    // whole 16-lane groups leave together
-    const int64_t bh = row / slots;
-    const int32_t token = rows[row - bh * slots];
-    float s = 0.f;
-    V8 b;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) b[e] = (T)0.f;
-    if (token >= 0) {
-        const int64_t at = (bh / Hn), hd = (bh % Hn);
-        const V8 a = *reinterpret_cast<const V8*>(o + at * oB + hd * oH + (int64_t)token * oS + c * 8);
-        b = *reinterpret_cast<const V8*>(dout + at * dB + hd * dH + (int64_t)token * dS + c * 8);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s += (float)a[e] * (float)b[e];
+    const int lane = threadIdx.x & 63, c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
+    const int w = blockIdx.x;
+    if (w >= wg_q + wg_k) {
+        const int64_t i = (int64_t)(w - wg_q - wg_k) * 256 + threadIdx.x;
+        if (i < a.n_bits) a.bits[i] = 0u;
+        return;
     }
-    *reinterpret_cast<V8*>(dout_blocked + row * kD + c * 8) = b;
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if (c == 0) {
-        delta[row] = -s;
-        const float l = token >= 0 ? lse[bh * tokens + token] : -INFINITY;
-        m2[row] = l == -INFINITY ? -INFINITY : -(l * kRcpLn2);
+    const bool queries = w < wg_q;
+    const Grid3& g = queries ? a.gq : a.gk;
+    const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
+    const int id = queries ? w : w - wg_q, bh = id / tiles, tile = id - bh * tiles;
+    const int batch = bh / a.Hn, head = bh - batch * a.Hn;
+    const Slots s = slots_of(g, tile / per_chunk, tile % per_chunk, lane);
+    if (bh == 0 && threadIdx.x < 64) {
+        (queries ? a.q_rows : a.k_rows)[(int64_t)tile * kTile + lane] = s.token;
+        if (!queries && lane == 0) a.valid[tile] = s.word;
     }
-}
-
-// bwd_scale_kernel for k in token order: k_s in blocked order, padded slots zero.  One 16-lane group per slot.
-template <typename T>
-__global__ __launch_bounds__(256) void bwd_scale_thw_kernel(const T* __restrict__ k, int64_t kB, int64_t kH, int64_t kS,
-                                                            const int32_t* __restrict__ rows, int Hn, int64_t slots,
-                                                            T* __restrict__ ks, float c, int64_t total) {
-    typedef typename Vec8<T>::type V8;
-    const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-    if (row >= total) return;
-    const int64_t bh = row / slots;
-    const int32_t token = rows[row - bh * slots];
-    V8 x;
+    const int64_t row0 = (int64_t)id * kTile + rg;             // of the blocked tensors
+    int token[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = (T)0.f;
-    if (token >= 0) {
-        x = *reinterpret_cast<const V8*>(k + (bh / Hn) * kB + (bh % Hn) * kH + (int64_t)token * kS + (threadIdx.x & 15) * 8);
+    for (int i = 0; i < 4; ++i) token[i] = max(__shfl(s.token, rg + 16 * i), 0);
+    auto at = [&](const uint16_t* p, const int64_t (&st)[3], int i) -> uint4 {
+        return *reinterpret_cast<const uint4*>(p + batch * st[0] + head * st[1] + (int64_t)token[i] * st[2] + c16 * 8);
+    };
+    auto put = [&](uint16_t* p, int i, const uint4& x) { *reinterpret_cast<uint4*>(p + (row0 + 16 * i) * kD + c16 * 8) = x; };
+    if (queries) {
+        uint4 q[4], o[4], d[4];
+        float l[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * c);
+        for (int i = 0; i < 4; ++i) { q[i] = at(a.q, a.q_st, i); o[i] = at(a.o, a.o_st, i); d[i] = at(a.dout, a.do_st, i); }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) l[i] = a.lse[bh * a.q_tokens + token[i]];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool real = (s.word >> (rg + 16 * i)) & 1ull;
+            keep_if(q[i], real); keep_if(o[i], real); keep_if(d[i], real);
+            float sum = dot8(__builtin_bit_cast(V8, o[i]), __builtin_bit_cast(V8, d[i]));
+#pragma unroll
+            for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+            put(a.q_blocked, i, q[i]);
+            put(a.dout_blocked, i, d[i]);
+            if (c16 == 0) {
+                a.delta[row0 + 16 * i] = -sum;
+                a.m2[row0 + 16 * i] = !real || l[i] == -INFINITY ? -INFINITY : -(l[i] * kRcpLn2);
+            }
+        }
+    } else {
+        uint4 k[4], v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { k[i] = at(a.k, a.k_st, i); v[i] = at(a.v, a.v_st, i); }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool real = (s.word >> (rg + 16 * i)) & 1ull;
+            V8 x = __builtin_bit_cast(V8, k[i]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * a.c);
+            uint4 ks = __builtin_bit_cast(uint4, x);
+            keep_if(ks, real); keep_if(v[i], real);
+            put(a.ks, i, ks);
+            put(a.v_blocked, i, v[i]);
+        }
     }
-    *reinterpret_cast<V8*>(ks + row * kD + (threadIdx.x & 15) * 8) = x;
 }
 
 __global__ void bwd_zero_kernel(uint32_t* p, int64_t n) {
@@ -158,29 +204,14 @@ __global__ void bwd_zero_kernel(uint32_t* p, int64_t n) {
     if (i < n) p[i] = 0u;
 }
 
-// bits[bh][kv block][query block / 32] |= 1 << (query block % 32) for every list entry; block indices are clamped
-// to the valid range as the forward kernels do.
-__global__ __launch_bounds__(256) void bwd_mask_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ lens,
-                                                       uint32_t* __restrict__ bits, int nbq, int nbk, int stride,
-                                                       int words, int64_t rows) {
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const int lane = threadIdx.x & 63;
-    const int64_t bh = row / nbq;
-    const int m = (int)(row % nbq);
-    const int n = min(max(lens[row], 0), stride);
-    for (int e = lane; e < n; e += 64) {
-        const int j = min(max(idx[row * stride + e], 0), nbk - 1);
-        atomicOr(bits + (bh * nbk + j) * words + (m >> 5), 1u << (m & 31));
-    }
-}
-
 // counts[bh * nbk + j] = number of query blocks that selected KV block j (bits set in its row of the bit matrix); with `base`
-// also the number of tile pairs of the head's blocks in front of j (per_entry pairs for each entry of a list).  One workgroup
-// per head.
+// also the number of tile pairs of the head's blocks in front of j (per_entry pairs for each entry of a list); order: the head's
+// KV tiles by descending count, a counting sort (tiles of one count in no particular order).  One workgroup per head.  LDS: a
+// bin per count, 0 .. nbq, and four words at least.
 __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restrict__ bits, int32_t* __restrict__ counts,
-                                                        int32_t* __restrict__ base, int words, int nbk, int per_entry) {
-    __shared__ int part[4];
+                                                        int32_t* __restrict__ base, int32_t* __restrict__ order, int words, int nbk, int nbq,
+                                                        int tiles_per_block, int per_entry) {
+    extern __shared__ int bins[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t head = (int64_t)blockIdx.x * nbk;
     int before = 0;
@@ -197,12 +228,38 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
             const int t = __shfl_up(upto, off);
             if (lane >= off) upto += t;
         }
-        if (lane == 63) part[wave] = upto;
+        if (lane == 63) bins[wave] = upto;
         __syncthreads();
-        for (int w = 0; w < wave; ++w) upto += part[w];
+        for (int w = 0; w < wave; ++w) upto += bins[w];
         if (j < nbk) base[head + j] = (before + upto - c) * per_entry;
-        before += part[0] + part[1] + part[2] + part[3];
+        before += bins[0] + bins[1] + bins[2] + bins[3];
         __syncthreads();
+    }
+    for (int i = threadIdx.x; i <= nbq; i += 256) bins[i] = 0;
+    __syncthreads();
+    for (int j = threadIdx.x; j < nbk; j += 256) atomicAdd(&bins[counts[head + j]], tiles_per_block);       // this thread's own counts
+    __syncthreads();
+    // offsets in descending count: lane l of the first wavefront takes the l-th share of the bins, from the top
+    if (wave == 0) {
+        const int per = (nbq + 64) / 64, top = nbq - lane * per;
+        int mine = 0;
+        for (int i = 0; i < per; ++i)
+            if (top - i >= 0) mine += bins[top - i];
+        int run = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int t = __shfl_up(run, off);
+            if (lane >= off) run += t;
+        }
+        run -= mine;
+        for (int i = 0; i < per; ++i)
+            if (top - i >= 0) { const int n = bins[top - i]; bins[top - i] = run; run += n; }
+    }
+    __syncthreads();
+    const int first_tile = (int)blockIdx.x * nbk * tiles_per_block;
+    for (int j = threadIdx.x; j < nbk; j += 256) {
+        const int to = atomicAdd(&bins[counts[head + j]], tiles_per_block);
+        for (int i = 0; i < tiles_per_block; ++i) order[first_tile + to + i] = first_tile + j * tiles_per_block + i;
     }
 }
 
@@ -1062,31 +1119,34 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     int32_t* place = reinterpret_cast<int32_t*>(ws + at.place);
     const int per_entry = (bs_q / kTile) * (bs_k / kTile);
 
-    const int64_t qrows = (int64_t)bh * Sq, krows = (int64_t)bh * Sk;
+    const size_t count_lds = (size_t)(nbq + 1 > 4 ? nbq + 1 : 4) * sizeof(int);
+    if (count_lds > 64 * 1024) return hipErrorInvalidValue;      // bwd_count_kernel's bins: 16 383 query blocks
+    const int64_t qrows = (int64_t)bh * Sq, krows = (int64_t)bh * Sk, nwords = (int64_t)bh * nbk * words;
     const float c = sm_scale * kRcpLn2;
     BwdStore dq_to = {nullptr, 0, 0, 0, Hn}, dk_to = dq_to, dv_to = dq_to;
     if (thw != nullptr) {
-        // o, dO, lse and k in token order: the two passes read them through the row tables, and dO comes out in
-        // blocked order for the kernels; q and v are the caller's blocked-order copies
         dq_to = {thw->q_rows, thw->dq_st[0], thw->dq_st[1], thw->dq_st[2], Hn};
         dk_to = {thw->k_rows, thw->dk_st[0], thw->dk_st[1], thw->dk_st[2], Hn};
         dv_to = {thw->k_rows, thw->dv_st[0], thw->dv_st[1], thw->dv_st[2], Hn};
         dq = thw->dq; dk = thw->dk; dv = thw->dv;
-        dout = thw->dout_blocked;
-        const dim3 gq((unsigned)((qrows + 15) / 16)), gk((unsigned)((krows + 15) / 16)), blk(256);
-        if (dtype == BSA_BF16) {
-            hipLaunchKernelGGL((bwd_rows_thw_kernel<__bf16>), gq, blk, 0, st, (const __bf16*)thw->o, thw->o_st[0], thw->o_st[1], thw->o_st[2],
-                               (const __bf16*)thw->dout, thw->do_st[0], thw->do_st[1], thw->do_st[2], thw->lse, thw->q_rows, thw->q_tokens, Hn,
-                               Sq, (__bf16*)thw->dout_blocked, delta, m2, qrows);
-            hipLaunchKernelGGL((bwd_scale_thw_kernel<__bf16>), gk, blk, 0, st, (const __bf16*)thw->k, thw->k_st[0], thw->k_st[1], thw->k_st[2],
-                               thw->k_rows, Hn, Sk, (__bf16*)ks, c, krows);
-        } else {
-            hipLaunchKernelGGL((bwd_rows_thw_kernel<_Float16>), gq, blk, 0, st, (const _Float16*)thw->o, thw->o_st[0], thw->o_st[1], thw->o_st[2],
-                               (const _Float16*)thw->dout, thw->do_st[0], thw->do_st[1], thw->do_st[2], thw->lse, thw->q_rows, thw->q_tokens, Hn,
-                               Sq, (_Float16*)thw->dout_blocked, delta, m2, qrows);
-            hipLaunchKernelGGL((bwd_scale_thw_kernel<_Float16>), gk, blk, 0, st, (const _Float16*)thw->k, thw->k_st[0], thw->k_st[1], thw->k_st[2],
-                               thw->k_rows, Hn, Sk, (_Float16*)ks, c, krows);
+        q = thw->q_blocked; v = thw->v_blocked; dout = thw->dout_blocked;
+        BwdPrep a = {};
+        a.gq = thw->gq; a.gk = thw->gk; a.Hn = Hn;
+        a.q = (const uint16_t*)thw->q; a.o = (const uint16_t*)thw->o; a.dout = (const uint16_t*)thw->dout; a.k = (const uint16_t*)thw->k;
+        a.v = (const uint16_t*)thw->v;
+        for (int i = 0; i < 3; ++i) {
+            a.q_st[i] = thw->q_st[i]; a.o_st[i] = thw->o_st[i]; a.do_st[i] = thw->do_st[i]; a.k_st[i] = thw->k_st[i]; a.v_st[i] = thw->v_st[i];
         }
+        a.lse = thw->lse; a.q_tokens = (int64_t)thw->gq.T * thw->gq.H * thw->gq.W;
+        a.q_blocked = (uint16_t*)thw->q_blocked; a.dout_blocked = (uint16_t*)thw->dout_blocked; a.ks = (uint16_t*)ks;
+        a.v_blocked = (uint16_t*)thw->v_blocked;
+        a.delta = delta; a.m2 = m2; a.q_rows = thw->q_rows; a.k_rows = thw->k_rows; a.valid = thw->valid;
+        a.bits = bits; a.n_bits = nwords; a.c = c;
+        const int64_t wg_q = qrows / kTile, wg_k = krows / kTile, wg_bits = (nwords + 255) / 256;
+        if (wg_q + wg_k + wg_bits > 0x7fffffff) return hipErrorInvalidValue;
+        const dim3 grid((unsigned)(wg_q + wg_k + wg_bits)), blk(256);
+        if (dtype == BSA_BF16) hipLaunchKernelGGL((bwd_prepare_kernel<__bf16>), grid, blk, 0, st, a, (int)wg_q, (int)wg_k);
+        else hipLaunchKernelGGL((bwd_prepare_kernel<_Float16>), grid, blk, 0, st, a, (int)wg_q, (int)wg_k);
     } else if (dtype == BSA_BF16) {
         hipLaunchKernelGGL((bwd_rows_kernel<__bf16>), dim3((unsigned)((qrows + 15) / 16)), dim3(256), 0, st, (const __bf16*)o,
                            (const __bf16*)dout, lse, delta, m2, qrows);
@@ -1098,17 +1158,14 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         hipLaunchKernelGGL((bwd_scale_kernel<_Float16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
                            (const _Float16*)k, (_Float16*)ks, c, krows * 16);
     }
-    const int64_t nwords = (int64_t)bh * nbk * words;
-    hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, bits, nwords);
+    if (thw == nullptr) hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, bits, nwords);
     const int64_t lrows = (int64_t)bh * nbq;
-    hipLaunchKernelGGL(bwd_mask_kernel, dim3((unsigned)((lrows + 3) / 4)), dim3(256), 0, st, idx, lens, bits, nbq, nbk, idx_stride,
-                       words, lrows);
     hipError_t e;
-    hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)bh), dim3(256), 0, st, bits, counts, kept.keep ? base : nullptr, words, nbk, per_entry);
-    if ((e = launch_order_by_length(counts, order, (int)bh, nbk, bs_k / kTile, nbq, st)) != hipSuccess) return e;
     // dQ walks every list in the forward kernel's visiting order when the list is ascending (a selection in block
     // order); any other order is walked as given.  The order only moves fp32 roundings of the dQ sum.
-    if ((e = launch_pace_order(idx, paced, lens, (int64_t)bh * nbq, nbk, idx_stride, st)) != hipSuccess) return e;
+    if ((e = launch_pace_order(idx, paced, lens, lrows, nbk, idx_stride, st, {}, {bits, nbq, words})) != hipSuccess) return e;
+    hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)bh), dim3(256), count_lds, st, bits, counts, kept.keep ? base : nullptr, order, words, nbk, nbq,
+                       bs_k / kTile, per_entry);
 
     const dim3 block(64);
     // the dK / dV kernel's LDS: four stages of half a Q tile, half a dO tile and the queries' M2 / delta, then a KV block's query blocks

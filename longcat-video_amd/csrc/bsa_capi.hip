@@ -662,6 +662,11 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     BSA_TRY(check_tensor(o, o_strides, p, "o"));
     BSA_TRY(check_kv_views(pl, k_strides, v_strides, "fwd_3d"));
 
+    // the lists that the caller keeps for a backward are written where it wants them, not copied there: 8 us of a call
+    if (walk_out != nullptr) {
+        w.idx_sorted = walk_out;
+        w.lens = lens_out;
+    }
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
 #define BSA_HIP(call, what) do { e = (call); if (e != hipSuccess) return hip_fail(e, what); } while (0)
@@ -718,9 +723,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     const size_t bh = (size_t)p->B * p->Hn;
     if (idx_out && pl.sel_width > 0)
         BSA_HIP(hipMemcpyAsync(idx_out, w.idx, bh * pl.nbq * pl.sel_width * sizeof(int32_t), hipMemcpyDeviceToDevice, st), "copy idx");
-    if (walk_out && pl.sel_width > 0)
-        BSA_HIP(hipMemcpyAsync(walk_out, w.idx_sorted, bh * pl.nbq * pl.sel_width * sizeof(int32_t), hipMemcpyDeviceToDevice, st), "copy walk order");
-    if (lens_out) BSA_HIP(hipMemcpyAsync(lens_out, w.lens, bh * pl.nbq * sizeof(int32_t), hipMemcpyDeviceToDevice, st), "copy lens");
+    if (lens_out && lens_out != w.lens) BSA_HIP(hipMemcpyAsync(lens_out, w.lens, bh * pl.nbq * sizeof(int32_t), hipMemcpyDeviceToDevice, st), "copy lens");
     if (score_out) BSA_HIP(hipMemcpyAsync(score_out, w.score, bh * pl.nbq * (size_t)pl.nbk * pl.es, hipMemcpyDeviceToDevice, st), "copy score");
 #undef BSA_HIP
     return BSA_OK;
@@ -943,30 +946,21 @@ int bsa_bwd_3d(const bsa_3d_params* p, const void* q, const int64_t q_strides[3]
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0) return set_error(BSA_ERR_BAD_ARG, "bwd_3d: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
     hipStream_t st = (hipStream_t)stream;
-    int32_t* q_rows = reinterpret_cast<int32_t*>(ws + pl.off_qrows);
-    int32_t* k_rows = reinterpret_cast<int32_t*>(ws + pl.off_krows);
-    uint64_t* valid = reinterpret_cast<uint64_t*>(ws + pl.off_valid);
-    // q and v in blocked order (the kernels stream their tiles as they lie in memory); the passes write the row tables
-    // of both grids and the validity words of the keys on the way
-    hipError_t e = launch_permute(q, q_strides, ws + pl.off_qp, nullptr, nullptr, p->B, p->Hn, pl.gq, p->D, p->dtype, st, false, q_rows);
-    if (e != hipSuccess) return hip_fail(e, "bwd_3d: permute q");
-    e = launch_permute(v, v_strides, ws + pl.off_vp, nullptr, valid, p->B, p->Hn, pl.gk, p->D, p->dtype, st, false, k_rows);
-    if (e != hipSuccess) return hip_fail(e, "bwd_3d: permute v");
     BwdThw t;
-    t.q_rows = q_rows;
-    t.k_rows = k_rows;
-    t.q_tokens = (int64_t)p->Tq * p->Hq * p->Wq;
-    t.k_tokens = (int64_t)p->Tk * p->Hk * p->Wk;
-    t.o = o; t.dout = d_o; t.lse = lse; t.k = k;
-    t.dout_blocked = ws + pl.off_dop;
+    t.gq = pl.gq; t.gk = pl.gk;
+    t.q = q; t.k = k; t.v = v; t.o = o; t.dout = d_o; t.lse = lse;
+    t.q_blocked = ws + pl.off_qp; t.v_blocked = ws + pl.off_vp; t.dout_blocked = ws + pl.off_dop;
+    t.q_rows = reinterpret_cast<int32_t*>(ws + pl.off_qrows);
+    t.k_rows = reinterpret_cast<int32_t*>(ws + pl.off_krows);
+    t.valid = reinterpret_cast<uint64_t*>(ws + pl.off_valid);
     t.dq = dq; t.dk = dk; t.dv = dv;
     for (int i = 0; i < 3; ++i) {
-        t.o_st[i] = o_strides[i]; t.do_st[i] = do_strides[i]; t.k_st[i] = k_strides[i];
+        t.q_st[i] = q_strides[i]; t.k_st[i] = k_strides[i]; t.v_st[i] = v_strides[i]; t.o_st[i] = o_strides[i]; t.do_st[i] = do_strides[i];
         t.dq_st[i] = dq_strides[i]; t.dk_st[i] = dk_strides[i]; t.dv_st[i] = dv_strides[i];
     }
-    e = launch_bwd(ws + pl.off_qp, nullptr, ws + pl.off_vp, nullptr, nullptr, nullptr, idx, lens, kv_padded(p) ? valid : nullptr, nullptr,
-                   nullptr, nullptr, p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype,
-                   ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t);
+    const hipError_t e = launch_bwd(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, idx, lens, kv_padded(p) ? t.valid : nullptr, nullptr, nullptr, nullptr,
+                                    p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype,
+                                    ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "bwd_3d launch");
 }
 

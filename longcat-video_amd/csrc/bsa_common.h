@@ -180,8 +180,14 @@ hipError_t launch_fwd_f32(const void* q, const void* k, const void* v, const int
 
 // Rewrites every row's ascending list of KV blocks into the order the attention kernel visits them in (see
 // pace_order_kernel).  rows of `stride` entries, lens[row] of them in use; in == out allowed; stride <= 5000.
+// With `bits` the lists are also written down the other way: words[bh][block][row / 32] gets bit row % 32 of every block in
+// row `row` of (batch, head) bh, `rows` rows each (cleared by the caller).
+struct ListBits {
+    uint32_t* words;
+    int rows, per_row;
+};
 hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* lens, int64_t rows, int nbk, int stride,
-                             hipStream_t st, HalfLists halves = {});
+                             hipStream_t st, HalfLists halves = {}, ListBits bits = {});
 // order: for every (batch, head) its 64-row query tiles by descending list length (lens is per query
 // block of tiles_per_block tiles, clamped to [0, max_len]); with `order` and a two-word `queue`
 // launch_fwd enqueues the 16-bit kernel both as rounds and as one launch whose workgroups draw items
@@ -255,19 +261,18 @@ size_t frag_fallback_ints(int64_t items);
 // those with `least` (then dS is not kept between the kernels and dQ is computed from scratch).
 size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, bool least = false);
 int bwd_max_query_blocks();      // the dK / dV kernel stages a KV block's query blocks in LDS: Sq / bs_q may not exceed this
-// With `thw` the caller's o, dO, lse, k and the three gradients are in token order: the passes that take delta and k_s
-// read them through the row tables (token of every blocked-order slot of one (batch, head), -1 = padding) and the
-// kernels store the gradient rows at their tokens.  q and v are then blocked-order copies (launch_permute), and the
-// arguments k, o, dout, lse, dq, dk, dv of launch_bwd are not used.  Strides count elements.
+// With `thw` the caller's tensors are in token order: a pass in front brings q, v, dO and k_s into blocked order, with the row
+// tables (token of every blocked-order slot of one (batch, head), -1 = padding) and the validity words, and the kernels store
+// the gradient rows at their tokens.  Of launch_bwd's own tensors only idx, lens and tile_valid are then used.  Strides count
+// elements.
 struct BwdThw {
-    const int32_t* q_rows;
-    const int32_t* k_rows;
-    int64_t q_tokens, k_tokens;       // real tokens per (batch, head)
-    const void* o; int64_t o_st[3];
-    const void* dout; int64_t do_st[3];
-    const float* lse;                 // [B * Hn][q_tokens]
-    const void* k; int64_t k_st[3];
-    void* dout_blocked;               // B * Hn * Sq rows of 128 elements
+    Grid3 gq, gk;
+    const void *q, *k, *v, *o, *dout;
+    int64_t q_st[3], k_st[3], v_st[3], o_st[3], do_st[3];
+    const float* lse;                 // [B * Hn][tokens]
+    void *q_blocked, *v_blocked, *dout_blocked;      // B * Hn * Sq (v: Sk) rows of 128 elements
+    int32_t *q_rows, *k_rows;         // Sq and Sk entries
+    uint64_t* valid;                  // Sk / 64 words
     void* dq; int64_t dq_st[3];
     void* dk; int64_t dk_st[3];
     void* dv; int64_t dv_st[3];

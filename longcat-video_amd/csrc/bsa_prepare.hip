@@ -10,6 +10,7 @@
 // part, each with the form and the registers that suit it (kOneLaunchGroups).
 #include "bsa_mfma.h"
 #include "bsa_rope.h"
+#include "bsa_slots.h"
 
 namespace bsa {
 namespace {
@@ -58,36 +59,6 @@ __global__ __launch_bounds__(256) void head_norm_kernel(const float* __restrict_
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = best;
     __syncthreads();
     if (threadIdx.x == 0) key_norm[blockIdx.x] = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
-}
-
-__device__ __forceinline__ void keep_if(uint4& x, bool keep) {
-    const uint32_t m = keep ? ~0u : 0u;
-    x.x &= m; x.y &= m; x.z &= m; x.w &= m;
-}
-
-// The 64 slots of a tile as a wavefront sees them, one per lane: grid position, token row (-1: padding), and the word of
-// the real ones.
-struct Slots {
-    int token, loc;        // loc: position inside the chunk, ti | hi << 8 | wi << 16
-    uint64_t word;
-};
-__device__ __forceinline__ Slots slots_of(const Grid3& g, int blk, int sub, int lane) {
-    const int nw = blk % g.Nw, nh = (blk / g.Nw) % g.Nh, nt = blk / (g.Nw * g.Nh);
-    const int r = sub * kTile + lane;
-    int wi, hi, ti;
-    if (((g.w & (g.w - 1)) | (g.h & (g.h - 1))) == 0) {           // the usual chunks: shifts instead of three divisions
-        const int ws = __builtin_ctz(g.w), hs = __builtin_ctz(g.h);
-        wi = r & (g.w - 1); hi = (r >> ws) & (g.h - 1); ti = r >> (ws + hs);
-    } else {
-        wi = r % g.w; hi = (r / g.w) % g.h; ti = r / (g.w * g.h);
-    }
-    const int tt = nt * g.t + ti, hh = nh * g.h + hi, ww = nw * g.w + wi;
-    const bool ok = tt < g.T && hh < g.H && ww < g.W;
-    Slots s;
-    s.token = ok ? (tt * g.H + hh) * g.W + ww : -1;
-    s.loc = ti | (hi << 8) | (wi << 16);
-    s.word = __ballot(ok);
-    return s;
 }
 
 // Where a slot of a tile goes: the real ones (bits of `word`) to the front, both groups in slot order.  The keys of a tile

@@ -544,13 +544,20 @@ __device__ inline const int32_t* pace_row(int32_t* work, int n, int cap, int nbk
     wave_sync();
     return spare;
 }
-__global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32_t* out, const int32_t* __restrict__ lens, int nbk, int stride, HalfLists halves) {
+__global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32_t* out, const int32_t* __restrict__ lens, int nbk, int stride, HalfLists halves,
+                                                        ListBits bits) {
     extern __shared__ int32_t pace_lds[];
     const int lane = threadIdx.x;
     const int64_t row = blockIdx.x;
     const int32_t* src = in + row * stride;
     int32_t* dst = out + row * stride;
     const int n = min(max(lens[row], 0), stride);
+    if (bits.words != nullptr) {
+        const int64_t bh = row / bits.rows;
+        const int m = (int)(row - bh * bits.rows);
+        for (int e = lane; e < n; e += 64)
+            atomicOr(bits.words + (bh * nbk + min(max(src[e], 0), nbk - 1)) * bits.per_row + (m >> 5), 1u << (m & 31));
+    }
     if (src != dst)
         for (int e = n + lane; e < stride; e += 64) dst[e] = src[e];
     if (n <= kPaceWidth && halves.lists == nullptr) {
@@ -887,12 +894,12 @@ hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int
 }
 
 hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* lens, int64_t rows, int nbk, int stride,
-                             hipStream_t st, HalfLists halves) {
+                             hipStream_t st, HalfLists halves, ListBits bits) {
     if (rows <= 0 || stride <= 0) return hipSuccess;
     const int groups = (stride + kPaceWidth - 1) / kPaceWidth;
     const size_t lds = ((size_t)3 * stride + groups) * sizeof(int32_t);
     if (lds > 64 * 1024 || rows > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pace_order_kernel, dim3((unsigned)rows), dim3(64), lds, st, in, out, lens, nbk, stride, halves);
+    hipLaunchKernelGGL(pace_order_kernel, dim3((unsigned)rows), dim3(64), lds, st, in, out, lens, nbk, stride, halves, bits);
     return hipGetLastError();
 }
 

@@ -289,3 +289,22 @@ def test_argument_checks():
                                                   p(t), st, p(t), st, p(t), st, p(ws), ws_bytes, None)
     assert call(p(t), 16) == _capi.BSA_ERR_WORKSPACE
     assert call(None, 1 << 20) == _capi.BSA_ERR_BAD_ARG
+
+
+@pytest.mark.parametrize("lq,chunk,sparsity", [
+    ((4, 4, 4), (4, 4, 4), 0.0),            # one block, one bin
+    ((4, 4, 36), (4, 4, 4), 0.5),           # nine blocks: fewer than the threads, words of one
+    ((12, 41, 50), (4, 4, 4), 0.9),         # 429 blocks: more than 256, words with a remainder, a ragged grid
+    ((9, 17, 30), (4, 4, 8), 0.5),          # two tiles a block, tiles without rows
+])
+def test_key_blocks_are_counted_and_sorted(lq, chunk, sparsity):
+    """The bit matrix, its counts, the prefix sums behind kept dS and the order of the key tiles, over few and many blocks: the
+    gradients of the rearranging route, and of a workspace without room for dS, bit for bit."""
+    bi = I()
+    H, S = 3, int(np.prod(lq))
+    g = torch.Generator("cuda").manual_seed(12)
+    q, k, v, do = (torch.randn(2, H, S, 128, generator=g, device="cuda").half() for _ in range(4))
+    o, walk, lens, lse = bi._bsa_3d(q, k, v, lq, lq, sparsity, chunk, chunk, for_backward=True)
+    args = (do, q, k, v, o, lse, walk, lens, lq, lq, chunk, chunk, 128 ** -0.5)
+    for a, b in zip(bi._bsa_3d_backward(*args), bi._bsa_3d_backward_by_rearranging(*args)):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)
