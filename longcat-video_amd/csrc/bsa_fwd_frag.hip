@@ -71,6 +71,20 @@ __device__ __forceinline__ float dot2_self(f16x8 x, int e, float acc) {
     return __builtin_amdgcn_fdot2(p, p, acc, false);
 }
 
+// n / d for 0 <= n < 2^31 by a product: m = ceil(2^p / d) with p = 31 + ceil(log2 d), so m d - 2^p < d <= 2^(p - 31) and the error
+// n (m d - 2^p) / (d 2^p) of the quotient stays below 1 / d.  A division by a number that the compiler does not know costs
+// 25 (32 bits) to 120 instructions (64), one after another, and an item has nine of them in front of its first product.
+struct Divisor {
+    uint32_t m, p;
+};
+static Divisor divisor(int d) {
+    uint32_t l = 0;
+    while (((int64_t)1 << l) < d) ++l;
+    const uint32_t p = 31 + l;
+    return {(uint32_t)((((unsigned __int128)1 << p) + d - 1) / d), p};
+}
+__device__ __forceinline__ int operator/(int n, const Divisor& d) { return (int)(((uint64_t)(uint32_t)n * d.m) >> d.p); }
+
 struct FragLayout {
     const int32_t* q_rows;        // token row of every blocked-order query slot, -1 = padding; null: q, o in blocked order
     int64_t q_st[3], o_st[3];     // element strides: batch, head, row
@@ -78,6 +92,7 @@ struct FragLayout {
     // tiles[u % n_live] of (batch, head) u / n_live.
     const int32_t* tiles;
     int n_live;
+    Divisor by_live, by_tiles, by_block, by_heads, by_sub;       // n_live; query tiles of a (batch, head), of a block; heads; tiles of a KV block
 };
 // The tile number (over all heads) of work item u.  The table was written by an earlier kernel and is read through the scalar
 // cache: the wait for it is its own, not one for every load of the wavefront, and all that is derived from it stays scalar.
@@ -85,7 +100,7 @@ struct FragLayout {
 // at 32 heads of 720p.)
 __device__ __forceinline__ int item_at(const FragLayout& L, int u, int nqt) {
     if (L.tiles == nullptr) return u;
-    const int bh = u / L.n_live;
+    const int bh = u / L.by_live;
     return bh * nqt + *(const __attribute__((address_space(4))) int32_t*)(L.tiles + (u - bh * L.n_live));
 }
 
@@ -127,6 +142,7 @@ constexpr int kPartFloats = kTile * kD + 2 * kTile;
 struct Parts {
     float* buf;
     int count, items;
+    Divisor by_count, by_items;
 };
 
 // The schedule for lists of unequal length: a queue per XCD.  Section x holds the items [section_begin(x), section_begin(x + 1))
@@ -134,6 +150,17 @@ struct Parts {
 constexpr int kQueues = 8, kQueueChoice = kQueues, kQueueWords = kQueues + 1;      // a counter per section, the choice of schedule
 static_assert(kQueueWords <= kFragQueueWords, "the caller's buffer holds the words");
 __device__ __forceinline__ int section_begin(int n, int x) { return (int)(((int64_t)n * x) >> 3); }
+
+// The kernel's arguments fill six cache lines, and the compiler loads them where it first needs them: six waits for memory, one
+// after another, in front of a launch's first item.  Asked for together they cost one, 0.36 us for 0.7 to 1.1.  With what an item
+// that nothing has prepared now asks for at once (below) and the divisions that went, the kernel of a single round is 1.3 us
+// shorter: 15.1 -> 13.8 us for 5 heads of 9x27x12, 25.4 -> 24.2 for two prompts of 8 heads of 7x15x26.
+__device__ __forceinline__ void touch_arguments() {
+    uint32_t a, b, c, d, e, f;
+    asm volatile("s_load_dword %0, %6, 0x0\n\ts_load_dword %1, %6, 0x40\n\ts_load_dword %2, %6, 0x80\n\ts_load_dword %3, %6, 0xc0\n\t"
+                 "s_load_dword %4, %6, 0x100\n\ts_load_dword %5, %6, 0x13c\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(a), "=&s"(b), "=&s"(c), "=&s"(d), "=&s"(e), "=&s"(f) : "s"(__builtin_amdgcn_kernarg_segment_ptr()));
+}
 
 template <typename T, int kWalk, bool kBounded>
 __global__ __launch_bounds__(64) void fwd_frag_kernel(
@@ -158,6 +185,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     constexpr float kSlack = 60.0f;
     static_assert(!kBounded || std::is_same<T, __bf16>::value, "fp16 probabilities need the running maximum");
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    touch_arguments();
     if (gate != nullptr && *gate != gate_want) return;
     // output staging: 64 rows of 256 B, 272 B apart.  The same memory stages a list that is too long for the small
     // buffers (kListEntries words at most) during the tile loop of an item that was not prepared ahead of time.
@@ -171,11 +199,9 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
 
     const int lane = threadIdx.x;
     const int lr = lane & 31, lh = lane >> 5;
-    const int nbq = (int)(Sq / bs_q);
     const int nqt = (int)(Sq / kTile);
     const int nsub = kWalk == kBlocks ? bs_k / kTile : 1;
-    const int nbk = (int)(Sk / bs_k);
-    const int tiles_bh = (int)(Sk / kTile);
+    const int tiles_bh = (int)(Sk / kTile), nbk = kWalk == kBlocks ? tiles_bh / L.by_sub : tiles_bh;     // kHalves does not ask for it
     const uint32_t lane_off = (uint32_t)lane * 16u;
     // the kernel that runs the fallback list takes as many items as the list holds
     const int n_launch = kBounded ? item_end - item_begin : parts.count > 1 ? parts.count * parts.items
@@ -210,6 +236,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // From the queues (queue_plan_kernel): the section of this workgroup's XCD first, then what the others have left.
     int section_turn = 0;
     auto draw = [&]() -> int {
+#pragma unroll 1
         for (; section_turn < kQueues; ++section_turn) {
             const int x = (blockIdx.x + section_turn) & (kQueues - 1);
             const int begin = section_begin(n_launch, x), n = section_begin(n_launch, x + 1) - begin;
@@ -228,16 +255,15 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     auto fetch = [&](int local) -> Desc {
         Desc d = {-1, 0, {0, 0}, local, INFINITY};
         if (local < 0) return d;
-        if (!kBounded && parts.count > 1) local %= parts.items;
+        if (!kBounded && parts.count > 1) local -= local / parts.by_items * parts.items;
         d.item = order != nullptr ? item_begin + order[local] : item_at(L, item_begin + local, nqt);
-        const int bh = d.item / nqt, qblock = (int)((int64_t)(d.item % nqt) * kTile / bs_q);
-        const int64_t row = (int64_t)bh * nbq + qblock;
+        const int64_t row = d.item / L.by_block;
         d.nent = lens[row];
         if (idx_stride > 0) {
             d.ent[0] = idx[row * idx_stride];
             if (kWalk == kHalves) d.ent[1] = idx[row * idx_stride + 1];
         }
-        if (key_norm != nullptr) d.kn = key_norm[bh];
+        if (key_norm != nullptr) d.kn = key_norm[d.item / L.by_tiles];
         return d;
     };
     // The descriptor's loads are vector loads of one address (behind the stores of an earlier item the compiler
@@ -252,7 +278,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     };
     // the pair of halves that position 0 of d's walk names
     auto first_pair = [&](const Desc& d, uint32_t (&h)[2]) {
-        const uint32_t base = (uint32_t)((d.item / nqt - bh_first) * tiles_bh) * 2u;
+        const uint32_t base = (uint32_t)((d.item / L.by_tiles - bh_first) * tiles_bh) * 2u;
         if (kWalk == kHalves) {
             h[0] = base + ((uint32_t)uni(d.ent[0]) & kHalfId);
             h[1] = base + ((uint32_t)uni(d.ent[1]) & kHalfId);
@@ -320,7 +346,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             const uint2 x = *reinterpret_cast<const uint2*>(ents + 2 * tc);               // the same address in every lane
             r.e[0] = x.x; r.e[1] = x.y;
         } else {
-            r.e[0] = ents[kWalk == kTiles ? tc : tc / nsub];
+            r.e[0] = ents[kWalk == kTiles ? tc : tc / L.by_sub];
         }
         return r;
     };
@@ -334,7 +360,8 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         }
         if (tp >= npairs) { h[0] = beyond[0]; h[1] = beyond[1]; return; }
         const int blk = min(max(uni((int)raw.e[0]), 0), nbk - 1);                          // a malformed list: wrong numbers, never a fault
-        h[0] = half_base + 2u * (uint32_t)(kWalk == kTiles ? blk : blk * nsub + (tp + pair0) % nsub);
+        const int tc = tp + pair0;
+        h[0] = half_base + 2u * (uint32_t)(kWalk == kTiles ? blk : blk * nsub + tc - tc / L.by_sub * nsub);
         h[1] = h[0] + 1u;
     };
     // the validity word of a pair's tile (all keys valid without padding; kHalves: the entries say it), in two steps so that
@@ -530,24 +557,36 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     };
 
     // ---- the workgroup's items
-    Desc cur = fetch(next_local());
-    Desc nxt = fetch(next_local());
+    Desc cur, nxt;
+#pragma unroll 1
+    for (int i = 0; i < 2; ++i) {        // one copy of the code: a launch's first item pays for every line of it, cold
+        cur = nxt;
+        nxt = fetch(next_local());
+    }
     bool prepared = false;           // the current item's list, Q rows and first fragments were requested by the item before it
     int list_buf = 0;                // which of the small list buffers holds the current item's list, if prepared
     while (uni(cur.item) >= 0) {
         cur.item = uni(cur.item);
         const Desc nx2 = fetch(next_local());                    // in flight while this item runs
-        const int bh = cur.item / nqt;
-        const int qtile = cur.item % nqt;
+        const int bh = cur.item / L.by_tiles;
+        const int qtile = cur.item - bh * nqt;
         const int64_t qrow0 = (int64_t)qtile * kTile;
-        const int qblock = (int)(qrow0 / bs_q);
-        const int64_t o_bh = (int64_t)(bh / Hn) * L.o_st[0] + (int64_t)(bh % Hn) * L.o_st[1];
+        const int batch = bh / L.by_heads;
+        const int64_t o_bh = (int64_t)batch * L.o_st[0] + (int64_t)(bh - batch * Hn) * L.o_st[1];
+        // the token rows of an item that nothing has prepared: asked for beside its descriptor
+        int32_t first_rows[3] = {0, 0, 0};
+        if (!prepared && L.q_rows != nullptr) {
+            first_rows[0] = L.q_rows[qrow0 + lr];
+            first_rows[1] = L.q_rows[qrow0 + 32 + lr];
+            first_rows[2] = L.q_rows[qrow0 + lane];
+        }
+        __builtin_amdgcn_sched_barrier(0);
         const int nent = list_length(cur);
         npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
         if (!kBounded && parts.count > 1) {
-            const int part = cur.local / parts.items;
-            pair0 = (int)((int64_t)npairs * part / parts.count);
-            npairs = (int)((int64_t)npairs * (part + 1) / parts.count) - pair0;
+            const int part = cur.local / parts.by_items;        // at most kMaxParts: the products fit 32 bits
+            pair0 = npairs * part / parts.by_count;
+            npairs = npairs * (part + 1) / parts.by_count - pair0;
         }
         half_base = (uint32_t)uni((bh - bh_first) * tiles_bh) * 2u;
         // the next item can be prepared while this one runs if this one has a loop to hide it behind, the next one
@@ -562,29 +601,57 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         } else {
             beyond[0] = beyond[1] = half_base;
         }
-        const int nbh = prepare_next ? nxt.item / nqt : 0;
-        const int64_t nqrow0 = prepare_next ? (int64_t)(nxt.item % nqt) * kTile : 0;
-        const int32_t* nlist = idx + ((int64_t)nbh * nbq + nqrow0 / bs_q) * idx_stride;
+        const int nitem = prepare_next ? nxt.item : 0, nbh = nitem / L.by_tiles;
+        const int64_t nqrow0 = (int64_t)(nitem - nbh * nqt) * kTile;
+        const int32_t* nlist = idx + (int64_t)(nitem / L.by_block) * idx_stride;
 
+        const bool early = kBounded || parts.count == 1;         // the walk starts at the list's first entry
+        auto first_fragments = [&](uint32_t h0, uint32_t h1) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(h0, c);                       // K(0)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) kb[1][c] = k_frag(h1, c);                       // K(1)
+#pragma unroll
+            for (int f = 0; f < 8; ++f) vb[0][f] = v_frag(h0, f);                       // V_A(0), V_B(0)
+#pragma unroll
+            for (int f = 0; f < 4; ++f) vb[1][f] = v_frag(h1, f);                       // V_A(1)
+        };
         if (!prepared) {
-            // Q as the B operand of S^T: lane holds rows lr and 32 + lr, d = 16 c + 8 lh .. +8.  Requested before the
-            // list is staged, so that the two chains of dependent loads (row table -> Q rows, list -> LDS) run side by side.
-            const int64_t q_bh = (int64_t)(bh / Hn) * L.q_st[0] + (int64_t)(bh % Hn) * L.q_st[1];
-#pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                int64_t row = qrow0 + 32 * qq + lr;
-                if (L.q_rows != nullptr) row = max(L.q_rows[row], 0);          // padded slots read token 0, never stored
-                const T* qp = q + q_bh + row * L.q_st[2] + 8 * lh;
-                V8 rows[8];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) rows[c] = *reinterpret_cast<const V8*>(qp + 16 * c);
-                take_q(qq, rows);
-            }
-            const int32_t* list = idx + ((int64_t)bh * nbq + qblock) * idx_stride;
+            // Nothing of this item is on its way yet.  Everything that its first product waits for is asked for before any of
+            // it is waited for: the list, Q as the B operand of S^T (lane holds rows lr and 32 + lr, d = 16 c + 8 lh .. +8) and,
+            // where the walk starts at the list's first entry, which the descriptor holds, the first K and V fragments.
             int lane_now = lane;                                     // see the epilogue
             asm volatile("" : "+v"(lane_now));
-            if (L.q_rows != nullptr) out_rows[list_buf][lane_now] = L.q_rows[qrow0 + lane_now];
-            for (int e = lane_now; e < nent; e += 64) big[e] = (uint32_t)list[e];
+            const int32_t* list = idx + (int64_t)(cur.item / L.by_block) * idx_stride;
+            constexpr int kAhead = 4;
+            int32_t entry[kAhead] = {0, 0, 0, 0};
+            if (nent > 0) {
+#pragma unroll
+                for (int e = 0; e < kAhead; ++e) entry[e] = list[min(lane_now + 64 * e, nent - 1)];
+            }
+            const int64_t q_bh = (int64_t)batch * L.q_st[0] + (int64_t)(bh - batch * Hn) * L.q_st[1];
+            V8 rows[2][8];
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq) {
+                const int64_t row = L.q_rows != nullptr ? (int64_t)max(first_rows[qq], 0) : qrow0 + 32 * qq + lr;      // padded slots read token 0, never stored
+                const T* qp = q + q_bh + row * L.q_st[2] + 8 * lh;
+#pragma unroll
+                for (int c = 0; c < 8; ++c) rows[qq][c] = *reinterpret_cast<const V8*>(qp + 16 * c);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (early && npairs > 0) {
+                uint32_t h[2];
+                first_pair(cur, h);
+                first_fragments((uint32_t)uni((int)h[0]), (uint32_t)uni((int)h[1]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (L.q_rows != nullptr) out_rows[list_buf][lane_now] = first_rows[2];
+#pragma unroll
+            for (int e = 0; e < kAhead; ++e)
+                if (lane_now + 64 * e < nent) big[lane_now + 64 * e] = (uint32_t)entry[e];
+            for (int e = lane_now + 64 * kAhead; e < nent; e += 64) big[e] = (uint32_t)list[e];
+            take_q(0, rows[0]);
+            take_q(1, rows[1]);
             ents = big;
             __syncthreads();
         } else {
@@ -629,16 +696,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             // ---- prologue.  In flight when the loop starts: K(1), K(2), V_A(0), V_B(0), V_A(1); the ring slot of
             // V_B(1) holds zeros, which the first step multiplies with P = 0 (there is no step -1).  A prepared item
             // finds all of them but K(2) requested already (K(0) sits where K(2) belongs until S(0) has been issued).
-            if (!prepared) {
-#pragma unroll
-                for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(half0, c);                    // K(0)
-#pragma unroll
-                for (int c = 0; c < 8; ++c) kb[1][c] = k_frag(w_half[0], c);                // K(1)
-#pragma unroll
-                for (int f = 0; f < 8; ++f) vb[0][f] = v_frag(half0, f);                    // V_A(0), V_B(0)
-#pragma unroll
-                for (int f = 0; f < 4; ++f) vb[1][f] = v_frag(w_half[0], f);                // V_A(1)
-            }
+            if (!prepared && !early) first_fragments(half0, w_half[0]);
 #pragma unroll
             for (int f = 4; f < 8; ++f)
 #pragma unroll
@@ -720,7 +778,8 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 // and the token rows of its 64 query slots, which its epilogue stores through
                 if (L.q_rows != nullptr)
                     load_to_lds_4(L.q_rows + nqrow0, (uint32_t)lane * 4u, (uint32_t)uni((int)lds_address(&out_rows[list_buf ^ 1][0])));
-                const int64_t nq_bh = (int64_t)(nbh / Hn) * L.q_st[0] + (int64_t)(nbh % Hn) * L.q_st[1];
+                const int nbatch = nbh / L.by_heads;
+                const int64_t nq_bh = (int64_t)nbatch * L.q_st[0] + (int64_t)(nbh - nbatch * Hn) * L.q_st[1];
                 const char* qsrc = reinterpret_cast<const char*>(q + nq_bh);
 #pragma unroll
                 for (int qq = 0; qq < 2; ++qq) {
@@ -863,8 +922,8 @@ template <typename T>
 __global__ __launch_bounds__(256) void merge_parts_kernel(Parts parts, T* __restrict__ o, float* __restrict__ lse, int item_begin,
                                                           int nqt, int Hn, int64_t lse_S, FragLayout L) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 31, lh = lane >> 5;
-    const int item = item_at(L, item_begin + blockIdx.x, nqt), bh = item / nqt;
-    const int64_t qrow0 = (int64_t)(item % nqt) * kTile;
+    const int item = item_at(L, item_begin + blockIdx.x, nqt), bh = item / L.by_tiles;
+    const int64_t qrow0 = (int64_t)(item - bh * nqt) * kTile;
     const float* first = parts.buf + (int64_t)blockIdx.x * kPartFloats;
     const int64_t stride = (int64_t)parts.items * kPartFloats;
     float M[2] = {-INFINITY, -INFINITY}, inv[2] = {0.f, 0.f};
@@ -920,7 +979,7 @@ constexpr float kClassesPerOctave = 1.0f;
 // tiles in its L2.  The last workgroup clears the counters and chooses between rounds and queues: a round lasts as long as
 // its longest list, the queues keep every workgroup busy but walk out of step.
 constexpr int kPlanThreads = 1024, kPlanClasses = 12, kPlanRounds = 8192;
-__global__ __launch_bounds__(kPlanThreads) void queue_plan_kernel(const int32_t* __restrict__ lens, int tiles_per_block, int nqt, FragLayout L,
+__global__ __launch_bounds__(kPlanThreads) void queue_plan_kernel(const int32_t* __restrict__ lens, int nqt, FragLayout L,
                                                                   int total, int resident, int max_len, int32_t* __restrict__ order,
                                                                   uint32_t* __restrict__ queue) {
     __shared__ int sm[kPlanClasses * kPlanThreads];
@@ -928,7 +987,7 @@ __global__ __launch_bounds__(kPlanThreads) void queue_plan_kernel(const int32_t*
     __shared__ int longest_sm;
     __shared__ unsigned long long sum_sm;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    auto length_of = [&](int item) { return min(max(lens[item / tiles_per_block], 0), max_len); };
+    auto length_of = [&](int item) { return min(max(lens[item / L.by_block], 0), max_len); };
     auto wave_max = [](int x) {
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) x = max(x, __shfl_xor(x, off));
@@ -1096,6 +1155,11 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const int total = B * Hn * n_live;
     L.tiles = n_live < per_head ? q_rows + Sq : nullptr;
     L.n_live = n_live;
+    L.by_live = divisor(n_live);
+    L.by_tiles = divisor(per_head);
+    L.by_block = divisor(bs_q / kTile);
+    L.by_heads = divisor(Hn);
+    L.by_sub = divisor(bs_k / kTile);
     const uint32_t whole_span = one_span ? (uint32_t)((int64_t)B * Hn * kv_bh_bytes) : 0u;
     // the LDS DMA that brings the next item's Q rows forms its addresses from 32-bit row offsets
     const int64_t q_rows_max = q_rows != nullptr ? lse_rows : Sq;
@@ -1104,7 +1168,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     // the items it has to leave to the other kernel is given, and that kernel can reach every head from one buffer.
     // A call of one round runs the exact kernel alone: its steps are 3 % longer, but a last launch that finds nothing to do
     // costs 3.6 us, a fifth of a small call's attention.
-    Parts parts = {nullptr, 1, 0};
+    Parts parts = {nullptr, 1, 0, divisor(1), divisor(1)};
     const bool bounded = dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident;      // (see `whole` below)
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
@@ -1126,7 +1190,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     } while (0)
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
     if (queue != nullptr && one_span) {
-        hipLaunchKernelGGL(queue_plan_kernel, dim3(kQueues + 1), dim3(kPlanThreads), 0, st, lens, bs_q / kTile, per_head, L, total, resident, idx_stride,
+        hipLaunchKernelGGL(queue_plan_kernel, dim3(kQueues + 1), dim3(kPlanThreads), 0, st, lens, per_head, L, total, resident, idx_stride,
                            order, queue);
         gate = queue + kQueueChoice;
         const dim3 grid((unsigned)(total < resident ? total : resident));
@@ -1157,7 +1221,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         first = end;
     }
     if (n_parts > 1) {
-        parts = {part_buf, n_parts, tail};
+        parts = {part_buf, n_parts, tail, divisor(n_parts), divisor(tail)};
         const int n = tail * n_parts;
         const dim3 grid((unsigned)(n < resident ? n : resident));
         BSA_FRAG_LAUNCH(false, grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
@@ -1165,7 +1229,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
             hipLaunchKernelGGL((merge_parts_kernel<__bf16>), dim3(tail), dim3(256), 0, st, parts, (__bf16*)o, lse, whole, per_head, Hn, lse_rows, L);
         else
             hipLaunchKernelGGL((merge_parts_kernel<_Float16>), dim3(tail), dim3(256), 0, st, parts, (_Float16*)o, lse, whole, per_head, Hn, lse_rows, L);
-        parts = {nullptr, 1, 0};
+        parts = {nullptr, 1, 0, divisor(1), divisor(1)};
     }
     if (bounded) {
         // what the schedule that ran left over, be it the rounds or the queues: as many items as the list holds,
