@@ -43,6 +43,34 @@ __host__ __device__ inline int live_query_tiles(const Grid3& g) { return live_ti
 // tiles that hold real rows, ascending.
 inline size_t row_table_ints(int64_t slots) { return (size_t)(slots + slots / 64); }
 
+// n / d for 0 <= n < 2^31 by a product: m = ceil(2^p / d) with p = 31 + ceil(log2 d), so m d - 2^p < d <= 2^(p - 31) and the error
+// n (m d - 2^p) / (d 2^p) of the quotient stays below 1 / d.  A division by a number that the compiler does not know costs
+// 25 (32 bits) to 120 instructions (64), one after another.
+struct Divisor {
+    uint32_t m, p;
+};
+inline Divisor divisor(int d) {
+    uint32_t l = 0;
+    while (((int64_t)1 << l) < d) ++l;
+    const uint32_t p = 31 + l;
+    return {(uint32_t)((((unsigned __int128)1 << p) + d - 1) / d), p};
+}
+__device__ __forceinline__ int operator/(int n, const Divisor& d) { return (int)(((uint64_t)(uint32_t)n * d.m) >> d.p); }
+
+// The compiler loads a kernel's arguments where it first needs them, a wait for memory for every cache line of them in front of
+// the first useful load of a launch.  Asked for together they cost one.  kBytes: of the arguments, at most 384.
+template <int kBytes>
+__device__ __forceinline__ void touch_arguments() {
+    static_assert(kBytes >= 4 && kBytes <= 384 && kBytes % 4 == 0, "");
+    uint32_t a, b, c, d, e, f;
+    constexpr int last = kBytes - 4;
+    asm volatile("s_load_dword %0, %6, %7\n\ts_load_dword %1, %6, %8\n\ts_load_dword %2, %6, %9\n\ts_load_dword %3, %6, %10\n\t"
+                 "s_load_dword %4, %6, %11\n\ts_load_dword %5, %6, %12\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&s"(a), "=&s"(b), "=&s"(c), "=&s"(d), "=&s"(e), "=&s"(f)
+                 : "s"(__builtin_amdgcn_kernarg_segment_ptr()), "i"(0), "i"(64 < last ? 64 : last), "i"(128 < last ? 128 : last),
+                   "i"(192 < last ? 192 : last), "i"(256 < last ? 256 : last), "i"(last));
+}
+
 // Where the rows of the attention operands live.  Blocked order: tile i of a (batch, head) is rows
 // 64*i .. 64*i+63 of a contiguous [B, Hn, S, D] tensor.  THW order: tile i is (a 64-slot part of)
 // chunk i of the grid and its slots are gathered from / scattered to token positions, so the

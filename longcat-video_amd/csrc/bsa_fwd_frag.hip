@@ -71,20 +71,6 @@ __device__ __forceinline__ float dot2_self(f16x8 x, int e, float acc) {
     return __builtin_amdgcn_fdot2(p, p, acc, false);
 }
 
-// n / d for 0 <= n < 2^31 by a product: m = ceil(2^p / d) with p = 31 + ceil(log2 d), so m d - 2^p < d <= 2^(p - 31) and the error
-// n (m d - 2^p) / (d 2^p) of the quotient stays below 1 / d.  A division by a number that the compiler does not know costs
-// 25 (32 bits) to 120 instructions (64), one after another, and an item has nine of them in front of its first product.
-struct Divisor {
-    uint32_t m, p;
-};
-static Divisor divisor(int d) {
-    uint32_t l = 0;
-    while (((int64_t)1 << l) < d) ++l;
-    const uint32_t p = 31 + l;
-    return {(uint32_t)((((unsigned __int128)1 << p) + d - 1) / d), p};
-}
-__device__ __forceinline__ int operator/(int n, const Divisor& d) { return (int)(((uint64_t)(uint32_t)n * d.m) >> d.p); }
-
 struct FragLayout {
     const int32_t* q_rows;        // token row of every blocked-order query slot, -1 = padding; null: q, o in blocked order
     int64_t q_st[3], o_st[3];     // element strides: batch, head, row
@@ -151,17 +137,6 @@ constexpr int kQueues = 8, kQueueChoice = kQueues, kQueueWords = kQueues + 1;   
 static_assert(kQueueWords <= kFragQueueWords, "the caller's buffer holds the words");
 __device__ __forceinline__ int section_begin(int n, int x) { return (int)(((int64_t)n * x) >> 3); }
 
-// The kernel's arguments fill six cache lines, and the compiler loads them where it first needs them: six waits for memory, one
-// after another, in front of a launch's first item.  Asked for together they cost one, 0.36 us for 0.7 to 1.1.  With what an item
-// that nothing has prepared now asks for at once (below) and the divisions that went, the kernel of a single round is 1.3 us
-// shorter: 15.1 -> 13.8 us for 5 heads of 9x27x12, 25.4 -> 24.2 for two prompts of 8 heads of 7x15x26.
-__device__ __forceinline__ void touch_arguments() {
-    uint32_t a, b, c, d, e, f;
-    asm volatile("s_load_dword %0, %6, 0x0\n\ts_load_dword %1, %6, 0x40\n\ts_load_dword %2, %6, 0x80\n\ts_load_dword %3, %6, 0xc0\n\t"
-                 "s_load_dword %4, %6, 0x100\n\ts_load_dword %5, %6, 0x13c\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&s"(a), "=&s"(b), "=&s"(c), "=&s"(d), "=&s"(e), "=&s"(f) : "s"(__builtin_amdgcn_kernarg_segment_ptr()));
-}
-
 template <typename T, int kWalk, bool kBounded>
 __global__ __launch_bounds__(64) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
@@ -185,7 +160,10 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     constexpr float kSlack = 60.0f;
     static_assert(!kBounded || std::is_same<T, __bf16>::value, "fp16 probabilities need the running maximum");
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    touch_arguments();
+    // six lines: 0.36 us for 0.7 to 1.1.  With what an item that nothing has prepared asks for at once (below) and the divisions
+    // that went, the kernel of a single round is 1.3 us shorter: 15.1 -> 13.8 us for 5 heads of 9x27x12, 25.4 -> 24.2 for two
+    // prompts of 8 heads of 7x15x26.
+    touch_arguments<320>();
     if (gate != nullptr && *gate != gate_want) return;
     // output staging: 64 rows of 256 B, 272 B apart.  The same memory stages a list that is too long for the small
     // buffers (kListEntries words at most) during the tile loop of an item that was not prepared ahead of time.

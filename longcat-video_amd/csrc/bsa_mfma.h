@@ -11,6 +11,7 @@ namespace mfma {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4_ __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 
@@ -49,6 +50,13 @@ __device__ inline void load_to_lds_16_once(const void* sbase, uint32_t voff, uin
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
                  :: "s"(lds_addr), "v"(voff), "s"(sbase) : "memory");
 }
+// Four of them, 1 KB apart on both sides (an instruction's offset counts for both addresses): load i reads
+// sbase + voff[i] + 1024 i.  One setting of m0 instead of four.
+__device__ inline void load_to_lds_4x16(const void* sbase, const uint32_t (&voff)[4], uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072"
+                 :: "s"(lds_addr), "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(sbase) : "memory");
+}
 // The same with 4 bytes per lane: the LDS address is m0 + 4*lane.
 __device__ inline void load_to_lds_4(const void* sbase, uint32_t voff, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
@@ -60,6 +68,14 @@ __device__ inline uint32_t lds_address(const void* p) {
 // 4 keys x 16 d patch -> this lane's d, 4 keys (see the header comment)
 __device__ inline s16x4 lds_read_tr16(const void* p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)p);
+}
+
+// LDS by address (lds_address): a constant that is added to the address goes into the instruction, which it does not when the
+// address is that of dynamic shared memory, a number the compiler learns too late.
+template <typename V>
+__device__ __forceinline__ V lds_read_at(uint32_t address) { return *(const __attribute__((address_space(3))) V*)(uintptr_t)address; }
+__device__ __forceinline__ s16x4 lds_read_tr16_at(uint32_t address) {
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(uintptr_t)address);
 }
 
 // S^T accumulators must sit in ordinary VGPRs, where the softmax reads them, while the (four times larger)
