@@ -1246,9 +1246,13 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         if (masked) BSA_BY_TYPE(BSA_DKDV, true, true);
         else BSA_BY_TYPE(BSA_DKDV, false, true);
     }
-    // from kept dS one launch: its stream is read once whatever the walks' pace (32 heads of 24x30x52: 1.81 ms by two rounds, 1.77 by
-    // five, 1.76 at once)
-    const int span = kept.keep ? total_q : 2 * round;
+    // One launch where a list may hold every block (the CDF rule), since rounds would wait for their longest list (dQ from
+    // scratch, 8 heads of 24x30x52, threshold 0.5, smooth inputs: 1.69 against 1.10 ms; random inputs, lists of one length: 2.46
+    // and 2.45), and from kept dS, whose stream is read once whatever the walks' pace, up to half of the blocks (density 1/16, 32
+    // heads of 24x30x52: 1.81 by two rounds, 1.76 at once; 1/4, 24 heads of 12x30x52: 1.32 and 1.31; 1/2, 12 heads: 1.27 and 1.28;
+    // every block, 8 heads of 12x32x48: 1.51 and 1.67, which lists of unequal length make up for).
+    const bool any_length = idx_stride >= nbk, once = any_length || (kept.keep && 2 * idx_stride < nbk);
+    const int span = once ? total_q : 2 * round;
     for (int first = 0; first < total_q; first += span) {
         const int end = first + span < total_q ? first + span : total_q;
         if (kept.keep) BSA_BY_TYPE(BSA_DQ_DS);

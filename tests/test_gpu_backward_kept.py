@@ -67,3 +67,23 @@ def test_without_room_for_ds(grid, chunk, monkeypatch):
     assert sizes[0][1] < sizes[0][0]
     assert torch.equal(dk0, dk1) and torch.equal(dv0, dv1)
     assert (dq0.float() - dq1.float()).norm() <= 2 * 2.0 ** -11 * dq1.float().norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_lists_of_any_length_run_in_one_launch(dtype, monkeypatch):
+    """2 304 query tiles and lists of 1 to 192 of 192 blocks, dQ from scratch: as wide as the blocks (one launch) and cut to the
+    longest list (rounds), bit for bit the same."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    lq, chunk, H = (12, 32, 32), (4, 4, 4), 12
+    S = lq[0] * lq[1] * lq[2]
+    g = torch.Generator("cuda").manual_seed(14)
+    q, k, v, do = (torch.randn(1, H, S, 128, generator=g, device="cuda").to(dtype) for _ in range(4))
+    lens = torch.randint(1, 40, (1, H, 192), generator=g, device="cuda", dtype=torch.int32)
+    lens[..., ::37] = 150
+    walk = torch.rand(1, H, 192, 192, generator=g, device="cuda").argsort(dim=-1).int()
+    walk[..., :150] = walk[..., :150].sort(dim=-1).values
+    o, lse = bi.ThwAttention(k, v, lq, lq, chunk, chunk)(q, walk, lens, return_lse=True)
+    monkeypatch.setattr(bi, "_backward_workspace", lambda need, least, device: torch.empty(least, dtype=torch.uint8, device=device))
+    wide, cut = (bi._bsa_3d_backward(do, q, k, v, o, lse, w, lens, lq, lq, chunk, chunk, 128 ** -0.5) for w in (walk, walk[..., :150].contiguous()))
+    for a, b in zip(wide, cut):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)
