@@ -1148,8 +1148,30 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     int32_t* place = reinterpret_cast<int32_t*>(ws + at.place);
     const int per_entry = (bs_q / kTile) * (bs_k / kTile);
 
+    // the dK / dV kernel's LDS: four stages of half a Q tile, half a dO tile and the queries' M2 / delta, then a KV block's query
+    // blocks; bwd_count_kernel has a bin for each of their numbers, less than that
+    const size_t lds = bwd_dkdv_lds_bytes(nbq);
+    if (lds > kBwdLdsLimit) return hipErrorInvalidValue;          // the C-ABI layer has rejected such a shape already
     const size_t count_lds = (size_t)(nbq + 1 > 4 ? nbq + 1 : 4) * sizeof(int);
-    if (count_lds > 64 * 1024) return hipErrorInvalidValue;      // bwd_count_kernel's bins: 16 383 query blocks
+    // Per device, once: the dK / dV instantiations and bwd_count_kernel may use all of the LDS, and the number of compute units.
+    static std::atomic<int> device_cus[64];
+    int dev = 0;
+    hipError_t e;
+    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+    if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
+    int cus = device_cus[dev].load(std::memory_order_acquire);
+    if (cus == 0) {
+        const void* kernels[9] = {
+            reinterpret_cast<const void*>(bwd_count_kernel),
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, false>),
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, true>),
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, false>),
+            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, true>)};
+        for (const void* kf : kernels)
+            if ((e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBwdLdsLimit)) != hipSuccess) return e;
+        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
+        device_cus[dev].store(cus, std::memory_order_release);   // threads racing here set the same attributes
+    }
     const int64_t qrows = (int64_t)bh * Sq, krows = (int64_t)bh * Sk, nwords = (int64_t)bh * nbk * words;
     const float c = sm_scale * kRcpLn2;
     BwdStore dq_to = {nullptr, 0, 0, 0, Hn}, dk_to = dq_to, dv_to = dq_to;
@@ -1189,7 +1211,6 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     }
     if (thw == nullptr) hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, bits, nwords);
     const int64_t lrows = (int64_t)bh * nbq;
-    hipError_t e;
     // dQ walks every list in the forward kernel's visiting order when the list is ascending (a selection in block
     // order); any other order is walked as given.  The order only moves fp32 roundings of the dQ sum.
     if ((e = launch_pace_order(idx, paced, lens, lrows, nbk, idx_stride, st, {}, {bits, nbq, words})) != hipSuccess) return e;
@@ -1197,27 +1218,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
                        bs_k / kTile, per_entry);
 
     const dim3 block(64);
-    // the dK / dV kernel's LDS: four stages of half a Q tile, half a dO tile and the queries' M2 / delta, then a KV block's query blocks
-    const size_t lds = bwd_dkdv_lds_bytes(nbq);
-    if (lds > kBwdLdsLimit) return hipErrorInvalidValue;          // the C-ABI layer has rejected such a shape already
     const bool masked = tile_valid != nullptr;
-    // Per device, once: the dK / dV instantiations may use all of the LDS, and the number of compute units.
-    static std::atomic<int> device_cus[64];
-    int dev = 0;
-    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-    if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
-    int cus = device_cus[dev].load(std::memory_order_acquire);
-    if (cus == 0) {
-        const void* kernels[8] = {
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, false>),
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, true>),
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, false>),
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, true>)};
-        for (const void* kf : kernels)
-            if ((e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBwdLdsLimit)) != hipSuccess) return e;
-        if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
-        device_cus[dev].store(cus, std::memory_order_release);   // threads racing here set the same attributes
-    }
     // dQ from scratch: rounds of as many wavefronts as the device runs at once (one per SIMD), two rounds per launch.  The dK / dV
     // kernel runs as one grid, longest list first: its lists (the query blocks of a KV block) differ in length, and
     // rounds that wait for the longest list cost more than they bring.

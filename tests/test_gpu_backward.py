@@ -308,3 +308,27 @@ def test_key_blocks_are_counted_and_sorted(lq, chunk, sparsity):
     args = (do, q, k, v, o, lse, walk, lens, lq, lq, chunk, chunk, 128 ** -0.5)
     for a, b in zip(bi._bsa_3d_backward(*args), bi._bsa_3d_backward_by_rearranging(*args)):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+def test_more_query_blocks_than_64_kb_of_bins():
+    """20 000 query blocks over two KV blocks of 64 keys, one head: bwd_count_kernel's bins take 80 KB.  Lists of both blocks and of
+    the first alone, so that the counts differ.  Against fp32 products of the same tensors; the tolerance of the roundings
+    of p, ds (an ulp each, relative to a row's terms) and of the result."""
+    g = torch.Generator("cuda").manual_seed(15)
+    nbq, sm = 20000, 128 ** -0.5
+    q, do = (torch.randn(1, 1, nbq * 64, 128, generator=g, device="cuda").bfloat16() for _ in range(2))
+    k, v = (torch.randn(1, 1, 128, 128, generator=g, device="cuda").bfloat16() for _ in range(2))
+    idx = torch.arange(2, device="cuda", dtype=torch.int32).expand(1, 1, nbq, 2).contiguous()
+    lens = 1 + (torch.arange(nbq, device="cuda", dtype=torch.int32) % 3 == 0).int().view(1, 1, nbq)
+    bi = I()
+    o, lse = bi.attn_fwd_bsa_varlen(q, k, v, sm, idx, lens, 64, 64)
+    dq, dk, dv = (torch.full_like(t, float("nan")) for t in (q, k, v))
+    bi.attn_bwd_bsa_varlen(do, q, k, v, o, dq, dk, dv, sm, lse, idx, lens, 64, 64)
+    qf, kf, vf, dof = (t[0, 0].float() for t in (q, k, v, do))
+    s = qf @ kf.T * sm
+    s.view(nbq, 64, 128)[lens.view(-1) == 1, :, 64:] = float("-inf")
+    p = s.softmax(-1)
+    dp = dof @ vf.T
+    ds = p * (dp - (p * dp).sum(-1, keepdim=True)) * sm
+    for got, want in ((dq, ds @ kf), (dk, ds.T @ qf), (dv, p.T @ dof)):
+        assert (got[0, 0].float() - want).norm() <= 2.0 ** -7 * want.norm()
