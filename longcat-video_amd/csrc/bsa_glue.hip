@@ -55,8 +55,12 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__
 // for 32 760 rows of 4 096, 2.6 TB/s of x and out).  A workgroup therefore holds them in LDS for kLnRows rows of a group
 // (in two planes of four, so that the lanes' 16-byte reads fall on different banks).  With a modulation row for every row
 // (kShared false) there is nothing to hold: 32 760 rows of 4 096 take 313 us from memory and 373 through LDS (from two rows
-// a group on LDS is the faster: 220 against 231).
-constexpr int kLnRows = 32;
+// a group on LDS is the faster: 220 against 231).  A wavefront's next row is requested before the sums over the one it holds (and
+// its first before the modulation is staged), and a workgroup takes few rows, since its staging hides behind the others'
+// rows and the last round of workgroups behind nothing.  us by rows a workgroup, 32 (rows requested when needed) / 32 / 16 / 8:
+// 32 760 rows of 4 096, 1 560 a group, 149 / 123 / 111 / 104 (5.2 TB/s); 24 960 rows 92 / 96 / 92 / 85; 86 400, 3 600 a group, 288 /
+// 287 / 271 / 260; 2 730 rows of 1 024, 390 a group, 12.8 / 12.9 / 7.9 / 5.7; 8 000 rows of 8 192, 500 a group, 116 / 64 / 56 / 59.
+constexpr int kLnRows = 8;
 template <typename T, int kPieces, bool kShared>        // 16-byte pieces of a row per lane: dim <= 512 kPieces
 __global__ __launch_bounds__(256, kPieces <= 8 ? 4 : 2) void layernorm_modulate_kernel(const T* __restrict__ x, const float* __restrict__ shift,
                                                                  const float* __restrict__ scale, T* __restrict__ out,
@@ -66,6 +70,14 @@ __global__ __launch_bounds__(256, kPieces <= 8 ? 4 : 2) void layernorm_modulate_
     const int group = blockIdx.x / per_group, row0 = (blockIdx.x - group * per_group) * kLnRows;
     const int64_t first = kShared ? (int64_t)group * rows_per_group + row0 : (int64_t)blockIdx.x * 4;
     const int n = kShared ? min(kLnRows, rows_per_group - row0) : (int)min((int64_t)4, rows - first), plane = dim / 2;
+    uint4 raw[kPieces], ahead[kPieces];         // a row stays in registers in its storage type; the wavefront's next one is on its way
+    auto request = [&](int r) {
+        const T* xr = x + (first + r) * dim + lane * 8;
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            if (j * 512 + lane * 8 < dim) ahead[j] = *reinterpret_cast<const uint4*>(xr + j * 512);
+    };
+    if (wave < n) request(wave);
     float* const sc = ln_lds;                    // scale + 1
     float* const sh = ln_lds + dim;
     auto plus_one = [](float4 a) { return make_float4(__fadd_rn(a.x, 1.0f), __fadd_rn(a.y, 1.0f), __fadd_rn(a.z, 1.0f), __fadd_rn(a.w, 1.0f)); };
@@ -79,12 +91,10 @@ __global__ __launch_bounds__(256, kPieces <= 8 ? 4 : 2) void layernorm_modulate_
     }
     for (int r = wave; r < n; r += 4) {
         const int64_t row = first + r;
-        const T* xr = x + row * dim;
-        uint4 raw[kPieces];                     // the row stays in registers in its storage type
         float sum = 0.f;
 #pragma unroll
-        for (int j = 0; j < kPieces; ++j)
-            if (j * 512 + lane * 8 < dim) raw[j] = *reinterpret_cast<const uint4*>(xr + j * 512 + lane * 8);
+        for (int j = 0; j < kPieces; ++j) raw[j] = ahead[j];
+        if (r + 4 < n) request(r + 4);
 #pragma unroll
         for (int j = 0; j < kPieces; ++j)
             if (j * 512 + lane * 8 < dim) {

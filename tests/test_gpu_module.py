@@ -503,9 +503,9 @@ def test_workgroups_of_several_heads(Hn, dtype, cond):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("frames,per,dim", [(3, 1, 8), (2, 33, 2048), (2, 32, 2056), (1, 31, 4096), (3, 70, 4104), (2, 5, 8192)])
+@pytest.mark.parametrize("frames,per,dim", [(3, 1, 8), (2, 33, 2048), (2, 32, 2056), (1, 31, 4096), (3, 70, 4104), (2, 5, 8192), (2, 8, 512), (2, 9, 4096), (1, 4, 64)])
 def test_layernorm_modulate_sizes(dtype, frames, per, dim):
-    """Rows per frame around a workgroup's 32, rows around the 2 048 and 4 096 that change the instantiation: within one
+    """Rows per frame around a workgroup's eight and its wavefronts' two, rows around the 2 048 and 4 096 that change the instantiation: within one
     ulp of the fp32 expression (one rounding at the end)."""
     g = torch.Generator().manual_seed(dim)
     x = torch.randn(2, frames * per, dim, generator=g).to(dtype)
