@@ -85,15 +85,22 @@ __global__ __launch_bounds__(256) void bwd_rows_kernel(const T* __restrict__ o, 
 }
 
 // k_s = k * c, rounded once to the storage type (the product is formed in fp32, as torch does for a tensor times
-// a Python scalar).
+// a Python scalar).  Padded keys' rows (bits of tile_valid, optional, a word for 64 of a head's Sk keys) become zeros, whatever k
+// holds there: the kernels start their products from -inf, and an infinite product would make a NaN of that.
 template <typename T>
-__global__ __launch_bounds__(256) void bwd_scale_kernel(const T* __restrict__ k, T* __restrict__ ks, float c, int64_t n8) {
+__global__ __launch_bounds__(256) void bwd_scale_kernel(const T* __restrict__ k, T* __restrict__ ks, float c, int64_t n8,
+                                                        const uint64_t* __restrict__ tile_valid, uint32_t Sk) {
     typedef typename Vec8<T>::type V8;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n8) return;
     V8 x = *reinterpret_cast<const V8*>(k + i * 8);
+    bool real = true;
+    if (tile_valid != nullptr) {
+        const uint32_t key = (uint32_t)(i >> 4) % Sk;              // all heads' rows fit 32 bits: 2^32 of them would be a terabyte
+        real = (tile_valid[key / kTile] >> (key % kTile)) & 1ull;
+    }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * c);
+    for (int e = 0; e < 8; ++e) x[e] = real ? (T)((float)x[e] * c) : (T)0.f;
     *reinterpret_cast<V8*>(ks + i * 8) = x;
 }
 
@@ -910,7 +917,8 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     // NEXT half (into a second pair of accumulators) are issued between the exponentials of this one.  S and dP
     // accumulate in ordinary registers, where the exponentials read them: MFMAs from inline assembly, behind which
     // the compiler adds no wait states - a pair is read a whole group of 16 MFMAs after it was written.
-    // the queries' M2 as this lane's key sees them: -inf for a padded key, whose chains then give p = exp2(-inf) = 0
+    // the queries' M2 as this lane's key sees them: -inf for a padded key, whose chains (its row of k_s is zeros) then give
+    // p = exp2(-inf) = 0
     uint32_t numbers = lds0 + (uint32_t)(kBwdNumbers + 16 * lh), m2_at = numbers + (kMasked && !key_ok ? 256u : 0u);
     auto starts = [&](int stage, f32x16& from_m, f32x16& from_d) {
 #pragma unroll
@@ -1060,8 +1068,8 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
                     T xk[4], xv[4];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        xk[j] = (T)(acc_dk[t][4 * g4 + j] * dk_scale);
-                        xv[j] = (T)acc_dv[t][4 * g4 + j];
+                        xk[j] = kMasked && !key_ok ? (T)0.f : (T)(acc_dk[t][4 * g4 + j] * dk_scale);
+                        xv[j] = kMasked && !key_ok ? (T)0.f : (T)acc_dv[t][4 * g4 + j];
                     }
                     *reinterpret_cast<uint2*>(out_k + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(xk);
                     *reinterpret_cast<uint2*>(out_v + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(xv);
@@ -1202,12 +1210,12 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         hipLaunchKernelGGL((bwd_rows_kernel<__bf16>), dim3((unsigned)((qrows + 15) / 16)), dim3(256), 0, st, (const __bf16*)o,
                            (const __bf16*)dout, lse, delta, m2, qrows);
         hipLaunchKernelGGL((bwd_scale_kernel<__bf16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
-                           (const __bf16*)k, (__bf16*)ks, c, krows * 16);
+                           (const __bf16*)k, (__bf16*)ks, c, krows * 16, tile_valid, (uint32_t)Sk);
     } else {
         hipLaunchKernelGGL((bwd_rows_kernel<_Float16>), dim3((unsigned)((qrows + 15) / 16)), dim3(256), 0, st, (const _Float16*)o,
                            (const _Float16*)dout, lse, delta, m2, qrows);
         hipLaunchKernelGGL((bwd_scale_kernel<_Float16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
-                           (const _Float16*)k, (_Float16*)ks, c, krows * 16);
+                           (const _Float16*)k, (_Float16*)ks, c, krows * 16, tile_valid, (uint32_t)Sk);
     }
     if (thw == nullptr) hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, bits, nwords);
     const int64_t lrows = (int64_t)bh * nbq;

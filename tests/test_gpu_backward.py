@@ -99,6 +99,31 @@ def test_padded_keys_and_rows_without_keys():
     assert torch.all(dq[0, 0, 128:192] == 0)
 
 
+@pytest.mark.parametrize("fill", [3e38, float("inf"), float("nan")])
+@pytest.mark.parametrize("bs_k", [64, 128])
+@pytest.mark.parametrize("keep_ds", [True, False])
+def test_rows_of_padded_keys_may_hold_anything(fill, bs_k, keep_ds, monkeypatch):
+    """K rows of padded keys whose products with q are infinite or no numbers: the bits that zeros there give, zero gradients for
+    them, with dS kept and from scratch."""
+    bi = I()
+    if not keep_ds:
+        monkeypatch.setattr(bi, "_backward_workspace", lambda need, least, device: torch.empty(least, dtype=torch.uint8, device=device))
+    q, k, v, do, idx, lens = make_case(9, 2, 6, 4, 3, torch.bfloat16, bs_k=bs_k, min_len=1)
+    q = q * 16                                        # the rows of fill * 128 ** -0.5 * log2(e) overflow fp32 in a product
+    Sk = k.shape[2]
+    valid = torch.ones(Sk, dtype=torch.bool)
+    valid[Sk - 70:] = False                           # a tile without keys, one with 58
+    valid[17:49] = False                              # across a wavefront's 32 keys
+    k[:, :, ~valid] = 0
+    want = run_gpu(q, k, v, do, idx, lens, 64, bs_k, 128 ** -0.5, words_of(valid))
+    k[:, :, ~valid] = fill
+    got = run_gpu(q, k, v, do, idx, lens, 64, bs_k, 128 ** -0.5, words_of(valid))
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert all(torch.isfinite(a.float()).all() for a in got[2:])
+    assert not got[3][:, :, ~valid].any() and not got[4][:, :, ~valid].any()
+
+
 def test_medium_case_against_autograd():
     """40 x 40 blocks, density 1/4: against the gradients of fp32 masked-dense attention."""
     sm = 1 / math.sqrt(128)
