@@ -276,8 +276,9 @@ int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const vo
  * every tensor left in (T, H, W) token order.  Same arithmetic and rounding points as bsa_bwd.
  *   q, o, d_o, dq [B, Hn, Tq*Hq*Wq, D] and k, v, dk, dv [B, Hn, Tk*Hk*Wk, D]: element strides as in bsa_fwd_3d,
  *   bf16 / fp16, D == 128, 16-byte aligned; lse [B, Hn, Tq*Hq*Wq] fp32 contiguous and idx [B, Hn, nbq, idx_stride],
- *   lens [B, Hn, nbq] as bsa_fwd_3d_lse returned them (blocks counted in the padded chunk grids).  p->k_sel and
- *   p->cdf_threshold are not read.  Padded keys give and get no gradient; dq, dk, dv are written at every token.
+ *   lens [B, Hn, nbq] as bsa_fwd_3d_lse returned them (blocks counted in the padded chunk grids).  p->k_sel is not
+ *   read; p->cdf_threshold > 0 says that the lists differ in length, which only decides how the dQ kernel is launched.
+ *   Padded keys give and get no gradient; dq, dk, dv are written at every token.
  *   workspace: bsa_bwd_3d_workspace_bytes() bytes, 256-byte aligned: blocked-order copies of q, v and d_o (the kernels
  *   stream their tiles as they lie in memory), the row tables of both grids, and bsa_bwd's workspace.  o, d_o, lse
  *   and k are read through the row tables by the passes that take delta and the scaled k, and the kernels store the

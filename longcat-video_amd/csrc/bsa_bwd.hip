@@ -1137,7 +1137,7 @@ size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int 
 hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,
                       const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv,
                       int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
-                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw) {
+                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw, bool unequal) {
     const size_t bh = (size_t)B * Hn;
     KeptDs kept = plan_ds((int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
     kept.keep = kept.keep && bwd_ws(kept, (int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride).total <= workspace_bytes;
@@ -1255,12 +1255,16 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         if (masked) BSA_BY_TYPE(BSA_DKDV, true, true);
         else BSA_BY_TYPE(BSA_DKDV, false, true);
     }
-    // One launch where a list may hold every block (the CDF rule), since rounds would wait for their longest list (dQ from
-    // scratch, 8 heads of 24x30x52, threshold 0.5, smooth inputs: 1.69 against 1.10 ms; random inputs, lists of one length: 2.46
-    // and 2.45), and from kept dS, whose stream is read once whatever the walks' pace, up to half of the blocks (density 1/16, 32
-    // heads of 24x30x52: 1.81 by two rounds, 1.76 at once; 1/4, 24 heads of 12x30x52: 1.32 and 1.31; 1/2, 12 heads: 1.27 and 1.28;
-    // every block, 8 heads of 12x32x48: 1.51 and 1.67, which lists of unequal length make up for).
-    const bool any_length = idx_stride >= nbk, once = any_length || (kept.keep && 2 * idx_stride < nbk);
+    // One launch for lists that the caller declares unequal, since rounds would wait for their longest list: the whole backward by
+    // rounds / at once, us, smooth inputs, from kept dS 8 heads of 12x32x48 at threshold 0.75 (28 to 89 of 288 blocks) 1 027 / 982,
+    // at 0.5 (28 to 42) 607 / 600, from scratch 8 heads of 24x30x52 at 0.5 (62 to 185 of 624) 3 438 / 2 848; random inputs (141
+    // and 142 of 288) 2 329 / 2 378 and (307 to 309) 10 227 / 10 286.
+    // From kept dS, whose stream is read once whatever the walks' pace, also up to half of the blocks (dQ alone, ms, density 1/16, 32
+    // heads of 24x30x52: 1.81 by two rounds, 1.76 at once; 1/4, 24 heads of 12x30x52: 1.32 and 1.31; 1/2, 12 heads: 1.27 and 1.28);
+    // equal lists of every block keep their rounds (8 heads of 12x32x48 4 655 / 4 793, of 4 heads 2 789 / 2 770).  From scratch a list
+    // as wide as the blocks may be of any length, and where all are full it makes no difference (24 heads of 12x32x48 13 576 /
+    // 13 463, 2 of 24x45x80 27 916 / 27 980).
+    const bool once = unequal || (kept.keep ? 2 * idx_stride < nbk : idx_stride >= nbk);
     const int span = once ? total_q : 2 * round;
     for (int first = 0; first < total_q; first += span) {
         const int end = first + span < total_q ? first + span : total_q;

@@ -960,7 +960,7 @@ int bsa_bwd_3d(const bsa_3d_params* p, const void* q, const int64_t q_strides[3]
     }
     const hipError_t e = launch_bwd(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, idx, lens, kv_padded(p) ? t.valid : nullptr, nullptr, nullptr, nullptr,
                                     p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype,
-                                    ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t);
+                                    ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t, p->cdf_threshold > 0.f);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "bwd_3d launch");
 }
 

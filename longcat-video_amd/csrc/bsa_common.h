@@ -305,9 +305,10 @@ struct BwdThw {
     void* dk; int64_t dk_st[3];
     void* dv; int64_t dv_st[3];
 };
+// unequal: the lists may differ much in length (for the schedule of dQ alone).
 hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,
                       const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv,
                       int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
-                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw = nullptr);
+                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw = nullptr, bool unequal = false);
 
 }  // namespace bsa

@@ -720,21 +720,22 @@ class _Bsa3dWithGrad(torch.autograd.Function):
         o, walk, lens, lse = _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
                                      cdf_threshold=cdf_threshold, for_backward=True)
         ctx.save_for_backward(q, k, v, o, lse, walk, lens)
-        ctx.args = (tuple(latent_shape_q), tuple(latent_shape_k), tuple(chunk_q), tuple(chunk_k), 1 / q.shape[-1] ** 0.5)
+        ctx.args = (tuple(latent_shape_q), tuple(latent_shape_k), tuple(chunk_q), tuple(chunk_k), 1 / q.shape[-1] ** 0.5,
+                    cdf_threshold is not None)
         return o
 
     @staticmethod
     def backward(ctx, do):
         q, k, v, o, lse, walk, lens = ctx.saved_tensors
-        latent_q, latent_k, chunk_q, chunk_k, sm_scale = ctx.args
-        return _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_q, chunk_k, sm_scale) + (None,) * 6
+        return _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, *ctx.args) + (None,) * 6
 
 
 @functools.lru_cache(maxsize=256)
-def _plan_3d_backward(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, sm_scale, width):
+def _plan_3d_backward(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, sm_scale, width, unequal_lengths=False):
     """C-ABI parameters of a backward call and the most and the least workspace it takes."""
     lib = _capi.load()
-    prm = C.byref(_capi.Bsa3dParams(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, 0, sm_scale, 0.0))
+    prm = C.byref(_capi.Bsa3dParams(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk, wk, 0, sm_scale,
+                                    1.0 if unequal_lengths else 0.0))
     need = lib.bsa_bwd_3d_workspace_bytes(prm, width)
     if need == 0:        # the call itself names what is wrong with the shape
         _capi.check(lib.bsa_bwd_3d(prm, *([None] * 10), None, None, None, width, *([None] * 6), None, 0, None), "bsa_bwd_3d")
@@ -742,15 +743,17 @@ def _plan_3d_backward(B, H, D, code, Tq, Hq, Wq, Tk, Hk, Wk, tq, hq, wq, tk, hk,
     return prm, need, lib.bsa_bwd_3d_workspace_least_bytes(prm, width)
 
 
-def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_q, chunk_k, sm_scale):
+def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_q, chunk_k, sm_scale, unequal_lengths=False):
     """bsa_bwd_3d: dq, dk, dv in token order from token-order tensors (bsa_interface.py:570-596 between the
-    rearrangements of :650-652 and :659, of which only those of q and v are made, inside the call)."""
+    rearrangements of :650-652 and :659, of which only those of q, v and do are made, inside the call).  unequal_lengths: the
+    lists come from the CDF rule (for the schedule alone)."""
     _need_gpu(do, q, k, v, o)
     B, H, Sq, D = q.shape
     lib = _capi.load()
     q, k, v, o, do = (_rows_ok(t) for t in (q, k, v, o, do))
     width = walk.shape[3]
-    prm, need, least = _plan_3d_backward(B, H, D, _code(q), *latent_q, *latent_k, *chunk_q, *chunk_k, float(sm_scale), width)
+    prm, need, least = _plan_3d_backward(B, H, D, _code(q), *latent_q, *latent_k, *chunk_q, *chunk_k, float(sm_scale), width,
+                                         unequal_lengths)
     ws = _backward_workspace(need, least, q.device)
     dq, dk, dv = (torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in (q, k, v))
     lse, walk, lens = lse.contiguous(), walk.contiguous(), lens.contiguous()

@@ -1,4 +1,5 @@
 """dQ from the dS that the dK / dV kernel keeps, against dQ from scratch."""
+import ctypes
 import math
 
 import pytest
@@ -87,3 +88,57 @@ def test_lists_of_any_length_run_in_one_launch(dtype, monkeypatch):
     wide, cut = (bi._bsa_3d_backward(do, q, k, v, o, lse, w, lens, lq, lq, chunk, chunk, 128 ** -0.5) for w in (walk, walk[..., :150].contiguous()))
     for a, b in zip(wide, cut):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
+def launches(f):
+    """Nodes of the graph that a capture of f gives: its kernel launches."""
+    f()                                              # set-up of the device, outside the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        f()
+    hip = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64.so" in line)
+    n = ctypes.c_size_t(0)
+    count = ctypes.CDLL(hip).hipGraphGetNodes
+    count.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_size_t)]
+    assert count(graph.raw_cuda_graph(), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+def test_launches_follow_the_rule_not_the_width(monkeypatch):
+    """2 560 query tiles and every block kept, dS kept: rounds (two launches of dQ) for the top-k rule, whose lists are equal, one
+    launch for the CDF rule, whose lists may be as wide; the same bits."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    lq, chunk, H = (8, 16, 16), (4, 4, 4), 80
+    S = lq[0] * lq[1] * lq[2]
+    g = torch.Generator("cuda").manual_seed(16)
+    q, k, v = (torch.randn(1, H, S, 128, generator=g, device="cuda").bfloat16().requires_grad_() for _ in range(3))
+    do = torch.randn(1, H, S, 128, generator=g, device="cuda").bfloat16()
+    calls, backward = [], bi._bsa_3d_backward
+    monkeypatch.setattr(bi, "_bsa_3d_backward", lambda *a: calls.append(a) or backward(*a))
+    grads = [torch.autograd.grad(bi.flash_attn_bsa_3d(q, k, v, lq, lq, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk, **rule), (q, k, v), do)
+             for rule in (dict(sparsity=0.0), dict(sparsity=0.0, cdf_threshold=0.5))]
+    with torch.no_grad():
+        counts = [launches(lambda: backward(*a)) for a in calls]      # noqa: B023
+    assert counts[0] == counts[1] + 1, counts
+    assert all(torch.isfinite(a.float()).all() and torch.equal(a, b) for a, b in zip(*grads))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_kept_ds_in_rounds_and_in_one_launch(dtype):
+    """2 304 query tiles and lists of 1 to 150 of 192 blocks, dS kept: declared unequal (one launch) and not (rounds), as wide as the
+    blocks and cut to the longest list, bit for bit the same."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    lq, chunk, H = (12, 32, 32), (4, 4, 4), 12
+    S = lq[0] * lq[1] * lq[2]
+    g = torch.Generator("cuda").manual_seed(17)
+    q, k, v, do = (torch.randn(1, H, S, 128, generator=g, device="cuda").to(dtype) for _ in range(4))
+    lens = torch.randint(1, 40, (1, H, 192), generator=g, device="cuda", dtype=torch.int32)
+    lens[..., ::37] = 150
+    walk = torch.rand(1, H, 192, 192, generator=g, device="cuda").argsort(dim=-1).int()
+    walk[..., :150] = walk[..., :150].sort(dim=-1).values
+    o, lse = bi.ThwAttention(k, v, lq, lq, chunk, chunk)(q, walk, lens, return_lse=True)
+    runs = [bi._bsa_3d_backward(do, q, k, v, o, lse, w, lens, lq, lq, chunk, chunk, 128 ** -0.5, unequal)
+            for w in (walk, walk[..., :150].contiguous()) for unequal in (False, True)]
+    for run_ in runs[1:]:
+        assert all(torch.isfinite(a.float()).all() and torch.equal(a, b) for a, b in zip(run_, runs[0]))
