@@ -448,12 +448,15 @@ constexpr int64_t kOneLaunchGroups = 20480;
 // the loads in front and by 2 404 / 337, 4 362 / 307, 8 352 / 295, 16 354 / 297; with fewer registers (row_part) 8 317 / 275 = 4.6 and
 // 5.1 TB/s.  Calls of fewer chunks than kGroupedChunks keep the workgroups instead, and rows as they are gain nothing (229
 // by one head, 253 by four).
+// The launch of k is held to the registers of five wavefronts a SIMD, but not the form with a cache, which would spill three: held /
+// as it is, this launch takes 179 / 169 us for 32 heads of 24x30x52 behind 4 cached frames, 140 / 142 for 16 behind 5, where five
+// wavefronts fit the call's workgroups into two whole rounds; the whole call 1 094 / 1 086 and 720 / 720, of 24x45x80 3 992 / 3 974.
 constexpr int kHeadsPerGroup = 8;
 constexpr int64_t kGroupedChunks = 8192;
 
 enum { kAllParts, kKeys, kValues, kQueries };
 template <bool kBf16, int kMode, int kPart>
-__global__ __launch_bounds__(256, kPart == kKeys && kMode != kPlain ? 5 : 1) void prepare_kernel(PrepArgs a, int wg_k, int wg_v, int64_t chunks_q) {
+__global__ __launch_bounds__(256, kPart == kKeys && kMode == kNorm ? 5 : 1) void prepare_kernel(PrepArgs a, int wg_k, int wg_v, int64_t chunks_q) {
     constexpr bool kTransform = kMode != kPlain;
     __shared__ __attribute__((aligned(16))) uint16_t tile[kPart == kQueries && !kTransform ? 8 : kTile * kPitchV];
     __shared__ float2 cs[kTransform && kPart != kValues ? 8 * 64 : 1];
