@@ -794,7 +794,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     extern __shared__ __attribute__((aligned(1024))) char bwd_lds[];
     const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    touch_arguments<256>();
+    touch_arguments<decltype(bwd_dkdv_kernel<T, kMasked, kKeep>)>();
     // items longest list first, every XCD on a contiguous run of each group of `round` (see launch_bwd); a scalar, and with it
     // all that is derived from it (left to the compiler, addresses of the loop were made scalars half by half)
     int item;

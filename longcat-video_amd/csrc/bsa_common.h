@@ -57,11 +57,24 @@ inline Divisor divisor(int d) {
 }
 __device__ __forceinline__ int operator/(int n, const Divisor& d) { return (int)(((uint64_t)(uint32_t)n * d.m) >> d.p); }
 
+// The bytes of a kernel's arguments, laid out one after another, each at its alignment.
+template <typename Kernel>
+struct ArgumentBytes;
+template <typename... A>
+struct ArgumentBytes<void(A...)> {
+    static constexpr int count() {
+        size_t at = 0;
+        ((at = (at + alignof(A) - 1) / alignof(A) * alignof(A) + sizeof(A)), ...);
+        return (int)((at + 3) / 4 * 4);
+    }
+};
+
 // The compiler loads a kernel's arguments where it first needs them, a wait for memory for every cache line of them in front of
-// the first useful load of a launch.  Asked for together they cost one.  kBytes: of the arguments, at most 384.
-template <int kBytes>
+// the first useful load of a launch.  Asked for together they cost one.  Kernel: the type of the kernel, of 384 bytes at most.
+template <typename Kernel>
 __device__ __forceinline__ void touch_arguments() {
-    static_assert(kBytes >= 4 && kBytes <= 384 && kBytes % 4 == 0, "");
+    constexpr int kBytes = ArgumentBytes<Kernel>::count();
+    static_assert(kBytes >= 4 && kBytes <= 384, "six cache lines are asked for");
     uint32_t a, b, c, d, e, f;
     constexpr int last = kBytes - 4;
     asm volatile("s_load_dword %0, %6, %7\n\ts_load_dword %1, %6, %8\n\ts_load_dword %2, %6, %9\n\ts_load_dword %3, %6, %10\n\t"

@@ -160,10 +160,11 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     constexpr float kSlack = 60.0f;
     static_assert(!kBounded || std::is_same<T, __bf16>::value, "fp16 probabilities need the running maximum");
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    // six lines: 0.36 us for 0.7 to 1.1.  With what an item that nothing has prepared asks for at once (below) and the divisions
+    // six lines: 0.36 us for the first five where one by one they took 0.7 to 1.1; with the sixth a call of two prompts of 8 heads,
+    // 7x15x26, takes 41.4 us for 41.9.  With what an item that nothing has prepared asks for at once (below) and the divisions
     // that went, the kernel of a single round is 1.3 us shorter: 15.1 -> 13.8 us for 5 heads of 9x27x12, 25.4 -> 24.2 for two
     // prompts of 8 heads of 7x15x26.
-    touch_arguments<320>();
+    touch_arguments<decltype(fwd_frag_kernel<T, kWalk, kBounded>)>();
     if (gate != nullptr && *gate != gate_want) return;
     // output staging: 64 rows of 256 B, 272 B apart.  The same memory stages a list that is too long for the small
     // buffers (kListEntries words at most) during the tile loop of an item that was not prepared ahead of time.

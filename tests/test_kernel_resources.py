@@ -42,3 +42,27 @@ def test_the_preparation_pass_stays_in_registers(code_objects):
     """It runs at the rate of a copy; a row's values through scratch memory would be another pass."""
     for symbol, entry in metadata(code_objects, "14prepare_kernel").items():
         assert number(entry, "vgpr_spill_count") == 0 and number(entry, "private_segment_fixed_size") == 0, symbol
+
+
+def asked_for_together(code_objects, symbol):
+    """Offsets of the first six scalar loads of one dword that stand in a row."""
+    for obj in code_objects:
+        text = subprocess.run([LLVM + "llvm-objdump", "-d", "--disassemble-symbols=" + symbol, obj], check=True, capture_output=True, text=True).stdout
+        run = []
+        for op, offset in re.findall(r"^\t(\S+)(?: s\d+, s\[\d+:\d+\], (0x[0-9a-f]+))?", text, re.M):
+            run = run + [int(offset, 16)] if op == "s_load_dword" and offset else []
+            if len(run) == 6:
+                return run
+    return []
+
+
+@pytest.mark.parametrize("name", ["15fwd_frag_kernel", "15bwd_dkdv_kernel"])
+def test_every_line_of_the_arguments_is_asked_for(code_objects, name):
+    """A 64-byte line of them that is left out is a wait for memory of its own; a load behind them may read past their segment."""
+    for symbol, entry in metadata(code_objects, name).items():
+        args = [(int(at), int(size)) for at, size, kind in re.findall(r"\.offset: +(\d+)\s+\.size: +(\d+)\s+\.value_kind: +(\S+)", entry)
+                if not kind.startswith("hidden")]
+        end = max(at + size for at, size in args)
+        asked = asked_for_together(code_objects, symbol)
+        assert asked and max(asked) + 4 <= end, (symbol, asked, end)
+        assert {at // 64 for at in asked} == set(range((end + 63) // 64)), (symbol, asked, end)
