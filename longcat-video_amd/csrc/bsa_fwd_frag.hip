@@ -536,7 +536,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     };
 
     // ---- the workgroup's items
-    Desc cur, nxt;
+    Desc cur = {-1, 0, {0, 0}, -1, INFINITY}, nxt = cur;
 #pragma unroll 1
     for (int i = 0; i < 2; ++i) {        // one copy of the code: a launch's first item pays for every line of it, cold
         cur = nxt;
