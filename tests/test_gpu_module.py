@@ -349,19 +349,20 @@ def test_lora_linear_random_inputs():
     assert (want - plain).abs().mean() > 10 * (got - want).abs().mean()      # the side branch is not lost in the tolerance
 
 
+@pytest.mark.parametrize("multiplier,alpha_scale", [(0.5, 0.5), (0.7, 1 / 3)])      # exact, and rounding at both scalings
 @pytest.mark.parametrize("M,r,n_sep,per", [
     (1, 16, 1, 64), (31, 48, 1, 192), (33, 128, 3, 128), (65, 64, 8, 64),       # edges of the 32 tokens of a turn and the 256 columns
     (700, 112, 1, 320), (40, 96, 5, 64),
-    (24700, 32, 1, 64),                                                        # more turns than workgroups
+    (24700, 32, 1, 64), (12400, 16, 1, 512),                                   # more turns than workgroups, one column block and two
     (50, 24, 1, 64), (50, 16, 2, 96), (50, 144, 1, 64),                        # not built in one pass: rank, slice, rank
 ])
-def test_lora_up_projection_and_sum(M, r, n_sep, per):
-    """Small integers are exact in every product and sum: the one-pass kernel, and the separate passes where it is not built,
-    give the oracle's bits, whole tokens and columns included.  An up weight that is a transposed view is read as it is."""
+def test_lora_up_projection_and_sum(M, r, n_sep, per, multiplier, alpha_scale):
+    """Small integers are exact in every product and its sum: the one-pass kernel, and the separate passes where it is not built,
+    give the oracle's bits, whole tokens and columns included, also where each scaling and the sum round.  An up weight that is a transposed view is read as it is."""
     g = torch.Generator().manual_seed(M + r)
     K, N = 64, n_sep * per
     x, w = (torch.randint(-2, 3, s, generator=g).bfloat16() for s in ((M, K), (N, K)))
-    br, term = _branch(g, K, N, r, n_sep, 0.5, r / 2, integers=True)
+    br, term = _branch(g, K, N, r, n_sep, multiplier, r * alpha_scale, integers=True)
     br.lora_down.mul_(0.25)                                                    # products of up to 2^12 quarters: 16 bits at most
     want = O.lora_linear(x, w, None, [term])
     br.to("cuda")
