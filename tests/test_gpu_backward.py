@@ -322,17 +322,34 @@ def test_argument_checks():
     ((12, 41, 50), (4, 4, 4), 0.9),         # 429 blocks: more than 256, words with a remainder, a ragged grid
     ((9, 17, 30), (4, 4, 8), 0.5),          # two tiles a block, tiles without rows
 ])
-def test_key_blocks_are_counted_and_sorted(lq, chunk, sparsity):
-    """The bit matrix, its counts, the prefix sums behind kept dS and the order of the key tiles, over few and many blocks: the
-    gradients of the rearranging route, and of a workspace without room for dS, bit for bit."""
+def test_key_blocks_are_counted_and_sorted(lq, chunk, sparsity, monkeypatch):
+    """The bit matrix, its counts, the prefix sums behind kept dS and the order of the key tiles, over few and many blocks.  dv of
+    every block of a head against fp32 products with the queries that list it (p and dv are rounded once each, 2^-11: a lost
+    block of queries would be far outside); dq from kept dS against dq from scratch, which walks the lists alone (tolerance as in
+    test_gpu_backward_kept.py); and the rearranging route bit for bit."""
     bi = I()
     H, S = 3, int(np.prod(lq))
     g = torch.Generator("cuda").manual_seed(12)
     q, k, v, do = (torch.randn(2, H, S, 128, generator=g, device="cuda").half() for _ in range(4))
     o, walk, lens, lse = bi._bsa_3d(q, k, v, lq, lq, sparsity, chunk, chunk, for_backward=True)
     args = (do, q, k, v, o, lse, walk, lens, lq, lq, chunk, chunk, 128 ** -0.5)
-    for a, b in zip(bi._bsa_3d_backward(*args), bi._bsa_3d_backward_by_rearranging(*args)):
+    dq, dk, dv = bi._bsa_3d_backward(*args)
+    for a, b in zip((dq, dk, dv), bi._bsa_3d_backward_by_rearranging(*args)):
         assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+    tokens = bi._slot_tokens(lq, chunk, "cuda").view(-1, int(np.prod(chunk)))
+    listed = torch.zeros(walk.shape[2], tokens.shape[0] + 1, dtype=torch.bool, device="cuda")      # the last column: behind a list's end
+    entry = torch.arange(walk.shape[3], device="cuda") < lens[1, 2, :, None]
+    listed.scatter_(1, torch.where(entry, walk[1, 2], tokens.shape[0]).long(), True)
+    qf, kf, vf, dof = (t[1, 2].float() for t in (q, k, v, do))
+    for j in range(tokens.shape[0]):
+        tq, tk = tokens[listed[:, j]].flatten(), tokens[j]
+        tq, tk = tq[tq >= 0], tk[tk >= 0]
+        p = torch.exp(qf[tq] @ kf[tk].T * 128 ** -0.5 - lse[1, 2, tq, None])
+        assert (dv[1, 2, tk].float() - p.T @ dof[tq]).norm() <= 2.0 ** -10 * (p.T @ dof[tq].abs()).norm(), j
+    monkeypatch.setattr(bi, "_backward_workspace", lambda need, least, device: torch.empty(least, dtype=torch.uint8, device=device))
+    dq0, dk0, dv0 = bi._bsa_3d_backward(*args)
+    assert torch.equal(dk0, dk) and torch.equal(dv0, dv)
+    assert (dq0.float() - dq.float()).norm() <= 2 * 2.0 ** -11 * dq.float().norm()
 
 
 def test_more_query_blocks_than_64_kb_of_bins():
