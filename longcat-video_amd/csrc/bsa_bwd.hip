@@ -93,14 +93,14 @@ __global__ __launch_bounds__(256) void bwd_scale_kernel(const T* __restrict__ k,
     typedef typename Vec8<T>::type V8;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= n8) return;
-    V8 x = *reinterpret_cast<const V8*>(k + i * 8);
-    bool real = true;
+    uint4 raw = *reinterpret_cast<const uint4*>(k + i * 8);
     if (tile_valid != nullptr) {
         const uint32_t key = (uint32_t)(i >> 4) % Sk;              // all heads' rows fit 32 bits: 2^32 of them would be a terabyte
-        real = (tile_valid[key / kTile] >> (key % kTile)) & 1ull;
+        keep_if(raw, (tile_valid[key / kTile] >> (key % kTile)) & 1ull);
     }
+    V8 x = __builtin_bit_cast(V8, raw);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = real ? (T)((float)x[e] * c) : (T)0.f;
+    for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * c);
     *reinterpret_cast<V8*>(ks + i * 8) = x;
 }
 
@@ -1068,8 +1068,10 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
                     T xk[4], xv[4];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        xk[j] = kMasked && !key_ok ? (T)0.f : (T)(acc_dk[t][4 * g4 + j] * dk_scale);
-                        xv[j] = kMasked && !key_ok ? (T)0.f : (T)acc_dv[t][4 * g4 + j];
+                        // padded keys' sums are replaced before the product, which fp16 would otherwise round with the conversion
+                        const float sum_k = kMasked && !key_ok ? 0.f : acc_dk[t][4 * g4 + j], sum_v = kMasked && !key_ok ? 0.f : acc_dv[t][4 * g4 + j];
+                        xk[j] = (T)(sum_k * dk_scale);
+                        xv[j] = (T)sum_v;
                     }
                     *reinterpret_cast<uint2*>(out_k + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(xk);
                     *reinterpret_cast<uint2*>(out_v + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(xv);

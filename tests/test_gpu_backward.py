@@ -226,6 +226,7 @@ def test_autograd_through_the_operator_with_the_cdf_rule():
     (torch.float16, (5, 9, 14), (5, 9, 14), (4, 4, 4), (4, 4, 4), False),
     (torch.bfloat16, (4, 8, 12), (8, 8, 12), (4, 4, 4), (4, 4, 8), False),      # fewer queries than keys, 128-token key chunks
     (torch.bfloat16, (7, 9, 17), (7, 9, 17), (4, 4, 8), (4, 4, 8), True),
+    (torch.float16, (19, 15, 56), (19, 15, 56), (4, 4, 4), (4, 4, 4), False),   # 12 million elements of k: a rounding of k_s that differs is met
 ])
 def test_the_token_order_backward_equals_the_rearranging_route(dtype, lq, lk, chunk_q, chunk_k, token_major):
     """bsa_bwd_3d reads o, dO, lse and k through the row tables and stores the gradients at their tokens; five
