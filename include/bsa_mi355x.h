@@ -204,8 +204,9 @@ int bsa_fwd_fragment(const void* q, const void* k, const void* v, const int32_t*
  *   row, and idx_out has that many columns.  workspace: bsa_workspace_bytes() bytes, 256-byte
  *   aligned.  idx_out/lens_out/score_out are optional copies for inspection
  *   (shapes as in bsa_score_topk).  With cdf_threshold the lists differ in length: the work is then also
- *   enqueued as one launch whose workgroups draw the query tiles longest list first, and a kernel decides
- *   from the lengths, on the device, whether that or the usual rounds of equal tiles run (bf16 / fp16).
+ *   enqueued as one launch whose workgroups draw the query tiles from a queue per XCD, in classes of list length,
+ *   longest first, and a kernel decides from the lengths, on the device, whether that or the usual rounds of
+ *   equal tiles run (bf16 / fp16).
  * For bf16 / fp16 no permuted copy of q, k, v or o is made: one pass over q and k
  * produces the pooled means (and the tables of bsa_thw_prepare), and the attention
  * kernel reads and writes THW order directly; k and v must then share one token
@@ -280,9 +281,9 @@ int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const vo
  *   read; p->cdf_threshold > 0 says that the lists differ in length, which only decides how the dQ kernel is launched.
  *   Padded keys give and get no gradient; dq, dk, dv are written at every token.
  *   workspace: bsa_bwd_3d_workspace_bytes() bytes, 256-byte aligned: blocked-order copies of q, v and d_o (the kernels
- *   stream their tiles as they lie in memory), the row tables of both grids, and bsa_bwd's workspace.  o, d_o, lse
- *   and k are read through the row tables by the passes that take delta and the scaled k, and the kernels store the
- *   gradient rows at their tokens: five of the eight rearrangements a caller of bsa_bwd would run are not made.
+ *   stream their tiles as they lie in memory), the row tables of both grids, and bsa_bwd's workspace.  One pass makes
+ *   the copies, the scaled k, delta and the tables from the tensors where they lie, and the kernels store the gradient
+ *   rows at their tokens: five of the eight rearrangements a caller of bsa_bwd would run are not made.
  */
 size_t bsa_bwd_3d_workspace_least_bytes(const bsa_3d_params* p, int idx_stride);      /* without the kept dS */
 size_t bsa_bwd_3d_workspace_bytes(const bsa_3d_params* p, int idx_stride);

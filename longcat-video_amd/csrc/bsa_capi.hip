@@ -636,7 +636,7 @@ int bsa_fwd_thw(const bsa_3d_params* p, const void* q, const int64_t q_strides[3
     BSA_TRY(check_kv_views(pl, k_strides, v_strides, "fwd_thw"));
     if (!lens || idx_stride < 0 || (!idx && idx_stride > 0)) return set_error(BSA_ERR_BAD_ARG, "fwd_thw: selection is missing");
     hipError_t e = hipSuccess;
-    // p->cdf_threshold > 0 declares lists of unequal length: work items by length, both schedules enqueued
+    // p->cdf_threshold > 0 declares lists of unequal length: both schedules are enqueued, and the LDS-tiled kernel draws its items by length
     if (pl.cdf && !pl.frag && idx_stride > 0)
         e = launch_order_by_length(lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, idx_stride, (hipStream_t)stream);
     if (e == hipSuccess)
@@ -704,7 +704,8 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
             BSA_HIP(launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st, halves), "visit order");
     }
     if (!pl.f32) {
-        // lists of unequal length: one launch whose workgroups draw the items, longest lists first
+        // lists of unequal length: a launch whose workgroups draw the items besides the rounds, for the LDS-tiled kernel longest list first
+        // (the fragment-order kernel's own plan kernel fills a queue per XCD)
         const bool by_half = w.halves != nullptr;
         const int32_t *walk = by_half ? w.halves : w.idx_sorted, *walk_lens = by_half ? w.half_lens : w.lens;
         const int walk_width = by_half ? pl.half_width : pl.sel_width;

@@ -16,7 +16,7 @@ constexpr int kMaxSlices = 8, kMaxRank = 128;
 constexpr int kCols = 256;           // output columns of a workgroup, 64 per wavefront
 constexpr int kRows = 32;              // tokens of a turn
 constexpr int kPitch = kCols + 8;    // elements between the staged rows
-constexpr int kGroups = 768;         // workgroups of a launch, about: three a CU (1 536: 543 us, 6 144: 595)
+constexpr int kGroups = 768;         // workgroups of a launch, about: three a CU (1 536: 543 us, 6 144: 595, sizes below); never more than turns
 
 struct UpSlices {
     const __bf16* w[kMaxSlices];     // [per, rank]
@@ -30,7 +30,10 @@ struct UpSlices {
 //
 // 32 760 tokens, rank 128, 12 288 columns in three slices and 4 096 in one: 537 us = 4.0 TB/s, for 943 us of up-projections
 // (hipBLASLt, 364) and lora_add_kernel (579) before.  64 tokens a turn, two workgroups a CU 631; org a turn ahead 566 (its
-// registers cost more than the wait).
+// registers cost more than the wait).  It is taken wherever it is built: one pass / separate ones, us, by tokens 1, 256, 4 096,
+// 32 760: 4 096 columns, rank 16 4.3 / 20.8, 4.0 / 20.7, 12.0 / 32.6, 86 / 242, rank 128 4.5 / 20.6, 6.0 / 20.4, 22.8 / 29.3, 120 / 230;
+// 12 288 in three, rank 16 4.0 / 41, 4.8 / 41, 33 / 85, 310 / 701, rank 128 4.5 / 41, 9.5 / 41, 50 / 80, 369 / 675; 512 columns, rank 128,
+// 4.4 / 20.4, 5.7 / 20.2, 6.4 / 20.3, 23.7 / 31.4 (below 30 us the separate ones wait for the host).
 template <int kSteps>
 __global__ __launch_bounds__(256, 3) void lora_up_add_kernel(const __bf16* org, const __bf16* __restrict__ t, int64_t ldt, UpSlices up,
                                                              float multiplier, float alpha, __bf16* out, int64_t M, int N, int col_blocks,

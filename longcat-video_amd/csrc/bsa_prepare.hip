@@ -446,8 +446,10 @@ constexpr int64_t kOneLaunchGroups = 20480;
 // the same for all of them, and a head's rows are on their way while the one before it is transformed and written.  By heads to a
 // workgroup (32 heads of 24x45x80, k / q, us): 1 445 / 392 (a workgroup's loads behind its look-up of the angles), then with
 // the loads in front and by 2 404 / 337, 4 362 / 307, 8 352 / 295, 16 354 / 297; with fewer registers (row_part) 8 317 / 275 = 4.6 and
-// 5.1 TB/s.  Calls of fewer chunks than kGroupedChunks keep the workgroups instead, and rows as they are gain nothing (229
-// by one head, 253 by four).
+// 5.1 TB/s.  Rows as they are gain nothing (229 by one head, 253 by four).  Calls of fewer chunks than kGroupedChunks keep the
+// workgroups instead; the whole operator at that line, sparsity 0.985, us by one head / by eight, which also brings more calls into
+// one launch: 4 160 chunks of k 181 / 174, 6 656 267 / 252, 8 320 422 / 394, 9 984 492 / 453, 13 312 642 / 605, 19 968 1 128 / 1 089; behind four
+// cached frames 4 160 136 / 136, 6 656 270 / 260, 8 320 360 / 320, 13 312 555 / 513.
 // The launch of k is held to the registers of five wavefronts a SIMD, but not the form with a cache, which would spill three: held /
 // as it is, this launch takes 179 / 169 us for 32 heads of 24x30x52 behind 4 cached frames, 140 / 142 for 16 behind 5, where five
 // wavefronts fit the call's workgroups into two whole rounds; the whole call 1 094 / 1 086 and 720 / 720, of 24x45x80 3 992 / 3 974.

@@ -67,7 +67,8 @@ def _up_projection(lx: torch.Tensor, branch: LoRABranch, workspace: torch.Tensor
 
 
 def _one_pass(b: LoRABranch) -> bool:
-    """What bsa_lora_up_add is built for; other branches, and sums over several, take the up-projection as a tensor."""
+    """What bsa_lora_up_add is built for, and faster at from 1 to 32 760 tokens, rank 16 to 128 and 64 to 12 288 columns (figures at the
+    kernel); other branches, and sums over several, take the up-projection as a tensor."""
     per = b.lora_up[0].shape[0]
     return (b.rank % 16 == 0 and b.rank <= 128 and len(b.lora_up) <= 8 and per % 64 == 0
             and all(u.dtype == torch.bfloat16 and (not u.is_contiguous() or u.data_ptr() % 16 == 0) for u in b.lora_up))
