@@ -32,6 +32,7 @@
 #include "bsa_mfma.h"
 #include "bsa_slots.h"
 
+#include <algorithm>
 #include <atomic>
 
 namespace bsa {
@@ -123,6 +124,10 @@ __device__ __forceinline__ T* store_row(T* blocked, const BwdStore& w, int64_t b
 // M2 per slot (padded slots: zero rows, delta -0, M2 -inf, so that their p is 0), the row tables of both grids, the validity
 // words of the keys, and the bit matrix cleared.  A workgroup per 64-slot tile; workgroups 0 .. wg_q - 1 take tiles of the
 // queries, the next wg_k tiles of the keys, the rest words of the matrix.  delta and M2 as bwd_rows_kernel takes them.
+// On a padded grid the real rows of a chunk come first, so that the halves of 32 slots behind them hold none: these are neither
+// written nor walked by the kernels, which take from `q_live` and `k_live` how many halves of a block to walk.  Forward and
+// backward with slots as they lie / packed: 6 heads of 9x17x30 (a third of the halves are empty) 266.6 / 235.1 us, 32 heads of
+// 24x30x52 (an eighth of the tiles have one half) 7 895 / 7 793.
 // Five launches less in front of a small backward, at 4 us each; at 32 heads of 24x30x52 it takes what the separate passes took.
 struct BwdPrep {
     Grid3 gq, gk;
@@ -138,6 +143,9 @@ struct BwdPrep {
     uint32_t* bits;
     int64_t n_bits;
     float c;                                                   // of k_s
+    int32_t *q_live, *k_live;                                  // of the grid's blocks; null: no padding, slots as they lie
+    uint32_t* planes;                                          // with q_live: LiveHalves::planes
+    int n_planes, plane_words;
 };
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, int wg_k) {
@@ -147,18 +155,29 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, i
     if (w >= wg_q + wg_k) {
         const int64_t i = (int64_t)(w - wg_q - wg_k) * 256 + threadIdx.x;
         if (i < a.n_bits) a.bits[i] = 0u;
+        if (a.k_live != nullptr && i < a.gk.blocks()) a.k_live[i] = live_halves(a.gk, (int)i);
+        if (a.q_live != nullptr && (i & ~63ll) < a.gq.blocks()) {              // whole wavefronts
+            const int n = i < a.gq.blocks() ? live_halves(a.gq, (int)i) : 0;
+            if (i < a.gq.blocks()) a.q_live[i] = n;
+            for (int p = 0; p < a.n_planes; ++p) {
+                const uint64_t bit = __ballot((n >> p) & 1);
+                if (lane < 2) a.planes[p * a.plane_words + (i >> 6) * 2 + lane] = (uint32_t)(bit >> (32 * lane));
+            }
+        }
         return;
     }
-    const bool queries = w < wg_q;
+    const bool queries = w < wg_q, packed = (queries ? a.q_live : a.k_live) != nullptr;
     const Grid3& g = queries ? a.gq : a.gk;
     const int per_chunk = g.chunk() / kTile, tiles = g.blocks() * per_chunk;
     const int id = queries ? w : w - wg_q, bh = id / tiles, tile = id - bh * tiles;
     const int batch = bh / a.Hn, head = bh - batch * a.Hn;
-    const Slots s = slots_of(g, tile / per_chunk, tile % per_chunk, lane);
+    const Slots s = packed ? packed_slots_of(g, tile / per_chunk, tile % per_chunk, lane) : slots_of(g, tile / per_chunk, tile % per_chunk, lane);
     if (bh == 0 && threadIdx.x < 64) {
         (queries ? a.q_rows : a.k_rows)[(int64_t)tile * kTile + lane] = s.token;
         if (!queries && lane == 0) a.valid[tile] = s.word;
     }
+    // 16-row sweeps: of both halves, of the first alone, none
+    const int sweeps = !packed || (s.word >> 32) != 0ull ? 4 : s.word != 0ull ? 2 : 0;
     const int64_t row0 = (int64_t)id * kTile + rg;             // of the blocked tensors
     int token[4];
 #pragma unroll
@@ -171,11 +190,14 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, i
         uint4 q[4], o[4], d[4];
         float l[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { q[i] = at(a.q, a.q_st, i); o[i] = at(a.o, a.o_st, i); d[i] = at(a.dout, a.do_st, i); }
+        for (int i = 0; i < 4; ++i)
+            if (i < sweeps) { q[i] = at(a.q, a.q_st, i); o[i] = at(a.o, a.o_st, i); d[i] = at(a.dout, a.do_st, i); }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) l[i] = a.lse[bh * a.q_tokens + token[i]];
+        for (int i = 0; i < 4; ++i)
+            if (i < sweeps) l[i] = a.lse[bh * a.q_tokens + token[i]];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            if (i >= sweeps) break;
             const bool real = (s.word >> (rg + 16 * i)) & 1ull;
             keep_if(q[i], real); keep_if(o[i], real); keep_if(d[i], real);
             float sum = dot8(__builtin_bit_cast(V8, o[i]), __builtin_bit_cast(V8, d[i]));
@@ -191,9 +213,11 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, i
     } else {
         uint4 k[4], v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { k[i] = at(a.k, a.k_st, i); v[i] = at(a.v, a.v_st, i); }
+        for (int i = 0; i < 4; ++i)
+            if (i < sweeps) { k[i] = at(a.k, a.k_st, i); v[i] = at(a.v, a.v_st, i); }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
+            if (i >= sweeps) break;
             const bool real = (s.word >> (rg + 16 * i)) & 1ull;
             V8 x = __builtin_bit_cast(V8, k[i]);
 #pragma unroll
@@ -211,13 +235,29 @@ __global__ void bwd_zero_kernel(uint32_t* p, int64_t n) {
     if (i < n) p[i] = 0u;
 }
 
-// counts[bh * nbk + j] = number of query blocks that selected KV block j (bits set in its row of the bit matrix); with `base`
-// also the number of tile pairs of the head's blocks in front of j (per_entry pairs for each entry of a list); order: the head's
-// KV tiles by descending count, a counting sort (tiles of one count in no particular order).  One workgroup per head.  LDS: a
-// bin per count, 0 .. nbq, and four words at least.
+// The halves (32 slots) of a block that hold rows.  live null: all of them, `full`.
+struct LiveHalves {
+    const int32_t* live;             // per block of the grid
+    // Of the query blocks also bit by bit: bit m % 32 of word p * plane_words + m / 32 is bit p of live[m], so that the halves of a
+    // set of query blocks, a row of the bit matrix, are counted a word at a time.
+    const uint32_t* planes;
+    int n_planes, plane_words, full;
+};
+// halves of the query blocks of `bits`, word w of a row of the bit matrix
+__device__ __forceinline__ int halves_of(const LiveHalves& q, uint32_t bits, int w) {
+    if (q.live == nullptr) return q.full * __popc(bits);
+    int n = 0;
+    for (int p = 0; p < q.n_planes; ++p) n += __popc(bits & q.planes[p * q.plane_words + w]) << p;
+    return n;
+}
+
+// counts[bh * nbk + j] = number of query halves that KV block j meets (those of the blocks set in its row of the bit matrix); with
+// `base` also the number of dS units (kDsUnitBytes) of the head's blocks in front of j; order: the head's KV tiles by descending
+// count in whole blocks, a counting sort (tiles of one count in no particular order).  One workgroup per head.  LDS: a bin per
+// count, 0 .. nbq, and four words at least.
 __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restrict__ bits, int32_t* __restrict__ counts,
                                                         int32_t* __restrict__ base, int32_t* __restrict__ order, int words, int nbk, int nbq,
-                                                        int tiles_per_block, int per_entry) {
+                                                        int tiles_per_block, LiveHalves q, Divisor by_full) {
     extern __shared__ int bins[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t head = (int64_t)blockIdx.x * nbk;
@@ -226,7 +266,7 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
         const int j = j0 + threadIdx.x;
         int c = 0;
         if (j < nbk)
-            for (int w = 0; w < words; ++w) c += __popc(bits[(head + j) * words + w]);
+            for (int w = 0; w < words; ++w) c += halves_of(q, bits[(head + j) * words + w], w);
         if (j < nbk) counts[head + j] = c;
         if (base == nullptr) continue;
         int upto = c;
@@ -238,13 +278,14 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
         if (lane == 63) bins[wave] = upto;
         __syncthreads();
         for (int w = 0; w < wave; ++w) upto += bins[w];
-        if (j < nbk) base[head + j] = (before + upto - c) * per_entry;
+        if (j < nbk) base[head + j] = (before + upto - c) * tiles_per_block;
         before += bins[0] + bins[1] + bins[2] + bins[3];
         __syncthreads();
     }
     for (int i = threadIdx.x; i <= nbq; i += 256) bins[i] = 0;
     __syncthreads();
-    for (int j = threadIdx.x; j < nbk; j += 256) atomicAdd(&bins[counts[head + j]], tiles_per_block);       // this thread's own counts
+    auto bin = [&](int j) -> int { return (counts[head + j] + q.full - 1) / by_full; };
+    for (int j = threadIdx.x; j < nbk; j += 256) atomicAdd(&bins[bin(j)], tiles_per_block);       // this thread's own counts
     __syncthreads();
     // offsets in descending count: lane l of the first wavefront takes the l-th share of the bins, from the top
     if (wave == 0) {
@@ -265,18 +306,18 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
     __syncthreads();
     const int first_tile = (int)blockIdx.x * nbk * tiles_per_block;
     for (int j = threadIdx.x; j < nbk; j += 256) {
-        const int to = atomicAdd(&bins[counts[head + j]], tiles_per_block);
+        const int to = atomicAdd(&bins[bin(j)], tiles_per_block);
         for (int i = 0; i < tiles_per_block; ++i) order[first_tile + to + i] = first_tile + j * tiles_per_block + i;
     }
 }
 
-// place[row * stride + e] = the first tile pair of list entry e in the order in which the dK / dV kernel walks the pairs of its
-// head: KV blocks ascending, inside a block its query blocks ascending (the rank of this query block among the bits of the
-// block's row).
+// place[row * stride + e] = the first dS unit of list entry e in the order in which the dK / dV kernel walks its head: KV blocks
+// ascending, inside a block its query blocks ascending (the halves of the query blocks in front of this one among the bits of
+// the block's row).
 __global__ __launch_bounds__(256) void bwd_place_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ lens,
                                                         const uint32_t* __restrict__ bits, const int32_t* __restrict__ base,
                                                         int32_t* __restrict__ place, int nbq, int nbk, int stride, int words,
-                                                        int per_entry, int64_t rows) {
+                                                        int tiles_per_block, int64_t rows, LiveHalves q) {
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int64_t bh = row / nbq;
@@ -285,9 +326,9 @@ __global__ __launch_bounds__(256) void bwd_place_kernel(const int32_t* __restric
     for (int e = threadIdx.x & 63; e < n; e += 64) {
         const int64_t j = bh * nbk + min(max(idx[row * stride + e], 0), nbk - 1);
         const uint32_t* r = bits + j * words;
-        int rank = __popc(r[m >> 5] & ((1u << (m & 31)) - 1u));
-        for (int w = 0; w < (m >> 5); ++w) rank += __popc(r[w]);
-        place[row * stride + e] = base[j] + rank * per_entry;
+        int rank = halves_of(q, r[m >> 5] & ((1u << (m & 31)) - 1u), m >> 5);
+        for (int w = 0; w < (m >> 5); ++w) rank += halves_of(q, r[w], w);
+        place[row * stride + e] = base[j] + rank * tiles_per_block;
     }
 }
 
@@ -343,6 +384,17 @@ struct DqSizes {
     int tiles;                       // query tiles of a (batch, head)
     Divisor by_tiles, by_block, by_sub, by_round;      // ... of a query block; tiles of a KV block; items of a round
 };
+// Halves with rows of query tile `item`, tile `sub` of its block: 2 where nothing is padded.
+__device__ __forceinline__ int query_halves(const int32_t* q_live, int item, int head, const DqSizes& sz, int tiles_per_block) {
+    if (q_live == nullptr) return 2;
+    const int tile = item - head * sz.tiles, block = tile / sz.by_block;
+    return min(max(__builtin_amdgcn_readfirstlane(q_live[block]) - 2 * (tile - block * tiles_per_block), 0), 2);
+}
+__device__ __forceinline__ int wave_sum(int x) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
+    return __builtin_amdgcn_readfirstlane(x);
+}
 template <typename T, bool kMasked>
 __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q, const T* __restrict__ dout,
                                                         const T* __restrict__ ks, const T* __restrict__ v,
@@ -350,7 +402,8 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
                                                         const int32_t* __restrict__ idx, const int32_t* __restrict__ lens,
                                                         const uint64_t* __restrict__ tile_valid, T* __restrict__ dq,
                                                         int64_t Sq, int64_t Sk, int bs_q, int bs_k, int stride, int item_begin,
-                                                        int item_end, int round, BwdStore dq_to, DqSizes sz) {
+                                                        int item_end, int round, BwdStore dq_to, DqSizes sz, const int32_t* __restrict__ q_live,
+                                                        const int32_t* __restrict__ k_live) {
     typedef typename Vec8<T>::type V8;
     extern __shared__ __attribute__((aligned(1024))) char dq_ring[];
     const int lane = threadIdx.x, lr = lane & 31, lh = lane >> 5;
@@ -363,6 +416,7 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
     const int head = item / sz.by_tiles;
     const int64_t bh = head, qrow0 = (int64_t)(item - head * sz.tiles) * kTile, lrow = item / sz.by_block;      // the tiles of a block lie next to each other
     const int nbk = (int)(Sk / kTile) / sz.by_sub, nsub = bs_k / kTile;
+    if (query_halves(q_live, item, head, sz, bs_q / kTile) == 0) return;
     const int n = __builtin_amdgcn_readfirstlane(min(max(lens[lrow], 0), stride));
     const int32_t* list = idx + lrow * stride;
     const char* k_src = reinterpret_cast<const char*>(ks) + bh * Sk * (int64_t)(kD * 2);
@@ -394,12 +448,20 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
 #pragma unroll
         for (int i = 0; i < 16; ++i) neg_m[qq][i] = m_row[qq];       // m2 and delta come negated
 
-    const int ntiles = n * nsub, nhalves = 2 * ntiles;
-    auto tile_at = [&](int tp) -> int64_t {
-        const int tc = min(tp, ntiles - 1);
-        const int e = tc / sz.by_sub;
-        return (int64_t)min(max(list[e], 0), nbk - 1) * nsub + tc - e * nsub;
-    };
+    // the walk: the halves with keys of one listed block after another
+    auto block_at = [&](int e) -> int { return __builtin_amdgcn_readfirstlane(min(max(list[min(e, n - 1)], 0), nbk - 1)); };
+    auto halves_of_block = [&](int block) -> int { return k_live != nullptr ? __builtin_amdgcn_readfirstlane(k_live[block]) : 2 * nsub; };
+    int nhalves = 2 * n * nsub;
+    if (k_live != nullptr) {
+        int mine = 0;
+        for (int e = lane; e < n; e += 64) mine += k_live[min(max(list[e], 0), nbk - 1)];
+        nhalves = wave_sum(mine);
+    }
+    // halves come in pairs: an odd number of them ends with the last one again, all of its keys masked
+    const int n_real = nhalves;
+    nhalves = (nhalves + 1) & ~1;
+    int entry = 0, next_block = 0, block_half = 0, half = 0, halves = 0;
+    if (n > 0) next_block = block_at(0);
     // ---- global -> LDS: 16 loads of 1 KB per half
     const uint32_t lds0 = lds_address(dq_ring);
     uint32_t voff[4];
@@ -412,9 +474,18 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
     uint32_t hv_ahead = ~0u;                     // validity of the keys of the half tile requested last
     auto issue = [&](int hp) {
         if (hp >= nhalves) return;
-        const int64_t tile = (int64_t)__builtin_amdgcn_readfirstlane((int)tile_at(hp >> 1));
-        if (kMasked) hv_ahead = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(tile_valid[tile] >> (32 * (hp & 1))));
-        const int64_t off = tile * kTileBytes + (hp & 1) * kBwdHalfTileBytes;
+        if (hp < n_real) {
+            if (half == halves) {
+                block_half = next_block * 2 * nsub;
+                halves = halves_of_block(next_block);
+                half = 0;
+                next_block = block_at(++entry);
+            }
+            ++half;
+        }
+        const int at = block_half + half - 1;
+        if (kMasked) hv_ahead = hp < n_real ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(tile_valid[at >> 1] >> (32 * (at & 1)))) : 0u;
+        const int64_t off = (int64_t)at * kBwdHalfTileBytes;
         const uint32_t dst = lds0 + (hp & 1) * kDqStage;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -569,11 +640,12 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
 // LDS stages, and both operands come out with transposing reads: the next half's while this one's sixteen MFMAs run, so all
 // three stages can be on their way.  Bound by the 24 KB per pair that enter the CU (32 MFMAs take two thirds of the time of
 // their loads at 64 B/clk); dS is read once, from beyond the L2.
-//   dS of a pair: [query half][key half][16-query step st][lane][8 elements], lane = 32 lh + key: the queries 16 st + 4 lh .. + 3
-//   and 8 further (the accumulator order of the dK / dV kernel), 1 KB per store instruction.
+//   dS in units of 32 queries against a 64-key tile, in the order in which the dK / dV kernel walks them (the tiles of a KV block next
+//   to one another): [key half][16-query step st][lane][8 elements], lane = 32 lh + key: the queries 16 st + 4 lh .. + 3 and 8
+//   further (the accumulator order of the dK / dV kernel), 1 KB per store instruction.
 //   In LDS: unit (key, lh, st) at 16-byte slot 4 key + 2 lh + st of its 2 KB block, so that the 32 lanes of a pass of a
 //   transposing read (4 keys x 16 queries, two groups) cover 256 consecutive bytes.
-constexpr int kDsPairBytes = kTile * kTile * 2;
+constexpr int kDsPairBytes = kTile * kTile * 2, kDsUnitBytes = kDsPairBytes / 2;
 constexpr int kDsqStage = kBwdHalfTileBytes + kDsPairBytes / 2;
 constexpr int kDsqStages = 3;
 constexpr int kDsqLoads = kDsqStage / 1024;      // LDS DMA instructions per half
@@ -583,7 +655,8 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
                                                             const int32_t* __restrict__ idx, const int32_t* __restrict__ place,
                                                             const int32_t* __restrict__ lens, T* __restrict__ dq, int64_t Sq,
                                                             int64_t Sk, int bs_q, int bs_k, int stride, int item_begin, int item_end,
-                                                            int round, int64_t pairs_per_head, BwdStore dq_to, DqSizes sz) {
+                                                            int round, int64_t pairs_per_head, BwdStore dq_to, DqSizes sz,
+                                                            const int32_t* __restrict__ q_live, const int32_t* __restrict__ k_live) {
     typedef typename Vec8<T>::type V8;
     extern __shared__ __attribute__((aligned(1024))) char dsq_ring[];
     const int lane = threadIdx.x, lr = lane & 31, lh = lane >> 5;
@@ -596,6 +669,8 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
     const int head = item / sz.by_tiles, lrow_n = item / sz.by_block;          // the tiles of a block lie next to each other
     const int64_t bh = head, qrow0 = (int64_t)(item - head * sz.tiles) * kTile, lrow = lrow_n;
     const int nbk = (int)(Sk / kTile) / sz.by_sub, nsub = bs_k / kTile, sub_q = item - lrow_n * (bs_q / kTile);
+    const int q_halves = query_halves(q_live, item, head, sz, bs_q / kTile);
+    if (q_halves == 0) return;
     const int n = __builtin_amdgcn_readfirstlane(min(max(lens[lrow], 0), stride));
     const char* k_src = reinterpret_cast<const char*>(ks) + bh * Sk * (int64_t)(kD * 2);
     const char* ds_src = ds + bh * pairs_per_head * kDsPairBytes;
@@ -606,16 +681,17 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
         for (int qq = 0; qq < 2; ++qq)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[t][qq][i] = 0.f;
-    const int nhalves = 2 * n * nsub;
+    int nhalves = 2 * n * nsub;
 
     // ---- the list, 64 entries at a time in a register each, an entry per lane (no vector load between the counted DMA loads
-    // but one pair every 64 entries)
-    int list_j = 0, list_p = 0;
+    // but these every 64 entries): block, dS unit, halves with keys
+    int list_j = 0, list_p = 0, list_n = 2 * nsub;
     auto take_entries = [&](int e0) {
         const int e = min(e0 + lane, n - 1);
         list_j = min(max(idx[lrow * stride + e], 0), nbk - 1);
         list_p = place[lrow * stride + e];
-        asm volatile("" : "+v"(list_j), "+v"(list_p));
+        if (k_live != nullptr) list_n = k_live[list_j];
+        asm volatile("" : "+v"(list_j), "+v"(list_p), "+v"(list_n));
     };
     // ---- global -> LDS
     const uint32_t lds0 = lds_address(dsq_ring);
@@ -627,19 +703,20 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
         voff[i] = (uint32_t)((row - 4 * i) * 256 + (((lane & 15) ^ f) << 4));    // load i adds 1 KB on both sides
     }
     const uint32_t voff_ds = (uint32_t)((lane & 1) * 1024 + ((lane >> 1) & 1) * 512 + (lane >> 2) * 16);
-    int entry = 0, sub = 0, key_half = 0, issued = 0, issue_stage = 0;
+    // a tile with rows in its first half alone takes that half's dS twice (the second sums are not stored)
+    const uint32_t second_half = q_halves == 2 ? (uint32_t)(nsub * kDsUnitBytes) : 0u;
+    int entry = 0, half = 0, issued = 0, issue_stage = 0;
     auto issue = [&]() {                          // the next half of the walk
         if (issued >= nhalves) return;
-        if (key_half == 0 && sub == 0 && entry > 0 && (entry & 63) == 0) take_entries(entry);
-        const int64_t tile = (int64_t)__builtin_amdgcn_readlane(list_j, entry & 63) * nsub + sub;
-        const int64_t pair = (int64_t)__builtin_amdgcn_readlane(list_p, entry & 63) + sub_q * nsub + sub;
+        const int64_t at = (int64_t)__builtin_amdgcn_readlane(list_j, entry & 63) * (2 * nsub) + half;
+        const int64_t unit = (int64_t)__builtin_amdgcn_readlane(list_p, entry & 63) + 2 * sub_q * nsub + (half >> 1);
         auto uniform = [](const char* x) -> const char* {          // the compiler cannot tell
             const uint64_t a = reinterpret_cast<uint64_t>(x);
             return reinterpret_cast<const char*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
                                                  ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32));
         };
-        const char* kp = uniform(k_src + tile * kTileBytes + key_half * kBwdHalfTileBytes);
-        const char* dp = uniform(ds_src + pair * kDsPairBytes + key_half * 2048);
+        const char* kp = uniform(k_src + at * kBwdHalfTileBytes);
+        const char* dp = uniform(ds_src + unit * kDsUnitBytes + (half & 1) * 2048);
         const uint32_t dst = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + issue_stage * kDsqStage));
         // an SGPR that a VALU instruction wrote may be a VMEM address five wait states later; the compiler does not count them
         // in front of an assembly statement (it left two)
@@ -650,11 +727,13 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
 #pragma unroll
         for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int i = 0; i < 2; ++i) load_to_lds_16_once(dp + h * 4096 + i * 256, voff_ds, dst + kBwdHalfTileBytes + h * 2048 + i * 1024);
+            for (int i = 0; i < 2; ++i) load_to_lds_16_once(dp + h * second_half + i * 256, voff_ds, dst + kBwdHalfTileBytes + h * 2048 + i * 1024);
         ++issued;
         issue_stage = issue_stage == kDsqStages - 1 ? 0 : issue_stage + 1;
-        key_half ^= 1;
-        if (key_half == 0 && ++sub == nsub) { sub = 0; ++entry; }
+        if (++half == __builtin_amdgcn_readlane(list_n, entry & 63)) {
+            half = 0;
+            if ((++entry & 63) == 0 && entry < n) take_entries(entry);
+        }
     };
     // ---- LDS -> fragments
     const int s16 = lane & 15, g1 = (lane >> 4) & 1, tx = s16 >> 2, ty = (s16 & 3) >> 1, tz = s16 & 1;
@@ -716,19 +795,26 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
     if (nhalves > 0) {
         V8 kt[2][8], d[2][2][2];
         take_entries(0);
+        if (k_live != nullptr) {
+            int mine = lane < n ? list_n : 0;
+            for (int e = 64 + lane; e < n; e += 64) mine += k_live[min(max(idx[lrow * stride + e], 0), nbk - 1)];
+            nhalves = wave_sum(mine);
+        }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // from here on the DMA loads are counted by hand
         issue();
         issue();
         issue();
         if (nhalves > 2) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        else if (nhalves > 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         take(kt[0], d[0]);
         reads_done();
         issue();
-        for (int hp = 0; hp < nhalves; hp += 2) {                                // halves come in pairs
+        for (int hp = 0; hp + 1 < nhalves; hp += 2) {
             step(hp, kt[0], d[0], kt[1], d[1]);
             step(hp + 1, kt[1], d[1], kt[0], d[0]);
         }
+        if (nhalves & 1) multiply(kt[0], d[0]);
     }
     // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, query lr (+ 32)
 #pragma unroll
@@ -762,12 +848,15 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
 // f(r) = ((r & 3) << 2) | ((r >> 2) & 3): 16 consecutive rows, and the 4 rows x 4 units of a transposing read's 32 lanes,
 // land on different banks.
 constexpr int kBwdHalfTile = kTileBytes / 2;                 // 32 query rows of Q or of dO
-constexpr int kBwdStats = 1024;                              // M2 (128 B), delta (128 B), -inf (128 B, for padded keys)
+constexpr int kBwdStats = 1024;                              // M2 (128 B), delta (128 B), -inf (128 B, for padded keys and repeated halves)
 constexpr int kBwdStage = 2 * kBwdHalfTile + kBwdStats;      // one half tile of queries: Q rows, dO rows, M2, delta
 constexpr int kBwdStages = 4;                                // two in use (this half, the next half's rows), two on their way
 // The Q parts of all stages, then their dO parts, then their numbers: every LDS read of the loop is a lane's offset, which changes
 // with the pair of stages by one bit, and a constant below 2^16, which the instruction holds.
 constexpr int kBwdDout = kBwdStages * kBwdHalfTile, kBwdNumbers = 2 * kBwdStages * kBwdHalfTile;
+// The list of a KV block's query blocks, in LDS: the block, and above kBlockBits its halves with rows (where any are padded).
+constexpr int kBlockBits = 15, kMostLiveHalves = (1 << (32 - kBlockBits)) - 1;
+constexpr int kPlanesAtHand = 4;                             // chunks of less than 512 tokens
 
 // What bounds it is issue: a wavefront has its SIMD to itself and issues one instruction after another, 337 of them a half beside
 // 1 024 clocks of products.  249 are left, with addresses that are scalars and stay so, no division for the list position, constants
@@ -777,7 +866,7 @@ constexpr int kBwdDout = kBwdStages * kBwdHalfTile, kBwdNumbers = 2 * kBwdStages
 // kKeep: dS, rounded as for the product, is also written out for bwd_dq_from_ds_kernel (pair_base: bwd_count_kernel's base).
 // what the dK / dV kernel would divide by or divide to get
 struct DkdvSizes {
-    int tiles, nbq, qsub, nsub;      // key tiles of a (batch, head), query blocks, tiles of a query block and of a KV block
+    int tiles, nbq, nsub;            // key tiles of a (batch, head), query blocks, tiles of a KV block
     Divisor by_tiles, by_block, by_round;
 };
 template <typename T, bool kMasked, bool kKeep>
@@ -789,7 +878,9 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
                                                        T* __restrict__ dv, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int words,
                                                        float dk_scale, const int32_t* __restrict__ order, int n_items, int round,
                                                        BwdStore dk_to, BwdStore dv_to, char* __restrict__ ds_out,
-                                                       const int32_t* __restrict__ pair_base, int64_t pairs_per_head, DkdvSizes sz) {
+                                                       char* __restrict__ ds_spare, const int32_t* __restrict__ unit_base, int64_t pairs_per_head, DkdvSizes sz,
+                                                       LiveHalves q_live, const int32_t* __restrict__ k_live,
+                                                       const int32_t* __restrict__ counts) {
     typedef typename Vec8<T>::type V8;
     extern __shared__ __attribute__((aligned(1024))) char bwd_lds[];
     const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
@@ -806,8 +897,17 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     const int head = item / sz.by_tiles, block = item / sz.by_block;          // the tiles of a block lie next to each other, over all heads
     const int64_t bh = head;
     const int64_t krow0 = (int64_t)(item - head * sz.tiles) * kTile;
-    const int nbq = sz.nbq, qsub = sz.qsub, nsub = sz.nsub;
+    const int nbq = sz.nbq, nsub = sz.nsub;
     const uint32_t* mask_row = bits + (int64_t)block * words;
+    // halves of this tile that hold keys: the second wavefront of a tile with one half brings its share of the rows, no more
+    int key_halves = 2;
+    if (k_live != nullptr) {
+        const int in_head = block - head * (sz.tiles / sz.by_block);
+        key_halves = __builtin_amdgcn_readfirstlane(k_live[in_head]) - 2 * (item - block * nsub);
+        if (key_halves <= 0) return;
+    }
+    // halves come in pairs: an odd number of them ends with the last one again, whose p are 0 (M2 = -inf)
+    const int n_real = __builtin_amdgcn_readfirstlane(counts[block]), nhalves = (n_real + 1) & ~1;
 
     // resident: K_s and V rows of this wavefront's 32 keys, as B operands (lane = key lr, 8 consecutive d)
     V8 kreg[8], vreg[8];
@@ -828,13 +928,19 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         for (int i = 0; i < 16; ++i) { acc_dk[t][i] = 0.f; acc_dv[t][i] = 0.f; }
 
     // behind every stage's numbers: M2 for padded keys
-    if (kMasked) *reinterpret_cast<float*>(bwd_lds + kBwdNumbers + (threadIdx.x >> 5) * kBwdStats + 256 + (threadIdx.x & 31) * 4) = -INFINITY;
+    *reinterpret_cast<float*>(bwd_lds + kBwdNumbers + (threadIdx.x >> 5) * kBwdStats + 256 + (threadIdx.x & 31) * 4) = -INFINITY;
     // the query blocks of this KV block, ascending, from the bit matrix into LDS (behind the stages)
     int32_t* qlist = reinterpret_cast<int32_t*>(bwd_lds + kBwdStages * kBwdStage);
     int count = 0;
     for (int w0 = 0; w0 < words; w0 += 64) {
         const int w = w0 + lane;
         uint32_t word = w < words ? mask_row[w] : 0u;
+        uint32_t plane[kPlanesAtHand] = {};
+        if (q_live.live != nullptr) {
+#pragma unroll
+            for (int p = 0; p < kPlanesAtHand; ++p)
+                if (p < q_live.n_planes && w < words) plane[p] = q_live.planes[p * q_live.plane_words + w];
+        }
         if (w == words - 1 && (nbq & 31)) word &= (1u << (nbq & 31)) - 1u;
         int mine = __popc(word), upto = mine;
 #pragma unroll
@@ -845,25 +951,37 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         int pos = count + upto - mine;
         if (wave == 0)
             while (word != 0u) {
-                qlist[pos++] = 32 * w + __builtin_ctz(word);
+                const int b = __builtin_ctz(word);
+                uint32_t n = 0;
+                if (q_live.live != nullptr) {
+                    if (q_live.n_planes <= kPlanesAtHand) {
+#pragma unroll
+                        for (int p = 0; p < kPlanesAtHand; ++p) n |= ((plane[p] >> b) & 1u) << p;
+                    } else {
+                        n = (uint32_t)q_live.live[32 * w + b];
+                    }
+                }
+                qlist[pos++] = (int32_t)((uint32_t)(32 * w + b) | n << kBlockBits);
                 word &= word - 1u;
             }
         count += __shfl(upto, 63);
     }
     __syncthreads();
-    const int count_u = __builtin_amdgcn_readfirstlane(count), ntiles = count_u * qsub;          // the same in every lane; the compiler cannot tell
-    // the walk's tiles one after another; the entry of the next block is read from LDS a pair of halves before it is used
-    int next_block = 0, next_sub = 0, next_entry = 0, block_tile = 0;
-    if (ntiles > 0) next_block = qlist[0];
-    auto next_tile = [&]() -> int {
-        if (next_sub == 0) {
-            block_tile = __builtin_amdgcn_readfirstlane(next_block) * qsub;
+    const int count_u = __builtin_amdgcn_readfirstlane(count);          // the same in every lane; the compiler cannot tell
+    // the walk's halves one after another; the entry of the next block is read from LDS while this one's are walked
+    int next_block = 0, next_entry = 0, block_half = 0, half = 0, halves = 0;
+    if (nhalves > 0) next_block = qlist[0];
+    auto next_half = [&]() -> int {
+        if (half == halves) {
+            const uint32_t entry = (uint32_t)__builtin_amdgcn_readfirstlane(next_block);
+            block_half = (int)(entry & ((1u << kBlockBits) - 1u)) * q_live.full;
+            halves = q_live.live != nullptr ? (int)(entry >> kBlockBits) : q_live.full;
+            half = 0;
             next_entry = min(next_entry + 1, count_u - 1);
             next_block = qlist[next_entry];
         }
-        const int tile = block_tile + next_sub;
-        next_sub = next_sub + 1 == qsub ? 0 : next_sub + 1;
-        return tile;
+        ++half;
+        return block_half + half - 1;
     };
 
     // ---- global -> LDS
@@ -879,19 +997,16 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     const uint32_t voff_stats = (lane < 32 ? stat_gap : 0u) + (uint32_t)((lane & 31) * 4);      // 32 x M2, 32 x delta
     const char* tile_src = reinterpret_cast<const char*>(wave == 0 ? q : dout) + bh * Sq * (int64_t)(kD * 2);
     const char* stat_src = reinterpret_cast<const char*>(delta) + bh * Sq * 4;
-    const int nhalves = 2 * ntiles;
-    // half hp = query half hp & 1 of the walk's tile hp / 2, into stage hp % kBwdStages; called for hp = 0, 1, 2, ...
-    int64_t tile = 0;
+    // half hp of the walk into stage hp % kBwdStages; called for hp = 0, 1, 2, ...
     auto issue = [&](int hp, int stage) {
         if (hp >= nhalves) return;
-        const int h = hp & 1;
-        if (h == 0) tile = next_tile();
-        const char* src = tile_src + tile * kTileBytes + h * kBwdHalfTile;
+        const int64_t at = hp < n_real ? next_half() : block_half + half - 1;
+        const char* src = tile_src + at * kBwdHalfTile;
         const uint32_t dst = lds0 + wave * kBwdDout + stage * kBwdHalfTile;
 #pragma unroll
         for (int j = 0; j < 2; ++j) load_to_lds_4x16(src + j * 4096, voff, dst + j * 4096);
         if (wave == 0)
-            load_to_lds_4(stat_src + tile * (kTile * 4) + h * 128, voff_stats, lds0 + kBwdNumbers + stage * kBwdStats);
+            load_to_lds_4(stat_src + at * 128, voff_stats, lds0 + kBwdNumbers + stage * kBwdStats);
     };
 
     // ---- LDS -> fragments
@@ -920,23 +1035,24 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     // the queries' M2 as this lane's key sees them: -inf for a padded key, whose chains (its row of k_s is zeros) then give
     // p = exp2(-inf) = 0
     uint32_t numbers = lds0 + (uint32_t)(kBwdNumbers + 16 * lh), m2_at = numbers + (kMasked && !key_ok ? 256u : 0u);
-    auto starts = [&](int stage, f32x16& from_m, f32x16& from_d) {
+    auto starts = [&](int stage, bool real, f32x16& from_m, f32x16& from_d) {
+        const uint32_t m2_here = real ? m2_at : numbers + 256;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const f32x4_ mm = lds_read_at<f32x4_>(m2_at + (stage * kBwdStats + 32 * g));
+            const f32x4_ mm = lds_read_at<f32x4_>(m2_here + (stage * kBwdStats + 32 * g));
             const f32x4_ dd = lds_read_at<f32x4_>(numbers + (stage * kBwdStats + 128 + 32 * g));
             from_m[4 * g] = mm.x; from_m[4 * g + 1] = mm.y; from_m[4 * g + 2] = mm.z; from_m[4 * g + 3] = mm.w;
             from_d[4 * g] = dd.x; from_d[4 * g + 1] = dd.y; from_d[4 * g + 2] = dd.z; from_d[4 * g + 3] = dd.w;
         }
     };
-    auto products_and_exponentials = [&](auto stage_c, f32x16& s, f32x16& dp, f32x16& s_next, f32x16& dp_next, auto&& behind_requests) {
+    auto products_and_exponentials = [&](auto stage_c, bool next_real, f32x16& s, f32x16& dp, f32x16& s_next, f32x16& dp_next, auto&& behind_requests) {
         constexpr int stage = decltype(stage_c)::value;             // of the next half, in its pair
         constexpr uint32_t qn = stage * kBwdHalfTile, dn = qn + kBwdDout;
         // The chains of the next half start from its queries' -M2 and -delta (accumulator i <-> query
         // 8 (i / 4) + 4 lh + i % 4 of the half, key lr), so S - M2 and dP - delta come out of the products and the
         // exponentials need no subtraction.
         f32x16 from_m, from_d;
-        starts(stage, from_m, from_d);
+        starts(stage, next_real, from_m, from_d);
         // Volatile assembly keeps the compiler from moving LDS reads across it, so the operands of a group of four
         // MFMAs are requested a group ahead by hand.
         V8 fq[2][2], fd[2][2];
@@ -972,15 +1088,15 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         }
     };
     char* ds_item = !kKeep ? nullptr
-        : ds_out + (bh * pairs_per_head + __builtin_amdgcn_readfirstlane(pair_base[block]) + (item - block * nsub)) * kDsPairBytes + wave * 2048;
-    auto gradients = [&](auto stage_c, const f32x16& p, const f32x16& ds) {
+        : ds_out + bh * pairs_per_head * kDsPairBytes + ((int64_t)__builtin_amdgcn_readfirstlane(unit_base[block]) + (item - block * nsub)) * kDsUnitBytes + wave * 2048;
+    auto gradients = [&](auto stage_c, char* ds_to, const f32x16& p, const f32x16& ds) {
         constexpr int stage = decltype(stage_c)::value;             // of this half, in its pair
         constexpr uint32_t qt = stage * kBwdHalfTile, dt = qt + kBwdDout;
 #pragma unroll
         for (int st2 = 0; st2 < 2; ++st2) {
             const V8 bp = pack8<T, V8>(p, st2), bds = pack8<T, V8>(ds, st2);
             if (kKeep)
-                __builtin_nontemporal_store(bds, reinterpret_cast<V8*>(ds_item + (stage & 1) * 4096 + st2 * 1024 + lane * 16));
+                __builtin_nontemporal_store(bds, reinterpret_cast<V8*>(ds_to + st2 * 1024 + lane * 16));
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 acc_dv[t] = mfma32(frag_tr_lds(dt, st2, t), bp, acc_dv[t]);
@@ -1001,14 +1117,15 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
             m2_at ^= 2 * kBwdStats;
         }
         // half hp + 3 takes the stage that half hp - 1 was read from: both wavefronts are past the barrier behind it
-        products_and_exponentials(std::integral_constant<int, odd ^ 1>{}, s, dp, s_next, dp_next, [&]() { issue(hp + 3, (hp + 3) & 3); });
+        // the halves with an odd number alone may be the one that repeats
+        products_and_exponentials(std::integral_constant<int, odd ^ 1>{}, odd || hp + 1 < n_real, s, dp, s_next, dp_next, [&]() { issue(hp + 3, (hp + 3) & 3); });
         __builtin_amdgcn_sched_barrier(0);
-        gradients(odd_c, s, dp);
+        gradients(odd_c, !odd || hp < n_real ? ds_item : ds_spare, s, dp);
         if (odd) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) { toff[t][0] ^= 2 * kBwdHalfTile; toff[t][1] ^= 2 * kBwdHalfTile; }
-            if (kKeep) ds_item += (int64_t)nsub * kDsPairBytes;
         }
+        if (kKeep) ds_item += (int64_t)nsub * kDsUnitBytes;
         // the chains into (s_next, dp_next) end here, sixteen MFMAs behind their last one
         mfma_chain_end(s_next); mfma_chain_end(dp_next);
         // With kKeep the two stores of this half and those of the one before may be on their way as well: a store is
@@ -1035,11 +1152,20 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __builtin_amdgcn_s_barrier();
+        if (wave >= key_halves) {                // no keys: the rows alone
+            for (int hp = 0; hp < nhalves; ++hp) {
+                issue(hp + 3, (hp + 3) & 3);
+                if (hp + 3 >= nhalves) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+            }
+            return;
+        }
         f32x16 s0, dp0, s1, dp1;
         {
             constexpr uint32_t qn = 0, dn = kBwdDout;
             f32x16 from_m, from_d;
-            starts(0, from_m, from_d);
+            starts(0, true, from_m, from_d);
             mfma_from_v(s0, lds_read_at<V8>(roff[0] + qn), kreg[0], from_m);
             mfma_from_v(dp0, lds_read_at<V8>(roff[0] + dn), vreg[0], from_d);
 #pragma unroll
@@ -1085,6 +1211,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
 constexpr size_t kBwdLdsLimit = 160 * 1024;
 // LDS of the dK / dV kernel for nbq query blocks: its stages, then the list of a KV block's query blocks
 size_t bwd_dkdv_lds_bytes(int nbq) { return (size_t)kBwdStages * kBwdStage + (size_t)nbq * sizeof(int32_t); }
+static_assert((kBwdLdsLimit - (size_t)kBwdStages * kBwdStage) / sizeof(int32_t) < ((size_t)1 << kBlockBits), "a list entry holds the block");
 int bwd_max_query_blocks() { return (int)((kBwdLdsLimit - (size_t)kBwdStages * kBwdStage) / sizeof(int32_t)); }
 
 // dS is kept between the two kernels where all of it (every list full) fits kDsBytes: 6.4 GB for 32 heads of 480p, where the
@@ -1106,11 +1233,19 @@ static KeptDs plan_ds(int64_t bh, int64_t Sq, int64_t Sk, int bs_q, int bs_k, in
 // The pieces of the backward's workspace.
 struct BwdWs {
     size_t ks, delta, m2, bits, paced, counts, order;      // k_s in blocked order; delta and M2; the bit matrix; the lists in the dQ
-                                                           // kernel's visiting order; per KV block its number of query blocks; the KV
+                                                           // kernel's visiting order; per KV block its number of query halves; the KV
                                                            // tiles of every head by that number
-    size_t base, place, ds;                                // with kept dS: pairs in front of a KV block, the pair of a list entry, dS
+    size_t q_live, k_live, planes;                         // LiveHalves of both grids (token order, where they are padded)
+    size_t base, place, ds, ds_spare;                      // with kept dS: units in front of a KV block, the first unit of a list entry, dS,
+                                                           // where a repeated half's goes
     size_t total;
 };
+static int plane_words(int64_t blocks) { return (int)((blocks + 63) / 64 * 2); }
+static int plane_count(int chunk) {
+    int bits = 0;
+    while ((chunk / 32) >> bits) ++bits;
+    return bits;
+}
 static BwdWs bwd_ws(const KeptDs& kept, int64_t bh, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride) {
     BwdWs w;
     size_t off = 0;
@@ -1123,9 +1258,13 @@ static BwdWs bwd_ws(const KeptDs& kept, int64_t bh, int64_t Sq, int64_t Sk, int 
     w.paced = take(bh * nbq * (size_t)idx_stride * 4);
     w.counts = take(bh * nbk * 4);
     w.order = take(bh * (size_t)(Sk / kTile) * 4);
+    w.q_live = take(nbq * 4);
+    w.k_live = take(nbk * 4);
+    w.planes = take((size_t)plane_count(bs_q) * plane_words((int64_t)nbq) * 4);
     w.base = take(kept.keep ? bh * nbk * 4 : 0);
     w.place = take(kept.keep ? bh * nbq * (size_t)idx_stride * 4 : 0);
     w.ds = take(kept.keep ? (size_t)bh * (size_t)kept.pairs_per_head * kDsPairBytes : 0);
+    w.ds_spare = take(kept.keep ? kDsUnitBytes : 0);
     w.total = off;
     return w;
 }
@@ -1156,7 +1295,14 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     int32_t* order = reinterpret_cast<int32_t*>(ws + at.order);
     int32_t* base = reinterpret_cast<int32_t*>(ws + at.base);
     int32_t* place = reinterpret_cast<int32_t*>(ws + at.place);
-    const int per_entry = (bs_q / kTile) * (bs_k / kTile);
+    const int nsub = bs_k / kTile;
+    // On a padded grid the real rows of a chunk come first, and the halves behind them are left out
+    auto packs = [](const Grid3& g) { return (g.T % g.t || g.H % g.h || g.W % g.w) && g.chunk() / 32 <= kMostLiveHalves; };
+    LiveHalves q_live = {nullptr, nullptr, 0, 0, bs_q / 32};
+    int32_t* k_live = nullptr;
+    if (thw != nullptr && packs(thw->gq))
+        q_live = {reinterpret_cast<int32_t*>(ws + at.q_live), reinterpret_cast<uint32_t*>(ws + at.planes), plane_count(bs_q), plane_words(nbq), bs_q / 32};
+    if (thw != nullptr && packs(thw->gk)) k_live = reinterpret_cast<int32_t*>(ws + at.k_live);
 
     // the dK / dV kernel's LDS: four stages of half a Q tile, half a dO tile and the queries' M2 / delta, then a KV block's query
     // blocks; bwd_count_kernel has a bin for each of their numbers, less than that
@@ -1203,7 +1349,10 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         a.v_blocked = (uint16_t*)thw->v_blocked;
         a.delta = delta; a.m2 = m2; a.q_rows = thw->q_rows; a.k_rows = thw->k_rows; a.valid = thw->valid;
         a.bits = bits; a.n_bits = nwords; a.c = c;
-        const int64_t wg_q = qrows / kTile, wg_k = krows / kTile, wg_bits = (nwords + 255) / 256;
+        a.q_live = const_cast<int32_t*>(q_live.live); a.k_live = k_live;
+        a.planes = const_cast<uint32_t*>(q_live.planes); a.n_planes = q_live.n_planes; a.plane_words = q_live.plane_words;
+        const int64_t wg_q = qrows / kTile, wg_k = krows / kTile;
+        const int64_t last = std::max(nwords, (int64_t)std::max(q_live.live != nullptr ? nbq : 0, k_live != nullptr ? nbk : 0)), wg_bits = (last + 255) / 256;
         if (wg_q + wg_k + wg_bits > 0x7fffffff) return hipErrorInvalidValue;
         const dim3 grid((unsigned)(wg_q + wg_k + wg_bits)), blk(256);
         if (dtype == BSA_BF16) hipLaunchKernelGGL((bwd_prepare_kernel<__bf16>), grid, blk, 0, st, a, (int)wg_q, (int)wg_k);
@@ -1225,7 +1374,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     // order); any other order is walked as given.  The order only moves fp32 roundings of the dQ sum.
     if ((e = launch_pace_order(idx, paced, lens, lrows, nbk, idx_stride, st, {}, {bits, nbq, words})) != hipSuccess) return e;
     hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)bh), dim3(256), count_lds, st, bits, counts, kept.keep ? base : nullptr, order, words, nbk, nbq,
-                       bs_k / kTile, per_entry);
+                       nsub, q_live, divisor(q_live.full));
 
     const dim3 block(64);
     const bool masked = tile_valid != nullptr;
@@ -1234,18 +1383,18 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     // rounds that wait for the longest list cost more than they bring.
     const int round = 4 * cus;
     const DqSizes dq_sizes = {(int)(Sq / kTile), divisor((int)(Sq / kTile)), divisor(bs_q / kTile), divisor(bs_k / kTile), divisor(round)};
-    const DkdvSizes sizes = {(int)(Sk / kTile), nbq, bs_q / kTile, bs_k / kTile, divisor((int)(Sk / kTile)), divisor(bs_k / kTile), divisor(round)};
+    const DkdvSizes sizes = {(int)(Sk / kTile), nbq, nsub, divisor((int)(Sk / kTile)), divisor(bs_k / kTile), divisor(round)};
     const int total_q = (int)(bh * (Sq / kTile)), total_k = (int)(bh * (Sk / kTile));
 #define BSA_DKDV(T, M, K)                                                                                                              \
     hipLaunchKernelGGL((bwd_dkdv_kernel<T, M, K>), dim3((unsigned)total_k), dim3(128), lds, st, (const T*)q, (const T*)dout, (const T*)ks,  \
                        (const T*)v, m2, delta, bits, tile_valid, (T*)dk, (T*)dv, Sq, Sk, bs_q, bs_k, words, sm_scale, order, total_k, round,  \
-                       dk_to, dv_to, ws + at.ds, base, kept.pairs_per_head, sizes)
+                       dk_to, dv_to, ws + at.ds, ws + at.ds_spare, base, kept.pairs_per_head, sizes, q_live, k_live, counts)
 #define BSA_DQ(T, M)                                                                                                                   \
     hipLaunchKernelGGL((bwd_dq_lds_kernel<T, M>), dim3(end - first), block, kDqRingLds, st, (const T*)q, (const T*)dout, (const T*)ks, (const T*)v,  \
-                       m2, delta, paced, lens, tile_valid, (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, dq_to, dq_sizes)
+                       m2, delta, paced, lens, tile_valid, (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, dq_to, dq_sizes, q_live.live, k_live)
 #define BSA_DQ_DS(T)                                                                                                                   \
     hipLaunchKernelGGL((bwd_dq_from_ds_kernel<T>), dim3(end - first), block, kDsqStages* kDsqStage, st, (const T*)ks, ws + at.ds, paced, place, lens,  \
-                       (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, kept.pairs_per_head, dq_to, dq_sizes)
+                       (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, kept.pairs_per_head, dq_to, dq_sizes, q_live.live, k_live)
 #define BSA_BY_TYPE(F, ...)                                     \
     do {                                                        \
         if (dtype == BSA_BF16) F(__bf16, ##__VA_ARGS__);        \
@@ -1253,7 +1402,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     } while (0)
     if (kept.keep) {
         hipLaunchKernelGGL(bwd_place_kernel, dim3((unsigned)((lrows + 3) / 4)), dim3(256), 0, st, paced, lens, bits, base, place, nbq, nbk, idx_stride,
-                           words, per_entry, lrows);
+                           words, nsub, lrows, q_live);
         if (masked) BSA_BY_TYPE(BSA_DKDV, true, true);
         else BSA_BY_TYPE(BSA_DKDV, false, true);
     }

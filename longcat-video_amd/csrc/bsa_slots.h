@@ -36,4 +36,23 @@ __device__ __forceinline__ Slots slots_of(const Grid3& g, int blk, int sub, int 
     return s;
 }
 
+// The same where the real slots of the chunk come first, in their order, and the padding behind them.
+__device__ __forceinline__ Slots packed_slots_of(const Grid3& g, int blk, int sub, int lane) {
+    const int nw = blk % g.Nw, nh = (blk / g.Nw) % g.Nh, nt = blk / (g.Nw * g.Nh);
+    const int ew = min(g.w, g.W - nw * g.w), eh = min(g.h, g.H - nh * g.h), et = min(g.t, g.T - nt * g.t);
+    const int rows = et * eh * ew;
+    if (rows == g.chunk()) return slots_of(g, blk, sub, lane);
+    const int r = sub * kTileSlots + lane, plane = r / ew, ti = plane / eh;
+    const int wi = r - plane * ew, hi = plane - ti * eh;
+    Slots s;
+    s.token = r < rows ? ((nt * g.t + ti) * g.H + nh * g.h + hi) * g.W + nw * g.w + wi : -1;
+    s.loc = ti | (hi << 8) | (wi << 16);
+    s.word = __ballot(r < rows);
+    return s;
+}
+// Halves of 32 slots that then hold real ones.
+__device__ __forceinline__ int live_halves(const Grid3& g, int blk) {
+    return (chunk_rows(g, blk / (g.Nw * g.Nh), (blk / g.Nw) % g.Nh, blk % g.Nw) + 31) / 32;
+}
+
 }  // namespace bsa

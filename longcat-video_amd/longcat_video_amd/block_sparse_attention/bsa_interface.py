@@ -767,21 +767,32 @@ def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_
 
 def _bsa_3d_backward_by_rearranging(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_q, chunk_k, sm_scale):
     """The same gradients the way a caller of the blocked-order entry points gets them: five rearrangements in
-    (bsa_interface.py:650-652 and their like for o and dO), bsa_bwd, three out.  Kept for the tests."""
+    (bsa_interface.py:650-652 and their like for o and dO), bsa_bwd, three out.  Inside a chunk the real slots come first, the
+    order bsa_bwd_3d sums them in.  Kept for the tests."""
     bs_q, bs_k = int(math.prod(chunk_q)), int(math.prod(chunk_k))
-    qp, _, _ = _permute(q, latent_q, chunk_q)
-    kp, _, valid = _permute(k, latent_k, chunk_k, want_valid=True)
-    vp, _, _ = _permute(v, latent_k, chunk_k)
-    op, _, _ = _permute(o, latent_q, chunk_q)
-    dop, _, _ = _permute(do, latent_q, chunk_q)                      # padded slots get a zero gradient
+    slots_q, order_q = _real_slots_first(latent_q, chunk_q, q.device)
+    slots_k, order_k = _real_slots_first(latent_k, chunk_k, q.device)
+    qp, op, dop = (_permute(t, latent_q, chunk_q)[0][:, :, order_q] for t in (q, o, do))      # padded slots get a zero gradient
+    kp, vp = (_permute(t, latent_k, chunk_k)[0][:, :, order_k] for t in (k, v))
+    valid = ((slots_k >= 0).view(-1, 64).long() << torch.arange(64, device=q.device)).sum(-1)
     padded_k = kp.shape[2] != k.shape[2]
     # lse in blocked order; a padded query slot has no keys as far as the backward is concerned (its p is 0)
-    slots = _slot_tokens(latent_q, chunk_q, q.device)
-    lse_p = torch.where(slots >= 0, lse[..., slots.clamp(min=0)], torch.full((), float("-inf"), device=q.device))
+    lse_p = torch.where(slots_q >= 0, lse[..., slots_q.clamp(min=0)], torch.full((), float("-inf"), device=q.device))
     dqp, dkp, dvp = (torch.empty_like(t) for t in (qp, kp, vp))
     attn_bwd_bsa_varlen(dop, qp, kp, vp, op, dqp, dkp, dvp, sm_scale, lse_p, walk, lens, bs_q, bs_k, None,
                         valid if padded_k else None)
-    return _unpermute(dqp, latent_q, chunk_q), _unpermute(dkp, latent_k, chunk_k), _unpermute(dvp, latent_k, chunk_k)
+    return (_unpermute(dqp[:, :, order_q.argsort()], latent_q, chunk_q),
+            *(_unpermute(t[:, :, order_k.argsort()], latent_k, chunk_k) for t in (dkp, dvp)))
+
+
+def _real_slots_first(latent_shape, chunk, device):
+    """The slots of every chunk with the padded ones behind the real ones: their tokens (-1: padding) and where in the blocked
+    order they lie."""
+    slots = _slot_tokens(latent_shape, chunk, device)
+    n = int(math.prod(chunk))
+    order = (slots < 0).view(-1, n).int().argsort(dim=-1, stable=True)
+    order = (order + torch.arange(0, slots.numel(), n, device=device).view(-1, 1)).reshape(-1)
+    return slots[order], order
 
 
 def _unpermute(xp, latent_shape, chunk):
