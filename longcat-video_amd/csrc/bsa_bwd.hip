@@ -361,14 +361,6 @@ __device__ inline void mfma_from(f32x16& acc, bf16x8 a, bf16x8 b, const f32x16& 
 __device__ inline void mfma_from(f32x16& acc, f16x8 a, f16x8 b, const f32x16& init) {
     asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "a"(b), "v"(init));
 }
-// the same with the B operand in an ordinary register
-__device__ inline void mfma_from_v(f32x16& acc, bf16x8 a, bf16x8 b, const f32x16& init) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(init));
-}
-__device__ inline void mfma_from_v(f32x16& acc, f16x8 a, f16x8 b, const f32x16& init) {
-    asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %3" : "=&v"(acc) : "v"(a), "v"(b), "v"(init));
-}
-
 // An MFMA reads its C operand for as long as its passes run, and nothing holds back a VALU write to those registers meanwhile
 // (fifteen wait states; the compiler adds them behind its own MFMAs, not behind an assembly statement, where it sees the
 // registers free at once).  The blocks that start a chain stay allocated up to here, at least two MFMAs on.
@@ -851,6 +843,7 @@ constexpr int kBwdHalfTile = kTileBytes / 2;                 // 32 query rows of
 constexpr int kBwdStats = 1024;                              // M2 (128 B), delta (128 B), -inf (128 B, for padded keys and repeated halves)
 constexpr int kBwdStage = 2 * kBwdHalfTile + kBwdStats;      // one half tile of queries: Q rows, dO rows, M2, delta
 constexpr int kBwdStages = 4;                                // two in use (this half, the next half's rows), two on their way
+constexpr int kBwdLoads = 9;                                 // DMA loads of a wavefront per half: its rows, 8 KB, and the numbers
 // The Q parts of all stages, then their dO parts, then their numbers: every LDS read of the loop is a lane's offset, which changes
 // with the pair of stages by one bit, and a constant below 2^16, which the instruction holds.
 constexpr int kBwdDout = kBwdStages * kBwdHalfTile, kBwdNumbers = 2 * kBwdStages * kBwdHalfTile;
@@ -915,8 +908,10 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         const int64_t row = bh * Sk + krow0 + 32 * wave + lr;
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            kreg[c] = *reinterpret_cast<const V8*>(ks + row * kD + 16 * c + 8 * lh);
-            vreg[c] = *reinterpret_cast<const V8*>(v + row * kD + 16 * c + 8 * lh);
+            const V8 a = *reinterpret_cast<const V8*>(ks + row * kD + 16 * c + 8 * lh), b = *reinterpret_cast<const V8*>(v + row * kD + 16 * c + 8 * lh);
+            // read by assembly MFMAs from accumulation registers
+            asm volatile("" : "=a"(kreg[c]) : "0"(a));
+            asm volatile("" : "=a"(vreg[c]) : "0"(b));
         }
     }
     bool key_ok = true;
@@ -968,19 +963,17 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     }
     __syncthreads();
     const int count_u = __builtin_amdgcn_readfirstlane(count);          // the same in every lane; the compiler cannot tell
-    // the walk's halves one after another; the entry of the next block is read from LDS while this one's are walked
+    // the walk's halves one after another, without a branch; the entry of the next block is read from LDS a half before it is used
     int next_block = 0, next_entry = 0, block_half = 0, half = 0, halves = 0;
     if (nhalves > 0) next_block = qlist[0];
-    auto next_half = [&]() -> int {
-        if (half == halves) {
-            const uint32_t entry = (uint32_t)__builtin_amdgcn_readfirstlane(next_block);
-            block_half = (int)(entry & ((1u << kBlockBits) - 1u)) * q_live.full;
-            halves = q_live.live != nullptr ? (int)(entry >> kBlockBits) : q_live.full;
-            half = 0;
-            next_entry = min(next_entry + 1, count_u - 1);
-            next_block = qlist[next_entry];
-        }
-        ++half;
+    auto next_half = [&](bool more) -> int {                     // !more: the last one again
+        const uint32_t entry = (uint32_t)__builtin_amdgcn_readfirstlane(next_block);
+        const bool fresh = more && half == halves;
+        block_half = fresh ? (int)(entry & ((1u << kBlockBits) - 1u)) * q_live.full : block_half;
+        halves = fresh ? (q_live.live != nullptr ? (int)(entry >> kBlockBits) : q_live.full) : halves;
+        half = (fresh ? 0 : half) + (more ? 1 : 0);
+        next_entry = min(next_entry + (fresh ? 1 : 0), count_u - 1);
+        next_block = qlist[next_entry];
         return block_half + half - 1;
     };
 
@@ -997,16 +990,26 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     const uint32_t voff_stats = (lane < 32 ? stat_gap : 0u) + (uint32_t)((lane & 31) * 4);      // 32 x M2, 32 x delta
     const char* tile_src = reinterpret_cast<const char*>(wave == 0 ? q : dout) + bh * Sq * (int64_t)(kD * 2);
     const char* stat_src = reinterpret_cast<const char*>(delta) + bh * Sq * 4;
-    // half hp of the walk into stage hp % kBwdStages; called for hp = 0, 1, 2, ...
-    auto issue = [&](int hp, int stage) {
-        if (hp >= nhalves) return;
-        const int64_t at = hp < n_real ? next_half() : block_half + half - 1;
-        const char* src = tile_src + at * kBwdHalfTile;
-        const uint32_t dst = lds0 + wave * kBwdDout + stage * kBwdHalfTile;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) load_to_lds_4x16(src + j * 4096, voff, dst + j * 4096);
-        if (wave == 0)
-            load_to_lds_4(stat_src + at * 128, voff_stats, lds0 + kBwdNumbers + stage * kBwdStats);
+    // half hp of the walk into stage hp % kBwdStages; called for hp = 0, 1, 2, ...  Behind the last half come copies of it, so that
+    // every half has kBwdLoads loads behind it to count; both wavefronts bring the numbers.
+    const char *src_now = nullptr, *stat_now = nullptr;
+    uint32_t dst_now = 0, stat_dst = 0;
+    auto issue_begin = [&](int hp) {
+        const int64_t at = next_half(hp < n_real);
+        const uint32_t stage = (uint32_t)hp & (kBwdStages - 1);
+        src_now = tile_src + at * kBwdHalfTile;
+        stat_now = stat_src + at * 128;
+        dst_now = lds0 + wave * kBwdDout + stage * kBwdHalfTile;
+        stat_dst = lds0 + kBwdNumbers + stage * kBwdStats;
+    };
+    auto issue_piece = [&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        if constexpr (i < 8) load_to_lds_16_at<1024 * (i & 3)>(src_now + (i >> 2) * 4096, voff[i & 3], dst_now + (i >> 2) * 4096);
+        else load_to_lds_4(stat_now, voff_stats, stat_dst);
+    };
+    auto issue = [&](int hp) {
+        issue_begin(hp);
+        static_for<kBwdLoads>([&](auto i_c) { issue_piece(i_c); });
     };
 
     // ---- LDS -> fragments
@@ -1022,165 +1025,178 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         for (int hi = 0; hi < 2; ++hi)
             toff[t][hi] = lds0 + (uint32_t)((4 * lh + tx + 8 * hi) * 256) + ((((uint32_t)(4 * t + 2 * g1 + ty)) ^ (uint32_t)((4 * tx) | (lh + 2 * hi))) << 4) +
                           (uint32_t)(tz * 8);
-    auto frag_tr_lds = [&](uint32_t part, int st2, int t) -> V8 {
-        const uint32_t base = part + (16 * st2) * 256;
-        const s16x4 lo = lds_read_tr16_at(toff[t][0] + base), hi = lds_read_tr16_at(toff[t][1] + base);
-        return __builtin_bit_cast(V8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    };
-    // One half tile of queries (32) against this wavefront's 32 keys is 32 MFMAs in two groups with the exponentials
-    // between them.  A wavefront has a SIMD to itself, so it overlaps them on its own: the S and dP products of the
-    // NEXT half (into a second pair of accumulators) are issued between the exponentials of this one.  S and dP
-    // accumulate in ordinary registers, where the exponentials read them: MFMAs from inline assembly, behind which
-    // the compiler adds no wait states - a pair is read a whole group of 16 MFMAs after it was written.
     // the queries' M2 as this lane's key sees them: -inf for a padded key, whose chains (its row of k_s is zeros) then give
     // p = exp2(-inf) = 0
     uint32_t numbers = lds0 + (uint32_t)(kBwdNumbers + 16 * lh), m2_at = numbers + (kMasked && !key_ok ? 256u : 0u);
-    auto starts = [&](int stage, bool real, f32x16& from_m, f32x16& from_d) {
-        const uint32_t m2_here = real ? m2_at : numbers + 256;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const f32x4_ mm = lds_read_at<f32x4_>(m2_here + (stage * kBwdStats + 32 * g));
-            const f32x4_ dd = lds_read_at<f32x4_>(numbers + (stage * kBwdStats + 128 + 32 * g));
-            from_m[4 * g] = mm.x; from_m[4 * g + 1] = mm.y; from_m[4 * g + 2] = mm.z; from_m[4 * g + 3] = mm.w;
-            from_d[4 * g] = dd.x; from_d[4 * g + 1] = dd.y; from_d[4 * g + 2] = dd.z; from_d[4 * g + 3] = dd.w;
-        }
-    };
-    auto products_and_exponentials = [&](auto stage_c, bool next_real, f32x16& s, f32x16& dp, f32x16& s_next, f32x16& dp_next, auto&& behind_requests) {
-        constexpr int stage = decltype(stage_c)::value;             // of the next half, in its pair
-        constexpr uint32_t qn = stage * kBwdHalfTile, dn = qn + kBwdDout;
-        // The chains of the next half start from its queries' -M2 and -delta (accumulator i <-> query
-        // 8 (i / 4) + 4 lh + i % 4 of the half, key lr), so S - M2 and dP - delta come out of the products and the
-        // exponentials need no subtraction.
-        f32x16 from_m, from_d;
-        starts(stage, next_real, from_m, from_d);
-        // Volatile assembly keeps the compiler from moving LDS reads across it, so the operands of a group of four
-        // MFMAs are requested a group ahead by hand.
-        V8 fq[2][2], fd[2][2];
-        auto request = [&](int g, int b) {
-            fq[b][0] = lds_read_at<V8>(roff[2 * g] + qn);
-            fd[b][0] = lds_read_at<V8>(roff[2 * g] + dn);
-            fq[b][1] = lds_read_at<V8>(roff[2 * g + 1] + qn);
-            fd[b][1] = lds_read_at<V8>(roff[2 * g + 1] + dn);
-        };
-        request(0, 0);
-        behind_requests();                       // the DMA set-up runs while the first LDS reads are on their way
-#pragma unroll
-        for (int g4 = 0; g4 < 4; ++g4) {
-            const int c = 2 * g4, b = g4 & 1;
-            if (g4 < 3) request(g4 + 1, b ^ 1);
-            if (g4 == 0) {
-                mfma_from_v(s_next, fq[b][0], kreg[0], from_m);
-                mfma_from_v(dp_next, fd[b][0], vreg[0], from_d);
-            } else {
-                mfma_s<false, false>(s_next, fq[b][0], kreg[c]);
-                mfma_s<false, false>(dp_next, fd[b][0], vreg[c]);
-            }
-            mfma_s<false, false>(s_next, fq[b][1], kreg[c + 1]);
-            mfma_s<false, false>(dp_next, fd[b][1], vreg[c + 1]);
-            if (g4 == 0) keep_start(from_m, from_d);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int i = 4 * g4 + j;
-                const float pi = __builtin_amdgcn_exp2f(s[i]);  // s holds S - M2, dp holds dP - delta
-                s[i] = pi;                                   // P
-                dp[i] = pi * dp[i];                          // dS
-            }
-        }
-    };
     char* ds_item = !kKeep ? nullptr
         : ds_out + bh * pairs_per_head * kDsPairBytes + ((int64_t)__builtin_amdgcn_readfirstlane(unit_base[block]) + (item - block * nsub)) * kDsUnitBytes + wave * 2048;
-    auto gradients = [&](auto stage_c, char* ds_to, const f32x16& p, const f32x16& ds) {
-        constexpr int stage = decltype(stage_c)::value;             // of this half, in its pair
-        constexpr uint32_t qt = stage * kBwdHalfTile, dt = qt + kBwdDout;
-#pragma unroll
-        for (int st2 = 0; st2 < 2; ++st2) {
-            const V8 bp = pack8<T, V8>(p, st2), bds = pack8<T, V8>(ds, st2);
-            if (kKeep)
-                __builtin_nontemporal_store(bds, reinterpret_cast<V8*>(ds_to + st2 * 1024 + lane * 16));
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                acc_dv[t] = mfma32(frag_tr_lds(dt, st2, t), bp, acc_dv[t]);
-                acc_dk[t] = mfma32(frag_tr_lds(qt, st2, t), bds, acc_dk[t]);
-            }
-        }
-    };
-    // During half hp the rows of half hp + 1 are read, so at its end the loads of half hp + 2 must have landed; the
-    // half requested after it may still be on its way (wavefront 0 issues 9 loads per half, wavefront 1 issues 8).
+    // P and dS of a half as B operands, and the transposed fragments of its rows (dO and Q of d tile t at 2 t and 2 t + 1): its first
+    // and its last 16 queries
+    V8 p_ab[2], ds_ab[2], tr_ab[2][8];
+    V8 fq[4], fd[4];                                             // row fragments c & 3
+    // One half tile of queries (32) against this wavefront's 32 keys is 32 MFMAs, and a wavefront has a SIMD to itself: what it
+    // does besides has to stand between them, and what they read has to be asked for long before.  A step issues, in slots of one
+    // MFMA each, with half hp's S - M2 and dP - delta complete (s, dp):
+    //    0 ..  7   dV, dK += the last 16 queries of half hp - 1 (their operands are in registers: nothing is waited for behind the barrier)
+    //    8 .. 23   S, dP of half hp + 1, into (s_next, dp_next)
+    //   24 .. 31   dV, dK += the first 16 queries of half hp
+    // and behind the MFMA of a slot its share of the rest: the chains' start values and row fragments of half hp + 1 four to eight
+    // slots before their MFMA, the transposed fragments of half hp sixteen, its exponentials, products and roundings, the DMA
+    // loads of half hp + 3.  (Left to the compiler, the transposed reads stood right in front of their MFMAs, four round trips to
+    // LDS a half, and the exponentials in bunches: 2 150 clocks a half beside 1 024 of products.)
+    // S and dP accumulate in ordinary registers, where the exponentials read them: MFMAs from inline assembly, behind which the
+    // compiler adds no wait states - a pair is first read nine MFMAs after its last product.
     auto step = [&](auto odd_c, int hp, f32x16& s, f32x16& dp, f32x16& s_next, f32x16& dp_next) {
         constexpr int odd = decltype(odd_c)::value;                  // hp & 1
-        // The stages come in two pairs; a lane's offsets point into the pair that is read next and go over to the other
-        // one with a bit, the rows' behind the even half (whose successor's successor lies there), the transposed reads' behind the odd.
-        if (odd) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) roff[c] ^= 2 * kBwdHalfTile;
-            numbers ^= 2 * kBwdStats;
-            m2_at ^= 2 * kBwdStats;
-        }
-        // half hp + 3 takes the stage that half hp - 1 was read from: both wavefronts are past the barrier behind it
+        constexpr uint32_t qn = (odd ^ 1) * kBwdHalfTile, dn = qn + kBwdDout;      // rows of half hp + 1, in its pair of stages
+        constexpr uint32_t qt = odd * kBwdHalfTile, dt = qt + kBwdDout;            // rows of half hp
         // the halves with an odd number alone may be the one that repeats
-        products_and_exponentials(std::integral_constant<int, odd ^ 1>{}, odd || hp + 1 < n_real, s, dp, s_next, dp_next, [&]() { issue(hp + 3, (hp + 3) & 3); });
+        const uint32_t m2_here = odd || hp + 1 < n_real ? m2_at : numbers + 256;
+        char* const ds_to = !odd || hp < n_real ? ds_item : ds_spare;
+        auto exponential = [&](int e) {
+            s[e] = __builtin_amdgcn_exp2f(s[e]);                     // S - M2 -> P
+            asm volatile("" : "+v"(s[e]));
+        };
+        auto product = [&](int e) {
+            dp[e] = s[e] * dp[e];                                    // dP - delta -> dS
+            asm volatile("" : "+v"(dp[e]));
+        };
+        auto round_pair = [&](V8& to, const f32x16& x, int e) {
+            to[e & 7] = (T)x[e];
+            to[(e + 1) & 7] = (T)x[e + 1];
+            asm volatile("" : "+v"(to));
+        };
+        s16x4 lo[2];                                                 // first halves of transposed fragments on their way
+        auto read_transposed = [&](auto n_c) {                       // n = 0 .. 31: 16 st2 + 4 t + 2 (Q or dO) + which half
+            constexpr int n = decltype(n_c)::value, st2 = n >> 4, t = (n >> 2) & 3, of_q = (n >> 1) & 1;
+            constexpr uint32_t base = (of_q ? qt : dt) + 16 * st2 * 256;
+            if constexpr ((n & 1) == 0) {
+                lo[st2] = lds_read_tr16_at(toff[t][0] + base);
+            } else {
+                const s16x4 hi = lds_read_tr16_at(toff[t][1] + base);
+                tr_ab[st2][2 * t + of_q] = __builtin_bit_cast(V8, (s16x8)__builtin_shufflevector(lo[st2], hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+        };
         __builtin_amdgcn_sched_barrier(0);
-        gradients(odd_c, !odd || hp < n_real ? ds_item : ds_spare, s, dp);
-        if (odd) {
-#pragma unroll
-            for (int t = 0; t < 4; ++t) { toff[t][0] ^= 2 * kBwdHalfTile; toff[t][1] ^= 2 * kBwdHalfTile; }
-        }
+        static_for<32>([&](auto slot_c) {
+            constexpr int i = decltype(slot_c)::value;
+            // ---- the MFMA
+            if constexpr (i < 8 || i >= 24) {
+                constexpr int st2 = i < 8 ? 1 : 0, x = i & 7, t = x >> 1;
+                if constexpr ((x & 1) == 0) acc_dv[t] = mfma32(tr_ab[st2][x], p_ab[st2], acc_dv[t]);
+                else acc_dk[t] = mfma32(tr_ab[st2][x], ds_ab[st2], acc_dk[t]);
+            } else {
+                constexpr int c = (i - 8) >> 1;
+                if constexpr ((i & 1) == 0) mfma_s<false, true>(s_next, fq[c & 3], kreg[c]);
+                else mfma_s<false, true>(dp_next, fd[c & 3], vreg[c]);
+            }
+            // ---- LDS
+            if constexpr (i < 4) {                                   // accumulator e <-> query 8 (e / 4) + 4 lh + e % 4 of the half, key lr
+                const f32x4_ mm = lds_read_at<f32x4_>(m2_here + ((odd ^ 1) * kBwdStats + 32 * i));
+                const f32x4_ dd = lds_read_at<f32x4_>(numbers + ((odd ^ 1) * kBwdStats + 128 + 32 * i));
+                s_next[4 * i] = mm.x; s_next[4 * i + 1] = mm.y; s_next[4 * i + 2] = mm.z; s_next[4 * i + 3] = mm.w;
+                dp_next[4 * i] = dd.x; dp_next[4 * i + 1] = dd.y; dp_next[4 * i + 2] = dd.z; dp_next[4 * i + 3] = dd.w;
+            } else if constexpr (i < 8) {
+                fq[i - 4] = lds_read_at<V8>(roff[i - 4] + qn);
+                fd[i - 4] = lds_read_at<V8>(roff[i - 4] + dn);
+            } else if constexpr (i < 16) {
+                constexpr int c = 4 + ((i - 8) >> 1);
+                if constexpr ((i & 1) == 0) fq[c & 3] = lds_read_at<V8>(roff[c] + qn);
+                else fd[c & 3] = lds_read_at<V8>(roff[c] + dn);
+            }
+            if constexpr (i >= 8 && i < 24) read_transposed(std::integral_constant<int, i - 8>{});
+            if constexpr (i >= 16 && i < 24) read_transposed(std::integral_constant<int, i>{});
+            if constexpr (i >= 24 && i < 28) {
+                read_transposed(std::integral_constant<int, 24 + 2 * (i - 24)>{});
+                read_transposed(std::integral_constant<int, 25 + 2 * (i - 24)>{});
+            }
+            // ---- the DMA loads of half hp + 3, into the stage that half hp - 1 was read from: both wavefronts are past the barrier behind it
+            if constexpr (i == 0) issue_begin(hp + 3);
+            if constexpr (i >= 1 && i <= kBwdLoads) issue_piece(std::integral_constant<int, i - 1>{});
+            // ---- exponentials behind slots 0, 1, 3, 4, 6, 7, ..., each product a slot later
+            if constexpr (i < 24 && i % 3 != 2) exponential(i / 3 * 2 + i % 3);
+            if constexpr (i < 24 && i % 3 != 0) product(i / 3 * 2 + i % 3 - 1);
+            // ---- roundings: the first 16 queries' elements are there behind slot 11, all behind slot 23
+            if constexpr (i == 12 || i == 15 || i == 18 || i == 21) {
+                constexpr int e = 2 * ((i - 12) / 3);
+                round_pair(p_ab[0], s, e);
+                round_pair(ds_ab[0], dp, e);
+            }
+            if constexpr (i >= 24 && i < 28) {
+                constexpr int e = 8 + 2 * (i - 24);
+                round_pair(p_ab[1], s, e);
+                round_pair(ds_ab[1], dp, e);
+            }
+            if constexpr (kKeep && (i == 24 || i == 28))
+                __builtin_nontemporal_store(ds_ab[i == 24 ? 0 : 1], reinterpret_cast<V8*>(ds_to + (i == 24 ? 0 : 1024) + lane * 16));
+            // ---- The stages come in two pairs; a lane's offsets point into the pair that is read next and go over to the other one
+            // with a bit, the rows' behind the even half (whose successor's successor lies there), the transposed reads' behind the odd.
+            if constexpr (!odd && i >= 24) roff[i - 24] ^= 2 * kBwdHalfTile;
+            if constexpr (!odd && i == 30) { numbers ^= 2 * kBwdStats; m2_at ^= 2 * kBwdStats; }
+            if constexpr (odd && i >= 28) { toff[i - 28][0] ^= 2 * kBwdHalfTile; toff[i - 28][1] ^= 2 * kBwdHalfTile; }
+            __builtin_amdgcn_sched_barrier(0);
+        });
         if (kKeep) ds_item += (int64_t)nsub * kDsUnitBytes;
-        // the chains into (s_next, dp_next) end here, sixteen MFMAs behind their last one
+        // the chains into (s_next, dp_next) end here, eight MFMAs behind their last one
         mfma_chain_end(s_next); mfma_chain_end(dp_next);
-        // With kKeep the two stores of this half and those of the one before may be on their way as well: a store is
-        // acknowledged later than a load (waiting for those of the half before cost 0.4 of 4.2 ms at 480p).
-        if (hp + 3 >= nhalves) {
-            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(kKeep ? 4 : 0) : "memory");
-        } else if (kKeep && hp == 0) {                           // no half before
-            if (wave == 0) asm volatile("s_waitcnt vmcnt(11) lgkmcnt(0)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(10) lgkmcnt(0)" ::: "memory");
-        } else {
-            if (wave == 0) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(kKeep ? 13 : 9) : "memory");
-            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(kKeep ? 12 : 8) : "memory");
-        }
+        // The loads of half hp + 2 must have landed; behind them are on their way those of half hp + 3 and, with kKeep, the two stores
+        // of this half and those of the one before: a store is acknowledged later than a load (waiting for those of the half before
+        // cost 0.4 of 4.2 ms at 480p).
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kKeep ? kBwdLoads + 4 : kBwdLoads) : "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);                          // lgkmcnt(0): this half's stage has been read
+        asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
     };
     if (nhalves > 0) {
-        issue(0, 0);
-        issue(1, 1);
-        issue(2, 2);
-        if (nhalves > 2) {
-            if (wave == 0) asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
-        } else {
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        issue(0);
+        issue(1);
+        issue(2);
+        if (kKeep) {                             // as many stores as a half before the first would have left on their way
+            const V8 none = {};
+            __builtin_nontemporal_store(none, reinterpret_cast<V8*>(ds_spare + lane * 16));
+            __builtin_nontemporal_store(none, reinterpret_cast<V8*>(ds_spare + 1024 + lane * 16));
         }
+        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kKeep ? kBwdLoads + 2 : kBwdLoads) : "memory");
         __builtin_amdgcn_s_barrier();
         if (wave >= key_halves) {                // no keys: the rows alone
             for (int hp = 0; hp < nhalves; ++hp) {
-                issue(hp + 3, (hp + 3) & 3);
-                if (hp + 3 >= nhalves) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                else asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+                issue(hp + 3);
+                asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kBwdLoads) : "memory");
                 __builtin_amdgcn_s_barrier();
             }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS that is no longer this workgroup's
             return;
         }
         f32x16 s0, dp0, s1, dp1;
-        {
-            constexpr uint32_t qn = 0, dn = kBwdDout;
-            f32x16 from_m, from_d;
-            starts(0, true, from_m, from_d);
-            mfma_from_v(s0, lds_read_at<V8>(roff[0] + qn), kreg[0], from_m);
-            mfma_from_v(dp0, lds_read_at<V8>(roff[0] + dn), vreg[0], from_d);
 #pragma unroll
-            for (int c = 1; c < 8; ++c) {
-                mfma_s<false, false>(s0, lds_read_at<V8>(roff[c] + qn), kreg[c]);
-                mfma_s<false, false>(dp0, lds_read_at<V8>(roff[c] + dn), vreg[c]);
-            }
-            keep_start(from_m, from_d);
-            asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
-            mfma_chain_end(s0); mfma_chain_end(dp0);
+        for (int g = 0; g < 4; ++g) {
+            const f32x4_ mm = lds_read_at<f32x4_>(m2_at + 32 * g), dd = lds_read_at<f32x4_>(numbers + (128 + 32 * g));
+            s0[4 * g] = mm.x; s0[4 * g + 1] = mm.y; s0[4 * g + 2] = mm.z; s0[4 * g + 3] = mm.w;
+            dp0[4 * g] = dd.x; dp0[4 * g + 1] = dd.y; dp0[4 * g + 2] = dd.z; dp0[4 * g + 3] = dd.w;
         }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            mfma_s<false, true>(s0, lds_read_at<V8>(roff[c]), kreg[c]);
+            mfma_s<false, true>(dp0, lds_read_at<V8>(roff[c] + kBwdDout), vreg[c]);
+        }
+        asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+        mfma_chain_end(s0); mfma_chain_end(dp0);
+        // nothing lies in front of the first half
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { p_ab[1][e] = (T)0.f; ds_ab[1][e] = (T)0.f; }
+#pragma unroll
+        for (int x = 0; x < 8; ++x) tr_ab[1][x] = p_ab[1];
         for (int hp = 0; hp < nhalves; hp += 2) {                                // halves come in pairs
             step(std::integral_constant<int, 0>{}, hp, s0, dp0, s1, dp1);
             step(std::integral_constant<int, 1>{}, hp + 1, s1, dp1, s0, dp0);
         }
+        // the last 16 queries of the last half
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            acc_dv[t] = mfma32(tr_ab[1][2 * t], p_ab[1], acc_dv[t]);
+            acc_dk[t] = mfma32(tr_ab[1][2 * t + 1], ds_ab[1], acc_dk[t]);
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // nothing may land in LDS that is no longer this workgroup's
     }
     // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, key lr
     {

@@ -48,17 +48,6 @@ constexpr int kListEntries = 4096;    // longest list a work item can walk (its 
 constexpr int kHalfEntries = 4096;    // ... of halves
 
 // ------------------------------------------------------------------ attention
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant expression
-// in every copy of the body (the register arrays of the kernel must never be indexed by a run-time value).
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
 // acc + x[2e]^2 + x[2e+1]^2 for a fragment of eight 16-bit values
 __device__ __forceinline__ float dot2_self(bf16x8 x, int e, float acc) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));

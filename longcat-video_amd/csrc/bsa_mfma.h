@@ -4,6 +4,7 @@
 #include "bsa_common.h"
 
 #include <type_traits>
+#include <utility>
 
 namespace bsa {
 namespace mfma {
@@ -56,6 +57,12 @@ __device__ inline void load_to_lds_4x16(const void* sbase, const uint32_t (&voff
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
                  "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072"
                  :: "s"(lds_addr), "v"(voff[0]), "v"(voff[1]), "v"(voff[2]), "v"(voff[3]), "s"(sbase) : "memory");
+}
+// One of them: kOffset counts for both addresses.
+template <int kOffset>
+__device__ inline void load_to_lds_16_at(const void* sbase, uint32_t voff, uint32_t lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%3"
+                 :: "s"(lds_addr), "v"(voff), "s"(sbase), "n"(kOffset) : "memory");
 }
 // The same with 4 bytes per lane: the LDS address is m0 + 4*lane.
 __device__ inline void load_to_lds_4(const void* sbase, uint32_t voff, uint32_t lds_addr) {
@@ -112,6 +119,17 @@ __device__ inline void mfma_s(f32x16& acc, f16x8 a, f16x8 b) {
         if (kAgprB) asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
         else asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
     }
+}
+
+// f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant expression
+// in every copy of the body (register arrays must never be indexed by a run-time value).
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
 }
 
 // Marks the end of a chain of assembly MFMAs into `acc`: from here on the accumulators may be read, written or
