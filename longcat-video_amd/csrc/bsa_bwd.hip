@@ -105,6 +105,51 @@ __global__ __launch_bounds__(256) void bwd_scale_kernel(const T* __restrict__ k,
     *reinterpret_cast<V8*>(ks + i * 8) = x;
 }
 
+// Transposed fragments of k_s, what the dQ product takes as its A operand: per 64-key tile (16 KB) [half kh][key step st][d tile
+// t][lane l][8 elements], element j of lane l = k_s[key 32 kh + 16 st + 8 (j >> 2) + 4 (l >> 5) + (j & 3)][d = 32 t + (l & 31)], the
+// keys of a step in accumulator order.  A workgroup of 256 turns its tile in 16 KB of LDS: row r of a half lies there with unit
+// p ^ f(r) at its 16-byte slot p, f(r) = ((r & 3) << 2) | ((r >> 2) & 3), as transposing reads want it.
+__device__ __forceinline__ void put_turned_row(char* lds, int row, int c16, const uint4& x) {
+    const int r = row & 31, f = ((r & 3) << 2) | ((r >> 2) & 3);
+    *reinterpret_cast<uint4*>(lds + (row >> 5) * kBwdHalfTileBytes + r * 256 + ((c16 ^ f) << 4)) = x;
+}
+// The lane's offset of the first (hi: second) four keys of a fragment of d tile t in a half that lies like this; 4096 further per
+// step of 16 keys.
+__device__ __forceinline__ uint32_t turned_offset(int lane, int t, int hi) {
+    const int lh = lane >> 5, s16 = lane & 15, g1 = (lane >> 4) & 1, tx = s16 >> 2, ty = (s16 & 3) >> 1, tz = s16 & 1;
+    return (uint32_t)((4 * lh + tx + 8 * hi) * 256) + ((((uint32_t)(4 * t + 2 * g1 + ty)) ^ (uint32_t)((4 * tx) | (lh + 2 * hi))) << 4) +
+           (uint32_t)(tz * 8);
+}
+__device__ __forceinline__ void store_turned_tile(const char* lds, char* out, int halves) {
+    const int lane = threadIdx.x & 63, t = threadIdx.x >> 6;                 // a wavefront per d tile
+    const uint32_t lo_at = turned_offset(lane, t, 0), hi_at = turned_offset(lane, t, 1);
+    for (int x = 0; x < 2 * halves; ++x) {                                   // 16-key steps
+        const s16x4 lo = lds_read_tr16(lds + x * 4096 + lo_at), hi = lds_read_tr16(lds + x * 4096 + hi_at);
+        *reinterpret_cast<s16x8*>(out + x * 4096 + t * 1024 + lane * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+}
+// k_s as bwd_scale_kernel makes it, in transposed fragments: a workgroup per tile of 64 rows.
+template <typename T>
+__global__ __launch_bounds__(256) void bwd_scale_turned_kernel(const T* __restrict__ k, char* __restrict__ ks_turned, float c,
+                                                               const uint64_t* __restrict__ tile_valid, int tiles) {
+    typedef typename Vec8<T>::type V8;
+    __shared__ __attribute__((aligned(16))) char turned[kTileBytes];
+    const int c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
+    const int64_t tile = blockIdx.x;
+    const uint64_t word = tile_valid != nullptr ? tile_valid[tile % tiles] : ~0ull;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        V8 x = *reinterpret_cast<const V8*>(k + (tile * kTile + rg + 16 * i) * kD + c16 * 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * c);
+        uint4 raw = __builtin_bit_cast(uint4, x);
+        keep_if(raw, (word >> (rg + 16 * i)) & 1ull);
+        put_turned_row(turned, rg + 16 * i, c16, raw);
+    }
+    __syncthreads();
+    store_turned_tile(turned, ks_turned + tile * kTileBytes, 2);
+}
+
 // Where a gradient row goes when the caller's tensors are in token order: the token of every blocked-order slot of one
 // (batch, head) (-1: padding, nothing is stored) and the element strides of the destination.  rows null: blocked order.
 struct BwdStore {
@@ -112,16 +157,14 @@ struct BwdStore {
     int64_t sB, sH, sS;
     int Hn;
 };
-template <typename T>
-__device__ __forceinline__ T* store_row(T* blocked, const BwdStore& w, int64_t bh, int64_t rows_per_bh, int64_t slot) {
-    if (w.rows == nullptr) return blocked + (bh * rows_per_bh + slot) * kD;
-    const int32_t token = w.rows[slot];
-    if (token < 0) return nullptr;
-    return blocked + (bh / w.Hn) * w.sB + (bh % w.Hn) * w.sH + (int64_t)token * w.sS;
-}
+// Where the kernels read k and v: element strides (in blocked order as in token order).
+struct BwdLoad {
+    const void* p;
+    int64_t sB, sH, sS;
+};
 
-// What the kernels below need of tensors in token order, in one launch (HBM-bound): q, dO and v in blocked order, k_s, delta and
-// M2 per slot (padded slots: zero rows, delta -0, M2 -inf, so that their p is 0), the row tables of both grids, the validity
+// What the kernels below need of tensors in token order, in one launch (HBM-bound): q and dO in blocked order, k_s in transposed
+// fragments (where dS is kept) or in blocked order beside v (for dQ from scratch), delta and M2 per slot (padded slots: zero rows, delta -0, M2 -inf, so that their p is 0), the row tables of both grids, the validity
 // words of the keys, and the bit matrix cleared.  A workgroup per 64-slot tile; workgroups 0 .. wg_q - 1 take tiles of the
 // queries, the next wg_k tiles of the keys, the rest words of the matrix.  delta and M2 as bwd_rows_kernel takes them.
 // On a padded grid the real rows of a chunk come first, so that the halves of 32 slots behind them hold none: these are neither
@@ -136,7 +179,7 @@ struct BwdPrep {
     int64_t q_st[3], o_st[3], do_st[3], k_st[3], v_st[3];      // element strides {batch, head, token}
     const float* lse;                                          // [B * Hn][tokens]
     int64_t q_tokens;
-    uint16_t *q_blocked, *dout_blocked, *ks, *v_blocked;
+    uint16_t *q_blocked, *dout_blocked, *ks, *v_blocked;      // v_blocked null: k_s in transposed fragments
     float *delta, *m2;
     int32_t *q_rows, *k_rows;
     uint64_t* valid;
@@ -150,6 +193,7 @@ struct BwdPrep {
 template <typename T>
 __global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, int wg_k) {
     typedef typename Vec8<T>::type V8;
+    __shared__ __attribute__((aligned(16))) char turned[kTileBytes];
     const int lane = threadIdx.x & 63, c16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
     const int w = blockIdx.x;
     if (w >= wg_q + wg_k) {
@@ -211,10 +255,14 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, i
             }
         }
     } else {
+        const bool rows = a.v_blocked != nullptr;
         uint4 k[4], v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (i < sweeps) { k[i] = at(a.k, a.k_st, i); v[i] = at(a.v, a.v_st, i); }
+            if (i < sweeps) {
+                k[i] = at(a.k, a.k_st, i);
+                if (rows) v[i] = at(a.v, a.v_st, i);
+            }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             if (i >= sweeps) break;
@@ -223,10 +271,18 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(BwdPrep a, int wg_q, i
 #pragma unroll
             for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * a.c);
             uint4 ks = __builtin_bit_cast(uint4, x);
-            keep_if(ks, real); keep_if(v[i], real);
-            put(a.ks, i, ks);
-            put(a.v_blocked, i, v[i]);
+            keep_if(ks, real);
+            if (rows) {
+                keep_if(v[i], real);
+                put(a.ks, i, ks);
+                put(a.v_blocked, i, v[i]);
+            } else {
+                put_turned_row(turned, rg + 16 * i, c16, ks);
+            }
         }
+        if (rows) return;
+        __syncthreads();
+        store_turned_tile(turned, reinterpret_cast<char*>(a.ks) + (int64_t)id * kTileBytes, sweeps / 2);
     }
 }
 
@@ -313,11 +369,12 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
 
 // place[row * stride + e] = the first dS unit of list entry e in the order in which the dK / dV kernel walks its head: KV blocks
 // ascending, inside a block its query blocks ascending (the halves of the query blocks in front of this one among the bits of
-// the block's row).
+// the block's row).  zeros: kDsUnitBytes to clear.
 __global__ __launch_bounds__(256) void bwd_place_kernel(const int32_t* __restrict__ idx, const int32_t* __restrict__ lens,
                                                         const uint32_t* __restrict__ bits, const int32_t* __restrict__ base,
                                                         int32_t* __restrict__ place, int nbq, int nbk, int stride, int words,
-                                                        int tiles_per_block, int64_t rows, LiveHalves q) {
+                                                        int tiles_per_block, int64_t rows, LiveHalves q, uint4* __restrict__ zeros) {
+    if (blockIdx.x == 0) zeros[threadIdx.x] = make_uint4(0u, 0u, 0u, 0u);
     const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= rows) return;
     const int64_t bh = row / nbq;
@@ -381,6 +438,37 @@ __device__ __forceinline__ int query_halves(const int32_t* q_live, int item, int
     if (q_live == nullptr) return 2;
     const int tile = item - head * sz.tiles, block = tile / sz.by_block;
     return min(max(__builtin_amdgcn_readfirstlane(q_live[block]) - 2 * (tile - block * tiles_per_block), 0), 2);
+}
+// Sixteen values of a lane's row, accumulator i <-> column 8 (i / 4) + 4 lh + i % 4, rounded and stored as 16-byte pieces: lanes l
+// and l + 32, which hold one row, trade so that each has eight columns in a row of two of the four groups.
+template <typename T>
+__device__ __forceinline__ void store_columns(T* row, bool real, const float (&x)[16], int lane) {
+    typedef T T4 __attribute__((ext_vector_type(4)));
+    uint2 p[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) p[g] = __builtin_bit_cast(uint2, T4{(T)x[4 * g], (T)x[4 * g + 1], (T)x[4 * g + 2], (T)x[4 * g + 3]});
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+        const auto a = __builtin_amdgcn_permlane32_swap(p[g].x, p[g + 1].x, false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(p[g].y, p[g + 1].y, false, false);
+        if (real) *reinterpret_cast<uint4*>(row + 8 * g + 8 * (lane >> 5)) = make_uint4(a[0], b[0], a[1], b[1]);
+    }
+}
+// dQ of a wavefront's 64 rows: accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, query lr (+ 32), row `rows` of the
+// destination (negative: a padded slot of a token-order destination)
+template <typename T>
+__device__ __forceinline__ void store_dq(const f32x16 (&acc)[4][2], T* dq, const BwdStore& w, int64_t bh, int64_t Sq, const int64_t (&rows)[2], int lane) {
+    T* const base = w.rows == nullptr ? dq + bh * Sq * kD : dq + (bh / w.Hn) * w.sB + (bh % w.Hn) * w.sH;
+    const int64_t pitch = w.rows == nullptr ? kD : w.sS;
+#pragma unroll
+    for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            float x[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[i] = acc[t][qq][i] * kLn2;
+            store_columns(base + rows[qq] * pitch + 32 * t, rows[qq] >= 0, x, lane);
+        }
 }
 __device__ __forceinline__ int wave_sum(int x) {
 #pragma unroll
@@ -608,50 +696,41 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
             step(hp + 1, sb, dpb, sa, dpa);
         }
     }
-    // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, query lr (+ 32)
-#pragma unroll
-    for (int qq = 0; qq < 2; ++qq) {
-        T* out = store_row(dq, dq_to, bh, Sq, qrow0 + 32 * qq + lr);
-        if (out == nullptr) continue;                            // a padded slot of a token-order destination
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                T x[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) x[j] = (T)(acc[t][qq][4 * g4 + j] * kLn2);
-                *reinterpret_cast<uint2*>(out + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(x);
-            }
-    }
+    int64_t rows[2] = {qrow0 + lr, qrow0 + 32 + lr};
+    if (dq_to.rows != nullptr) { rows[0] = dq_to.rows[rows[0]]; rows[1] = dq_to.rows[rows[1]]; }
+    store_dq<T>(acc, dq, dq_to, bh, Sq, rows, lane);
 }
 
 // ------------------------------------------------------------------ dQ from kept dS
-// Where the dK / dV kernel keeps the dS it rounds for its own product (kDsPairBytes per tile pair), dQ^T += K_s^T dS^T is all
-// that is left to do: one product of three and no exponentials.  A wavefront walks the list of its 64 query rows as in
-// bwd_dq_lds_kernel; per half tile (32 keys) the K_s rows (8 KB) and the dS of its 64 queries (4 KB) go into one of three
-// LDS stages, and both operands come out with transposing reads: the next half's while this one's sixteen MFMAs run, so all
-// three stages can be on their way.  Bound by the 24 KB per pair that enter the CU (32 MFMAs take two thirds of the time of
-// their loads at 64 B/clk); dS is read once, from beyond the L2.
+// Where the dK / dV kernel keeps the dS it rounds for its own product (kDsUnitBytes per 32 queries and tile), dQ^T += K_s^T dS^T
+// is all that is left to do: one product of three and no exponentials.  A wavefront walks the list of its 64 query rows as in
+// bwd_dq_lds_kernel.  Per half tile (32 keys) the transposed fragments of K_s (8 KB) come straight into the registers of the A
+// operand; the dS of its 64 queries (4 KB) come into registers too and go through 4 KB of LDS, out of which transposing reads make
+// the B operand.  kDsqAhead halves are on their way: a wavefront has its SIMD and all of its registers to itself, and what a
+// half needs is dealt out behind the sixteen MFMAs of the one before.  (Both through three stages of LDS, 36 KB a wavefront: the
+// loads could only be issued once the reads before them were done, in front of the products: 1.75 ms for 32 heads of 24x30x52,
+// 1.50 with everything in L2.)
 //   dS in units of 32 queries against a 64-key tile, in the order in which the dK / dV kernel walks them (the tiles of a KV block next
 //   to one another): [key half][16-query step st][lane][8 elements], lane = 32 lh + key: the queries 16 st + 4 lh .. + 3 and 8
 //   further (the accumulator order of the dK / dV kernel), 1 KB per store instruction.
-//   In LDS: unit (key, lh, st) at 16-byte slot 4 key + 2 lh + st of its 2 KB block, so that the 32 lanes of a pass of a
-//   transposing read (4 keys x 16 queries, two groups) cover 256 consecutive bytes.
+//   In LDS: unit (key, lh, st) at 16-byte slot 4 key + ((2 lh + st) ^ (key >> 1 & 3)) of its 2 KB block: the 32 lanes of a pass of
+//   a transposing read (4 keys x 16 queries, two groups) cover 256 consecutive bytes, and eight lanes that write lie on different
+//   banks.  (The order of the slots on the global side instead, as the LDS DMA needs it, gives every lane of a load a cache
+//   line of its own: 64 clocks of the address unit for 16, and 1.81 ms.)
 constexpr int kDsPairBytes = kTile * kTile * 2, kDsUnitBytes = kDsPairBytes / 2;
-constexpr int kDsqStage = kBwdHalfTileBytes + kDsPairBytes / 2;
-constexpr int kDsqStages = 3;
-constexpr int kDsqLoads = kDsqStage / 1024;      // LDS DMA instructions per half
+constexpr int kDsqAhead = 4;
 
 template <typename T>
-__global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict__ ks, const char* __restrict__ ds,
+__global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const char* __restrict__ ks_turned, const char* __restrict__ ds, const char* __restrict__ zeros,
                                                             const int32_t* __restrict__ idx, const int32_t* __restrict__ place,
                                                             const int32_t* __restrict__ lens, T* __restrict__ dq, int64_t Sq,
                                                             int64_t Sk, int bs_q, int bs_k, int stride, int item_begin, int item_end,
                                                             int round, int64_t pairs_per_head, BwdStore dq_to, DqSizes sz,
                                                             const int32_t* __restrict__ q_live, const int32_t* __restrict__ k_live) {
     typedef typename Vec8<T>::type V8;
-    extern __shared__ __attribute__((aligned(1024))) char dsq_ring[];
+    __shared__ __attribute__((aligned(16))) char turn[2 * 2048];
     const int lane = threadIdx.x, lr = lane & 31, lh = lane >> 5;
+    touch_arguments<decltype(bwd_dq_from_ds_kernel<T>)>();
     int item;
     {
         const int local = blockIdx.x, r0 = local / sz.by_round * round;
@@ -661,10 +740,31 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
     const int head = item / sz.by_tiles, lrow_n = item / sz.by_block;          // the tiles of a block lie next to each other
     const int64_t bh = head, qrow0 = (int64_t)(item - head * sz.tiles) * kTile, lrow = lrow_n;
     const int nbk = (int)(Sk / kTile) / sz.by_sub, nsub = bs_k / kTile, sub_q = item - lrow_n * (bs_q / kTile);
-    const int q_halves = query_halves(q_live, item, head, sz, bs_q / kTile);
-    if (q_halves == 0) return;
+    // the list, 64 entries at a time in a register each, an entry per lane: block, dS unit, halves with keys
     const int n = __builtin_amdgcn_readfirstlane(min(max(lens[lrow], 0), stride));
-    const char* k_src = reinterpret_cast<const char*>(ks) + bh * Sk * (int64_t)(kD * 2);
+    int list_j = 0, list_p = 0, list_n = 2 * nsub;
+    auto take_entries = [&](int e0) {
+        const int e = max(min(e0 + lane, n - 1), 0);
+        list_j = min(max(idx[lrow * stride + e], 0), nbk - 1);
+        list_p = place[lrow * stride + e];
+        if (k_live != nullptr) list_n = k_live[list_j];
+    };
+    // waited for where they are loaded: the compiler would otherwise wait for them, and with them for every load before, at each half
+    auto entries_there = [&]() { asm volatile("" : "+v"(list_j), "+v"(list_p), "+v"(list_n)); };
+    take_entries(0);
+    const int q_halves = query_halves(q_live, item, head, sz, bs_q / kTile);
+    // the tokens of this lane's two rows; the epilogue stores through them
+    int64_t rows[2] = {qrow0 + lr, qrow0 + 32 + lr};
+    if (dq_to.rows != nullptr) { rows[0] = dq_to.rows[rows[0]]; rows[1] = dq_to.rows[rows[1]]; }
+    if (q_halves == 0) return;
+    int n_real = 2 * n * nsub;
+    if (k_live != nullptr) {
+        int mine = lane < n ? list_n : 0;
+        for (int e = 64 + lane; e < n; e += 64) mine += k_live[min(max(idx[lrow * stride + e], 0), nbk - 1)];
+        n_real = wave_sum(mine);
+    }
+    entries_there();
+    const char* k_src = ks_turned + bh * Sk * (int64_t)(kD * 2);
     const char* ds_src = ds + bh * pairs_per_head * kDsPairBytes;
     f32x16 acc[4][2];
 #pragma unroll
@@ -673,156 +773,96 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const T* __restrict_
         for (int qq = 0; qq < 2; ++qq)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[t][qq][i] = 0.f;
-    int nhalves = 2 * n * nsub;
 
-    // ---- the list, 64 entries at a time in a register each, an entry per lane (no vector load between the counted DMA loads
-    // but these every 64 entries): block, dS unit, halves with keys
-    int list_j = 0, list_p = 0, list_n = 2 * nsub;
-    auto take_entries = [&](int e0) {
-        const int e = min(e0 + lane, n - 1);
-        list_j = min(max(idx[lrow * stride + e], 0), nbk - 1);
-        list_p = place[lrow * stride + e];
-        if (k_live != nullptr) list_n = k_live[list_j];
-        asm volatile("" : "+v"(list_j), "+v"(list_p), "+v"(list_n));
-    };
-    // ---- global -> LDS
-    const uint32_t lds0 = lds_address(dsq_ring);
-    uint32_t voff[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = 4 * i + (lane >> 4);                                     // + 16 j
-        const int f = ((row & 3) << 2) | ((row >> 2) & 3);
-        voff[i] = (uint32_t)((row - 4 * i) * 256 + (((lane & 15) ^ f) << 4));    // load i adds 1 KB on both sides
-    }
-    const uint32_t voff_ds = (uint32_t)((lane & 1) * 1024 + ((lane >> 1) & 1) * 512 + (lane >> 2) * 16);
-    // a tile with rows in its first half alone takes that half's dS twice (the second sums are not stored)
-    const uint32_t second_half = q_halves == 2 ? (uint32_t)(nsub * kDsUnitBytes) : 0u;
-    int entry = 0, half = 0, issued = 0, issue_stage = 0;
-    auto issue = [&]() {                          // the next half of the walk
-        if (issued >= nhalves) return;
-        const int64_t at = (int64_t)__builtin_amdgcn_readlane(list_j, entry & 63) * (2 * nsub) + half;
-        const int64_t unit = (int64_t)__builtin_amdgcn_readlane(list_p, entry & 63) + 2 * sub_q * nsub + (half >> 1);
-        auto uniform = [](const char* x) -> const char* {          // the compiler cannot tell
-            const uint64_t a = reinterpret_cast<uint64_t>(x);
-            return reinterpret_cast<const char*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
-                                                 ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32));
-        };
-        const char* kp = uniform(k_src + at * kBwdHalfTileBytes);
-        const char* dp = uniform(ds_src + unit * kDsUnitBytes + (half & 1) * 2048);
-        const uint32_t dst = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + issue_stage * kDsqStage));
-        // an SGPR that a VALU instruction wrote may be a VMEM address five wait states later; the compiler does not count them
-        // in front of an assembly statement (it left two)
-        asm volatile("s_nop 4" : "+s"(kp), "+s"(dp));
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-            load_to_lds_4x16(kp + j * 4096, voff, dst + j * 4096);
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) load_to_lds_16_once(dp + h * second_half + i * 256, voff_ds, dst + kBwdHalfTileBytes + h * 2048 + i * 1024);
-        ++issued;
-        issue_stage = issue_stage == kDsqStages - 1 ? 0 : issue_stage + 1;
-        if (++half == __builtin_amdgcn_readlane(list_n, entry & 63)) {
-            half = 0;
-            if ((++entry & 63) == 0 && entry < n) take_entries(entry);
+    // ---- the walk: where half hp's fragments and its dS lie, for hp = 0, 1, 2, ...; behind the last half its fragments again, with
+    // zeros for dS.  A tile with rows in its first half alone takes that half's dS twice (the second sums are not stored).
+    const int second_half = q_halves == 2 ? nsub * kDsUnitBytes : 0;
+    int entry = 0, half = 0, walked = 0;
+    int64_t k_at = 0;
+    struct At { const char *k, *d0, *d1; };
+    auto next = [&]() -> At {
+        const bool more = walked < n_real;
+        const int j = __builtin_amdgcn_readlane(list_j, entry & 63), p = __builtin_amdgcn_readlane(list_p, entry & 63);
+        const int of_block = __builtin_amdgcn_readlane(list_n, entry & 63);
+        k_at = more ? ((int64_t)j * (2 * nsub) + half) * kBwdHalfTileBytes : k_at;
+        const char* d0 = more ? ds_src + ((int64_t)p + 2 * sub_q * nsub + (half >> 1)) * kDsUnitBytes + (half & 1) * 2048 : zeros;
+        const char* d1 = more ? d0 + second_half : zeros;
+        ++walked;
+        const bool done = more && half + 1 == of_block;
+        half = done ? 0 : half + 1;
+        entry += done ? 1 : 0;
+        if (done && (entry & 63) == 0 && entry < n) {
+            take_entries(entry);
+            entries_there();
         }
+        return {k_src + k_at, d0, d1};
     };
-    // ---- LDS -> fragments
+    // dS i: query half i >> 1, 16-query step i & 1
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    auto load_ds = [&](const At& a, int i) -> u32x4 {
+        return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>((i < 2 ? a.d0 : a.d1) + (i & 1) * 1024 + lane * 16));
+    };
+    auto load_k = [&](const At& a, int f) -> V8 { return *reinterpret_cast<const V8*>(a.k + f * 1024 + lane * 16); };      // f = 4 st + t
+
     const int s16 = lane & 15, g1 = (lane >> 4) & 1, tx = s16 >> 2, ty = (s16 & 3) >> 1, tz = s16 & 1;
-    uint32_t toff[4][2];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int hi = 0; hi < 2; ++hi)
-            toff[t][hi] = (uint32_t)((4 * lh + tx + 8 * hi) * 256) + ((((uint32_t)(4 * t + 2 * g1 + ty)) ^ (uint32_t)((4 * tx) | (lh + 2 * hi))) << 4) +
-                          (uint32_t)(tz * 8);
-    const uint32_t doff = (uint32_t)((4 * (4 * lh + tx) + 2 * tz + g1) * 16 + 8 * ty);      // chunk s16 & 3: lh' = its bit 0, the unit's half its bit 1
-    int read_stage = 0;
-    auto take = [&](V8 (&kt)[8], V8 (&dst)[2][2]) {
-        const char* part = dsq_ring + read_stage * kDsqStage;
-        auto both = [](s16x4 lo, s16x4 hi) { return __builtin_bit_cast(V8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)); };
-#pragma unroll
-        for (int st = 0; st < 2; ++st) {
-#pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                const char* d = part + kBwdHalfTileBytes + qq * 2048 + st * 1024 + doff;
-                dst[qq][st] = both(lds_read_tr16(d), lds_read_tr16(d + 512));
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const char* k = part + st * 4096;
-                kt[4 * st + t] = both(lds_read_tr16(k + toff[t][0]), lds_read_tr16(k + toff[t][1]));
-            }
-        }
-        read_stage = read_stage == kDsqStages - 1 ? 0 : read_stage + 1;
+    const uint32_t turn0 = lds_address(turn);
+    const int turn_x = (lr >> 1) & 3;            // of the writing lane's key
+    const uint32_t put_at[2] = {turn0 + (uint32_t)((4 * lr + ((2 * lh) ^ turn_x)) * 16), turn0 + (uint32_t)((4 * lr + ((2 * lh + 1) ^ turn_x)) * 16)};
+    // chunk s16 & 3: lh' = its bit 0, the unit's half its bit 1; the keys 8 and 16 further have the same two bits
+    const uint32_t take_at = turn0 + (uint32_t)((4 * (4 * lh + tx) + ((2 * tz + g1) ^ ((2 * lh + (tx >> 1)) & 3))) * 16 + 8 * ty);
+    auto put = [&](int i, const u32x4& x) { *(__attribute__((address_space(3))) u32x4*)(uintptr_t)(put_at[i & 1] + (i >> 1) * 2048) = x; };
+    V8 k[kDsqAhead][8], d[2][2][2];              // fragments by half; the B operand [half & 1][query half][16-key step]
+    u32x4 raw[kDsqAhead][4];
+    s16x4 lo = {};
+    auto turn_read = [&](V8 (&to)[2][2], int i) {                // i = 4 st + 2 qq + which four keys
+        const s16x4 x = lds_read_tr16_at(take_at + ((i >> 1) & 1) * 2048 + (i >> 2) * 1024 + (i & 1) * 512);
+        if ((i & 1) == 0) lo = x;
+        else to[(i >> 1) & 1][i >> 2] = __builtin_bit_cast(V8, (s16x8)__builtin_shufflevector(lo, x, 0, 1, 2, 3, 4, 5, 6, 7));
     };
-    auto multiply = [&](const V8 (&kt)[8], const V8 (&dst)[2][2]) {
-#pragma unroll
-        for (int st = 0; st < 2; ++st)
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int qq = 0; qq < 2; ++qq) acc[t][qq] = mfma32(kt[4 * st + t], dst[qq][st], acc[t][qq]);
-    };
-    // lgkmcnt(0) as the builtin: in assembly the compiler would not know of it and wait again in front of the products
-    auto reads_done = [&]() {
-        __builtin_amdgcn_s_waitcnt(0xc07f);
-        asm volatile("" ::: "memory");
-    };
-    // half hp in (kt, d); the next half's operands are read, then its stage is free for half hp + 4
-    auto step = [&](int hp, const V8 (&kt)[8], const V8 (&d)[2][2], V8 (&nkt)[8], V8 (&nd)[2][2]) {
-        if (hp + 1 < nhalves) {
-            static_assert(kDsqLoads == 12, "the counts below");
-            if (hp + 3 < nhalves) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");          // halves hp + 2 and hp + 3 may be on their way
-            else if (hp + 2 < nhalves) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            take(nkt, nd);
-        }
+    // Half hp, ring slot r, in sixteen slots of an MFMA each.  Its fragments are replaced by those of half hp + kDsqAhead as soon as
+    // their second MFMA is out; the dS of half hp + 1 goes into LDS and out of it, its registers take half hp + 1 + kDsqAhead.
+    auto step = [&](auto r_c, const At& a, At& ahead) {
+        constexpr int r = decltype(r_c)::value, r1 = (r + 1) % kDsqAhead;
+        ahead = next();
         __builtin_amdgcn_sched_barrier(0);
-        multiply(kt, d);
-        __builtin_amdgcn_sched_barrier(0);
-        reads_done();
-        issue();
+        static_for<16>([&](auto slot_c) {
+            constexpr int i = decltype(slot_c)::value, st = i >> 3, t = (i >> 1) & 3, qq = i & 1;
+            acc[t][qq] = mfma32(k[r][4 * st + t], d[r & 1][qq][st], acc[t][qq]);
+            if constexpr (i < 4) put(i, raw[r1][i]);
+            else if constexpr (i < 12) turn_read(d[r1 & 1], i - 4);
+            if constexpr (qq == 1) k[r][4 * st + t] = load_k(a, 4 * st + t);
+            if constexpr (i >= 4 && i < 12 && qq == 0) raw[r1][(i - 4) >> 1] = load_ds(ahead, (i - 4) >> 1);
+            __builtin_amdgcn_sched_barrier(0);
+        });
     };
-    if (nhalves > 0) {
-        V8 kt[2][8], d[2][2][2];
-        take_entries(0);
-        if (k_live != nullptr) {
-            int mine = lane < n ? list_n : 0;
-            for (int e = 64 + lane; e < n; e += 64) mine += k_live[min(max(idx[lrow * stride + e], 0), nbk - 1)];
-            nhalves = wave_sum(mine);
+    if (n_real > 0) {
+        At at[kDsqAhead];
+#pragma unroll
+        for (int r = 0; r < kDsqAhead; ++r) at[r] = next();
+#pragma unroll
+        for (int r = 0; r < kDsqAhead; ++r) {
+#pragma unroll
+            for (int f = 0; f < 8; ++f) k[r][f] = load_k(at[r], f);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) raw[r][i] = load_ds(at[r], i);
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // from here on the DMA loads are counted by hand
-        issue();
-        issue();
-        issue();
-        if (nhalves > 2) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-        else if (nhalves > 1) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        take(kt[0], d[0]);
-        reads_done();
-        issue();
-        for (int hp = 0; hp + 1 < nhalves; hp += 2) {
-            step(hp, kt[0], d[0], kt[1], d[1]);
-            step(hp + 1, kt[1], d[1], kt[0], d[0]);
+        // the first half's dS, whose registers take half kDsqAhead
+        At a = next(), ahead;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) put(i, raw[0][i]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) turn_read(d[0], i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) raw[0][i] = load_ds(a, i);
+        static_assert(kDsqAhead % 2 == 0, "d alternates");
+        for (int hp = 0; hp < n_real; hp += kDsqAhead) {
+            static_for<kDsqAhead>([&](auto r_c) {
+                step(r_c, a, ahead);
+                a = ahead;
+            });
         }
-        if (nhalves & 1) multiply(kt[0], d[0]);
     }
-    // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, query lr (+ 32)
-#pragma unroll
-    for (int qq = 0; qq < 2; ++qq) {
-        T* out = store_row(dq, dq_to, bh, Sq, qrow0 + 32 * qq + lr);
-        if (out == nullptr) continue;                            // a padded slot of a token-order destination
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                T x[4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) x[j] = (T)(acc[t][qq][4 * g4 + j] * kLn2);
-                *reinterpret_cast<uint2*>(out + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(x);
-            }
-    }
+    store_dq<T>(acc, dq, dq_to, bh, Sq, rows, lane);
 }
 
 // ------------------------------------------------------------------ dK and dV in one kernel, Q and dO through LDS
@@ -864,11 +904,11 @@ struct DkdvSizes {
 };
 template <typename T, bool kMasked, bool kKeep>
 __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, const T* __restrict__ dout,
-                                                       const T* __restrict__ ks, const T* __restrict__ v,
+                                                       BwdLoad k_from, BwdLoad v_from,
                                                        const float* __restrict__ m2, const float* __restrict__ delta,
                                                        const uint32_t* __restrict__ bits,
                                                        const uint64_t* __restrict__ tile_valid, T* __restrict__ dk,
-                                                       T* __restrict__ dv, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int words,
+                                                       T* __restrict__ dv, int64_t Sq, int64_t Sk, int words, float ks_scale,
                                                        float dk_scale, const int32_t* __restrict__ order, int n_items, int round,
                                                        BwdStore dk_to, BwdStore dv_to, char* __restrict__ ds_out,
                                                        char* __restrict__ ds_spare, const int32_t* __restrict__ unit_base, int64_t pairs_per_head, DkdvSizes sz,
@@ -894,26 +934,12 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     const uint32_t* mask_row = bits + (int64_t)block * words;
     // halves of this tile that hold keys: the second wavefront of a tile with one half brings its share of the rows, no more
     int key_halves = 2;
-    if (k_live != nullptr) {
-        const int in_head = block - head * (sz.tiles / sz.by_block);
-        key_halves = __builtin_amdgcn_readfirstlane(k_live[in_head]) - 2 * (item - block * nsub);
-        if (key_halves <= 0) return;
-    }
+    if (k_live != nullptr) key_halves = __builtin_amdgcn_readfirstlane(k_live[block - head * (sz.tiles / sz.by_block)]) - 2 * (item - block * nsub);
     // halves come in pairs: an odd number of them ends with the last one again, whose p are 0 (M2 = -inf)
     const int n_real = __builtin_amdgcn_readfirstlane(counts[block]), nhalves = (n_real + 1) & ~1;
-
-    // resident: K_s and V rows of this wavefront's 32 keys, as B operands (lane = key lr, 8 consecutive d)
-    V8 kreg[8], vreg[8];
-    {
-        const int64_t row = bh * Sk + krow0 + 32 * wave + lr;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            const V8 a = *reinterpret_cast<const V8*>(ks + row * kD + 16 * c + 8 * lh), b = *reinterpret_cast<const V8*>(v + row * kD + 16 * c + 8 * lh);
-            // read by assembly MFMAs from accumulation registers
-            asm volatile("" : "=a"(kreg[c]) : "0"(a));
-            asm volatile("" : "=a"(vreg[c]) : "0"(b));
-        }
-    }
+    // the row of this lane's key: its token, or in blocked order its slot
+    int64_t key_row = krow0 + 32 * wave + lr;
+    if (dk_to.rows != nullptr) key_row = dk_to.rows[key_row];
     bool key_ok = true;
     if (kMasked) key_ok = (tile_valid[krow0 / kTile] >> (32 * wave + lr)) & 1ull;
     f32x16 acc_dk[4], acc_dv[4];
@@ -926,16 +952,38 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     *reinterpret_cast<float*>(bwd_lds + kBwdNumbers + (threadIdx.x >> 5) * kBwdStats + 256 + (threadIdx.x & 31) * 4) = -INFINITY;
     // the query blocks of this KV block, ascending, from the bit matrix into LDS (behind the stages)
     int32_t* qlist = reinterpret_cast<int32_t*>(bwd_lds + kBwdStages * kBwdStage);
-    int count = 0;
-    for (int w0 = 0; w0 < words; w0 += 64) {
-        const int w = w0 + lane;
-        uint32_t word = w < words ? mask_row[w] : 0u;
-        uint32_t plane[kPlanesAtHand] = {};
+    uint32_t word_now = 0, plane[kPlanesAtHand] = {};
+    auto take_words = [&](int w) {
+        word_now = w < words ? mask_row[w] : 0u;
         if (q_live.live != nullptr) {
 #pragma unroll
             for (int p = 0; p < kPlanesAtHand; ++p)
                 if (p < q_live.n_planes && w < words) plane[p] = q_live.planes[p * q_live.plane_words + w];
         }
+    };
+    take_words(lane);
+    if (key_halves <= 0) return;
+    // Resident: K_s and V rows of this wavefront's 32 keys, as B operands (lane = key lr, 8 consecutive d), from where the caller's
+    // rows lie.  Asked for here, behind the look-up of their token and in front of the list's: what is waited for before the first
+    // product is one chain of dependent loads, not two.
+    V8 k_rows[8], v_rows[8];
+    {
+        const int64_t at_row = max(key_row, (int64_t)0);
+        const int batch = head / dk_to.Hn, in_batch = head - batch * dk_to.Hn;
+        const T* kp = static_cast<const T*>(k_from.p) + batch * k_from.sB + in_batch * k_from.sH + at_row * k_from.sS + 8 * lh;
+        const T* vp = static_cast<const T*>(v_from.p) + batch * v_from.sB + in_batch * v_from.sH + at_row * v_from.sS + 8 * lh;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            k_rows[c] = *reinterpret_cast<const V8*>(kp + 16 * c);
+            v_rows[c] = *reinterpret_cast<const V8*>(vp + 16 * c);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    int count = 0;
+    for (int w0 = 0; w0 < words; w0 += 64) {
+        const int w = w0 + lane;
+        if (w0 > 0) take_words(w);
+        uint32_t word = word_now;
         if (w == words - 1 && (nbq & 31)) word &= (1u << (nbq & 31)) - 1u;
         int mine = __popc(word), upto = mine;
 #pragma unroll
@@ -1046,6 +1094,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     // LDS a half, and the exponentials in bunches: 2 150 clocks a half beside 1 024 of products.)
     // S and dP accumulate in ordinary registers, where the exponentials read them: MFMAs from inline assembly, behind which the
     // compiler adds no wait states - a pair is first read nine MFMAs after its last product.
+    V8 kreg[8], vreg[8];
     auto step = [&](auto odd_c, int hp, f32x16& s, f32x16& dp, f32x16& s_next, f32x16& dp_next) {
         constexpr int odd = decltype(odd_c)::value;                  // hp & 1
         constexpr uint32_t qn = (odd ^ 1) * kBwdHalfTile, dn = qn + kBwdDout;      // rows of half hp + 1, in its pair of stages
@@ -1150,24 +1199,39 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     if (nhalves > 0) {
         issue(0);
         issue(1);
+        // k_s = k * c, rounded once to the storage type (as bwd_scale_kernel); padded keys' rows are zeros, whatever lies there: their
+        // products start from -inf, and an infinite one would make a NaN of that.  (The wait for the rows is one for all that is
+        // on its way; the first two halves have to be there as well.)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            V8 x = k_rows[c];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = (T)((float)x[e] * ks_scale);
+            uint4 kr = __builtin_bit_cast(uint4, x), vr = __builtin_bit_cast(uint4, v_rows[c]);
+            if (kMasked) { keep_if(kr, key_ok); keep_if(vr, key_ok); }
+            // read by assembly MFMAs from accumulation registers
+            asm volatile("" : "=a"(kreg[c]) : "0"(__builtin_bit_cast(V8, kr)));
+            asm volatile("" : "=a"(vreg[c]) : "0"(__builtin_bit_cast(V8, vr)));
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
         issue(2);
         if (kKeep) {                             // as many stores as a half before the first would have left on their way
             const V8 none = {};
             __builtin_nontemporal_store(none, reinterpret_cast<V8*>(ds_spare + lane * 16));
             __builtin_nontemporal_store(none, reinterpret_cast<V8*>(ds_spare + 1024 + lane * 16));
         }
-        asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kKeep ? kBwdLoads + 2 : kBwdLoads) : "memory");
-        __builtin_amdgcn_s_barrier();
         if (wave >= key_halves) {                // no keys: the rows alone
             for (int hp = 0; hp < nhalves; ++hp) {
                 issue(hp + 3);
-                asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kBwdLoads) : "memory");
+                asm volatile("s_waitcnt vmcnt(%0)" :: "n"(kBwdLoads) : "memory");      // (the stores in front of the first count for nothing)
                 __builtin_amdgcn_s_barrier();
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS that is no longer this workgroup's
             return;
         }
         f32x16 s0, dp0, s1, dp1;
+        V8 first_q[8], first_d[8];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const f32x4_ mm = lds_read_at<f32x4_>(m2_at + 32 * g), dd = lds_read_at<f32x4_>(numbers + (128 + 32 * g));
@@ -1176,8 +1240,13 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         }
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
-            mfma_s<false, true>(s0, lds_read_at<V8>(roff[c]), kreg[c]);
-            mfma_s<false, true>(dp0, lds_read_at<V8>(roff[c] + kBwdDout), vreg[c]);
+            first_q[c] = lds_read_at<V8>(roff[c]);
+            first_d[c] = lds_read_at<V8>(roff[c] + kBwdDout);
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            mfma_s<false, true>(s0, first_q[c], kreg[c]);
+            mfma_s<false, true>(dp0, first_d[c], vreg[c]);
         }
         asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
         mfma_chain_end(s0); mfma_chain_end(dp0);
@@ -1200,24 +1269,21 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     }
     // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, key lr
     {
-        T* out_k = store_row(dk, dk_to, bh, Sk, krow0 + 32 * wave + lr);
-        T* out_v = store_row(dv, dv_to, bh, Sk, krow0 + 32 * wave + lr);
-        if (out_k != nullptr && out_v != nullptr) {              // both or neither: one row table serves dk and dv
+        const int batch = head / dk_to.Hn, in_batch = head - batch * dk_to.Hn;
+        const bool blocked = dk_to.rows == nullptr;
+        T* out_k = dk + (blocked ? (bh * Sk + key_row) * kD : batch * dk_to.sB + in_batch * dk_to.sH + key_row * dk_to.sS);
+        T* out_v = dv + (blocked ? (bh * Sk + key_row) * kD : batch * dv_to.sB + in_batch * dv_to.sH + key_row * dv_to.sS);
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+        for (int t = 0; t < 4; ++t) {
+            float xk[16], xv[16];
 #pragma unroll
-                for (int g4 = 0; g4 < 4; ++g4) {
-                    T xk[4], xv[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        // padded keys' sums are replaced before the product, which fp16 would otherwise round with the conversion
-                        const float sum_k = kMasked && !key_ok ? 0.f : acc_dk[t][4 * g4 + j], sum_v = kMasked && !key_ok ? 0.f : acc_dv[t][4 * g4 + j];
-                        xk[j] = (T)(sum_k * dk_scale);
-                        xv[j] = (T)sum_v;
-                    }
-                    *reinterpret_cast<uint2*>(out_k + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(xk);
-                    *reinterpret_cast<uint2*>(out_v + 32 * t + 8 * g4 + 4 * lh) = *reinterpret_cast<const uint2*>(xv);
-                }
+            for (int i = 0; i < 16; ++i) {
+                // padded keys' sums are replaced before the product, which fp16 would otherwise round with the conversion
+                xk[i] = (kMasked && !key_ok ? 0.f : acc_dk[t][i]) * dk_scale;
+                xv[i] = kMasked && !key_ok ? 0.f : acc_dv[t][i];
+            }
+            store_columns(out_k + 32 * t, key_row >= 0, xk, lane);
+            store_columns(out_v + 32 * t, key_row >= 0, xv, lane);
         }
     }
 }
@@ -1252,8 +1318,8 @@ struct BwdWs {
                                                            // kernel's visiting order; per KV block its number of query halves; the KV
                                                            // tiles of every head by that number
     size_t q_live, k_live, planes;                         // LiveHalves of both grids (token order, where they are padded)
-    size_t base, place, ds, ds_spare;                      // with kept dS: units in front of a KV block, the first unit of a list entry, dS,
-                                                           // where a repeated half's goes
+    size_t base, place, ds, ds_spare, ds_zeros;                      // with kept dS: units in front of a KV block, the first unit of a list entry, dS,
+                                                           // where a repeated half's goes, a unit of zeros
     size_t total;
 };
 static int plane_words(int64_t blocks) { return (int)((blocks + 63) / 64 * 2); }
@@ -1281,6 +1347,7 @@ static BwdWs bwd_ws(const KeptDs& kept, int64_t bh, int64_t Sq, int64_t Sk, int 
     w.place = take(kept.keep ? bh * nbq * (size_t)idx_stride * 4 : 0);
     w.ds = take(kept.keep ? (size_t)bh * (size_t)kept.pairs_per_head * kDsPairBytes : 0);
     w.ds_spare = take(kept.keep ? kDsUnitBytes : 0);
+    w.ds_zeros = take(kept.keep ? kDsUnitBytes : 0);
     w.total = off;
     return w;
 }
@@ -1347,11 +1414,14 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     const int64_t qrows = (int64_t)bh * Sq, krows = (int64_t)bh * Sk, nwords = (int64_t)bh * nbk * words;
     const float c = sm_scale * kRcpLn2;
     BwdStore dq_to = {nullptr, 0, 0, 0, Hn}, dk_to = dq_to, dv_to = dq_to;
+    BwdLoad k_from = {k, Hn * Sk * kD, Sk * kD, kD}, v_from = {v, Hn * Sk * kD, Sk * kD, kD};
     if (thw != nullptr) {
         dq_to = {thw->q_rows, thw->dq_st[0], thw->dq_st[1], thw->dq_st[2], Hn};
         dk_to = {thw->k_rows, thw->dk_st[0], thw->dk_st[1], thw->dk_st[2], Hn};
         dv_to = {thw->k_rows, thw->dv_st[0], thw->dv_st[1], thw->dv_st[2], Hn};
         dq = thw->dq; dk = thw->dk; dv = thw->dv;
+        k_from = {thw->k, thw->k_st[0], thw->k_st[1], thw->k_st[2]};
+        v_from = {thw->v, thw->v_st[0], thw->v_st[1], thw->v_st[2]};
         q = thw->q_blocked; v = thw->v_blocked; dout = thw->dout_blocked;
         BwdPrep a = {};
         a.gq = thw->gq; a.gk = thw->gk; a.Hn = Hn;
@@ -1362,7 +1432,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         }
         a.lse = thw->lse; a.q_tokens = (int64_t)thw->gq.T * thw->gq.H * thw->gq.W;
         a.q_blocked = (uint16_t*)thw->q_blocked; a.dout_blocked = (uint16_t*)thw->dout_blocked; a.ks = (uint16_t*)ks;
-        a.v_blocked = (uint16_t*)thw->v_blocked;
+        a.v_blocked = kept.keep ? nullptr : (uint16_t*)thw->v_blocked;
         a.delta = delta; a.m2 = m2; a.q_rows = thw->q_rows; a.k_rows = thw->k_rows; a.valid = thw->valid;
         a.bits = bits; a.n_bits = nwords; a.c = c;
         a.q_live = const_cast<int32_t*>(q_live.live); a.k_live = k_live;
@@ -1376,13 +1446,15 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     } else if (dtype == BSA_BF16) {
         hipLaunchKernelGGL((bwd_rows_kernel<__bf16>), dim3((unsigned)((qrows + 15) / 16)), dim3(256), 0, st, (const __bf16*)o,
                            (const __bf16*)dout, lse, delta, m2, qrows);
-        hipLaunchKernelGGL((bwd_scale_kernel<__bf16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
-                           (const __bf16*)k, (__bf16*)ks, c, krows * 16, tile_valid, (uint32_t)Sk);
+        if (kept.keep) hipLaunchKernelGGL((bwd_scale_turned_kernel<__bf16>), dim3((unsigned)(krows / kTile)), dim3(256), 0, st, (const __bf16*)k, ks, c, tile_valid, (int)(Sk / kTile));
+        else hipLaunchKernelGGL((bwd_scale_kernel<__bf16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
+                                (const __bf16*)k, (__bf16*)ks, c, krows * 16, tile_valid, (uint32_t)Sk);
     } else {
         hipLaunchKernelGGL((bwd_rows_kernel<_Float16>), dim3((unsigned)((qrows + 15) / 16)), dim3(256), 0, st, (const _Float16*)o,
                            (const _Float16*)dout, lse, delta, m2, qrows);
-        hipLaunchKernelGGL((bwd_scale_kernel<_Float16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
-                           (const _Float16*)k, (_Float16*)ks, c, krows * 16, tile_valid, (uint32_t)Sk);
+        if (kept.keep) hipLaunchKernelGGL((bwd_scale_turned_kernel<_Float16>), dim3((unsigned)(krows / kTile)), dim3(256), 0, st, (const _Float16*)k, ks, c, tile_valid, (int)(Sk / kTile));
+        else hipLaunchKernelGGL((bwd_scale_kernel<_Float16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
+                                (const _Float16*)k, (_Float16*)ks, c, krows * 16, tile_valid, (uint32_t)Sk);
     }
     if (thw == nullptr) hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, bits, nwords);
     const int64_t lrows = (int64_t)bh * nbq;
@@ -1402,14 +1474,14 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     const DkdvSizes sizes = {(int)(Sk / kTile), nbq, nsub, divisor((int)(Sk / kTile)), divisor(bs_k / kTile), divisor(round)};
     const int total_q = (int)(bh * (Sq / kTile)), total_k = (int)(bh * (Sk / kTile));
 #define BSA_DKDV(T, M, K)                                                                                                              \
-    hipLaunchKernelGGL((bwd_dkdv_kernel<T, M, K>), dim3((unsigned)total_k), dim3(128), lds, st, (const T*)q, (const T*)dout, (const T*)ks,  \
-                       (const T*)v, m2, delta, bits, tile_valid, (T*)dk, (T*)dv, Sq, Sk, bs_q, bs_k, words, sm_scale, order, total_k, round,  \
+    hipLaunchKernelGGL((bwd_dkdv_kernel<T, M, K>), dim3((unsigned)total_k), dim3(128), lds, st, (const T*)q, (const T*)dout, k_from, v_from,  \
+                       m2, delta, bits, tile_valid, (T*)dk, (T*)dv, Sq, Sk, words, c, sm_scale, order, total_k, round,  \
                        dk_to, dv_to, ws + at.ds, ws + at.ds_spare, base, kept.pairs_per_head, sizes, q_live, k_live, counts)
 #define BSA_DQ(T, M)                                                                                                                   \
     hipLaunchKernelGGL((bwd_dq_lds_kernel<T, M>), dim3(end - first), block, kDqRingLds, st, (const T*)q, (const T*)dout, (const T*)ks, (const T*)v,  \
                        m2, delta, paced, lens, tile_valid, (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, dq_to, dq_sizes, q_live.live, k_live)
 #define BSA_DQ_DS(T)                                                                                                                   \
-    hipLaunchKernelGGL((bwd_dq_from_ds_kernel<T>), dim3(end - first), block, kDsqStages* kDsqStage, st, (const T*)ks, ws + at.ds, paced, place, lens,  \
+    hipLaunchKernelGGL((bwd_dq_from_ds_kernel<T>), dim3(end - first), block, 0, st, ks, ws + at.ds, ws + at.ds_zeros, paced, place, lens,  \
                        (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, kept.pairs_per_head, dq_to, dq_sizes, q_live.live, k_live)
 #define BSA_BY_TYPE(F, ...)                                     \
     do {                                                        \
@@ -1418,7 +1490,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     } while (0)
     if (kept.keep) {
         hipLaunchKernelGGL(bwd_place_kernel, dim3((unsigned)((lrows + 3) / 4)), dim3(256), 0, st, paced, lens, bits, base, place, nbq, nbk, idx_stride,
-                           words, nsub, lrows, q_live);
+                           words, nsub, lrows, q_live, reinterpret_cast<uint4*>(ws + at.ds_zeros));
         if (masked) BSA_BY_TYPE(BSA_DKDV, true, true);
         else BSA_BY_TYPE(BSA_DKDV, false, true);
     }
