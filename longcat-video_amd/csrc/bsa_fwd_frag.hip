@@ -126,8 +126,17 @@ constexpr int kQueues = 8, kQueueChoice = kQueues, kQueueWords = kQueues + 1;   
 static_assert(kQueueWords <= kFragQueueWords, "the caller's buffer holds the words");
 __device__ __forceinline__ int section_begin(int n, int x) { return (int)(((int64_t)n * x) >> 3); }
 
-template <typename T, int kWalk, bool kBounded>
-__global__ __launch_bounds__(64) void fwd_frag_kernel(
+// kTeam: wavefronts that share an item, a workgroup on the SIMDs of one compute unit.  Each walks a share of the item's pairs
+// (a part's share, where the item is in parts as well) from the list that they stage together; then their sums are put
+// together in LDS, in the order of the shares, wavefront w those of its 4 / kTeam tiles of d, and the rows leave as from one
+// wavefront.  One item per workgroup, nothing prepared ahead.  For calls of so few items that most SIMDs would have none: see
+// choose_split.
+template <int kTeam>
+constexpr int kTeamBytes = kTeam * (kTile * kD + 2 * kTile) * 4;      // the sums, maxima and row sums of every wavefront
+static_assert(kTeamBytes<4> <= 160 * 1024 && 2 * (kTeamBytes<2> + 512) <= 160 * 1024, "LDS of a compute unit with four wavefronts");
+
+template <typename T, int kWalk, bool kBounded, int kTeam>
+__global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
     const int32_t* __restrict__ idx, const int32_t* __restrict__ lens, const uint64_t* __restrict__ tile_valid,
     T* __restrict__ o, float* __restrict__ lse, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride,
@@ -148,24 +157,29 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // fewer).
     constexpr float kSlack = 60.0f;
     static_assert(!kBounded || std::is_same<T, __bf16>::value, "fp16 probabilities need the running maximum");
+    static_assert(!kBounded || kTeam == 1, "a team leaves nothing to another launch");
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     // six lines: 0.36 us for the first five where one by one they took 0.7 to 1.1; with the sixth a call of two prompts of 8 heads,
     // 7x15x26, takes 41.4 us for 41.9.  With what an item that nothing has prepared asks for at once (below) and the divisions
     // that went, the kernel of a single round is 1.3 us shorter: 15.1 -> 13.8 us for 5 heads of 9x27x12, 25.4 -> 24.2 for two
     // prompts of 8 heads of 7x15x26.
-    touch_arguments<decltype(fwd_frag_kernel<T, kWalk, kBounded>)>();
+    touch_arguments<decltype(fwd_frag_kernel<T, kWalk, kBounded, kTeam>)>();
     if (gate != nullptr && *gate != gate_want) return;
     // output staging: 64 rows of 256 B, 272 B apart.  The same memory stages a list that is too long for the small
     // buffers (kListEntries words at most) during the tile loop of an item that was not prepared ahead of time.
     constexpr int kOutPitch = kD + 8;
-    __shared__ __attribute__((aligned(16))) T ost[kTile * kOutPitch];
+    // A team has its list there, then the wavefronts' sums, then the rows of the output.
+    constexpr int kOutBytes = kTile * kOutPitch * (int)sizeof(T);
+    __shared__ __attribute__((aligned(16))) char ost_bytes[kTeam > 1 ? kTeamBytes<kTeam> : kOutBytes];
+    T* const ost = reinterpret_cast<T*>(ost_bytes);
     constexpr int kWords = kWalk == kHalves ? 2 : 1;              // list words of a pair
-    __shared__ __attribute__((aligned(8))) uint32_t lists[2][kPipeList * kWords];
+    __shared__ __attribute__((aligned(8))) uint32_t lists[2][kTeam > 1 ? 2 : kPipeList * kWords];
     __shared__ int32_t out_rows[2][kTile];       // token rows of this and the next item's 64 query slots (row table given)
-    __shared__ __attribute__((aligned(16))) char qstage[kTileBytes];      // Q of the next item, in register order
+    __shared__ __attribute__((aligned(16))) char qstage[kTeam > 1 ? 16 : kTileBytes];      // Q of the next item, in register order
     uint32_t* const big = reinterpret_cast<uint32_t*>(ost);
 
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = kTeam > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
     const int lr = lane & 31, lh = lane >> 5;
     const int nqt = (int)(Sq / kTile);
     const int nsub = kWalk == kBlocks ? bs_k / kTile : 1;
@@ -298,6 +312,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
 
     // ---- per item
     int npairs = 0, pair0 = 0;       // the walk covers the pairs pair0 .. pair0 + npairs - 1 of the list
+    int n_halves = 0;                // a team's walk over halves: those of this wavefront's share, from ents on
     uint32_t half_base = 0;          // first half of the item's (batch, head)
     uint32_t beyond[2] = {0, 0};     // what the positions behind the end of the list name
     const uint32_t* ents = big;      // the item's list in LDS
@@ -310,7 +325,11 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     auto pair_raw = [&](int tp) -> Raw {
         const int tc = min(tp, npairs - 1) + pair0;
         Raw r;
-        if constexpr (kWalk == kHalves) {
+        if constexpr (kWalk == kHalves && kTeam > 1) {
+            r.e[0] = ents[2 * tc];
+            r.e[1] = ents[min(2 * tc + 1, n_halves - 1)];
+            if (2 * tc + 1 >= n_halves) r.e[1] &= kHalfId;      // an odd share: its last half once more, no key of it
+        } else if constexpr (kWalk == kHalves) {
             const uint2 x = *reinterpret_cast<const uint2*>(ents + 2 * tc);               // the same address in every lane
             r.e[0] = x.x; r.e[1] = x.y;
         } else {
@@ -373,7 +392,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // mx0, mx1: this lane's unscaled maxima over its 16 accumulators of the step that comes next.  The test
     // needs no exchange between the two key groups of a query: some lane exceeds the limit exactly when the
     // combined maximum does.
-    auto raise_max = [&](float mx0, float mx1) {
+    auto raise_max = [&](float mx0, float mx1) __attribute__((always_inline)) {
         if (__builtin_expect(__any(mx0 > raise_at[0] || mx1 > raise_at[1]), 0)) {
             const float mx[2] = {finish_max(mx0) * qk_scale, finish_max(mx1) * qk_scale};
 #pragma unroll
@@ -392,7 +411,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // The output accumulators live in AGPRs, which the VALU cannot multiply in place.  Written out register by
     // register through one temporary, so that this rare path does not make the compiler reserve VGPRs for a copy
     // of the accumulators.
-    auto rescale_out = [&]() {
+    auto rescale_out = [&]() __attribute__((always_inline)) {
         asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMA into the accumulators has retired
         static_for<128>([&](auto n_c) {
             constexpr int n = decltype(n_c)::value, qq = n >> 6, t = (n >> 4) & 3, i = n & 15;
@@ -419,7 +438,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
     // fragment is requested two steps before it is used.  Within a burst the fragment that is used first is
     // requested last: loads return in order, so the wait in front of its first use covers the whole burst and
     // the fragments behind it need none of their own.
-    auto step = [&](auto jj) {
+    auto step = [&](auto jj) __attribute__((always_inline)) {
         constexpr int j = decltype(jj)::value;
         constexpr int sc = j & 1, sn = sc ^ 1;                 // S(u) and S(u+1) alternate between two register sets
         constexpr int kslot = (j + 1) & 1;                     // ring slot of K(u+1), then of K(u+3)
@@ -548,10 +567,13 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             first_rows[1] = L.q_rows[qrow0 + 32 + lr];
             first_rows[2] = L.q_rows[qrow0 + lane];
         }
+        // ... and so is a team's list, as far as one entry a thread goes (what lies behind its end is not used)
+        int32_t team_entry = 0;
+        if (kTeam > 1 && idx_stride > 0) team_entry = idx[(int64_t)(cur.item / L.by_block) * idx_stride + min((int)threadIdx.x, idx_stride - 1)];
         __builtin_amdgcn_sched_barrier(0);
         const int nent = list_length(cur);
         npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
-        if (!kBounded && parts.count > 1) {
+        if (kTeam == 1 && !kBounded && parts.count > 1) {
             const int part = cur.local / parts.by_items;        // at most kMaxParts: the products fit 32 bits
             pair0 = npairs * part / parts.by_count;
             npairs = npairs * (part + 1) / parts.by_count - pair0;
@@ -561,7 +583,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         // has a first tile to point the walk at, a list that fits a small buffer, and Q rows the LDS DMA can address
         const int next_nent = list_length(nxt);
         // (an item in parts has no first pair that is known ahead)
-        const bool prepare_next = (kBounded || parts.count == 1) && nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
+        const bool prepare_next = kTeam == 1 && (kBounded || parts.count == 1) && nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
         if (prepare_next) {
             first_pair(nxt, beyond);
             beyond[0] = (uint32_t)uni((int)beyond[0]);
@@ -573,7 +595,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
         const int64_t nqrow0 = (int64_t)(nitem - nbh * nqt) * kTile;
         const int32_t* nlist = idx + (int64_t)(nitem / L.by_block) * idx_stride;
 
-        const bool early = kBounded || parts.count == 1;         // the walk starts at the list's first entry
+        const bool early = kTeam == 1 && (kBounded || parts.count == 1);         // the walk starts at the list's first entry
         auto first_fragments = [&](uint32_t h0, uint32_t h1) {
 #pragma unroll
             for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(h0, c);                       // K(0)
@@ -593,7 +615,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             const int32_t* list = idx + (int64_t)(cur.item / L.by_block) * idx_stride;
             constexpr int kAhead = 4;
             int32_t entry[kAhead] = {0, 0, 0, 0};
-            if (nent > 0) {
+            if (kTeam == 1 && nent > 0) {
 #pragma unroll
                 for (int e = 0; e < kAhead; ++e) entry[e] = list[min(lane_now + 64 * e, nent - 1)];
             }
@@ -613,15 +635,51 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 first_fragments((uint32_t)uni((int)h[0]), (uint32_t)uni((int)h[1]));
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (L.q_rows != nullptr) out_rows[list_buf][lane_now] = first_rows[2];
+            if (L.q_rows != nullptr && (kTeam == 1 || wave == 0)) out_rows[list_buf][lane_now] = first_rows[2];
+            if constexpr (kTeam == 1) {
 #pragma unroll
-            for (int e = 0; e < kAhead; ++e)
-                if (lane_now + 64 * e < nent) big[lane_now + 64 * e] = (uint32_t)entry[e];
-            for (int e = lane_now + 64 * kAhead; e < nent; e += 64) big[e] = (uint32_t)list[e];
+                for (int e = 0; e < kAhead; ++e)
+                    if (lane_now + 64 * e < nent) big[lane_now + 64 * e] = (uint32_t)entry[e];
+                for (int e = lane_now + 64 * kAhead; e < nent; e += 64) big[e] = (uint32_t)list[e];
+            } else {
+                if ((int)threadIdx.x < nent) big[threadIdx.x] = (uint32_t)team_entry;
+                for (int e = threadIdx.x + 64 * kTeam; e < nent; e += 64 * kTeam) big[e] = (uint32_t)list[e];
+            }
             take_q(0, rows[0]);
             take_q(1, rows[1]);
             ents = big;
             __syncthreads();
+            if constexpr (kTeam > 1) {
+                // This wavefront's share of the list, whole KV blocks of it, so that a walk over halves and one over tiles that masks
+                // the empty halves cut at the same keys (and give the same bits).
+                const int share = (parts.count > 1 ? cur.local / parts.by_items : 0) * kTeam + wave, shares = parts.count * kTeam;
+                if constexpr (kWalk == kHalves) {
+                    const int used = min(max(uni(cur.nent), 0), idx_stride);      // without the repeat that makes the number even
+                    auto starts_block = [&](int base) -> uint64_t {       // of the list's entries base .. base + 63
+                        const uint32_t h = base + lane < used ? ents[base + lane] & kHalfId : 1u;
+                        return __ballot((h & 1u) == 0u && (int)(h >> 1) == (int)(h >> 1) / L.by_sub * (bs_k / kTile));
+                    };
+                    int n_blocks = 0;
+                    for (int base = 0; base < used; base += 64) n_blocks += __builtin_popcountll(starts_block(base));
+                    const int b0 = n_blocks * share / shares, b1 = n_blocks * (share + 1) / shares;      // 4 096 entries, 64 shares at most
+                    int p0 = 0, p1 = used, seen = 0;
+                    for (int base = 0; base < used; base += 64) {
+                        const uint64_t m = starts_block(base);
+                        const int rank = seen + __builtin_popcountll(m & (((uint64_t)1 << lane) - 1));
+                        const uint64_t at0 = __ballot(((m >> lane) & 1) != 0 && rank == b0), at1 = __ballot(((m >> lane) & 1) != 0 && rank == b1);
+                        if (at0 != 0) p0 = base + __builtin_ctzll(at0);
+                        if (at1 != 0) p1 = base + __builtin_ctzll(at1);
+                        seen += __builtin_popcountll(m);
+                    }
+                    ents += p0;
+                    n_halves = b1 > b0 ? p1 - p0 : 0;
+                    npairs = (n_halves + 1) >> 1;
+                } else {
+                    const int b0 = nent * share / shares, b1 = nent * (share + 1) / shares;
+                    pair0 = b0 * nsub;
+                    npairs = (b1 - b0) * nsub;
+                }
+            }
         } else {
             ents = lists[list_buf];
 #pragma unroll
@@ -781,7 +839,7 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
                 raw = pair_raw(g + 5);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            __syncthreads();                          // the list in LDS has been read: the memory may become the staging tile
+            if (kTeam == 1) __syncthreads();          // the list in LDS has been read: the memory may become the staging tile (a team: below)
             if (prepare_next) {
                 // The DMA of the next item's list and Q rows was issued in front of the loop and every iteration has
                 // issued 32 loads since; loads complete in order, so all but the newest 24 done (the next item's first
@@ -799,6 +857,116 @@ __global__ __launch_bounds__(64) void fwd_frag_kernel(
             }   // run
         }   // npairs > 0
 
+        if constexpr (kTeam > 1) {
+            // ---- the wavefronts' sums together: sums[wave][register order of a part], then maxima and row sums [wave][query].
+            // 128 KB through LDS for a team of four, a microsecond; the rows leave from all wavefronts.
+            float* const sums = reinterpret_cast<float*>(ost_bytes);
+            float* const stats = sums + kTeam * kTile * kD;
+            float inv[2], M[2], l_all[2];
+            __syncthreads();                          // the list has been read
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq) {
+                const float l = l_i[qq] + __shfl_xor(l_i[qq], 32);
+                if (lh == 0) {
+                    stats[(2 * wave) * kTile + 32 * qq + lr] = m_i[qq];
+                    stats[(2 * wave + 1) * kTile + 32 * qq + lr] = l;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+                    for (int gq = 0; gq < 4; ++gq)
+                        *reinterpret_cast<float4*>(sums + wave * (kTile * kD) + (((t * 2 + qq) * 4 + gq) * 64 + lane) * 4) =
+                            make_float4(oacc[t][qq][4 * gq], oacc[t][qq][4 * gq + 1], oacc[t][qq][4 * gq + 2], oacc[t][qq][4 * gq + 3]);
+            __syncthreads();
+            float factor[2][kTeam];
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq) {
+                float m[kTeam];
+#pragma unroll
+                for (int w = 0; w < kTeam; ++w) m[w] = stats[(2 * w) * kTile + 32 * qq + lr];
+                M[qq] = m[0];
+#pragma unroll
+                for (int w = 1; w < kTeam; ++w) M[qq] = fmaxf(M[qq], m[w]);
+                l_all[qq] = 0.f;
+#pragma unroll
+                for (int w = 0; w < kTeam; ++w) {
+                    factor[qq][w] = m[w] > -INFINITY ? __builtin_amdgcn_exp2f(m[w] - M[qq]) : 0.f;      // a share without keys: no maximum, sums 0
+                    l_all[qq] += stats[(2 * w + 1) * kTile + 32 * qq + lr] * factor[qq][w];
+                }
+                inv[qq] = l_all[qq] > 0.f ? 1.0f / l_all[qq] : 0.f;
+            }
+            constexpr int kOwn = 4 / kTeam;           // tiles of d that a wavefront puts together
+            float4 own[kOwn][2][4];
+#pragma unroll
+            for (int t = 0; t < kOwn; ++t)
+#pragma unroll
+                for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+                    for (int gq = 0; gq < 4; ++gq) {
+                        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                        for (int w = 0; w < kTeam; ++w) {
+                            const float4 x = *reinterpret_cast<const float4*>(sums + w * (kTile * kD) + ((((wave * kOwn + t) * 2 + qq) * 4 + gq) * 64 + lane) * 4);
+                            const float fw = factor[qq][w];
+                            sum.x = fmaf(x.x, fw, sum.x); sum.y = fmaf(x.y, fw, sum.y); sum.z = fmaf(x.z, fw, sum.z); sum.w = fmaf(x.w, fw, sum.w);
+                        }
+                        own[t][qq][gq] = sum;
+                    }
+            if (parts.count > 1) {
+                float* const out = parts.buf + (int64_t)cur.local * kPartFloats;
+#pragma unroll
+                for (int t = 0; t < kOwn; ++t)
+#pragma unroll
+                    for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+                        for (int gq = 0; gq < 4; ++gq)
+                            *reinterpret_cast<float4*>(out + ((((wave * kOwn + t) * 2 + qq) * 4 + gq) * 64 + lane) * 4) = own[t][qq][gq];
+                if (wave == 0 && lh == 0) {
+#pragma unroll
+                    for (int qq = 0; qq < 2; ++qq) {
+                        out[kTile * kD + 32 * qq + lr] = M[qq];
+                        out[kTile * kD + kTile + 32 * qq + lr] = l_all[qq];
+                    }
+                }
+                return;
+            }
+            if (lse != nullptr && wave == 0 && lh == 0) {
+#pragma unroll
+                for (int qq = 0; qq < 2; ++qq) {
+                    int64_t row = qrow0 + 32 * qq + lr;
+                    if (L.q_rows != nullptr) row = out_rows[list_buf][32 * qq + lr];
+                    if (row >= 0) lse[(int64_t)bh * lse_S + row] = l_all[qq] > 0.f ? (M[qq] + __builtin_log2f(l_all[qq])) * kLn2 : -INFINITY;
+                }
+            }
+            __syncthreads();                          // the sums have been read: the memory becomes the staging tile
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+                for (int t = 0; t < kOwn; ++t)
+#pragma unroll
+                    for (int gq = 0; gq < 4; ++gq) {
+                        const float4 x = own[t][qq][gq];
+                        T out4[4] = {(T)(x.x * inv[qq]), (T)(x.y * inv[qq]), (T)(x.z * inv[qq]), (T)(x.w * inv[qq])};
+                        *reinterpret_cast<uint2*>(ost + (32 * qq + lr) * kOutPitch + 32 * (wave * kOwn + t) + 8 * gq + 4 * lh) = *reinterpret_cast<uint2*>(out4);
+                    }
+            __syncthreads();
+            const int kc = threadIdx.x & 15, kr = threadIdx.x >> 4;
+            constexpr int kRows = 4 * kTeam, kTurns = kTile / kRows;
+            u32x4 pieces[kTurns];
+            int32_t rows[kTurns];
+#pragma unroll
+            for (int i = 0; i < kTurns; ++i) {
+                rows[i] = L.q_rows != nullptr ? out_rows[list_buf][kr + kRows * i] : kr + kRows * i;
+                pieces[i] = *reinterpret_cast<const u32x4*>(ost + (kr + kRows * i) * kOutPitch + kc * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < kTurns; ++i)
+                if (rows[i] >= 0) *reinterpret_cast<u32x4*>(o + o_bh + ((L.q_rows != nullptr ? 0 : qrow0) + rows[i]) * L.o_st[2] + kc * 8) = pieces[i];
+            return;
+        }
         if (!kBounded && parts.count > 1) {
             float* const out = parts.buf + (int64_t)cur.local * kPartFloats;
 #pragma unroll
@@ -1038,6 +1206,8 @@ constexpr int kRoundsPerLaunch = 5;
 constexpr int kRoundsPerLaunchShort = 8;     // lists of at most kShortList tiles
 constexpr int kShortList = 64;
 
+constexpr int kOneRound = 1 << 30;           // more than a launch's items: each workgroup has one (the team kernels)
+
 // Workgroups (of one wavefront) the device runs at once with this kernel: one per SIMD, at most kMostResident (256 compute
 // units).
 constexpr int kMostResident = 1024;
@@ -1063,26 +1233,32 @@ __global__ void frag_zero_kernel(uint32_t* p, int n) {
     if (i < n) p[i] = 0u;
 }
 
-// How many parts the last, partial round of `items` work items with lists of list_tiles tiles is cut into, so that the
-// wavefronts it leaves idle share its walk: the count with the least estimated time.  A 64-key tile of a list takes 1.72 us of a
-// wavefront when the chip is full, 1.15 us when it is half empty (its power then allows the full clock: with one price for
-// both, rounds of 512 and 640 items were cut and a 480p layer took 1 838 us instead of 1 826, four heads of 720p 1 113 instead
-// of 1 095), a part 6 us to start and end, the merge a launch and the parts' bytes (33 KB written and read).  Shares of
-// fewer than 10 tiles are not worth it.
+// Into how many shares the items of the last, partial round are cut along their lists, so that the wavefronts it would leave
+// idle help: a team of `team` wavefronts an item, or `parts` parts of such teams, whichever has the least estimated time.  A
+// 64-key tile of a list takes 1.72 us of a wavefront when the chip is full, 1.15 us when it is half empty (its power then
+// allows the full clock: with one price for both, rounds of 512 and 640 items were cut and a 480p layer took 1 838 us instead
+// of 1 826, four heads of 720p 1 113 instead of 1 095); an item 6 us to start and end, 4.3 with a team of two, which stores
+// side by side, 5.8 with one of four; the merge of parts a launch and their bytes (33 KB written and read).  Shares of fewer
+// than 10 tiles are not worth a part.  Whole operator, one wavefront an item / two / four / two parts of teams of four, us: 16
+// items of 2 tiles 20.3 / 17.4 / 18.5, 64 of 4 23.4 / 19.4 / 19.9, 64 of 8 29.3 / 23.0 / 22.2, 128 of 32 60.7 / 40.5 / 33.0 /
+// 41.7, 128 of 128 184 / 108 / 71.5 / 64.3, 240 of 16 47.8 / 36.5 / 34.0 / 50.9, 384 of 32 72.4 / 52.9 / 62.9, 512 of 2 33.0 /
+// 31.0 / 37.7, 512 of 64 120 / 87 / 95.
 constexpr int kMaxParts = 16, kMaxPartRounds = 2, kMinPartTiles = 10;
-static int choose_parts(int items, int list_tiles, int resident) {
-    int best = 1;
+struct Split { int team, parts; };
+static Split choose_split(int items, int list_tiles, int resident, int most_team, bool parts_allowed) {
+    Split best = {1, 1};
     float best_us = 0.f;
-    for (int p = 1; p == 1 || (p <= kMaxParts && p * kMinPartTiles <= list_tiles && (int64_t)items * p <= kMaxPartRounds * resident); ++p) {
-        const int rounds = (int)(((int64_t)items * p + resident - 1) / resident);
-        const float full = (float)items * p / ((float)rounds * resident), tile_us = 1.15f + 1.14f * (full > 0.5f ? full - 0.5f : 0.f);
-        const float us = rounds * (tile_us * list_tiles / p + 6.f) + (p > 1 ? 5.f + 0.0125f * items * p : 0.f);
-        if (p == 1 || us < best_us) { best = p; best_us = us; }
-    }
+    for (int team = 1; team <= most_team && team <= list_tiles; team *= 2)
+        for (int p = 1; p == 1 || (parts_allowed && p <= kMaxParts && p * team * kMinPartTiles <= list_tiles && (int64_t)items * p * team <= kMaxPartRounds * resident); ++p) {
+            const int groups = resident / team, rounds = (int)(((int64_t)items * p + groups - 1) / groups);
+            const float full = (float)items * p / ((float)rounds * groups), tile_us = 1.15f + 1.14f * (full > 0.5f ? full - 0.5f : 0.f);
+            const float us = rounds * (tile_us * list_tiles / (p * team) + (team == 1 ? 6.f : team == 2 ? 4.3f : 5.8f)) + (p > 1 ? 5.f + 0.0125f * items * p : 0.f);
+            if ((team == 1 && p == 1) || us < best_us) { best = {team, p}; best_us = us; }
+        }
     return best;
 }
 // floats of the parts' buffer, whatever the length of the lists and whichever device runs the call (a caller asks for the size
-// of a workspace once, for all of its devices): a partial round has no more items than the call, choose_parts the limits
+// of a workspace once, for all of its devices): a partial round has no more items than the call, choose_split the limits
 size_t frag_part_floats(const Grid3& g, int64_t heads) {
     const int64_t all = heads * live_query_tiles(g) * kMaxParts, most = (int64_t)kMaxPartRounds * kMostResident;
     return (size_t)(all < most ? all : most) * kPartFloats;
@@ -1106,7 +1282,6 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const int per_head = (int)(Sq / kTile);
     const int all_tiles = B * Hn * per_head;
     const int resident = resident_wavefronts();
-    const dim3 block(64);
     const uint32_t* gate = nullptr;
     // The kernel addresses K and V through a buffer of less than 4 GB that starts at the first (batch, head) of a
     // launch: a launch covers as many heads as fit.  One head always does (fewer than 2^24 keys of 256 B).
@@ -1140,24 +1315,29 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const bool bounded = dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident;      // (see `whole` below)
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
-#define BSA_FRAG_LAUNCH_T(T, WALK, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
-    hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD>), grid, block, 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
-                       lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, resident, Hn, lse_rows, \
+#define BSA_FRAG_LAUNCH_T(T, WALK, BD, TEAM, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
+    hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD, TEAM>), grid, dim3(64 * TEAM), 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
+                       lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, TEAM > 1 ? kOneRound : resident, Hn, lse_rows, \
                        L, ord, que, gate, want, bh0, span, q_offsets_32, key_norm, fbl, fbc, parts)
-#define BSA_FRAG_LAUNCH(BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                                     \
+#define BSA_FRAG_LAUNCH_W(T, BD, TEAM, ...)                                                                            \
     do {                                                                                                               \
-        if (dtype == BSA_BF16) {                                                                                       \
-            if (halves) BSA_FRAG_LAUNCH_T(__bf16, kHalves, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
-            else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(__bf16, kTiles, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
-            else BSA_FRAG_LAUNCH_T(__bf16, kBlocks, BD, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);        \
-        } else {                                                                                                       \
-            if (halves) BSA_FRAG_LAUNCH_T(_Float16, kHalves, false, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
-            else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(_Float16, kTiles, false, grid, begin, end, ord, que, want, bh0, span, fbl, fbc); \
-            else BSA_FRAG_LAUNCH_T(_Float16, kBlocks, false, grid, begin, end, ord, que, want, bh0, span, fbl, fbc);   \
-        }                                                                                                              \
+        if (halves) BSA_FRAG_LAUNCH_T(T, kHalves, BD, TEAM, __VA_ARGS__);                                              \
+        else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(T, kTiles, BD, TEAM, __VA_ARGS__);                                   \
+        else BSA_FRAG_LAUNCH_T(T, kBlocks, BD, TEAM, __VA_ARGS__);                                                     \
+    } while (0)
+#define BSA_FRAG_LAUNCH(BD, ...)                                                                                       \
+    do {                                                                                                               \
+        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, BD, 1, __VA_ARGS__);                                          \
+        else BSA_FRAG_LAUNCH_W(_Float16, false, 1, __VA_ARGS__);                                                       \
+    } while (0)
+#define BSA_FRAG_LAUNCH_TEAM(TEAM, ...)                                                                                \
+    do {                                                                                                               \
+        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, __VA_ARGS__);                                    \
+        else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, __VA_ARGS__);                                                    \
     } while (0)
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
-    if (queue != nullptr && one_span) {
+    // Lists of unequal length of one round need no plan: every item has a wavefront of its own from the start.
+    if (queue != nullptr && one_span && total > resident) {
         hipLaunchKernelGGL(queue_plan_kernel, dim3(kQueues + 1), dim3(kPlanThreads), 0, st, lens, per_head, L, total, resident, idx_stride,
                            order, queue);
         gate = queue + kQueueChoice;
@@ -1169,11 +1349,15 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
     const int list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
     const int span = (list_tiles <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
-    // The last, partial round in parts when its wavefronts would leave too much of the chip idle (and the exact kernel
-    // reaches every head from one buffer; the caller gives a buffer for lists of one length only).
+    // The items of the last, partial round are cut when its wavefronts would leave too much of the chip idle (and the exact
+    // kernel reaches every head from one buffer): into parts only where the caller gives a buffer, for lists of one length; into
+    // teams only where there is no other round, so that calls with and without a buffer, with and without the queues, and over
+    // lists of halves and of blocks cut alike.
     const int tail = total % resident;
-    const int n_parts = part_buf != nullptr && one_span && queue == nullptr && tail > 0 ? choose_parts(tail, list_tiles, resident) : 1;
-    const int whole = n_parts > 1 ? total - tail : total;
+    Split split = {1, 1};
+    if (one_span && tail > 0 && (part_buf != nullptr || total < resident))
+        split = choose_split(tail, list_tiles, resident, total < resident ? 4 : 1, part_buf != nullptr);
+    const int whole = split.team * split.parts > 1 ? total - tail : total;
     for (int first = 0; first < whole;) {
         int end = first + span < whole ? first + span : whole;
         const int bh0 = one_span ? 0 : first / per_head;
@@ -1188,11 +1372,17 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                             (int32_t*)nullptr, (uint32_t*)nullptr);
         first = end;
     }
-    if (n_parts > 1) {
-        parts = {part_buf, n_parts, tail, divisor(n_parts), divisor(tail)};
-        const int n = tail * n_parts;
-        const dim3 grid((unsigned)(n < resident ? n : resident));
-        BSA_FRAG_LAUNCH(false, grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
+    if (whole < total) {
+        if (split.parts > 1) parts = {part_buf, split.parts, tail, divisor(split.parts), divisor(tail)};
+        const int n = tail * split.parts;
+        const dim3 grid((unsigned)(split.team == 1 && n > resident ? resident : n));
+#define BSA_FRAG_TAIL grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr
+        if (split.team == 4) BSA_FRAG_LAUNCH_TEAM(4, BSA_FRAG_TAIL);
+        else if (split.team == 2) BSA_FRAG_LAUNCH_TEAM(2, BSA_FRAG_TAIL);
+        else BSA_FRAG_LAUNCH(false, BSA_FRAG_TAIL);
+#undef BSA_FRAG_TAIL
+    }
+    if (split.parts > 1) {
         if (dtype == BSA_BF16)
             hipLaunchKernelGGL((merge_parts_kernel<__bf16>), dim3(tail), dim3(256), 0, st, parts, (__bf16*)o, lse, whole, per_head, Hn, lse_rows, L);
         else
@@ -1207,6 +1397,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         BSA_FRAG_LAUNCH(false, grid, 0, all_tiles, (const int32_t*)fb_list, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, fb_count);
     }
 #undef BSA_FRAG_LAUNCH
+#undef BSA_FRAG_LAUNCH_TEAM
+#undef BSA_FRAG_LAUNCH_W
 #undef BSA_FRAG_LAUNCH_T
     return hipGetLastError();
 }

@@ -1,0 +1,40 @@
+"""Work items of the attention kernel that several wavefronts of a workgroup share, against one wavefront an item."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent,chunk,width", [
+    ((4, 4, 8), (4, 4, 4), 2),           # two items: lists of 0, 1 and 2 tiles
+    ((5, 9, 13), (4, 4, 4), 5),          # shares of one tile and of two, padded tiles among them
+    ((5, 9, 20), (2, 8, 16), 3),         # blocks of four tiles, some of padding alone
+    ((13, 10, 11), (4, 4, 8), 20),       # blocks of two tiles
+    ((8, 16, 40), (4, 4, 4), 71),        # 80 items: more entries than a wavefront has lanes
+    ((8, 34, 40), (4, 4, 4), 180),       # 180 items and lists beyond the small buffers
+])
+def test_teams_equal_single_wavefronts(dtype, latent, chunk, width):
+    """The heads of a call of few items (teams of two and of four) and the same heads among so many that every item has one
+    wavefront, over caller's lists of 0 to `width` blocks.  Two orders of the same fp32 sums and two roundings of P: max-abs
+    1.6e-2 and mean-abs 1e-3 of outputs near 1, lse 2e-3."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    S = math.prod(latent)
+    blocks = math.prod(-(-n // c) for n, c in zip(latent, chunk))
+    tiles = math.prod(chunk) // 64
+    g = torch.Generator(device="cuda").manual_seed(21)
+    for few in (1, max(1, 300 // (blocks * tiles))):              # up to 256 items a team of four, up to 512 one of two
+        q, k, v = (torch.randn(1, few, S, 128, generator=g, device="cuda").to(dtype) for _ in range(3))
+        walk = torch.rand(1, few, blocks, blocks, generator=g, device="cuda").argsort(dim=-1)[..., :width].int().contiguous()
+        lens = torch.randint(0, width + 1, (1, few, blocks), generator=g, device="cuda", dtype=torch.int32)
+        many = -(-1100 // (few * blocks))
+        got, lse = bi.ThwAttention(k, v, latent, latent, chunk, chunk)(q, walk, lens, return_lse=True)
+        rep = lambda x: x.repeat(1, many, *([1] * (x.dim() - 2)))      # noqa: E731
+        want, want_lse = bi.ThwAttention(rep(k), rep(v), latent, latent, chunk, chunk)(rep(q), rep(walk), rep(lens), return_lse=True)
+        want, want_lse = want[:, :few], want_lse[:, :few]
+        d = (got.float() - want.float()).abs()
+        assert d.max() <= 1.6e-2 and d.mean() <= 1e-3, (float(d.max()), float(d.mean()))
+        assert torch.equal(torch.isinf(lse), torch.isinf(want_lse))
+        assert (lse - want_lse).nan_to_num().abs().max() <= 2e-3
