@@ -126,17 +126,18 @@ constexpr int kQueues = 8, kQueueChoice = kQueues, kQueueWords = kQueues + 1;   
 static_assert(kQueueWords <= kFragQueueWords, "the caller's buffer holds the words");
 __device__ __forceinline__ int section_begin(int n, int x) { return (int)(((int64_t)n * x) >> 3); }
 
-// kTeam: wavefronts that share an item, a workgroup on the SIMDs of one compute unit.  Each walks a share of the item's pairs
-// (a part's share, where the item is in parts as well) from the list that they stage together; then their sums are put
-// together in LDS, in the order of the shares, wavefront w those of its 4 / kTeam tiles of d, and the rows leave as from one
-// wavefront.  One item per workgroup, nothing prepared ahead.  For calls of so few items that most SIMDs would have none: see
-// choose_split.
+// kTeam: 0, one wavefront a workgroup, which runs one item after another as above; otherwise a workgroup runs one item, with
+// nothing prepared ahead and none of the code for it, as wavefronts that have a SIMD of a compute unit each.  1: a call of one
+// round (two prompts of 8 heads, 7x15x26: 40.0 -> 38.0 us).  2, 4: a team.  Each of its wavefronts walks a share of the item's pairs (of a part's
+// share, where the item is in parts as well) from the list that they stage together; then their sums are put together in LDS, in the
+// order of the shares, wavefront w those of its 4 / kTeam tiles of d, and the rows leave from all of them.  For calls of so few
+// items that most SIMDs would have none: see choose_split.
 template <int kTeam>
 constexpr int kTeamBytes = kTeam * (kTile * kD + 2 * kTile) * 4;      // the sums, maxima and row sums of every wavefront
 static_assert(kTeamBytes<4> <= 160 * 1024 && 2 * (kTeamBytes<2> + 512) <= 160 * 1024, "LDS of a compute unit with four wavefronts");
 
 template <typename T, int kWalk, bool kBounded, int kTeam>
-__global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
+__global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
     const int32_t* __restrict__ idx, const int32_t* __restrict__ lens, const uint64_t* __restrict__ tile_valid,
     T* __restrict__ o, float* __restrict__ lse, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride,
@@ -145,6 +146,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
     int bh_first, uint32_t kv_span_bytes, int q_offsets_32, const float* __restrict__ key_norm,
     int32_t* __restrict__ fallback, uint32_t* __restrict__ fallback_count, Parts parts) {
     typedef typename Vec8<T>::type V8;
+    constexpr bool kOnce = kTeam > 0;
     // log2 headroom before the running maximum is raised: probabilities reach 2^kTau, which the storage type of P
     // must hold (fp16 ends at 65 504) and the fp32 sums must hold times the number of keys
     constexpr float kTau = std::is_same<T, _Float16>::value ? 14.0f : 30.0f;
@@ -157,7 +159,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
     // fewer).
     constexpr float kSlack = 60.0f;
     static_assert(!kBounded || std::is_same<T, __bf16>::value, "fp16 probabilities need the running maximum");
-    static_assert(!kBounded || kTeam == 1, "a team leaves nothing to another launch");
+    static_assert(!kBounded || kTeam == 0, "a call of one round leaves nothing to another launch");
     typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
     // six lines: 0.36 us for the first five where one by one they took 0.7 to 1.1; with the sixth a call of two prompts of 8 heads,
     // 7x15x26, takes 41.4 us for 41.9.  With what an item that nothing has prepared asks for at once (below) and the divisions
@@ -173,9 +175,9 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
     __shared__ __attribute__((aligned(16))) char ost_bytes[kTeam > 1 ? kTeamBytes<kTeam> : kOutBytes];
     T* const ost = reinterpret_cast<T*>(ost_bytes);
     constexpr int kWords = kWalk == kHalves ? 2 : 1;              // list words of a pair
-    __shared__ __attribute__((aligned(8))) uint32_t lists[2][kTeam > 1 ? 2 : kPipeList * kWords];
+    __shared__ __attribute__((aligned(8))) uint32_t lists[2][kOnce ? 2 : kPipeList * kWords];
     __shared__ int32_t out_rows[2][kTile];       // token rows of this and the next item's 64 query slots (row table given)
-    __shared__ __attribute__((aligned(16))) char qstage[kTeam > 1 ? 16 : kTileBytes];      // Q of the next item, in register order
+    __shared__ __attribute__((aligned(16))) char qstage[kOnce ? 16 : kTileBytes];      // Q of the next item, in register order
     uint32_t* const big = reinterpret_cast<uint32_t*>(ost);
 
     const int lane = threadIdx.x & 63;
@@ -230,14 +232,14 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
         return -1;
     };
     int rounds_taken = 0;
-    auto next_local = [&]() -> int { return queue != nullptr ? draw() : round_local(rounds_taken++); };
+    auto next_local = [&]() -> int { return !kOnce && queue != nullptr ? draw() : round_local(rounds_taken++); };
     // what is known of an item ahead of time: its number, the length of its list and its first entry (both as
     // they lie in memory; they are clamped where they are used)
     struct Desc { int item, nent, ent[2], local; float kn; };       // ent: the first list entry (kHalves: the first two)
     auto fetch = [&](int local) -> Desc {
         Desc d = {-1, 0, {0, 0}, local, INFINITY};
         if (local < 0) return d;
-        if (!kBounded && parts.count > 1) local -= local / parts.by_items * parts.items;
+        if (!kBounded && kTeam != 1 && parts.count > 1) local -= local / parts.by_items * parts.items;
         d.item = order != nullptr ? item_begin + order[local] : item_at(L, item_begin + local, nqt);
         const int64_t row = d.item / L.by_block;
         d.nent = lens[row];
@@ -546,15 +548,16 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
     // ---- the workgroup's items
     Desc cur = {-1, 0, {0, 0}, -1, INFINITY}, nxt = cur;
 #pragma unroll 1
-    for (int i = 0; i < 2; ++i) {        // one copy of the code: a launch's first item pays for every line of it, cold
+    for (int i = 0; i < (kOnce ? 1 : 2); ++i) {        // one copy of the code: a launch's first item pays for every line of it, cold
         cur = nxt;
         nxt = fetch(next_local());
     }
+    if (kOnce) cur = nxt;
     bool prepared = false;           // the current item's list, Q rows and first fragments were requested by the item before it
     int list_buf = 0;                // which of the small list buffers holds the current item's list, if prepared
     while (uni(cur.item) >= 0) {
         cur.item = uni(cur.item);
-        const Desc nx2 = fetch(next_local());                    // in flight while this item runs
+        const Desc nx2 = kOnce ? cur : fetch(next_local());      // in flight while this item runs
         const int bh = cur.item / L.by_tiles;
         const int qtile = cur.item - bh * nqt;
         const int64_t qrow0 = (int64_t)qtile * kTile;
@@ -569,11 +572,11 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
         }
         // ... and so is a team's list, as far as one entry a thread goes (what lies behind its end is not used)
         int32_t team_entry = 0;
-        if (kTeam > 1 && idx_stride > 0) team_entry = idx[(int64_t)(cur.item / L.by_block) * idx_stride + min((int)threadIdx.x, idx_stride - 1)];
+        if (kOnce && idx_stride > 0) team_entry = idx[(int64_t)(cur.item / L.by_block) * idx_stride + min((int)threadIdx.x, idx_stride - 1)];
         __builtin_amdgcn_sched_barrier(0);
         const int nent = list_length(cur);
         npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
-        if (kTeam == 1 && !kBounded && parts.count > 1) {
+        if (!kOnce && !kBounded && parts.count > 1) {
             const int part = cur.local / parts.by_items;        // at most kMaxParts: the products fit 32 bits
             pair0 = npairs * part / parts.by_count;
             npairs = npairs * (part + 1) / parts.by_count - pair0;
@@ -583,7 +586,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
         // has a first tile to point the walk at, a list that fits a small buffer, and Q rows the LDS DMA can address
         const int next_nent = list_length(nxt);
         // (an item in parts has no first pair that is known ahead)
-        const bool prepare_next = kTeam == 1 && (kBounded || parts.count == 1) && nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
+        const bool prepare_next = !kOnce && (kBounded || parts.count == 1) && nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
         if (prepare_next) {
             first_pair(nxt, beyond);
             beyond[0] = (uint32_t)uni((int)beyond[0]);
@@ -595,7 +598,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
         const int64_t nqrow0 = (int64_t)(nitem - nbh * nqt) * kTile;
         const int32_t* nlist = idx + (int64_t)(nitem / L.by_block) * idx_stride;
 
-        const bool early = kTeam == 1 && (kBounded || parts.count == 1);         // the walk starts at the list's first entry
+        const bool early = kTeam == 1 || (!kOnce && (kBounded || parts.count == 1));         // the walk starts at the list's first entry
         auto first_fragments = [&](uint32_t h0, uint32_t h1) {
 #pragma unroll
             for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(h0, c);                       // K(0)
@@ -615,7 +618,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
             const int32_t* list = idx + (int64_t)(cur.item / L.by_block) * idx_stride;
             constexpr int kAhead = 4;
             int32_t entry[kAhead] = {0, 0, 0, 0};
-            if (kTeam == 1 && nent > 0) {
+            if (!kOnce && nent > 0) {
 #pragma unroll
                 for (int e = 0; e < kAhead; ++e) entry[e] = list[min(lane_now + 64 * e, nent - 1)];
             }
@@ -635,8 +638,8 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
                 first_fragments((uint32_t)uni((int)h[0]), (uint32_t)uni((int)h[1]));
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (L.q_rows != nullptr && (kTeam == 1 || wave == 0)) out_rows[list_buf][lane_now] = first_rows[2];
-            if constexpr (kTeam == 1) {
+            if (L.q_rows != nullptr && wave == 0) out_rows[list_buf][lane_now] = first_rows[2];
+            if constexpr (!kOnce) {
 #pragma unroll
                 for (int e = 0; e < kAhead; ++e)
                     if (lane_now + 64 * e < nent) big[lane_now + 64 * e] = (uint32_t)entry[e];
@@ -839,7 +842,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
                 raw = pair_raw(g + 5);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (kTeam == 1) __syncthreads();          // the list in LDS has been read: the memory may become the staging tile (a team: below)
+            if (kTeam <= 1) __syncthreads();          // the list in LDS has been read: the memory may become the staging tile (a team: below)
             if (prepare_next) {
                 // The DMA of the next item's list and Q rows was issued in front of the loop and every iteration has
                 // issued 32 loads since; loads complete in order, so all but the newest 24 done (the next item's first
@@ -967,7 +970,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
                 if (rows[i] >= 0) *reinterpret_cast<u32x4*>(o + o_bh + ((L.q_rows != nullptr ? 0 : qrow0) + rows[i]) * L.o_st[2] + kc * 8) = pieces[i];
             return;
         }
-        if (!kBounded && parts.count > 1) {
+        if (!kOnce && !kBounded && parts.count > 1) {
             float* const out = parts.buf + (int64_t)cur.local * kPartFloats;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
@@ -1043,6 +1046,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_frag_kernel(
                 if (rows[i] >= 0) *reinterpret_cast<u32x4*>(o + o_bh + (row_base + rows[i]) * L.o_st[2] + kc * 8) = pieces[i];
         }
         }   // run
+        if constexpr (kOnce) return;
         // ---- on to the next item
         prepared = prepare_next && run;
         if (prepared) list_buf ^= 1;
@@ -1206,7 +1210,7 @@ constexpr int kRoundsPerLaunch = 5;
 constexpr int kRoundsPerLaunchShort = 8;     // lists of at most kShortList tiles
 constexpr int kShortList = 64;
 
-constexpr int kOneRound = 1 << 30;           // more than a launch's items: each workgroup has one (the team kernels)
+constexpr int kOneRound = 1 << 30;           // more than a launch's items: each workgroup has one (kTeam > 0)
 
 // Workgroups (of one wavefront) the device runs at once with this kernel: one per SIMD, at most kMostResident (256 compute
 // units).
@@ -1316,8 +1320,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
 #define BSA_FRAG_LAUNCH_T(T, WALK, BD, TEAM, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
-    hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD, TEAM>), grid, dim3(64 * TEAM), 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
-                       lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, TEAM > 1 ? kOneRound : resident, Hn, lse_rows, \
+    hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD, TEAM>), grid, dim3(TEAM > 1 ? 64 * TEAM : 64), 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
+                       lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, TEAM > 0 ? kOneRound : resident, Hn, lse_rows, \
                        L, ord, que, gate, want, bh0, span, q_offsets_32, key_norm, fbl, fbc, parts)
 #define BSA_FRAG_LAUNCH_W(T, BD, TEAM, ...)                                                                            \
     do {                                                                                                               \
@@ -1327,10 +1331,10 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     } while (0)
 #define BSA_FRAG_LAUNCH(BD, ...)                                                                                       \
     do {                                                                                                               \
-        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, BD, 1, __VA_ARGS__);                                          \
-        else BSA_FRAG_LAUNCH_W(_Float16, false, 1, __VA_ARGS__);                                                       \
+        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, BD, 0, __VA_ARGS__);                                          \
+        else BSA_FRAG_LAUNCH_W(_Float16, false, 0, __VA_ARGS__);                                                       \
     } while (0)
-#define BSA_FRAG_LAUNCH_TEAM(TEAM, ...)                                                                                \
+#define BSA_FRAG_LAUNCH_ONCE(TEAM, ...)                                                                                \
     do {                                                                                                               \
         if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, __VA_ARGS__);                                    \
         else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, __VA_ARGS__);                                                    \
@@ -1357,7 +1361,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     Split split = {1, 1};
     if (one_span && tail > 0 && (part_buf != nullptr || total < resident))
         split = choose_split(tail, list_tiles, resident, total < resident ? 4 : 1, part_buf != nullptr);
-    const int whole = split.team * split.parts > 1 ? total - tail : total;
+    const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
+    const int whole = once ? 0 : split.parts > 1 ? total - tail : total;
     for (int first = 0; first < whole;) {
         int end = first + span < whole ? first + span : whole;
         const int bh0 = one_span ? 0 : first / per_head;
@@ -1374,11 +1379,12 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     }
     if (whole < total) {
         if (split.parts > 1) parts = {part_buf, split.parts, tail, divisor(split.parts), divisor(tail)};
-        const int n = tail * split.parts;
+        const int n = (total - whole) * split.parts;
         const dim3 grid((unsigned)(split.team == 1 && n > resident ? resident : n));
 #define BSA_FRAG_TAIL grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr
-        if (split.team == 4) BSA_FRAG_LAUNCH_TEAM(4, BSA_FRAG_TAIL);
-        else if (split.team == 2) BSA_FRAG_LAUNCH_TEAM(2, BSA_FRAG_TAIL);
+        if (split.team == 4) BSA_FRAG_LAUNCH_ONCE(4, BSA_FRAG_TAIL);
+        else if (split.team == 2) BSA_FRAG_LAUNCH_ONCE(2, BSA_FRAG_TAIL);
+        else if (once) BSA_FRAG_LAUNCH_ONCE(1, BSA_FRAG_TAIL);
         else BSA_FRAG_LAUNCH(false, BSA_FRAG_TAIL);
 #undef BSA_FRAG_TAIL
     }
@@ -1397,7 +1403,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         BSA_FRAG_LAUNCH(false, grid, 0, all_tiles, (const int32_t*)fb_list, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, fb_count);
     }
 #undef BSA_FRAG_LAUNCH
-#undef BSA_FRAG_LAUNCH_TEAM
+#undef BSA_FRAG_LAUNCH_ONCE
 #undef BSA_FRAG_LAUNCH_W
 #undef BSA_FRAG_LAUNCH_T
     return hipGetLastError();
