@@ -1210,6 +1210,10 @@ constexpr int kRoundsPerLaunch = 5;
 constexpr int kRoundsPerLaunchShort = 8;     // lists of at most kShortList tiles
 constexpr int kShortList = 64;
 
+// Tiles a wavefront walks in all of a call's rounds, up to which it runs the exact kernel alone (bounded / exact, us: 1 120 items
+// of 4 tiles 55.0 / 52.8, of 16, the last round in teams, 83.3 / 81.4, of 32 116.9 / 115.6, of 64 183.5 / 184.0; 2 160 of 4 87.8 /
+// 87.4, of 16 133.0 / 132.4, of 32 196.0 / 196.5; 2 700 of 11 132.6 / 133.8).
+constexpr int kExactRoundTiles = 24;
 constexpr int kOneRound = 1 << 30;           // more than a launch's items: each workgroup has one (kTeam > 0)
 
 // Workgroups (of one wavefront) the device runs at once with this kernel: one per SIMD, at most kMostResident (256 compute
@@ -1247,16 +1251,22 @@ __global__ void frag_zero_kernel(uint32_t* p, int n) {
 // items of 2 tiles 20.3 / 17.4 / 18.5, 64 of 4 23.4 / 19.4 / 19.9, 64 of 8 29.3 / 23.0 / 22.2, 128 of 32 60.7 / 40.5 / 33.0 /
 // 41.7, 128 of 128 184 / 108 / 71.5 / 64.3, 240 of 16 47.8 / 36.5 / 34.0 / 50.9, 384 of 32 72.4 / 52.9 / 62.9, 512 of 2 33.0 /
 // 31.0 / 37.7, 512 of 64 120 / 87 / 95.
+// Uncut, the items behind whole rounds (is_tail) were prepared by those before them and start at once; cut, they wait for
+// another launch (4 us).  Items of one length behind one whole round, uncut / teams of two / of four: 56 of 8 64.3 / 63.9 / 64.0,
+// of 16 88.9 / 84.6 / 82.7, of 64 225 / 197 / 183; 272 of 8 68.3 / 70.7, of 16 91.7 / 90.0, of 64 231 / 206; 416 of 16 94.2 / 93.0,
+// of 64 232 / 214; behind two, 512 of 16 144.3 / 144.8, of 64 368 / 361.  As many shares as there are wavefronts are not made behind
+// whole rounds: little is gained, and a call by the CDF rule, which is not cut there, gives the bits of one by the top-k rule.
 constexpr int kMaxParts = 16, kMaxPartRounds = 2, kMinPartTiles = 10;
 struct Split { int team, parts; };
-static Split choose_split(int items, int list_tiles, int resident, int most_team, bool parts_allowed) {
+static Split choose_split(int items, int list_tiles, int resident, bool is_tail, bool parts_allowed) {
     Split best = {1, 1};
     float best_us = 0.f;
-    for (int team = 1; team <= most_team && team <= list_tiles; team *= 2)
+    for (int team = 1; team <= 4 && team <= list_tiles && !(is_tail && team > 1 && items * team >= resident); team *= 2)
         for (int p = 1; p == 1 || (parts_allowed && p <= kMaxParts && p * team * kMinPartTiles <= list_tiles && (int64_t)items * p * team <= kMaxPartRounds * resident); ++p) {
             const int groups = resident / team, rounds = (int)(((int64_t)items * p + groups - 1) / groups);
+            const float start = team == 2 ? 4.3f : team == 4 ? 5.8f : is_tail && p == 1 ? 0.f : 6.f;
             const float full = (float)items * p / ((float)rounds * groups), tile_us = 1.15f + 1.14f * (full > 0.5f ? full - 0.5f : 0.f);
-            const float us = rounds * (tile_us * list_tiles / (p * team) + (team == 1 ? 6.f : team == 2 ? 4.3f : 5.8f)) + (p > 1 ? 5.f + 0.0125f * items * p : 0.f);
+            const float us = rounds * (tile_us * list_tiles / (p * team) + start) + (p > 1 ? 5.f + 0.0125f * items * p : 0.f) + (is_tail && p * team > 1 ? 4.f : 0.f);
             if ((team == 1 && p == 1) || us < best_us) { best = {team, p}; best_us = us; }
         }
     return best;
@@ -1313,10 +1323,11 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const int q_offsets_32 = q_rows_max * q_st[2] * 2 + 512 < ((int64_t)1 << 32) ? 1 : 0;
     // The bf16 rounds run the kernel whose steps take no row maxima when the key norms are known, a place for the list of
     // the items it has to leave to the other kernel is given, and that kernel can reach every head from one buffer.
-    // A call of one round runs the exact kernel alone: its steps are 3 % longer, but a last launch that finds nothing to do
-    // costs 3.6 us, a fifth of a small call's attention.
+    // A short call runs the exact kernel alone: its steps are 3 % longer, but a last launch that finds nothing to do costs 4.7 us.
     Parts parts = {nullptr, 1, 0, divisor(1), divisor(1)};
-    const bool bounded = dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident;      // (see `whole` below)
+    const int list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
+    const bool bounded = dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident &&
+                         (int64_t)total * list_tiles > (int64_t)kExactRoundTiles * resident;
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
 #define BSA_FRAG_LAUNCH_T(T, WALK, BD, TEAM, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
@@ -1351,7 +1362,6 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     }
     // kRoundsPerLaunch rounds per launch, every workgroup running one item of each: the items of a round start
     // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
-    const int list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
     const int span = (list_tiles <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
     // The items of the last, partial round are cut when its wavefronts would leave too much of the chip idle (and the exact
     // kernel reaches every head from one buffer): into parts only where the caller gives a buffer, for lists of one length; into
@@ -1360,9 +1370,9 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const int tail = total % resident;
     Split split = {1, 1};
     if (one_span && tail > 0 && (part_buf != nullptr || total < resident))
-        split = choose_split(tail, list_tiles, resident, total < resident ? 4 : 1, part_buf != nullptr);
+        split = choose_split(tail, list_tiles, resident, total > resident, part_buf != nullptr);
     const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
-    const int whole = once ? 0 : split.parts > 1 ? total - tail : total;
+    const int whole = once ? 0 : split.team * split.parts > 1 ? total - tail : total;
     for (int first = 0; first < whole;) {
         int end = first + span < whole ? first + span : whole;
         const int bh0 = one_span ? 0 : first / per_head;

@@ -38,3 +38,21 @@ def test_teams_equal_single_wavefronts(dtype, latent, chunk, width):
         assert d.max() <= 1.6e-2 and d.mean() <= 1e-3, (float(d.max()), float(d.mean()))
         assert torch.equal(torch.isinf(lse), torch.isinf(want_lse))
         assert (lse - want_lse).nan_to_num().abs().max() <= 2e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads,sparsity", [(9, 0.5), (9, 0.75), (11, 0.5)])      # 128 items behind 1 024 (teams of four), 384 (teams of two)
+def test_last_round_in_teams(heads, sparsity, dtype):
+    """The items behind whole rounds in teams, against the kernel on whole lists (ThwAttention, which cuts nothing there): the same
+    bits in the whole rounds, two summation orders behind them (max-abs 1.6e-2, mean-abs 1e-3, lse 2e-3)."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    latent, chunk = (8, 32, 32), (4, 4, 4)
+    S = math.prod(latent)
+    g = torch.Generator(device="cuda").manual_seed(22)
+    q, k, v = (torch.randn(1, heads, S, 128, generator=g, device="cuda").to(dtype) for _ in range(3))
+    o, walk, lens, lse = bi._bsa_3d(q, k, v, latent, latent, sparsity, chunk, chunk, for_backward=True)
+    want, want_lse = bi.ThwAttention(k, v, latent, latent, chunk, chunk)(q, walk, lens, return_lse=True)
+    assert torch.equal(o[:, :8], want[:, :8]) and torch.equal(lse[:, :8], want_lse[:, :8])
+    d = (o.float() - want.float()).abs()
+    assert d.max() <= 1.6e-2 and d.mean() <= 1e-3, (float(d.max()), float(d.mean()))
+    assert not torch.equal(o, want) and torch.allclose(lse, want_lse, atol=2e-3)
