@@ -720,17 +720,23 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
 constexpr int kDsPairBytes = kTile * kTile * 2, kDsUnitBytes = kDsPairBytes / 2;
 constexpr int kDsqAhead = 4;
 
-template <typename T>
-__global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const char* __restrict__ ks_turned, const char* __restrict__ ds, const char* __restrict__ zeros,
+// kTeam: wavefronts of a workgroup that share the list of its query rows, a contiguous share of the entries each; their sums are
+// put together in LDS, in the order of the shares, 4 / kTeam tiles of d to a wavefront.  For calls whose query tiles would leave
+// most SIMDs without one (launch_bwd).
+template <typename T, int kTeam>
+__global__ __launch_bounds__(64 * kTeam, 1) void bwd_dq_from_ds_kernel(const char* __restrict__ ks_turned, const char* __restrict__ ds, const char* __restrict__ zeros,
                                                             const int32_t* __restrict__ idx, const int32_t* __restrict__ place,
                                                             const int32_t* __restrict__ lens, T* __restrict__ dq, int64_t Sq,
                                                             int64_t Sk, int bs_q, int bs_k, int stride, int item_begin, int item_end,
                                                             int round, int64_t pairs_per_head, BwdStore dq_to, DqSizes sz,
                                                             const int32_t* __restrict__ q_live, const int32_t* __restrict__ k_live) {
     typedef typename Vec8<T>::type V8;
-    __shared__ __attribute__((aligned(16))) char turn[2 * 2048];
-    const int lane = threadIdx.x, lr = lane & 31, lh = lane >> 5;
-    touch_arguments<decltype(bwd_dq_from_ds_kernel<T>)>();
+    constexpr int kTurnBytes = 2 * 2048, kSumFloats = kTile * kD;
+    __shared__ __attribute__((aligned(16))) char turns[kTeam > 1 ? kTeam * kSumFloats * 4 : kTurnBytes];      // a team's sums lie where its dS was
+    const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
+    const int wave = kTeam > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
+    char* const turn = turns + wave * kTurnBytes;
+    touch_arguments<decltype(bwd_dq_from_ds_kernel<T, kTeam>)>();
     int item;
     {
         const int local = blockIdx.x, r0 = local / sz.by_round * round;
@@ -741,10 +747,11 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const char* __restri
     const int64_t bh = head, qrow0 = (int64_t)(item - head * sz.tiles) * kTile, lrow = lrow_n;
     const int nbk = (int)(Sk / kTile) / sz.by_sub, nsub = bs_k / kTile, sub_q = item - lrow_n * (bs_q / kTile);
     // the list, 64 entries at a time in a register each, an entry per lane: block, dS unit, halves with keys
-    const int n = __builtin_amdgcn_readfirstlane(min(max(lens[lrow], 0), stride));
+    const int n_all = __builtin_amdgcn_readfirstlane(min(max(lens[lrow], 0), stride));
+    const int e_begin = n_all * wave / kTeam, n = n_all * (wave + 1) / kTeam - e_begin;      // this wavefront's share
     int list_j = 0, list_p = 0, list_n = 2 * nsub;
     auto take_entries = [&](int e0) {
-        const int e = max(min(e0 + lane, n - 1), 0);
+        const int e = max(min(e_begin + e0 + lane, e_begin + n - 1), 0);
         list_j = min(max(idx[lrow * stride + e], 0), nbk - 1);
         list_p = place[lrow * stride + e];
         if (k_live != nullptr) list_n = k_live[list_j];
@@ -760,7 +767,7 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const char* __restri
     int n_real = 2 * n * nsub;
     if (k_live != nullptr) {
         int mine = lane < n ? list_n : 0;
-        for (int e = 64 + lane; e < n; e += 64) mine += k_live[min(max(idx[lrow * stride + e], 0), nbk - 1)];
+        for (int e = 64 + lane; e < n; e += 64) mine += k_live[min(max(idx[lrow * stride + e_begin + e], 0), nbk - 1)];
         n_real = wave_sum(mine);
     }
     entries_there();
@@ -862,6 +869,41 @@ __global__ __launch_bounds__(64) void bwd_dq_from_ds_kernel(const char* __restri
             });
         }
     }
+    if constexpr (kTeam > 1) {
+        float* const sums = reinterpret_cast<float*>(turns);
+        __syncthreads();                          // every wavefront is through with its dS
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<float4*>(sums + wave * kSumFloats + (((t * 2 + qq) * 4 + g) * 64 + lane) * 4) =
+                        make_float4(acc[t][qq][4 * g], acc[t][qq][4 * g + 1], acc[t][qq][4 * g + 2], acc[t][qq][4 * g + 3]);
+        __syncthreads();
+        constexpr int kOwn = 4 / kTeam;
+        T* const base = dq_to.rows == nullptr ? dq + bh * Sq * kD : dq + (bh / dq_to.Hn) * dq_to.sB + (bh % dq_to.Hn) * dq_to.sH;
+        const int64_t pitch = dq_to.rows == nullptr ? kD : dq_to.sS;
+#pragma unroll
+        for (int qq = 0; qq < 2; ++qq)
+#pragma unroll
+            for (int own = 0; own < kOwn; ++own) {
+                const int t = wave * kOwn + own;
+                float x[16];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                    for (int w = 0; w < kTeam; ++w) {
+                        const float4 part = *reinterpret_cast<const float4*>(sums + w * kSumFloats + (((t * 2 + qq) * 4 + g) * 64 + lane) * 4);
+                        sum.x += part.x; sum.y += part.y; sum.z += part.z; sum.w += part.w;
+                    }
+                    x[4 * g] = sum.x * kLn2; x[4 * g + 1] = sum.y * kLn2; x[4 * g + 2] = sum.z * kLn2; x[4 * g + 3] = sum.w * kLn2;
+                }
+                store_columns(base + rows[qq] * pitch + 32 * t, rows[qq] >= 0, x, lane);
+            }
+        return;
+    }
     store_dq<T>(acc, dq, dq_to, bh, Sq, rows, lane);
 }
 
@@ -902,8 +944,11 @@ struct DkdvSizes {
     int tiles, nbq, nsub;            // key tiles of a (batch, head), query blocks, tiles of a KV block
     Divisor by_tiles, by_block, by_round;
 };
-template <typename T, bool kMasked, bool kKeep>
-__global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, const T* __restrict__ dout,
+// kGroups: pairs of wavefronts that share a tile's list of query blocks, a half of its entries each, every pair with stages of its
+// own; at the end one adds up dK and the other dV, through LDS.  2 for calls of no more key tiles than there are compute units,
+// which leave two of four SIMDs without a wavefront: see launch_bwd.
+template <typename T, bool kMasked, bool kKeep, int kGroups>
+__global__ __launch_bounds__(128 * kGroups, 1) void bwd_dkdv_kernel(const T* __restrict__ q, const T* __restrict__ dout,
                                                        BwdLoad k_from, BwdLoad v_from,
                                                        const float* __restrict__ m2, const float* __restrict__ delta,
                                                        const uint32_t* __restrict__ bits,
@@ -917,8 +962,9 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     typedef typename Vec8<T>::type V8;
     extern __shared__ __attribute__((aligned(1024))) char bwd_lds[];
     const int lane = threadIdx.x & 63, lr = lane & 31, lh = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    touch_arguments<decltype(bwd_dkdv_kernel<T, kMasked, kKeep>)>();
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) & 1);
+    const int group = kGroups > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 7)) : 0;
+    touch_arguments<decltype(bwd_dkdv_kernel<T, kMasked, kKeep, kGroups>)>();
     // items longest list first, every XCD on a contiguous run of each group of `round` (see launch_bwd); a scalar, and with it
     // all that is derived from it (left to the compiler, addresses of the loop were made scalars half by half)
     int item;
@@ -936,7 +982,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     int key_halves = 2;
     if (k_live != nullptr) key_halves = __builtin_amdgcn_readfirstlane(k_live[block - head * (sz.tiles / sz.by_block)]) - 2 * (item - block * nsub);
     // halves come in pairs: an odd number of them ends with the last one again, whose p are 0 (M2 = -inf)
-    const int n_real = __builtin_amdgcn_readfirstlane(counts[block]), nhalves = (n_real + 1) & ~1;
+    int n_real = __builtin_amdgcn_readfirstlane(counts[block]), nhalves = (n_real + 1) & ~1;
     // the row of this lane's key: its token, or in blocked order its slot
     int64_t key_row = krow0 + 32 * wave + lr;
     if (dk_to.rows != nullptr) key_row = dk_to.rows[key_row];
@@ -949,9 +995,10 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         for (int i = 0; i < 16; ++i) { acc_dk[t][i] = 0.f; acc_dv[t][i] = 0.f; }
 
     // behind every stage's numbers: M2 for padded keys
-    *reinterpret_cast<float*>(bwd_lds + kBwdNumbers + (threadIdx.x >> 5) * kBwdStats + 256 + (threadIdx.x & 31) * 4) = -INFINITY;
+    char* const stages = bwd_lds + group * (kBwdStages * kBwdStage);
+    *reinterpret_cast<float*>(stages + kBwdNumbers + ((threadIdx.x >> 5) & 3) * kBwdStats + 256 + (threadIdx.x & 31) * 4) = -INFINITY;
     // the query blocks of this KV block, ascending, from the bit matrix into LDS (behind the stages)
-    int32_t* qlist = reinterpret_cast<int32_t*>(bwd_lds + kBwdStages * kBwdStage);
+    int32_t* qlist = reinterpret_cast<int32_t*>(bwd_lds + kGroups * kBwdStages * kBwdStage);
     uint32_t word_now = 0, plane[kPlanesAtHand] = {};
     auto take_words = [&](int w) {
         word_now = w < words ? mask_row[w] : 0u;
@@ -992,7 +1039,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
             if (lane >= off) upto += t;
         }
         int pos = count + upto - mine;
-        if (wave == 0)
+        if (wave == 0 && group == 0)
             while (word != 0u) {
                 const int b = __builtin_ctz(word);
                 uint32_t n = 0;
@@ -1010,23 +1057,41 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         count += __shfl(upto, 63);
     }
     __syncthreads();
-    const int count_u = __builtin_amdgcn_readfirstlane(count);          // the same in every lane; the compiler cannot tell
+    int count_u = __builtin_amdgcn_readfirstlane(count);          // the same in every lane; the compiler cannot tell
+    // This pair's share of the list: entries, halves, and the halves in front of it.  Both pairs walk as many as the one that has more:
+    // the barriers are the workgroup's.
+    int halves_before = 0;
+    if constexpr (kGroups > 1) {
+        const int all = n_real, middle = count_u >> 1;
+        int mine = 0;
+        for (int e = lane; e < middle; e += 64) mine += q_live.live != nullptr ? (int)((uint32_t)qlist[e] >> kBlockBits) : q_live.full;
+        const int first_share = wave_sum(mine);
+        halves_before = group == 0 ? 0 : first_share;
+        n_real = group == 0 ? first_share : all - first_share;
+        nhalves = (max(first_share, all - first_share) + 1) & ~1;
+        qlist += group == 0 ? 0 : middle;
+        count_u = group == 0 ? middle : count_u - middle;
+    }
     // the walk's halves one after another, without a branch; the entry of the next block is read from LDS a half before it is used
     int next_block = 0, next_entry = 0, block_half = 0, half = 0, halves = 0;
     if (nhalves > 0) next_block = qlist[0];
+    if (kGroups > 1 && n_real == 0) {            // an empty share: the other pair's only block, all of it a repeat
+        block_half = (int)((uint32_t)__builtin_amdgcn_readfirstlane(next_block) & ((1u << kBlockBits) - 1u)) * q_live.full;
+        half = halves = 1;
+    }
     auto next_half = [&](bool more) -> int {                     // !more: the last one again
         const uint32_t entry = (uint32_t)__builtin_amdgcn_readfirstlane(next_block);
         const bool fresh = more && half == halves;
         block_half = fresh ? (int)(entry & ((1u << kBlockBits) - 1u)) * q_live.full : block_half;
         halves = fresh ? (q_live.live != nullptr ? (int)(entry >> kBlockBits) : q_live.full) : halves;
         half = (fresh ? 0 : half) + (more ? 1 : 0);
-        next_entry = min(next_entry + (fresh ? 1 : 0), count_u - 1);
+        next_entry = min(next_entry + (fresh ? 1 : 0), kGroups > 1 ? max(count_u - 1, 0) : count_u - 1);
         next_block = qlist[next_entry];
         return block_half + half - 1;
     };
 
     // ---- global -> LDS
-    const uint32_t lds0 = lds_address(bwd_lds);
+    const uint32_t lds0 = lds_address(bwd_lds) + (uint32_t)(group * (kBwdStages * kBwdStage));
     uint32_t voff[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1077,7 +1142,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
     // p = exp2(-inf) = 0
     uint32_t numbers = lds0 + (uint32_t)(kBwdNumbers + 16 * lh), m2_at = numbers + (kMasked && !key_ok ? 256u : 0u);
     char* ds_item = !kKeep ? nullptr
-        : ds_out + bh * pairs_per_head * kDsPairBytes + ((int64_t)__builtin_amdgcn_readfirstlane(unit_base[block]) + (item - block * nsub)) * kDsUnitBytes + wave * 2048;
+        : ds_out + bh * pairs_per_head * kDsPairBytes + ((int64_t)__builtin_amdgcn_readfirstlane(unit_base[block]) + (item - block * nsub) + (int64_t)halves_before * nsub) * kDsUnitBytes + wave * 2048;
     // P and dS of a half as B operands, and the transposed fragments of its rows (dO and Q of d tile t at 2 t and 2 t + 1): its first
     // and its last 16 queries
     V8 p_ab[2], ds_ab[2], tr_ab[2][8];
@@ -1099,9 +1164,9 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         constexpr int odd = decltype(odd_c)::value;                  // hp & 1
         constexpr uint32_t qn = (odd ^ 1) * kBwdHalfTile, dn = qn + kBwdDout;      // rows of half hp + 1, in its pair of stages
         constexpr uint32_t qt = odd * kBwdHalfTile, dt = qt + kBwdDout;            // rows of half hp
-        // the halves with an odd number alone may be the one that repeats
-        const uint32_t m2_here = odd || hp + 1 < n_real ? m2_at : numbers + 256;
-        char* const ds_to = !odd || hp < n_real ? ds_item : ds_spare;
+        // the halves with an odd number alone may be the one that repeats (with two pairs, all behind this one's share)
+        const uint32_t m2_here = (odd && kGroups == 1) || hp + 1 < n_real ? m2_at : numbers + 256;
+        char* const ds_to = (!odd && kGroups == 1) || hp < n_real ? ds_item : ds_spare;
         auto exponential = [&](int e) {
             s[e] = __builtin_amdgcn_exp2f(s[e]);                     // S - M2 -> P
             asm volatile("" : "+v"(s[e]));
@@ -1228,13 +1293,14 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
                 __builtin_amdgcn_s_barrier();
             }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // nothing may land in LDS that is no longer this workgroup's
+            if (kGroups > 1) { __syncthreads(); __syncthreads(); }       // where the others put their sums together
             return;
         }
         f32x16 s0, dp0, s1, dp1;
         V8 first_q[8], first_d[8];
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const f32x4_ mm = lds_read_at<f32x4_>(m2_at + 32 * g), dd = lds_read_at<f32x4_>(numbers + (128 + 32 * g));
+            const f32x4_ mm = lds_read_at<f32x4_>((kGroups == 1 || n_real > 0 ? m2_at : numbers + 256) + 32 * g), dd = lds_read_at<f32x4_>(numbers + (128 + 32 * g));
             s0[4 * g] = mm.x; s0[4 * g + 1] = mm.y; s0[4 * g + 2] = mm.z; s0[4 * g + 3] = mm.w;
             dp0[4 * g] = dd.x; dp0[4 * g + 1] = dd.y; dp0[4 * g + 2] = dd.z; dp0[4 * g + 3] = dd.w;
         }
@@ -1267,6 +1333,30 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // nothing may land in LDS that is no longer this workgroup's
     }
+    if constexpr (kGroups > 1) {
+        // The first pair leaves its dV, the second its dK, 16 KB a wavefront, and takes the other: first pair's sum plus second's.
+        if (nhalves > 0) {
+            __syncthreads();
+            float* const mine = reinterpret_cast<float*>(bwd_lds) + (2 * group + wave) * (32 * kD);
+            const float* const theirs = reinterpret_cast<const float*>(bwd_lds) + (2 * (group ^ 1) + wave) * (32 * kD);
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x16& x = group == 0 ? acc_dv[t] : acc_dk[t];
+                    *reinterpret_cast<float4*>(mine + ((t * 4 + g) * 64 + lane) * 4) = make_float4(x[4 * g], x[4 * g + 1], x[4 * g + 2], x[4 * g + 3]);
+                }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const float4 y = *reinterpret_cast<const float4*>(theirs + ((t * 4 + g) * 64 + lane) * 4);
+                    f32x16& x = group == 0 ? acc_dk[t] : acc_dv[t];
+                    x[4 * g] += y.x; x[4 * g + 1] += y.y; x[4 * g + 2] += y.z; x[4 * g + 3] += y.w;
+                }
+        }
+    }
     // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, key lr
     {
         const int batch = head / dk_to.Hn, in_batch = head - batch * dk_to.Hn;
@@ -1282,8 +1372,8 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
                 xk[i] = (kMasked && !key_ok ? 0.f : acc_dk[t][i]) * dk_scale;
                 xv[i] = kMasked && !key_ok ? 0.f : acc_dv[t][i];
             }
-            store_columns(out_k + 32 * t, key_row >= 0, xk, lane);
-            store_columns(out_v + 32 * t, key_row >= 0, xv, lane);
+            if (kGroups == 1 || group == 0) store_columns(out_k + 32 * t, key_row >= 0, xk, lane);
+            if (kGroups == 1 || group == 1) store_columns(out_v + 32 * t, key_row >= 0, xv, lane);
         }
     }
 }
@@ -1292,7 +1382,7 @@ __global__ __launch_bounds__(128) void bwd_dkdv_kernel(const T* __restrict__ q, 
 
 constexpr size_t kBwdLdsLimit = 160 * 1024;
 // LDS of the dK / dV kernel for nbq query blocks: its stages, then the list of a KV block's query blocks
-size_t bwd_dkdv_lds_bytes(int nbq) { return (size_t)kBwdStages * kBwdStage + (size_t)nbq * sizeof(int32_t); }
+size_t bwd_dkdv_lds_bytes(int nbq, int groups = 1) { return (size_t)groups * kBwdStages * kBwdStage + (size_t)nbq * sizeof(int32_t); }
 static_assert((kBwdLdsLimit - (size_t)kBwdStages * kBwdStage) / sizeof(int32_t) < ((size_t)1 << kBlockBits), "a list entry holds the block");
 int bwd_max_query_blocks() { return (int)((kBwdLdsLimit - (size_t)kBwdStages * kBwdStage) / sizeof(int32_t)); }
 
@@ -1400,12 +1490,12 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     if (dev < 0 || dev >= 64) return hipErrorInvalidDevice;
     int cus = device_cus[dev].load(std::memory_order_acquire);
     if (cus == 0) {
-        const void* kernels[9] = {
-            reinterpret_cast<const void*>(bwd_count_kernel),
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, false>),
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<__bf16, false, true>),
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, false>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, false>),
-            reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, true, true>), reinterpret_cast<const void*>(bwd_dkdv_kernel<_Float16, false, true>)};
+#define BSA_KERNELS(T, G)                                                                                                                   \
+    reinterpret_cast<const void*>(bwd_dkdv_kernel<T, true, false, G>), reinterpret_cast<const void*>(bwd_dkdv_kernel<T, false, false, G>),  \
+    reinterpret_cast<const void*>(bwd_dkdv_kernel<T, true, true, G>), reinterpret_cast<const void*>(bwd_dkdv_kernel<T, false, true, G>)
+        const void* kernels[] = {reinterpret_cast<const void*>(bwd_count_kernel), BSA_KERNELS(__bf16, 1), BSA_KERNELS(__bf16, 2),
+                                 BSA_KERNELS(_Float16, 1), BSA_KERNELS(_Float16, 2)};
+#undef BSA_KERNELS
         for (const void* kf : kernels)
             if ((e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBwdLdsLimit)) != hipSuccess) return e;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
@@ -1473,26 +1563,36 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     const DqSizes dq_sizes = {(int)(Sq / kTile), divisor((int)(Sq / kTile)), divisor(bs_q / kTile), divisor(bs_k / kTile), divisor(round)};
     const DkdvSizes sizes = {(int)(Sk / kTile), nbq, nsub, divisor((int)(Sk / kTile)), divisor(bs_k / kTile), divisor(round)};
     const int total_q = (int)(bh * (Sq / kTile)), total_k = (int)(bh * (Sk / kTile));
-#define BSA_DKDV(T, M, K)                                                                                                              \
-    hipLaunchKernelGGL((bwd_dkdv_kernel<T, M, K>), dim3((unsigned)total_k), dim3(128), lds, st, (const T*)q, (const T*)dout, k_from, v_from,  \
+#define BSA_DKDV(T, M, K, G)                                                                                                           \
+    hipLaunchKernelGGL((bwd_dkdv_kernel<T, M, K, G>), dim3((unsigned)total_k), dim3(128 * G), bwd_dkdv_lds_bytes(nbq, G), st, (const T*)q, (const T*)dout, k_from, v_from,  \
                        m2, delta, bits, tile_valid, (T*)dk, (T*)dv, Sq, Sk, words, c, sm_scale, order, total_k, round,  \
                        dk_to, dv_to, ws + at.ds, ws + at.ds_spare, base, kept.pairs_per_head, sizes, q_live, k_live, counts)
 #define BSA_DQ(T, M)                                                                                                                   \
     hipLaunchKernelGGL((bwd_dq_lds_kernel<T, M>), dim3(end - first), block, kDqRingLds, st, (const T*)q, (const T*)dout, (const T*)ks, (const T*)v,  \
                        m2, delta, paced, lens, tile_valid, (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, dq_to, dq_sizes, q_live.live, k_live)
-#define BSA_DQ_DS(T)                                                                                                                   \
-    hipLaunchKernelGGL((bwd_dq_from_ds_kernel<T>), dim3(end - first), block, 0, st, ks, ws + at.ds, ws + at.ds_zeros, paced, place, lens,  \
+#define BSA_DQ_DS(T, TEAM)                                                                                                             \
+    hipLaunchKernelGGL((bwd_dq_from_ds_kernel<T, TEAM>), dim3(end - first), dim3(64 * TEAM), 0, st, ks, ws + at.ds, ws + at.ds_zeros, paced, place, lens,  \
                        (T*)dq, Sq, Sk, bs_q, bs_k, idx_stride, first, end, round, kept.pairs_per_head, dq_to, dq_sizes, q_live.live, k_live)
 #define BSA_BY_TYPE(F, ...)                                     \
     do {                                                        \
         if (dtype == BSA_BF16) F(__bf16, ##__VA_ARGS__);        \
         else F(_Float16, ##__VA_ARGS__);                        \
     } while (0)
+    // Two pairs of wavefronts to a key tile where there are no more tiles than compute units (a workgroup's stages then fill a unit's LDS) and its
+    // list has blocks to share: us, one pair / two, 252 tiles of 2 heads of 28x8x34 136 / 107, 240 of 13x8x58 75 / 61, 180 of 3
+    // heads of 11x17x16 71 / 53.
+    const bool two_pairs = total_k <= cus && bwd_dkdv_lds_bytes(nbq, 2) <= kBwdLdsLimit && (int64_t)nbq * idx_stride >= 4 * (int64_t)nbk;
+#define BSA_DKDV_OF(K)                                                     \
+    do {                                                                   \
+        if (masked && two_pairs) BSA_BY_TYPE(BSA_DKDV, true, K, 2);        \
+        else if (two_pairs) BSA_BY_TYPE(BSA_DKDV, false, K, 2);            \
+        else if (masked) BSA_BY_TYPE(BSA_DKDV, true, K, 1);                \
+        else BSA_BY_TYPE(BSA_DKDV, false, K, 1);                           \
+    } while (0)
     if (kept.keep) {
         hipLaunchKernelGGL(bwd_place_kernel, dim3((unsigned)((lrows + 3) / 4)), dim3(256), 0, st, paced, lens, bits, base, place, nbq, nbk, idx_stride,
                            words, nsub, lrows, q_live, reinterpret_cast<uint4*>(ws + at.ds_zeros));
-        if (masked) BSA_BY_TYPE(BSA_DKDV, true, true);
-        else BSA_BY_TYPE(BSA_DKDV, false, true);
+        BSA_DKDV_OF(true);
     }
     // One launch for lists that the caller declares unequal, since rounds would wait for their longest list: the whole backward by
     // rounds / at once, us, smooth inputs, from kept dS 8 heads of 12x32x48 at threshold 0.75 (28 to 89 of 288 blocks) 1 027 / 982,
@@ -1504,17 +1604,21 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     // as wide as the blocks may be of any length, and where all are full it makes no difference (24 heads of 12x32x48 13 576 /
     // 13 463, 2 of 24x45x80 27 916 / 27 980).
     const bool once = unequal || (kept.keep ? 2 * idx_stride < nbk : idx_stride >= nbk);
-    const int span = once ? total_q : 2 * round;
+    const int span = once ? total_q : 2 * round, list_tiles = idx_stride * nsub;
+    // As many wavefronts to a list as SIMDs would be left without one, while each has tiles: us, one / four, 252 query tiles of 2
+    // heads of 28x8x34 77 / 52, 240 of 13x8x58 30 / 23, 180 of 3 heads of 11x17x16 29 / 20.
     for (int first = 0; first < total_q; first += span) {
         const int end = first + span < total_q ? first + span : total_q;
-        if (kept.keep) BSA_BY_TYPE(BSA_DQ_DS);
+        if (kept.keep && 4 * total_q <= round && list_tiles >= 8) BSA_BY_TYPE(BSA_DQ_DS, 4);
+        else if (kept.keep && 2 * total_q <= round && list_tiles >= 2) BSA_BY_TYPE(BSA_DQ_DS, 2);
+        else if (kept.keep) BSA_BY_TYPE(BSA_DQ_DS, 1);
         else if (masked) BSA_BY_TYPE(BSA_DQ, true);
         else BSA_BY_TYPE(BSA_DQ, false);
     }
     if (!kept.keep) {
-        if (masked) BSA_BY_TYPE(BSA_DKDV, true, false);
-        else BSA_BY_TYPE(BSA_DKDV, false, false);
+        BSA_DKDV_OF(false);
     }
+#undef BSA_DKDV_OF
 #undef BSA_DKDV
 #undef BSA_DQ
 #undef BSA_DQ_DS

@@ -56,3 +56,35 @@ def test_last_round_in_teams(heads, sparsity, dtype):
     d = (o.float() - want.float()).abs()
     assert d.max() <= 1.6e-2 and d.mean() <= 1e-3, (float(d.max()), float(d.mean()))
     assert not torch.equal(o, want) and torch.allclose(lse, want_lse, atol=2e-3)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent,chunk,width", [
+    ((4, 4, 8), (4, 4, 4), 2),           # two blocks: lists of one entry, and empty ones, are shared
+    ((5, 9, 13), (4, 4, 4), 9),          # ragged: tiles of one half, an odd number of halves
+    ((13, 10, 11), (4, 4, 8), 20),       # blocks of two tiles, tiles without rows
+    ((8, 32, 32), (4, 4, 4), 100),       # 128 tiles, more entries than lanes
+])
+def test_shared_gradient_lists(latent, chunk, width, dtype):
+    """dQ by teams of two and four wavefronts and dK / dV by two pairs of them, against the same heads among so many that every tile
+    has its own: the same P and dS, fp32 sums in two orders.  These differ by some 2^-22 of the sum, so one element in
+    thousands rounds the other way and the 2-norms differ by far less than an eighth of a rounding."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    S = math.prod(latent)
+    blocks = math.prod(-(-n // c) for n, c in zip(latent, chunk))
+    tiles = math.prod(chunk) // 64
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    g = torch.Generator(device="cuda").manual_seed(23)
+    for few in (1, max(1, 250 // (blocks * tiles)), max(1, 500 // (blocks * tiles))):
+        q, k, v, do = (torch.randn(1, few, S, 128, generator=g, device="cuda").to(dtype) for _ in range(4))
+        walk = torch.rand(1, few, blocks, blocks, generator=g, device="cuda").argsort(dim=-1)[..., :width].sort(dim=-1).values.int().contiguous()
+        lens = torch.randint(0, width + 1, (1, few, blocks), generator=g, device="cuda", dtype=torch.int32)
+        o, lse = bi.ThwAttention(k, v, latent, latent, chunk, chunk)(q, walk, lens, return_lse=True)
+        args = (latent, latent, chunk, chunk, 128 ** -0.5)
+        got = bi._bsa_3d_backward(do, q, k, v, o, lse, walk, lens, *args)
+        many = -(-1100 // (few * blocks))
+        rep = [x.repeat(1, many, *([1] * (x.dim() - 2))) for x in (do, q, k, v, o, lse, walk, lens)]
+        for a, w in zip(got, bi._bsa_3d_backward(*rep, *args)):
+            w = w[:, :few].float()
+            assert torch.isfinite(a.float()).all()
+            assert float((a.float() - w).norm()) <= ulp / 8 * float(w.norm())
