@@ -325,12 +325,7 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
             for (int w = 0; w < words; ++w) c += halves_of(q, bits[(head + j) * words + w], w);
         if (j < nbk) counts[head + j] = c;
         if (base == nullptr) continue;
-        int upto = c;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(upto, off);
-            if (lane >= off) upto += t;
-        }
+        int upto = wave_scan(c);
         if (lane == 63) bins[wave] = upto;
         __syncthreads();
         for (int w = 0; w < wave; ++w) upto += bins[w];
@@ -349,13 +344,7 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
         int mine = 0;
         for (int i = 0; i < per; ++i)
             if (top - i >= 0) mine += bins[top - i];
-        int run = mine;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(run, off);
-            if (lane >= off) run += t;
-        }
-        run -= mine;
+        int run = wave_scan(mine) - mine;
         for (int i = 0; i < per; ++i)
             if (top - i >= 0) { const int n = bins[top - i]; bins[top - i] = run; run += n; }
     }
@@ -471,9 +460,7 @@ __device__ __forceinline__ void store_dq(const f32x16 (&acc)[4][2], T* dq, const
         }
 }
 __device__ __forceinline__ int wave_sum(int x) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-    return __builtin_amdgcn_readfirstlane(x);
+    return __builtin_amdgcn_readlane(wave_scan(x), 63);
 }
 template <typename T, bool kMasked>
 __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q, const T* __restrict__ dout,
@@ -1032,12 +1019,7 @@ __global__ __launch_bounds__(128 * kGroups, 1) void bwd_dkdv_kernel(const T* __r
         if (w0 > 0) take_words(w);
         uint32_t word = word_now;
         if (w == words - 1 && (nbq & 31)) word &= (1u << (nbq & 31)) - 1u;
-        int mine = __popc(word), upto = mine;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int t = __shfl_up(upto, off);
-            if (lane >= off) upto += t;
-        }
+        const int mine = __popc(word), upto = wave_scan(mine);
         int pos = count + upto - mine;
         if (wave == 0 && group == 0)
             while (word != 0u) {
@@ -1054,7 +1036,7 @@ __global__ __launch_bounds__(128 * kGroups, 1) void bwd_dkdv_kernel(const T* __r
                 qlist[pos++] = (int32_t)((uint32_t)(32 * w + b) | n << kBlockBits);
                 word &= word - 1u;
             }
-        count += __shfl(upto, 63);
+        count += __builtin_amdgcn_readlane(upto, 63);
     }
     __syncthreads();
     int count_u = __builtin_amdgcn_readfirstlane(count);          // the same in every lane; the compiler cannot tell

@@ -57,6 +57,28 @@ inline Divisor divisor(int d) {
 }
 __device__ __forceinline__ int operator/(int n, const Divisor& d) { return (int)(((uint64_t)(uint32_t)n * d.m) >> d.p); }
 
+// Over a wavefront whose lanes all take part, by DPP moves: a few clocks a step, where a __shfl is a round trip to LDS.  Lanes that
+// a move leaves without a source add 0.
+__device__ __forceinline__ int wave_scan(int x) {                // the sum over lanes 0 .. lane
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);      // row_shr:1, 2, 4, 8: inside rows of 16 lanes
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);      // row_bcast:15 into rows 1 and 3, row_bcast:31 into 2 and 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return x;
+}
+__device__ __forceinline__ uint32_t wave_max(uint32_t x) {       // the same in every lane, a scalar
+    auto step = [&](uint32_t y) { x = x > y ? x : y; };
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false));
+    step((uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false));
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
 // The bytes of a kernel's arguments, laid out one after another, each at its alignment.
 template <typename Kernel>
 struct ArgumentBytes;

@@ -202,8 +202,7 @@ __device__ inline void kth_value(const uint32_t (&val)[N], InRange in_range, int
         uint32_t mx = 0;
 #pragma unroll
         for (int j = 0; j < N; ++j) mx = max(mx, val[j]);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o));
+        mx = wave_max(mx);
         *reinterpret_cast<uint4*>(h + 4 * lane) = make_uint4(0u, 0u, 0u, 0u);
         __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
         __builtin_amdgcn_wave_barrier();
@@ -216,12 +215,7 @@ __device__ inline void kth_value(const uint32_t (&val)[N], InRange in_range, int
         __builtin_amdgcn_wave_barrier();
         const uint4 c = *reinterpret_cast<const uint4*>(h + 4 * lane);
         const int own = (int)(c.x + c.y + c.z + c.w);
-        int upto = own;                                    // columns within bins 0 .. 4 lane + 3
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(upto, o);
-            if (lane >= o) upto += t;
-        }
+        const int upto = wave_scan(own);                   // columns within bins 0 .. 4 lane + 3
         const int before = upto - own;
         const uint64_t holder = __ballot(before < k_sel && k_sel <= upto);
         if (holder != 0) {
@@ -230,9 +224,9 @@ __device__ inline void kth_value(const uint32_t (&val)[N], InRange in_range, int
                 if (run + (int)c.y < k_sel) { run += (int)c.y; ++bin; in_bin = (int)c.z;
                     if (run + (int)c.z < k_sel) { run += (int)c.z; ++bin; in_bin = (int)c.w; } } }
             const int src = __builtin_ctzll(holder);
-            thr = mx - (uint32_t)__shfl(bin, src);
-            cnt_gt = __shfl(run, src);
-            cnt_eq = __shfl(in_bin, src);
+            thr = mx - (uint32_t)__builtin_amdgcn_readlane(bin, src);
+            cnt_gt = __builtin_amdgcn_readlane(run, src);
+            cnt_eq = __builtin_amdgcn_readlane(in_bin, src);
             found = true;
         }
     }
@@ -404,14 +398,9 @@ __global__ __launch_bounds__(256) void topk_blocked_kernel(const uint16_t* __res
             }
             // of the columns equal to t the first need_eq in column order win
             const int n_eq = __popc(eq);
-            int upto = n_eq;
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int t = __shfl_up(upto, o);
-                if (lane >= o) upto += t;
-            }
+            const int upto = wave_scan(n_eq);
             int take = min(max(need_eq - (eq_seen + upto - n_eq), 0), n_eq);
-            eq_seen += __shfl(upto, 63);
+            eq_seen += __builtin_amdgcn_readlane(upto, 63);
             win = gt;
             while (take > 0) {
                 const uint32_t low = eq & (0u - eq);
@@ -421,14 +410,9 @@ __global__ __launch_bounds__(256) void topk_blocked_kernel(const uint16_t* __res
             }
         }
         const int n_win = __popc(win);
-        int upto = n_win;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int t = __shfl_up(upto, o);
-            if (lane >= o) upto += t;
-        }
+        const int upto = wave_scan(n_win);
         int p = pos + upto - n_win;
-        pos += __shfl(upto, 63);
+        pos += __builtin_amdgcn_readlane(upto, 63);
         while (win != 0u) {
             out[p++] = 512 * j + 8 * lane + __builtin_ctz(win);
             win &= win - 1u;
@@ -458,7 +442,8 @@ __device__ __forceinline__ void wave_sync() {
 }
 // A visiting list of n blocks (LDS, visible to the wavefront) as the halves that hold keys, for the attention kernel's
 // kHalves walk: half of the (batch, head) | real keys << 20.  An odd number is made even with a repeat that holds no key.
-__device__ inline void expand_row(const int32_t* list, int n, const HalfLists& h, int64_t row, int lane) {
+// counts: the keys of every tile, in LDS; null: from the validity words.
+__device__ inline void expand_row(const int32_t* list, int n, const HalfLists& h, int64_t row, int lane, const uint8_t* counts = nullptr) {
     int32_t* const out = h.lists + row * h.stride;
     const uint64_t below = ((uint64_t)1 << lane) - 1;
     const int tiles = n * h.nsub;
@@ -469,7 +454,7 @@ __device__ inline void expand_row(const int32_t* list, int n, const HalfLists& h
         if (e < tiles) {
             const int j = h.nsub == 1 ? e : e / h.nsub;
             tile = list[j] * h.nsub + (e - j * h.nsub);
-            keys = __popcll(h.valid[tile]);
+            keys = counts != nullptr ? (int)counts[tile] : __popcll(h.valid[tile]);
         }
         const uint64_t one = __ballot(keys > 0), two = __ballot(keys > 32);
         const int at = total + __popcll(one & below) + __popcll(two & below);
@@ -489,9 +474,13 @@ __device__ inline void expand_row(const int32_t* list, int n, const HalfLists& h
 
 // 32-bit words of LDS that pace_row needs for lists of n entries
 __host__ __device__ inline int pace_words(int n) { return 3 * n + (n + kPaceWidth - 1) / kPaceWidth; }
+// nbk * kPaceWidth, where the products that pace_row divides by it fit 31 bits, otherwise m = 0.
+inline Divisor pace_divisor(int nbk, int stride) {
+    return (int64_t)nbk * (stride > kPaceWidth ? stride : kPaceWidth) <= 0x7fffffff ? divisor(nbk * kPaceWidth) : Divisor{0, 0};
+}
 // work[0 .. n): the ascending list, clamped to the valid range; dst: where its visiting order goes.  Returns the visiting
 // order in LDS.
-__device__ inline const int32_t* pace_row(int32_t* work, int n, int cap, int nbk, int lane, int32_t* __restrict__ dst) {
+__device__ inline const int32_t* pace_row(int32_t* work, int n, int cap, int nbk, int lane, int32_t* __restrict__ dst, const Divisor& by_span) {
     int32_t* const lst = work;                   // [cap] the row, ascending
     int32_t* const slots = lst + cap;            // [cap] block per visit slot, -1 = empty
     int32_t* const spare = slots + cap;          // [cap] blocks over their group's room, ascending
@@ -499,7 +488,10 @@ __device__ inline const int32_t* pace_row(int32_t* work, int n, int cap, int nbk
     const int groups = (n + kPaceWidth - 1) / kPaceWidth;
     // n < 2^13 (the LDS that the callers ask for bounds it) and b < nbk: 32-bit products and quotients
     const uint32_t span = (uint32_t)nbk * kPaceWidth;
-    auto group_of = [&](int32_t b) { return (int)min((uint32_t)b * (uint32_t)n / span, (uint32_t)groups - 1u); };
+    auto group_of = [&](int32_t b) {
+        const uint32_t x = (uint32_t)b * (uint32_t)n;
+        return (int)min(by_span.m != 0u ? (uint32_t)((int)x / by_span) : x / span, (uint32_t)groups - 1u);
+    };
     for (int e = lane; e < n; e += 64) slots[e] = -1;
     for (int g = lane; g < groups; g += 64) first[g] = 0;
     wave_sync();
@@ -545,7 +537,7 @@ __device__ inline const int32_t* pace_row(int32_t* work, int n, int cap, int nbk
     return spare;
 }
 __global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32_t* out, const int32_t* __restrict__ lens, int nbk, int stride, HalfLists halves,
-                                                        ListBits bits) {
+                                                        ListBits bits, Divisor by_span) {
     extern __shared__ int32_t pace_lds[];
     const int lane = threadIdx.x;
     const int64_t row = blockIdx.x;
@@ -568,7 +560,7 @@ __global__ __launch_bounds__(64) void pace_order_kernel(const int32_t* in, int32
     for (int e = lane; e < n; e += 64) pace_lds[e] = min(max(src[e], 0), nbk - 1);
     wave_sync();
     const int32_t* order = pace_lds;
-    if (n > kPaceWidth) order = pace_row(pace_lds, n, stride, nbk, lane, dst);
+    if (n > kPaceWidth) order = pace_row(pace_lds, n, stride, nbk, lane, dst, by_span);
     else if (src != dst)
         for (int e = lane; e < n; e += 64) dst[e] = src[e];
     if (halves.lists != nullptr) expand_row(order, n, halves, row, lane);
@@ -596,7 +588,8 @@ __host__ __device__ inline int gate_wave_words(int k_sel) { const int w = pace_w
 
 template <typename T, int NPL>
 __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict__ qc, const T* __restrict__ kc, int32_t* __restrict__ lists,
-                                                            int32_t* __restrict__ lens, int nbq, int nbk, int k_sel, int paced, HeadNorms norms, HalfLists halves) {
+                                                            int32_t* __restrict__ lens, int nbq, int nbk, int k_sel, int paced, HeadNorms norms, HalfLists halves,
+                                                            int counts_at, Divisor by_span) {
     typedef typename GateRows<T>::bits S;
     constexpr int D = 128, R = GateRows<T>::kRows;
     extern __shared__ __attribute__((aligned(16))) unsigned char gate_lds[];
@@ -604,7 +597,12 @@ __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict_
     T* const scores = reinterpret_cast<T*>(gate_lds);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     uint32_t* const mine = reinterpret_cast<uint32_t*>(gate_lds + (size_t)R * pitch * sizeof(T)) + wave * words;
+    touch_arguments<decltype(gate_kernel<T, NPL>)>();
     const int bh = blockIdx.y, m0 = blockIdx.x * R;
+    // the keys of every tile, which the lists of halves ask for one after another at the end: looked up here, beside the scores
+    uint8_t* const counts = counts_at > 0 ? gate_lds + counts_at : nullptr;
+    if (counts_at > 0)
+        for (int i = threadIdx.x; i < nbk * halves.nsub; i += kGateThreads) counts[i] = (uint8_t)__popcll(halves.valid[i]);
     if (norms.tile_norm != nullptr && wave == kGateThreads / 64 - 1 && blockIdx.x == 0 && blockIdx.z == 0) head_norm(norms, bh, lane);
     const T* qb = qc + (int64_t)bh * nbq * D;
     const T* kb = kc + (int64_t)bh * nbk * D;
@@ -667,10 +665,10 @@ __global__ __launch_bounds__(kGateThreads) void gate_kernel(const T* __restrict_
         wave_sync();
         int32_t* const dst = lists + row * k_sel;
         const int32_t* order = list;
-        if (paced && k_sel > kPaceWidth) order = pace_row(list, k_sel, k_sel, nbk, lane, dst);
+        if (paced && k_sel > kPaceWidth) order = pace_row(list, k_sel, k_sel, nbk, lane, dst, by_span);
         else
             for (int e = lane; e < k_sel; e += 64) dst[e] = list[e];
-        if (halves.lists != nullptr) expand_row(order, k_sel, halves, row, lane);
+        if (halves.lists != nullptr) expand_row(order, k_sel, halves, row, lane, counts);
         wave_sync();
     }
 }
@@ -687,17 +685,24 @@ size_t gate_lds_bytes(int nbk, int k_sel) {
 template <typename T>
 hipError_t launch_gate_t(const T* qc, const T* kc, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel, bool paced,
                          hipStream_t st, HeadNorms norms, HalfLists halves) {
-    const size_t lds = gate_lds_bytes<T>(nbk, k_sel);
+    size_t lds = gate_lds_bytes<T>(nbk, k_sel);
+    const int64_t tiles = (int64_t)nbk * halves.nsub;
+    int counts_at = 0;
+    if (halves.lists != nullptr && tiles <= (int64_t)(kLdsLimit - lds)) {
+        counts_at = (int)lds;
+        lds += (size_t)tiles;
+    }
     const int blocks = (nbq + GateRows<T>::kRows - 1) / GateRows<T>::kRows;
     const int parts = GateRows<T>::kRows > kGateThreads / 64 && blocks * BH <= kGateMaxGroups / 2 ? 2 : 1;
     const dim3 grid(blocks, BH, parts), block(kGateThreads);
+    const Divisor by_span = pace_divisor(nbk, k_sel);
 #define BSA_GATE(N)                                                                                                          \
     do {                                                                                                                     \
         if (lds > 64 * 1024) {                                                                                               \
             const hipError_t ea = hipFuncSetAttribute((const void*)gate_kernel<T, N>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsLimit); \
             if (ea != hipSuccess) return ea;                                                                                 \
         }                                                                                                                    \
-        hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0, norms, halves);  \
+        hipLaunchKernelGGL((gate_kernel<T, N>), grid, block, lds, st, qc, kc, lists, lens, nbq, nbk, k_sel, paced ? 1 : 0, norms, halves, counts_at, by_span);  \
     } while (0)
     if (nbk <= 64) BSA_GATE(1);
     else if (nbk <= 128) BSA_GATE(2);
@@ -899,7 +904,7 @@ hipError_t launch_pace_order(const int32_t* in, int32_t* out, const int32_t* len
     const int groups = (stride + kPaceWidth - 1) / kPaceWidth;
     const size_t lds = ((size_t)3 * stride + groups) * sizeof(int32_t);
     if (lds > 64 * 1024 || rows > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(pace_order_kernel, dim3((unsigned)rows), dim3(64), lds, st, in, out, lens, nbk, stride, halves, bits);
+    hipLaunchKernelGGL(pace_order_kernel, dim3((unsigned)rows), dim3(64), lds, st, in, out, lens, nbk, stride, halves, bits, pace_divisor(nbk, stride));
     return hipGetLastError();
 }
 
