@@ -571,11 +571,12 @@ hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, cons
 hipError_t attention_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, const void* q, const int64_t q_strides[3],
                          const void* k, const int64_t k_strides[3], const void* v, const int64_t v_strides[3], void* o,
                          const int64_t o_strides[3], const int32_t* idx, const int32_t* lens, int idx_stride, float* lse,
-                         hipStream_t st, bool by_length = false, bool fallback_cleared = false, bool halves = false, float* parts = nullptr) {
+                         hipStream_t st, bool by_length = false, bool fallback_cleared = false, bool halves = false, float* parts = nullptr,
+                         const GateCall* gate = nullptr) {
     if (pl.frag)
         return launch_fwd_frag(q, w.kp, w.vp, idx, lens, kv_padded(p) ? w.valid : nullptr, o, lse, p->B, p->Hn, pl.Sqp, pl.Skp,
                                pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype, st, w.qrows, q_strides, o_strides,
-                               (int64_t)p->Tq * p->Hq * p->Wq, &pl.gq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves, parts);
+                               (int64_t)p->Tq * p->Hq * p->Wq, &pl.gq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves, parts, gate);
     FwdLayout L;
     L.q_rows = w.qrows;
     L.k_tiles = w.ktiles;
@@ -689,8 +690,10 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     const int64_t sel_rows = (int64_t)p->B * p->Hn * pl.nbq;
     const HeadNorms norms = {pl.frag ? w.knorm + tile_norm_offset(p->B, p->Hn) : nullptr, w.knorm, (int)(pl.Skp / 64)};
     const HalfLists halves = {w.valid, pl.gk.chunk() / 64, w.halves, w.half_lens, pl.half_width};
+    GateCall gate = {};              // made in front of the attention kernel or by it (launch_fwd_frag)
     if (!pl.cdf && idx_out == nullptr && score_out == nullptr && gate_fits(p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, p->dtype)) {
-        BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st, norms, halves), "gate");
+        gate = {w.qc, w.kc, w.idx_sorted, w.lens, pl.nbq, pl.nbk, p->k_sel, walk_out != nullptr || lens_out != nullptr, norms, halves};
+        if (!pl.frag) BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st, norms, halves), "gate");
     } else {
         BSA_HIP(launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st, norms), "score");
         if (pl.cdf) {
@@ -712,7 +715,8 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         if (pl.cdf && !pl.frag)
             BSA_HIP(launch_order_by_length(walk_lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, walk_width, st), "order by length");
         BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, walk, walk_lens, walk_width,
-                              lse_out, st, pl.cdf, pl.frag, by_half, pl.cdf ? nullptr : w.parts), "attention");
+                              lse_out, st, pl.cdf, pl.frag, by_half, pl.cdf ? nullptr : w.parts, pl.frag && gate.q_cmp != nullptr ? &gate : nullptr),
+                "gate and attention");
     } else {
         F32Layout L;
         L.q_rows = w.qrows; L.k_rows = w.krows;

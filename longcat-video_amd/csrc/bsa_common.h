@@ -217,6 +217,15 @@ struct HalfLists {
 // visiting order, lens = k_sel.  The same lists as launch_score, launch_topk and launch_pace_order; gate_fits says for
 // which sizes it is built and the better choice.
 bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype);
+// What launch_gate takes, for launch_fwd_frag, which runs it or lets the attention kernel select for itself.
+struct GateCall {
+    const void *q_cmp, *k_cmp;
+    int32_t *lists, *lens;           // lists [BH][nbq][k_sel]
+    int nbq, nbk, k_sel;
+    bool wanted;                     // lists and lens are read behind the attention
+    HeadNorms norms;
+    HalfLists halves;
+};
 hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
                        bool paced, int dtype, hipStream_t st, HeadNorms norms = {nullptr, nullptr, 0}, HalfLists halves = {});
 // lens[row] = number of columns the CDF rule keeps, clamped to [k_min, cap]
@@ -306,7 +315,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const Grid3* q_grid = nullptr, int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
-                           int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false, float* part_buf = nullptr);
+                           int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false, float* part_buf = nullptr,
+                           const GateCall* gate_call = nullptr);
 // order (B * Hn * Sq / 64 int32) and queue (kFragQueueWords), both or none: scratch for the schedule of lists of unequal length,
 // enqueued besides the rounds; which of the two runs is decided on the device.
 constexpr int kFragQueueWords = 16;
@@ -317,6 +327,7 @@ constexpr int kFragQueueWords = 16;
 // part_buf (optional, frag_part_floats() floats): the last, partial round may be cut into parts, merged at the end.
 size_t frag_part_floats(const Grid3& q_grid, int64_t heads);
 // halves: idx and lens are HalfLists, idx_stride their row pitch (at most 4 096).
+// gate_call (optional): idx and lens are still to be made.
 size_t frag_fallback_ints(int64_t items);
 
 

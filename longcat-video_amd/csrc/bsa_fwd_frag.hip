@@ -33,6 +33,7 @@
 // bf16 a form that takes no maxima where the norms bound the logits (kBounded); numerics
 // follow flash_attn_bsa_varlen_mask.py:242-285: fp32 logits, scale * log2(e) applied after the
 // dot, exp2, P rounded to the storage type for the P V product, fp32 row sum, one final rounding.
+#include "bsa_gate.h"
 #include "bsa_mfma.h"
 
 #include <type_traits>
@@ -136,7 +137,24 @@ template <int kTeam>
 constexpr int kTeamBytes = kTeam * (kTile * kD + 2 * kTile) * 4;      // the sums, maxima and row sums of every wavefront
 static_assert(kTeamBytes<4> <= 160 * 1024 && 2 * (kTeamBytes<2> + 512) <= 160 * 1024, "LDS of a compute unit with four wavefronts");
 
-template <typename T, int kWalk, bool kBounded, int kTeam>
+// kGate: the item's list does not exist yet.  The workgroup makes it from the chunk means, as gate_kernel does (the same products and
+// roundings, the same lists), in front of its walk: the scores of its block against every key block, a share of 32 of them to a
+// wavefront at a time, then the first wavefront selects and orders.  Instead of another launch, its start and its end.
+// Whole operator, us, with gate_kernel in front / like this: 2 heads of 16x22x12 23.0 / 19.9, 4 of 9x13x10 30.2 / 26.3, two prompts of
+// 13 heads of 7x8x8 24.2 / 21.6, of 8 heads of 7x15x26 40.3 / 38.2.
+struct FragGate {
+    const uint16_t *qc, *kc;         // chunk means, 16-bit storage
+    int nbk, k_sel;
+    Divisor by_span;
+};
+constexpr int kGateWaveBlocks = 128, kGateMostBlocks = 256;      // key blocks to a wavefront, to a workgroup
+// LDS of the selection: the list of halves; scores; keys of every tile; where the first wavefront works; the list's length
+__host__ __device__ inline int gate_list_words(int k_sel, int nsub, bool halves) { return halves ? (2 * k_sel * nsub + 3) / 4 * 4 : 0; }
+__host__ __device__ inline int gate_here_bytes(int nbk, int k_sel, int nsub, bool halves) {
+    return (gate_list_words(k_sel, nsub, halves) + gate_wave_words(k_sel) + 4) * 4 + (nbk + 31) / 32 * 64 + (halves ? (nbk * nsub + 15) / 16 * 16 : 0);
+}
+
+template <typename T, int kWalk, bool kBounded, int kTeam, bool kGate>
 __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
     const int32_t* __restrict__ idx, const int32_t* __restrict__ lens, const uint64_t* __restrict__ tile_valid,
@@ -144,9 +162,10 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
     float qk_scale, int item_begin, int item_end, int round, int Hn, int64_t lse_S, FragLayout L,
     const int32_t* __restrict__ order, uint32_t* __restrict__ queue, const uint32_t* __restrict__ gate, uint32_t gate_want,
     int bh_first, uint32_t kv_span_bytes, int q_offsets_32, const float* __restrict__ key_norm,
-    int32_t* __restrict__ fallback, uint32_t* __restrict__ fallback_count, Parts parts) {
+    int32_t* __restrict__ fallback, uint32_t* __restrict__ fallback_count, Parts parts, FragGate G) {
     typedef typename Vec8<T>::type V8;
     constexpr bool kOnce = kTeam > 0;
+    static_assert(!kGate || kOnce, "a workgroup that selects has one item");
     // log2 headroom before the running maximum is raised: probabilities reach 2^kTau, which the storage type of P
     // must hold (fp16 ends at 65 504) and the fp32 sums must hold times the number of keys
     constexpr float kTau = std::is_same<T, _Float16>::value ? 14.0f : 30.0f;
@@ -165,7 +184,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
     // 7x15x26, takes 41.4 us for 41.9.  With what an item that nothing has prepared asks for at once (below) and the divisions
     // that went, the kernel of a single round is 1.3 us shorter: 15.1 -> 13.8 us for 5 heads of 9x27x12, 25.4 -> 24.2 for two
     // prompts of 8 heads of 7x15x26.
-    touch_arguments<decltype(fwd_frag_kernel<T, kWalk, kBounded, kTeam>)>();
+    touch_arguments<decltype(fwd_frag_kernel<T, kWalk, kBounded, kTeam, kGate>)>();
     if (gate != nullptr && *gate != gate_want) return;
     // output staging: 64 rows of 256 B, 272 B apart.  The same memory stages a list that is too long for the small
     // buffers (kListEntries words at most) during the tile loop of an item that was not prepared ahead of time.
@@ -184,7 +203,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
     const int wave = kTeam > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
     const int lr = lane & 31, lh = lane >> 5;
     const int nqt = (int)(Sq / kTile);
-    const int nsub = kWalk == kBlocks ? bs_k / kTile : 1;
+    const int nsub = kWalk == kBlocks ? bs_k / kTile : 1, nsub_of_block = bs_k / kTile;
     const int tiles_bh = (int)(Sk / kTile), nbk = kWalk == kBlocks ? tiles_bh / L.by_sub : tiles_bh;     // kHalves does not ask for it
     const uint32_t lane_off = (uint32_t)lane * 16u;
     // the kernel that runs the fallback list takes as many items as the list holds
@@ -241,6 +260,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         if (local < 0) return d;
         if (!kBounded && kTeam != 1 && parts.count > 1) local -= local / parts.by_items * parts.items;
         d.item = order != nullptr ? item_begin + order[local] : item_at(L, item_begin + local, nqt);
+        if (kGate) return d;
         const int64_t row = d.item / L.by_block;
         d.nent = lens[row];
         if (idx_stride > 0) {
@@ -572,9 +592,9 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         }
         // ... and so is a team's list, as far as one entry a thread goes (what lies behind its end is not used)
         int32_t team_entry = 0;
-        if (kOnce && idx_stride > 0) team_entry = idx[(int64_t)(cur.item / L.by_block) * idx_stride + min((int)threadIdx.x, idx_stride - 1)];
+        if (kOnce && !kGate && idx_stride > 0) team_entry = idx[(int64_t)(cur.item / L.by_block) * idx_stride + min((int)threadIdx.x, idx_stride - 1)];
         __builtin_amdgcn_sched_barrier(0);
-        const int nent = list_length(cur);
+        int nent = list_length(cur);
         npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
         if (!kOnce && !kBounded && parts.count > 1) {
             const int part = cur.local / parts.by_items;        // at most kMaxParts: the products fit 32 bits
@@ -598,7 +618,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         const int64_t nqrow0 = (int64_t)(nitem - nbh * nqt) * kTile;
         const int32_t* nlist = idx + (int64_t)(nitem / L.by_block) * idx_stride;
 
-        const bool early = kTeam == 1 || (!kOnce && (kBounded || parts.count == 1));         // the walk starts at the list's first entry
+        const bool early = (kTeam == 1 && !kGate) || (!kOnce && (kBounded || parts.count == 1));         // the walk starts at the list's first entry
         auto first_fragments = [&](uint32_t h0, uint32_t h1) {
 #pragma unroll
             for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(h0, c);                       // K(0)
@@ -644,14 +664,86 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 for (int e = 0; e < kAhead; ++e)
                     if (lane_now + 64 * e < nent) big[lane_now + 64 * e] = (uint32_t)entry[e];
                 for (int e = lane_now + 64 * kAhead; e < nent; e += 64) big[e] = (uint32_t)list[e];
+            } else if constexpr (kGate) {
+                char* const work = ost_bytes;
+                const int words = gate_list_words(G.k_sel, nsub_of_block, kWalk == kHalves);
+                int32_t* const halves_list = reinterpret_cast<int32_t*>(work);
+                uint32_t* const mine = reinterpret_cast<uint32_t*>(work) + words;
+                int* const total_at = reinterpret_cast<int*>(mine + gate_wave_words(G.k_sel));
+                T* const scores = reinterpret_cast<T*>(total_at + 4);
+                uint8_t* const counts = reinterpret_cast<uint8_t*>(scores + (G.nbk + 31) / 32 * 32);
+                const int64_t brow = cur.item / L.by_block;
+                if (kWalk == kHalves)
+                    for (int i = threadIdx.x; i < G.nbk * nsub_of_block; i += 64 * kTeam) counts[i] = (uint8_t)__popcll(tile_valid[i]);
+                const T* const qm = reinterpret_cast<const T*>(G.qc) + brow * kD + lh * 8;      // its mean as every row of the product
+                const T* const km = reinterpret_cast<const T*>(G.kc) + (int64_t)bh * G.nbk * kD + lh * 8;
+                V8 qa[8], kr[4][8];
+#pragma unroll
+                for (int c = 0; c < 8; ++c) qa[c] = *reinterpret_cast<const V8*>(qm + 16 * c);
+                constexpr int kTurns = kTeam == 1 ? kGateWaveBlocks / 32 : kGateMostBlocks / 32 / kTeam;
+#pragma unroll
+                for (int t = 0; t < kTurns; ++t) {
+                    const int n0 = 32 * (wave + kTeam * t);
+                    if (n0 < G.nbk) {
+                        const T* const kt = km + (int64_t)min(n0 + lr, G.nbk - 1) * kD;
+#pragma unroll
+                        for (int c = 0; c < 8; ++c) kr[t][c] = *reinterpret_cast<const V8*>(kt + 16 * c);
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < kTurns; ++t) {
+                    const int n0 = 32 * (wave + kTeam * t);
+                    if (n0 < G.nbk) {
+                        f32x16 acc;
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+#pragma unroll
+                        for (int c = 0; c < 8; ++c) acc = mfma32(qa[c], kr[t][c], acc);
+                        if (lh == 0) scores[n0 + lr] = (T)acc[0];
+                    }
+                }
+                __syncthreads();
+                if (wave == 0) {
+                    constexpr int kPerLane = kTeam == 1 ? kGateWaveBlocks / 64 : kGateMostBlocks / 64;
+                    uint32_t val[kPerLane];
+                    const uint16_t* const raw = reinterpret_cast<const uint16_t*>(scores);
+#pragma unroll
+                    for (int j = 0; j < kPerLane; ++j) {
+                        const int i = j * 64 + lane;
+                        const uint16_t x = raw[min(i, G.nbk - 1)];
+                        val[j] = i < G.nbk ? ord_of(x) : 0u;
+                    }
+                    int32_t* const list = reinterpret_cast<int32_t*>(mine);
+                    select_row<uint16_t, kPerLane, false>(val, [&](int i) { return raw[i]; }, lane, G.nbk, G.k_sel, nullptr, list, nullptr, mine);
+                    wave_sync();
+                    int32_t* const dst = idx != nullptr ? const_cast<int32_t*>(idx) + brow * G.k_sel : nullptr;
+                    const int32_t* order_here = list;
+                    if (G.k_sel > kPaceWidth) order_here = pace_row(list, G.k_sel, G.k_sel, G.nbk, lane, dst, G.by_span);
+                    else if (dst != nullptr)
+                        for (int e = lane; e < G.k_sel; e += 64) dst[e] = list[e];
+                    if (lens != nullptr && lane == 0) const_cast<int32_t*>(lens)[brow] = G.k_sel;
+                    int total = G.k_sel;
+                    if constexpr (kWalk == kHalves) total = expand_list(order_here, G.k_sel, nsub_of_block, halves_list, lane, [&](int tile) { return (int)counts[tile]; });
+                    if (lane == 0) {
+                        total_at[0] = total;
+                        total_at[1] = (int)(order_here - list);
+                    }
+                }
+                __syncthreads();
+                cur.nent = total_at[0];
+                nent = list_length(cur);
+                ents = kWalk == kHalves ? reinterpret_cast<const uint32_t*>(halves_list) : mine + uni(total_at[1]);
+                if (kTeam == 1) npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
             } else {
                 if ((int)threadIdx.x < nent) big[threadIdx.x] = (uint32_t)team_entry;
                 for (int e = threadIdx.x + 64 * kTeam; e < nent; e += 64 * kTeam) big[e] = (uint32_t)list[e];
             }
             take_q(0, rows[0]);
             take_q(1, rows[1]);
-            ents = big;
-            __syncthreads();
+            if constexpr (!kGate) {
+                ents = big;
+                __syncthreads();
+            }
             if constexpr (kTeam > 1) {
                 // This wavefront's share of the list, whole KV blocks of it, so that a walk over halves and one over tiles that masks
                 // the empty halves cut at the same keys (and give the same bits).
@@ -1286,7 +1378,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const Grid3* q_grid, int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
-                           bool halves, float* part_buf) {
+                           bool halves, float* part_buf, const GateCall* gate_call) {
     // the C-ABI layer keeps lists within these limits (a list that is too long for the small buffers is staged in `ost`)
     if (idx_stride > (halves ? kHalfEntries : kListEntries)) return hipErrorInvalidValue;
     const float qk_scale = sm_scale * kLog2e;
@@ -1330,25 +1422,31 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                          (int64_t)total * list_tiles > (int64_t)kExactRoundTiles * resident;
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
-#define BSA_FRAG_LAUNCH_T(T, WALK, BD, TEAM, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
-    hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD, TEAM>), grid, dim3(TEAM > 1 ? 64 * TEAM : 64), 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
+    FragGate here = {nullptr, nullptr, 0, 0, {0, 0}};
+#define BSA_FRAG_LAUNCH_T(T, WALK, BD, TEAM, GATE, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
+    hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD, TEAM, GATE>), grid, dim3(TEAM > 1 ? 64 * TEAM : 64), 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
                        lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, TEAM > 0 ? kOneRound : resident, Hn, lse_rows, \
-                       L, ord, que, gate, want, bh0, span, q_offsets_32, key_norm, fbl, fbc, parts)
-#define BSA_FRAG_LAUNCH_W(T, BD, TEAM, ...)                                                                            \
+                       L, ord, que, gate, want, bh0, span, q_offsets_32, key_norm, fbl, fbc, parts, here)
+#define BSA_FRAG_LAUNCH_W(T, BD, TEAM, GATE, ...)                                                                      \
     do {                                                                                                               \
-        if (halves) BSA_FRAG_LAUNCH_T(T, kHalves, BD, TEAM, __VA_ARGS__);                                              \
-        else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(T, kTiles, BD, TEAM, __VA_ARGS__);                                   \
-        else BSA_FRAG_LAUNCH_T(T, kBlocks, BD, TEAM, __VA_ARGS__);                                                     \
+        if (halves) BSA_FRAG_LAUNCH_T(T, kHalves, BD, TEAM, GATE, __VA_ARGS__);                                        \
+        else if (bs_k == kTile) BSA_FRAG_LAUNCH_T(T, kTiles, BD, TEAM, GATE, __VA_ARGS__);                             \
+        else BSA_FRAG_LAUNCH_T(T, kBlocks, BD, TEAM, GATE, __VA_ARGS__);                                               \
     } while (0)
 #define BSA_FRAG_LAUNCH(BD, ...)                                                                                       \
     do {                                                                                                               \
-        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, BD, 0, __VA_ARGS__);                                          \
-        else BSA_FRAG_LAUNCH_W(_Float16, false, 0, __VA_ARGS__);                                                       \
+        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, BD, 0, false, __VA_ARGS__);                                   \
+        else BSA_FRAG_LAUNCH_W(_Float16, false, 0, false, __VA_ARGS__);                                                \
     } while (0)
 #define BSA_FRAG_LAUNCH_ONCE(TEAM, ...)                                                                                \
     do {                                                                                                               \
-        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, __VA_ARGS__);                                    \
-        else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, __VA_ARGS__);                                                    \
+        if (here.qc != nullptr) {                                                                                      \
+            if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, true, __VA_ARGS__);                          \
+            else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, true, __VA_ARGS__);                                          \
+        } else {                                                                                                       \
+            if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, false, __VA_ARGS__);                         \
+            else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, false, __VA_ARGS__);                                         \
+        }                                                                                                              \
     } while (0)
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
     // Lists of unequal length of one round need no plan: every item has a wavefront of its own from the start.
@@ -1372,6 +1470,21 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     if (one_span && tail > 0 && (part_buf != nullptr || total < resident))
         split = choose_split(tail, list_tiles, resident, total > resident, part_buf != nullptr);
     const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
+    // The lists of a call of one round are made by the workgroups that walk them, where that is little work.
+    if (gate_call != nullptr) {
+        const GateCall& c = *gate_call;
+        const int nsub = bs_k / kTile;
+        if (once && split.parts == 1 && c.k_sel > 0 && c.nbk <= (split.team == 1 ? kGateWaveBlocks : kGateMostBlocks) &&
+            gate_here_bytes(c.nbk, c.k_sel, nsub, halves) <= kTile * (kD + 8) * 2) {
+            here = {static_cast<const uint16_t*>(c.q_cmp), static_cast<const uint16_t*>(c.k_cmp), c.nbk, c.k_sel, pace_divisor(c.nbk, c.k_sel)};
+            idx = c.wanted ? c.lists : nullptr;
+            lens = c.wanted ? c.lens : nullptr;
+            if (halves) tile_valid = c.halves.valid;
+        } else {
+            const hipError_t e = launch_gate(c.q_cmp, c.k_cmp, c.lists, c.lens, B * Hn, c.nbq, c.nbk, c.k_sel, true, dtype, st, c.norms, c.halves);
+            if (e != hipSuccess) return e;
+        }
+    }
     const int whole = once ? 0 : split.team * split.parts > 1 ? total - tail : total;
     for (int first = 0; first < whole;) {
         int end = first + span < whole ? first + span : whole;

@@ -1,0 +1,41 @@
+"""Calls of one round, whose workgroups make the lists that they walk, against the kernels that make them by themselves."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent,chunk,heads,sparsity", [
+    ((4, 4, 4), (4, 4, 4), 1, 0.0),             # one block
+    ((4, 32, 32), (4, 4, 4), 2, 0.9),           # 64 blocks, a team of four, 6 kept: no visiting order
+    ((4, 32, 32), (4, 4, 4), 8, 0.8),           # ... 512 items, teams of two
+    ((4, 32, 32), (4, 4, 4), 9, 0.8),           # ... 576, one wavefront an item
+    ((4, 20, 52), (4, 4, 4), 3, 0.5),           # 65 blocks
+    ((8, 32, 32), (4, 4, 4), 8, 0.75),          # 128 blocks, one wavefront an item, the most it scores
+    ((4, 12, 172), (4, 4, 4), 7, 0.75),         # 129: 903 items, the kernel in front
+    ((16, 32, 32), (4, 4, 4), 1, 0.3),          # 256 blocks: the most a team scores; 179 kept
+    ((4, 4, 1028), (4, 4, 4), 1, 0.9),          # 257: the kernel in front
+    ((5, 9, 13), (4, 4, 4), 2, 0.5),            # ragged: halves
+    ((5, 33, 30), (4, 4, 4), 7, 0.7),           # ... 144 blocks, 1 008 items
+    ((13, 10, 11), (4, 4, 8), 3, 0.4),          # blocks of two tiles, tiles of padding alone
+    ((8, 16, 32), (4, 8, 8), 2, 0.5),           # blocks of four tiles without padding
+])
+def test_lists_made_by_the_attention_kernel(latent, chunk, heads, sparsity, dtype):
+    """The lists that a backward would be given are those of score, top-k and visiting order one after another, with equal scores
+    among them (repeated key chunks: ties go to the lowest block), and the output is theirs bit for bit, with and without lists."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    S, blocks = math.prod(latent), math.prod(-(-n // c) for n, c in zip(latent, chunk))
+    g = torch.Generator(device="cuda").manual_seed(31)
+    for ties in (False, True):
+        q, k, v = (torch.randn(2, heads, S, 128, generator=g, device="cuda").to(dtype)[:1] for _ in range(3))
+        if ties:
+            k[:, :, S // 2:] = k[:, :, :1]
+        o, walk, lens, lse = bi._bsa_3d(q, k, v, latent, latent, sparsity, chunk, chunk, for_backward=True)
+        want_o, idx, want_lens, _ = bi._bsa_3d(q, k, v, latent, latent, sparsity, chunk, chunk, want_selection=True)
+        ascending = idx.sort(dim=-1).values.int().contiguous()
+        assert torch.equal(lens, want_lens) and torch.equal(walk, bi.visit_order(ascending, lens, blocks))
+        assert torch.isfinite(o.float()).all() and torch.equal(o, want_o)
+        assert torch.equal(bi.flash_attn_bsa_3d(q, k, v, latent, latent, sparsity=sparsity, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk), o)
