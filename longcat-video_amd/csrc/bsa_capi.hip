@@ -690,22 +690,27 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     const int64_t sel_rows = (int64_t)p->B * p->Hn * pl.nbq;
     const HeadNorms norms = {pl.frag ? w.knorm + tile_norm_offset(p->B, p->Hn) : nullptr, w.knorm, (int)(pl.Skp / 64)};
     const HalfLists halves = {w.valid, pl.gk.chunk() / 64, w.halves, w.half_lens, pl.half_width};
-    GateCall gate = {};              // made in front of the attention kernel or by it (launch_fwd_frag)
-    if (!pl.cdf && idx_out == nullptr && score_out == nullptr && gate_fits(p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, p->dtype)) {
-        gate = {w.qc, w.kc, w.idx_sorted, w.lens, pl.nbq, pl.nbk, p->k_sel, walk_out != nullptr || lens_out != nullptr, norms, halves};
-        if (!pl.frag) BSA_HIP(launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st, norms, halves), "gate");
-    } else {
-        BSA_HIP(launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st, norms), "score");
-        if (pl.cdf) {
-            BSA_HIP(launch_cdf_count(w.score, w.lens, sel_rows, pl.nbk, p->cdf_threshold, p->sm_scale, p->k_sel < pl.sel_width ? p->k_sel : pl.sel_width,
-                                     pl.sel_width, p->dtype, st), "cdf count");
-            BSA_HIP(launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, 0, p->dtype, st, w.lens, pl.sel_width), "top-k");
-        } else {
-            BSA_HIP(launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, p->k_sel, p->dtype, st), "top-k");
-        }
-        if (pl.frag && pl.sel_width > 0)
-            BSA_HIP(launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st, halves), "visit order");
-    }
+    const int k_min = p->k_sel < pl.sel_width ? p->k_sel : pl.sel_width;
+    auto select = [&]() -> hipError_t {
+        if (!pl.cdf && idx_out == nullptr && score_out == nullptr && gate_fits(p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, p->dtype))
+            return launch_gate(w.qc, w.kc, w.idx_sorted, w.lens, p->B * p->Hn, pl.nbq, pl.nbk, p->k_sel, pl.frag, p->dtype, st, norms, halves);
+        hipError_t r = launch_score(w.qc, w.kc, w.score, p->B * p->Hn, pl.nbq, pl.nbk, p->D, p->dtype, st, norms);
+        if (r == hipSuccess && pl.cdf)
+            r = launch_cdf_count(w.score, w.lens, sel_rows, pl.nbk, p->cdf_threshold, p->sm_scale, k_min, pl.sel_width, p->dtype, st);
+        if (r == hipSuccess)
+            r = pl.cdf ? launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, 0, p->dtype, st, w.lens, pl.sel_width)
+                       : launch_topk(w.score, idx_out ? w.idx : nullptr, w.idx_sorted, w.lens, sel_rows, pl.nbk, p->k_sel, p->dtype, st);
+        if (r == hipSuccess && pl.frag && pl.sel_width > 0)
+            r = launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st, halves);
+        return r;
+    };
+    // made in front of the attention kernel, or by it where the caller asks for nothing but what it walks (launch_fwd_frag)
+    const bool by_attention = pl.frag && idx_out == nullptr && score_out == nullptr && pl.sel_width > 0;
+    const bool lists_wanted = walk_out != nullptr || lens_out != nullptr;
+    const GateCall gate = {w.qc, w.kc, lists_wanted ? w.idx_sorted : nullptr, lists_wanted ? w.lens : nullptr, w.valid, pl.nbk, pl.sel_width,
+                           pl.cdf ? p->cdf_threshold : 0.f, p->sm_scale, k_min,
+                           [](void* ctx) { return (*static_cast<decltype(select)*>(ctx))(); }, &select};
+    if (!by_attention) BSA_HIP(select(), "selection");
     if (!pl.f32) {
         // lists of unequal length: a launch whose workgroups draw the items besides the rounds, for the LDS-tiled kernel longest list first
         // (the fragment-order kernel's own plan kernel fills a queue per XCD)
@@ -715,8 +720,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         if (pl.cdf && !pl.frag)
             BSA_HIP(launch_order_by_length(walk_lens, w.order, p->B * p->Hn, pl.nbq, pl.gq.chunk() / 64, walk_width, st), "order by length");
         BSA_HIP(attention_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, o, o_strides, walk, walk_lens, walk_width,
-                              lse_out, st, pl.cdf, pl.frag, by_half, pl.cdf ? nullptr : w.parts, pl.frag && gate.q_cmp != nullptr ? &gate : nullptr),
-                "gate and attention");
+                              lse_out, st, pl.cdf, pl.frag, by_half, pl.cdf ? nullptr : w.parts, by_attention ? &gate : nullptr), by_attention ? "selection and attention" : "attention");
     } else {
         F32Layout L;
         L.q_rows = w.qrows; L.k_rows = w.krows;

@@ -217,14 +217,16 @@ struct HalfLists {
 // visiting order, lens = k_sel.  The same lists as launch_score, launch_topk and launch_pace_order; gate_fits says for
 // which sizes it is built and the better choice.
 bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype);
-// What launch_gate takes, for launch_fwd_frag, which runs it or lets the attention kernel select for itself.
+// A selection that launch_fwd_frag lets the attention kernel make, or has made in front of it by make(ctx).
 struct GateCall {
-    const void *q_cmp, *k_cmp;
-    int32_t *lists, *lens;           // lists [BH][nbq][k_sel]
-    int nbq, nbk, k_sel;
-    bool wanted;                     // lists and lens are read behind the attention
-    HeadNorms norms;
-    HalfLists halves;
+    const void *q_cmp, *k_cmp;       // chunk means
+    int32_t *lists, *lens;           // where the lists go ([BH][nbq][width]), null: they are not read behind the attention
+    const uint64_t* valid;           // validity words of the key tiles
+    int nbk, width;                  // width: the top-k rule's count, the most of the CDF rule's
+    float threshold, scale;          // CDF rule (launch_cdf_count), threshold 0: top-k
+    int k_min;
+    hipError_t (*make)(void* ctx);
+    void* ctx;
 };
 hipError_t launch_gate(const void* q_cmp, const void* k_cmp, int32_t* lists, int32_t* lens, int BH, int nbq, int nbk, int k_sel,
                        bool paced, int dtype, hipStream_t st, HeadNorms norms = {nullptr, nullptr, 0}, HalfLists halves = {});

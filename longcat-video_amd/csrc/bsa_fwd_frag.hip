@@ -144,14 +144,16 @@ static_assert(kTeamBytes<4> <= 160 * 1024 && 2 * (kTeamBytes<2> + 512) <= 160 * 
 // 13 heads of 7x8x8 24.2 / 21.6, of 8 heads of 7x15x26 40.3 / 38.2.
 struct FragGate {
     const uint16_t *qc, *kc;         // chunk means, 16-bit storage
-    int nbk, k_sel;
+    int nbk, width;                  // entries of a list: the top-k rule's count, the most of the CDF rule's
+    float threshold, scale;          // of the CDF rule, as cdf_count_kernel's; threshold 0: top-k
+    int k_min;
     Divisor by_span;
 };
 constexpr int kGateWaveBlocks = 128, kGateMostBlocks = 256;      // key blocks to a wavefront, to a workgroup
 // LDS of the selection: the list of halves; scores; keys of every tile; where the first wavefront works; the list's length
-__host__ __device__ inline int gate_list_words(int k_sel, int nsub, bool halves) { return halves ? (2 * k_sel * nsub + 3) / 4 * 4 : 0; }
-__host__ __device__ inline int gate_here_bytes(int nbk, int k_sel, int nsub, bool halves) {
-    return (gate_list_words(k_sel, nsub, halves) + gate_wave_words(k_sel) + 4) * 4 + (nbk + 31) / 32 * 64 + (halves ? (nbk * nsub + 15) / 16 * 16 : 0);
+__host__ __device__ inline int gate_list_words(int width, int nsub, bool halves) { return halves ? (2 * width * nsub + 3) / 4 * 4 : 0; }
+__host__ __device__ inline int gate_here_bytes(int nbk, int width, int nsub, bool halves) {
+    return (gate_list_words(width, nsub, halves) + gate_wave_words(width) + 4) * 4 + (nbk + 31) / 32 * 64 + (halves ? (nbk * nsub + 15) / 16 * 16 : 0);
 }
 
 template <typename T, int kWalk, bool kBounded, int kTeam, bool kGate>
@@ -666,10 +668,10 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 for (int e = lane_now + 64 * kAhead; e < nent; e += 64) big[e] = (uint32_t)list[e];
             } else if constexpr (kGate) {
                 char* const work = ost_bytes;
-                const int words = gate_list_words(G.k_sel, nsub_of_block, kWalk == kHalves);
+                const int words = gate_list_words(G.width, nsub_of_block, kWalk == kHalves);
                 int32_t* const halves_list = reinterpret_cast<int32_t*>(work);
                 uint32_t* const mine = reinterpret_cast<uint32_t*>(work) + words;
-                int* const total_at = reinterpret_cast<int*>(mine + gate_wave_words(G.k_sel));
+                int* const total_at = reinterpret_cast<int*>(mine + gate_wave_words(G.width));
                 T* const scores = reinterpret_cast<T*>(total_at + 4);
                 uint8_t* const counts = reinterpret_cast<uint8_t*>(scores + (G.nbk + 31) / 32 * 32);
                 const int64_t brow = cur.item / L.by_block;
@@ -714,16 +716,25 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                         val[j] = i < G.nbk ? ord_of(x) : 0u;
                     }
                     int32_t* const list = reinterpret_cast<int32_t*>(mine);
-                    select_row<uint16_t, kPerLane, false>(val, [&](int i) { return raw[i]; }, lane, G.nbk, G.k_sel, nullptr, list, nullptr, mine);
+                    int k_sel = G.width;
+                    if (G.threshold > 0.f) {
+                        float e[kPerLane];
+#pragma unroll
+                        for (int j = 0; j < kPerLane; ++j) e[j] = j * 64 + lane < G.nbk ? (float)scores[min(j * 64 + lane, G.nbk - 1)] : -INFINITY;
+                        k_sel = cdf_row<16>(val, e, lane, G.nbk, G.threshold, G.scale, G.k_min, G.width);
+                    }
+                    int32_t* const dst = idx != nullptr ? const_cast<int32_t*>(idx) + brow * G.width : nullptr;
+                    if (k_sel > 0) select_row<uint16_t, kPerLane, false>(val, [&](int i) { return raw[i]; }, lane, G.nbk, k_sel, nullptr, list, nullptr, mine);
                     wave_sync();
-                    int32_t* const dst = idx != nullptr ? const_cast<int32_t*>(idx) + brow * G.k_sel : nullptr;
                     const int32_t* order_here = list;
-                    if (G.k_sel > kPaceWidth) order_here = pace_row(list, G.k_sel, G.k_sel, G.nbk, lane, dst, G.by_span);
+                    if (k_sel > kPaceWidth) order_here = pace_row(list, k_sel, k_sel, G.nbk, lane, dst, G.by_span);
                     else if (dst != nullptr)
-                        for (int e = lane; e < G.k_sel; e += 64) dst[e] = list[e];
-                    if (lens != nullptr && lane == 0) const_cast<int32_t*>(lens)[brow] = G.k_sel;
-                    int total = G.k_sel;
-                    if constexpr (kWalk == kHalves) total = expand_list(order_here, G.k_sel, nsub_of_block, halves_list, lane, [&](int tile) { return (int)counts[tile]; });
+                        for (int e = lane; e < k_sel; e += 64) dst[e] = list[e];
+                    if (dst != nullptr)
+                        for (int e = k_sel + lane; e < G.width; e += 64) dst[e] = -1;
+                    if (lens != nullptr && lane == 0) const_cast<int32_t*>(lens)[brow] = k_sel;
+                    int total = k_sel;
+                    if constexpr (kWalk == kHalves) total = expand_list(order_here, k_sel, nsub_of_block, halves_list, lane, [&](int tile) { return (int)counts[tile]; });
                     if (lane == 0) {
                         total_at[0] = total;
                         total_at[1] = (int)(order_here - list);
@@ -1422,7 +1433,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                          (int64_t)total * list_tiles > (int64_t)kExactRoundTiles * resident;
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
-    FragGate here = {nullptr, nullptr, 0, 0, {0, 0}};
+    FragGate here = {};
 #define BSA_FRAG_LAUNCH_T(T, WALK, BD, TEAM, GATE, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
     hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD, TEAM, GATE>), grid, dim3(TEAM > 1 ? 64 * TEAM : 64), 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
                        lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, TEAM > 0 ? kOneRound : resident, Hn, lse_rows, \
@@ -1448,19 +1459,6 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
             else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, false, __VA_ARGS__);                                         \
         }                                                                                                              \
     } while (0)
-    if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
-    // Lists of unequal length of one round need no plan: every item has a wavefront of its own from the start.
-    if (queue != nullptr && one_span && total > resident) {
-        hipLaunchKernelGGL(queue_plan_kernel, dim3(kQueues + 1), dim3(kPlanThreads), 0, st, lens, per_head, L, total, resident, idx_stride,
-                           order, queue);
-        gate = queue + kQueueChoice;
-        const dim3 grid((unsigned)(total < resident ? total : resident));
-        if (bounded) BSA_FRAG_LAUNCH(true, grid, 0, total, order, queue, 1u, 0, whole_span, fb_list, fb_count);
-        else BSA_FRAG_LAUNCH(false, grid, 0, total, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
-    }
-    // kRoundsPerLaunch rounds per launch, every workgroup running one item of each: the items of a round start
-    // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
-    const int span = (list_tiles <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
     // The items of the last, partial round are cut when its wavefronts would leave too much of the chip idle (and the exact
     // kernel reaches every head from one buffer): into parts only where the caller gives a buffer, for lists of one length; into
     // teams only where there is no other round, so that calls with and without a buffer, with and without the queues, and over
@@ -1474,17 +1472,31 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     if (gate_call != nullptr) {
         const GateCall& c = *gate_call;
         const int nsub = bs_k / kTile;
-        if (once && split.parts == 1 && c.k_sel > 0 && c.nbk <= (split.team == 1 ? kGateWaveBlocks : kGateMostBlocks) &&
-            gate_here_bytes(c.nbk, c.k_sel, nsub, halves) <= kTile * (kD + 8) * 2) {
-            here = {static_cast<const uint16_t*>(c.q_cmp), static_cast<const uint16_t*>(c.k_cmp), c.nbk, c.k_sel, pace_divisor(c.nbk, c.k_sel)};
-            idx = c.wanted ? c.lists : nullptr;
-            lens = c.wanted ? c.lens : nullptr;
-            if (halves) tile_valid = c.halves.valid;
+        if (once && split.parts == 1 && c.nbk <= (split.team == 1 ? kGateWaveBlocks : kGateMostBlocks) &&
+            gate_here_bytes(c.nbk, c.width, nsub, halves) <= kTile * (kD + 8) * 2) {
+            here = {static_cast<const uint16_t*>(c.q_cmp), static_cast<const uint16_t*>(c.k_cmp), c.nbk, c.width, c.threshold, c.scale, c.k_min,
+                    pace_divisor(c.nbk, c.width)};
+            idx = c.lists;
+            lens = c.lens;
+            if (halves) tile_valid = c.valid;
         } else {
-            const hipError_t e = launch_gate(c.q_cmp, c.k_cmp, c.lists, c.lens, B * Hn, c.nbq, c.nbk, c.k_sel, true, dtype, st, c.norms, c.halves);
+            const hipError_t e = c.make(c.ctx);
             if (e != hipSuccess) return e;
         }
     }
+    if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
+    // Lists of unequal length of one round need no plan: every item has a wavefront of its own from the start.
+    if (queue != nullptr && one_span && total > resident) {
+        hipLaunchKernelGGL(queue_plan_kernel, dim3(kQueues + 1), dim3(kPlanThreads), 0, st, lens, per_head, L, total, resident, idx_stride,
+                           order, queue);
+        gate = queue + kQueueChoice;
+        const dim3 grid((unsigned)(total < resident ? total : resident));
+        if (bounded) BSA_FRAG_LAUNCH(true, grid, 0, total, order, queue, 1u, 0, whole_span, fb_list, fb_count);
+        else BSA_FRAG_LAUNCH(false, grid, 0, total, order, queue, 1u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr);
+    }
+    // kRoundsPerLaunch rounds per launch, every workgroup running one item of each: the items of a round start
+    // together and keep in step (with many more rounds per launch they drift apart and the L2 hit rate falls).
+    const int span = (list_tiles <= kShortList ? kRoundsPerLaunchShort : kRoundsPerLaunch) * resident;
     const int whole = once ? 0 : split.team * split.parts > 1 ? total - tail : total;
     for (int first = 0; first < whole;) {
         int end = first + span < whole ? first + span : whole;

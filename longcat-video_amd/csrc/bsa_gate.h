@@ -160,6 +160,107 @@ __device__ inline void select_row(const uint32_t (&val)[NPL], RawAt raw_at, int 
     }
 }
 
+// ---------------------------------------------------------------- CDF rule
+__device__ inline float score_value(uint16_t s, int dtype) {
+    if (dtype == BSA_F16) return (float)__builtin_bit_cast(_Float16, s);
+    return __uint_as_float((uint32_t)s << 16);
+}
+__device__ inline float score_value(uint32_t s, int) { return __uint_as_float(s); }
+// The sum over the lanes l, l ^ 32, l ^ 16, ... of a butterfly, by moves between registers: the halves of the wavefront and of its
+// rows trade, and inside a row a rotation by 8 (4, 2, 1) reaches lane l ^ 8 (a lane that holds what l ^ 4 does, ...).  A sum of
+// doubles by __shfl is twelve round trips to LDS, and the search below makes sixteen of them (cdf_count_kernel, 16 heads of
+// 20x30x52: 34 us that way).
+__device__ __forceinline__ double wave_sum(double x) {
+    auto halves = [](double y, uint32_t& lo, uint32_t& hi) {
+        const uint64_t b = (uint64_t)__double_as_longlong(y);
+        lo = (uint32_t)b; hi = (uint32_t)(b >> 32);
+    };
+    auto whole = [](uint32_t lo, uint32_t hi) { return __longlong_as_double((long long)((uint64_t)hi << 32 | lo)); };
+    uint32_t lo, hi;
+    halves(x, lo, hi);
+    {
+        const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false), b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        x = whole(a[0], b[0]) + whole(a[1], b[1]);
+    }
+    halves(x, lo, hi);
+    {
+        const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false), b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        x = whole(a[0], b[0]) + whole(a[1], b[1]);
+    }
+#define BSA_ROTATED(N)                                                                                  \
+    halves(x, lo, hi);                                                                                  \
+    x += whole((uint32_t)__builtin_amdgcn_update_dpp(0, (int)lo, 0x120 + N, 0xf, 0xf, false), (uint32_t)__builtin_amdgcn_update_dpp(0, (int)hi, 0x120 + N, 0xf, 0xf, false))
+    BSA_ROTATED(8);
+    BSA_ROTATED(4);
+    BSA_ROTATED(2);
+    BSA_ROTATED(1);
+#undef BSA_ROTATED
+    return x;
+}
+
+// How many columns the CDF rule keeps per row: with the columns sorted by descending score (ties towards
+// the lowest index) and weights softmax(score * scale), the number of leading columns whose running sum
+// of weights stays at or below `threshold`; never fewer than k_min (the "cdf + top-k" rule) and never
+// more than `cap`.  Sums run in double precision on the unnormalised weights
+// e_i = exp((s_i - max) * scale): sum_top(e) <= threshold * sum_all(e).  The columns at or above a score
+// value t form a prefix of the sorted order, so a bitwise binary search over t finds the value group in
+// which the running sum crosses the threshold; inside that group every column weighs the same.
+// val: the order-preserving images of the row's columns l, l + 64, ... in lane l, 0 past its end; e: the scores.
+template <int kValueBits, int NPL>
+__device__ inline int cdf_row(const uint32_t (&val)[NPL], float (&e)[NPL], int lane, int nbk, float threshold, float scale, int k_min, int cap) {
+    float mx = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) mx = fmaxf(mx, e[j]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    double total = 0.0;
+#pragma unroll
+    for (int j = 0; j < NPL; ++j) {
+        e[j] = j * 64 + lane < nbk ? expf((e[j] - mx) * scale) : 0.f;
+        total += (double)e[j];
+    }
+    total = wave_sum(total);
+    const double budget = (double)threshold * total;
+    // largest t whose columns at or above t outweigh the budget (t = 0: all columns, if even that holds)
+    auto mass_ge = [&](uint32_t t) {
+        double m = 0.0;
+#pragma unroll
+        for (int j = 0; j < NPL; ++j) m += val[j] >= t ? (double)e[j] : 0.0;     // padding has e = 0
+        return wave_sum(m);
+    };
+    int n;
+    // NaN by its bits: a file may be built without regard for them
+    const bool nan = ((uint64_t)__double_as_longlong(total) << 1) > 0xffe0000000000000ull;
+    if (nan || !(total > budget)) {
+        n = nbk;                                  // threshold >= 1: everything
+    } else {
+        uint32_t thr = 0;
+        for (int bit = kValueBits - 1; bit >= 0; --bit) {
+            const uint32_t cand = thr | (1u << bit);
+            if (mass_ge(cand) > budget) thr = cand;
+        }
+        // columns above thr fit; the group equal to thr crosses: take as many of it as still fit
+        double above = 0.0, one = 0.0;
+        int cnt_gt = 0, cnt_eq = 0;
+#pragma unroll
+        for (int j = 0; j < NPL; ++j) {
+            const bool real = j * 64 + lane < nbk;
+            above += val[j] > thr ? (double)e[j] : 0.0;
+            cnt_gt += __popcll(__ballot(val[j] > thr));
+            const bool eq = real && val[j] == thr;
+            cnt_eq += __popcll(__ballot(eq));
+            if (eq) one = (double)e[j];
+        }
+        above = wave_sum(above);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) one = fmax(one, __shfl_xor(one, o));
+        int fit = one > 0.0 ? (int)floor((budget - above) / one) : cnt_eq;
+        fit = max(0, min(fit, cnt_eq));
+        n = cnt_gt + fit;
+    }
+    return __builtin_amdgcn_readfirstlane(min(max(n, k_min), min(cap, nbk)));
+}
+
 // The order in which the attention kernel visits one row's selected KV blocks.  Softmax attention does not
 // depend on it beyond rounding, so it is chosen for the L2 cache: the query tiles that run side by side walk
 // the KV sequence together when slot s of every list holds a block near s/n of the sequence, and then share

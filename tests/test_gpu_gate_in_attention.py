@@ -39,3 +39,38 @@ def test_lists_made_by_the_attention_kernel(latent, chunk, heads, sparsity, dtyp
         assert torch.equal(lens, want_lens) and torch.equal(walk, bi.visit_order(ascending, lens, blocks))
         assert torch.isfinite(o.float()).all() and torch.equal(o, want_o)
         assert torch.equal(bi.flash_attn_bsa_3d(q, k, v, latent, latent, sparsity=sparsity, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk), o)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("latent,chunk,heads,threshold,sparsity", [
+    ((4, 4, 4), (4, 4, 4), 1, 0.5, None),             # one block, which alone is more than the threshold: an empty list
+    ((4, 32, 32), (4, 4, 4), 2, 0.5, None),           # a team of four
+    ((4, 32, 32), (4, 4, 4), 9, 0.25, 0.9),           # one wavefront an item, never fewer than six blocks
+    ((16, 32, 32), (4, 4, 4), 1, 1.0, None),          # every one of 256 blocks
+    ((5, 9, 13), (4, 4, 4), 2, 0.75, 0.5),            # ragged: halves
+    ((13, 10, 11), (4, 4, 8), 3, 0.5, None),          # blocks of two tiles, tiles of padding alone
+    ((8, 32, 36), (4, 4, 4), 8, 0.5, None),           # 1 152 items: the kernels in front
+])
+def test_cdf_lists_made_by_the_attention_kernel(latent, chunk, heads, threshold, sparsity, dtype):
+    """The same for the CDF rule, with scores that differ in their spread from block to block, with equal ones, and with a NaN
+    (its rows keep every block)."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    S, blocks = math.prod(latent), math.prod(-(-n // c) for n, c in zip(latent, chunk))
+    g = torch.Generator(device="cuda").manual_seed(32)
+    for kind in ("spread", "ties", "nan"):
+        q, k, v = (torch.randn(1, heads, S, 128, generator=g, device="cuda") for _ in range(3))
+        k = k + 3 * torch.randn(1, heads, 1, 128, generator=g, device="cuda")
+        q = q * torch.rand(1, heads, S, 1, generator=g, device="cuda") * 4
+        if kind == "ties":
+            k[:, :, S // 2:] = k[:, :, :1]
+        q, k, v = (x.to(dtype) for x in (q, k, v))
+        if kind == "nan":
+            q[0, 0, 0, 0] = float("nan")
+        args = (q, k, v, latent, latent, sparsity, chunk, chunk)
+        o, walk, lens, _ = bi._bsa_3d(*args, for_backward=True, cdf_threshold=threshold)
+        want_o, idx, want_lens, _ = bi._bsa_3d(*args, want_selection=True, cdf_threshold=threshold)
+        ascending = torch.where(idx < 0, torch.full_like(idx, blocks), idx).sort(dim=-1).values
+        want = bi.visit_order(torch.where(ascending == blocks, torch.zeros_like(ascending), ascending).int(), want_lens, blocks)
+        used = torch.arange(blocks, device="cuda") < want_lens[..., None]
+        assert torch.equal(lens, want_lens) and torch.equal(walk[used], want[used]) and (walk[~used] == -1).all()
+        assert torch.equal(o.nan_to_num(), want_o.nan_to_num()) and torch.equal(o.isnan(), want_o.isnan())
