@@ -149,7 +149,7 @@ struct FragGate {
     int k_min;
     Divisor by_span;
 };
-constexpr int kGateWaveBlocks = 128, kGateMostBlocks = 256;      // key blocks to a wavefront, to a workgroup
+constexpr int kGateWaveBlocks = 256, kGateMostBlocks = 512;      // key blocks that one wavefront scores, that a team does
 // LDS of the selection: the list of halves; scores; keys of every tile; where the first wavefront works; the list's length
 __host__ __device__ inline int gate_list_words(int width, int nsub, bool halves) { return halves ? (2 * width * nsub + 3) / 4 * 4 : 0; }
 __host__ __device__ inline int gate_here_bytes(int nbk, int width, int nsub, bool halves) {
@@ -679,52 +679,63 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                     for (int i = threadIdx.x; i < G.nbk * nsub_of_block; i += 64 * kTeam) counts[i] = (uint8_t)__popcll(tile_valid[i]);
                 const T* const qm = reinterpret_cast<const T*>(G.qc) + brow * kD + lh * 8;      // its mean as every row of the product
                 const T* const km = reinterpret_cast<const T*>(G.kc) + (int64_t)bh * G.nbk * kD + lh * 8;
-                V8 qa[8], kr[4][8];
+                V8 qa[8];
 #pragma unroll
                 for (int c = 0; c < 8; ++c) qa[c] = *reinterpret_cast<const V8*>(qm + 16 * c);
-                constexpr int kTurns = kTeam == 1 ? kGateWaveBlocks / 32 : kGateMostBlocks / 32 / kTeam;
+                // four of this wavefront's blocks of 32 are on their way at a time
+                for (int n_first = 32 * wave; n_first < G.nbk; n_first += 4 * 32 * kTeam) {
+                    V8 kr[4][8];
 #pragma unroll
-                for (int t = 0; t < kTurns; ++t) {
-                    const int n0 = 32 * (wave + kTeam * t);
-                    if (n0 < G.nbk) {
-                        const T* const kt = km + (int64_t)min(n0 + lr, G.nbk - 1) * kD;
+                    for (int t = 0; t < 4; ++t) {
+                        const int n0 = n_first + 32 * kTeam * t;
+                        if (n0 < G.nbk) {
+                            const T* const kt = km + (int64_t)min(n0 + lr, G.nbk - 1) * kD;
 #pragma unroll
-                        for (int c = 0; c < 8; ++c) kr[t][c] = *reinterpret_cast<const V8*>(kt + 16 * c);
+                            for (int c = 0; c < 8; ++c) kr[t][c] = *reinterpret_cast<const V8*>(kt + 16 * c);
+                        }
                     }
-                }
 #pragma unroll
-                for (int t = 0; t < kTurns; ++t) {
-                    const int n0 = 32 * (wave + kTeam * t);
-                    if (n0 < G.nbk) {
-                        f32x16 acc;
+                    for (int t = 0; t < 4; ++t) {
+                        const int n0 = n_first + 32 * kTeam * t;
+                        if (n0 < G.nbk) {
+                            f32x16 acc;
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+                            for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-                        for (int c = 0; c < 8; ++c) acc = mfma32(qa[c], kr[t][c], acc);
-                        if (lh == 0) scores[n0 + lr] = (T)acc[0];
+                            for (int c = 0; c < 8; ++c) acc = mfma32(qa[c], kr[t][c], acc);
+                            if (lh == 0) scores[n0 + lr] = (T)acc[0];
+                        }
                     }
                 }
                 __syncthreads();
                 if (wave == 0) {
-                    constexpr int kPerLane = kTeam == 1 ? kGateWaveBlocks / 64 : kGateMostBlocks / 64;
-                    uint32_t val[kPerLane];
                     const uint16_t* const raw = reinterpret_cast<const uint16_t*>(scores);
-#pragma unroll
-                    for (int j = 0; j < kPerLane; ++j) {
-                        const int i = j * 64 + lane;
-                        const uint16_t x = raw[min(i, G.nbk - 1)];
-                        val[j] = i < G.nbk ? ord_of(x) : 0u;
-                    }
                     int32_t* const list = reinterpret_cast<int32_t*>(mine);
-                    int k_sel = G.width;
-                    if (G.threshold > 0.f) {
-                        float e[kPerLane];
+                    auto select = [&](auto n_c) -> int {                 // by columns to a lane
+                        constexpr int kPerLane = decltype(n_c)::value;
+                        uint32_t val[kPerLane];
 #pragma unroll
-                        for (int j = 0; j < kPerLane; ++j) e[j] = j * 64 + lane < G.nbk ? (float)scores[min(j * 64 + lane, G.nbk - 1)] : -INFINITY;
-                        k_sel = cdf_row<16>(val, e, lane, G.nbk, G.threshold, G.scale, G.k_min, G.width);
-                    }
+                        for (int j = 0; j < kPerLane; ++j) {
+                            const int i = j * 64 + lane;
+                            const uint16_t x = raw[min(i, G.nbk - 1)];
+                            val[j] = i < G.nbk ? ord_of(x) : 0u;
+                        }
+                        int n = G.width;
+                        if (G.threshold > 0.f) {
+                            float e[kPerLane];
+#pragma unroll
+                            for (int j = 0; j < kPerLane; ++j) e[j] = j * 64 + lane < G.nbk ? (float)scores[min(j * 64 + lane, G.nbk - 1)] : -INFINITY;
+                            n = cdf_row<16>(val, e, lane, G.nbk, G.threshold, G.scale, G.k_min, G.width);
+                        }
+                        if (n > 0) select_row<uint16_t, kPerLane, false>(val, [&](int i) { return raw[i]; }, lane, G.nbk, n, nullptr, list, nullptr, mine);
+                        return n;
+                    };
+                    int k_sel;
+                    if (G.nbk <= 64) k_sel = select(std::integral_constant<int, 1>{});
+                    else if (G.nbk <= 128) k_sel = select(std::integral_constant<int, 2>{});
+                    else if (kTeam == 1 || G.nbk <= 256) k_sel = select(std::integral_constant<int, 4>{});
+                    else k_sel = select(std::integral_constant<int, 8>{});
                     int32_t* const dst = idx != nullptr ? const_cast<int32_t*>(idx) + brow * G.width : nullptr;
-                    if (k_sel > 0) select_row<uint16_t, kPerLane, false>(val, [&](int i) { return raw[i]; }, lane, G.nbk, k_sel, nullptr, list, nullptr, mine);
                     wave_sync();
                     const int32_t* order_here = list;
                     if (k_sel > kPaceWidth) order_here = pace_row(list, k_sel, k_sel, G.nbk, lane, dst, G.by_span);
@@ -1468,11 +1479,13 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     if (one_span && tail > 0 && (part_buf != nullptr || total < resident))
         split = choose_split(tail, list_tiles, resident, total > resident, part_buf != nullptr);
     const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
-    // The lists of a call of one round are made by the workgroups that walk them, where that is little work.
+    // The lists of a call whose workgroups all run at once are made by those that walk them.  The kernels in front / like this, us, density
+    // 1/16: 4 heads of 192 blocks (one wavefront an item) 48.1 / 46.1, 4 of 256 64.6 / 64.8, one of 320 (teams of four) 43.7 / 40.0, of 512
+    // 66.6 / 62.5; one workgroup behind another pays for it twice (2 heads of 320 blocks, teams of four, density 1/4, 147 / 156).
     if (gate_call != nullptr) {
         const GateCall& c = *gate_call;
         const int nsub = bs_k / kTile;
-        if (once && split.parts == 1 && c.nbk <= (split.team == 1 ? kGateWaveBlocks : kGateMostBlocks) &&
+        if (once && split.parts == 1 && total * split.team <= resident && c.nbk <= (split.team == 1 ? kGateWaveBlocks : kGateMostBlocks) &&
             gate_here_bytes(c.nbk, c.width, nsub, halves) <= kTile * (kD + 8) * 2) {
             here = {static_cast<const uint16_t*>(c.q_cmp), static_cast<const uint16_t*>(c.k_cmp), c.nbk, c.width, c.threshold, c.scale, c.k_min,
                     pace_divisor(c.nbk, c.width)};

@@ -14,10 +14,12 @@ pytestmark = pytest.mark.gpu
     ((4, 32, 32), (4, 4, 4), 8, 0.8),           # ... 512 items, teams of two
     ((4, 32, 32), (4, 4, 4), 9, 0.8),           # ... 576, one wavefront an item
     ((4, 20, 52), (4, 4, 4), 3, 0.5),           # 65 blocks
-    ((8, 32, 32), (4, 4, 4), 8, 0.75),          # 128 blocks, one wavefront an item, the most it scores
-    ((4, 12, 172), (4, 4, 4), 7, 0.75),         # 129: 903 items, the kernel in front
-    ((16, 32, 32), (4, 4, 4), 1, 0.3),          # 256 blocks: the most a team scores; 179 kept
-    ((4, 4, 1028), (4, 4, 4), 1, 0.9),          # 257: the kernel in front
+    ((8, 32, 32), (4, 4, 4), 8, 0.75),          # 128 blocks, one wavefront an item
+    ((4, 12, 172), (4, 4, 4), 7, 0.75),         # 129: more than two columns a lane
+    ((16, 32, 32), (4, 4, 4), 4, 0.3),          # 256 blocks, the most a wavefront scores; 179 kept
+    ((4, 4, 1028), (4, 4, 4), 3, 0.9),          # 257, 771 items: the kernel in front
+    ((8, 64, 64), (4, 4, 4), 1, 0.8),           # 512: the most a team scores
+    ((4, 4, 2052), (4, 4, 4), 1, 0.9),          # 513: the kernels in front
     ((5, 9, 13), (4, 4, 4), 2, 0.5),            # ragged: halves
     ((5, 33, 30), (4, 4, 4), 7, 0.7),           # ... 144 blocks, 1 008 items
     ((13, 10, 11), (4, 4, 8), 3, 0.4),          # blocks of two tiles, tiles of padding alone
