@@ -705,7 +705,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         return r;
     };
     // made in front of the attention kernel, or by it where the caller asks for nothing but what it walks (launch_fwd_frag)
-    const bool by_attention = pl.frag && idx_out == nullptr && score_out == nullptr && pl.sel_width > 0;
+    const bool by_attention = (pl.frag || pl.f32) && idx_out == nullptr && score_out == nullptr && pl.sel_width > 0;
     const bool lists_wanted = walk_out != nullptr || lens_out != nullptr;
     const GateCall gate = {w.qc, w.kc, lists_wanted ? w.idx_sorted : nullptr, lists_wanted ? w.lens : nullptr, w.valid, pl.nbk, pl.sel_width,
                            pl.cdf ? p->cdf_threshold : 0.f, p->sm_scale, k_min,
@@ -727,7 +727,7 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
         L.lse_rows = (int64_t)p->Tq * p->Hq * p->Wq;
         for (int i = 0; i < 3; ++i) { L.q_st[i] = q_strides[i]; L.k_st[i] = k_strides[i]; L.v_st[i] = v_strides[i]; L.o_st[i] = o_strides[i]; }
         BSA_HIP(launch_fwd_f32(q, k, v, w.idx_sorted, w.lens, nullptr, o, nullptr, p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(),
-                               pl.sel_width, p->sm_scale, st, &L), "attention");
+                               pl.sel_width, p->sm_scale, st, &L, by_attention ? &gate : nullptr), by_attention ? "selection and attention" : "attention");
     }
     const size_t bh = (size_t)p->B * p->Hn;
     if (idx_out && pl.sel_width > 0)

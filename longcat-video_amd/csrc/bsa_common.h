@@ -217,7 +217,7 @@ struct HalfLists {
 // visiting order, lens = k_sel.  The same lists as launch_score, launch_topk and launch_pace_order; gate_fits says for
 // which sizes it is built and the better choice.
 bool gate_fits(int BH, int nbq, int nbk, int k_sel, int dtype);
-// A selection that launch_fwd_frag lets the attention kernel make, or has made in front of it by make(ctx).
+// A selection that launch_fwd_frag and launch_fwd_f32 let the attention kernel make, or has made in front of it by make(ctx).
 struct GateCall {
     const void *q_cmp, *k_cmp;       // chunk means
     int32_t *lists, *lens;           // where the lists go ([BH][nbq][width]), null: they are not read behind the attention
@@ -250,7 +250,7 @@ hipError_t launch_pool_f32(const void* q, const int64_t q_st[3], const Grid3& gq
                            const int64_t k_st[3], const Grid3& gk, float* k_pooled, int32_t* k_rows, int B, int Hn, hipStream_t st);
 hipError_t launch_fwd_f32(const void* q, const void* k, const void* v, const int32_t* idx, const int32_t* lens,
                           const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k,
-                          int idx_stride, float sm_scale, hipStream_t st, const F32Layout* layout = nullptr);
+                          int idx_stride, float sm_scale, hipStream_t st, const F32Layout* layout = nullptr, const GateCall* gate_call = nullptr);
 
 // Rewrites every row's ascending list of KV blocks into the order the attention kernel visits them in (see
 // pace_order_kernel).  rows of `stride` entries, lens[row] of them in use; in == out allowed; stride <= 5000.

@@ -5,6 +5,7 @@
 // the 1 024 SIMDs a call of a few dozen query rows reaches and how many launches it makes.  256 tokens x 4 heads took
 // 93 us with a plain kernel behind four copies (62 us for 16 workgroups that walked their keys one by one, 20 us for
 // the copies, 12 us for scores computed one column per lane).
+#include "bsa_gate.h"
 #include "bsa_mfma.h"
 
 namespace bsa {
@@ -16,9 +17,11 @@ using mfma::kLn2;
 using mfma::kLog2e;
 using mfma::kTile;
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int64_t kF32SplitUnits = 4096;
+// Units, and units times key blocks, up to which they select for themselves; the four units of a query block make its list four
+// times.  With gate_kernel in front / like this, us: 64 units and 4 blocks 16.7 / 14.1, 512 and 128 44.5 / 40.9, 1 024 and 32 39.9 /
+// 37.1, 1 024 and 64 50.8 / 48.1, 1 024 and 128 72.7 / 74.1, 2 048 and 64 83.6 / 87.2.
+constexpr int64_t kF32GateUnits = 1024, kF32GateScores = 64 * 1024;
 
 // ------------------------------------------------------------------ chunk means and row tables
 // blockIdx.z 0: q, 1: k.  One workgroup per (chunk, batch * head): a thread sums 16-byte piece c of the rows rg, rg + 8,
@@ -94,9 +97,15 @@ struct F32Args {
     int64_t Sq, Sk, lse_rows;
     int Hn, bs_q, bs_k, idx_stride;
     float qk_scale;
+    const float *qc, *kc;             // kGate: chunk means
+    int k_sel;
 };
 
-template <int kSplit>
+// kGate: the workgroup makes its block's list itself, as gate_kernel does (the same scores and choice, blocks ascending), instead
+// of a launch in front that is longer than that.  Of the wavefronts' scores, 16 at a time, each
+// is made once; the first wavefront selects.
+constexpr int kF32GateBlocks = 128;
+template <int kSplit, bool kGate>
 __global__ __launch_bounds__(256) void fwd_f32_kernel(F32Args a) {
     constexpr int kPitch = kD + 4;
     __shared__ __attribute__((aligned(16))) float part_o[kSplit == 1 ? 1 : kSplit * 16 * kPitch];
@@ -112,9 +121,11 @@ __global__ __launch_bounds__(256) void fwd_f32_kernel(F32Args a) {
     const float* vb = a.v + at * a.v_st[0] + hd * a.v_st[1];
     const int nbq = (int)(a.Sq / a.bs_q), nbk = (int)(a.Sk / a.bs_k), per_block = a.bs_k / 16;
     const int64_t lrow = bh * nbq + slot0 / a.bs_q;
-    const int32_t* list = a.idx + lrow * a.idx_stride;
+    __shared__ float gate_scores[kGate ? kF32GateBlocks : 1];
+    __shared__ int32_t gate_list[kGate ? kF32GateBlocks : 1];
+    const int32_t* list = kGate ? nullptr : a.idx + lrow * a.idx_stride;
     const int qtok = a.q_rows != nullptr ? a.q_rows[slot0 + n16] : (int)slot0 + n16;
-    int ngroups = __builtin_amdgcn_readfirstlane(min(max(a.lens[lrow], 0), a.idx_stride)) * per_block;
+    int ngroups = (kGate ? a.k_sel : __builtin_amdgcn_readfirstlane(min(max(a.lens[lrow], 0), a.idx_stride))) * per_block;
     if (!__any(qtok >= 0)) ngroups = 0;                               // query rows of padding only
 
     f32x4 qv[8], o[8];
@@ -126,9 +137,30 @@ __global__ __launch_bounds__(256) void fwd_f32_kernel(F32Args a) {
             o[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
+    if constexpr (kGate) {
+        f32x4 qm[8], km[8];
+        score_row_f32(a.qc + lrow * kD + 4 * g, qm);                  // the block's mean as every row of the product
+        for (int n0 = 16 * wave; n0 < nbk; n0 += 64) {
+            score_row_f32(a.kc + (bh * nbk + min(n0 + n16, nbk - 1)) * kD + 4 * g, km);
+            const f32x4 acc = score_tile_f32(qm, km);
+            if (g == 0) gate_scores[n0 + n16] = acc[0];
+        }
+        __syncthreads();
+        if (wave == 0) {
+            uint32_t val[kF32GateBlocks / 64];
+#pragma unroll
+            for (int j = 0; j < kF32GateBlocks / 64; ++j) {
+                const int i = j * 64 + lane;
+                val[j] = i < nbk ? ord_of(__float_as_uint(gate_scores[min(i, nbk - 1)])) : 0u;
+            }
+            select_row<uint32_t, kF32GateBlocks / 64, false>(val, [&](int i) { return __float_as_uint(gate_scores[i]); }, lane, nbk, a.k_sel, nullptr,
+                                                             gate_list, nullptr, nullptr);
+        }
+        __syncthreads();
+    }
     // key group gi of the walk: its first blocked-order slot; tokens of its keys (-1: padding or masked)
     auto slot_of = [&](int gi) -> int64_t {
-        const int blk = min(max(__builtin_amdgcn_readfirstlane(list[gi / per_block]), 0), nbk - 1);
+        const int blk = min(max(__builtin_amdgcn_readfirstlane(kGate ? gate_list[gi / per_block] : list[gi / per_block]), 0), nbk - 1);
         return (int64_t)blk * a.bs_k + (gi % per_block) * 16;
     };
     struct Rows { int k; int v[4]; };                                 // key n16 of the group; keys 4 g .. 4 g + 3
@@ -277,7 +309,7 @@ hipError_t launch_pool_f32(const void* q, const int64_t q_st[3], const Grid3& gq
 
 hipError_t launch_fwd_f32(const void* q, const void* k, const void* v, const int32_t* idx, const int32_t* lens,
                           const uint64_t* tile_valid, void* o, float* lse, int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k,
-                          int idx_stride, float sm_scale, hipStream_t st, const F32Layout* layout) {
+                          int idx_stride, float sm_scale, hipStream_t st, const F32Layout* layout, const GateCall* gate_call) {
     F32Args a = {};
     a.q = (const float*)q; a.k = (const float*)k; a.v = (const float*)v; a.o = (float*)o;
     a.lse = lse; a.idx = idx; a.lens = lens; a.tile_valid = tile_valid;
@@ -299,10 +331,22 @@ hipError_t launch_fwd_f32(const void* q, const void* k, const void* v, const int
     // Up to 4 096 16-row units one workgroup each still is at most four wavefronts' worth per SIMD: the split walk is a
     // quarter as long.  Beyond, four units share a workgroup, and what they read of k and v.
     const int64_t units = (int64_t)B * Hn * (Sq / 16);
+    if (gate_call != nullptr) {
+        const GateCall& c = *gate_call;
+        if (units <= kF32GateUnits && units * c.nbk <= kF32GateScores && c.nbk <= kF32GateBlocks && c.lists == nullptr && c.threshold == 0.f && c.width > 0) {
+            a.qc = static_cast<const float*>(c.q_cmp);
+            a.kc = static_cast<const float*>(c.k_cmp);
+            a.k_sel = c.width;
+            hipLaunchKernelGGL((fwd_f32_kernel<4, true>), dim3((unsigned)units), dim3(256), 0, st, a);
+            return hipGetLastError();
+        }
+        const hipError_t e = c.make(c.ctx);
+        if (e != hipSuccess) return e;
+    }
     if (units <= kF32SplitUnits)
-        hipLaunchKernelGGL((fwd_f32_kernel<4>), dim3((unsigned)units), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((fwd_f32_kernel<4, false>), dim3((unsigned)units), dim3(256), 0, st, a);
     else
-        hipLaunchKernelGGL((fwd_f32_kernel<1>), dim3((unsigned)(units / 4)), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((fwd_f32_kernel<1, false>), dim3((unsigned)(units / 4)), dim3(256), 0, st, a);
     return hipGetLastError();
 }
 

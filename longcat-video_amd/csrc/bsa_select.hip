@@ -118,21 +118,6 @@ __global__ __launch_bounds__(256) void score_mfma_kernel(const T* __restrict__ q
     }
 }
 
-// fp32 storage type: v_mfma_f32_16x16x4, a wavefront per 16 x 16 scores.  Step (j, e) contracts d = 16 j + 4 (lane / 16) + e,
-// so that a lane reads its row in 16-byte pieces.  score_tile_f32 is also what the one-launch gating runs: the same bits.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void score_row_f32(const float* row, f32x4 (&x)[8]) {       // row + 4 (lane / 16)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = *reinterpret_cast<const f32x4*>(row + 16 * j);
-}
-__device__ __forceinline__ f32x4 score_tile_f32(const f32x4 (&a)[8], const f32x4 (&b)[8]) {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j][e], b[j][e], acc, 0, 0, 0);
-    return acc;                              // accumulator i of lane l: row 4 (l / 16) + i, column l % 16
-}
 __global__ __launch_bounds__(256) void score_f32_kernel(const float* __restrict__ qc, const float* __restrict__ kc,
                                                         float* __restrict__ score, int nbq, int nbk) {
     constexpr int D = 128;

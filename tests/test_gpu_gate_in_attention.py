@@ -76,3 +76,27 @@ def test_cdf_lists_made_by_the_attention_kernel(latent, chunk, heads, threshold,
         used = torch.arange(blocks, device="cuda") < want_lens[..., None]
         assert torch.equal(lens, want_lens) and torch.equal(walk[used], want[used]) and (walk[~used] == -1).all()
         assert torch.equal(o.nan_to_num(), want_o.nan_to_num()) and torch.equal(o.isnan(), want_o.isnan())
+
+
+@pytest.mark.parametrize("latent,chunk,heads,sparsity", [
+    ((4, 4, 4), (4, 4, 4), 1, 0.0),
+    ((4, 8, 8), (4, 4, 4), 4, 0.5),
+    ((4, 32, 32), (4, 4, 4), 4, 0.9),           # 64 blocks, 1 024 units: the most
+    ((4, 20, 52), (4, 4, 4), 2, 0.5),           # 65
+    ((8, 32, 32), (4, 4, 4), 1, 0.75),          # 128: the most
+    ((4, 12, 172), (4, 4, 4), 1, 0.75),         # 129: the kernel in front
+    ((5, 9, 13), (4, 4, 4), 2, 0.5),            # ragged
+    ((13, 10, 11), (4, 4, 8), 1, 0.4),          # blocks of eight units, some of padding alone
+])
+def test_fp32_lists_made_by_the_attention_kernel(latent, chunk, heads, sparsity):
+    """The same for fp32 operands, by the output alone: another list would be another output."""
+    from longcat_video_amd.block_sparse_attention import bsa_interface as bi
+    S = math.prod(latent)
+    g = torch.Generator(device="cuda").manual_seed(33)
+    for ties in (False, True):
+        q, k, v = (torch.randn(2, heads, S, 128, generator=g, device="cuda")[:1] for _ in range(3))
+        if ties:
+            k[:, :, S // 2:] = k[:, :, :1]
+        want = bi._bsa_3d(q, k, v, latent, latent, sparsity, chunk, chunk, want_selection=True)[0]
+        got = bi.flash_attn_bsa_3d(q, k, v, latent, latent, sparsity=sparsity, chunk_3d_shape_q=chunk, chunk_3d_shape_k=chunk)
+        assert torch.isfinite(got).all() and torch.equal(got, want)
