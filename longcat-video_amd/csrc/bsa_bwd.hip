@@ -310,33 +310,44 @@ __device__ __forceinline__ int halves_of(const LiveHalves& q, uint32_t bits, int
 // counts[bh * nbk + j] = number of query halves that KV block j meets (those of the blocks set in its row of the bit matrix); with
 // `base` also the number of dS units (kDsUnitBytes) of the head's blocks in front of j; order: the head's KV tiles by descending
 // count in whole blocks, a counting sort (tiles of one count in no particular order).  One workgroup per head.  LDS: a bin per
-// count, 0 .. nbq, and four words at least.
-__global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restrict__ bits, int32_t* __restrict__ counts,
+// count, 0 .. nbq, and a word per wavefront at least.
+constexpr int kCountThreads = 1024;      // of 256 where there are no more blocks
+__global__ __launch_bounds__(kCountThreads) void bwd_count_kernel(const uint32_t* __restrict__ bits, int32_t* __restrict__ counts,
                                                         int32_t* __restrict__ base, int32_t* __restrict__ order, int words, int nbk, int nbq,
                                                         int tiles_per_block, LiveHalves q, Divisor by_full) {
     extern __shared__ int bins[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), threads = blockDim.x;
     const int64_t head = (int64_t)blockIdx.x * nbk;
     int before = 0;
-    for (int j0 = 0; j0 < nbk; j0 += 256) {
+    for (int j0 = 0; j0 < nbk; j0 += threads) {
         const int j = j0 + threadIdx.x;
         int c = 0;
-        if (j < nbk)
-            for (int w = 0; w < words; ++w) c += halves_of(q, bits[(head + j) * words + w], w);
+        if (j < nbk) {
+            const uint32_t* row = bits + (head + j) * words;
+            for (int w0 = 0; w0 < words; w0 += 8) {                // eight words on their way
+                uint32_t x[8];
+#pragma unroll
+                for (int w = 0; w < 8; ++w) x[w] = row[min(w0 + w, words - 1)];
+#pragma unroll
+                for (int w = 0; w < 8; ++w)
+                    if (w0 + w < words) c += halves_of(q, x[w], w0 + w);
+            }
+        }
         if (j < nbk) counts[head + j] = c;
         if (base == nullptr) continue;
         int upto = wave_scan(c);
         if (lane == 63) bins[wave] = upto;
         __syncthreads();
-        for (int w = 0; w < wave; ++w) upto += bins[w];
+        const int sums = wave_scan(lane < threads / 64 ? bins[lane] : 0);         // the wavefronts in front, then all of them
+        upto += wave > 0 ? __builtin_amdgcn_readlane(sums, wave - 1) : 0;
         if (j < nbk) base[head + j] = (before + upto - c) * tiles_per_block;
-        before += bins[0] + bins[1] + bins[2] + bins[3];
+        before += __builtin_amdgcn_readlane(sums, 63);
         __syncthreads();
     }
-    for (int i = threadIdx.x; i <= nbq; i += 256) bins[i] = 0;
+    for (int i = threadIdx.x; i <= nbq; i += threads) bins[i] = 0;
     __syncthreads();
     auto bin = [&](int j) -> int { return (counts[head + j] + q.full - 1) / by_full; };
-    for (int j = threadIdx.x; j < nbk; j += 256) atomicAdd(&bins[bin(j)], tiles_per_block);       // this thread's own counts
+    for (int j = threadIdx.x; j < nbk; j += threads) atomicAdd(&bins[bin(j)], tiles_per_block);       // this thread's own counts
     __syncthreads();
     // offsets in descending count: lane l of the first wavefront takes the l-th share of the bins, from the top
     if (wave == 0) {
@@ -350,7 +361,7 @@ __global__ __launch_bounds__(256) void bwd_count_kernel(const uint32_t* __restri
     }
     __syncthreads();
     const int first_tile = (int)blockIdx.x * nbk * tiles_per_block;
-    for (int j = threadIdx.x; j < nbk; j += 256) {
+    for (int j = threadIdx.x; j < nbk; j += threads) {
         const int to = atomicAdd(&bins[bin(j)], tiles_per_block);
         for (int i = 0; i < tiles_per_block; ++i) order[first_tile + to + i] = first_tile + j * tiles_per_block + i;
     }
@@ -1463,7 +1474,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     // blocks; bwd_count_kernel has a bin for each of their numbers, less than that
     const size_t lds = bwd_dkdv_lds_bytes(nbq);
     if (lds > kBwdLdsLimit) return hipErrorInvalidValue;          // the C-ABI layer has rejected such a shape already
-    const size_t count_lds = (size_t)(nbq + 1 > 4 ? nbq + 1 : 4) * sizeof(int);
+    const size_t count_lds = (size_t)(nbq + 1 > kCountThreads / 64 ? nbq + 1 : kCountThreads / 64) * sizeof(int);
     // Per device, once: the dK / dV instantiations and bwd_count_kernel may use all of the LDS, and the number of compute units.
     static std::atomic<int> device_cus[64];
     int dev = 0;
@@ -1533,7 +1544,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     // dQ walks every list in the forward kernel's visiting order when the list is ascending (a selection in block
     // order); any other order is walked as given.  The order only moves fp32 roundings of the dQ sum.
     if ((e = launch_pace_order(idx, paced, lens, lrows, nbk, idx_stride, st, {}, {bits, nbq, words})) != hipSuccess) return e;
-    hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)bh), dim3(256), count_lds, st, bits, counts, kept.keep ? base : nullptr, order, words, nbk, nbq,
+    hipLaunchKernelGGL(bwd_count_kernel, dim3((unsigned)bh), dim3(nbk <= 256 ? 256 : kCountThreads), count_lds, st, bits, counts, kept.keep ? base : nullptr, order, words, nbk, nbq,
                        nsub, q_live, divisor(q_live.full));
 
     const dim3 block(64);

@@ -454,9 +454,13 @@ template <typename S>
 hipError_t launch_cdf_count_t(const S* score, int32_t* lens, int64_t rows, int nbk, float threshold, float scale,
                               int k_min, int cap, int dtype, hipStream_t st) {
     dim3 grid((unsigned)((rows + 3) / 4)), block(256);
+    // bound by the sixteen masked sums of doubles over a lane's columns, past the row's end too: many widths
 #define BSA_CDF(N) hipLaunchKernelGGL((cdf_count_kernel<S, N>), grid, block, 0, st, score, lens, rows, nbk, threshold, scale, k_min, cap, dtype)
     if (nbk <= 4 * 64) BSA_CDF(4);
+    else if (nbk <= 6 * 64) BSA_CDF(6);
     else if (nbk <= 8 * 64) BSA_CDF(8);
+    else if (nbk <= 10 * 64) BSA_CDF(10);
+    else if (nbk <= 12 * 64) BSA_CDF(12);
     else if (nbk <= 16 * 64) BSA_CDF(16);
     else if (nbk <= 24 * 64) BSA_CDF(24);
     else if (nbk <= 32 * 64) BSA_CDF(32);
