@@ -86,6 +86,15 @@ def _rows_ok(t: torch.Tensor) -> torch.Tensor:
     return t if ok else t.contiguous()
 
 
+def _operand(t: torch.Tensor):
+    """_rows_ok, with the pointer and the strides that the C ABI takes, each asked for once."""
+    at, s = t.data_ptr(), t.stride()
+    if at == 0 or s[3] != 1 or (at | (s[0] | s[1] | s[2]) * t.element_size()) % 16 != 0 or t.is_neg():
+        t = _rows_ok(t)
+        at, s = t.data_ptr(), t.stride()
+    return t, at, _strides_of(s[0], s[1], s[2])
+
+
 _WORKSPACES: dict = {}
 
 
@@ -473,8 +482,8 @@ class _AttentionBsa(torch.autograd.Function):
         return dq, dk, dv, None, None, None, None, None, None
 
 
-def _wants_grad(*tensors: torch.Tensor) -> bool:
-    return torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+def _wants_grad(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    return torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
 
 
 def flash_attn_bsa(q, k, v, chunk_size_q, chunk_size_k, sparsity, cdf_threshold, sm_scale,
@@ -531,8 +540,11 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
     knows grids, chunks and rules to be plain numbers (see _plan_of)."""
     _need_gpu(q, k, v)
     B, H, Sq, D = q.shape
-    q, k, v = _rows_ok(q), _rows_ok(k), _rows_ok(v)
+    q, q_at, q_st = _operand(q)
+    k, k_at, k_st = _operand(k)
+    v, v_at, v_st = _operand(v)
     lib = _capi.load()
+    dtype, device = q.dtype, q.device
     if plain:
         plan = _plan_3d(B, H, D, _code(q), *latent_shape_q, *latent_shape_k, *chunk_q, *chunk_k, sparsity, cdf_threshold)
     else:
@@ -542,45 +554,45 @@ def _bsa_3d(q, k, v, latent_shape_q, latent_shape_k, sparsity, chunk_q, chunk_k,
         # this route gathers k and v tiles with one set of in-tile offsets (32 bits); views that
         # do not fit are copied once
         k, v = k.contiguous(), v.contiguous()
-    ws = None if static_scratch else _workspace(need, q.device)
-    o = torch.empty(B, H, Sq, D, dtype=q.dtype, device=q.device) if out is None else out
-    assert o.shape == (B, H, Sq, D) and o.dtype == q.dtype and o.stride(3) == 1
+        k_at, k_st, v_at, v_st = _ptr(k), _st(k), _ptr(v), _st(v)
+    ws = None if static_scratch else _workspace(need, device)
+    if out is None:
+        o = torch.empty(B, H, Sq, D, dtype=dtype, device=device)
+    else:
+        o = out
+        assert o.shape == (B, H, Sq, D) and o.dtype == dtype and o.stride(3) == 1
     idx = lens = score = None
     if want_selection:
         idx = torch.empty(B, H, nbq, width, dtype=torch.int32, device=q.device)
         lens = torch.empty(B, H, nbq, dtype=torch.int32, device=q.device)
         score = torch.empty(B, H, nbq, nbk, dtype=q.dtype, device=q.device)
     if for_backward:
-        walk = torch.empty(B, H, nbq, max(width, 1), dtype=torch.int32, device=q.device)[..., :width]
-        lens = torch.empty(B, H, nbq, dtype=torch.int32, device=q.device)
-        lse = torch.empty(B, H, Sq, dtype=torch.float32, device=q.device)
+        walk = torch.empty(B, H, nbq, max(width, 1), dtype=torch.int32, device=device)[..., :width]
+        lens = torch.empty(B, H, nbq, dtype=torch.int32, device=device)
+        lse = torch.empty(B, H, Sq, dtype=torch.float32, device=device)
         with _on_device(q):
             _capi.check(lib.bsa_fwd_3d_lse(
-                prm, _ptr(q), _st(q), _ptr(k), _st(k),
-                _ptr(v), _st(v), _ptr(o), _st(o),
+                prm, q_at, q_st, k_at, k_st, v_at, v_st, _ptr(o), _st(o),
                 _ptr(lse), _ptr(walk), _ptr(lens), _ptr(ws), need, _stream(q)), "flash_attn_bsa_3d (with lse)")
         return o, walk, lens, lse
     with _on_device(q):
         if qk_norm is not None:
             qw, kw, tab, table_T, t_off_q, t_off_k, eps = qk_norm
             qw, kw = qw.to(q.dtype).contiguous(), kw.to(q.dtype).contiguous()
-            q_normed = torch.empty(B, H, Sq, D, dtype=q.dtype, device=q.device)
+            q_normed = torch.empty(B, H, Sq, D, dtype=dtype, device=device)
             n = _capi.BsaQkNorm(_ptr(qw), _ptr(kw), _ptr(tab), int(table_T), int(t_off_q), int(t_off_k), float(eps))
             c = _kv_cache_arg(q, k, int(latent_shape_k[1]) * int(latent_shape_k[2]), kv_cache, kv_out)
             _capi.check(lib.bsa_fwd_3d_qknorm_kv(
-                prm, C.byref(n), None if c is None else C.byref(c), _ptr(q), _st(q), _ptr(q_normed),
-                _st(q_normed), _ptr(k), _st(k),
-                _ptr(v), _st(v), _ptr(o), _st(o),
+                prm, C.byref(n), None if c is None else C.byref(c), q_at, q_st, _ptr(q_normed),
+                _st(q_normed), k_at, k_st, v_at, v_st, _ptr(o), _st(o),
                 _ptr(ws), need, _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d (q/k norm inside)")
         elif static_scratch:
             _capi.check(lib.bsa_fwd_3d_static(
-                prm, _ptr(q), _st(q), _ptr(k), _st(k),
-                _ptr(v), _st(v), _ptr(o), _st(o),
+                prm, q_at, q_st, k_at, k_st, v_at, v_st, _ptr(o), _st(o),
                 _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d (static scratch)")
         else:
             _capi.check(lib.bsa_fwd_3d(
-                prm, _ptr(q), _st(q), _ptr(k), _st(k),
-                _ptr(v), _st(v), _ptr(o), _st(o),
+                prm, q_at, q_st, k_at, k_st, v_at, v_st, _ptr(o), _st(o),
                 _ptr(ws), need, _ptr(idx), _ptr(lens), _ptr(score), _stream(q)), "flash_attn_bsa_3d")
     return (o, idx, lens, score) if want_selection else o
 
@@ -750,17 +762,16 @@ def _bsa_3d_backward(do, q, k, v, o, lse, walk, lens, latent_q, latent_k, chunk_
     _need_gpu(do, q, k, v, o)
     B, H, Sq, D = q.shape
     lib = _capi.load()
-    q, k, v, o, do = (_rows_ok(t) for t in (q, k, v, o, do))
+    (q, q_at, q_st), (k, k_at, k_st), (v, v_at, v_st), (o, o_at, o_st), (do, do_at, do_st) = map(_operand, (q, k, v, o, do))
     width = walk.shape[3]
     prm, need, least = _plan_3d_backward(B, H, D, _code(q), *latent_q, *latent_k, *chunk_q, *chunk_k, float(sm_scale), width,
                                          unequal_lengths)
     ws = _backward_workspace(need, least, q.device)
     dq, dk, dv = (torch.empty(t.shape, dtype=t.dtype, device=t.device) for t in (q, k, v))
     lse, walk, lens = lse.contiguous(), walk.contiguous(), lens.contiguous()
-    st = _st
     with _on_device(q):
-        _capi.check(lib.bsa_bwd_3d(prm, _ptr(q), st(q), _ptr(k), st(k), _ptr(v), st(v), _ptr(o), st(o), _ptr(do), st(do),
-                                   _ptr(lse), _ptr(walk), _ptr(lens), width, _ptr(dq), st(dq), _ptr(dk), st(dk), _ptr(dv), st(dv),
+        _capi.check(lib.bsa_bwd_3d(prm, q_at, q_st, k_at, k_st, v_at, v_st, o_at, o_st, do_at, do_st,
+                                   _ptr(lse), _ptr(walk), _ptr(lens), width, _ptr(dq), _st(dq), _ptr(dk), _st(dk), _ptr(dv), _st(dv),
                                    _ptr(ws), ws.numel(), _stream(q)), "bsa_bwd_3d")
     return dq, dk, dv
 
@@ -813,8 +824,10 @@ def _bsa_3d_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, latent_shape_q
 def _calls_directly(*tensors: torch.Tensor) -> bool:
     """Plain tensors on the GPU and nothing that wants to see the operator go by (tracing, a dispatch or function mode,
     functorch): the custom op's dispatch, 20 us of a call, is then left out."""
-    return (all((type(t) is torch.Tensor or type(t) is torch.nn.Parameter) and t.is_cuda for t in tensors)
-            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
+    for t in tensors:
+        if not ((type(t) is torch.Tensor or type(t) is torch.nn.Parameter) and t.is_cuda):
+            return False
+    return (torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0
             and torch._C._functorch.peek_interpreter_stack() is None and torch._C._get_tracing_state() is None)
 
 

@@ -81,11 +81,15 @@ _GEMM_WORKSPACES = _Bounded(16)          # 64 MiB each
 
 def _gemm_workspace(device) -> torch.Tensor:
     """64 MiB per device and stream, kept: calls on one stream run one after the other."""
-    key = (str(device), torch._C._cuda_getCurrentRawStream(device.index))
+    key = (device.index, torch._C._cuda_getCurrentRawStream(device.index))
     ws = _GEMM_WORKSPACES.get(key)
     if ws is None:
         ws = _GEMM_WORKSPACES[key] = torch.empty(64 << 20, dtype=torch.uint8, device=device)
     return ws
+
+
+def _bf16(t: torch.Tensor) -> torch.Tensor:
+    return t if t.dtype == torch.bfloat16 and t.is_contiguous() else t.to(torch.bfloat16).contiguous()
 
 
 def linear_bf16(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
@@ -99,22 +103,24 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     K = x.shape[-1]
     N = weight.shape[0]
     assert weight.shape[1] == K
-    x2 = x.reshape(-1, K).contiguous()
-    w = weight.to(torch.bfloat16).contiguous()
-    b = None if bias is None else bias.to(torch.bfloat16).contiguous()
+    x2 = x if x.is_contiguous() else x.reshape(-1, K).contiguous()
+    M = x2.numel() // K
+    w, b = _bf16(weight), None if bias is None else _bf16(bias)
+    shape = (*x.shape[:-1], N)
     if out is None:
-        out = torch.empty(x2.shape[0], N, dtype=torch.bfloat16, device=x.device)
-    assert out.shape == (x2.shape[0], N) and out.dtype == torch.bfloat16 and out.is_contiguous()
+        out = torch.empty(shape, dtype=torch.bfloat16, device=x.device)
+    else:
+        assert out.shape == (M, N) and out.dtype == torch.bfloat16 and out.is_contiguous()
     r = None
     if residual is not None:
-        r = residual.reshape(-1, N).contiguous()
-        assert r.shape == out.shape and r.dtype == torch.bfloat16
+        r = residual if residual.is_contiguous() else residual.reshape(-1, N).contiguous()
+        assert r.numel() == M * N and r.dtype == torch.bfloat16
     if workspace is None:
         workspace = _gemm_workspace(x.device)
     with _on_device(x):
-        _capi.check(_capi.load().bsa_linear_bf16(_ptr(x2), _ptr(w), _ptr(b), _ptr(r), _ptr(out), x2.shape[0], N, K,
+        _capi.check(_capi.load().bsa_linear_bf16(_ptr(x2), _ptr(w), _ptr(b), _ptr(r), _ptr(out), M, N, K,
                                                  _ptr(workspace), workspace.numel(), _stream(x)), "linear")
-    return out.view(*x.shape[:-1], N)
+    return out if out.shape == shape else out.view(shape)
 
 
 def tune_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], residual: bool = False,
