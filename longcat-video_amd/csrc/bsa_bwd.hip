@@ -931,10 +931,10 @@ constexpr int kBwdDout = kBwdStages * kBwdHalfTile, kBwdNumbers = 2 * kBwdStages
 constexpr int kBlockBits = 15, kMostLiveHalves = (1 << (32 - kBlockBits)) - 1;
 constexpr int kPlanesAtHand = 4;                             // chunks of less than 512 tokens
 
-// What bounds it is issue: a wavefront has its SIMD to itself and issues one instruction after another, 337 of them a half beside
-// 1 024 clocks of products.  249 are left, with addresses that are scalars and stay so, no division for the list position, constants
-// in the LDS reads, one setting of m0 for four loads, and padded keys that start their chains from -inf instead of a test an
-// element: 4.01 -> 3.74 ms at 32 heads of 24x30x52 (with dS kept), 18.25 -> 17.25 ms at 24x45x80.
+// What bounds it: with every instruction in a slot behind an MFMA (see the step) the matrix pipes are busy 54 % of the clocks at
+// 1.59 GHz, which is what the board's power limit leaves; a wavefront waits 22 % of its time, a quarter of that for LDS.  3.13 ms at 32
+// heads of 24x30x52 with dS kept (3.69 before the slots, 4.01 with 337 instructions a half beside the products, 249 since addresses are
+// scalars, lists are walked without divisions and padded keys start their chains from -inf).
 // kMasked: as in the dQ kernel - without validity words no key is padding and the test is compiled out.
 // kKeep: dS, rounded as for the product, is also written out for bwd_dq_from_ds_kernel (pair_base: bwd_count_kernel's base).
 // what the dK / dV kernel would divide by or divide to get

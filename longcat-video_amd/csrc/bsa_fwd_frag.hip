@@ -21,7 +21,8 @@
 //      = the A operand of O^T (32 d x 32 queries) += V^T . P^T, with the 16 keys of a step in the
 //        order in which the accumulator registers of S^T hold them, so that P^T needs no shuffle.
 //
-// Work decomposition.  One wavefront (a workgroup of 64 threads, one per SIMD) = one work item =
+// Work decomposition.  One wavefront (a workgroup of 64 threads, one per SIMD; of small calls two or four,
+// see kTeam) = one work item =
 // 64 query rows against its list of KV blocks, walked in steps of 32 keys (half a tile).  Per
 // step: 16 MFMAs for S^T of the next step interleaved with the exp2 / row sum / rounding of the
 // current one, then 16 MFMAs for O^T += V^T P^T interleaved with the row maximum of the next.
