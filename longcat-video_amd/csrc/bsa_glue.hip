@@ -1,11 +1,12 @@
 // Glue of the attention module around the block-sparse operator: row RMSNorm,
 // fused per-head QK RMSNorm + 3-D RoPE, and bf16 linear layers (hipBLASLt,
-// a plain library GEMM with bias / residual epilogue).
+// a plain library GEMM with a bias epilogue; a residual is added by a pass of its own).
 #include "bsa_common.h"
 #include "bsa_rope.h"
 
 #include <hipblaslt/hipblaslt.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <shared_mutex>
@@ -275,14 +276,47 @@ __global__ __launch_bounds__(256) void norm_rope_kernel(const T* __restrict__ sr
 }
 
 // ------------------------------------------------------------- linear (GEMM)
+// out = bf16(y + bias + residual) of a product left in fp32, rows of y dense: the sums in fp32 and one rounding, as in a GEMM's
+// epilogue.  kWide: eight elements a thread, everything 16-byte aligned; otherwise one.
+// The library is never asked for the residual itself (beta = 1, C beside D): at 86 400 x 4 096 x 4 096 that product came out with
+// the bias missing from the last two of every 32 rows of a 128 x 128 part in 5 of 4 170 equal calls, and differed from itself in 11
+// of 6 000 without a bias; with beta = 0 none of 29 000 calls did.
+// HBM-bound (6 bytes in and 2 out an element).  us, fp32 product and this pass / product with beta = 1 / the engine's GEMM: 86 400 rows
+// of 4 096 x 4 096 2 693 / 2 094 / 2 831, 24 960 854 / 672 / 901, 2 000 73 / 59 / 132, 256 23 / 19 / 98.
+template <bool kWide>
+__global__ __launch_bounds__(256) void residual_add_kernel(const float* __restrict__ y, const __bf16* bias, const __bf16* residual,
+                                                           __bf16* out, int64_t ldo, uint32_t n, uint32_t per_row) {
+    constexpr int kEach = kWide ? 8 : 1;
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t row = i / per_row, col = (i - row * per_row) * kEach;
+    const int64_t at = row * ldo + col;
+    float v[kEach];
+    __bf16 r[kEach], b[kEach], res[kEach];
+    if constexpr (kWide) {
+        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(y + (uint64_t)i * 8);
+        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(y + (uint64_t)i * 8 + 4);
+        *reinterpret_cast<uint4*>(r) = *reinterpret_cast<const uint4*>(residual + at);
+        if (bias != nullptr) *reinterpret_cast<uint4*>(b) = *reinterpret_cast<const uint4*>(bias + col);
+    } else {
+        v[0] = y[i];
+        r[0] = residual[at];
+        if (bias != nullptr) b[0] = bias[col];
+    }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) res[k] = (__bf16)((bias != nullptr ? v[k] + (float)b[k] : v[k]) + (float)r[k]);
+    if constexpr (kWide) *reinterpret_cast<uint4*>(out + at) = *reinterpret_cast<const uint4*>(res);
+    else out[at] = res[0];
+}
+
 // Shape of a linear call on a device -> the algorithm it runs with: the one bsa_linear_bf16_tune measured to be
 // the fastest, else hipBLASLt's first proposal that fits the workspace (asked for once per shape, not per call).
 struct LinearKey {
     int64_t M, ldx, ldw, ldo;
-    int N, K, bias, residual, device;
+    int N, K, bias, fp32_out, device;
     bool operator<(const LinearKey& o) const {
-        return std::tie(M, ldx, ldw, ldo, N, K, bias, residual, device) <
-               std::tie(o.M, o.ldx, o.ldw, o.ldo, o.N, o.K, o.bias, o.residual, o.device);
+        return std::tie(M, ldx, ldw, ldo, N, K, bias, fp32_out, device) <
+               std::tie(o.M, o.ldx, o.ldw, o.ldo, o.N, o.K, o.bias, o.fp32_out, o.device);
     }
 };
 struct TunedAlgo {
@@ -498,17 +532,10 @@ int bsa_linear_bf16_tune(const void* x, int64_t ldx, const void* w, int64_t ldw,
     return linear_impl(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K, workspace, workspace_bytes, stream, true, default_ms, best_ms);
 }
 
-static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
-                       void* out, int64_t ldo, int64_t M, int N, int K, void* workspace, size_t workspace_bytes,
-                       void* stream, bool tune, float* default_ms, float* best_ms) {
-    if (!x || !w || !out) return set_error(BSA_ERR_BAD_ARG, "linear: null pointer");
-    if (M <= 0 || N <= 0 || K <= 0) return set_error(BSA_ERR_BAD_ARG, "linear: sizes must be positive");
-    if (ldx < K || ldw < K || ldo < N) return set_error(BSA_ERR_BAD_ARG, "linear: a row stride is shorter than its row");
-    // hipBLASLt has been seen to write through the workspace pointer for large problems even when it was
-    // told that there is none, so a workspace is mandatory.  Its best algorithms for the 720p projections
-    // want just under 64 MiB (1.52 PFLOP/s instead of 1.24 with 32 MiB); more brings nothing.
-    if (!workspace || workspace_bytes < ((size_t)64 << 20))
-        return set_error(BSA_ERR_WORKSPACE, "linear: a workspace of at least 64 MiB is required (got %zu bytes)", workspace_bytes);
+// The product itself, bf16 or fp32 out.
+static int lt_product(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, void* out, int64_t ldo, bool fp32_out,
+                      int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream, bool tune, float* default_ms,
+                      float* best_ms) {
     LtState& st = lt_state();
     int device = 0;
     if (hipGetDevice(&device) != hipSuccess) return set_error(BSA_ERR_HIP, "linear: hipGetDevice failed");
@@ -526,7 +553,7 @@ static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, c
     {
         // row-major out[M,N] = x[M,K] . w[N,K]^T  ==  column-major out'(N x M) = w'(K x N)^T . x'(K x M)
         const hipblasOperation_t ta = HIPBLAS_OP_T, tb = HIPBLAS_OP_N;
-        const float alpha = 1.f, beta = residual ? 1.f : 0.f;
+        const float alpha = 1.f, beta = 0.f;
         BSA_LT(hipblasLtMatmulDescCreate(&desc, HIPBLAS_COMPUTE_32F, HIP_R_32F));
         BSA_LT(hipblasLtMatmulDescSetAttribute(desc, HIPBLASLT_MATMUL_DESC_TRANSA, &ta, sizeof(ta)));
         BSA_LT(hipblasLtMatmulDescSetAttribute(desc, HIPBLASLT_MATMUL_DESC_TRANSB, &tb, sizeof(tb)));
@@ -539,11 +566,11 @@ static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, c
         }
         BSA_LT(hipblasLtMatrixLayoutCreate(&la, HIP_R_16BF, K, N, ldw));
         BSA_LT(hipblasLtMatrixLayoutCreate(&lb, HIP_R_16BF, K, M, ldx));
-        BSA_LT(hipblasLtMatrixLayoutCreate(&lc, HIP_R_16BF, N, M, ldo));
+        BSA_LT(hipblasLtMatrixLayoutCreate(&lc, fp32_out ? HIP_R_32F : HIP_R_16BF, N, M, ldo));
         BSA_LT(hipblasLtMatmulPreferenceCreate(&pref));
         const uint64_t wsb = workspace_bytes;
         BSA_LT(hipblasLtMatmulPreferenceSetAttribute(pref, HIPBLASLT_MATMUL_PREF_MAX_WORKSPACE_BYTES, &wsb, sizeof(wsb)));
-        const LinearKey key{M, ldx, ldw, ldo, N, K, bias ? 1 : 0, residual ? 1 : 0, device};
+        const LinearKey key{M, ldx, ldw, ldo, N, K, bias ? 1 : 0, fp32_out ? 1 : 0, device};
         if (!tune) {
             TunedAlgo known;
             bool have = false;
@@ -553,7 +580,7 @@ static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, c
                 if (hit != st.chosen.end() && hit->second.workspace <= workspace_bytes) { known = hit->second; have = true; }
             }
             if (have) {
-                BSA_LT(hipblasLtMatmul(handle, desc, &alpha, w, la, x, lb, &beta, residual ? residual : out, lc, out, lc,
+                BSA_LT(hipblasLtMatmul(handle, desc, &alpha, w, la, x, lb, &beta, out, lc, out, lc,
                                        &known.algo, workspace, workspace_bytes, (hipStream_t)stream));
                 goto done;
             }
@@ -581,7 +608,7 @@ static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, c
                 bool ok = true;
                 for (int r = 0; r < 4 && ok; ++r) {
                     if (r == 1) ok = hipEventRecord(e0, (hipStream_t)stream) == hipSuccess;
-                    ok = ok && hipblasLtMatmul(handle, desc, &alpha, w, la, x, lb, &beta, residual ? residual : out, lc, out, lc,
+                    ok = ok && hipblasLtMatmul(handle, desc, &alpha, w, la, x, lb, &beta, out, lc, out, lc,
                                                &heur[i].algo, workspace, workspace_bytes, (hipStream_t)stream) == HIPBLAS_STATUS_SUCCESS;
                 }
                 float ms = 0.f;
@@ -610,7 +637,7 @@ static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, c
             std::unique_lock<std::shared_mutex> lock(st.mu);
             st.chosen.emplace(key, TunedAlgo{heur[pick].algo, heur[pick].workspaceSize});      // a measured choice stays
         }
-        BSA_LT(hipblasLtMatmul(handle, desc, &alpha, w, la, x, lb, &beta, residual ? residual : out, lc, out, lc,
+        BSA_LT(hipblasLtMatmul(handle, desc, &alpha, w, la, x, lb, &beta, out, lc, out, lc,
                                &heur[pick].algo, workspace, workspace_bytes, (hipStream_t)stream));
     }
 done:
@@ -621,6 +648,59 @@ done:
     if (desc) hipblasLtMatmulDescDestroy(desc);
 #undef BSA_LT
     return rc;
+}
+
+constexpr size_t kLtWorkspace = (size_t)64 << 20;
+
+size_t bsa_linear_bf16_workspace_bytes(int64_t M, int N, int with_residual) {
+    if (M <= 0 || N <= 0) return 0;
+    return kLtWorkspace + (with_residual ? ((size_t)M * N * sizeof(float) + 255) / 256 * 256 + 256 : 0);
+}
+
+static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
+                       void* out, int64_t ldo, int64_t M, int N, int K, void* workspace, size_t workspace_bytes,
+                       void* stream, bool tune, float* default_ms, float* best_ms) {
+    if (!x || !w || !out) return set_error(BSA_ERR_BAD_ARG, "linear: null pointer");
+    if (M <= 0 || N <= 0 || K <= 0) return set_error(BSA_ERR_BAD_ARG, "linear: sizes must be positive");
+    if (ldx < K || ldw < K || ldo < N) return set_error(BSA_ERR_BAD_ARG, "linear: a row stride is shorter than its row");
+    // hipBLASLt has been seen to write through the workspace pointer for large problems even when it was
+    // told that there is none, so a workspace is mandatory.  Its best algorithms for the 720p projections
+    // want just under 64 MiB (1.52 PFLOP/s instead of 1.24 with 32 MiB); more brings nothing.
+    if (!workspace || workspace_bytes < kLtWorkspace)
+        return set_error(BSA_ERR_WORKSPACE, "linear: a workspace of at least 64 MiB is required (got %zu bytes)", workspace_bytes);
+    if (!residual) return lt_product(x, ldx, w, ldw, bias, out, ldo, false, M, N, K, workspace, workspace_bytes, stream, tune, default_ms, best_ms);
+
+    // With a residual the product goes to fp32 behind the library's share of the workspace, as many rows (and columns) at a time
+    // as there is room for: all of them in bsa_linear_bf16_workspace_bytes, in the least workspace of 64 MiB half of it.
+    const size_t fp32_bytes = (size_t)M * N * sizeof(float) + 256;
+    const size_t lt_bytes = workspace_bytes - kLtWorkspace >= std::min(fp32_bytes, kLtWorkspace) ? kLtWorkspace : workspace_bytes / 2;
+    const uintptr_t at = (reinterpret_cast<uintptr_t>(workspace) + lt_bytes + 255) / 256 * 256;
+    float* const y = reinterpret_cast<float*>(at);
+    const int64_t room = std::min<int64_t>((int64_t)((reinterpret_cast<uintptr_t>(workspace) + workspace_bytes - at) / sizeof(float)), (int64_t)1 << 31);
+    const int cols = (int)std::min<int64_t>(N, room);
+    int64_t rows = std::min(M, room / cols);
+    if (rows < M && rows > 256) rows = rows / 256 * 256;
+    const uint16_t *xp = static_cast<const uint16_t*>(x), *wp = static_cast<const uint16_t*>(w), *bp = static_cast<const uint16_t*>(bias),
+                   *rp = static_cast<const uint16_t*>(residual);
+    uint16_t* const op = static_cast<uint16_t*>(out);
+    if (tune) return lt_product(x, ldx, w, ldw, nullptr, y, cols, true, rows, cols, K, workspace, lt_bytes, stream, true, default_ms, best_ms);
+    for (int64_t m = 0; m < M; m += rows)
+        for (int n = 0; n < N; n += cols) {
+            const int64_t mr = std::min(rows, M - m);
+            const int nc = std::min(cols, N - n);
+            const int rc = lt_product(xp + m * ldx, ldx, wp + n * ldw, ldw, nullptr, y, nc, true, mr, nc, K, workspace, lt_bytes, stream, false, nullptr, nullptr);
+            if (rc != BSA_OK) return rc;
+            const uint16_t *b = bp == nullptr ? nullptr : bp + n, *r = rp + m * ldo + n;
+            uint16_t* const o = op + m * ldo + n;
+            const bool wide = nc % 8 == 0 && ldo % 8 == 0 && ((reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(r) | reinterpret_cast<uintptr_t>(o)) & 15u) == 0;
+            const uint32_t per_row = (uint32_t)(wide ? nc / 8 : nc), all = (uint32_t)(mr * per_row);
+            const dim3 grid((unsigned)(((uint64_t)all + 255) / 256)), block(256);
+            if (wide) hipLaunchKernelGGL((residual_add_kernel<true>), grid, block, 0, (hipStream_t)stream, y, (const __bf16*)b, (const __bf16*)r, (__bf16*)o, ldo, all, per_row);
+            else hipLaunchKernelGGL((residual_add_kernel<false>), grid, block, 0, (hipStream_t)stream, y, (const __bf16*)b, (const __bf16*)r, (__bf16*)o, ldo, all, per_row);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return set_error(BSA_ERR_HIP, "linear: residual launch: %s", hipGetErrorString(e));
+        }
+    return BSA_OK;
 }
 
 }  // extern "C"

@@ -30,7 +30,7 @@ import torch
 import torch.nn as nn
 
 from .. import _capi
-from ..block_sparse_attention.bsa_interface import _bsa_3d, _on_device, _ptr, _st, _stream
+from ..block_sparse_attention.bsa_interface import _backward_workspace, _bsa_3d, _on_device, _ptr, _st, _stream
 
 
 class RMSNorm_FP32(nn.Module):
@@ -88,6 +88,15 @@ def _gemm_workspace(device) -> torch.Tensor:
     return ws
 
 
+def _linear_workspace(M: int, N: int, residual: bool, device) -> torch.Tensor:
+    """What a linear of M rows and N columns works in: with a residual also the fp32 product, from torch's allocator for the one
+    call where the card has room for it, and otherwise in groups of rows."""
+    if not residual:
+        return _gemm_workspace(device)
+    need = _capi.load().bsa_linear_bf16_workspace_bytes(M, N, 1)
+    return _backward_workspace(need, 64 << 20, device)
+
+
 def _bf16(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.bfloat16 and t.is_contiguous() else t.to(torch.bfloat16).contiguous()
 
@@ -116,7 +125,7 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
         r = residual if residual.is_contiguous() else residual.reshape(-1, N).contiguous()
         assert r.numel() == M * N and r.dtype == torch.bfloat16
     if workspace is None:
-        workspace = _gemm_workspace(x.device)
+        workspace = _linear_workspace(M, N, r is not None, x.device)
     with _on_device(x):
         _capi.check(_capi.load().bsa_linear_bf16(_ptr(x2), _ptr(w), _ptr(b), _ptr(r), _ptr(out), M, N, K,
                                                  _ptr(workspace), workspace.numel(), _stream(x)), "linear")
@@ -137,7 +146,7 @@ def tune_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     out = torch.empty(x2.shape[0], N, dtype=torch.bfloat16, device=x.device)
     r = torch.zeros_like(out) if residual else None
     if workspace is None:
-        workspace = _gemm_workspace(x.device)
+        workspace = _linear_workspace(x2.shape[0], N, residual, x.device)
     d, best = C.c_float(0), C.c_float(0)
     with _on_device(x):
         n = _capi.load().bsa_linear_bf16_tune(_ptr(x2), K, _ptr(w), K, _ptr(b), _ptr(r), _ptr(out), N, x2.shape[0], N, K,
@@ -375,7 +384,7 @@ class Attention(nn.Module):
     @torch.no_grad()
     def forward(self, x: torch.Tensor, shape=None, num_cond_latents=None, return_kv=False,
                 residual: Optional[torch.Tensor] = None):
-        """attention.py:107-147.  `residual` (extension): added to the projection output inside the GEMM."""
+        """attention.py:107-147.  `residual` (extension): added to the fp32 projection, one rounding."""
         B, N, C = x.shape
         Hn, D = self.num_heads, self.head_dim
         eps = self.q_norm.eps
