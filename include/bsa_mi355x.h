@@ -232,6 +232,13 @@ int bsa_fwd_3d(const bsa_3d_params* p,
                int32_t* idx_out, int32_t* lens_out, void* score_out, void* stream);
 
 /*
+ * How bsa_fwd_3d schedules a call of these sizes on the current device (no counterpart in the reference; for tests and tuning):
+ * out = {work items of 64 query rows, those of the last, partial round, wavefronts that share one of these, parts that its
+ * list is cut into}.  Runs on the host.  bf16 / fp16.
+ */
+int bsa_fwd_3d_last_round(const bsa_3d_params* p, int32_t out[4]);
+
+/*
  * bsa_fwd_3d for a caller that will ask for gradients: the same kernels and the same output bit for bit
  * (_attention_bsa.forward runs one kernel with and without grad and keeps lse, bsa:538-568), plus what the
  * backward needs: lse_out [B, Hn, Tq*Hq*Wq] fp32 in token order (natural log; -inf for a query without keys),

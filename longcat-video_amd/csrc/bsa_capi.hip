@@ -443,6 +443,17 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
 }
 }  // namespace
 
+int bsa_fwd_3d_last_round(const bsa_3d_params* p, int32_t out[4]) {
+    Plan pl;
+    BSA_TRY(make_plan(p, &pl));
+    if (!out) return set_error(BSA_ERR_BAD_ARG, "fwd_3d_last_round: null pointer");
+    if (!pl.frag) return set_error(BSA_ERR_UNSUPPORTED, "fwd_3d_last_round: 16-bit types only");
+    const bool by_half = pl.half_width > 0;
+    const LastRound r = frag_last_round((int64_t)p->B * p->Hn, pl.Sqp, pl.Skp, pl.gk.chunk(), by_half ? pl.half_width : pl.sel_width, by_half, &pl.gq, !pl.cdf);
+    out[0] = r.total; out[1] = r.items; out[2] = r.team; out[3] = r.parts;
+    return BSA_OK;
+}
+
 size_t bsa_workspace_bytes(const bsa_3d_params* p) {
     Plan pl;
     if (make_plan(p, &pl) != BSA_OK) return 0;

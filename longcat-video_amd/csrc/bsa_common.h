@@ -326,8 +326,11 @@ constexpr int kFragQueueWords = 16;
 // takes no row maxima and list here the items whose logits it cannot bound; a last launch computes those.  Its first word
 // counts them: fallback_cleared says that it is zero already.
 // q_grid (optional, with q_rows): the grid whose row table (row_table_ints) q_rows is; tiles without real rows are then left out.
-// part_buf (optional, frag_part_floats() floats): the last, partial round may be cut into parts, merged at the end.
+// part_buf (optional, frag_part_floats() floats, lists of one length): the last, partial round may be cut into parts, merged at the end.
 size_t frag_part_floats(const Grid3& q_grid, int64_t heads);
+// Work items of a call, those of its last, partial round, and how these are shared: `parts` parts of an item, `team` wavefronts a part.
+struct LastRound { int total, items, team, parts; };
+LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, bool halves, const Grid3* q_grid, bool one_length);
 // halves: idx and lens are HalfLists, idx_stride their row pitch (at most 4 096).
 // gate_call (optional): idx and lens are still to be made.
 size_t frag_fallback_ints(int64_t items);

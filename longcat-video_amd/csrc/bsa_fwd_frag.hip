@@ -1370,14 +1370,19 @@ __global__ void frag_zero_kernel(uint32_t* p, int n) {
 // another launch (4 us).  Items of one length behind one whole round, uncut / teams of two / of four: 56 of 8 64.3 / 63.9 / 64.0,
 // of 16 88.9 / 84.6 / 82.7, of 64 225 / 197 / 183; 272 of 8 68.3 / 70.7, of 16 91.7 / 90.0, of 64 231 / 206; 416 of 16 94.2 / 93.0,
 // of 64 232 / 214; behind two, 512 of 16 144.3 / 144.8, of 64 368 / 361.  As many shares as there are wavefronts are not made behind
-// whole rounds: little is gained, and a call by the CDF rule, which is not cut there, gives the bits of one by the top-k rule.
+// whole rounds: little is gained.
+// Lists that may be shorter than their width (the CDF rule's, a caller's: one_length false) are cut where all teams run at once,
+// which pays from two tiles on, and not into more.  Priced by the width, 600 items by the CDF rule became three rounds of teams of
+// four behind kernels that select.  Those / one round of wavefronts, at threshold 0.03, 0.0625, 0.25 and 1, whole operator, us: 600
+// items of 100 blocks 56.1 / 30.4, 63.0 / 35.2, 88.5 / 59.0, 171 / 153; 768 of 256 72.9 / 47.5, 87.4 / 56.2, 148.5 / 126.2, 404 / 410; 640
+// of 320, which no wavefront scores by itself, 76.1 / 53.5, 88.0 / 65.7, 162 / 148, 444 / 454.
 constexpr int kMaxParts = 16, kMaxPartRounds = 2, kMinPartTiles = 10;
 struct Split { int team, parts; };
-static Split choose_split(int items, int list_tiles, int resident, bool is_tail, bool parts_allowed) {
+static Split choose_split(int items, int list_tiles, int resident, bool is_tail, bool one_length) {
     Split best = {1, 1};
     float best_us = 0.f;
-    for (int team = 1; team <= 4 && team <= list_tiles && !(is_tail && team > 1 && items * team >= resident); team *= 2)
-        for (int p = 1; p == 1 || (parts_allowed && p <= kMaxParts && p * team * kMinPartTiles <= list_tiles && (int64_t)items * p * team <= kMaxPartRounds * resident); ++p) {
+    for (int team = 1; team <= 4 && team <= list_tiles && !(is_tail && team > 1 && items * team >= resident) && (one_length || items * team <= resident); team *= 2)
+        for (int p = 1; p == 1 || (one_length && p <= kMaxParts && p * team * kMinPartTiles <= list_tiles && (int64_t)items * p * team <= kMaxPartRounds * resident); ++p) {
             const int groups = resident / team, rounds = (int)(((int64_t)items * p + groups - 1) / groups);
             const float start = team == 2 ? 4.3f : team == 4 ? 5.8f : is_tail && p == 1 ? 0.f : 6.f;
             const float full = (float)items * p / ((float)rounds * groups), tile_us = 1.15f + 1.14f * (full > 0.5f ? full - 0.5f : 0.f);
@@ -1385,6 +1390,38 @@ static Split choose_split(int items, int list_tiles, int resident, bool is_tail,
             if ((team == 1 && p == 1) || us < best_us) { best = {team, p}; best_us = us; }
         }
     return best;
+}
+struct Rounds {
+    int heads_per_span;              // (batch, head)s that one buffer of K reaches
+    bool one_span;
+    int n_live, total, resident, list_tiles, tail;
+    Split split;
+};
+static Rounds plan_rounds(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, bool halves, const Grid3* q_grid, bool one_length) {
+    Rounds r;
+    // The kernel addresses K and V through a buffer of less than 4 GB that starts at the first (batch, head) of a
+    // launch: a launch covers as many heads as fit.  One head always does (fewer than 2^24 keys of 256 B).
+    r.heads_per_span = (int)((((int64_t)1 << 32) - 1) / ((Sk / kTile) * (int64_t)kTileBytes));
+    r.one_span = heads <= r.heads_per_span;
+    // Query tiles without real rows drop out; they would walk their lists for nothing.  A 13x30x53 grid in 4x4x8 chunks has
+    // 448 tiles, 371 of them with rows: 820 -> 727 us for 16 heads in fp16.  (Tiles with at most 32 rows, an eighth of a 30-row
+    // grid's, stay whole: a walk with half of the MFMAs and the same loads took longer per tile, 206 against 179 us a round at
+    // 720p, and a third longer overall where such tiles ran between full ones and put the items of an XCD out of step.)
+    r.n_live = q_grid != nullptr && r.one_span ? live_query_tiles(*q_grid) : (int)(Sq / kTile);
+    r.total = (int)(heads * r.n_live);
+    r.resident = resident_wavefronts();
+    r.list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
+    // The items of the last, partial round are cut when its wavefronts would leave too much of the chip idle (and the exact
+    // kernel reaches every head from one buffer); behind whole rounds and into parts only for lists of one length.
+    r.tail = r.total % r.resident;
+    r.split = {1, 1};
+    if (r.one_span && r.tail > 0 && (one_length || r.total < r.resident))
+        r.split = choose_split(r.tail, r.list_tiles, r.resident, r.total > r.resident, one_length);
+    return r;
+}
+LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, bool halves, const Grid3* q_grid, bool one_length) {
+    const Rounds r = plan_rounds(heads, Sq, Sk, bs_k, idx_stride, halves, q_grid, one_length);
+    return {r.total, r.tail, r.split.team, r.split.parts};
 }
 // floats of the parts' buffer, whatever the length of the lists and whichever device runs the call (a caller asks for the size
 // of a workspace once, for all of its devices): a partial round has no more items than the call, choose_split the limits
@@ -1410,21 +1447,12 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     for (int i = 0; i < 3; ++i) { L.q_st[i] = q_st[i]; L.o_st[i] = o_st[i]; }
     const int per_head = (int)(Sq / kTile);
     const int all_tiles = B * Hn * per_head;
-    const int resident = resident_wavefronts();
     const uint32_t* gate = nullptr;
-    // The kernel addresses K and V through a buffer of less than 4 GB that starts at the first (batch, head) of a
-    // launch: a launch covers as many heads as fit.  One head always does (fewer than 2^24 keys of 256 B).
     const int64_t kv_bh_bytes = (Sk / kTile) * (int64_t)kTileBytes;
-    const int64_t span_limit = ((int64_t)1 << 32) - 1;
-    if (kv_bh_bytes > span_limit) return hipErrorInvalidValue;
-    const int heads_per_span = (int)(span_limit / kv_bh_bytes);
-    const bool one_span = (int64_t)B * Hn <= heads_per_span;
-    // Query tiles without real rows drop out; they would walk their lists for nothing.  A 13x30x53 grid in 4x4x8 chunks has
-    // 448 tiles, 371 of them with rows: 820 -> 727 us for 16 heads in fp16.  (Tiles with at most 32 rows, an eighth of a 30-row
-    // grid's, stay whole: a walk with half of the MFMAs and the same loads took longer per tile, 206 against 179 us a round at
-    // 720p, and a third longer overall where such tiles ran between full ones and put the items of an XCD out of step.)
-    const int n_live = q_grid != nullptr && one_span ? live_query_tiles(*q_grid) : per_head;
-    const int total = B * Hn * n_live;
+    if (kv_bh_bytes > ((int64_t)1 << 32) - 1) return hipErrorInvalidValue;
+    // a buffer for parts comes with lists of one length
+    const auto [heads_per_span, one_span, n_live, total, resident, list_tiles, tail, split] =
+        plan_rounds((int64_t)B * Hn, Sq, Sk, bs_k, idx_stride, halves, q_grid, part_buf != nullptr);
     L.tiles = n_live < per_head ? q_rows + Sq : nullptr;
     L.n_live = n_live;
     L.by_live = divisor(n_live);
@@ -1440,7 +1468,6 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     // the items it has to leave to the other kernel is given, and that kernel can reach every head from one buffer.
     // A short call runs the exact kernel alone: its steps are 3 % longer, but a last launch that finds nothing to do costs 4.7 us.
     Parts parts = {nullptr, 1, 0, divisor(1), divisor(1)};
-    const int list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
     const bool bounded = dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident &&
                          (int64_t)total * list_tiles > (int64_t)kExactRoundTiles * resident;
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
@@ -1471,14 +1498,6 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
             else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, false, __VA_ARGS__);                                         \
         }                                                                                                              \
     } while (0)
-    // The items of the last, partial round are cut when its wavefronts would leave too much of the chip idle (and the exact
-    // kernel reaches every head from one buffer): into parts only where the caller gives a buffer, for lists of one length; into
-    // teams only where there is no other round, so that calls with and without a buffer, with and without the queues, and over
-    // lists of halves and of blocks cut alike.
-    const int tail = total % resident;
-    Split split = {1, 1};
-    if (one_span && tail > 0 && (part_buf != nullptr || total < resident))
-        split = choose_split(tail, list_tiles, resident, total > resident, part_buf != nullptr);
     const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
     // The lists of a call whose workgroups all run at once are made by those that walk them.  The kernels in front / like this, us, density
     // 1/16: 4 heads of 192 blocks (one wavefront an item) 48.1 / 46.1, 4 of 256 64.6 / 64.8, one of 320 (teams of four) 43.7 / 40.0, of 512

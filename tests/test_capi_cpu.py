@@ -251,3 +251,22 @@ def test_workspace_holds_for_devices_of_any_size(cus):
         items, round_ = heads * 64 * frames // 4, 4 * cus
         parts = size(0.0) - size(0.5) + 4 * items + 256                  # its order, its queue
         assert parts >= min(items % round_ * 16, 2 * round_) * 33280
+
+
+def test_lists_of_unknown_length_are_shared_where_all_run_at_once():
+    """A list by the CDF rule may be a sixteenth of its width: its items go to teams of wavefronts only where all teams run at once
+    (1 024 wavefronts without a device), and its last round is not cut into parts.  By the top-k rule the estimate decides."""
+    lib = _capi.load()
+    out = (C.c_int32 * 4)()
+    for heads in range(1, 24):
+        for frames, chunk in ((4, (4, 4, 4)), (13, (4, 4, 8))):
+            prm = _capi.Bsa3dParams(1, heads, 128, _capi.BSA_BF16, frames, 40, 40, frames, 40, 40, *chunk, *chunk, 0, 0.1, 0.5)
+            assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == 0
+            total, items, team, parts = out
+            assert items == total % 1024 and parts == 1 and team in (1, 2, 4) and items * team <= 1024
+            assert team > 1 if total <= 512 else team == 1
+    prm = _capi.Bsa3dParams(1, 6, 128, _capi.BSA_BF16, 4, 40, 40, 4, 40, 40, 4, 4, 4, 4, 4, 4, 100, 0.1, 0.0)
+    assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == 0 and tuple(out) == (600, 600, 4, 1)
+    assert lib.bsa_fwd_3d_last_round(C.byref(prm), None) == _capi.BSA_ERR_BAD_ARG
+    prm.dtype = _capi.BSA_F32
+    assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == _capi.BSA_ERR_UNSUPPORTED
