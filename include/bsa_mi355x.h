@@ -270,6 +270,8 @@ int bsa_fwd_3d_lse(const bsa_3d_params* p,
  *   walked in bsa_visit_order's order by the dQ kernel (fp32 roundings only).  Where it comes to at most 8 GB, the dS
  *   of every pair of tiles is kept in it too and spares the dQ kernel two of its three products; a workspace of
  *   bsa_bwd_workspace_least_bytes() has no room for that and is accepted all the same.
+ *   Gradients may be stored over the inputs (dk over k, dv over v); over k in another place than its own rows, from a copy of it
+ *   and without the kept dS.
  */
 size_t bsa_bwd_workspace_least_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int D, int bs_q, int bs_k, int idx_stride, int dtype);
 size_t bsa_bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int D, int bs_q, int bs_k, int idx_stride, int dtype);
@@ -286,7 +288,7 @@ int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const vo
  *   bf16 / fp16, D == 128, 16-byte aligned; lse [B, Hn, Tq*Hq*Wq] fp32 contiguous and idx [B, Hn, nbq, idx_stride],
  *   lens [B, Hn, nbq] as bsa_fwd_3d_lse returned them (blocks counted in the padded chunk grids).  p->k_sel is not
  *   read; p->cdf_threshold > 0 says that the lists differ in length, which only decides how the dQ kernel is launched.
- *   Padded keys give and get no gradient; dq, dk, dv are written at every token.
+ *   Padded keys give and get no gradient; dq, dk, dv are written at every token.  They may lie over the inputs, as bsa_bwd's.
  *   workspace: bsa_bwd_3d_workspace_bytes() bytes, 256-byte aligned: blocked-order copies of q, v and d_o (the kernels
  *   stream their tiles as they lie in memory), the row tables of both grids, and bsa_bwd's workspace.  One pass makes
  *   the copies, the scaled k, delta and the tables from the tensors where they lie, and the kernels store the gradient

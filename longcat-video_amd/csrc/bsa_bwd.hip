@@ -157,7 +157,8 @@ struct BwdStore {
     int64_t sB, sH, sS;
     int Hn;
 };
-// Where the kernels read k and v: element strides (in blocked order as in token order).
+// Where the dK / dV kernel reads k and v: element strides; rows by token or, with rows_by_slot, by slot (the same where no row table is
+// stored through).
 struct BwdLoad {
     const void* p;
     int64_t sB, sH, sS;
@@ -952,7 +953,7 @@ __global__ __launch_bounds__(128 * kGroups, 1) void bwd_dkdv_kernel(const T* __r
                                                        const uint32_t* __restrict__ bits,
                                                        const uint64_t* __restrict__ tile_valid, T* __restrict__ dk,
                                                        T* __restrict__ dv, int64_t Sq, int64_t Sk, int words, float ks_scale,
-                                                       float dk_scale, const int32_t* __restrict__ order, int n_items, int round,
+                                                       float dk_scale, int rows_by_slot, const int32_t* __restrict__ order, int n_items, int round,
                                                        BwdStore dk_to, BwdStore dv_to, char* __restrict__ ds_out,
                                                        char* __restrict__ ds_spare, const int32_t* __restrict__ unit_base, int64_t pairs_per_head, DkdvSizes sz,
                                                        LiveHalves q_live, const int32_t* __restrict__ k_live,
@@ -1013,7 +1014,7 @@ __global__ __launch_bounds__(128 * kGroups, 1) void bwd_dkdv_kernel(const T* __r
     // product is one chain of dependent loads, not two.
     V8 k_rows[8], v_rows[8];
     {
-        const int64_t at_row = max(key_row, (int64_t)0);
+        const int64_t at_row = rows_by_slot ? krow0 + 32 * wave + lr : max(key_row, (int64_t)0);
         const int batch = head / dk_to.Hn, in_batch = head - batch * dk_to.Hn;
         const T* kp = static_cast<const T*>(k_from.p) + batch * k_from.sB + in_batch * k_from.sH + at_row * k_from.sS + 8 * lh;
         const T* vp = static_cast<const T*>(v_from.p) + batch * v_from.sB + in_batch * v_from.sH + at_row * v_from.sS + 8 * lh;
@@ -1444,10 +1445,10 @@ size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int 
 hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,
                       const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv,
                       int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
-                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw, bool unequal) {
+                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw, bool unequal, bool read_copies) {
     const size_t bh = (size_t)B * Hn;
     KeptDs kept = plan_ds((int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
-    kept.keep = kept.keep && bwd_ws(kept, (int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride).total <= workspace_bytes;
+    kept.keep = kept.keep && !read_copies && bwd_ws(kept, (int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride).total <= workspace_bytes;
     const BwdWs at = bwd_ws(kept, (int64_t)bh, Sq, Sk, bs_q, bs_k, idx_stride);
     char* ws = static_cast<char*>(workspace);
     char* ks = ws + at.ks;
@@ -1498,6 +1499,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     const float c = sm_scale * kRcpLn2;
     BwdStore dq_to = {nullptr, 0, 0, 0, Hn}, dk_to = dq_to, dv_to = dq_to;
     BwdLoad k_from = {k, Hn * Sk * kD, Sk * kD, kD}, v_from = {v, Hn * Sk * kD, Sk * kD, kD};
+    float rows_scale = c;            // what makes k_s of the rows at k_from
     if (thw != nullptr) {
         dq_to = {thw->q_rows, thw->dq_st[0], thw->dq_st[1], thw->dq_st[2], Hn};
         dk_to = {thw->k_rows, thw->dk_st[0], thw->dk_st[1], thw->dk_st[2], Hn};
@@ -1505,6 +1507,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         dq = thw->dq; dk = thw->dk; dv = thw->dv;
         k_from = {thw->k, thw->k_st[0], thw->k_st[1], thw->k_st[2]};
         v_from = {thw->v, thw->v_st[0], thw->v_st[1], thw->v_st[2]};
+        if (read_copies) v_from = {thw->v_blocked, Hn * Sk * kD, Sk * kD, kD};
         q = thw->q_blocked; v = thw->v_blocked; dout = thw->dout_blocked;
         BwdPrep a = {};
         a.gq = thw->gq; a.gk = thw->gk; a.Hn = Hn;
@@ -1539,6 +1542,10 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
         else hipLaunchKernelGGL((bwd_scale_kernel<_Float16>), dim3((unsigned)((krows * 16 + 255) / 256)), dim3(256), 0, st,
                                 (const _Float16*)k, (_Float16*)ks, c, krows * 16, tile_valid, (uint32_t)Sk);
     }
+    if (read_copies) {
+        k_from = {ks, Hn * Sk * kD, Sk * kD, kD};
+        rows_scale = 1.f;
+    }
     if (thw == nullptr) hipLaunchKernelGGL(bwd_zero_kernel, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, st, bits, nwords);
     const int64_t lrows = (int64_t)bh * nbq;
     // dQ walks every list in the forward kernel's visiting order when the list is ascending (a selection in block
@@ -1558,7 +1565,7 @@ hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o
     const int total_q = (int)(bh * (Sq / kTile)), total_k = (int)(bh * (Sk / kTile));
 #define BSA_DKDV(T, M, K, G)                                                                                                           \
     hipLaunchKernelGGL((bwd_dkdv_kernel<T, M, K, G>), dim3((unsigned)total_k), dim3(128 * G), bwd_dkdv_lds_bytes(nbq, G), st, (const T*)q, (const T*)dout, k_from, v_from,  \
-                       m2, delta, bits, tile_valid, (T*)dk, (T*)dv, Sq, Sk, words, c, sm_scale, order, total_k, round,  \
+                       m2, delta, bits, tile_valid, (T*)dk, (T*)dv, Sq, Sk, words, rows_scale, sm_scale, read_copies ? 1 : 0, order, total_k, round,  \
                        dk_to, dv_to, ws + at.ds, ws + at.ds_spare, base, kept.pairs_per_head, sizes, q_live, k_live, counts)
 #define BSA_DQ(T, M)                                                                                                                   \
     hipLaunchKernelGGL((bwd_dq_lds_kernel<T, M>), dim3(end - first), block, kDqRingLds, st, (const T*)q, (const T*)dout, (const T*)ks, (const T*)v,  \

@@ -343,6 +343,30 @@ size_t bsa_bwd_workspace_least_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int 
                ? 0 : bwd_workspace_bytes(B, Hn, Sq, Sk, bs_q, bs_k, idx_stride, true);
 }
 
+// The memory of a [B, Hn, S, 128] tensor of 16-bit elements.
+struct Span {
+    const void* p;
+    int64_t st[3];
+    uintptr_t lo, hi;
+    Span(const void* t, const int64_t strides[3], int64_t B, int64_t Hn, int64_t S) : p(t) {
+        int64_t first = 0, last = 128;
+        const int64_t most[3] = {B - 1, Hn - 1, S - 1};
+        for (int i = 0; i < 3; ++i) {
+            st[i] = strides[i];
+            (strides[i] < 0 ? first : last) += most[i] * strides[i];
+        }
+        lo = reinterpret_cast<uintptr_t>(t) + (uintptr_t)(first * 2);
+        hi = reinterpret_cast<uintptr_t>(t) + (uintptr_t)(last * 2);
+    }
+    bool meets(const Span& o) const { return lo < o.hi && o.lo < hi; }
+    bool same(const Span& o) const { return p == o.p && st[0] == o.st[0] && st[1] == o.st[1] && st[2] == o.st[2]; }
+};
+// The dK / dV kernel reads the rows of `in` (k or v) as it comes to them.  dk and dv may be the tensor itself, whose rows are read by
+// the workgroup that stores them; any other overlap, and one with dq, which may be stored in front, needs a copy.
+static bool needs_copy(const Span& in, const Span& dq, const Span& dk, const Span& dv) {
+    return in.meets(dq) || (in.meets(dk) && !in.same(dk)) || (in.meets(dv) && !in.same(dv));
+}
+
 int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o, const float* lse,
             const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv, int B,
             int Hn, int64_t Sq, int64_t Sk, int D, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
@@ -357,8 +381,10 @@ int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const vo
         return set_error(BSA_ERR_BAD_ARG, "bwd: tensors must be 16-byte aligned, the workspace 256-byte aligned");
     const size_t need = bwd_workspace_bytes(B, Hn, Sq, Sk, bs_q, bs_k, idx_stride, true);
     if (workspace_bytes < need) return set_error(BSA_ERR_WORKSPACE, "bwd: workspace of %zu bytes, %zu needed", workspace_bytes, need);
+    const int64_t q_st[3] = {(int64_t)Hn * Sq * D, Sq * D, D}, k_st[3] = {(int64_t)Hn * Sk * D, Sk * D, D};
+    const bool read_copies = needs_copy(Span(k, k_st, B, Hn, Sk), Span(dq, q_st, B, Hn, Sq), Span(dk, k_st, B, Hn, Sk), Span(dv, k_st, B, Hn, Sk));
     const hipError_t e = launch_bwd(q, k, v, o, d_o, lse, idx, lens, tile_valid, dq, dk, dv, B, Hn, Sq, Sk, bs_q, bs_k, idx_stride,
-                                    sm_scale, dtype, workspace, workspace_bytes, (hipStream_t)stream);
+                                    sm_scale, dtype, workspace, workspace_bytes, (hipStream_t)stream, nullptr, false, read_copies);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "bwd launch");
 }
 
@@ -978,9 +1004,13 @@ int bsa_bwd_3d(const bsa_3d_params* p, const void* q, const int64_t q_strides[3]
         t.q_st[i] = q_strides[i]; t.k_st[i] = k_strides[i]; t.v_st[i] = v_strides[i]; t.o_st[i] = o_strides[i]; t.do_st[i] = do_strides[i];
         t.dq_st[i] = dq_strides[i]; t.dk_st[i] = dk_strides[i]; t.dv_st[i] = dv_strides[i];
     }
+    const int64_t nq = (int64_t)p->Tq * p->Hq * p->Wq, nk = (int64_t)p->Tk * p->Hk * p->Wk;
+    const Span dq_at(dq, dq_strides, p->B, p->Hn, nq), dk_at(dk, dk_strides, p->B, p->Hn, nk), dv_at(dv, dv_strides, p->B, p->Hn, nk);
+    const bool read_copies = needs_copy(Span(k, k_strides, p->B, p->Hn, nk), dq_at, dk_at, dv_at) ||
+                             needs_copy(Span(v, v_strides, p->B, p->Hn, nk), dq_at, dk_at, dv_at);
     const hipError_t e = launch_bwd(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, idx, lens, kv_padded(p) ? t.valid : nullptr, nullptr, nullptr, nullptr,
                                     p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype,
-                                    ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t, p->cdf_threshold > 0.f);
+                                    ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t, p->cdf_threshold > 0.f, read_copies);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "bwd_3d launch");
 }
 

@@ -349,17 +349,18 @@ struct BwdThw {
     const void *q, *k, *v, *o, *dout;
     int64_t q_st[3], k_st[3], v_st[3], o_st[3], do_st[3];
     const float* lse;                 // [B * Hn][tokens]
-    void *q_blocked, *v_blocked, *dout_blocked;      // B * Hn * Sq (v: Sk) rows of 128 elements
+    void *q_blocked, *v_blocked, *dout_blocked;      // B * Hn * Sq (v: Sk) rows of 128 elements; v where dS is not kept
     int32_t *q_rows, *k_rows;         // Sq and Sk entries
     uint64_t* valid;                  // Sk / 64 words
     void* dq; int64_t dq_st[3];
     void* dk; int64_t dk_st[3];
     void* dv; int64_t dv_st[3];
 };
-// unequal: the lists may differ much in length (for the schedule of dQ alone).
+// unequal: the lists may differ much in length (for the schedule of dQ alone).  read_copies: a gradient is stored over k (with thw: or
+// v) before the dK / dV kernel has read all of it, which then reads k_s and v in blocked order from the workspace; dS is not kept.
 hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* dout, const float* lse,
                       const int32_t* idx, const int32_t* lens, const uint64_t* tile_valid, void* dq, void* dk, void* dv,
                       int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype,
-                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw = nullptr, bool unequal = false);
+                      void* workspace, size_t workspace_bytes, hipStream_t st, const BwdThw* thw = nullptr, bool unequal = false, bool read_copies = false);
 
 }  // namespace bsa
