@@ -289,10 +289,11 @@ int bsa_bwd(const void* q, const void* k, const void* v, const void* o, const vo
  *   lens [B, Hn, nbq] as bsa_fwd_3d_lse returned them (blocks counted in the padded chunk grids).  p->k_sel is not
  *   read; p->cdf_threshold > 0 says that the lists differ in length, which only decides how the dQ kernel is launched.
  *   Padded keys give and get no gradient; dq, dk, dv are written at every token.  They may lie over the inputs, as bsa_bwd's.
- *   workspace: bsa_bwd_3d_workspace_bytes() bytes, 256-byte aligned: blocked-order copies of q, v and d_o (the kernels
- *   stream their tiles as they lie in memory), the row tables of both grids, and bsa_bwd's workspace.  One pass makes
- *   the copies, the scaled k, delta and the tables from the tensors where they lie, and the kernels store the gradient
- *   rows at their tokens: five of the eight rearrangements a caller of bsa_bwd would run are not made.
+ *   workspace: bsa_bwd_3d_workspace_bytes() bytes, 256-byte aligned: blocked-order copies of q and d_o (the kernels
+ *   stream their tiles as they lie in memory), the row tables of both grids, and bsa_bwd's workspace; in less than that, down to
+ *   bsa_bwd_3d_workspace_least_bytes(), a copy of v in the place of the kept dS.  One pass makes the copies, the scaled k, delta and
+ *   the tables from the tensors where they lie, and the kernels store the gradient rows at their tokens: the rearrangements a caller
+ *   of bsa_bwd would run are not made.
  */
 size_t bsa_bwd_3d_workspace_least_bytes(const bsa_3d_params* p, int idx_stride);      /* without the kept dS */
 size_t bsa_bwd_3d_workspace_bytes(const bsa_3d_params* p, int idx_stride);

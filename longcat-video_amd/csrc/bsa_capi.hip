@@ -2,6 +2,7 @@
 // sequencing.  Nothing here allocates device memory or waits for the GPU.
 #include "bsa_common.h"
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <cmath>
@@ -948,14 +949,19 @@ int make_bwd3d_plan(const bsa_3d_params* p, int idx_stride, Bwd3dPlan* pl) {
     size_t off = 0;
     auto take = [&](size_t bytes) { const size_t o = off; off += up256(bytes); return o; };
     pl->off_qp = take(bh * pl->Sqp * row);
-    pl->off_vp = take(bh * pl->Skp * row);
     pl->off_dop = take(bh * pl->Sqp * row);
     pl->off_qrows = take((size_t)pl->Sqp * sizeof(int32_t));
     pl->off_krows = take((size_t)pl->Skp * sizeof(int32_t));
     pl->off_valid = take((size_t)(pl->Skp / 64) * sizeof(uint64_t));
+    // Behind them bsa_bwd's workspace: with the dS of all pairs, or without it and with v in blocked order.  In `total` the first has
+    // room, in less, down to `least`, only the second.
     pl->off_bwd = off;
-    pl->least = off + up256(bwd_workspace_bytes(p->B, p->Hn, pl->Sqp, pl->Skp, pl->gq.chunk(), pl->gk.chunk(), idx_stride, true));
-    pl->total = off + up256(bwd_workspace_bytes(p->B, p->Hn, pl->Sqp, pl->Skp, pl->gq.chunk(), pl->gk.chunk(), idx_stride));
+    const size_t scratch = bwd_workspace_bytes(p->B, p->Hn, pl->Sqp, pl->Skp, pl->gq.chunk(), pl->gk.chunk(), idx_stride, true);
+    const size_t most = bwd_workspace_bytes(p->B, p->Hn, pl->Sqp, pl->Skp, pl->gq.chunk(), pl->gk.chunk(), idx_stride);
+    take(scratch);
+    pl->off_vp = take(bh * pl->Skp * row);
+    pl->least = off;
+    pl->total = most > scratch ? std::max(pl->off_bwd + up256(most), off + 256) : off;
     return BSA_OK;
 }
 }  // namespace
@@ -1010,7 +1016,7 @@ int bsa_bwd_3d(const bsa_3d_params* p, const void* q, const int64_t q_strides[3]
                              needs_copy(Span(v, v_strides, p->B, p->Hn, nk), dq_at, dk_at, dv_at);
     const hipError_t e = launch_bwd(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, idx, lens, kv_padded(p) ? t.valid : nullptr, nullptr, nullptr, nullptr,
                                     p->B, p->Hn, pl.Sqp, pl.Skp, pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype,
-                                    ws + pl.off_bwd, workspace_bytes - pl.off_bwd, st, &t, p->cdf_threshold > 0.f, read_copies);
+                                    ws + pl.off_bwd, (workspace_bytes >= pl.total ? workspace_bytes : pl.off_vp) - pl.off_bwd, st, &t, p->cdf_threshold > 0.f, read_copies);
     return e == hipSuccess ? BSA_OK : hip_fail(e, "bwd_3d launch");
 }
 

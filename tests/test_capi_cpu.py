@@ -270,3 +270,21 @@ def test_lists_of_unknown_length_are_shared_where_all_run_at_once():
     assert lib.bsa_fwd_3d_last_round(C.byref(prm), None) == _capi.BSA_ERR_BAD_ARG
     prm.dtype = _capi.BSA_F32
     assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == _capi.BSA_ERR_UNSUPPORTED
+
+
+def test_backward_workspace_holds_v_only_without_the_kept_ds():
+    """With dS kept no kernel reads v in blocked order: beside bsa_bwd's workspace there are q, dO and the tables; a workspace of the
+    least size has v in the place of dS, and is always smaller."""
+    lib = _capi.load()
+    for heads, grid, width in ((32, (24, 30, 52), 78), (1, (4, 4, 4), 1), (3, (5, 9, 13), 4), (32, (24, 45, 80), 90)):
+        prm = C.byref(_capi.Bsa3dParams(1, heads, 128, _capi.BSA_BF16, *grid, *grid, 4, 4, 4, 4, 4, 4, 0, 0.1, 0.0))
+        S = lib.bsa_padded_tokens(*grid, 4, 4, 4)
+        total, least = lib.bsa_bwd_3d_workspace_bytes(prm, width), lib.bsa_bwd_3d_workspace_least_bytes(prm, width)
+        sizes = (1, heads, S, S, 128, 64, 64, width, _capi.BSA_BF16)
+        most, scratch = lib.bsa_bwd_workspace_bytes(*sizes), lib.bsa_bwd_workspace_least_bytes(*sizes)
+        own = 2 * heads * S * 256 + 2 * 4 * S + S // 8 + 6 * 256
+        assert scratch + heads * S * 256 <= least <= scratch + heads * S * 256 + own
+        if most == scratch:                       # 24x45x80: more than is kept
+            assert total == least
+        else:
+            assert least < total <= max(most + own, least + 256)
