@@ -142,7 +142,9 @@ static_assert(kTeamBytes<4> <= 160 * 1024 && 2 * (kTeamBytes<2> + 512) <= 160 * 
 // roundings, the same lists), in front of its walk: the scores of its block against every key block, a share of 32 of them to a
 // wavefront at a time, then the first wavefront selects and orders.  Instead of another launch, its start and its end.
 // Whole operator, us, with gate_kernel in front / like this: 2 heads of 16x22x12 23.0 / 19.9, 4 of 9x13x10 30.2 / 26.3, two prompts of
-// 13 heads of 7x8x8 24.2 / 21.6, of 8 heads of 7x15x26 40.3 / 38.2.
+// 13 heads of 7x8x8 24.2 / 21.6, of 8 heads of 7x15x26 40.3 / 38.2.  `fallback` and `fallback_count` are then where the lists
+// ([BH][nbq][width]) and their lengths go, null: nowhere.  (As arguments of their own they would be 392 bytes, beyond what is asked for
+// together, and two arguments that the kernel can do without in their place cost the layers 0.3 to 0.7 %, by where the loop then lies.)
 struct FragGate {
     const uint16_t *qc, *kc;         // chunk means, 16-bit storage
     int nbk, width;                  // entries of a list: the top-k rule's count, the most of the CDF rule's
@@ -211,7 +213,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
     const uint32_t lane_off = (uint32_t)lane * 16u;
     // the kernel that runs the fallback list takes as many items as the list holds
     const int n_launch = kBounded ? item_end - item_begin : parts.count > 1 ? parts.count * parts.items
-                                  : (fallback_count != nullptr ? __builtin_amdgcn_readfirstlane((int)min(*fallback_count, (uint32_t)(item_end - item_begin)))
+                                  : (!kGate && fallback_count != nullptr ? __builtin_amdgcn_readfirstlane((int)min(*fallback_count, (uint32_t)(item_end - item_begin)))
                                                                : item_end - item_begin);
 
     const int64_t kv_bh_bytes = (int64_t)tiles_bh * kTileBytes;
@@ -736,7 +738,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                     else if (G.nbk <= 128) k_sel = select(std::integral_constant<int, 2>{});
                     else if (kTeam == 1 || G.nbk <= 256) k_sel = select(std::integral_constant<int, 4>{});
                     else k_sel = select(std::integral_constant<int, 8>{});
-                    int32_t* const dst = idx != nullptr ? const_cast<int32_t*>(idx) + brow * G.width : nullptr;
+                    int32_t* const dst = fallback != nullptr ? fallback + brow * G.width : nullptr;
                     wave_sync();
                     const int32_t* order_here = list;
                     if (k_sel > kPaceWidth) order_here = pace_row(list, k_sel, k_sel, G.nbk, lane, dst, G.by_span);
@@ -744,7 +746,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                         for (int e = lane; e < k_sel; e += 64) dst[e] = list[e];
                     if (dst != nullptr)
                         for (int e = k_sel + lane; e < G.width; e += 64) dst[e] = -1;
-                    if (lens != nullptr && lane == 0) const_cast<int32_t*>(lens)[brow] = k_sel;
+                    if (fallback_count != nullptr && lane == 0) fallback_count[brow] = (uint32_t)k_sel;
                     int total = k_sel;
                     if constexpr (kWalk == kHalves) total = expand_list(order_here, k_sel, nsub_of_block, halves_list, lane, [&](int tile) { return (int)counts[tile]; });
                     if (lane == 0) {
@@ -1473,6 +1475,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
     FragGate here = {};
+    int32_t* gate_lists = nullptr;      // with `here`: where the lists that the kernel makes go
+    uint32_t* gate_lens = nullptr;
 #define BSA_FRAG_LAUNCH_T(T, WALK, BD, TEAM, GATE, grid, begin, end, ord, que, want, bh0, span, fbl, fbc)                           \
     hipLaunchKernelGGL((fwd_frag_kernel<T, WALK, BD, TEAM, GATE>), grid, dim3(TEAM > 1 ? 64 * TEAM : 64), 0, st, (const T*)q, (const char*)kf, (const char*)vf, idx, \
                        lens, tile_valid, (T*)o, lse, Sq, Sk, bs_q, bs_k, idx_stride, qk_scale, begin, end, TEAM > 0 ? kOneRound : resident, Hn, lse_rows, \
@@ -1509,8 +1513,9 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
             gate_here_bytes(c.nbk, c.width, nsub, halves) <= kTile * (kD + 8) * 2) {
             here = {static_cast<const uint16_t*>(c.q_cmp), static_cast<const uint16_t*>(c.k_cmp), c.nbk, c.width, c.threshold, c.scale, c.k_min,
                     pace_divisor(c.nbk, c.width)};
-            idx = c.lists;
-            lens = c.lens;
+            gate_lists = c.lists;
+            gate_lens = reinterpret_cast<uint32_t*>(c.lens);
+            idx = lens = nullptr;
             if (halves) tile_valid = c.valid;
         } else {
             const hipError_t e = c.make(c.ctx);
@@ -1549,7 +1554,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         if (split.parts > 1) parts = {part_buf, split.parts, tail, divisor(split.parts), divisor(tail)};
         const int n = (total - whole) * split.parts;
         const dim3 grid((unsigned)(split.team == 1 && n > resident ? resident : n));
-#define BSA_FRAG_TAIL grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, (int32_t*)nullptr, (uint32_t*)nullptr
+#define BSA_FRAG_TAIL grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, gate_lists, gate_lens
         if (split.team == 4) BSA_FRAG_LAUNCH_ONCE(4, BSA_FRAG_TAIL);
         else if (split.team == 2) BSA_FRAG_LAUNCH_ONCE(2, BSA_FRAG_TAIL);
         else if (once) BSA_FRAG_LAUNCH_ONCE(1, BSA_FRAG_TAIL);
