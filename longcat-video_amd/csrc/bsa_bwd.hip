@@ -1,7 +1,7 @@
-// Block-sparse flash-attention backward for gfx950 (bf16 / fp16 MFMA).  The kernels work on blocked-order q, k_s, v,
-// dO; the caller's tensors are either in blocked order too (launch_bwd without `thw`) or in (T, H, W) token order, in
-// which case the two small passes read o, dO, lse and k through row tables and the kernels store every gradient row
-// at its token (BwdThw, BwdStore).
+// Block-sparse flash-attention backward for gfx950 (bf16 / fp16 MFMA).  The kernels walk q and dO in blocked order.  The caller's
+// tensors are either in blocked order too (launch_bwd without `thw`: small passes make delta, M2 and k_s) or in (T, H, W) token
+// order, where one pass (bwd_prepare_kernel) makes what they need of the tensors where these lie, the real rows of a ragged chunk
+// in front of its padding, and the kernels store every gradient row at its token (BwdThw, BwdStore).
 //
 // Follows the reference's backward (bsa_interface.py:341-461; kernels flash_attn_bsa_varlen_mask.py:288-360
 // for dK/dV and :428-462 for dQ, wrappers :630-642 and :943-945) with the same rounding points:
@@ -11,18 +11,19 @@
 //   ds = p * (dp - delta) rounded to the storage type, p rounded to the storage type for dV;
 //   dV = sum p^T do,  dK = sm_scale * sum ds^T q,  dQ = ln 2 * sum ds k_s  (fp32 accumulators, one final rounding).
 //
-// Data movement: k (pre-scaled) and v, q and dO are read as they lie in memory, in blocked order, through LDS
-// (global_load_lds_dwordx4): no fragment-order copies.  Row fragments (A operand whose rows are tokens) come out of
-// LDS with ds_read_b128, transposed ones (A operand whose rows are head-dim columns, contraction over 16 tokens in
-// accumulator order) with ds_read_b64_tr_b16.
+// Data movement.  dK / dV: k and v rows from where the caller has them (BwdLoad) into registers, scaled there; q and dO in blocked order
+// through LDS (global_load_lds_dwordx4): row fragments (A operand whose rows are tokens) come out of it with ds_read_b128,
+// transposed ones (A operand whose rows are head-dim columns, contraction over 16 tokens in accumulator order) with
+// ds_read_b64_tr_b16.  dQ from kept dS: k_s as transposed fragments, written once by the pass in front, straight into registers.
+// dQ from scratch: k_s and v in blocked order through LDS, q and dO rows in registers.
 //
-// dQ: one wavefront per 64 query rows (two halves of 32, so that every K_s and V fragment feeds two MFMAs).
+// dQ from scratch: one wavefront per 64 query rows (two halves of 32, so that every K_s and V fragment feeds two MFMAs).
 // S^T = K_s Q^T and dP^T = V dO^T (Q and dO rows in registers as B operands) put one query per lane, so M2 and
 // delta are one scalar per lane and dS^T in the accumulator registers is already the B operand of
 // dQ^T += K_s^T dS^T.
 // dK, dV: one kernel, a workgroup of two wavefronts per 64 keys.  S = Q K_s^T and dP = dO V^T (K_s and V rows in
 // registers as B operands) put one key per lane; P and dS in the accumulator registers are the B operands of
-// dV^T += dO^T P and dK^T += Q^T dS.  Q and dO are read as they lie in memory, through LDS (see that kernel).
+// dV^T += dO^T P and dK^T += Q^T dS.
 // Where its dS fits in memory the dK / dV kernel runs first and keeps it, and dQ is one product instead of three
 // (bwd_dq_from_ds_kernel).
 // The query blocks of a KV block come from a bit matrix [KV block][query block] that a small kernel fills from
@@ -113,8 +114,8 @@ __device__ __forceinline__ void put_turned_row(char* lds, int row, int c16, cons
     const int r = row & 31, f = ((r & 3) << 2) | ((r >> 2) & 3);
     *reinterpret_cast<uint4*>(lds + (row >> 5) * kBwdHalfTileBytes + r * 256 + ((c16 ^ f) << 4)) = x;
 }
-// The lane's offset of the first (hi: second) four keys of a fragment of d tile t in a half that lies like this; 4096 further per
-// step of 16 keys.
+// The lane's offset of the first (hi: second) four rows of a transposed fragment of d tile t in a half that lies like this; 4096
+// further per step of 16 rows.
 __device__ __forceinline__ uint32_t turned_offset(int lane, int t, int hi) {
     const int lh = lane >> 5, s16 = lane & 15, g1 = (lane >> 4) & 1, tx = s16 >> 2, ty = (s16 & 3) >> 1, tz = s16 & 1;
     return (uint32_t)((4 * lh + tx + 8 * hi) * 256) + ((((uint32_t)(4 * t + 2 * g1 + ty)) ^ (uint32_t)((4 * tx) | (lh + 2 * hi))) << 4) +
@@ -579,7 +580,7 @@ __global__ __launch_bounds__(64) void bwd_dq_lds_kernel(const T* __restrict__ q,
 #pragma unroll
     for (int c = 0; c < 8; ++c) roff[c] = (uint32_t)(lr * 256) + ((((uint32_t)(2 * c + lh)) ^ fl) << 4);
     const int s16 = lane & 15, g1 = (lane >> 4) & 1, tx = s16 >> 2, ty = (s16 & 3) >> 1, tz = s16 & 1;
-    uint32_t toff[4][2];
+    uint32_t toff[4][2];                         // turned_offset, written out: as a call the kernels came out 0.3 % slower in small clips
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -1125,7 +1126,7 @@ __global__ __launch_bounds__(128 * kGroups, 1) void bwd_dkdv_kernel(const T* __r
 #pragma unroll
     for (int c = 0; c < 8; ++c) roff[c] = lds0 + (uint32_t)(lr * 256) + ((((uint32_t)(2 * c + lh)) ^ fl) << 4);
     const int s16 = lane & 15, g1 = (lane >> 4) & 1, tx = s16 >> 2, ty = (s16 & 3) >> 1, tz = s16 & 1;
-    uint32_t toff[4][2];
+    uint32_t toff[4][2];                         // turned_offset, written out
 #pragma unroll
     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -1398,7 +1399,7 @@ static KeptDs plan_ds(int64_t bh, int64_t Sq, int64_t Sk, int bs_q, int bs_k, in
 
 // The pieces of the backward's workspace.
 struct BwdWs {
-    size_t ks, delta, m2, bits, paced, counts, order;      // k_s in blocked order; delta and M2; the bit matrix; the lists in the dQ
+    size_t ks, delta, m2, bits, paced, counts, order;      // k_s, with kept dS in transposed fragments, otherwise in blocked order; delta and M2; the bit matrix; the lists in the dQ
                                                            // kernel's visiting order; per KV block its number of query halves; the KV
                                                            // tiles of every head by that number
     size_t q_live, k_live, planes;                         // LiveHalves of both grids (token order, where they are padded)

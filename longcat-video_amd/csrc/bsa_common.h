@@ -340,8 +340,8 @@ size_t frag_fallback_ints(int64_t items);
 // those with `least` (then dS is not kept between the kernels and dQ is computed from scratch).
 size_t bwd_workspace_bytes(int B, int Hn, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride, bool least = false);
 int bwd_max_query_blocks();      // the dK / dV kernel stages a KV block's query blocks in LDS: Sq / bs_q may not exceed this
-// With `thw` the caller's tensors are in token order: a pass in front brings q, v, dO and k_s into blocked order, with the row
-// tables (token of every blocked-order slot of one (batch, head), -1 = padding) and the validity words, and the kernels store
+// With `thw` the caller's tensors are in token order: a pass in front brings q and dO into blocked order, k_s into transposed fragments
+// (dS not kept: k_s and v into blocked order), with the row tables (token of every blocked-order slot of one (batch, head), -1 = padding) and the validity words, and the kernels store
 // the gradient rows at their tokens.  Of launch_bwd's own tensors only idx, lens and tile_valid are then used.  Strides count
 // elements.
 struct BwdThw {

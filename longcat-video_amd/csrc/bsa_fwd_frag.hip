@@ -1504,8 +1504,9 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     } while (0)
     const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
     // The lists of a call whose workgroups all run at once are made by those that walk them.  The kernels in front / like this, us, density
-    // 1/16: 4 heads of 192 blocks (one wavefront an item) 48.1 / 46.1, 4 of 256 64.6 / 64.8, one of 320 (teams of four) 43.7 / 40.0, of 512
-    // 66.6 / 62.5; one workgroup behind another pays for it twice (2 heads of 320 blocks, teams of four, density 1/4, 147 / 156).
+    // 1/16: one wavefront an item, 768 items of 192 blocks 48.3 / 46.7, 672 of 224 49.0 / 47.3, 768 of 256 54.8 / 53.9, 1 024 of 256, the most
+    // that there are, 64.1 / 64.3 (at density 1/4 151.2 / 151.0); teams of four, 320 of 320 43.7 / 40.0, 512 of 512 66.6 / 62.5; one
+    // workgroup behind another pays for it twice (2 heads of 320 blocks, teams of four, density 1/4, 147 / 156).
     if (gate_call != nullptr) {
         const GateCall& c = *gate_call;
         const int nsub = bs_k / kTile;
