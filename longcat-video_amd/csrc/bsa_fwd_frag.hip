@@ -1373,9 +1373,10 @@ __global__ void frag_zero_kernel(uint32_t* p, int n) {
 // of 16 88.9 / 84.6 / 82.7, of 64 225 / 197 / 183; 272 of 8 68.3 / 70.7, of 16 91.7 / 90.0, of 64 231 / 206; 416 of 16 94.2 / 93.0,
 // of 64 232 / 214; behind two, 512 of 16 144.3 / 144.8, of 64 368 / 361.  As many shares as there are wavefronts are not made behind
 // whole rounds: little is gained.
-// Lists that may be shorter than their width (the CDF rule's, a caller's: one_length false) are cut where all teams run at once,
-// which pays from two tiles on, and not into more.  Priced by the width, 600 items by the CDF rule became three rounds of teams of
-// four behind kernels that select.  Those / one round of wavefronts, at threshold 0.03, 0.0625, 0.25 and 1, whole operator, us: 600
+// Teams are made where all of them run at once.  Three rounds of teams of four were priced 8 % too low: three parts / teams, us, 544 items
+// of 200 tiles 259 / 284, 640 of 200 282 / 292, of 280 368 / 383; a wavefront an item / teams, 640 of 100 177 / 173, 700 of 100 198 / 205,
+// of 200 339 / 331, 768 of 64 131 / 138, of 200 327 / 320.  Where a list may be shorter than its width (the CDF rule, a caller's: one_length
+// false) they lost more, behind kernels that select; teams / one round of wavefronts, at threshold 0.03, 0.0625, 0.25 and 1, us: 600
 // items of 100 blocks 56.1 / 30.4, 63.0 / 35.2, 88.5 / 59.0, 171 / 153; 768 of 256 72.9 / 47.5, 87.4 / 56.2, 148.5 / 126.2, 404 / 410; 640
 // of 320, which no wavefront scores by itself, 76.1 / 53.5, 88.0 / 65.7, 162 / 148, 444 / 454.
 constexpr int kMaxParts = 16, kMaxPartRounds = 2, kMinPartTiles = 10;
@@ -1383,7 +1384,7 @@ struct Split { int team, parts; };
 static Split choose_split(int items, int list_tiles, int resident, bool is_tail, bool one_length) {
     Split best = {1, 1};
     float best_us = 0.f;
-    for (int team = 1; team <= 4 && team <= list_tiles && !(is_tail && team > 1 && items * team >= resident) && (one_length || items * team <= resident); team *= 2)
+    for (int team = 1; team <= 4 && team <= list_tiles && (team == 1 || items * team + (is_tail ? 1 : 0) <= resident); team *= 2)
         for (int p = 1; p == 1 || (one_length && p <= kMaxParts && p * team * kMinPartTiles <= list_tiles && (int64_t)items * p * team <= kMaxPartRounds * resident); ++p) {
             const int groups = resident / team, rounds = (int)(((int64_t)items * p + groups - 1) / groups);
             const float start = team == 2 ? 4.3f : team == 4 ? 5.8f : is_tail && p == 1 ? 0.f : 6.f;

@@ -253,9 +253,9 @@ def test_workspace_holds_for_devices_of_any_size(cus):
         assert parts >= min(items % round_ * 16, 2 * round_) * 33280
 
 
-def test_lists_of_unknown_length_are_shared_where_all_run_at_once():
-    """A list by the CDF rule may be a sixteenth of its width: its items go to teams of wavefronts only where all teams run at once
-    (1 024 wavefronts without a device), and its last round is not cut into parts.  By the top-k rule the estimate decides."""
+def test_items_are_shared_where_all_teams_run_at_once():
+    """Teams of wavefronts of a last round run at once (1 024 wavefronts without a device); a list by the CDF rule, which may be a
+    sixteenth of its width, is not cut into parts.  By the top-k rule the estimate decides."""
     lib = _capi.load()
     out = (C.c_int32 * 4)()
     for heads in range(1, 24):
@@ -265,8 +265,10 @@ def test_lists_of_unknown_length_are_shared_where_all_run_at_once():
             total, items, team, parts = out
             assert items == total % 1024 and parts == 1 and team in (1, 2, 4) and items * team <= 1024
             assert team > 1 if total <= 512 else team == 1
-    prm = _capi.Bsa3dParams(1, 6, 128, _capi.BSA_BF16, 4, 40, 40, 4, 40, 40, 4, 4, 4, 4, 4, 4, 100, 0.1, 0.0)
-    assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == 0 and tuple(out) == (600, 600, 4, 1)
+    for heads, grid, k_sel, want in ((6, (4, 40, 40), 100, (600, 600, 1, 1)), (1, (8, 64, 68), 200, (544, 544, 1, 3)),
+                                     (1, (8, 64, 68), 64, (544, 544, 1, 1)), (1, (8, 64, 64), 100, (512, 512, 2, 1))):
+        prm = _capi.Bsa3dParams(1, heads, 128, _capi.BSA_BF16, *grid, *grid, 4, 4, 4, 4, 4, 4, k_sel, 0.1, 0.0)
+        assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == 0 and tuple(out) == want
     assert lib.bsa_fwd_3d_last_round(C.byref(prm), None) == _capi.BSA_ERR_BAD_ARG
     prm.dtype = _capi.BSA_F32
     assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == _capi.BSA_ERR_UNSUPPORTED
