@@ -476,7 +476,7 @@ int bsa_fwd_3d_last_round(const bsa_3d_params* p, int32_t out[4]) {
     if (!out) return set_error(BSA_ERR_BAD_ARG, "fwd_3d_last_round: null pointer");
     if (!pl.frag) return set_error(BSA_ERR_UNSUPPORTED, "fwd_3d_last_round: 16-bit types only");
     const bool by_half = pl.half_width > 0;
-    const LastRound r = frag_last_round((int64_t)p->B * p->Hn, pl.Sqp, pl.Skp, pl.gk.chunk(), by_half ? pl.half_width : pl.sel_width, by_half, &pl.gq, !pl.cdf);
+    const LastRound r = frag_last_round((int64_t)p->B * p->Hn, pl.Sqp, pl.Skp, pl.gk.chunk(), by_half ? pl.half_width : pl.sel_width, by_half ? &pl.gk : nullptr, &pl.gq, !pl.cdf);
     out[0] = r.total; out[1] = r.items; out[2] = r.team; out[3] = r.parts;
     return BSA_OK;
 }
@@ -614,7 +614,7 @@ hipError_t attention_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, co
     if (pl.frag)
         return launch_fwd_frag(q, w.kp, w.vp, idx, lens, kv_padded(p) ? w.valid : nullptr, o, lse, p->B, p->Hn, pl.Sqp, pl.Skp,
                                pl.gq.chunk(), pl.gk.chunk(), idx_stride, p->sm_scale, p->dtype, st, w.qrows, q_strides, o_strides,
-                               (int64_t)p->Tq * p->Hq * p->Wq, &pl.gq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves, parts, gate);
+                               (int64_t)p->Tq * p->Hq * p->Wq, &pl.gq, by_length ? w.order : nullptr, by_length ? w.queue : nullptr, w.knorm, w.fallback, fallback_cleared, halves ? &pl.gk : nullptr, parts, gate);
     FwdLayout L;
     L.q_rows = w.qrows;
     L.k_tiles = w.ktiles;

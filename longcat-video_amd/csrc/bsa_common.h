@@ -317,7 +317,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const Grid3* q_grid = nullptr, int32_t* order = nullptr, uint32_t* queue = nullptr, const float* key_norm = nullptr,
-                           int32_t* fallback = nullptr, bool fallback_cleared = false, bool halves = false, float* part_buf = nullptr,
+                           int32_t* fallback = nullptr, bool fallback_cleared = false, const Grid3* halves_of = nullptr, float* part_buf = nullptr,
                            const GateCall* gate_call = nullptr);
 // order (B * Hn * Sq / 64 int32) and queue (kFragQueueWords), both or none: scratch for the schedule of lists of unequal length,
 // enqueued besides the rounds; which of the two runs is decided on the device.
@@ -330,8 +330,8 @@ constexpr int kFragQueueWords = 16;
 size_t frag_part_floats(const Grid3& q_grid, int64_t heads);
 // Work items of a call, those of its last, partial round, and how these are shared: `parts` parts of an item, `team` wavefronts a part.
 struct LastRound { int total, items, team, parts; };
-LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, bool halves, const Grid3* q_grid, bool one_length);
-// halves: idx and lens are HalfLists, idx_stride their row pitch (at most 4 096).
+LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length);
+// halves_of (optional): idx and lens are HalfLists, idx_stride their row pitch (at most 4 096), of this grid of keys.
 // gate_call (optional): idx and lens are still to be made.
 size_t frag_fallback_ints(int64_t items);
 

@@ -1379,17 +1379,30 @@ __global__ void frag_zero_kernel(uint32_t* p, int n) {
 // false) they lost more, behind kernels that select; teams / one round of wavefronts, at threshold 0.03, 0.0625, 0.25 and 1, us: 600
 // items of 100 blocks 56.1 / 30.4, 63.0 / 35.2, 88.5 / 59.0, 171 / 153; 768 of 256 72.9 / 47.5, 87.4 / 56.2, 148.5 / 126.2, 404 / 410; 640
 // of 320, which no wavefront scores by itself, 76.1 / 53.5, 88.0 / 65.7, 162 / 148, 444 / 454.
+// The shares of a team of two are whole KV blocks of the list, which visits the sequence in order, while parts of single wavefronts
+// are cut by halves.  On a grid whose last frames do not fill their chunks the second share is short: `heavier_half` is the first one's
+// part of the halves over the mean, of blocks spread evenly.  Its wavefront walks that much longer on a chip that is as much emptier.
+// Teams of two / parts, us, which were priced without it: 258 items of 13x26x43 in 4x4x8 chunks and 168 tiles 127 / 112, 342 of 9x36x57
+// and 344 251 / 219, 336 of 5x46x53 in 4x4x4 and 168 137 / 129, 468 of 9x50x46 and 234 210 / 215.  Teams of four come out right without
+// it: with it 80 items of 5x37x15 and 64 tiles would go to parts, 53 us for 41, 138 of 9x18x48 and 90 65 for 54.
+static float heavier_half(const Grid3& k) {
+    const int full = k.chunk() / 32, last = k.T % k.t == 0 ? full : (k.T % k.t * k.h * k.w + 31) / 32;      // halves of an inner chunk
+    const float layers = (float)k.Nt, span = 0.5f * layers, inner = fminf(span, layers - 1.f);
+    return 2.f * (inner * full + (span - inner) * last) / ((layers - 1.f) * full + last);
+}
 constexpr int kMaxParts = 16, kMaxPartRounds = 2, kMinPartTiles = 10;
 struct Split { int team, parts; };
-static Split choose_split(int items, int list_tiles, int resident, bool is_tail, bool one_length) {
+// halves_of: the grid of the keys where the lists are of halves, otherwise null
+static Split choose_split(int items, int list_tiles, int resident, bool is_tail, bool one_length, const Grid3* halves_of) {
     Split best = {1, 1};
     float best_us = 0.f;
     for (int team = 1; team <= 4 && team <= list_tiles && (team == 1 || items * team + (is_tail ? 1 : 0) <= resident); team *= 2)
         for (int p = 1; p == 1 || (one_length && p <= kMaxParts && p * team * kMinPartTiles <= list_tiles && (int64_t)items * p * team <= kMaxPartRounds * resident); ++p) {
             const int groups = resident / team, rounds = (int)(((int64_t)items * p + groups - 1) / groups);
             const float start = team == 2 ? 4.3f : team == 4 ? 5.8f : is_tail && p == 1 ? 0.f : 6.f;
-            const float full = (float)items * p / ((float)rounds * groups), tile_us = 1.15f + 1.14f * (full > 0.5f ? full - 0.5f : 0.f);
-            const float us = rounds * (tile_us * list_tiles / (p * team) + start) + (p > 1 ? 5.f + 0.0125f * items * p : 0.f) + (is_tail && p * team > 1 ? 4.f : 0.f);
+            const float weight = team == 2 && p == 1 && halves_of != nullptr ? heavier_half(*halves_of) : 1.f;
+            const float full = (float)items * p / ((float)rounds * groups) / weight, tile_us = 1.15f + 1.14f * (full > 0.5f ? full - 0.5f : 0.f);
+            const float us = rounds * (tile_us * list_tiles * weight / (p * team) + start) + (p > 1 ? 5.f + 0.0125f * items * p : 0.f) + (is_tail && p * team > 1 ? 4.f : 0.f);
             if ((team == 1 && p == 1) || us < best_us) { best = {team, p}; best_us = us; }
         }
     return best;
@@ -1400,7 +1413,7 @@ struct Rounds {
     int n_live, total, resident, list_tiles, tail;
     Split split;
 };
-static Rounds plan_rounds(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, bool halves, const Grid3* q_grid, bool one_length) {
+static Rounds plan_rounds(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length) {
     Rounds r;
     // The kernel addresses K and V through a buffer of less than 4 GB that starts at the first (batch, head) of a
     // launch: a launch covers as many heads as fit.  One head always does (fewer than 2^24 keys of 256 B).
@@ -1413,17 +1426,17 @@ static Rounds plan_rounds(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int i
     r.n_live = q_grid != nullptr && r.one_span ? live_query_tiles(*q_grid) : (int)(Sq / kTile);
     r.total = (int)(heads * r.n_live);
     r.resident = resident_wavefronts();
-    r.list_tiles = halves ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
+    r.list_tiles = halves_of != nullptr ? (idx_stride + 1) / 2 : idx_stride * (bs_k / kTile);
     // The items of the last, partial round are cut when its wavefronts would leave too much of the chip idle (and the exact
     // kernel reaches every head from one buffer); behind whole rounds and into parts only for lists of one length.
     r.tail = r.total % r.resident;
     r.split = {1, 1};
     if (r.one_span && r.tail > 0 && (one_length || r.total < r.resident))
-        r.split = choose_split(r.tail, r.list_tiles, r.resident, r.total > r.resident, one_length);
+        r.split = choose_split(r.tail, r.list_tiles, r.resident, r.total > r.resident, one_length, halves_of);
     return r;
 }
-LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, bool halves, const Grid3* q_grid, bool one_length) {
-    const Rounds r = plan_rounds(heads, Sq, Sk, bs_k, idx_stride, halves, q_grid, one_length);
+LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length) {
+    const Rounds r = plan_rounds(heads, Sq, Sk, bs_k, idx_stride, halves_of, q_grid, one_length);
     return {r.total, r.tail, r.split.team, r.split.parts};
 }
 // floats of the parts' buffer, whatever the length of the lists and whichever device runs the call (a caller asks for the size
@@ -1441,7 +1454,8 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
                            int bs_q, int bs_k, int idx_stride, float sm_scale, int dtype, hipStream_t st,
                            const int32_t* q_rows, const int64_t q_st[3], const int64_t o_st[3], int64_t lse_rows,
                            const Grid3* q_grid, int32_t* order, uint32_t* queue, const float* key_norm, int32_t* fallback, bool fallback_cleared,
-                           bool halves, float* part_buf, const GateCall* gate_call) {
+                           const Grid3* halves_of, float* part_buf, const GateCall* gate_call) {
+    const bool halves = halves_of != nullptr;
     // the C-ABI layer keeps lists within these limits (a list that is too long for the small buffers is staged in `ost`)
     if (idx_stride > (halves ? kHalfEntries : kListEntries)) return hipErrorInvalidValue;
     const float qk_scale = sm_scale * kLog2e;
@@ -1455,7 +1469,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     if (kv_bh_bytes > ((int64_t)1 << 32) - 1) return hipErrorInvalidValue;
     // a buffer for parts comes with lists of one length
     const auto [heads_per_span, one_span, n_live, total, resident, list_tiles, tail, split] =
-        plan_rounds((int64_t)B * Hn, Sq, Sk, bs_k, idx_stride, halves, q_grid, part_buf != nullptr);
+        plan_rounds((int64_t)B * Hn, Sq, Sk, bs_k, idx_stride, halves_of, q_grid, part_buf != nullptr);
     L.tiles = n_live < per_head ? q_rows + Sq : nullptr;
     L.n_live = n_live;
     L.by_live = divisor(n_live);

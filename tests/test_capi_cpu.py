@@ -269,6 +269,11 @@ def test_items_are_shared_where_all_teams_run_at_once():
                                      (1, (8, 64, 68), 64, (544, 544, 1, 1)), (1, (8, 64, 64), 100, (512, 512, 2, 1))):
         prm = _capi.Bsa3dParams(1, heads, 128, _capi.BSA_BF16, *grid, *grid, 4, 4, 4, 4, 4, 4, k_sel, 0.1, 0.0)
         assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == 0 and tuple(out) == want
+    # keys whose last frames fill a quarter or a half of their chunks: the second wavefront of a team of two would have less to do
+    for grid, chunk, k_sel, want in (((13, 26, 43), (4, 4, 8), 84, (1, 3)), ((9, 36, 57), (4, 4, 8), 172, (1, 5)), ((5, 46, 53), (4, 4, 4), 168, (1, 3)),
+                                     ((16, 26, 43), (4, 4, 8), 84, (2, 1)), ((9, 50, 46), (4, 4, 4), 234, (2, 1)), ((5, 37, 15), (4, 4, 4), 64, (4, 1))):
+        prm = _capi.Bsa3dParams(1, 1, 128, _capi.BSA_BF16, *grid, *grid, *chunk, *chunk, k_sel, 0.1, 0.0)
+        assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == 0 and tuple(out)[2:] == want, (grid, tuple(out))
     assert lib.bsa_fwd_3d_last_round(C.byref(prm), None) == _capi.BSA_ERR_BAD_ARG
     prm.dtype = _capi.BSA_F32
     assert lib.bsa_fwd_3d_last_round(C.byref(prm), out) == _capi.BSA_ERR_UNSUPPORTED
