@@ -89,9 +89,9 @@ def _gemm_workspace(device) -> torch.Tensor:
 
 
 def _linear_workspace(M: int, N: int, residual: bool, device) -> torch.Tensor:
-    """What a linear of M rows and N columns works in: with a residual also the fp32 product, from torch's allocator for the one
-    call where the card has room for it, and otherwise in groups of rows."""
-    if not residual:
+    """What a linear of M rows and N columns works in: with a residual also the fp32 product, in the kept workspace's second half
+    if that holds it, otherwise from torch's allocator for the one call, and where the card has no room for it in groups of rows."""
+    if not residual or 4 * M * N + 256 <= 32 << 20:
         return _gemm_workspace(device)
     need = _capi.load().bsa_linear_bf16_workspace_bytes(M, N, 1)
     return _backward_workspace(need, 64 << 20, device)
