@@ -418,10 +418,12 @@ int bsa_norm_rope(const void* src, const int64_t src_strides[3], void* dst, cons
                   int t_offset, int table_T, int D, float eps, int dtype, void* stream);
 
 /* out[M,N] = x[M,K] . w[N,K]^T (+ bias[N]) (+ residual[M,N]), bf16 in/out, fp32 accumulate, on MFMA
- * through hipBLASLt.  Replaces the nn.Linear calls attention.py:111 and :142.  `workspace`: at least
- * 64 MiB of device memory (BSA_ERR_WORKSPACE otherwise); its contents do not matter.  With a residual, which a
- * pass of its own adds to an fp32 product (one rounding), bsa_linear_bf16_workspace_bytes holds all of it;
- * in less, the call runs in groups of rows, slower.  out may be the residual.  Every calling thread
+ * through hipBLASLt, or through the engine's own GEMM where that is faster: most products with a residual, and short rows.
+ * Replaces the nn.Linear calls attention.py:111 and :142.  `workspace`: at least
+ * 64 MiB of device memory (BSA_ERR_WORKSPACE otherwise); its contents do not matter.  A residual that the engine's GEMM
+ * does not add (with the same single rounding) is added to an fp32 product by a pass of its own: bsa_linear_bf16_workspace_bytes holds all of that;
+ * in less, the call runs in groups of rows.  bsa_linear_bf16_ld_workspace_bytes: what the call with these very operands has use
+ * for.  out may be the residual.  Every calling thread
  * uses a hipBLASLt handle of its own per device; a thread that ends hands its handles to the next thread that
  * needs one, so their number stays at the largest number of threads that called at one time. */
 int bsa_linear_bf16(const void* x, const void* w, const void* bias, const void* residual, void* out,
@@ -435,11 +437,14 @@ size_t bsa_linear_bf16_workspace_bytes(int64_t M, int N, int with_residual);
 int bsa_linear_bf16_ld(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
                        void* out, int64_t ldo, int64_t M, int N, int K, void* workspace, size_t workspace_bytes,
                        void* stream);
+size_t bsa_linear_bf16_ld_workspace_bytes(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
+                                          const void* out, int64_t ldo, int64_t M, int N, int K);
 
 /* One-time tuning of a linear shape (no counterpart in the reference, whose nn.Linear leaves the choice to the
  * BLAS library): runs every algorithm hipBLASLt proposes for this call (up to 32, each four times on the given
  * buffers; `out` is overwritten), and remembers the fastest for later bsa_linear_bf16 / _ld calls with the same
- * M, N, K, row strides, bias / residual presence (and, with a residual, a workspace of the same size) in this process.  Unlike every other entry point it WAITS for
+ * M, N, K, row strides, bias / residual presence (and, with a residual, a workspace of the same size) in this process,
+ * as far as these go to the library.  Unlike every other entry point it WAITS for
  * the stream, so call it at set-up, outside graph capture.  Returns the number of algorithms timed (> 0) or a
  * negative status; default_ms / best_ms (optional) receive the time of the algorithm an untuned call uses and
  * of the one chosen.  Algorithms differ in summation order, so results can differ in the last bit. */

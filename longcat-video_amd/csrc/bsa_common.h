@@ -174,6 +174,8 @@ inline int dtype_size(int dtype) {
 
 // Records the message returned by bsa_last_error() and passes `code` through.
 int set_error(int code, const char* fmt, ...);
+bool gemm_serves_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual, const void* out, int64_t ldo,
+                        int64_t M, int N, int K);      // bsa_gemm.hip
 
 // Kernel launchers (one per source file); all validate nothing and assume the
 // C-ABI layer has checked shapes.  Each returns a hipError_t from the launch.

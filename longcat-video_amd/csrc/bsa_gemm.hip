@@ -3,61 +3,65 @@
 //   q, k, v   = split(x . w^T + bias) per head, q and k normalised per head (RMSNorm over the 128
 //               features of a head) and rotated (3-D RoPE), every head written as a contiguous
 //               [tokens, 128] tensor                                    (QKV epilogue)
-// bf16 operands, fp32 accumulation in v_mfma_f32_32x32x16_bf16.
+// bf16 operands, fp32 accumulation in v_mfma_f32_16x16x32_bf16.
 //
 // Shape of the computation.  Both operands have k as their fastest axis, which is the layout both MFMA
-// operands want: lane l of a 32x32x16 product holds 8 consecutive k of row l % 32, starting at k = 8 (l / 32).
+// operands want: lane l of a 16x16x32 product holds 8 consecutive k of row l % 16, starting at k = 8 (l / 16).
 // The weight rows are the A operand and the token rows the B operand, so an accumulator register holds
-// C^T: lane l has token l % 32 and, in its 16 registers, features 8 (r / 4) + 4 (l / 32) + r % 4 of the
-// 32x32 block.  A lane therefore owns whole rotation pairs (features 2i, 2i + 1) and half of the features of
-// its tokens: the per-head sum of squares is an in-lane sum plus one exchange between lane l and l ^ 32.
+// C^T: lane l has token l % 16 and, in its 4 registers, features 4 (l / 16) + r of the 16x16 block.  A lane
+// therefore owns whole rotation pairs (features 2i, 2i + 1) and a quarter of the features of its tokens: the per-head
+// sum of squares is an in-lane sum plus two exchanges.  16x16x32 and not 32x32x16: what bounds a large product is the
+// board's power, and the small form moves half as many accumulators per multiplication.  Registers alone, random data, nothing but
+// MFMAs: 2 080 TFLOP/s against 1 820; this kernel (then one tile a workgroup), 86 400 x 4 096 x 4 096: 2 149 us against 2 282, the
+// clock under it 1.78 GHz against 1.65.
 //
-// A workgroup of four wavefronts (one per SIMD, 512 registers each) computes a tile of 256 tokens x 256
-// features; every wavefront owns 128 x 128 of it (16 accumulator blocks = 256 registers), which for the QKV
-// projection is exactly one head of 128 tokens.  Per k block of 64 the workgroup brings 256 rows x 128 bytes of
+// A workgroup of eight wavefronts computes tiles of 256 tokens x 256 features, a wavefront 64 x 128 of a tile: for the
+// QKV projection one head of 64 tokens.  Waves w and w + 4 share a SIMD and take turns: while group 0 (features 0 .. 127 of the
+// tile) multiplies a k block of 64, 64 MFMAs, group 1 reads its operands of one from LDS and requests a slab of a later one, and
+// the other way round, with a barrier at every change.  One wavefront a SIMD (128 x 128 of the tile) has a third fewer
+// fragment reads but nothing to issue while it waits or requests: 2 500 us.  Per k block the workgroup brings 256 rows x 128 bytes of
 // either operand (a half-slab of 32 KB, whole cache lines) from global memory straight into LDS
-// (global_load_lds_dwordx4, no staging registers); five half-slab stages fill the 160 KB of LDS: two in use, up to
-// three on their way.  The LDS side of such a load is linear in the lane index, so the XOR swizzle that keeps the
-// fragment reads (ds_read_b128, rows 128 bytes apart; measured: bank-conflict cycles 4 % of the LDS-active ones)
-// free of bank conflicts is applied on the global side: the 16-byte slot p of row r receives k unit
-// p ^ ((r >> 1) & 7).
+// (global_load_lds_dwordx4, no staging registers); five half-slab stages fill the 160 KB of LDS.  The LDS side of such a load is
+// linear in the lane index, so the XOR swizzle that keeps the fragment reads (ds_read_b128, rows 128 bytes apart) free of bank
+// conflicts is applied on the global side: the 16-byte slot p of row r receives k unit p ^ ((r >> 1) & 7).
 //
-// One barrier per k block, after the third of its four k sub-steps: the fragments of a sub-step are read during
-// the MFMAs of the one before.  At the barrier every wavefront has awaited its own share of the next block's two
-// half-slabs and holds the last fragments of this one; the two stages so drained take the half-slabs five further
-// on, requested one load per four MFMAs over the k block that follows.
+// The stages, in phases (k block j is read by group 0 in phase 2j and by group 1 in phase 2j + 1): its two half-slabs are free from
+// phase 2j + 2 on.  Group 0 requests the weights of block j + 1 in phase 2j, into the stage of block j - 1's tokens, and waits for them
+// at the end of phase 2j + 1; group 1 requests the tokens of block j + 2 in phase 2j + 1, into the stage of block j - 1's
+// weights, and waits for those of block j + 1 there.
 //
-// Tiles are handed out so that the workgroups resident on one XCD (32 CUs, one shared L2; workgroup b runs
-// on XCD b % 8) form a block of 8 token tiles x 4 feature tiles: they run in step, so each slab fetched from
-// HBM serves 4 (token slab) or 8 (weight slab) workgroups out of L2 (measured at the 720p QKV shape: 15 GB leave
-// L2 per call for 65 GB that enter LDS).
+// A workgroup stays and goes from tile to tile; the requests run on over the change, so that the first blocks of the next tile
+// are there when it begins (one tile a workgroup: 2 135 us; 32 760 x 12 288 x 4 096 2 400 against 2 290).  The order of the tiles runs
+// over blocks of 8 token tiles, and the workgroups of an XCD have a contiguous share of it, 8 x 4 tiles at a time: in step, they
+// fetch a slab once for 4 or 8 of them.
 //
-// What bounds it (measured at [86400, 4096] x [4096, 12288]^T on random data): the board's power limit.  Under this
-// kernel the clock settles near 1.83 GHz instead of 2.4 (under hipBLASLt's kernel for the same product near
-// 1.72 GHz), so a gain in work per clock is partly paid back in clock.  Per clock the k loop reaches about 0.61 of
-// the MFMA rate.  Variants measured on the way: all sixteen loads of a k block in one burst after the barrier
-// 8.5 ms (the wavefronts then wait for the address unit, not for data: with a software barrier instead of
-// s_barrier no better, without any barrier 5.3 ms but wrong); two stages of a whole k block 8.0 ms; ten 16 KB
-// stages with paired loads of the two halves of a cache line 8.4 ms; register prefetch two blocks ahead with
-// compiler-placed waits 9.1 ms (the waits it places allow only one block in flight).
+// What bounds it: power, and the reading half of a phase.  Per k block and group 610 clocks to request 32 KB (the address unit of a
+// CU takes 16 a load of 1 KB, and a wavefront issues in order) and 500 to read 96 KB of fragments, against 1 009 of MFMAs, so the
+// MFMAs run 0.76 of the clocks at 1.87 GHz.  Measured and not kept: the requests between the fragment reads (R 1 170 clocks)
+// or between the MFMAs (both wait for the address unit: 0.66-0.70), MFMAs behind the barrier of a phase, with and without priority (0.75),
+// an L2 prefetch three to eight blocks ahead (1-2 % slower), one barrier a k block with the groups half a block apart (0.54-0.74).
+// hipBLASLt's kernel for the QKV shape reaches 0.80 at 1.80 GHz.
 #include "bsa_mfma.h"
+
+#include <algorithm>
 
 namespace bsa {
 namespace {
 
 using namespace mfma;
 
-constexpr int kTileM = 256;              // tokens per workgroup
-constexpr int kTileN = 256;              // features per workgroup
+constexpr int kTileM = 256;              // tokens of a tile
+constexpr int kTileN = 256;              // features of a tile
 constexpr int kBK = 64;                  // k per pipeline step
 constexpr int kPart = 256 * kBK * 2;     // bytes of one operand's slab
 constexpr int kStages = 5;               // half-slabs resident in LDS: 160 KB
-constexpr int kEpiPitch = 272;           // bytes per token row of the output staging area (256 + 16)
-constexpr int kEpiBytes = 64 * kEpiPitch;
-constexpr int kSuperM = 8, kSuperN = 4;  // tiles of one XCD's block
+constexpr int kThreads = 512;
+constexpr int kCus = 256;                // workgroups of a launch at most: one a CU
+constexpr int kBlockM = 8;               // token tiles that the order of the tiles stays with
 
 typedef bf16x8 V8;
-template <int N> using IC = std::integral_constant<int, N>;
+
+enum Epilogue { kPlain, kResidual, kQkv };
 
 struct GemmArgs {
     const __bf16* x; int64_t ldx;
@@ -66,7 +70,7 @@ struct GemmArgs {
     const __bf16* residual; int64_t ldr;
     __bf16* out; int64_t ldo;
     int M, N, K;
-    int tiles_m, tiles_n, super_m, super_total;
+    int tiles_m, tiles_n;
     // QKV epilogue
     __bf16* dst[3];
     int64_t dB, dH, dS;
@@ -76,289 +80,289 @@ struct GemmArgs {
     float eps;
 };
 
-template <bool QKV>
-__global__ __launch_bounds__(256) void gemm_nt_kernel(const GemmArgs a) {
+template <int kEpi>
+__global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) {
+    constexpr bool QKV = kEpi == kQkv;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave >> 1, wn = wave & 1;      // this wavefront's feature half and token half
+    const int group = wave >> 2, quarter = wave & 3;      // waves w and w + 4 share a SIMD
 
-    // tile of this workgroup
-    const int b = blockIdx.x;
-    const int super = (b >> 8) * 8 + (b & 7), pos = (b >> 3) & 31;
-    if (super >= a.super_total) return;
-    const int sf = super / a.super_m, sm = super - sf * a.super_m;
-    const int tile_f = sf * kSuperN + (pos & 3), tile_m = sm * kSuperM + (pos >> 2);
-    if (tile_f >= a.tiles_n || tile_m >= a.tiles_m) return;
-    const int f_tile0 = tile_f * kTileN, m_tile0 = tile_m * kTileM;
+    // ---- tiles of this workgroup: every per_xcd-th of its XCD's (workgroup b runs on XCD b % 8)
+    const int per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7;
+    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
+    const int t_end = (int)(tiles * (xcd + 1) >> 3), t_first = (int)(tiles * xcd >> 3) + (int)(blockIdx.x >> 3);
+    if (t_first >= t_end) return;
+    auto place = [&](int t, int& tile_m, int& tile_f) {
+        const int block = t / (kBlockM * a.tiles_n), in = t - block * (kBlockM * a.tiles_n);
+        const int rows = min(kBlockM, a.tiles_m - block * kBlockM);
+        tile_f = in / rows;
+        tile_m = block * kBlockM + in - tile_f * rows;
+    };
 
-    // ---- global -> LDS: this wavefront brings rows [64 wave, 64 wave + 64) of a half-slab, 8 rows (of 128 bytes:
-    // one cache line each) per load
-    uint32_t voff_w[8], voff_x[8];
+    // ---- global -> LDS: group 0 brings weight rows (odd half-slabs), group 1 token rows (even ones), a wavefront 64 of them,
+    // 8 rows (of 128 bytes: one cache line each) per load
+    const char* from;
+    uint32_t pitch;
+    int last_row;
+    int next_t = t_first, left = 0;                   // tile that is being brought, k blocks of it that are not yet
+    const int nblocks = a.K / kBK;
+    const uint32_t lds0 = lds_address(smem);
+    auto start_tile = [&]() __attribute__((always_inline)) {
+        int tm, tf;
+        place(next_t, tm, tf);
+        from = group ? reinterpret_cast<const char*>(a.x + (int64_t)tm * kTileM * a.ldx) : reinterpret_cast<const char*>(a.w + (int64_t)tf * kTileN * a.ldw);
+        pitch = (uint32_t)(group ? a.ldx : a.ldw) * 2u;
+        last_row = group ? a.M - 1 - tm * kTileM : a.N - 1 - tf * kTileN;
+        left = nblocks;
+    };
+    // half-slab h (even: token rows, odd: weight rows, of k block h / 2 of all of this workgroup's tiles) lives in stage h % kStages
+    auto bring = [&](int stage) __attribute__((always_inline)) {
+        const uint32_t to = lds0 + stage * kPart + quarter * 8192;
+        int l = lane;
+        asm volatile("" : "+v"(l));                   // eight offsets worked out anew cost less than registers for them
+        const uint32_t unit = ((l & 7) ^ (l >> 4)) * 16;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-        const int row = wave * 64 + r * 8 + (lane >> 3);
-        const int unit = (lane & 7) ^ ((row >> 1) & 7);
-        const int frow = min(row, a.N - 1 - f_tile0), mrow = min(row, a.M - 1 - m_tile0);   // edge tiles repeat their last row
-        voff_w[r] = (uint32_t)((int64_t)frow * a.ldw * 2 + unit * 16);
-        voff_x[r] = (uint32_t)((int64_t)mrow * a.ldx * 2 + unit * 16);
-    }
-    const char* wbase = reinterpret_cast<const char*>(a.w + (int64_t)f_tile0 * a.ldw);
-    const char* xbase = reinterpret_cast<const char*>(a.x + (int64_t)m_tile0 * a.ldx);
-    // Half-slab h (even: weight rows, odd: token rows, of k block h / 2) lives in stage h % kStages.
-    const uint32_t lds0 = lds_address(smem) + wave * 8192;
-    const int nblocks = a.K / kBK, nhalf = 2 * nblocks;
-    // load r (of eight) of half-slab h; `odd` = h & 1, known at compile time
-    auto issue_one = [&](int h, int stage, auto odd_c, int r) __attribute__((always_inline)) {
-        constexpr int odd = decltype(odd_c)::value;
-        if (h >= nhalf) return;
-        const char* base = (odd ? xbase : wbase) + (int64_t)(h >> 1) * (kBK * 2);
-        load_to_lds_16(base, odd ? voff_x[r] : voff_w[r], lds0 + stage * kPart + r * 1024);
+        for (int r = 0; r < 8; ++r) {
+            const int row = min(quarter * 64 + r * 8 + (l >> 3), last_row);       // edge tiles repeat their last row
+            load_to_lds_16(from, __umul24(row, pitch) + (r & 1 ? unit ^ 64u : unit), to + r * 1024);
+        }
+        from += kBK * 2;
+        if (--left == 0) {
+            next_t += per_xcd;
+            if (next_t < t_end) start_tile();
+        }
     };
 
     // ---- LDS -> fragments
-    const uint32_t swz = ((lane & 31) >> 1) & 7, g = lane >> 5;
-    const uint32_t a_lane = (wm * 128 + (lane & 31)) * 128, b_lane = (wn * 128 + (lane & 31)) * 128;
-    uint32_t unit_of[4];
+    const uint32_t lr = lane & 15, lg = lane >> 4;
+    uint32_t unit_of[2];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) unit_of[ks] = ((2 * ks + g) ^ swz) * 16;
-    V8 af[2][4], bf[2][4];
-    auto read_frags = [&](int stage_w, int stage_x, int ks) __attribute__((always_inline)) {
-        const char* sw = smem + stage_w * kPart + unit_of[ks] + a_lane;
-        const char* sx = smem + stage_x * kPart + unit_of[ks] + b_lane;
+    for (int ks = 0; ks < 2; ++ks) unit_of[ks] = ((4 * ks + lg) ^ ((lr >> 1) & 7)) * 16 + lr * 128;
+    V8 af[2][8], bf[2][4];
+    auto read_frags = [&](int stage_w, int stage_x) __attribute__((always_inline)) {
+        const uint32_t sw = lds0 + stage_w * kPart + group * (128 * 128), sx = lds0 + stage_x * kPart + quarter * (64 * 128);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) af[ks & 1][i] = *reinterpret_cast<const V8*>(sw + i * 4096);
+        for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bf[ks & 1][j] = *reinterpret_cast<const V8*>(sx + j * 4096);
-    };
-    f32x16 acc[4][4];
+            for (int i = 0; i < 8; ++i) af[ks][i] = lds_read_at<V8>(unit_of[ks] + sw + i * 2048);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-    // The sixteen MFMAs of k sub-step ks, and between them four of the sixteen loads requested at the last barrier
-    // (token half-slab pend_h first, then weight half-slab pend_h + 1): one load per four MFMAs.  Issued in one
-    // burst right after the barrier, the four wavefronts' loads queue up in the CU's one address unit and the
-    // wavefronts, which issue in order, cannot start their MFMAs until their last load is taken.
-    int pend_h = nhalf, pend_sw = 0, pend_sx = 0;
-    auto products = [&](auto ks_c) __attribute__((always_inline)) {
-        constexpr int ks = decltype(ks_c)::value;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = mfma32(af[ks & 1][i], bf[ks & 1][j], acc[i][j]);
-            constexpr int quarter = (ks + 1) & 3;            // sub-step 3 is the first after the barrier
-            const int n = 4 * quarter + i;
-            __builtin_amdgcn_sched_barrier(0);
-            if (n < 8) issue_one(pend_h, pend_sx, IC<1>{}, n); else issue_one(pend_h + 1, pend_sw, IC<0>{}, n - 8);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < 4; ++j) bf[ks][j] = lds_read_at<V8>(unit_of[ks] + sx + j * 2048);
         }
+    };
+    f32x4_ acc[8][4];
+    auto meet = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
     };
 
     // ---- pipeline
-#pragma unroll
-    for (int r = 0; r < 8; ++r) issue_one(0, 0, IC<0>{}, r);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) issue_one(1, 1, IC<1>{}, r);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) issue_one(2, 2, IC<0>{}, r);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) issue_one(3, 3, IC<1>{}, r);
-#pragma unroll
-    for (int r = 0; r < 8; ++r) issue_one(4, 4, IC<0>{}, r);
-    if (nhalf >= kStages) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");    // half-slabs 0 and 1 of five
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    read_frags(0, 1, 0);
-    // k block kb, with c = kb % kStages known at compile time
-    auto block = [&](int kb, auto c_) __attribute__((always_inline)) {
-        constexpr int c = decltype(c_)::value;
-        constexpr int sw = (2 * c) % kStages, sx = (2 * c + 1) % kStages;              // stages of this block
-        constexpr int nw = (2 * c + 2) % kStages, nx = (2 * c + 3) % kStages;          // ... of the next one
-        read_frags(sw, sx, 1);
-        products(IC<0>{});
-        read_frags(sw, sx, 2);
-        products(IC<1>{});
-        read_frags(sw, sx, 3);
-        products(IC<2>{});
-        // The next block's two half-slabs: this wavefront's share has landed (the one requested after them may still
-        // be on its way), then (barrier) everybody's; and everybody holds the last fragments of this block in
-        // registers, so its two stages can take the half-slabs five further on (tokens of block kb + 2, needed at
-        // the next barrier, then weights of block kb + 3), requested piecemeal by products().
-        if (2 * kb + 4 < nhalf) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        pend_h = 2 * kb + kStages;
-        pend_sx = sw;                    // half-slab 2 kb + 5 (tokens) takes the stage of half-slab 2 kb (weights)
-        pend_sw = sx;                    // half-slab 2 kb + 6 (weights) the stage of half-slab 2 kb + 1 (tokens)
-        if (kb + 1 < nblocks) read_frags(nw, nx, 0);
-        products(IC<3>{});
-    };
-    int kb = 0;
-    for (; kb + kStages <= nblocks; kb += kStages) {
-        block(kb, IC<0>{});
-        block(kb + 1, IC<1>{});
-        block(kb + 2, IC<2>{});
-        block(kb + 3, IC<3>{});
-        block(kb + 4, IC<4>{});
+    start_tile();
+    if (group) {
+        bring(0);
+        if (left) {
+            bring(2);
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+        } else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    } else {
+        bring(1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    if (kb < nblocks) { block(kb, IC<0>{}); ++kb; }
-    if (kb < nblocks) { block(kb, IC<1>{}); ++kb; }
-    if (kb < nblocks) { block(kb, IC<2>{}); ++kb; }
-    if (kb < nblocks) { block(kb, IC<3>{}); ++kb; }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();        // every wavefront is done with the slabs: the staging area may overwrite them
-
-    // ---- epilogue.  Feature of register r of block i: f0 + 32 i + 8 (r / 4) + 4 g + r % 4; token of block j: m0 + 32 j + lane % 32.
-    const int f0 = f_tile0 + wm * 128;                    // first feature of this wavefront
-    const int m0 = m_tile0 + wn * 128;                    // first token
-    if (f0 >= a.N) return;
-    char* stage_area = smem + wave * kEpiBytes;
-    // bias, four consecutive features at a time
-    if (a.bias != nullptr) {
+    meet();
+    if (group) meet();
+    int s_x = 0;                                     // stage of this block's token rows, (2 kb) % 5
+    for (int t = t_first; t < t_end; t += per_xcd) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint2 raw = *reinterpret_cast<const uint2*>(a.bias + f0 + 32 * i + 8 * q + 4 * g);
-                const __bf16* bv = reinterpret_cast<const __bf16*>(&raw);
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+        for (int kb = 0; kb < nblocks; ++kb) {
+            const int s_w = s_x + 1 >= kStages ? s_x + 1 - kStages : s_x + 1;
+            const int ahead = s_x + 3 + group, s_to = ahead >= kStages ? ahead - kStages : ahead;
+            const bool more = left != 0;
+            if (more) bring(s_to);
+            __builtin_amdgcn_sched_barrier(0);
+            read_frags(s_w, s_x);
+            __builtin_amdgcn_sched_barrier(0);
+            if (group && more) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+            else if (group) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            s_x = s_x + 2 >= kStages ? s_x + 2 - kStages : s_x + 2;
+            meet();
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += (float)bv[e];
-            }
-    }
-    if constexpr (!QKV) {
-        if (a.residual != nullptr) {
+            for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int tok = min(m0 + 32 * j + (lane & 31), a.M - 1);
-                const __bf16* rrow = a.residual + (int64_t)tok * a.ldr + f0 + 4 * g;
+                for (int i = 0; i < 8; ++i)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint2 raw = *reinterpret_cast<const uint2*>(rrow + 32 * i + 8 * q);
-                        const __bf16* rv = reinterpret_cast<const __bf16*>(&raw);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += (float)rv[e];
-                    }
-            }
+                    for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(af[ks][i], bf[ks][j], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!group) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (!group || kb + 1 < nblocks || t + per_xcd < t_end) meet();
         }
-    }
-    int section = 0, head = 0;
-    if constexpr (QKV) {
-        const int per_section = a.Hn * 128;
-        section = f0 / per_section;
-        head = (f0 - section * per_section) >> 7;
-        if (section < 2) {
+
+        // ---- epilogue.  Feature of register r of block i: f0 + 16 i + 4 lg + r; token of block j: m0 + 16 j + lr.
+        int tile_m, tile_f, el = lane;
+        asm volatile("" : "+v"(el));
+        const uint32_t lr = el & 15, lg = el >> 4;
+        place(t, tile_m, tile_f);
+        const int f0 = tile_f * kTileN + group * 128;         // first feature of this wavefront
+        const int m0 = tile_m * kTileM + quarter * 64;        // first token
+        if (f0 >= a.N) continue;
+        int section = 0, head = 0;
+        if constexpr (QKV) {
+            const int per_section = a.Hn * 128;
+            section = f0 / per_section;
+            head = (f0 - section * per_section) >> 7;
+            if (a.bias != nullptr) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const uint2 raw = *reinterpret_cast<const uint2*>(a.bias + f0 + 16 * i + 4 * lg);
+                    const __bf16* bv = reinterpret_cast<const __bf16*>(&raw);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][j][e] += (float)bv[e];
+                }
+            }
+            if (section < 2) {
 #pragma clang fp contract(off)       // every product and sum below is rounded on its own, as in the eager expressions
-            constexpr int D = 128;
-            constexpr int nt = (D - 4 * (D / 6)) / 2, nh = D / 6, nw = D / 6;    // rotation pairs per axis: 22, 21, 21
-            const __bf16* nwgt = a.norm_w[section];
-            // the projection output is a bf16 tensor in the module this replaces: round before normalising
+                constexpr int D = 128;
+                constexpr int nt = (D - 4 * (D / 6)) / 2, nh = D / 6, nw = D / 6;    // rotation pairs per axis: 22, 21, 21
+                const __bf16* nwgt = a.norm_w[section];
+                // the projection output is a bf16 tensor in the module this replaces: round before normalising
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                float ss = 0.f;
+                for (int j = 0; j < 4; ++j) {
+                    float ss = 0.f;
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                    for (int i = 0; i < 8; ++i)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const float v = (float)(__bf16)acc[i][j][r];
-                        acc[i][j][r] = v;
-                        ss = fmaf(v, v, ss);
-                    }
-                ss += __shfl_xor(ss, 32);
-                const float rs = __builtin_amdgcn_rsqf(ss * (1.0f / (float)D) + a.eps);    // as bsa_rope.h
-                // position of this lane's token of block j
-                const uint32_t tok = (uint32_t)min(m0 + 32 * j + (lane & 31), a.M - 1);
-                const uint32_t s = tok % (uint32_t)a.S;
-                const uint32_t u = s / (uint32_t)a.Wg, v2 = u / (uint32_t)a.Hg;
-                const int wi = (int)(s - u * a.Wg), hi = (int)(u - v2 * a.Hg), ti = a.t0 + (int)v2;
-                const int sin_t = a.Ttab * nt, cos_h = 2 * a.Ttab * nt, sin_h = a.Hg * nh, cos_w = cos_h + 2 * a.Hg * nh,
-                          sin_w = a.Wg * nw;
+                        for (int r = 0; r < 4; ++r) {
+                            const float v = (float)(__bf16)acc[i][j][r];
+                            acc[i][j][r] = v;
+                            ss = fmaf(v, v, ss);
+                        }
+                    ss += __shfl_xor(ss, 16);
+                    ss += __shfl_xor(ss, 32);
+                    const float rs = __builtin_amdgcn_rsqf(ss * (1.0f / (float)D) + a.eps);    // as bsa_rope.h
+                    // position of this lane's token of block j
+                    const uint32_t tok = (uint32_t)min(m0 + 16 * j + (int)lr, a.M - 1);
+                    const uint32_t s = tok % (uint32_t)a.S;
+                    const uint32_t u = s / (uint32_t)a.Wg, v2 = u / (uint32_t)a.Hg;
+                    const int wi = (int)(s - u * a.Wg), hi = (int)(u - v2 * a.Hg), ti = a.t0 + (int)v2;
+                    const int cos_h = 2 * a.Ttab * nt, cos_w = cos_h + 2 * a.Hg * nh;
+                    const int at_t = ti * nt, at_h = cos_h + hi * nh - nt, at_w = cos_w + wi * nw - nt - nh;     // + pair: cosines
+                    const int to_sin_t = a.Ttab * nt, to_sin_h = a.Hg * nh, to_sin_w = a.Wg * nw;
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint2 raw = *reinterpret_cast<const uint2*>(nwgt + 32 * i + 8 * q + 4 * g);
+                    for (int i = 0; i < 8; ++i) {
+                        const uint2 raw = *reinterpret_cast<const uint2*>(nwgt + 16 * i + 4 * lg);
                         const __bf16* wv = reinterpret_cast<const __bf16*>(&raw);
                         float f[4];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            f[e] = (float)(__bf16)((float)(__bf16)(acc[i][j][4 * q + e] * rs) * (float)wv[e]);
+                        for (int e = 0; e < 4; ++e) f[e] = (float)(__bf16)((float)(__bf16)(acc[i][j][e] * rs) * (float)wv[e]);
 #pragma unroll
                         for (int e = 0; e < 2; ++e) {
-                            const int pair = 16 * i + 4 * q + 2 * (int)g + e;
-                            int at, dsin;
-                            if (pair < nt) { at = ti * nt + pair; dsin = sin_t; }
-                            else if (pair < nt + nh) { at = cos_h + hi * nh + pair - nt; dsin = sin_h; }
-                            else { at = cos_w + wi * nw + pair - nt - nh; dsin = sin_w; }
-                            const float c = a.tab[at], sn = a.tab[at + dsin];
+                            const int pair = 8 * i + 2 * (int)lg + e;         // 8 i .. 8 i + 7: most blocks lie within one axis
+                            const bool in_t = 8 * i + 7 < nt || (8 * i < nt && pair < nt), in_w = 8 * i >= nt + nh || (8 * i + 7 >= nt + nh && pair >= nt + nh);
+                            const int at = (in_t ? at_t : in_w ? at_w : at_h) + pair;
+                            const float c = a.tab[at], sn = a.tab[at + (in_t ? to_sin_t : in_w ? to_sin_w : to_sin_h)];
                             const float x0 = f[2 * e], x1 = f[2 * e + 1];
                             // two products, then one add, each rounded: the order of operations of the eager expression
-                            acc[i][j][4 * q + 2 * e] = x0 * c + (-x1) * sn;
-                            acc[i][j][4 * q + 2 * e + 1] = x1 * c + x0 * sn;
+                            acc[i][j][2 * e] = x0 * c + (-x1) * sn;
+                            acc[i][j][2 * e + 1] = x1 * c + x0 * sn;
                         }
                     }
+                    __builtin_amdgcn_sched_barrier(0);       // one block's table entries at a time: registers
+                }
             }
         }
-    }
-    // through LDS into token rows, 64 tokens at a time, then 16 bytes per lane to global memory
+        // Two blocks of 16 features change places between the lanes so that a lane has eight features of its token in a row: 16
+        // bytes of it, 64 of the four lanes that share it.
+        const int piece = 16 * (lg & 1) + 8 * (lg >> 1);
+        uint2 bias[8];
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
+        for (int i = 0; i < 8; ++i) bias[i] = make_uint2(0, 0);
+        if (!QKV && a.bias != nullptr) {
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj) {
-            const int j = 2 * half + jj;
-            char* row = stage_area + (32 * jj + (lane & 31)) * kEpiPitch + 8 * g;
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    __bf16 v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = (__bf16)acc[i][j][4 * q + e];
-                    *reinterpret_cast<uint2*>(row + (32 * i + 8 * q) * 2) = *reinterpret_cast<const uint2*>(v);
-                }
+            for (int i = 0; i < 8; ++i) bias[i] = *reinterpret_cast<const uint2*>(a.bias + f0 + 16 * i + 4 * lg);
         }
-        __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0): this wavefront's LDS writes have landed
-#pragma unroll 4
-        for (int it = 0; it < 16; ++it) {
-            const int lrow = 4 * it + (lane >> 4);
-            const int tok = m0 + 64 * half + lrow;
-            const uint4 val = *reinterpret_cast<const uint4*>(stage_area + lrow * kEpiPitch + (lane & 15) * 16);
-            if (tok < a.M) {
-                __bf16* o;
+#pragma unroll
+        for (int jj = 0; jj < 4; jj += 2) {
+            uint4 res[2][4];
+            if constexpr (kEpi == kResidual) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const __bf16* row = a.residual + (int64_t)min(m0 + 16 * (jj + j) + (int)lr, a.M - 1) * a.ldr + f0 + piece;
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) res[j][p] = *reinterpret_cast<const uint4*>(row + 32 * p);
+                }
+            }
+#pragma unroll
+            for (int j = jj; j < jj + 2; ++j) {
+                const int tok = m0 + 16 * j + (int)lr;
+                __bf16* to;
                 if constexpr (QKV) {
                     const uint32_t bb = (uint32_t)tok / (uint32_t)a.S, s = (uint32_t)tok - bb * (uint32_t)a.S;
-                    o = a.dst[section] + bb * a.dB + head * a.dH + s * a.dS;
+                    to = a.dst[section] + bb * a.dB + head * a.dH + s * a.dS;
                 } else {
-                    o = a.out + (int64_t)tok * a.ldo + f0;
+                    to = a.out + (int64_t)tok * a.ldo + f0;
                 }
-                *reinterpret_cast<uint4*>(o + (lane & 15) * 8) = val;
+                uint4 o[4];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    float v[2][4];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            v[h][e] = QKV ? acc[2 * p + h][j][e] : acc[2 * p + h][j][e] + (float)reinterpret_cast<const __bf16*>(&bias[2 * p + h])[e];
+                    if constexpr (kEpi == kResidual) {
+                        const uint4 r = res[j - jj][p];
+                        const auto lo = __builtin_amdgcn_permlane16_swap(r.x, r.z, false, false);
+                        const auto hi = __builtin_amdgcn_permlane16_swap(r.y, r.w, false, false);
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const uint32_t raw[2] = {lo[h], hi[h]};
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) v[h][e] += (float)reinterpret_cast<const __bf16*>(raw)[e];
+                        }
+                    }
+                    uint32_t w[2][2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) {
+                            const __bf16 two[2] = {(__bf16)v[h][2 * e], (__bf16)v[h][2 * e + 1]};
+                            w[h][e] = *reinterpret_cast<const uint32_t*>(two);
+                        }
+                    const auto lo = __builtin_amdgcn_permlane16_swap(w[0][0], w[1][0], false, false);
+                    const auto hi = __builtin_amdgcn_permlane16_swap(w[0][1], w[1][1], false, false);
+                    o[p] = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+                }
+                if (tok < a.M) {
+#pragma unroll
+                    for (int p = 0; p < 4; ++p) *reinterpret_cast<uint4*>(to + 32 * p + piece) = o[p];
+                }
             }
         }
-        __builtin_amdgcn_s_waitcnt(0xc07f);   // the rows are read before the next half overwrites them
     }
 }
 
 
-template <bool QKV>
+template <int kEpi>
 int launch_gemm(GemmArgs& a, hipStream_t stream) {
     a.tiles_m = (a.M + kTileM - 1) / kTileM;
     a.tiles_n = (a.N + kTileN - 1) / kTileN;
-    a.super_m = (a.tiles_m + kSuperM - 1) / kSuperM;
-    a.super_total = a.super_m * ((a.tiles_n + kSuperN - 1) / kSuperN);
-    const unsigned grid = (unsigned)((a.super_total + 7) / 8) * 256u;
+    const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
+    const unsigned grid = (unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, kCus);
     const size_t lds = (size_t)kStages * kPart;
-    static_assert(kStages * kPart >= 4 * kEpiBytes, "the staging area reuses the slabs");
-    auto kernel = gemm_nt_kernel<QKV>;
+    auto kernel = gemm_nt_kernel<kEpi>;
     // more than the 64 KB a kernel gets without asking; the attribute is per device, so it is set on every call
     const hipError_t ea = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (ea != hipSuccess) return set_error(BSA_ERR_HIP, "gemm: LDS size: %s", hipGetErrorString(ea));
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), lds, stream, a);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), lds, stream, a);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? BSA_OK : set_error(BSA_ERR_HIP, "gemm launch: %s", hipGetErrorString(e));
 }
@@ -375,6 +379,28 @@ int check_gemm_operands(const char* what, const void* x, int64_t ldx, const void
 }
 
 }  // namespace
+
+// Which linear layers (bsa_linear_bf16) this kernel serves: us of hipBLASLt (with a residual: an fp32 product and residual_add_kernel) /
+// of this kernel.  With a residual where the tiles fill the rounds of 256 that they take to four fifths: 86 400 x 4 096 x 4 096 2 668 / 2 241, 4 096 rows
+// 123 / 106, 2 048 (128 tiles) 72 / 82, 256 (16 tiles) 23 / 74, 8 192 x 2 048 x 2 048 80 / 58, 16 384 x 1 024 x 1 024 58 / 36; and where K is short, whatever
+// the tiles: K = 256 16.9 / 10.7 for 16 rows, 60 / 33 for 86 400, 512 columns and K rows from 16 to 8 192 level.  Without one only there: K = 128 and
+// 384 columns 14.2 / 9.9 (1 000 rows) to 37.6 / 27.2 (86 400), K = 256 and 768 13.9 / 12.1 to 67 / 53; the library's host time is 14.
+// Rows must be those of whole 16-byte pieces, and out nowhere else than in a place of its own or the residual's: the
+// library's route has read x before it writes a result, this kernel has not.
+bool gemm_serves_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual, const void* out, int64_t ldo,
+                        int64_t M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || K % kBK || N % 128 || ldx % 8 || ldw % 8 || ldo % 8 || ldx < K || ldw < K || ldo < N || ldx >= (1 << 22) || ldw >= (1 << 22)) return false;
+    const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+    if (((at(x) | at(w) | at(out) | at(residual)) & 15u) || (at(bias) & 7u)) return false;
+    const auto rows = [](int64_t n, int64_t pitch, int64_t width) { return (uintptr_t)((n - 1) * pitch + width) * 2u; };
+    const uintptr_t o = at(out), o_end = o + rows(M, ldo, N);
+    const auto meets = [&](const void* p, uintptr_t bytes) { return p != nullptr && at(p) < o_end && o < at(p) + bytes; };
+    if (meets(x, rows(M, ldx, K)) || meets(w, rows(N, ldw, K)) || meets(bias, (uintptr_t)N * 2u) || (residual != out && meets(residual, o_end - o))) return false;
+    if (K <= 256) return true;
+    const int64_t tiles = (M + kTileM - 1) / kTileM * ((N + kTileN - 1) / kTileN), round = (tiles + kCus - 1) / kCus * kCus;
+    return residual != nullptr && 5 * tiles >= 4 * round;
+}
+
 }  // namespace bsa
 
 using namespace bsa;
@@ -394,7 +420,7 @@ int bsa_gemm_bf16(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
     a.x = (const __bf16*)x; a.ldx = ldx; a.w = (const __bf16*)w; a.ldw = ldw; a.bias = (const __bf16*)bias;
     a.residual = (const __bf16*)residual; a.ldr = ldr; a.out = (__bf16*)out; a.ldo = ldo;
     a.M = (int)M; a.N = N; a.K = K;
-    return launch_gemm<false>(a, (hipStream_t)stream);
+    return residual ? launch_gemm<kResidual>(a, (hipStream_t)stream) : launch_gemm<kPlain>(a, (hipStream_t)stream);
 }
 
 int bsa_qkv_projection(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* q_weight,
@@ -424,7 +450,7 @@ int bsa_qkv_projection(const void* x, int64_t ldx, const void* w, int64_t ldw, c
     a.dB = dst_strides[0]; a.dH = dst_strides[1]; a.dS = dst_strides[2];
     a.norm_w[0] = (const __bf16*)q_weight; a.norm_w[1] = (const __bf16*)k_weight;
     a.tab = rope_table; a.Hn = Hn; a.S = (int)S; a.Hg = H; a.Wg = W; a.t0 = t_offset; a.Ttab = table_T; a.eps = eps;
-    return launch_gemm<true>(a, (hipStream_t)stream);
+    return launch_gemm<kQkv>(a, (hipStream_t)stream);
 }
 
 }  // extern "C"

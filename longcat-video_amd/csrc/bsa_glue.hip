@@ -657,6 +657,12 @@ size_t bsa_linear_bf16_workspace_bytes(int64_t M, int N, int with_residual) {
     return kLtWorkspace + (with_residual ? ((size_t)M * N * sizeof(float) + 255) / 256 * 256 + 256 : 0);
 }
 
+size_t bsa_linear_bf16_ld_workspace_bytes(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
+                                          const void* out, int64_t ldo, int64_t M, int N, int K) {
+    if (!x || !w || !out) return 0;
+    return bsa_linear_bf16_workspace_bytes(M, N, residual != nullptr && !gemm_serves_linear(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K));
+}
+
 static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
                        void* out, int64_t ldo, int64_t M, int N, int K, void* workspace, size_t workspace_bytes,
                        void* stream, bool tune, float* default_ms, float* best_ms) {
@@ -668,6 +674,8 @@ static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, c
     // want just under 64 MiB (1.52 PFLOP/s instead of 1.24 with 32 MiB); more brings nothing.
     if (!workspace || workspace_bytes < kLtWorkspace)
         return set_error(BSA_ERR_WORKSPACE, "linear: a workspace of at least 64 MiB is required (got %zu bytes)", workspace_bytes);
+    if (!tune && gemm_serves_linear(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K))
+        return bsa_gemm_bf16(x, ldx, w, ldw, bias, residual, ldo, out, ldo, M, N, K, stream);
     if (!residual) return lt_product(x, ldx, w, ldw, bias, out, ldo, false, M, N, K, workspace, workspace_bytes, stream, tune, default_ms, best_ms);
 
     // With a residual the product goes to fp32 behind the library's share of the workspace, as many rows (and columns) at a time

@@ -88,13 +88,14 @@ def _gemm_workspace(device) -> torch.Tensor:
     return ws
 
 
-def _linear_workspace(M: int, N: int, residual: bool, device) -> torch.Tensor:
-    """What a linear of M rows and N columns works in: with a residual also the fp32 product, in the kept workspace's second half
-    if that holds it, otherwise from torch's allocator for the one call, and where the card has no room for it in groups of rows."""
-    if not residual or 4 * M * N + 256 <= 32 << 20:
+def _linear_workspace(M: int, N: int, need, device) -> torch.Tensor:
+    """What a linear of M rows and N columns works in: with a residual possibly also the fp32 product, in the kept workspace's second
+    half if that holds it, otherwise, if the call has use for more (`need` says), from torch's allocator for the one call, and where the
+    card has no room for it in groups of rows."""
+    if need is None or 4 * M * N + 256 <= 32 << 20:
         return _gemm_workspace(device)
-    need = _capi.load().bsa_linear_bf16_workspace_bytes(M, N, 1)
-    return _backward_workspace(need, 64 << 20, device)
+    nbytes = need()
+    return _gemm_workspace(device) if nbytes <= 64 << 20 else _backward_workspace(nbytes, 64 << 20, device)
 
 
 def _bf16(t: torch.Tensor) -> torch.Tensor:
@@ -125,7 +126,9 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
         r = residual if residual.is_contiguous() else residual.reshape(-1, N).contiguous()
         assert r.numel() == M * N and r.dtype == torch.bfloat16
     if workspace is None:
-        workspace = _linear_workspace(M, N, r is not None, x.device)
+        need = None if r is None else lambda: _capi.load().bsa_linear_bf16_ld_workspace_bytes(
+            _ptr(x2), K, _ptr(w), K, _ptr(b), _ptr(r), _ptr(out), N, M, N, K)
+        workspace = _linear_workspace(M, N, need, x.device)
     with _on_device(x):
         _capi.check(_capi.load().bsa_linear_bf16(_ptr(x2), _ptr(w), _ptr(b), _ptr(r), _ptr(out), M, N, K,
                                                  _ptr(workspace), workspace.numel(), _stream(x)), "linear")
@@ -146,7 +149,8 @@ def tune_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     out = torch.empty(x2.shape[0], N, dtype=torch.bfloat16, device=x.device)
     r = torch.zeros_like(out) if residual else None
     if workspace is None:
-        workspace = _linear_workspace(x2.shape[0], N, residual, x.device)
+        need = None if not residual else lambda: _capi.load().bsa_linear_bf16_workspace_bytes(x2.shape[0], N, 1)
+        workspace = _linear_workspace(x2.shape[0], N, need, x.device)
     d, best = C.c_float(0), C.c_float(0)
     with _on_device(x):
         n = _capi.load().bsa_linear_bf16_tune(_ptr(x2), K, _ptr(w), K, _ptr(b), _ptr(r), _ptr(out), N, x2.shape[0], N, K,

@@ -148,6 +148,30 @@ def test_fwd_3d_plan_and_workspace():
     assert lib.bsa_fwd_3d(None, *args, ws, need, None, None, None, None) == _capi.BSA_ERR_BAD_ARG
 
 
+def test_which_linear_layers_work_without_a_product():
+    """With a residual, a layer that the engine's GEMM serves needs the 64 MiB that every call brings; any other an fp32 product too."""
+    lib = _capi.load()
+    least = 64 << 20
+
+    def alone(x=0x100000000, ldx=1024, w=0x200000000, ldw=1024, bias=0x300000000, res=0x400000000, out=0x500000000, ldo=1024, M=65536, N=1024, K=1024):
+        p = lambda v: None if v is None else C.c_void_p(v)      # noqa: E731
+        got = lib.bsa_linear_bf16_ld_workspace_bytes(p(x), ldx, p(w), ldw, p(bias), p(res), p(out), ldo, M, N, K)
+        assert got in (least, lib.bsa_linear_bf16_workspace_bytes(M, N, 1)) and lib.bsa_linear_bf16_workspace_bytes(M, N, 1) > least
+        return got == least
+
+    assert alone() and alone(bias=None) and alone(out=0x400000000) and alone(M=16 * 256 * 4) and alone(K=64, M=3)
+    assert alone(res=None)                                          # no residual: no product either
+    assert not alone(M=256) and not alone(M=70 * 256)               # 4 tiles; 280: two rounds of 256, little more than half full
+    assert alone(M=90 * 256 * 4)
+    assert not alone(K=1000, ldx=1000) and not alone(N=1000) and not alone(ldx=1028) and not alone(ldo=1028)
+    for bad in ("x", "w", "res", "out"):
+        assert not alone(**{bad: 0x600000008})
+    assert not alone(bias=0x300000004) and alone(bias=0x300000008)
+    # results over operands that are still read: only in the residual's own place
+    assert not alone(out=0x100000000) and not alone(out=0x200000000) and not alone(out=0x400000800) and not alone(out=0x300000000)
+    assert not alone(out=0x100000000 + (65536 * 1024 * 2 - 16)) and alone(out=0x100000000 + 65536 * 1024 * 2)
+
+
 def test_gemm_and_qkv_projection_reject_bad_arguments():
     lib = _capi.load()
 

@@ -49,6 +49,21 @@ def test_gemm_is_exact_on_integers():
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 320, 384])
+@pytest.mark.parametrize("m,n", [(1, 128), (255, 256), (257, 384), (2309, 6656), (4864, 3456)])
+def test_gemm_goes_from_tile_to_tile(m, n, k):
+    """One tile, edges in both directions, and more tiles than workgroups (10 x 26, the second block of token tiles of two, and 19 x 14 of which the
+    last is half empty): the requests run on from a tile into the next, from a tile of one k block too.  Small integers, exact."""
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    ints = lambda *s: torch.randint(-2, 3, s, generator=g, device="cuda").bfloat16()      # noqa: E731
+    x, w, b, r = ints(m, k), ints(n, k), ints(n), ints(m, n) * 37
+    want = (x.float() @ w.float().T + b.float())
+    for res in (None, r):
+        got = M().gemm_bf16(x, w, b, residual=res)
+        assert torch.equal(got, (want if res is None else want + res.float()).bfloat16())
+    assert torch.equal(M().gemm_bf16(x, w, b, residual=r, out=r), got)                # in the residual's place
+
+
 def test_gemm_with_row_strides():
     """Operands and output as column slices of wider tensors (row strides above K and N)."""
     g = torch.Generator().manual_seed(6)
