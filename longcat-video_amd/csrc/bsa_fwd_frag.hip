@@ -5,7 +5,7 @@
 // byte is written once and read twice (two wavefronts share each 32-key half): 96 KB of LDS
 // traffic per 64 x 64 tile against 512 clocks of MFMA per SIMD, which makes LDS, not the matrix
 // unit, its roofline.  Here a wavefront owns all 64 query rows of a work item, so every K and V
-// fragment feeds two MFMAs (one per 32 query rows) and is needed by this wavefront alone: it is
+// fragment feeds four MFMAs (one per 16 query rows) and is needed by this wavefront alone: it is
 // loaded from global memory straight into registers, in exactly the lane order the MFMA operand
 // wants, and LDS carries nothing in the tile loop - no staging, no swizzle, no barrier.  That
 // needs K and V in a layout whose every 1 KB is one operand fragment (below), written once per
@@ -13,19 +13,22 @@
 // replaces the zero-filled copies of the chunks at the padded high edge of the grid).
 //
 // Fragment order, per 64-key tile (16 KB for K, 16 KB for V; two 8 KB halves of 32 keys):
-//   K: [half kh][d step c = 0..7][lane l = 0..63][8 elements]
-//        element j of lane l = K[key 32 kh + (l & 31)][d = 16 c + 8 (l >> 5) + j]
-//      = the A operand of v_mfma_f32_32x32x16 for S^T (32 keys x 32 queries) += K . Q^T.
-//   V: [half kh][key step s = 0..1][d tile t = 0..3][lane l][8 elements]
-//        element j of lane l = V[key 32 kh + 16 s + 8 (j >> 2) + 4 (l >> 5) + (j & 3)][d = 32 t + (l & 31)]
-//      = the A operand of O^T (32 d x 32 queries) += V^T . P^T, with the 16 keys of a step in the
+//   K: [half kh][d step c = 0..3][key block kb = 0..1][lane l = 0..63][8 elements]
+//        element j of lane l = K[key 32 kh + 16 kb + (l & 15)][d = 32 c + 8 (l >> 4) + j]
+//      = the A operand of v_mfma_f32_16x16x32 for S^T (16 keys x 16 queries) += K . Q^T.
+//   V: [half kh][d tile t = 0..7][lane l][8 elements]
+//        element j of lane l = V[key 32 kh + 16 (j >> 2) + 4 (l >> 4) + (j & 3)][d = 16 t + (l & 15)]
+//      = the A operand of O^T (16 d x 16 queries) += V^T . P^T, with the 32 keys of a step in the
 //        order in which the accumulator registers of S^T hold them, so that P^T needs no shuffle.
+//
+// 16x16x32 and not 32x32x16: the board's power is what bounds this kernel, and the small form moves half as many
+// accumulators per multiplication (MFMAs alone on random data: 2 080 TFLOP/s against 1 820).
 //
 // Work decomposition.  One wavefront (a workgroup of 64 threads, one per SIMD; of small calls two or four,
 // see kTeam) = one work item =
 // 64 query rows against its list of KV blocks, walked in steps of 32 keys (half a tile).  Per
-// step: 16 MFMAs for S^T of the next step interleaved with the exp2 / row sum / rounding of the
-// current one, then 16 MFMAs for O^T += V^T P^T interleaved with the row maximum of the next.
+// step: 32 MFMAs for S^T of the next step interleaved with the exp2 / row sum / rounding of the
+// current one, then 32 MFMAs for O^T += V^T P^T interleaved with the row maximum of the next.
 // K and V fragments of the following steps are in flight in register rings (kRing steps each).
 // The output accumulators (128 registers) and the rings live in the 512-register file that a
 // single wavefront per SIMD has to itself.
@@ -159,6 +162,16 @@ __host__ __device__ inline int gate_here_bytes(int nbk, int width, int nsub, boo
     return (gate_list_words(width, nsub, halves) + gate_wave_words(width) + 4) * 4 + (nbk + 31) / 32 * 64 + (halves ? (nbk * nsub + 15) / 16 * 16 : 0);
 }
 
+// The first of a step's 96 pieces (six a pair, nine instructions' time) that stands behind MFMA g or a later one, in the kernel with maxima.
+constexpr int first_piece(int g) {
+    for (int p = 0; p < 96; ++p) {
+        constexpr int before[6] = {0, 2, 3, 4, 6, 7};
+        const int t = 9 * (p / 6) + before[p % 6];
+        if ((t < 126 ? t * 48 / 126 : 48 + (t - 126) * 16 / 18) >= g) return p;
+    }
+    return 96;
+}
+
 template <typename T, int kWalk, bool kBounded, int kTeam, bool kGate>
 __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
@@ -202,11 +215,12 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
     __shared__ __attribute__((aligned(8))) uint32_t lists[2][kOnce ? 2 : kPipeList * kWords];
     __shared__ int32_t out_rows[2][kTile];       // token rows of this and the next item's 64 query slots (row table given)
     __shared__ __attribute__((aligned(16))) char qstage[kOnce ? 16 : kTileBytes];      // Q of the next item, in register order
+    __shared__ __attribute__((aligned(16))) char scale_room[kBounded ? 16 : kTeam > 1 ? 1024 * kTeam : 1024];
     uint32_t* const big = reinterpret_cast<uint32_t*>(ost);
 
     const int lane = threadIdx.x & 63;
     const int wave = kTeam > 1 ? __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : 0;
-    const int lr = lane & 31, lh = lane >> 5;
+    const int lr = lane & 15, lg = lane >> 4;
     const int nqt = (int)(Sq / kTile);
     const int nsub = kWalk == kBlocks ? bs_k / kTile : 1, nsub_of_block = bs_k / kTile;
     const int tiles_bh = (int)(Sk / kTile), nbk = kWalk == kBlocks ? tiles_bh / L.by_sub : tiles_bh;     // kHalves does not ask for it
@@ -221,14 +235,12 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kf) + bh_first * kv_bh_bytes, 0, (int)kv_span_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t vrs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(vf) + bh_first * kv_bh_bytes, 0, (int)kv_span_bytes, 0x00020000);
-    // half: index of the 32-key half counted from (batch, head) bh_first; c / f: fragment of the half
-    auto k_frag = [&](uint32_t half, int c) -> V8 {
-        const uint32_t so = half * (uint32_t)kHalfBytes + (uint32_t)((c >> 2) * 4096);
-        return __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(krs, lane_off + (uint32_t)((c & 3) * 1024), so, 0));
+    // at: byte offset of a 32-key half, counted from (batch, head) bh_first; c / f: fragment of the half
+    auto k_frag = [&](uint32_t at, int c) -> V8 {
+        return __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(krs, lane_off + (uint32_t)((c & 3) * 1024), at + (uint32_t)((c >> 2) * 4096), 0));
     };
-    auto v_frag = [&](uint32_t half, int f) -> V8 {          // f = 4 * key step + d tile
-        const uint32_t so = half * (uint32_t)kHalfBytes + (uint32_t)((f >> 2) * 4096);
-        return __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(vrs, lane_off + (uint32_t)((f & 3) * 1024), so, 0));
+    auto v_frag = [&](uint32_t at, int f) -> V8 {          // f: d tile
+        return __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(vrs, lane_off + (uint32_t)((f & 3) * 1024), at + (uint32_t)((f >> 2) * 4096), 0));
     };
 
     // ---- which items this workgroup runs
@@ -298,56 +310,66 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
     };
 
     // ---- registers that live across items
-    V8 qreg[2][8];
-    // Register rings: K fragments of two steps, V fragments of two steps (each step: 4 fragments for its
-    // first 16 keys, "A", and 4 for its last 16, "B").
+    V8 qreg[4][4];                                             // [16 queries][d step]
+    // Register rings: K and V fragments of two steps.
     V8 kb[2][8], vb[2][8];
-    f32x16 s[2][2];                                            // S^T of the current and of the next step
-    V8 pb[2][2];                                               // P^T as B operand: [query half][A | B]
-    f32x16 oacc[4][2];
-    float m_i[2], l_i[2];
-    // Softmax state per query half: running maximum m_i (scaled, log2 units), its negative for the exponent
-    // (0 while the maximum is -inf), and the unscaled logit above which the maximum has to be raised.
-    float neg_m[2], raise_at[2];
+    f32x4_ s[2][2][4];                                         // S^T of the current and of the next step: [][key block][16 queries]
+    V8 pb[4];                                                  // P^T as B operand, by 16 queries
+    f32x4_ oacc[8][4];
+    float m_i[4], l_i[4];
+    // Softmax state per 16 queries: running maximum m_i (scaled, log2 units), its negative for the exponent
+    // (0 while the maximum is -inf), and the unscaled logit above which the maximum has to be raised; the lowest of these.
+    float neg_m[4], raise_at[4], raise_low;
     const float inv_scale = 1.0f / qk_scale;
     // Raising the
     // maximum has two parts.  Here: the new maximum, the exponent offset, the row sum (which already holds
     // every probability of the current step).  The output accumulators are rescaled one quarter of a step later
-    // (rescale_out, behind slot 7 of the next step): the product of the current step's P_B, whose
-    // probabilities were taken relative to the old maximum, is only issued in slots 0 .. 7 of that step.
-    float alpha_p[2];
+    // (rescale_out, behind slot 7 of the next step): the products of the current step's queries 32 .. 63, whose
+    // probabilities were taken relative to the old maximum, are only issued in slots 0 .. 7 of that step.
+    float alpha_p[4];
     bool rescale_pending = false;
 
-    // Q fragments of one query half into their registers, and the lane's part of the rows' squared norms.  Half 1 is
-    // read by the assembly MFMAs from accumulation registers.  Its values pass through an assembly statement that
+    // Q fragments of 16 queries into their registers, and the lane's part of the rows' squared norms.  The queries 32 .. 63 are
+    // read by the assembly MFMAs from accumulation registers.  Their values pass through an assembly statement that
     // ties them to that register class: a value that C++ code also reads (the squares) the compiler would keep in
     // ordinary registers and copy in front of every MFMA that names it, without the wait states such a copy needs.
-    float q_sq[2] = {0.f, 0.f};
-    auto take_q = [&](int qq, V8 (&rows)[8]) {
+    float q_sq[4] = {0.f, 0.f, 0.f, 0.f};
+    auto take_q = [&](int qb, V8 (&rows)[4]) {
         float sq = 0.f;
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
+        for (int c = 0; c < 4; ++c)
 #pragma unroll
             for (int e = 0; e < 4; ++e) sq = dot2_self(rows[c], e, sq);
-        q_sq[qq] = sq;
+        q_sq[qb] = sq;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (qq == 1) asm volatile("" : "=a"(qreg[1][c]) : "0"(rows[c]));
-            else asm volatile("" : "=v"(qreg[0][c]) : "0"(rows[c]));
+        for (int c = 0; c < 4; ++c) {
+            asm volatile("" : "=a"(qreg[qb][c]) : "0"(rows[c]));
         }
     };
+    // a sum or a maximum over the four lanes that share a query
+    auto over_lanes = [](float x, auto f) -> float {
+        const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        const float y = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+        const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(y), __float_as_uint(y), false, false);
+        return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    };
+    const auto add = [](float a, float b) { return a + b; };
 
     // ---- per item
     int npairs = 0, pair0 = 0;       // the walk covers the pairs pair0 .. pair0 + npairs - 1 of the list
     int n_halves = 0;                // a team's walk over halves: those of this wavefront's share, from ents on
     uint32_t half_base = 0;          // first half of the item's (batch, head)
-    uint32_t beyond[2] = {0, 0};     // what the positions behind the end of the list name
+    uint32_t beyond[2] = {0, 0};     // the entries of the positions behind the end of the list
     const uint32_t* ents = big;      // the item's list in LDS
-    // window of the walk: the halves 2 g + 1 .. 2 g + 5 of loop iteration g (one pair per iteration) and the keys to keep
-    uint32_t w_half[5], w_mask[5];
+    // window of the walk: the entries of the halves 2 g + 1 .. 2 g + 5 of loop iteration g (one pair per iteration).  An entry is a half,
+    // counted from half_base, | real keys << 20, as kHalves lists hold them; what is above 2^19 halves is lost in the shift to
+    // bytes.
+    uint32_t w[5];
+    auto offset_of = [&](uint32_t entry) -> uint32_t { return (entry << 13) + (half_base << 13); };
+    static_assert(kHalfBytes == 1 << 13, "the shift");
 
-    // Pair tp of the walk -> its halves and the keys of theirs that count (bit i: key i).  Positions behind the list name
-    // `beyond` with every key masked out.  The entry is read from LDS (pair_raw, to be issued early) and decoded later.
+    // Pair tp of the walk -> its entries.  Positions behind the list name `beyond`, no key of theirs.  The list is read from LDS
+    // (pair_raw, to be issued early) and made into entries later.
     struct Raw { uint32_t e[kWords]; };
     auto pair_raw = [&](int tp) -> Raw {
         const int tc = min(tp, npairs - 1) + pair0;
@@ -364,210 +386,221 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         }
         return r;
     };
-    auto count_mask = [&](int n) -> uint64_t { return n >= 64 ? ~0ull : ((uint64_t)1 << n) - 1; };
-    auto pair_halves = [&](int tp, const Raw& raw, uint32_t (&h)[2]) {
-        if (kWalk == kHalves) {
-#pragma unroll
-            for (int x = 0; x < kWords; ++x)
-                h[x] = tp >= npairs ? beyond[x] : half_base + ((uint32_t)uni((int)raw.e[x]) & kHalfId);
-            return;
-        }
-        if (tp >= npairs) { h[0] = beyond[0]; h[1] = beyond[1]; return; }
+    // first half of the pair's tile, counted from half_base (kTiles, kBlocks)
+    auto tile_half = [&](int tp, const Raw& raw) -> uint32_t {
+        if (tp >= npairs) return 0;
         const int blk = min(max(uni((int)raw.e[0]), 0), nbk - 1);                          // a malformed list: wrong numbers, never a fault
         const int tc = tp + pair0;
-        h[0] = half_base + 2u * (uint32_t)(kWalk == kTiles ? blk : blk * nsub + tc - tc / L.by_sub * nsub);
-        h[1] = h[0] + 1u;
+        return 2u * (uint32_t)(kWalk == kTiles ? blk : blk * nsub + tc - tc / L.by_sub * nsub);
     };
     // the validity word of a pair's tile (all keys valid without padding; kHalves: the entries say it), in two steps so that
     // a caller can ask for several words before it waits for the first
-    auto pair_word = [&](int tp, const uint32_t (&h)[2]) -> uint64_t {
-        if (kWalk == kHalves || tile_valid == nullptr) return ~0ull;
-        return tile_valid[tp >= npairs ? 0u : (h[0] - half_base) >> 1];                    // behind the list: another head's tile
-    };
-    auto pair_masks = [&](int tp, const Raw& raw, uint64_t word, uint32_t (&m)[2]) {
-        const uint32_t keep = tp >= npairs ? 0u : ~0u;
-        if (kWalk == kHalves) {
+    auto pair_word = [&](uint32_t half) -> uint64_t { return kWalk == kHalves || tile_valid == nullptr ? ~0ull : tile_valid[half >> 1]; };
+    auto pair_entries = [&](int tp, const Raw& raw, uint32_t half, uint64_t word, uint32_t (&e)[2]) {
+        if (tp >= npairs) {
+            e[0] = beyond[0];
+            e[1] = beyond[1];
+        } else if (kWalk == kHalves) {
 #pragma unroll
-            for (int x = 0; x < kWords; ++x) m[x] = (uint32_t)count_mask(uni((int)raw.e[x]) >> kHalfCountShift) & keep;
-            return;
+            for (int x = 0; x < kWords; ++x) e[x] = (uint32_t)uni((int)raw.e[x]);
+        } else {
+            // the same word in every lane; made a scalar by hand (behind the stores of an earlier item's output the
+            // compiler reads it with a vector load)
+            const uint32_t lo = (uint32_t)uni((int)(uint32_t)word), hi = (uint32_t)uni((int)(uint32_t)(word >> 32));
+            const int n = __builtin_popcountll((uint64_t)lo | ((uint64_t)hi << 32));
+            e[0] = half | (uint32_t)min(n, 32) << kHalfCountShift;
+            e[1] = (half + 1u) | (uint32_t)max(n - 32, 0) << kHalfCountShift;
         }
-        // the same word in every lane; made a scalar by hand (behind the stores of an earlier item's output the
-        // compiler reads it with a vector load)
-        const uint32_t lo = (uint32_t)uni((int)(uint32_t)word), hi = (uint32_t)uni((int)(uint32_t)(word >> 32));
-        const uint64_t front = count_mask(__builtin_popcountll((uint64_t)lo | ((uint64_t)hi << 32)));
-        m[0] = (uint32_t)front & keep;
-        m[1] = (uint32_t)(front >> 32) & keep;
     };
-    // accumulator i <-> key 8 (i / 4) + 4 lh + i % 4 of the step's 32 keys, query lr (+32)
-    auto mask_pair = [&](f32x16 (&sv)[2], uint32_t half) {
-        if (__builtin_expect(half != ~0u, 0)) {
+    // accumulator i of key block kk <-> key 16 kk + 4 lg + i of the step's 32 keys, query lr (+16, 32, 48)
+    auto mask_pair = [&](f32x4_ (&sv)[2][4], uint32_t entry) {
+        if (__builtin_expect(entry < 32u << kHalfCountShift, 0)) {
             asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");       // the MFMAs into these accumulators have retired
-            // the lane's part of the shift first: the tests below then use constants, not sixteen per-lane bit masks
+            // the lane's part of the shift first: the tests below then use constants, not eight per-lane bit masks
             // that would have to be kept in registers (or spilled) all through the loop for this rare path
-            uint32_t mine = half >> (4 * lh);
+            uint32_t mine = ((1u << (entry >> kHalfCountShift)) - 1u) >> (4 * lg);
             asm volatile("" : "+v"(mine));
 #pragma unroll
-            for (int i = 0; i < 16; ++i)
-                if (!((mine >> (8 * (i / 4) + (i % 4))) & 1u)) { sv[0][i] = -INFINITY; sv[1][i] = -INFINITY; }
-        }
-    };
-    // combine a lane's maximum with the other key group of the same query (lane ^ 32)
-    auto finish_max = [&](float mx) -> float {
-        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-        return fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    };
-    // mx0, mx1: this lane's unscaled maxima over its 16 accumulators of the step that comes next.  The test
-    // needs no exchange between the two key groups of a query: some lane exceeds the limit exactly when the
-    // combined maximum does.
-    auto raise_max = [&](float mx0, float mx1) __attribute__((always_inline)) {
-        if (__builtin_expect(__any(mx0 > raise_at[0] || mx1 > raise_at[1]), 0)) {
-            const float mx[2] = {finish_max(mx0) * qk_scale, finish_max(mx1) * qk_scale};
+            for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                const float m_new = fmaxf(m_i[qq], mx[qq]);
-                const float alpha = __builtin_amdgcn_exp2f(m_i[qq] - ((m_new == -INFINITY) ? 0.f : m_new));
-                m_i[qq] = m_new;
-                neg_m[qq] = (m_new == -INFINITY) ? 0.f : -m_new;
-                raise_at[qq] = (m_new + kTau) * inv_scale;
-                l_i[qq] *= alpha;
-                alpha_p[qq] = alpha;
-            }
-            rescale_pending = true;
+                for (int i = 0; i < 4; ++i)
+                    if (!((mine >> (16 * kk + i)) & 1u)) {
+#pragma unroll
+                        for (int qb = 0; qb < 4; ++qb) sv[kk][qb][i] = -INFINITY;
+                    }
         }
     };
-    // The output accumulators live in AGPRs, which the VALU cannot multiply in place.  Written out register by
-    // register through one temporary, so that this rare path does not make the compiler reserve VGPRs for a copy
-    // of the accumulators.
+    // mx: this lane's unscaled maxima over its 8 accumulators per query of the step that comes next.  The test
+    // needs no exchange between the four key groups of a query: some lane exceeds the limit exactly when the
+    // combined maximum does.
+    auto raise_max = [&](const float (&mx)[4]) __attribute__((always_inline)) {
+        if (!__any(mx[0] > raise_at[0] || mx[1] > raise_at[1] || mx[2] > raise_at[2] || mx[3] > raise_at[3])) return;
+#pragma unroll
+        for (int qb = 0; qb < 4; ++qb) {
+            const float m_new = fmaxf(m_i[qb], over_lanes(mx[qb], [](float a, float b) { return fmaxf(a, b); }) * qk_scale);
+            const float alpha = __builtin_amdgcn_exp2f(m_i[qb] - ((m_new == -INFINITY) ? 0.f : m_new));
+            m_i[qb] = m_new;
+            neg_m[qb] = (m_new == -INFINITY) ? 0.f : -m_new;
+            raise_at[qb] = (m_new + kTau) * inv_scale;
+            l_i[qb] *= alpha;
+            alpha_p[qb] = alpha;
+        }
+        raise_low = fminf(fminf(raise_at[0], raise_at[1]), fminf(raise_at[2], raise_at[3]));
+        rescale_pending = true;
+    };
+    auto lane_max = [&](const f32x4_ (&sv)[2][4], float (&mx)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int qb = 0; qb < 4; ++qb) {
+            mx[qb] = fmaxf(sv[0][qb][0], sv[0][qb][1]);
+            mx[qb] = fmaxf(fmaxf(mx[qb], sv[0][qb][2]), sv[0][qb][3]);
+            mx[qb] = fmaxf(fmaxf(mx[qb], sv[1][qb][0]), sv[1][qb][1]);
+            mx[qb] = fmaxf(fmaxf(mx[qb], sv[1][qb][2]), sv[1][qb][3]);
+        }
+    };
+    // The output accumulators live in AGPRs, which the VALU cannot multiply in place.  Each goes through LDS and back into the
+    // registers it came from, so that this rare path does not make the compiler reserve registers for copies of
+    // them (element by element through moves it did, 220 to 340 of them, in scratch memory).
     auto rescale_out = [&]() __attribute__((always_inline)) {
         asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMA into the accumulators has retired
-        static_for<128>([&](auto n_c) {
-            constexpr int n = decltype(n_c)::value, qq = n >> 6, t = (n >> 4) & 3, i = n & 15;
-            float x = oacc[t][qq][i], tmp;
-            asm volatile("v_accvgpr_read_b32 %1, %0\n\tv_mul_f32 %1, %1, %2\n\ts_nop 1\n\tv_accvgpr_write_b32 %0, %1"
-                         : "+a"(x), "=&v"(tmp) : "v"(alpha_p[qq]));
-            oacc[t][qq][i] = x;
+        const uint32_t at = lds_address(scale_room) + threadIdx.x * 16u;
+        static_for<32>([&](auto n_c) {
+            constexpr int n = decltype(n_c)::value, qb = n & 3, t = n >> 2;
+            f32x4_ y;
+            asm volatile("ds_write_b128 %1, %2\n\ts_waitcnt lgkmcnt(0)\n\tds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(y) : "v"(at), "a"(oacc[t][qb]) : "memory");
+            y *= alpha_p[qb];
+            asm volatile("ds_write_b128 %1, %2\n\ts_waitcnt lgkmcnt(0)\n\tds_read_b128 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "+a"(oacc[t][qb]) : "v"(at), "v"(y) : "memory");
         });
         asm volatile("s_nop 7" ::: "memory");                        // AGPR writes before the next MFMA reads them
         rescale_pending = false;
     };
 
-    // Step u = 2 g + j (j static).  On entry S(u) is complete and the running maximum covers it; P_B(u-1) is
-    // complete.  The 32 MFMAs of a step, in issue order ("slots"):
-    //    0 ..  7   O^T += V_B(u-1)^T P_B(u-1)^T      the last 16 keys of the previous step
-    //    8 .. 23   S(u+1)^T = K(u+1) Q^T
-    //   24 .. 31   O^T += V_A(u)^T P_A(u)^T          the first 16 keys of this step
+    // Step u = 2 g + j (j static).  On entry S(u) is complete and the running maximum covers it; the P of queries 32 .. 63 of
+    // step u-1 are complete.  The 64 MFMAs of a step, in issue order (32 "slots" of two):
+    //    0 ..  7   O^T += V(u-1)^T P(u-1)^T      queries 32 .. 63 of the previous step, a tile of d a slot
+    //    8 .. 23   S(u+1)^T = K(u+1) Q^T         a fragment of K in two slots
+    //   24 .. 31   O^T += V(u)^T P(u)^T          queries 0 .. 31 of this step
     // The VALU work on S(u) - per pair of accumulators two fma, two exp2, two additions for the row sum and one
     // rounding of the pair to the storage type, 16 pairs - is cut into pieces that go between the MFMAs so that
-    // no gap holds more than an MFMA lasts: the first 14 pairs behind slots 0 .. 23 (the eight pairs of P_A
+    // no gap holds more than two MFMAs last: the first 14 pairs behind slots 0 .. 23 (the eight pairs of queries 0 .. 31
     // first: they are complete well before slot 24), the last two behind slots 24 .. 31 together with the row
     // maximum of S(u+1), which is complete by then.  Fragment registers are reloaded in bursts behind the last
-    // MFMA that reads them: V_B(u+1) behind slot 7, K(u+3) behind slot 23, V_A(u+2) behind slot 31, so that every
-    // fragment is requested two steps before it is used.  Within a burst the fragment that is used first is
+    // MFMA that reads them: V(u+1) behind slot 7, a step and a half before it is used, K(u+3) behind slot 23, two steps.
+    // Within a burst the fragment that is used first is
     // requested last: loads return in order, so the wait in front of its first use covers the whole burst and
     // the fragments behind it need none of their own.
-    auto step = [&](auto jj) __attribute__((always_inline)) {
+    // `between` puts scalar work of the walk behind the slots.
+    auto step = [&](auto jj, auto between) __attribute__((always_inline)) {
         constexpr int j = decltype(jj)::value;
         constexpr int sc = j & 1, sn = sc ^ 1;                 // S(u) and S(u+1) alternate between two register sets
         constexpr int kslot = (j + 1) & 1;                     // ring slot of K(u+1), then of K(u+3)
-        constexpr int vprev = (j + 1) & 1, vcur = j & 1;       // ring slots of V(u-1) / V(u+1) and of V(u) / V(u+2)
-        // pair n: query half n & 1, accumulators 2 (n >> 1), + 1.  Its arithmetic comes in three pieces of about the
-        // same cost - exponential of the first accumulator (h0), of the second (h1), and the use of both: row sum
-        // and rounding (t) - in the order h0(0) h1(0) h0(1) t(0) h1(1) h0(2) t(1) h1(2) ...: the result of a
-        // transcendental instruction cannot be consumed by the next instruction without a wait state.
-        float pa[2][2];
-        auto piece = [&](int p) {                               // p = 0 .. 47
-            // p = 0: h0(0); p = 1: h1(0); p = 2 + 3 k: h0(k + 1); p = 3 + 3 k: t(k); p = 4 + 3 k: h1(k + 1); p = 47: t(15)
-            const int k = p < 2 ? 0 : (p - 2) / 3, r = p < 2 ? 0 : (p - 2) % 3;
-            const bool is_t = p == 47 || (p >= 2 && r == 1);
-            const int n = p < 2 ? 0 : p == 47 ? 15 : (r == 1 ? k : k + 1);
-            const int e = p < 2 ? p : (r == 0 ? 0 : 1);         // which accumulator of the pair (h0 / h1)
-            const int qq = n & 1, i = 2 * (n >> 1);
-            if (is_t) {
-                l_i[qq] += pa[n & 1][0] + pa[n & 1][1];
-                pb[qq][i >> 3][i & 7] = (T)pa[n & 1][0];
-                pb[qq][i >> 3][(i + 1) & 7] = (T)pa[n & 1][1];
-                asm volatile("" : "+v"(l_i[qq]), "+v"(pb[qq][i >> 3]));
-            } else {
-                pa[n & 1][e] = __builtin_amdgcn_exp2f(fmaf(s[sc][qq][i + e], qk_scale, neg_m[qq]));
-                asm volatile("" : "+v"(pa[n & 1][e]));
+        constexpr int vprev = (j + 1) & 1, vcur = j & 1;       // ring slots of V(u-1), then V(u+1), and of V(u)
+        // pair n: queries 16 qb .. with qb = 2 (n >> 3) + (n & 1), keys 2 ((n >> 1) & 3), + 1 of the lane's eight.  Its instructions go in
+        // six: an exponential, an argument of the next pair, the sum of the pair before; the other exponential, the other argument, and
+        // the pair before added to the row sum and rounded.  (The result of a transcendental instruction cannot be consumed by the
+        // next instruction without a wait state.)
+        float fx[2][2], pa[2][2], both;
+        auto argument = [&](int m, int e) {
+            const int qb = 2 * (m >> 3) + (m & 1), i = 2 * ((m >> 1) & 3);
+            fx[m & 1][e] = fmaf(s[sc][i >> 2][qb][(i & 3) + e], qk_scale, neg_m[qb]);
+            asm volatile("" : "+v"(fx[m & 1][e]));
+        };
+        auto piece = [&](int p) {                               // p = 0 .. 97
+            const int n = p / 6, r = p % 6, m = n - 1;
+            if ((r == 0 || r == 3) && n < 16) {
+                pa[n & 1][r == 3] = __builtin_amdgcn_exp2f(fx[n & 1][r == 3]);
+                asm volatile("" : "+v"(pa[n & 1][r == 3]));
+            } else if ((r == 1 || r == 4) && n < 15) {
+                argument(n + 1, r == 4);
+            } else if (((r == 2 && n < 16) || p == 96) && m >= 0) {
+                both = pa[m & 1][0] + pa[m & 1][1];
+                asm volatile("" : "+v"(both));
+            } else if (((r == 5 && n < 16) || p == 97) && m >= 0) {
+                const int qb = 2 * (m >> 3) + (m & 1), i = 2 * ((m >> 1) & 3);
+                l_i[qb] += both;
+                pb[qb][i] = (T)pa[m & 1][0];
+                pb[qb][i + 1] = (T)pa[m & 1][1];
+                asm volatile("" : "+v"(l_i[qb]), "+v"(pb[qb]));
             }
         };
-        float mx[2];
+        // Behind MFMA g of 64.  An instruction takes four clocks of issue and an exponential eight; an MFMA sixteen in its pipe.
+        // Without maxima a pair takes four gaps - of an exponential, two instructions, an exponential, three - and everything fits; with
+        // them 14 pairs stand in the first 48 gaps, which leaves the last 16 room for the maxima of S(u+1).
+        auto gap = [&](auto g_c) __attribute__((always_inline)) {
+            constexpr int g = decltype(g_c)::value;
+            if constexpr (g == 0) { argument(0, 0); argument(0, 1); }
+            if constexpr (kBounded) {
+                constexpr int p0 = 6 * (g >> 2), r = g & 3;
+                if constexpr (r == 0) piece(p0);
+                if constexpr (r == 1) { piece(p0 + 1); piece(p0 + 2); }
+                if constexpr (r == 2) piece(p0 + 3);
+                if constexpr (r == 3) { piece(p0 + 4); piece(p0 + 5); }
+            } else {
+                constexpr int from = first_piece(g), to = first_piece(g + 1);
+                static_for<to - from>([&](auto p_c) { piece(from + decltype(p_c)::value); });
+            }
+            if constexpr (g == 63) { piece(96); piece(97); }
+        };
+        float highest = 0.f;                                    // of this lane's 32 accumulators of S(u+1), value n: key n / 4, queries n % 4
+        auto next_s = [&](int n) { return s[sn][n >> 4][n & 3][(n >> 2) & 3]; };
         __builtin_amdgcn_sched_barrier(0);
         static_for<32>([&](auto slot_c) {
             constexpr int slot = decltype(slot_c)::value;
-            // ---- the MFMA of this slot
+            // ---- the MFMAs of this slot
+            if constexpr (slot == 0) asm volatile("s_nop 1");       // the last of pb[3] was written in front of this step
             if constexpr (slot < 8) {
-                constexpr int t = slot >> 1, qq = slot & 1;
-                oacc[t][qq] = mfma32(vb[vprev][4 + t], pb[qq][1], oacc[t][qq]);
+                mfma_acc16(oacc[slot][2], vb[vprev][slot], pb[2]);
+                __builtin_amdgcn_sched_barrier(0);
+                gap(std::integral_constant<int, 2 * slot>{});
+                __builtin_amdgcn_sched_barrier(0);
+                mfma_acc16(oacc[slot][3], vb[vprev][slot], pb[3]);
             } else if constexpr (slot < 24) {
-                constexpr int c = (slot - 8) >> 1, qq = slot & 1;
-                if constexpr (qq == 0) {
-                    if constexpr (c == 0) mfma_s<true, false>(s[sn][0], kb[kslot][0], qreg[0][0]);
-                    else mfma_s<false, false>(s[sn][0], kb[kslot][c], qreg[0][c]);
-                } else {
-                    if constexpr (c == 0) mfma_s<true, true>(s[sn][1], kb[kslot][0], qreg[1][0]);
-                    else mfma_s<false, true>(s[sn][1], kb[kslot][c], qreg[1][c]);
-                }
+                constexpr int f = (slot - 8) >> 1, c = f >> 1, kk = f & 1, qb = 2 * (slot & 1);      // d step, key block
+                mfma_s16<c == 0, true>(s[sn][kk][qb], kb[kslot][f], qreg[qb][c]);
+                __builtin_amdgcn_sched_barrier(0);
+                gap(std::integral_constant<int, 2 * slot>{});
+                __builtin_amdgcn_sched_barrier(0);
+                mfma_s16<c == 0, true>(s[sn][kk][qb + 1], kb[kslot][f], qreg[qb + 1][c]);
             } else {
-                constexpr int t = (slot - 24) >> 1, qq = slot & 1;
-                oacc[t][qq] = mfma32(vb[vcur][t], pb[qq][0], oacc[t][qq]);
+                constexpr int t = slot - 24;
+                mfma_acc16(oacc[t][0], vb[vcur][t], pb[0]);
+                __builtin_amdgcn_sched_barrier(0);
+                gap(std::integral_constant<int, 2 * slot>{});
+                __builtin_amdgcn_sched_barrier(0);
+                mfma_acc16(oacc[t][1], vb[vcur][t], pb[1]);
             }
             // ---- reloads, in bursts behind the last MFMA that reads the fragments (single loads between the
-            // arithmetic cost more issue time than they take): V_B(u+1), K(u+3), V_A(u+2)
-            if constexpr (slot == 7) {
-#pragma unroll
-                for (int tt = 1; tt <= 4; ++tt) vb[vprev][4 + (tt & 3)] = v_frag(w_half[j], 4 + (tt & 3));
-            }
-            if constexpr (slot == 23) {
-#pragma unroll
-                for (int cc = 1; cc <= 8; ++cc) kb[kslot][cc & 7] = k_frag(w_half[j + 2], cc & 7);
-            }
-            if constexpr (slot == 31) {
-#pragma unroll
-                for (int tt = 1; tt <= 4; ++tt) vb[vcur][tt & 3] = v_frag(w_half[j + 1], tt & 3);
-            }
+            // arithmetic cost more issue time than they take): V(u+1), K(u+3)
+            if constexpr (slot < 8) vb[vprev][slot] = v_frag(offset_of(w[j]), slot);
+            if constexpr (slot >= 8 && slot < 24 && slot % 2 == 1) kb[kslot][(slot - 9) / 2] = k_frag(offset_of(w[j + 2]), (slot - 9) / 2);
             if constexpr (slot == 7) {
                 if (__builtin_expect(rescale_pending, 0)) rescale_out();
             }
-            // ---- VALU pieces: 42 of the 48 (14 pairs) behind slots 0 .. 23, one or two per slot; the other 6 behind
-            // slots 24 .. 31 next to the row maximum of S(u+1).  S(u+1) is first read behind slot 25: its last MFMA
-            // (slot 23) has retired by the time the MFMA of slot 25 has been issued, which the compiler cannot
-            // check for the assembly MFMAs.
-            if constexpr (slot < 24) {
-                constexpr int lo = (slot * 42) / 24, hi = ((slot + 1) * 42) / 24;      // one or two pieces
-                piece(lo);
-                if constexpr (hi - lo > 1) piece(lo + 1);
-            } else {
+            gap(std::integral_constant<int, 2 * slot + 1>{});
+            if constexpr (slot >= 24) {
                 constexpr int r = slot - 24;                    // 0 .. 7
-                if constexpr (r == 0) { piece(42); piece(43); }
                 if constexpr (r == 1) {
-                    mfma_chain_end(s[sn][0]);
-                    mfma_chain_end(s[sn][1]);
-                    mask_pair(s[sn], w_mask[j]);               // the keys of step u + 1
-                    if constexpr (!kBounded) {
-                        mx[0] = fmaxf(fmaxf(s[sn][0][0], s[sn][0][1]), s[sn][0][2]);
-                        mx[1] = fmaxf(fmaxf(s[sn][1][0], s[sn][1][1]), s[sn][1][2]);
-                        mx[0] = fmaxf(fmaxf(mx[0], s[sn][0][3]), s[sn][0][15]);
-                        mx[1] = fmaxf(fmaxf(mx[1], s[sn][1][3]), s[sn][1][15]);
-                    }
+#pragma unroll
+                    for (int x = 0; x < 8; ++x) mfma_chain_end(s[sn][x >> 2][x & 3]);
+                    mask_pair(s[sn], w[j]);                    // the keys of step u + 1
+                    if constexpr (!kBounded) highest = fmaxf(fmaxf(next_s(0), next_s(1)), next_s(2));
                 }
-                if constexpr (!kBounded && r >= 2 && r < 7) {   // accumulators 4 .. 13, two per slot and query half
-                    mx[0] = fmaxf(fmaxf(mx[0], s[sn][0][2 * r]), s[sn][0][2 * r + 1]);
-                    mx[1] = fmaxf(fmaxf(mx[1], s[sn][1][2 * r]), s[sn][1][2 * r + 1]);
+                if constexpr (!kBounded && r >= 2) {            // the other 29, five or four a slot
+                    constexpr int from = 3 + (29 * (r - 2) + 5) / 6, to = 3 + (29 * (r - 1) + 5) / 6;
+#pragma unroll
+                    for (int n = from; n < (to < 32 ? to : 32); ++n) highest = fmaxf(highest, next_s(n));
                 }
-                if constexpr (!kBounded && r == 7) {
-                    mx[0] = fmaxf(mx[0], s[sn][0][14]);
-                    mx[1] = fmaxf(mx[1], s[sn][1][14]);
-                }
-                if constexpr (r == 2) piece(44);
-                if constexpr (r == 4) piece(45);
-                if constexpr (r == 6) piece(46);
-                if constexpr (r == 7) piece(47);
             }
+            between(slot_c);
             __builtin_amdgcn_sched_barrier(0);
         });
-        if constexpr (!kBounded) raise_max(mx[0], mx[1]);
+        // One test for all queries, of the highest value and the lowest limit, seldom met; then of each query's own.
+        if constexpr (!kBounded) {
+            if (__builtin_expect(__any(highest > raise_low), 0)) {
+                float mx[4];
+                lane_max(s[sn], mx);
+                raise_max(mx);
+            }
+        }
     };
 
     // ---- the workgroup's items
@@ -589,11 +622,11 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         const int batch = bh / L.by_heads;
         const int64_t o_bh = (int64_t)batch * L.o_st[0] + (int64_t)(bh - batch * Hn) * L.o_st[1];
         // the token rows of an item that nothing has prepared: asked for beside its descriptor
-        int32_t first_rows[3] = {0, 0, 0};
+        int32_t first_rows[5] = {0, 0, 0, 0, 0};
         if (!prepared && L.q_rows != nullptr) {
-            first_rows[0] = L.q_rows[qrow0 + lr];
-            first_rows[1] = L.q_rows[qrow0 + 32 + lr];
-            first_rows[2] = L.q_rows[qrow0 + lane];
+#pragma unroll
+            for (int qb = 0; qb < 4; ++qb) first_rows[qb] = L.q_rows[qrow0 + 16 * qb + lr];
+            first_rows[4] = L.q_rows[qrow0 + lane];
         }
         // ... and so is a team's list, as far as one entry a thread goes (what lies behind its end is not used)
         int32_t team_entry = 0;
@@ -612,12 +645,11 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         const int next_nent = list_length(nxt);
         // (an item in parts has no first pair that is known ahead)
         const bool prepare_next = !kOnce && (kBounded || parts.count == 1) && nxt.item >= 0 && npairs > 0 && next_nent > 0 && next_nent <= kPipeList * kWords && q_offsets_32 != 0;
+        beyond[0] = beyond[1] = 0;
         if (prepare_next) {
             first_pair(nxt, beyond);
-            beyond[0] = (uint32_t)uni((int)beyond[0]);
-            beyond[1] = (uint32_t)uni((int)beyond[1]);
-        } else {
-            beyond[0] = beyond[1] = half_base;
+#pragma unroll
+            for (int x = 0; x < 2; ++x) beyond[x] = (uint32_t)uni((int)(beyond[x] - half_base)) & kHalfId;
         }
         const int nitem = prepare_next ? nxt.item : 0, nbh = nitem / L.by_tiles;
         const int64_t nqrow0 = (int64_t)(nitem - nbh * nqt) * kTile;
@@ -626,17 +658,15 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         const bool early = (kTeam == 1 && !kGate) || (!kOnce && (kBounded || parts.count == 1));         // the walk starts at the list's first entry
         auto first_fragments = [&](uint32_t h0, uint32_t h1) {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(h0, c);                       // K(0)
+            for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(h0 << 13, c);                 // K(0)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) kb[1][c] = k_frag(h1, c);                       // K(1)
+            for (int c = 0; c < 8; ++c) kb[1][c] = k_frag(h1 << 13, c);                 // K(1)
 #pragma unroll
-            for (int f = 0; f < 8; ++f) vb[0][f] = v_frag(h0, f);                       // V_A(0), V_B(0)
-#pragma unroll
-            for (int f = 0; f < 4; ++f) vb[1][f] = v_frag(h1, f);                       // V_A(1)
+            for (int f = 0; f < 8; ++f) vb[0][f] = v_frag(h0 << 13, f);                 // V(0)
         };
         if (!prepared) {
             // Nothing of this item is on its way yet.  Everything that its first product waits for is asked for before any of
-            // it is waited for: the list, Q as the B operand of S^T (lane holds rows lr and 32 + lr, d = 16 c + 8 lh .. +8) and,
+            // it is waited for: the list, Q as the B operand of S^T (lane holds rows lr, 16 + lr, ..., d = 32 c + 8 lg .. +8) and,
             // where the walk starts at the list's first entry, which the descriptor holds, the first K and V fragments.
             int lane_now = lane;                                     // see the epilogue
             asm volatile("" : "+v"(lane_now));
@@ -648,13 +678,13 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 for (int e = 0; e < kAhead; ++e) entry[e] = list[min(lane_now + 64 * e, nent - 1)];
             }
             const int64_t q_bh = (int64_t)batch * L.q_st[0] + (int64_t)(bh - batch * Hn) * L.q_st[1];
-            V8 rows[2][8];
+            V8 rows[4][4];
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                const int64_t row = L.q_rows != nullptr ? (int64_t)max(first_rows[qq], 0) : qrow0 + 32 * qq + lr;      // padded slots read token 0, never stored
-                const T* qp = q + q_bh + row * L.q_st[2] + 8 * lh;
+            for (int qb = 0; qb < 4; ++qb) {
+                const int64_t row = L.q_rows != nullptr ? (int64_t)max(first_rows[qb], 0) : qrow0 + 16 * qb + lr;      // padded slots read token 0, never stored
+                const T* qp = q + q_bh + row * L.q_st[2] + 8 * lg;
 #pragma unroll
-                for (int c = 0; c < 8; ++c) rows[qq][c] = *reinterpret_cast<const V8*>(qp + 16 * c);
+                for (int c = 0; c < 4; ++c) rows[qb][c] = *reinterpret_cast<const V8*>(qp + 32 * c);
             }
             __builtin_amdgcn_sched_barrier(0);
             if (early && npairs > 0) {
@@ -663,7 +693,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 first_fragments((uint32_t)uni((int)h[0]), (uint32_t)uni((int)h[1]));
             }
             __builtin_amdgcn_sched_barrier(0);
-            if (L.q_rows != nullptr && wave == 0) out_rows[list_buf][lane_now] = first_rows[2];
+            if (L.q_rows != nullptr && wave == 0) out_rows[list_buf][lane_now] = first_rows[4];
             if constexpr (!kOnce) {
 #pragma unroll
                 for (int e = 0; e < kAhead; ++e)
@@ -680,6 +710,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 const int64_t brow = cur.item / L.by_block;
                 if (kWalk == kHalves)
                     for (int i = threadIdx.x; i < G.nbk * nsub_of_block; i += 64 * kTeam) counts[i] = (uint8_t)__popcll(tile_valid[i]);
+                const int lr = lane & 31, lh = lane >> 5;
                 const T* const qm = reinterpret_cast<const T*>(G.qc) + brow * kD + lh * 8;      // its mean as every row of the product
                 const T* const km = reinterpret_cast<const T*>(G.kc) + (int64_t)bh * G.nbk * kD + lh * 8;
                 V8 qa[8];
@@ -763,8 +794,8 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 if ((int)threadIdx.x < nent) big[threadIdx.x] = (uint32_t)team_entry;
                 for (int e = threadIdx.x + 64 * kTeam; e < nent; e += 64 * kTeam) big[e] = (uint32_t)list[e];
             }
-            take_q(0, rows[0]);
-            take_q(1, rows[1]);
+#pragma unroll
+            for (int qb = 0; qb < 4; ++qb) take_q(qb, rows[qb]);
             if constexpr (!kGate) {
                 ents = big;
                 __syncthreads();
@@ -803,86 +834,89 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         } else {
             ents = lists[list_buf];
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                V8 rows[8];
+            for (int qb = 0; qb < 4; ++qb) {
+                V8 rows[4];
 #pragma unroll
-                for (int c = 0; c < 8; ++c) rows[c] = *reinterpret_cast<const V8*>(qstage + (qq * 8 + c) * 1024 + lane_off);
-                take_q(qq, rows);
+                for (int c = 0; c < 4; ++c) rows[c] = *reinterpret_cast<const V8*>(qstage + (qb * 4 + c) * 1024 + lane_off);
+                take_q(qb, rows);
             }
         }
-        m_i[0] = m_i[1] = -INFINITY;
-        l_i[0] = l_i[1] = 0.f;
 #pragma unroll
-        for (int t = 0; t < 4; ++t)
+        for (int qb = 0; qb < 4; ++qb) {
+            m_i[qb] = -INFINITY;
+            l_i[qb] = 0.f;
+        }
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq)
+        for (int t = 0; t < 8; ++t)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) oacc[t][qq][i] = 0.f;
+            for (int qb = 0; qb < 4; ++qb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) oacc[t][qb][i] = 0.f;
 
         bool run = true;                     // this kernel computes the item (see the bound on q . k below)
         if (npairs > 0) {
-            uint32_t half0, mask0;           // position 0 of the walk
+            uint32_t first;                  // position 0 of the walk
             {
                 // the three entries, then the three words, each kind in one sweep: one wait per kind instead of three
                 Raw raw3[3];
-                uint32_t h[3][2], m[3][2];
+                uint32_t h[3] = {0, 0, 0}, e[3][2];
                 uint64_t word3[3];
 #pragma unroll
                 for (int r = 0; r < 3; ++r) raw3[r] = pair_raw(r);
+                if (kWalk != kHalves) {
 #pragma unroll
-                for (int r = 0; r < 3; ++r) pair_halves(r, raw3[r], h[r]);
+                    for (int r = 0; r < 3; ++r) h[r] = tile_half(r, raw3[r]);
+                }
 #pragma unroll
-                for (int r = 0; r < 3; ++r) word3[r] = pair_word(r, h[r]);
+                for (int r = 0; r < 3; ++r) word3[r] = pair_word(h[r]);
 #pragma unroll
-                for (int r = 0; r < 3; ++r) pair_masks(r, raw3[r], word3[r], m[r]);
-                half0 = h[0][0]; mask0 = m[0][0];
-                w_half[0] = h[0][1]; w_half[1] = h[1][0]; w_half[2] = h[1][1]; w_half[3] = h[2][0]; w_half[4] = h[2][1];
-                w_mask[0] = m[0][1]; w_mask[1] = m[1][0]; w_mask[2] = m[1][1]; w_mask[3] = m[2][0]; w_mask[4] = m[2][1];
+                for (int r = 0; r < 3; ++r) pair_entries(r, raw3[r], h[r], word3[r], e[r]);
+                first = e[0][0];
+                w[0] = e[0][1]; w[1] = e[1][0]; w[2] = e[1][1]; w[3] = e[2][0]; w[4] = e[2][1];
             }
-            // ---- prologue.  In flight when the loop starts: K(1), K(2), V_A(0), V_B(0), V_A(1); the ring slot of
-            // V_B(1) holds zeros, which the first step multiplies with P = 0 (there is no step -1).  A prepared item
+            // ---- prologue.  In flight when the loop starts: K(1), K(2), V(0); the ring slot of
+            // V(1) holds zeros, which the first step multiplies with P = 0 (there is no step -1).  A prepared item
             // finds all of them but K(2) requested already (K(0) sits where K(2) belongs until S(0) has been issued).
-            if (!prepared && !early) first_fragments(half0, w_half[0]);
+            if (!prepared && !early) first_fragments(half_base + (first & kHalfId), half_base + (w[0] & kHalfId));
 #pragma unroll
-            for (int f = 4; f < 8; ++f)
+            for (int f = 0; f < 8; ++f)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) vb[1][f][e] = (T)0.f;
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq)
+            for (int qb = 0; qb < 4; ++qb) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) pb[qq][1][e] = (T)0.f;
-            neg_m[0] = neg_m[1] = 0.f;
-            raise_at[0] = raise_at[1] = -INFINITY;
-            alpha_p[0] = alpha_p[1] = 1.f;
+                for (int e = 0; e < 8; ++e) pb[qb][e] = (T)0.f;
+                neg_m[qb] = 0.f;
+                raise_at[qb] = -INFINITY;
+                alpha_p[qb] = 1.f;
+            }
+            raise_low = -INFINITY;
             // the token rows of the next item's queries are looked up now; its list and its Q rows are asked for once
             // it is known that this item runs here
-            int32_t next_rows[2] = {0, 0};
+            int32_t next_rows[4] = {0, 0, 0, 0};
             if (prepare_next) {
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq) {
-                    const int64_t row = nqrow0 + 32 * qq + lr;
-                    next_rows[qq] = L.q_rows != nullptr ? L.q_rows[row] : (int32_t)row;      // used (and clamped) behind S(0): no wait here
+                for (int qb = 0; qb < 4; ++qb) {
+                    const int64_t row = nqrow0 + 16 * qb + lr;
+                    next_rows[qb] = L.q_rows != nullptr ? L.q_rows[row] : (int32_t)row;      // used (and clamped) behind S(0): no wait here
                 }
             }
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                if (c == 0) { mfma_s<true, false>(s[0][0], kb[0][0], qreg[0][0]); mfma_s<true, true>(s[0][1], kb[0][0], qreg[1][0]); }
-                else { mfma_s<false, false>(s[0][0], kb[0][c], qreg[0][c]); mfma_s<false, true>(s[0][1], kb[0][c], qreg[1][c]); }
-            }
+            for (int f = 0; f < 8; ++f)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(w_half[1], c);                    // K(2), behind the last reader of K(0)
+                for (int qb = 0; qb < 4; ++qb) {
+                    if (f < 2) mfma_s16<true, true>(s[0][f & 1][qb], kb[0][f], qreg[qb][f >> 1]);
+                    else mfma_s16<false, true>(s[0][f & 1][qb], kb[0][f], qreg[qb][f >> 1]);
+                }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(offset_of(w[1]), c);              // K(2), behind the last reader of K(0)
             asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");           // MFMA results before the VALU reads them
-            mfma_chain_end(s[0][0]);
-            mfma_chain_end(s[0][1]);
-            mask_pair(s[0], mask0);
-            float mx[2];
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                mx[qq] = fmaxf(s[0][qq][0], s[0][qq][1]);
-#pragma unroll
-                for (int i = 2; i < 16; i += 2) mx[qq] = fmaxf(fmaxf(mx[qq], s[0][qq][i]), s[0][qq][i + 1]);
-            }
-            raise_max(mx[0], mx[1]);
+            for (int x = 0; x < 8; ++x) mfma_chain_end(s[0][x >> 2][x & 3]);
+            mask_pair(s[0], first);
+            float mx[4];
+            lane_max(s[0], mx);
+            raise_max(mx);
             rescale_pending = false;                                     // nothing accumulated yet
 
             // Cauchy-Schwarz: no logit of this item exceeds |q| times the largest key norm of the head.  If that bound
@@ -894,19 +928,19 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
             // after it starts from scratch.
             if constexpr (kBounded) {
                 const float kn = __uint_as_float((uint32_t)uni((int)__float_as_uint(cur.kn)));
-                bool fits[2];
+                bool fit = true;
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq) {
-                    const float bound = __builtin_sqrtf(q_sq[qq] + __shfl_xor(q_sq[qq], 32)) * 1.001f * kn * qk_scale;   // both halves of the row's d
-                    const float lowest = m_i[qq] == -INFINITY ? -bound : m_i[qq];       // the row's largest logit is no smaller
+                for (int qb = 0; qb < 4; ++qb) {
+                    const float bound = __builtin_sqrtf(over_lanes(q_sq[qb], add)) * 1.001f * kn * qk_scale;      // all of the row's d
+                    const float lowest = m_i[qb] == -INFINITY ? -bound : m_i[qb];       // the row's largest logit is no smaller
                     const float ref = bound - kTau;
-                    fits[qq] = ref <= lowest + kSlack;                                  // false for a NaN
-                    if (ref > m_i[qq]) {
-                        m_i[qq] = ref;
-                        neg_m[qq] = -ref;
+                    fit = fit && ref <= lowest + kSlack;                                // false for a NaN
+                    if (ref > m_i[qb]) {
+                        m_i[qb] = ref;
+                        neg_m[qb] = -ref;
                     }
                 }
-                run = __all(fits[0] && fits[1]);
+                run = __all(fit);
                 if (!run && lane == 0) fallback[atomicAdd(fallback_count, 1u)] = cur.item;
             }
             if (run) {
@@ -914,7 +948,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 // What the next item needs and what takes long to arrive is asked for now.  Its list goes from global
                 // memory straight into the list buffer that is not in use (LDS DMA, 64 entries per instruction; the
                 // lanes behind the end of the list repeat its last entry); its Q rows go into the staging tile,
-                // fragment (qq, c) as 1 KB in lane order.  These loads are invisible to the compiler's count of
+                // fragment (qb, c) as 1 KB in lane order.  These loads are invisible to the compiler's count of
                 // outstanding loads, which can only make its waits for the fragment loads stricter than they need
                 // be while the DMA is under way.
 #pragma unroll
@@ -928,36 +962,38 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 const int64_t nq_bh = (int64_t)nbatch * L.q_st[0] + (int64_t)(nbh - nbatch * Hn) * L.q_st[1];
                 const char* qsrc = reinterpret_cast<const char*>(q + nq_bh);
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq) {
-                    const uint32_t voff = (uint32_t)max(next_rows[qq], 0) * (uint32_t)(L.q_st[2] * 2) + (uint32_t)(16 * lh);   // padded slots read token 0
+                for (int qb = 0; qb < 4; ++qb) {
+                    const uint32_t voff = (uint32_t)max(next_rows[qb], 0) * (uint32_t)(L.q_st[2] * 2) + (uint32_t)(16 * lg);   // padded slots read token 0
 #pragma unroll
-                    for (int c = 0; c < 8; ++c) load_to_lds_16(qsrc + 32 * c, voff, lds_address(qstage + (qq * 8 + c) * 1024));
+                    for (int c = 0; c < 4; ++c) load_to_lds_16(qsrc + 64 * c, voff, lds_address(qstage + (qb * 4 + c) * 1024));
                 }
             }
-            // The entry that comes into the window is decoded one iteration before it enters (its validity word may
-            // be a load) and read from LDS one iteration before that.
-            uint32_t p_half[2], p_mask[2];
-            {
-                const Raw raw3 = pair_raw(3);
-                pair_halves(3, raw3, p_half);
-                pair_masks(3, raw3, pair_word(3, p_half), p_mask);
-            }
+            // The entries that come into the window are made one iteration before they enter (a validity word may
+            // be a load) and read from LDS one iteration before that.  All of it goes between the last MFMAs of an iteration: in a
+            // row behind them, with masks worked out for every half, it was 55 instructions, and the matrix pipe had nothing
+            // to do for 220 clocks of 2 048.
+            uint32_t in[2];
+            auto make = [&](int tp, const Raw& raw, uint32_t (&e)[2]) {
+                const uint32_t h = kWalk == kHalves ? 0u : tile_half(tp, raw);
+                pair_entries(tp, raw, h, pair_word(h), e);
+            };
+            make(3, pair_raw(3), in);
             Raw raw = pair_raw(4);
             for (int g = 0; g < npairs; ++g) {
-                step(std::integral_constant<int, 0>{});
-                step(std::integral_constant<int, 1>{});
-                w_half[0] = w_half[2]; w_mask[0] = w_mask[2];
-                w_half[1] = w_half[3]; w_mask[1] = w_mask[3];
-                w_half[2] = w_half[4]; w_mask[2] = w_mask[4];
+                step(std::integral_constant<int, 0>{}, [](auto) {});
+                step(std::integral_constant<int, 1>{}, [&](auto slot_c) __attribute__((always_inline)) {
+                    constexpr int slot = decltype(slot_c)::value;
+                    if constexpr (slot == 26) w[0] = w[2];
+                    if constexpr (slot == 27) { w[1] = w[3]; w[2] = w[4]; }
+                    if constexpr (slot == 28) { w[3] = in[0]; w[4] = in[1]; }
+                    if constexpr (slot == 29) make(g + 4, raw, in);
+                    if constexpr (slot == 30) raw = pair_raw(g + 5);
+                    if constexpr (slot >= 26) {
 #pragma unroll
-                for (int x = 0; x < 2; ++x) { w_half[3 + x] = p_half[x]; w_mask[3 + x] = p_mask[x]; }
-#pragma unroll
-                for (int x = 0; x < 5; ++x) asm volatile("" : "+s"(w_half[x]), "+s"(w_mask[x]));
-                pair_halves(g + 4, raw, p_half);
-                pair_masks(g + 4, raw, pair_word(g + 4, p_half), p_mask);
-                __builtin_amdgcn_sched_barrier(0);
-                raw = pair_raw(g + 5);
-                __builtin_amdgcn_sched_barrier(0);
+                        for (int x = 0; x < 5; ++x) asm volatile("" : "+s"(w[x]));
+                        if constexpr (slot >= 29) asm volatile("" : "+s"(in[0]), "+s"(in[1]));
+                    }
+                });
             }
             if (kTeam <= 1) __syncthreads();          // the list in LDS has been read: the memory may become the staging tile (a team: below)
             if (prepare_next) {
@@ -968,11 +1004,17 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 // the next item starts and the output accumulators are free.
                 asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
             }
-            // the last 16 keys of the last step (V_B of an odd step sits in ring slot 1)
+            // queries 32 .. 63 of the last step (V of an odd step sits in ring slot 1)
+            asm volatile("s_nop 1");
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 8; ++t)
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq) oacc[t][qq] = mfma32(vb[1][4 + t], pb[qq][1], oacc[t][qq]);
+                for (int qb = 2; qb < 4; ++qb) mfma_acc16(oacc[t][qb], vb[1][t], pb[qb]);
+            asm volatile("s_nop 15" ::: "memory");           // the last of them has retired before the VALU reads it
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+#pragma unroll
+                for (int qb = 0; qb < 4; ++qb) mfma_acc_end(oacc[t][qb]);
             if (rescale_pending) rescale_out();
             }   // run
         }   // npairs > 0
@@ -982,96 +1024,86 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
             // 128 KB through LDS for a team of four, a microsecond; the rows leave from all wavefronts.
             float* const sums = reinterpret_cast<float*>(ost_bytes);
             float* const stats = sums + kTeam * kTile * kD;
-            float inv[2], M[2], l_all[2];
+            float inv[4], M[4], l_all[4];
             __syncthreads();                          // the list has been read
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                const float l = l_i[qq] + __shfl_xor(l_i[qq], 32);
-                if (lh == 0) {
-                    stats[(2 * wave) * kTile + 32 * qq + lr] = m_i[qq];
-                    stats[(2 * wave + 1) * kTile + 32 * qq + lr] = l;
+            for (int qb = 0; qb < 4; ++qb) {
+                const float l = over_lanes(l_i[qb], add);
+                if (lg == 0) {
+                    stats[(2 * wave) * kTile + 16 * qb + lr] = m_i[qb];
+                    stats[(2 * wave + 1) * kTile + 16 * qb + lr] = l;
                 }
             }
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 8; ++t)
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq)
-#pragma unroll
-                    for (int gq = 0; gq < 4; ++gq)
-                        *reinterpret_cast<float4*>(sums + wave * (kTile * kD) + (((t * 2 + qq) * 4 + gq) * 64 + lane) * 4) =
-                            make_float4(oacc[t][qq][4 * gq], oacc[t][qq][4 * gq + 1], oacc[t][qq][4 * gq + 2], oacc[t][qq][4 * gq + 3]);
+                for (int qb = 0; qb < 4; ++qb) *reinterpret_cast<f32x4_*>(sums + wave * (kTile * kD) + ((t * 4 + qb) * 64 + lane) * 4) = oacc[t][qb];
             __syncthreads();
-            float factor[2][kTeam];
+            float factor[4][kTeam];
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
+            for (int qb = 0; qb < 4; ++qb) {
                 float m[kTeam];
 #pragma unroll
-                for (int w = 0; w < kTeam; ++w) m[w] = stats[(2 * w) * kTile + 32 * qq + lr];
-                M[qq] = m[0];
+                for (int w = 0; w < kTeam; ++w) m[w] = stats[(2 * w) * kTile + 16 * qb + lr];
+                M[qb] = m[0];
 #pragma unroll
-                for (int w = 1; w < kTeam; ++w) M[qq] = fmaxf(M[qq], m[w]);
-                l_all[qq] = 0.f;
+                for (int w = 1; w < kTeam; ++w) M[qb] = fmaxf(M[qb], m[w]);
+                l_all[qb] = 0.f;
 #pragma unroll
                 for (int w = 0; w < kTeam; ++w) {
-                    factor[qq][w] = m[w] > -INFINITY ? __builtin_amdgcn_exp2f(m[w] - M[qq]) : 0.f;      // a share without keys: no maximum, sums 0
-                    l_all[qq] += stats[(2 * w + 1) * kTile + 32 * qq + lr] * factor[qq][w];
+                    factor[qb][w] = m[w] > -INFINITY ? __builtin_amdgcn_exp2f(m[w] - M[qb]) : 0.f;      // a share without keys: no maximum, sums 0
+                    l_all[qb] += stats[(2 * w + 1) * kTile + 16 * qb + lr] * factor[qb][w];
                 }
-                inv[qq] = l_all[qq] > 0.f ? 1.0f / l_all[qq] : 0.f;
+                inv[qb] = l_all[qb] > 0.f ? 1.0f / l_all[qb] : 0.f;
             }
-            constexpr int kOwn = 4 / kTeam;           // tiles of d that a wavefront puts together
-            float4 own[kOwn][2][4];
+            constexpr int kOwn = 8 / kTeam;           // tiles of d that a wavefront puts together
+            float4 own[kOwn][4];
 #pragma unroll
             for (int t = 0; t < kOwn; ++t)
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq)
+                for (int qb = 0; qb < 4; ++qb) {
+                    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
-                    for (int gq = 0; gq < 4; ++gq) {
-                        float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-                        for (int w = 0; w < kTeam; ++w) {
-                            const float4 x = *reinterpret_cast<const float4*>(sums + w * (kTile * kD) + ((((wave * kOwn + t) * 2 + qq) * 4 + gq) * 64 + lane) * 4);
-                            const float fw = factor[qq][w];
-                            sum.x = fmaf(x.x, fw, sum.x); sum.y = fmaf(x.y, fw, sum.y); sum.z = fmaf(x.z, fw, sum.z); sum.w = fmaf(x.w, fw, sum.w);
-                        }
-                        own[t][qq][gq] = sum;
+                    for (int w = 0; w < kTeam; ++w) {
+                        const float4 x = *reinterpret_cast<const float4*>(sums + w * (kTile * kD) + (((wave * kOwn + t) * 4 + qb) * 64 + lane) * 4);
+                        const float fw = factor[qb][w];
+                        sum.x = fmaf(x.x, fw, sum.x); sum.y = fmaf(x.y, fw, sum.y); sum.z = fmaf(x.z, fw, sum.z); sum.w = fmaf(x.w, fw, sum.w);
                     }
+                    own[t][qb] = sum;
+                }
             if (parts.count > 1) {
                 float* const out = parts.buf + (int64_t)cur.local * kPartFloats;
 #pragma unroll
                 for (int t = 0; t < kOwn; ++t)
 #pragma unroll
-                    for (int qq = 0; qq < 2; ++qq)
+                    for (int qb = 0; qb < 4; ++qb)
+                        *reinterpret_cast<float4*>(out + (((wave * kOwn + t) * 4 + qb) * 64 + lane) * 4) = own[t][qb];
+                if (wave == 0 && lg == 0) {
 #pragma unroll
-                        for (int gq = 0; gq < 4; ++gq)
-                            *reinterpret_cast<float4*>(out + ((((wave * kOwn + t) * 2 + qq) * 4 + gq) * 64 + lane) * 4) = own[t][qq][gq];
-                if (wave == 0 && lh == 0) {
-#pragma unroll
-                    for (int qq = 0; qq < 2; ++qq) {
-                        out[kTile * kD + 32 * qq + lr] = M[qq];
-                        out[kTile * kD + kTile + 32 * qq + lr] = l_all[qq];
+                    for (int qb = 0; qb < 4; ++qb) {
+                        out[kTile * kD + 16 * qb + lr] = M[qb];
+                        out[kTile * kD + kTile + 16 * qb + lr] = l_all[qb];
                     }
                 }
                 return;
             }
-            if (lse != nullptr && wave == 0 && lh == 0) {
+            if (lse != nullptr && wave == 0 && lg == 0) {
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq) {
-                    int64_t row = qrow0 + 32 * qq + lr;
-                    if (L.q_rows != nullptr) row = out_rows[list_buf][32 * qq + lr];
-                    if (row >= 0) lse[(int64_t)bh * lse_S + row] = l_all[qq] > 0.f ? (M[qq] + __builtin_log2f(l_all[qq])) * kLn2 : -INFINITY;
+                for (int qb = 0; qb < 4; ++qb) {
+                    int64_t row = qrow0 + 16 * qb + lr;
+                    if (L.q_rows != nullptr) row = out_rows[list_buf][16 * qb + lr];
+                    if (row >= 0) lse[(int64_t)bh * lse_S + row] = l_all[qb] > 0.f ? (M[qb] + __builtin_log2f(l_all[qb])) * kLn2 : -INFINITY;
                 }
             }
             __syncthreads();                          // the sums have been read: the memory becomes the staging tile
 #pragma unroll
-            for (int qq = 0; qq < 2; ++qq)
+            for (int qb = 0; qb < 4; ++qb)
 #pragma unroll
-                for (int t = 0; t < kOwn; ++t)
-#pragma unroll
-                    for (int gq = 0; gq < 4; ++gq) {
-                        const float4 x = own[t][qq][gq];
-                        T out4[4] = {(T)(x.x * inv[qq]), (T)(x.y * inv[qq]), (T)(x.z * inv[qq]), (T)(x.w * inv[qq])};
-                        *reinterpret_cast<uint2*>(ost + (32 * qq + lr) * kOutPitch + 32 * (wave * kOwn + t) + 8 * gq + 4 * lh) = *reinterpret_cast<uint2*>(out4);
-                    }
+                for (int t = 0; t < kOwn; ++t) {
+                    const float4 x = own[t][qb];
+                    T out4[4] = {(T)(x.x * inv[qb]), (T)(x.y * inv[qb]), (T)(x.z * inv[qb]), (T)(x.w * inv[qb])};
+                    *reinterpret_cast<uint2*>(ost + (16 * qb + lr) * kOutPitch + 16 * (wave * kOwn + t) + 4 * lg) = *reinterpret_cast<uint2*>(out4);
+                }
             __syncthreads();
             const int kc = threadIdx.x & 15, kr = threadIdx.x >> 4;
             constexpr int kRows = 4 * kTeam, kTurns = kTile / kRows;
@@ -1090,47 +1122,41 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
         if (!kOnce && !kBounded && parts.count > 1) {
             float* const out = parts.buf + (int64_t)cur.local * kPartFloats;
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 8; ++t)
 #pragma unroll
-                for (int qq = 0; qq < 2; ++qq)
+                for (int qb = 0; qb < 4; ++qb) *reinterpret_cast<f32x4_*>(out + ((t * 4 + qb) * 64 + lane) * 4) = oacc[t][qb];
 #pragma unroll
-                    for (int gq = 0; gq < 4; ++gq)
-                        *reinterpret_cast<float4*>(out + (((t * 2 + qq) * 4 + gq) * 64 + lane) * 4) =
-                            make_float4(oacc[t][qq][4 * gq], oacc[t][qq][4 * gq + 1], oacc[t][qq][4 * gq + 2], oacc[t][qq][4 * gq + 3]);
-#pragma unroll
-            for (int qq = 0; qq < 2; ++qq) {
-                const float l = l_i[qq] + __shfl_xor(l_i[qq], 32);
-                if (lh == 0) {
-                    out[kTile * kD + 32 * qq + lr] = m_i[qq];
-                    out[kTile * kD + kTile + 32 * qq + lr] = l;
+            for (int qb = 0; qb < 4; ++qb) {
+                const float l = over_lanes(l_i[qb], add);
+                if (lg == 0) {
+                    out[kTile * kD + 16 * qb + lr] = m_i[qb];
+                    out[kTile * kD + kTile + 16 * qb + lr] = l;
                 }
             }
         } else if (run) {
-        // ---- epilogue: combine the two key groups of every query, normalise, store through LDS ----
-        float inv[2];
+        // ---- epilogue: combine the four key groups of every query, normalise, store through LDS ----
+        float inv[4];
 #pragma unroll
-        for (int qq = 0; qq < 2; ++qq) {
-            const float l = l_i[qq] + __shfl_xor(l_i[qq], 32);
-            inv[qq] = l > 0.f ? 1.0f / l : 0.f;
-            if (lse != nullptr && lh == 0) {
-                int64_t row = qrow0 + 32 * qq + lr;
-                if (L.q_rows != nullptr) row = out_rows[list_buf][32 * qq + lr];
-                if (row >= 0) lse[(int64_t)bh * lse_S + row] = l > 0.f ? (m_i[qq] + __builtin_log2f(l)) * kLn2 : -INFINITY;
+        for (int qb = 0; qb < 4; ++qb) {
+            const float l = over_lanes(l_i[qb], add);
+            inv[qb] = l > 0.f ? 1.0f / l : 0.f;
+            if (lse != nullptr && lg == 0) {
+                int64_t row = qrow0 + 16 * qb + lr;
+                if (L.q_rows != nullptr) row = out_rows[list_buf][16 * qb + lr];
+                if (row >= 0) lse[(int64_t)bh * lse_S + row] = l > 0.f ? ((kBounded ? -neg_m[qb] : m_i[qb]) + __builtin_log2f(l)) * kLn2 : -INFINITY;
             }
         }
-        // accumulator i of d tile t <-> d = 32 t + 8 (i / 4) + 4 lh + i % 4, query 32 qq + lr
+        // accumulator i of d tile t <-> d = 16 t + 4 lg + i, query 16 qb + lr
 #pragma unroll
-        for (int qq = 0; qq < 2; ++qq) {
-            T* orow = ost + (32 * qq + lr) * kOutPitch;
+        for (int qb = 0; qb < 4; ++qb) {
+            T* orow = ost + (16 * qb + lr) * kOutPitch;
 #pragma unroll
-            for (int t = 0; t < 4; ++t)
+            for (int t = 0; t < 8; ++t) {
+                T out4[4];
 #pragma unroll
-                for (int gq = 0; gq < 4; ++gq) {
-                    T out4[4];
-#pragma unroll
-                    for (int jx = 0; jx < 4; ++jx) out4[jx] = (T)(oacc[t][qq][4 * gq + jx] * inv[qq]);
-                    *reinterpret_cast<uint2*>(orow + 32 * t + 8 * gq + 4 * lh) = *reinterpret_cast<uint2*>(out4);
-                }
+                for (int jx = 0; jx < 4; ++jx) out4[jx] = (T)(oacc[t][qb][jx] * inv[qb]);
+                *reinterpret_cast<uint2*>(orow + 16 * t + 4 * lg) = *reinterpret_cast<uint2*>(out4);
+            }
         }
         __syncthreads();                          // one wavefront: orders its LDS writes before the reads below
         {
@@ -1178,42 +1204,42 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
 template <typename T>
 __global__ __launch_bounds__(256) void merge_parts_kernel(Parts parts, T* __restrict__ o, float* __restrict__ lse, int item_begin,
                                                           int nqt, int Hn, int64_t lse_S, FragLayout L) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 31, lh = lane >> 5;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lg = lane >> 4;
     const int item = item_at(L, item_begin + blockIdx.x, nqt), bh = item / L.by_tiles;
     const int64_t qrow0 = (int64_t)(item - bh * nqt) * kTile;
     const float* first = parts.buf + (int64_t)blockIdx.x * kPartFloats;
     const int64_t stride = (int64_t)parts.items * kPartFloats;
-    float M[2] = {-INFINITY, -INFINITY}, inv[2] = {0.f, 0.f};
-    int64_t row[2];
+    float M[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}, inv[4];
+    int64_t row[4];
 #pragma unroll
-    for (int qq = 0; qq < 2; ++qq) {
-        const int slot = 32 * qq + lr;
-        row[qq] = L.q_rows != nullptr ? (int64_t)L.q_rows[qrow0 + slot] : qrow0 + slot;
-        for (int p = 0; p < parts.count; ++p) M[qq] = fmaxf(M[qq], first[p * stride + kTile * kD + slot]);
+    for (int qb = 0; qb < 4; ++qb) {
+        const int slot = 16 * qb + lr;
+        row[qb] = L.q_rows != nullptr ? (int64_t)L.q_rows[qrow0 + slot] : qrow0 + slot;
+        for (int p = 0; p < parts.count; ++p) M[qb] = fmaxf(M[qb], first[p * stride + kTile * kD + slot]);
         float l = 0.f;
         for (int p = 0; p < parts.count; ++p) {
             const float m = first[p * stride + kTile * kD + slot];
-            if (m > -INFINITY) l += first[p * stride + kTile * kD + kTile + slot] * __builtin_amdgcn_exp2f(m - M[qq]);
+            if (m > -INFINITY) l += first[p * stride + kTile * kD + kTile + slot] * __builtin_amdgcn_exp2f(m - M[qb]);
         }
-        inv[qq] = l > 0.f ? 1.0f / l : 0.f;
-        if (lse != nullptr && wave == 0 && lh == 0 && row[qq] >= 0)
-            lse[(int64_t)bh * lse_S + row[qq]] = l > 0.f ? (M[qq] + __builtin_log2f(l)) * kLn2 : -INFINITY;
+        inv[qb] = l > 0.f ? 1.0f / l : 0.f;
+        if (lse != nullptr && wave == 0 && lg == 0 && row[qb] >= 0)
+            lse[(int64_t)bh * lse_S + row[qb]] = l > 0.f ? (M[qb] + __builtin_log2f(l)) * kLn2 : -INFINITY;
     }
     T* const out = o + (int64_t)(bh / Hn) * L.o_st[0] + (int64_t)(bh % Hn) * L.o_st[1];
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
-        const int chunk = wave * 8 + c, t = chunk >> 3, qq = (chunk >> 2) & 1, gq = chunk & 3;      // qq is c >> 2
+        const int chunk = wave * 8 + c, t = chunk >> 2, qb = c & 3;
         float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
         for (int p = 0; p < parts.count; ++p) {
-            const float m = first[p * stride + kTile * kD + 32 * qq + lr];
-            const float f = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M[c >> 2]) : 0.f;
+            const float m = first[p * stride + kTile * kD + 16 * qb + lr];
+            const float f = m > -INFINITY ? __builtin_amdgcn_exp2f(m - M[qb]) : 0.f;
             const float4 x = *reinterpret_cast<const float4*>(first + p * stride + (chunk * 64 + lane) * 4);
             sum.x = fmaf(x.x, f, sum.x); sum.y = fmaf(x.y, f, sum.y); sum.z = fmaf(x.z, f, sum.z); sum.w = fmaf(x.w, f, sum.w);
         }
-        if (row[c >> 2] < 0) continue;
-        const float n = inv[c >> 2];
+        if (row[qb] < 0) continue;
+        const float n = inv[qb];
         T x4[4] = {(T)(sum.x * n), (T)(sum.y * n), (T)(sum.z * n), (T)(sum.w * n)};
-        *reinterpret_cast<uint2*>(out + row[c >> 2] * L.o_st[2] + 32 * t + 8 * gq + 4 * lh) = *reinterpret_cast<const uint2*>(x4);
+        *reinterpret_cast<uint2*>(out + row[qb] * L.o_st[2] + 16 * t + 4 * lg) = *reinterpret_cast<const uint2*>(x4);
     }
 }
 

@@ -25,6 +25,9 @@ __device__ inline f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
 __device__ inline f32x4_ mfma16(bf16x8 a, bf16x8 b, f32x4_ c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+__device__ inline f32x4_ mfma16(f16x8 a, f16x8 b, f32x4_ c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
 template <typename T> struct Vec8;
 template <> struct Vec8<__bf16> { typedef bf16x8 type; };
 template <> struct Vec8<_Float16> { typedef f16x8 type; };
@@ -124,6 +127,39 @@ __device__ inline void mfma_s(f32x16& acc, f16x8 a, f16x8 b) {
     }
 }
 
+// The same for 16x16x32 products.
+template <bool kFirst, bool kAgprB>
+__device__ inline void mfma_s16(f32x4_& acc, bf16x8 a, bf16x8 b) {
+    if (kFirst) {
+        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
+        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+    } else {
+        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
+        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+    }
+}
+template <bool kFirst, bool kAgprB>
+__device__ inline void mfma_s16(f32x4_& acc, f16x8 a, f16x8 b) {
+    if (kFirst) {
+        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
+        else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
+    } else {
+        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
+        else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+    }
+}
+
+// An accumulation into AGPRs, in place: with the builtin, whose result may lie elsewhere than what it adds to, the compiler put 32
+// accumulators of four registers into other registers from step to step, a move for every register.  A and B in VGPRs, which a
+// VALU instruction must have written at least two wait states before.
+__device__ inline void mfma_acc16(f32x4_& acc, bf16x8 a, bf16x8 b) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+__device__ inline void mfma_acc16(f32x4_& acc, f16x8 a, f16x8 b) {
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma_acc_end(f32x4_& acc) { asm volatile("" : "+a"(acc)); }
+
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N - 1>): a loop whose index is a constant expression
 // in every copy of the body (register arrays must never be indexed by a run-time value).
 template <typename F, int... I>
@@ -139,6 +175,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 // reused.  Emits nothing; it only keeps `acc` allocated, and unchanged, between the chain's last MFMA and this
 // point, which the caller places at least eight MFMAs (or the equivalent s_nop) behind that MFMA.
 __device__ __forceinline__ void mfma_chain_end(f32x16& acc) { asm volatile("" : "+v"(acc)); }
+__device__ __forceinline__ void mfma_chain_end(f32x4_& acc) { asm volatile("" : "+v"(acc)); }
 
 }  // namespace mfma
 }  // namespace bsa

@@ -102,7 +102,7 @@ __device__ __forceinline__ void place(int id, int per_head, int heads, int head_
     }
 }
 
-constexpr int kPitchK = kD + 4;      // elements: 264-byte rows for 16-byte pieces read row by row
+constexpr int kPitchK = kD + 8;      // elements: 272-byte rows, sixteen of which read at one column fall on different banks
 constexpr int kPitchV = kD + 16;     // 288-byte rows: the transposing reads fetch 4 keys x 16 d per 16 lanes, and with rows 72 banks apart the four keys fall on different banks
 
 // kMode: rows as they are; with norm and rotation; and with a cache in front of k and v, or their rows written out.
@@ -269,9 +269,8 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         if (x.frag != nullptr) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                uint16_t* row = tile + front_place(s.word, rg + 16 * i) * kPitchK + c16 * 8;          // 8-byte aligned (pitch 264 B)
-                *reinterpret_cast<uint2*>(row) = make_uint2(xs[i].x, xs[i].y);
-                *reinterpret_cast<uint2*>(row + 4) = make_uint2(xs[i].z, xs[i].w);
+                uint16_t* row = tile + front_place(s.word, rg + 16 * i) * kPitchK + c16 * 8;
+                *reinterpret_cast<uint4*>(row) = xs[i];
             }
         }
         if (sub + 1 < per_chunk || hi + 1 < heads) {
@@ -288,10 +287,9 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int e = tid + 256 * i;                               // 16-byte piece of the output, 0..1023
-                const int l = e & 63, f = e >> 6;                          // lane and fragment: key half f / 8, d chunk f % 8
-                const uint16_t* p = tile + (32 * (f >> 3) + (l & 31)) * kPitchK + 16 * (f & 7) + 8 * (l >> 5);
-                const uint2 lo = *reinterpret_cast<const uint2*>(p), hi = *reinterpret_cast<const uint2*>(p + 4);
-                *reinterpret_cast<uint4*>(out + (int64_t)e * 16) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+                const int l = e & 63, f = e >> 6;                          // lane and fragment: key half f / 8, d chunk f / 2 % 4, its 16 keys f % 2
+                const uint16_t* p = tile + (32 * (f >> 3) + 16 * (f & 1) + (l & 15)) * kPitchK + 32 * ((f >> 1) & 3) + 8 * (l >> 4);
+                *reinterpret_cast<uint4*>(out + (int64_t)e * 16) = *reinterpret_cast<const uint4*>(p);
             }
             __syncthreads();                      // the next tile, or the sums below, may have the memory
         }
@@ -352,10 +350,9 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
         const int l = e & 63, f = e >> 6;
         // ds_read_b64_tr_b16: the 16 lanes of a group point at a 4-key x 16-d patch (lane s at key s / 4,
         // d 4 (s % 4) .. + 4) and each receives the 4 keys of one d
-        const int kh = f >> 3, s2 = (f >> 2) & 1, t = f & 3, lh = l >> 5;
-        const int s16 = l & 15, g1 = (l >> 4) & 1;
-        const uint16_t* from = tile + (32 * kh + 16 * s2 + 4 * lh + (s16 >> 2)) * kPitchV + 32 * t + 16 * g1 + 4 * (s16 & 3);
-        const s16x4 lo = lds_read_tr16(from), hi = lds_read_tr16(from + 8 * kPitchV);
+        const int kh = f >> 3, t = f & 7, s16 = l & 15, lg = l >> 4;
+        const uint16_t* from = tile + (32 * kh + 4 * lg + (s16 >> 2)) * kPitchV + 16 * t + 4 * (s16 & 3);
+        const s16x4 lo = lds_read_tr16(from), hi = lds_read_tr16(from + 16 * kPitchV);
         typedef short s16x8_ __attribute__((ext_vector_type(8)));
         *reinterpret_cast<s16x8_*>(out + (int64_t)e * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
