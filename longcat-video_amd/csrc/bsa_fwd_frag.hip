@@ -886,11 +886,8 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
             for (int qb = 0; qb < 4; ++qb) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) pb[qb][e] = (T)0.f;
-                neg_m[qb] = 0.f;
-                raise_at[qb] = -INFINITY;
                 alpha_p[qb] = 1.f;
             }
-            raise_low = -INFINITY;
             // the token rows of the next item's queries are looked up now; its list and its Q rows are asked for once
             // it is known that this item runs here
             int32_t next_rows[4] = {0, 0, 0, 0};
@@ -914,10 +911,17 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
 #pragma unroll
             for (int x = 0; x < 8; ++x) mfma_chain_end(s[0][x >> 2][x & 3]);
             mask_pair(s[0], first);
+            // the first maximum: nothing is accumulated yet that it would rescale
             float mx[4];
             lane_max(s[0], mx);
-            raise_max(mx);
-            rescale_pending = false;                                     // nothing accumulated yet
+#pragma unroll
+            for (int qb = 0; qb < 4; ++qb) {
+                m_i[qb] = over_lanes(mx[qb], [](float a, float b) { return fmaxf(a, b); }) * qk_scale;
+                neg_m[qb] = m_i[qb] == -INFINITY ? 0.f : -m_i[qb];
+                raise_at[qb] = (m_i[qb] + kTau) * inv_scale;
+            }
+            raise_low = fminf(fminf(raise_at[0], raise_at[1]), fminf(raise_at[2], raise_at[3]));
+            rescale_pending = false;
 
             // Cauchy-Schwarz: no logit of this item exceeds |q| times the largest key norm of the head.  If that bound
             // lies below the level at which the running maximum would be raised, no later step can raise it, and the steps

@@ -102,7 +102,7 @@ __device__ __forceinline__ void place(int id, int per_head, int heads, int head_
     }
 }
 
-constexpr int kPitchK = kD + 8;      // elements: 272-byte rows, sixteen of which read at one column fall on different banks
+constexpr int kPitchK = kD + 4;      // elements: 264-byte rows, read and written in 8-byte pieces (with rows of 272, whose pieces could be 16, the kernel has eight registers more, a wavefront a SIMD less, and a preview's launch takes 13.9 us for 13.2)
 constexpr int kPitchV = kD + 16;     // 288-byte rows: the transposing reads fetch 4 keys x 16 d per 16 lanes, and with rows 72 banks apart the four keys fall on different banks
 
 // kMode: rows as they are; with norm and rotation; and with a cache in front of k and v, or their rows written out.
@@ -270,7 +270,8 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 uint16_t* row = tile + front_place(s.word, rg + 16 * i) * kPitchK + c16 * 8;
-                *reinterpret_cast<uint4*>(row) = xs[i];
+                *reinterpret_cast<uint2*>(row) = make_uint2(xs[i].x, xs[i].y);
+                *reinterpret_cast<uint2*>(row + 4) = make_uint2(xs[i].z, xs[i].w);
             }
         }
         if (sub + 1 < per_chunk || hi + 1 < heads) {
@@ -284,12 +285,14 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         if (x.frag != nullptr) {
             __syncthreads();
             char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
+            // 16-byte piece tid + 256 i of the output: lane l of fragment w + 4 i, which is key half i / 2, d chunk w / 2 + 2 (i % 2), its 16 keys w % 2
+            const int l = tid & 63, w = tid >> 6;
+            const uint16_t* p = tile + (16 * (w & 1) + (l & 15)) * kPitchK + 32 * (w >> 1) + 8 * (l >> 4);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int e = tid + 256 * i;                               // 16-byte piece of the output, 0..1023
-                const int l = e & 63, f = e >> 6;                          // lane and fragment: key half f / 8, d chunk f / 2 % 4, its 16 keys f % 2
-                const uint16_t* p = tile + (32 * (f >> 3) + 16 * (f & 1) + (l & 15)) * kPitchK + 32 * ((f >> 1) & 3) + 8 * (l >> 4);
-                *reinterpret_cast<uint4*>(out + (int64_t)e * 16) = *reinterpret_cast<const uint4*>(p);
+                const uint16_t* at = p + 32 * (i >> 1) * kPitchK + 64 * (i & 1);
+                const uint2 lo = *reinterpret_cast<const uint2*>(at), hi = *reinterpret_cast<const uint2*>(at + 4);
+                *reinterpret_cast<uint4*>(out + (int64_t)(tid + 256 * i) * 16) = make_uint4(lo.x, lo.y, hi.x, hi.y);
             }
             __syncthreads();                      // the next tile, or the sums below, may have the memory
         }
@@ -344,17 +347,16 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(tile + front_place(s.word, rg + 16 * i) * kPitchV + c16 * 8) = xs[i];
     __syncthreads();
     char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
+    // ds_read_b64_tr_b16: the 16 lanes of a group point at a 4-key x 16-d patch (lane s at key s / 4,
+    // d 4 (s % 4) .. + 4) and each receives the 4 keys of one d.  Piece threadIdx.x + 256 i: lane l of fragment w + 4 i, key half i / 2, d tile w + 4 (i % 2)
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint16_t* from = tile + (4 * (l >> 4) + ((l & 15) >> 2)) * kPitchV + 16 * w + 4 * (l & 3);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int e = threadIdx.x + 256 * i;
-        const int l = e & 63, f = e >> 6;
-        // ds_read_b64_tr_b16: the 16 lanes of a group point at a 4-key x 16-d patch (lane s at key s / 4,
-        // d 4 (s % 4) .. + 4) and each receives the 4 keys of one d
-        const int kh = f >> 3, t = f & 7, s16 = l & 15, lg = l >> 4;
-        const uint16_t* from = tile + (32 * kh + 4 * lg + (s16 >> 2)) * kPitchV + 16 * t + 4 * (s16 & 3);
-        const s16x4 lo = lds_read_tr16(from), hi = lds_read_tr16(from + 16 * kPitchV);
+        const uint16_t* at = from + 32 * (i >> 1) * kPitchV + 64 * (i & 1);
+        const s16x4 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 16 * kPitchV);
         typedef short s16x8_ __attribute__((ext_vector_type(8)));
-        *reinterpret_cast<s16x8_*>(out + (int64_t)e * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        *reinterpret_cast<s16x8_*>(out + (int64_t)(threadIdx.x + 256 * i) * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
 }
 
