@@ -442,7 +442,7 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->off_kp = take(bh * kv_rows * p->D * pl->es);
     pl->off_vp = take(bh * kv_rows * p->D * pl->es);
     pl->off_qc = take(bh * pl->nbq * p->D * pl->es);
-    pl->off_kc = take(bh * pl->nbk * p->D * pl->es);
+    pl->off_kc = take(bh * ((pl->nbk + 31) / 32 * 32) * p->D * pl->es);      // in operand order groups of 32 are filled up
     pl->off_score = take(bh * pl->nbq * (size_t)pl->nbk * pl->es);
     pl->off_idx = take(bh * pl->nbq * (size_t)(pl->sel_width > 0 ? pl->sel_width : 1) * sizeof(int32_t));
     pl->off_idx_sorted = take(bh * pl->nbq * (size_t)(pl->sel_width > 0 ? pl->sel_width : 1) * sizeof(int32_t));
@@ -540,7 +540,7 @@ int check_kv_views(const Plan& pl, const int64_t k_strides[3], const int64_t v_s
 hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, const void* q, const int64_t q_strides[3],
                        const void* k, const int64_t k_strides[3], const void* v, const int64_t v_strides[3], bool pool,
                        hipStream_t st, const bsa_qk_norm* qkn = nullptr, void* q_normed = nullptr, const int64_t* qn_strides = nullptr,
-                       const bsa_kv_cache* c = nullptr) {
+                       const bsa_kv_cache* c = nullptr, bool operand_means = false) {
     hipError_t e;
     const bool padded_k = kv_padded(p);
     if (pl.frag) {
@@ -556,6 +556,7 @@ hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, cons
         a.v.frag = static_cast<char*>(w.vp);
         if (pool) {
             a.k.pooled = static_cast<uint16_t*>(w.kc);
+            a.k.pooled_operand = operand_means;
             a.q = prep_rows(q, q_strides);
             a.q.pooled = static_cast<uint16_t*>(w.qc);
             a.q.rows = w.qrows;
@@ -708,16 +709,21 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
     }
     hipStream_t st = (hipStream_t)stream;
     hipError_t e;
+    // the selection is made in front of the attention kernel, or by it where the caller asks for nothing but what it walks (launch_fwd_frag)
+    const bool by_attention = (pl.frag || pl.f32) && idx_out == nullptr && score_out == nullptr && pl.sel_width > 0;
+    const bool inside = by_attention && pl.frag &&
+                        frag_selects((int64_t)p->B * p->Hn, pl.Sqp, pl.Skp, pl.gk.chunk(), pl.half_width > 0 ? pl.half_width : pl.sel_width,
+                                     pl.half_width > 0 ? &pl.gk : nullptr, &pl.gq, !pl.cdf, pl.nbk, pl.sel_width);
 #define BSA_HIP(call, what) do { e = (call); if (e != hipSuccess) return hip_fail(e, what); } while (0)
     if (qkn != nullptr) {
         // q and k as the projection left them: the pass that takes q's chunk means also normalises and rotates its
         // rows into q_normed (what the attention kernel then reads), the pass that rewrites k in fragment order
         // normalises and rotates on the way
-        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, qkn, q_normed, qn_strides, kvc), "pool, norm, rotate and prepare");
+        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, qkn, q_normed, qn_strides, kvc, inside), "pool, norm, rotate and prepare");
         q = q_normed;
         q_strides = qn_strides;
     } else if (!pl.f32) {
-        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st), "pool and prepare");
+        BSA_HIP(prepare_thw(pl, p, w, q, q_strides, k, k_strides, v, v_strides, true, st, nullptr, nullptr, nullptr, nullptr, inside), "pool and prepare");
     } else {
         BSA_HIP(launch_pool_f32(q, q_strides, pl.gq, (float*)w.qc, w.qrows, k, k_strides, pl.gk, (float*)w.kc, w.krows, p->B, p->Hn, st),
                 "pool q and k");
@@ -742,11 +748,9 @@ int fwd_3d_impl(const Plan& pl, const bsa_3d_params* p, const void* q, const int
             r = launch_pace_order(w.idx_sorted, w.idx_sorted, w.lens, sel_rows, pl.nbk, pl.sel_width, st, halves);
         return r;
     };
-    // made in front of the attention kernel, or by it where the caller asks for nothing but what it walks (launch_fwd_frag)
-    const bool by_attention = (pl.frag || pl.f32) && idx_out == nullptr && score_out == nullptr && pl.sel_width > 0;
     const bool lists_wanted = walk_out != nullptr || lens_out != nullptr;
     const GateCall gate = {w.qc, w.kc, lists_wanted ? w.idx_sorted : nullptr, lists_wanted ? w.lens : nullptr, w.valid, pl.nbk, pl.sel_width,
-                           pl.cdf ? p->cdf_threshold : 0.f, p->sm_scale, k_min,
+                           pl.cdf ? p->cdf_threshold : 0.f, p->sm_scale, k_min, inside,
                            [](void* ctx) { return (*static_cast<decltype(select)*>(ctx))(); }, &select};
     if (!by_attention) BSA_HIP(select(), "selection");
     if (!pl.f32) {

@@ -227,6 +227,7 @@ struct GateCall {
     int nbk, width;                  // width: the top-k rule's count, the most of the CDF rule's
     float threshold, scale;          // CDF rule (launch_cdf_count), threshold 0: top-k
     int k_min;
+    bool inside;                     // launch_fwd_frag: the attention kernel makes it (frag_selects)
     hipError_t (*make)(void* ctx);
     void* ctx;
 };
@@ -286,6 +287,7 @@ struct PrepRows {
     int heads;                       // set by launch_prepare: heads of a chunk that a workgroup takes
     char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, the real slots of a tile first, zeros behind
     uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
+    int pooled_operand;              // k: ... in operand order instead (operand_mean_at)
     int32_t* rows;                   // q: row_table_ints() entries; the real slots of a chunk come first
     uint64_t* valid;                 // k, optional: bit s of word i = slot 64 i + s holds a real token
     const uint64_t* valid_in;        // k, v, optional: the real slots of every tile as the caller has them (instead of the grid's)
@@ -297,6 +299,11 @@ struct PrepRows {
     int head_fastest;                // set by launch_prepare: the order in which workgroups take (chunk, head)
     int offsets_32;                  // set by launch_prepare: the rows of a (batch, head) lie within 4 GB
 };
+// Chunk means of k as the attention kernel's products take them where it selects itself, 32 blocks of a (batch, head) to a group: a product's
+// fragment (16 of the 128 d) is 1 KB in lane order, lane l block l % 32 and d 8 (l / 32) .. + 8.  The last group is filled up.
+__host__ __device__ inline int64_t operand_mean_at(int64_t bh, int blocks, int blk, int d) {
+    return ((bh * ((blocks + 31) / 32) + blk / 32) * 8 + d / 16) * 512 + (d >> 3 & 1) * 256 + (blk & 31) * 8 + (d & 7);
+}
 struct PrepArgs {
     PrepRows q, k, v;
     Grid3 gq, gk;
@@ -332,6 +339,8 @@ constexpr int kFragQueueWords = 16;
 size_t frag_part_floats(const Grid3& q_grid, int64_t heads);
 // Work items of a call, those of its last, partial round, and how these are shared: `parts` parts of an item, `team` wavefronts a part.
 struct LastRound { int total, items, team, parts; };
+// Whether the attention kernel makes the lists of a call itself; then the chunk means of k are in operand order.
+bool frag_selects(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length, int nbk, int width);
 LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length);
 // halves_of (optional): idx and lens are HalfLists, idx_stride their row pitch (at most 4 096), of this grid of keys.
 // gate_call (optional): idx and lens are still to be made.

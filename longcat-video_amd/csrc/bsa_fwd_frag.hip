@@ -149,7 +149,7 @@ static_assert(kTeamBytes<4> <= 160 * 1024 && 2 * (kTeamBytes<2> + 512) <= 160 * 
 // ([BH][nbq][width]) and their lengths go, null: nowhere.  (As arguments of their own they would be 392 bytes, beyond what is asked for
 // together, and two arguments that the kernel can do without in their place cost the layers 0.3 to 0.7 %, by where the loop then lies.)
 struct FragGate {
-    const uint16_t *qc, *kc;         // chunk means, 16-bit storage
+    const uint16_t *qc, *kc;         // chunk means, 16-bit storage; k's in operand order (operand_mean_at)
     int nbk, width;                  // entries of a list: the top-k rule's count, the most of the CDF rule's
     float threshold, scale;          // of the CDF rule, as cdf_count_kernel's; threshold 0: top-k
     int k_min;
@@ -712,7 +712,8 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                     for (int i = threadIdx.x; i < G.nbk * nsub_of_block; i += 64 * kTeam) counts[i] = (uint8_t)__popcll(tile_valid[i]);
                 const int lr = lane & 31, lh = lane >> 5;
                 const T* const qm = reinterpret_cast<const T*>(G.qc) + brow * kD + lh * 8;      // its mean as every row of the product
-                const T* const km = reinterpret_cast<const T*>(G.kc) + (int64_t)bh * G.nbk * kD + lh * 8;
+                // k's means in whole kilobytes; as rows of 256 bytes a load took 32 bytes of each of 32
+                const T* const km = reinterpret_cast<const T*>(G.kc) + operand_mean_at(bh, G.nbk, 0, 0) + lane * 8;
                 V8 qa[8];
 #pragma unroll
                 for (int c = 0; c < 8; ++c) qa[c] = *reinterpret_cast<const V8*>(qm + 16 * c);
@@ -723,9 +724,9 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                     for (int t = 0; t < 4; ++t) {
                         const int n0 = n_first + 32 * kTeam * t;
                         if (n0 < G.nbk) {
-                            const T* const kt = km + (int64_t)min(n0 + lr, G.nbk - 1) * kD;
+                            const T* const kt = km + n0 / 32 * 4096;
 #pragma unroll
-                            for (int c = 0; c < 8; ++c) kr[t][c] = *reinterpret_cast<const V8*>(kt + 16 * c);
+                            for (int c = 0; c < 8; ++c) kr[t][c] = *reinterpret_cast<const V8*>(kt + 512 * c);
                         }
                     }
 #pragma unroll
@@ -1465,6 +1466,15 @@ static Rounds plan_rounds(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int i
         r.split = choose_split(r.tail, r.list_tiles, r.resident, r.total > r.resident, one_length, halves_of);
     return r;
 }
+// The lists of a call whose workgroups all run at once are made by those that walk them.  The kernels in front / like this, us, density
+// 1/16: one wavefront an item, 768 items of 192 blocks 48.3 / 46.7, 672 of 224 49.0 / 47.3, 768 of 256 54.8 / 53.9, 1 024 of 256, the most
+// that there are, 64.1 / 64.3 (at density 1/4 151.2 / 151.0); teams of four, 320 of 320 43.7 / 40.0, 512 of 512 66.6 / 62.5; one
+// workgroup behind another pays for it twice (2 heads of 320 blocks, teams of four, density 1/4, 147 / 156).
+bool frag_selects(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length, int nbk, int width) {
+    const Rounds r = plan_rounds(heads, Sq, Sk, bs_k, idx_stride, halves_of, q_grid, one_length);
+    return r.one_span && r.split.parts == 1 && r.total * r.split.team <= r.resident && nbk <= (r.split.team == 1 ? kGateWaveBlocks : kGateMostBlocks) &&
+           gate_here_bytes(nbk, width, bs_k / kTile, halves_of != nullptr) <= kTile * (kD + 8) * 2;
+}
 LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length) {
     const Rounds r = plan_rounds(heads, Sq, Sk, bs_k, idx_stride, halves_of, q_grid, one_length);
     return {r.total, r.tail, r.split.team, r.split.parts};
@@ -1548,15 +1558,9 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         }                                                                                                              \
     } while (0)
     const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
-    // The lists of a call whose workgroups all run at once are made by those that walk them.  The kernels in front / like this, us, density
-    // 1/16: one wavefront an item, 768 items of 192 blocks 48.3 / 46.7, 672 of 224 49.0 / 47.3, 768 of 256 54.8 / 53.9, 1 024 of 256, the most
-    // that there are, 64.1 / 64.3 (at density 1/4 151.2 / 151.0); teams of four, 320 of 320 43.7 / 40.0, 512 of 512 66.6 / 62.5; one
-    // workgroup behind another pays for it twice (2 heads of 320 blocks, teams of four, density 1/4, 147 / 156).
     if (gate_call != nullptr) {
         const GateCall& c = *gate_call;
-        const int nsub = bs_k / kTile;
-        if (once && split.parts == 1 && total * split.team <= resident && c.nbk <= (split.team == 1 ? kGateWaveBlocks : kGateMostBlocks) &&
-            gate_here_bytes(c.nbk, c.width, nsub, halves) <= kTile * (kD + 8) * 2) {
+        if (c.inside) {
             here = {static_cast<const uint16_t*>(c.q_cmp), static_cast<const uint16_t*>(c.k_cmp), c.nbk, c.width, c.threshold, c.scale, c.k_min,
                     pace_divisor(c.nbk, c.width)};
             gate_lists = c.lists;

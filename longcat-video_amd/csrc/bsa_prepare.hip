@@ -305,7 +305,8 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         if (threadIdx.x < kD) {
             float sum = 0.f;
             for (int i = 0; i < 16; ++i) sum += red[i * kD + threadIdx.x];
-            x.pooled[((int64_t)bh * g.blocks() + blk) * kD + threadIdx.x] = narrow<kBf16>(sum * (1.0f / g.chunk()));
+            const int64_t at = x.pooled_operand ? operand_mean_at(bh, g.blocks(), blk, threadIdx.x) : ((int64_t)bh * g.blocks() + blk) * kD + threadIdx.x;
+            x.pooled[at] = narrow<kBf16>(sum * (1.0f / g.chunk()));
         }
         __syncthreads();                          // the next head may have the memory
     }
