@@ -470,6 +470,13 @@ int bsa_lora_add(const void* org, const void* const* up, const float* multiplier
 int bsa_lora_up_add(const void* org, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank, float multiplier,
                     float alpha_scale, void* out, int64_t M, int N, void* stream);
 
+/* A Linear with one side branch from its down projection on: out = T(x . w^T + bias + s), s = multiplier * alpha_scale * up(t), bf16 in and
+ * out.  Operands as in bsa_linear_bf16 (rows of x, w and out next to each other, the workspace too) and bsa_lora_up_add.  Where the engine's
+ * GEMM serves it, all of it is accumulated in fp32 and rounded once; otherwise bsa_linear_bf16 and bsa_lora_up_add with
+ * their roundings, and what these are not built for is refused as there.  out must be memory of its own. */
+int bsa_linear_lora_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
+                         float multiplier, float alpha_scale, void* out, int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream);
+
 /* bsa_fwd_3d for the attention module (attention.py:116-137): q and k arrive as the QKV projection left them
  * (strided views into its output are fine) and go through the per-head RMSNorm (RMSNorm_FP32, blocks.py:42-53) and
  * the 3-D RoPE (rope_3d.py:100-120) inside the operator's own passes over them, at the rounding points of

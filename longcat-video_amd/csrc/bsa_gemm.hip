@@ -35,6 +35,9 @@
 // over blocks of 8 token tiles, and the workgroups of an XCD have a contiguous share of it, 8 x 4 tiles at a time: in step, they
 // fetch a slab once for 4 or 8 of them.
 //
+// A LoRA side branch is more of the same sum: a tile's first k blocks are those of the rank axis (t . up^T, scaled where they end), for a pass
+// that reads and writes the layer's output at 4 TB/s.  Its two blocks of 66 cost 3 % of the product (128 multiplications a lane included).
+//
 // What bounds it: power, and the reading half of a phase.  Per k block and group 610 clocks to request 32 KB (the address unit of a
 // CU takes 16 a load of 1 KB, and a wavefront issues in order) and 500 to read 96 KB of fragments, against 1 009 of MFMAs, so the
 // MFMAs run 0.76 of the clocks at 1.87 GHz.  Measured and not kept: the requests between the fragment reads (R 1 170 clocks)
@@ -61,7 +64,9 @@ constexpr int kBlockM = 8;               // token tiles that the order of the ti
 
 typedef bf16x8 V8;
 
-enum Epilogue { kPlain, kResidual, kQkv };
+constexpr int kMaxSlices = 8;
+
+enum Epilogue { kPlain, kResidual, kQkv, kLora };
 
 struct GemmArgs {
     const __bf16* x; int64_t ldx;
@@ -78,6 +83,11 @@ struct GemmArgs {
     const float* tab;
     int Hn, S, Hg, Wg, t0, Ttab;
     float eps;
+    // a LoRA side branch: t [M, slices * rank], up [per, rank] for every `per` features
+    const __bf16* t; int64_t ldt;
+    const __bf16* up[kMaxSlices];
+    int per, rank;
+    float scale;
 };
 
 template <int kEpi>
@@ -106,15 +116,23 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
     uint32_t pitch;
     int last_row;
     int next_t = t_first, left = 0;                   // tile that is being brought, k blocks of it that are not yet
-    const int nblocks = a.K / kBK;
+    const int side_blocks = kEpi == kLora ? a.rank / kBK : 0, nblocks = side_blocks + a.K / kBK;
+    bool side = kEpi == kLora;                        // a tile's blocks are those of its side branch, then those of the layer
     const uint32_t lds0 = lds_address(smem);
-    auto start_tile = [&]() __attribute__((always_inline)) {
+    auto start_part = [&]() __attribute__((always_inline)) {
         int tm, tf;
         place(next_t, tm, tf);
+        last_row = group ? a.M - 1 - tm * kTileM : a.N - 1 - tf * kTileN;
+        if (kEpi == kLora && side) {
+            const int f = tf * kTileN, slice = f / a.per;                     // slices are whole tiles
+            from = group ? reinterpret_cast<const char*>(a.t + (int64_t)tm * kTileM * a.ldt + slice * a.rank) : reinterpret_cast<const char*>(a.up[slice] + (int64_t)(f - slice * a.per) * a.rank);
+            pitch = (uint32_t)(group ? a.ldt : a.rank) * 2u;
+            left = side_blocks;
+            return;
+        }
         from = group ? reinterpret_cast<const char*>(a.x + (int64_t)tm * kTileM * a.ldx) : reinterpret_cast<const char*>(a.w + (int64_t)tf * kTileN * a.ldw);
         pitch = (uint32_t)(group ? a.ldx : a.ldw) * 2u;
-        last_row = group ? a.M - 1 - tm * kTileM : a.N - 1 - tf * kTileN;
-        left = nblocks;
+        left = nblocks - side_blocks;
     };
     // half-slab h (even: token rows, odd: weight rows, of k block h / 2 of all of this workgroup's tiles) lives in stage h % kStages
     auto bring = [&](int stage) __attribute__((always_inline)) {
@@ -129,8 +147,14 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
         }
         from += kBK * 2;
         if (--left == 0) {
-            next_t += per_xcd;
-            if (next_t < t_end) start_tile();
+            if (kEpi == kLora && side) {
+                side = false;
+                start_part();
+            } else {
+                next_t += per_xcd;
+                side = kEpi == kLora;
+                if (next_t < t_end) start_part();
+            }
         }
     };
 
@@ -158,7 +182,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
     };
 
     // ---- pipeline
-    start_tile();
+    start_part();
     if (group) {
         bring(0);
         if (left) {
@@ -198,6 +222,16 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
                 for (int i = 0; i < 8; ++i)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(af[ks][i], bf[ks][j], acc[i][j]);
+            if constexpr (kEpi == kLora) {
+                if (kb + 1 == side_blocks && a.scale != 1.f) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[i][j][r] *= a.scale;
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
             if (!group) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (!group || kb + 1 < nblocks || t + per_xcd < t_end) meet();
@@ -401,6 +435,27 @@ bool gemm_serves_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, 
     return residual != nullptr && 5 * tiles >= 4 * round;
 }
 
+// Which layers with a LoRA side branch run as one product, a rank of whole k blocks and slices of whole tiles: us, the library's product and
+// lora_up_add_kernel / this kernel.  Rank 128, tiles that fill their rounds: 32 760 x 12 288 x 4 096 2 471 / 2 386 (the library alone 2 115), x 4 096 x 4 096
+// 834 / 809, 86 400 x 4 096 x 4 096 2 276 / 2 192, 20 000 x 3 072 x 1 024 170 / 127.  Three quarters full 2 000 x 12 288 x 4 096 187 / 173, 0.73
+// 12 000 x 2 048 x 2 048 105 / 94, two thirds 1 560 x 12 288 x 4 096 152 / 169, 0.56 9 000 x 2 048 x 2 048 89 / 90.  A short K has less to lose: K = 1 024
+// 0.54 full 17 500 x 1 024 67 / 56, 3 000 x 3 072 45 / 29, a quarter full 4 000 x 1 024 24 / 27; K = 512 0.16 full 20.2 / 19.0, 0.09 level, K = 256 400 x 768
+// 16.5 / 12.9, 30 000 x 256 32 / 17.  Pointers and rows as above.
+static bool lora_serves(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
+                        const void* out, int64_t M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || n_sep <= 0 || n_sep > kMaxSlices || rank <= 0 || rank % kBK || rank > 128) return false;
+    if (K % kBK || K >= (1 << 22) || N % n_sep || N / n_sep % kTileN || ldt < (int64_t)n_sep * rank || ldt % 8 || ldt >= (1 << 22)) return false;
+    const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+    if (((at(x) | at(w) | at(t) | at(out)) & 15u) || (at(bias) & 7u)) return false;
+    const uintptr_t o = at(out), o_end = o + (uintptr_t)M * N * 2u;
+    const auto meets = [&](const void* p, uintptr_t bytes) { return p != nullptr && at(p) < o_end && o < at(p) + bytes; };
+    if (meets(x, (uintptr_t)M * K * 2u) || meets(w, (uintptr_t)N * K * 2u) || meets(bias, (uintptr_t)N * 2u) || meets(t, (uintptr_t)((M - 1) * ldt + n_sep * rank) * 2u)) return false;
+    for (int i = 0; i < n_sep; ++i)
+        if (!up[i] || (at(up[i]) & 15u) || meets(up[i], (uintptr_t)(N / n_sep) * rank * 2u)) return false;
+    const int64_t tiles = (M + kTileM - 1) / kTileM * (N / kTileN), round = (tiles + kCus - 1) / kCus * kCus;
+    return K <= 512 || 4 * tiles >= (K <= 1024 ? 2 : 3) * round;
+}
+
 }  // namespace bsa
 
 using namespace bsa;
@@ -421,6 +476,22 @@ int bsa_gemm_bf16(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
     a.residual = (const __bf16*)residual; a.ldr = ldr; a.out = (__bf16*)out; a.ldo = ldo;
     a.M = (int)M; a.N = N; a.K = K;
     return residual ? launch_gemm<kResidual>(a, (hipStream_t)stream) : launch_gemm<kPlain>(a, (hipStream_t)stream);
+}
+
+int bsa_linear_lora_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
+                         float multiplier, float alpha_scale, void* out, int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!x || !w || !t || !up || !out) return set_error(BSA_ERR_BAD_ARG, "linear_lora: null pointer");
+    if (!lora_serves(x, w, bias, t, ldt, up, n_sep, rank, out, M, N, K)) {
+        const int rc = bsa_linear_bf16(x, w, bias, nullptr, out, M, N, K, workspace, workspace_bytes, stream);
+        return rc != BSA_OK ? rc : bsa_lora_up_add(out, t, ldt, up, n_sep, rank, multiplier, alpha_scale, out, M, N, stream);
+    }
+    GemmArgs a = {};
+    a.x = (const __bf16*)x; a.ldx = K; a.w = (const __bf16*)w; a.ldw = K; a.bias = (const __bf16*)bias;
+    a.out = (__bf16*)out; a.ldo = N;
+    a.M = (int)M; a.N = N; a.K = K;
+    a.t = (const __bf16*)t; a.ldt = ldt; a.per = N / n_sep; a.rank = rank; a.scale = multiplier * alpha_scale;
+    for (int i = 0; i < n_sep; ++i) a.up[i] = (const __bf16*)up[i];
+    return launch_gemm<kLora>(a, (hipStream_t)stream);
 }
 
 int bsa_qkv_projection(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* q_weight,

@@ -30,7 +30,7 @@ struct UpSlices {
 //
 // 32 760 tokens, rank 128, 12 288 columns in three slices and 4 096 in one: 537 us = 4.0 TB/s, for 943 us of up-projections
 // (hipBLASLt, 364) and lora_add_kernel (579) before.  64 tokens a turn, two workgroups a CU 631; org a turn ahead 566 (its
-// registers cost more than the wait).  It is taken wherever it is built: one pass / separate ones, us, by tokens 1, 256, 4 096,
+// registers cost more than the wait).  It is taken wherever it is built and the engine's GEMM does not take the branch into its sum (lora_serves): one pass / separate ones, us, by tokens 1, 256, 4 096,
 // 32 760: 4 096 columns, rank 16 4.3 / 20.8, 4.0 / 20.7, 12.0 / 32.6, 86 / 242, rank 128 4.5 / 20.6, 6.0 / 20.4, 22.8 / 29.3, 120 / 230;
 // 12 288 in three, rank 16 4.0 / 41, 4.8 / 41, 33 / 85, 310 / 701, rank 128 4.5 / 41, 9.5 / 41, 50 / 80, 369 / 675; 512 columns, rank 128,
 // 4.4 / 20.4, 5.7 / 20.2, 6.4 / 20.3, 23.7 / 31.4 (below 30 us the separate ones wait for the host).

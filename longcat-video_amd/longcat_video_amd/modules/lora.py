@@ -3,18 +3,19 @@
 The reference patches the forward of every Linear a LoRA file names (longcat_video_dit.py:211-249):
 ``org_forward(x) + sum_i lora_up_i(lora_down_i(x)) * multiplier_i * alpha_scale_i``.  ``lora_up`` is either one
 Linear or, for fused projections such as qkv, one Linear per equal slice of the output features, each fed its own
-slice of the rank axis (lora_utils.py:12-21, 47-53).  Here the layer and the down projection go to hipBLASLt through the
-C ABI; the up-projection of a single branch, its scaling and the sum are one pass over the layer's output
-(bsa_lora_up_add).  Several branches, whose scaled terms are summed before the layer's output is added, take their
-up-projections from hipBLASLt too (the sliced one with row strides, in place) and one elementwise pass.  Both with the
-eager expression's roundings.
+slice of the rank axis (lora_utils.py:12-21, 47-53).  Here the down projection goes to hipBLASLt through the C ABI; the layer with
+a single branch is one call (bsa_linear_lora_bf16): one product of the engine's GEMM, in fp32 up to its one rounding, or the layer by
+hipBLASLt and one pass over its output with the eager expression's roundings.  Several branches, whose scaled terms are summed before the
+layer's output is added, take their up-projections from hipBLASLt too (the sliced one with row strides, in place) and one
+elementwise pass, with the eager roundings.
 """
+import ctypes as C
 from typing import List, Optional, Sequence
 
 import torch
 
 from .. import _capi
-from .attention import _gemm_workspace, _on_device, _ptr, _stream, linear_bf16
+from .attention import _bf16, _gemm_workspace, _on_device, _ptr, _stream, linear_bf16
 
 MAX_BRANCHES = 4
 
@@ -67,43 +68,58 @@ def _up_projection(lx: torch.Tensor, branch: LoRABranch, workspace: torch.Tensor
 
 
 def _one_pass(b: LoRABranch) -> bool:
-    """What bsa_lora_up_add is built for, and faster at from 1 to 32 760 tokens, rank 16 to 128 and 64 to 12 288 columns (figures at the
-    kernel); other branches, and sums over several, take the up-projection as a tensor."""
+    """What bsa_linear_lora_bf16 is built for, and faster at from 1 to 32 760 tokens, rank 16 to 128 and 64 to 12 288 columns (figures at the
+    kernels); other branches, and sums over several, take the up-projection as a tensor."""
     per = b.lora_up[0].shape[0]
     return (b.rank % 16 == 0 and b.rank <= 128 and len(b.lora_up) <= 8 and per % 64 == 0
             and all(u.dtype == torch.bfloat16 and (not u.is_contiguous() or u.data_ptr() % 16 == 0) for u in b.lora_up))
+
+
+def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace) -> torch.Tensor:
+    """The down projection, then the layer with its side branch."""
+    M, K, N = x2.shape[0], x2.shape[1], weight.shape[0]
+    assert weight.shape[1] == K and b.out_features == N and b.lora_down.shape[1] == K
+    if b.lora_down.dtype != torch.bfloat16:
+        raise NotImplementedError("LoRA weights must be bf16 (the reference moves them to the model dtype)")
+    x2 = x2.contiguous()
+    lx = linear_bf16(x2, b.lora_down, None, workspace=workspace)                  # [M, n_sep * rank]
+    w, bw = _bf16(weight), None if bias is None else _bf16(bias)
+    ups = [u.contiguous() for u in b.lora_up]
+    ptrs = (C.c_void_p * len(ups))(*[u.data_ptr() for u in ups])
+    out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
+    with _on_device(x):
+        _capi.check(_capi.load().bsa_linear_lora_bf16(_ptr(x2), _ptr(w), _ptr(bw), _ptr(lx), lx.shape[1], ptrs, len(ups), b.rank,
+                                                      float(b.multiplier), alpha, _ptr(out), M, N, K, _ptr(workspace),
+                                                      workspace.numel(), _stream(x)), "linear with a LoRA branch")
+    return out
 
 
 @torch.no_grad()
 def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                 loras: Optional[List[LoRABranch]] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The patched forward of longcat_video_dit.py:234-249 for a bf16 Linear."""
-    org = linear_bf16(x, weight, bias, workspace=workspace)
     active = [b for b in (loras or []) if b.use_lora]
     if not active:
-        return org                                 # `org_output + 0`
+        return linear_bf16(x, weight, bias, workspace=workspace)                    # `org_output + 0`
     if len(active) > MAX_BRANCHES:
         raise NotImplementedError("at most %d LoRA branches per Linear are built" % MAX_BRANCHES)
+    if not x.is_cuda:
+        raise RuntimeError("the engine runs on the GPU only")
     if workspace is None:
         workspace = _gemm_workspace(x.device)
     N = weight.shape[0]
     x2 = x.reshape(-1, x.shape[-1])
-    import ctypes as C
     # alpha_scale lives in a bf16 buffer in the reference
     alphas = [float(torch.tensor(b.alpha_scale, dtype=torch.bfloat16)) for b in active]
+    if len(active) == 1 and _one_pass(active[0]):
+        return _with_one_branch(x, x2, weight, bias, active[0], alphas[0], workspace)
+    org = linear_bf16(x, weight, bias, workspace=workspace)
     ups = []
     for b, a in zip(active, alphas):
         assert b.out_features == N and b.lora_down.shape[1] == x.shape[-1]
         if b.lora_down.dtype != torch.bfloat16:
             raise NotImplementedError("LoRA weights must be bf16 (the reference moves them to the model dtype)")
         lx = linear_bf16(x2, b.lora_down, None, workspace=workspace)              # [M, n_sep * rank]
-        if len(active) == 1 and _one_pass(b):
-            w = [u.contiguous() for u in b.lora_up]
-            ptrs = (C.c_void_p * len(w))(*[u.data_ptr() for u in w])
-            with _on_device(x):
-                _capi.check(_capi.load().bsa_lora_up_add(_ptr(org), _ptr(lx), lx.shape[1], ptrs, len(w), b.rank, float(b.multiplier), a,
-                                                         _ptr(org), lx.shape[0], N, _stream(x)), "lora_up_add")
-            return org
         ups.append(_up_projection(lx, b, workspace))
     n = len(ups)
     up_ptrs = (C.c_void_p * n)(*[u.data_ptr() for u in ups])

@@ -371,6 +371,27 @@ def test_lora_up_projection_and_sum(M, r, n_sep, per, multiplier, alpha_scale):
     assert torch.equal(L().lora_linear(x.cuda(), w.cuda(), None, [br]).cpu(), want)
 
 
+@pytest.mark.parametrize("scale", [1.0, 0.5])
+@pytest.mark.parametrize("M,K,r,n_sep,per", [
+    (4500, 64, 64, 3, 1024), (4417, 64, 128, 3, 1024), (4609, 320, 64, 3, 1024),      # one block of the side branch or of the layer, edges
+    (8961, 192, 128, 1, 3072), (52300, 128, 64, 1, 256), (17700, 128, 128, 3, 256),         # more tiles than workgroups
+    (1, 64, 64, 1, 256), (257, 512, 128, 8, 256),                                           # one tile, and one row in the second
+])
+def test_layer_with_lora_branch_in_one_product(M, K, r, n_sep, per, scale):
+    """Where the tiles fill the chip the side branch is a part of the layer's sum, which is rounded once: small integers are exact up to that, so
+    the result is that of the fp32 sum (the up-projection is no bf16 number: rounded by itself it would show)."""
+    g = torch.Generator(device="cuda").manual_seed(M + r)
+    ints = lambda lo, hi, *s: torch.randint(lo, hi, s, generator=g, device="cuda").bfloat16()      # noqa: E731
+    x, w, b = ints(-2, 3, M, K), ints(-2, 3, n_sep * per, K), ints(-2, 3, n_sep * per)
+    br = L().LoRABranch(ints(-1, 2, n_sep * r, K), [ints(-9, 10, per, r) for _ in range(n_sep)], scale, r)
+    t = (x.float() @ br.lora_down.float().T).bfloat16().float()
+    up = torch.cat([t[:, i * r:(i + 1) * r] @ u.float().T for i, u in enumerate(br.lora_up)], 1)
+    want = (x.float() @ w.float().T + b.float() + scale * up).bfloat16()
+    assert not torch.equal(up, up.bfloat16().float())
+    assert torch.equal(L().lora_linear(x, w, b, [br]), want)
+    assert torch.equal(L().lora_linear(x, w, None, [br]), (x.float() @ w.float().T + scale * up).bfloat16())
+
+
 def test_module_forward_with_lora_branches():
     """longcat_video_dit.py:211-249: LoRA branches on attn.qkv (up-projection split in three) and attn.proj."""
     shape = (4, 8, 8)
