@@ -477,6 +477,13 @@ int bsa_lora_up_add(const void* org, const void* t, int64_t ldt, const void* con
 int bsa_linear_lora_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
                          float multiplier, float alpha_scale, void* out, int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same behind a gate, as a DiT block adds its attention (longcat_video_dit.py:101-103): out = T(residual + gate * y), y the layer's output
+ * with its side branch, or, with t NULL, without one.  gate: fp32 [M / rows_per_group, N].  One rounding where the engine's GEMM serves
+ * it, otherwise that of y and that of bsa_gated_residual.  out must be memory of its own. */
+int bsa_linear_gated_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
+                          float multiplier, float alpha_scale, const void* residual, const float* gate, int rows_per_group, void* out,
+                          int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream);
+
 /* bsa_fwd_3d for the attention module (attention.py:116-137): q and k arrive as the QKV projection left them
  * (strided views into its output are fine) and go through the per-head RMSNorm (RMSNorm_FP32, blocks.py:42-53) and
  * the 3-D RoPE (rope_3d.py:100-120) inside the operator's own passes over them, at the rounding points of

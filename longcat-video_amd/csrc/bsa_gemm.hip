@@ -37,6 +37,8 @@
 //
 // A LoRA side branch is more of the same sum: a tile's first k blocks are those of the rank axis (t . up^T, scaled where they end), for a pass
 // that reads and writes the layer's output at 4 TB/s.  Its two blocks of 66 cost 3 % of the product (128 multiplications a lane included).
+// A gated residual is added in the epilogue, for the same reason: 24 960 x 4 096 x 4 096 as the library's product and gated_residual_kernel
+// 741 us, with the sum in this epilogue 673, 32 760 rows 836 / 823; with a side branch of rank 128 in front of it as well 0.04 ms of a segment's 5.5.
 //
 // What bounds it: power, and the reading half of a phase.  Per k block and group 610 clocks to request 32 KB (the address unit of a
 // CU takes 16 a load of 1 KB, and a wavefront issues in order) and 500 to read 96 KB of fragments, against 1 009 of MFMAs, so the
@@ -66,7 +68,7 @@ typedef bf16x8 V8;
 
 constexpr int kMaxSlices = 8;
 
-enum Epilogue { kPlain, kResidual, kQkv, kLora };
+enum Epilogue { kPlain, kResidual, kGated, kQkv };
 
 struct GemmArgs {
     const __bf16* x; int64_t ldx;
@@ -83,6 +85,7 @@ struct GemmArgs {
     const float* tab;
     int Hn, S, Hg, Wg, t0, Ttab;
     float eps;
+    const float* gate; int gate_rows;      // out = residual + gate * (...): a row of N for every gate_rows tokens
     // a LoRA side branch: t [M, slices * rank], up [per, rank] for every `per` features
     const __bf16* t; int64_t ldt;
     const __bf16* up[kMaxSlices];
@@ -90,7 +93,8 @@ struct GemmArgs {
     float scale;
 };
 
-template <int kEpi>
+// kSide: with a LoRA side branch.
+template <int kEpi, bool kSide>
 __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) {
     constexpr bool QKV = kEpi == kQkv;
     extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -116,14 +120,14 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
     uint32_t pitch;
     int last_row;
     int next_t = t_first, left = 0;                   // tile that is being brought, k blocks of it that are not yet
-    const int side_blocks = kEpi == kLora ? a.rank / kBK : 0, nblocks = side_blocks + a.K / kBK;
-    bool side = kEpi == kLora;                        // a tile's blocks are those of its side branch, then those of the layer
+    const int side_blocks = kSide ? a.rank / kBK : 0, nblocks = side_blocks + a.K / kBK;
+    bool side = kSide;                                // a tile's blocks are those of its side branch, then those of the layer
     const uint32_t lds0 = lds_address(smem);
     auto start_part = [&]() __attribute__((always_inline)) {
         int tm, tf;
         place(next_t, tm, tf);
         last_row = group ? a.M - 1 - tm * kTileM : a.N - 1 - tf * kTileN;
-        if (kEpi == kLora && side) {
+        if (kSide && side) {
             const int f = tf * kTileN, slice = f / a.per;                     // slices are whole tiles
             from = group ? reinterpret_cast<const char*>(a.t + (int64_t)tm * kTileM * a.ldt + slice * a.rank) : reinterpret_cast<const char*>(a.up[slice] + (int64_t)(f - slice * a.per) * a.rank);
             pitch = (uint32_t)(group ? a.ldt : a.rank) * 2u;
@@ -147,12 +151,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
         }
         from += kBK * 2;
         if (--left == 0) {
-            if (kEpi == kLora && side) {
+            if (kSide && side) {
                 side = false;
                 start_part();
             } else {
                 next_t += per_xcd;
-                side = kEpi == kLora;
+                side = kSide;
                 if (next_t < t_end) start_part();
             }
         }
@@ -222,7 +226,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
                 for (int i = 0; i < 8; ++i)
 #pragma unroll
                     for (int j = 0; j < 4; ++j) acc[i][j] = mfma16(af[ks][i], bf[ks][j], acc[i][j]);
-            if constexpr (kEpi == kLora) {
+            if constexpr (kSide) {
                 if (kb + 1 == side_blocks && a.scale != 1.f) {
 #pragma unroll
                     for (int i = 0; i < 8; ++i)
@@ -325,7 +329,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
 #pragma unroll
         for (int jj = 0; jj < 4; jj += 2) {
             uint4 res[2][4];
-            if constexpr (kEpi == kResidual) {
+            if constexpr (kEpi == kResidual || kEpi == kGated) {
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     const __bf16* row = a.residual + (int64_t)min(m0 + 16 * (jj + j) + (int)lr, a.M - 1) * a.ldr + f0 + piece;
@@ -343,6 +347,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
                 } else {
                     to = a.out + (int64_t)tok * a.ldo + f0;
                 }
+                const float* gate = nullptr;
+                if constexpr (kEpi == kGated) gate = a.gate + (int64_t)((uint32_t)min(tok, a.M - 1) / (uint32_t)a.gate_rows) * a.N + f0 + 4 * lg;
                 uint4 o[4];
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
@@ -352,15 +358,17 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
                             v[h][e] = QKV ? acc[2 * p + h][j][e] : acc[2 * p + h][j][e] + (float)reinterpret_cast<const __bf16*>(&bias[2 * p + h])[e];
-                    if constexpr (kEpi == kResidual) {
+                    if constexpr (kEpi == kResidual || kEpi == kGated) {
                         const uint4 r = res[j - jj][p];
                         const auto lo = __builtin_amdgcn_permlane16_swap(r.x, r.z, false, false);
                         const auto hi = __builtin_amdgcn_permlane16_swap(r.y, r.w, false, false);
 #pragma unroll
                         for (int h = 0; h < 2; ++h) {
                             const uint32_t raw[2] = {lo[h], hi[h]};
+                            f32x4_ g = {1.f, 1.f, 1.f, 1.f};
+                            if constexpr (kEpi == kGated) g = *reinterpret_cast<const f32x4_*>(gate + 32 * p + 16 * h);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) v[h][e] += (float)reinterpret_cast<const __bf16*>(raw)[e];
+                            for (int e = 0; e < 4; ++e) v[h][e] = (float)reinterpret_cast<const __bf16*>(raw)[e] + (kEpi == kGated ? g[e] * v[h][e] : v[h][e]);
                         }
                     }
                     uint32_t w[2][2];
@@ -385,14 +393,14 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
 }
 
 
-template <int kEpi>
+template <int kEpi, bool kSide = false>
 int launch_gemm(GemmArgs& a, hipStream_t stream) {
     a.tiles_m = (a.M + kTileM - 1) / kTileM;
     a.tiles_n = (a.N + kTileN - 1) / kTileN;
     const int64_t tiles = (int64_t)a.tiles_m * a.tiles_n;
     const unsigned grid = (unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, kCus);
     const size_t lds = (size_t)kStages * kPart;
-    auto kernel = gemm_nt_kernel<kEpi>;
+    auto kernel = gemm_nt_kernel<kEpi, kSide>;
     // more than the 64 KB a kernel gets without asking; the attribute is per device, so it is set on every call
     const hipError_t ea = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (ea != hipSuccess) return set_error(BSA_ERR_HIP, "gemm: LDS size: %s", hipGetErrorString(ea));
@@ -421,18 +429,23 @@ int check_gemm_operands(const char* what, const void* x, int64_t ldx, const void
 // 384 columns 14.2 / 9.9 (1 000 rows) to 37.6 / 27.2 (86 400), K = 256 and 768 13.9 / 12.1 to 67 / 53; the library's host time is 14.
 // Rows must be those of whole 16-byte pieces, and out nowhere else than in a place of its own or the residual's: the
 // library's route has read x before it writes a result, this kernel has not.
-bool gemm_serves_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual, const void* out, int64_t ldo,
-                        int64_t M, int N, int K) {
+static bool gemm_takes(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual, const void* out, int64_t ldo,
+                       int64_t M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || K % kBK || N % 128 || ldx % 8 || ldw % 8 || ldo % 8 || ldx < K || ldw < K || ldo < N || ldx >= (1 << 22) || ldw >= (1 << 22)) return false;
     const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
     if (((at(x) | at(w) | at(out) | at(residual)) & 15u) || (at(bias) & 7u)) return false;
     const auto rows = [](int64_t n, int64_t pitch, int64_t width) { return (uintptr_t)((n - 1) * pitch + width) * 2u; };
     const uintptr_t o = at(out), o_end = o + rows(M, ldo, N);
     const auto meets = [&](const void* p, uintptr_t bytes) { return p != nullptr && at(p) < o_end && o < at(p) + bytes; };
-    if (meets(x, rows(M, ldx, K)) || meets(w, rows(N, ldw, K)) || meets(bias, (uintptr_t)N * 2u) || (residual != out && meets(residual, o_end - o))) return false;
-    if (K <= 256) return true;
+    return !(meets(x, rows(M, ldx, K)) || meets(w, rows(N, ldw, K)) || meets(bias, (uintptr_t)N * 2u) || (residual != out && meets(residual, o_end - o)));
+}
+static bool residual_serves(int64_t M, int N, int K) {
     const int64_t tiles = (M + kTileM - 1) / kTileM * ((N + kTileN - 1) / kTileN), round = (tiles + kCus - 1) / kCus * kCus;
-    return residual != nullptr && 5 * tiles >= 4 * round;
+    return K <= 256 || 5 * tiles >= 4 * round;
+}
+bool gemm_serves_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual, const void* out, int64_t ldo,
+                        int64_t M, int N, int K) {
+    return (K <= 256 || residual != nullptr) && residual_serves(M, N, K) && gemm_takes(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K);
 }
 
 // Which layers with a LoRA side branch run as one product, a rank of whole k blocks and slices of whole tiles: us, the library's product and
@@ -454,6 +467,18 @@ static bool lora_serves(const void* x, const void* w, const void* bias, const vo
         if (!up[i] || (at(up[i]) & 15u) || meets(up[i], (uintptr_t)(N / n_sep) * rank * 2u)) return false;
     const int64_t tiles = (M + kTileM - 1) / kTileM * (N / kTileN), round = (tiles + kCus - 1) / kCus * kCus;
     return K <= 512 || 4 * tiles >= (K <= 1024 ? 2 : 3) * round;
+}
+
+static GemmArgs layer_args(const void* x, const void* w, const void* bias, void* out, int64_t M, int N, int K) {
+    GemmArgs a = {};
+    a.x = (const __bf16*)x; a.ldx = K; a.w = (const __bf16*)w; a.ldw = K; a.bias = (const __bf16*)bias;
+    a.out = (__bf16*)out; a.ldo = N;
+    a.M = (int)M; a.N = N; a.K = K;
+    return a;
+}
+static void add_side(GemmArgs& a, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank, float scale) {
+    a.t = (const __bf16*)t; a.ldt = ldt; a.per = a.N / n_sep; a.rank = rank; a.scale = scale;
+    for (int i = 0; i < n_sep; ++i) a.up[i] = (const __bf16*)up[i];
 }
 
 }  // namespace bsa
@@ -485,13 +510,32 @@ int bsa_linear_lora_bf16(const void* x, const void* w, const void* bias, const v
         const int rc = bsa_linear_bf16(x, w, bias, nullptr, out, M, N, K, workspace, workspace_bytes, stream);
         return rc != BSA_OK ? rc : bsa_lora_up_add(out, t, ldt, up, n_sep, rank, multiplier, alpha_scale, out, M, N, stream);
     }
-    GemmArgs a = {};
-    a.x = (const __bf16*)x; a.ldx = K; a.w = (const __bf16*)w; a.ldw = K; a.bias = (const __bf16*)bias;
-    a.out = (__bf16*)out; a.ldo = N;
-    a.M = (int)M; a.N = N; a.K = K;
-    a.t = (const __bf16*)t; a.ldt = ldt; a.per = N / n_sep; a.rank = rank; a.scale = multiplier * alpha_scale;
-    for (int i = 0; i < n_sep; ++i) a.up[i] = (const __bf16*)up[i];
-    return launch_gemm<kLora>(a, (hipStream_t)stream);
+    GemmArgs a = layer_args(x, w, bias, out, M, N, K);
+    add_side(a, t, ldt, up, n_sep, rank, multiplier * alpha_scale);
+    return launch_gemm<kPlain, true>(a, (hipStream_t)stream);
+}
+
+int bsa_linear_gated_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
+                          float multiplier, float alpha_scale, const void* residual, const float* gate, int rows_per_group, void* out,
+                          int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!x || !w || (t && !up) || !residual || !gate || !out) return set_error(BSA_ERR_BAD_ARG, "linear_gated: null pointer");
+    if (M <= 0 || N <= 0 || K <= 0) return set_error(BSA_ERR_BAD_ARG, "linear_gated: sizes must be positive");
+    if (rows_per_group <= 0 || M % rows_per_group != 0)
+        return set_error(BSA_ERR_SHAPE, "linear_gated: %lld rows do not split into groups of %d", (long long)M, rows_per_group);
+    if (out == residual) return set_error(BSA_ERR_BAD_ARG, "linear_gated: out must be memory of its own");
+    const uintptr_t o = reinterpret_cast<uintptr_t>(out), g = reinterpret_cast<uintptr_t>(gate);
+    const bool over_gate = g < o + (uintptr_t)M * N * 2u && o < g + (uintptr_t)(M / rows_per_group) * N * sizeof(float);
+    if (!(g & 15u) && !over_gate && gemm_takes(x, K, w, K, bias, residual, out, N, M, N, K) &&
+        (t ? lora_serves(x, w, bias, t, ldt, up, n_sep, rank, out, M, N, K) : residual_serves(M, N, K))) {
+        GemmArgs a = layer_args(x, w, bias, out, M, N, K);
+        a.residual = (const __bf16*)residual; a.ldr = N; a.gate = gate; a.gate_rows = rows_per_group;
+        if (!t) return launch_gemm<kGated>(a, (hipStream_t)stream);
+        add_side(a, t, ldt, up, n_sep, rank, multiplier * alpha_scale);
+        return launch_gemm<kGated, true>(a, (hipStream_t)stream);
+    }
+    const int rc = t ? bsa_linear_lora_bf16(x, w, bias, t, ldt, up, n_sep, rank, multiplier, alpha_scale, out, M, N, K, workspace, workspace_bytes, stream)
+                     : bsa_linear_bf16(x, w, bias, nullptr, out, M, N, K, workspace, workspace_bytes, stream);
+    return rc != BSA_OK ? rc : bsa_gated_residual(residual, out, gate, out, M, rows_per_group, N, BSA_BF16, stream);
 }
 
 int bsa_qkv_projection(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* q_weight,

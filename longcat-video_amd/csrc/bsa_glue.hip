@@ -151,8 +151,8 @@ __global__ __launch_bounds__(256, kPieces <= 8 ? 4 : 2) void layernorm_modulate_
 
 // out = T(float(x) + gate * float(y)), gate fp32 per group of rows (one latent frame).
 template <typename T>
-__global__ __launch_bounds__(256) void gated_residual_kernel(const T* __restrict__ x, const T* __restrict__ y,
-                                                             const float* __restrict__ gate, T* __restrict__ out,
+__global__ __launch_bounds__(256) void gated_residual_kernel(const T* __restrict__ x, const T* y,      // y may be out
+                                                             const float* __restrict__ gate, T* out,
                                                              int64_t rows, int rows_per_group, int dim) {
     // the launch is limited to 2^31 threads: 32-bit divisions (64-bit ones cost more than the 48 bytes moved)
     const uint32_t per_row = (uint32_t)dim / 8;

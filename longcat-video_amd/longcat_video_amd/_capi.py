@@ -91,6 +91,7 @@ SIGNATURES = {
     "bsa_linear_bf16_tune": (_i, [_p, _i64, _p, _i64, _p, _p, _p, _i64, _i64, _i, _i, _p, C.c_size_t, _p, _p, _p]),
     "bsa_lora_add": (_i, [_p, _p, _p, _p, _i, _p, _i64, _i, _p]),
     "bsa_linear_lora_bf16": (_i, [_p, _p, _p, _p, _i64, _p, _i, _i, _f, _f, _p, _i64, _i, _i, _p, C.c_size_t, _p]),
+    "bsa_linear_gated_bf16": (_i, [_p, _p, _p, _p, _i64, _p, _i, _i, _f, _f, _p, _p, _i, _p, _i64, _i, _i, _p, C.c_size_t, _p]),
     "bsa_lora_up_add": (_i, [_p, _p, _i64, _p, _i, _i, _f, _f, _p, _i64, _i, _p]),
     "bsa_gemm_bf16": (_i, [_p, _i64, _p, _i64, _p, _p, _i64, _p, _i64, _i64, _i, _i, _p]),
     "bsa_qkv_projection": (_i, [_p, _i64, _p, _i64, _p, _p, _p, _p, _p, _p, _p, _strides] + [_i] * 9 + [_f, _p]),

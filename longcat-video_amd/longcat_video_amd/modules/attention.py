@@ -135,6 +135,28 @@ def linear_bf16(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     return out if out.shape == shape else out.view(shape)
 
 
+def linear_gated(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], residual: torch.Tensor, gate: torch.Tensor,
+                 workspace: Optional[torch.Tensor] = None, side=(None, 0, None, 0, 0, 0.0, 0.0)) -> torch.Tensor:
+    """``gated_residual(residual, gate, x @ weight.T + bias)`` in one call; side: a LoRA branch, as bsa_linear_gated_bf16 takes it."""
+    if not x.is_cuda:
+        raise RuntimeError("the engine runs on the GPU only")
+    if x.dtype != torch.bfloat16 or residual.dtype != torch.bfloat16:
+        raise NotImplementedError("linear: only bf16 is built")
+    K, N = x.shape[-1], weight.shape[0]
+    gate, per = _frames(residual, gate, "gate")
+    assert weight.shape[1] == K and residual.shape[-1] == N and residual.numel() // N == x.numel() // K
+    x2 = x if x.is_contiguous() else x.reshape(-1, K).contiguous()
+    M = x2.numel() // K
+    w, b, r = _bf16(weight), None if bias is None else _bf16(bias), residual.contiguous()
+    out = torch.empty(residual.shape, dtype=torch.bfloat16, device=x.device)
+    if workspace is None:
+        workspace = _gemm_workspace(x.device)
+    with _on_device(x):
+        _capi.check(_capi.load().bsa_linear_gated_bf16(_ptr(x2), _ptr(w), _ptr(b), *side, _ptr(r), _ptr(gate), per, _ptr(out), M, N, K,
+                                                       _ptr(workspace), workspace.numel(), _stream(x)), "linear with a gate")
+    return out
+
+
 def tune_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], residual: bool = False,
                 workspace: Optional[torch.Tensor] = None):
     """One-time choice of the GEMM algorithm for ``linear_bf16`` calls of this shape (rows of x, weight shape, bias and
@@ -325,12 +347,20 @@ class Attention(nn.Module):
         # epilogue) and bsa_gemm_bf16.  Both round at the same points.
         self.projection_backend = "hipblaslt"
 
-    def _linear(self, x, layer, loras, residual=None):
+    def _linear(self, x, layer, loras, residual=None, gate=None):
+        engine = self.projection_backend == "engine" and layer.weight.shape[0] % 128 == 0 and layer.weight.shape[1] % 64 == 0
+        if gate is not None:                              # residual + gate * the layer
+            if any(b.use_lora for b in loras):
+                from .lora import lora_linear
+                return lora_linear(x, layer.weight, layer.bias, loras, residual=residual, gate=gate)
+            if engine:
+                return gated_residual(residual, gate, gemm_bf16(x, layer.weight, layer.bias))
+            return linear_gated(x, layer.weight, layer.bias, residual, gate)
         if any(b.use_lora for b in loras):
             from .lora import lora_linear
             y = lora_linear(x, layer.weight, layer.bias, loras)
             return y if residual is None else y + residual
-        if self.projection_backend == "engine" and layer.weight.shape[0] % 128 == 0 and layer.weight.shape[1] % 64 == 0:
+        if engine:
             return gemm_bf16(x, layer.weight, layer.bias, residual=residual)
         return linear_bf16(x, layer.weight, layer.bias, residual=residual)
 
@@ -387,8 +417,9 @@ class Attention(nn.Module):
 
     @torch.no_grad()
     def forward(self, x: torch.Tensor, shape=None, num_cond_latents=None, return_kv=False,
-                residual: Optional[torch.Tensor] = None):
-        """attention.py:107-147.  `residual` (extension): added to the fp32 projection, one rounding."""
+                residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None):
+        """attention.py:107-147.  `residual` (extension): added to the fp32 projection, one rounding; with `gate`, fp32 [B, T, 1, C]:
+        residual + gate * the projection."""
         B, N, C = x.shape
         Hn, D = self.num_heads, self.head_dim
         eps = self.q_norm.eps
@@ -413,7 +444,7 @@ class Attention(nn.Module):
                 self._process_attn(qs[:, :, n:], ks, vs, shape, out=ov[:, :, n:], qk_norm=norm(num_cond_latents), kv_out=kv_out)   # attention.py:132-133
             else:
                 self._process_attn(qs, ks, vs, shape, out=ov, qk_norm=norm(0), kv_out=kv_out)
-            y = self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual=residual)
+            y = self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
             return (y, kv_out) if return_kv else y
         else:
             # q moves into a per-head tensor on the way (the attention kernel fetches its rows tile by tile); k is
@@ -435,14 +466,14 @@ class Attention(nn.Module):
             self._process_attn(q[:, :, n:], k, v, shape, out=ov[:, :, n:])                       # attention.py:132-133
         else:
             self._process_attn(q, k, v, shape, out=ov)
-        y = self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual=residual)
+        y = self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
         if return_kv:
             return y, (k_cache, v.contiguous())
         return y
 
     @torch.no_grad()
     def forward_with_kv_cache(self, x: torch.Tensor, shape=None, num_cond_latents=None, kv_cache=None,
-                              residual: Optional[torch.Tensor] = None) -> torch.Tensor:
+                              residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
         """attention.py:149-181: the new tokens attend to the cached conditioning keys/values followed by
         their own.  The cache holds keys after the norm and before the rotation; cached and new keys are
         rotated together on a grid of T + num_cond_latents frames, the queries sit at its last T frames."""
@@ -468,7 +499,7 @@ class Attention(nn.Module):
             tab = rope_table(grid_full, D, x.device)
             self._process_attn(qs, ks, vs, shape, out=o.permute(0, 2, 1, 3), kv_cache=(kc, vc, int(num_cond_latents)),
                                qk_norm=(self.q_norm.weight, self.k_norm.weight, tab, T + num_cond_latents, num_cond_latents, 0, eps))
-            return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual=residual)
+            return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
         k_full = torch.empty(B, Hn, n_c + N, D, dtype=x.dtype, device=x.device)
         v_full = torch.empty_like(k_full)
         kc = k_cache.to(x.device).expand(B, -1, -1, -1)                            # attention.py:162-164
@@ -482,7 +513,7 @@ class Attention(nn.Module):
                       t_offset=num_cond_latents, table_grid=grid_full)
         o = torch.empty(B, N, Hn, D, dtype=x.dtype, device=x.device)
         self._process_attn(q, k_full, v_full, shape, out=o.permute(0, 2, 1, 3))
-        return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual=residual)
+        return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
 
 
 @torch.no_grad()
@@ -551,6 +582,14 @@ def dit_self_attention_branch(x: torch.Tensor, shift_msa: torch.Tensor, scale_ms
     small fp32 linear layer outside this path)."""
     x_m = layernorm_modulate(x, shift_msa, scale_msa)
     new_cache = None
+    # the gate and the sum inside the output projection, where nothing between the two can look at what it gives
+    if (type(attn) is Attention and x.dtype == torch.bfloat16 and not attn._forward_hooks and not attn._forward_pre_hooks
+            and not torch.nn.modules.module._has_any_global_hook() and not {"forward", "forward_with_kv_cache", "_linear"} & attn.__dict__.keys()):
+        inside = dict(shape=latent_shape, num_cond_latents=num_cond_latents, residual=x, gate=gate_msa)
+        if kv_cache is not None:
+            out = attn.forward_with_kv_cache(x_m, kv_cache=kv_cache, **inside)
+            return (out, None) if return_kv else out
+        return attn(x_m, return_kv=return_kv, **inside)
     if kv_cache is not None:
         x_s = attn.forward_with_kv_cache(x_m, shape=latent_shape, num_cond_latents=num_cond_latents, kv_cache=kv_cache)
     elif return_kv:

@@ -15,7 +15,7 @@ from typing import List, Optional, Sequence
 import torch
 
 from .. import _capi
-from .attention import _bf16, _gemm_workspace, _on_device, _ptr, _stream, linear_bf16
+from .attention import _bf16, _gemm_workspace, _on_device, _ptr, _stream, gated_residual, linear_bf16, linear_gated
 
 MAX_BRANCHES = 4
 
@@ -75,8 +75,8 @@ def _one_pass(b: LoRABranch) -> bool:
             and all(u.dtype == torch.bfloat16 and (not u.is_contiguous() or u.data_ptr() % 16 == 0) for u in b.lora_up))
 
 
-def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace) -> torch.Tensor:
-    """The down projection, then the layer with its side branch."""
+def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace, residual, gate) -> torch.Tensor:
+    """The down projection, then the layer with its side branch, and with a gate residual + gate * that."""
     M, K, N = x2.shape[0], x2.shape[1], weight.shape[0]
     assert weight.shape[1] == K and b.out_features == N and b.lora_down.shape[1] == K
     if b.lora_down.dtype != torch.bfloat16:
@@ -86,19 +86,24 @@ def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace
     w, bw = _bf16(weight), None if bias is None else _bf16(bias)
     ups = [u.contiguous() for u in b.lora_up]
     ptrs = (C.c_void_p * len(ups))(*[u.data_ptr() for u in ups])
+    side = (_ptr(lx), lx.shape[1], ptrs, len(ups), b.rank, float(b.multiplier), alpha)
+    if gate is not None:
+        return linear_gated(x2, w, bw, residual, gate, workspace, side)
     out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
     with _on_device(x):
-        _capi.check(_capi.load().bsa_linear_lora_bf16(_ptr(x2), _ptr(w), _ptr(bw), _ptr(lx), lx.shape[1], ptrs, len(ups), b.rank,
-                                                      float(b.multiplier), alpha, _ptr(out), M, N, K, _ptr(workspace),
+        _capi.check(_capi.load().bsa_linear_lora_bf16(_ptr(x2), _ptr(w), _ptr(bw), *side, _ptr(out), M, N, K, _ptr(workspace),
                                                       workspace.numel(), _stream(x)), "linear with a LoRA branch")
     return out
 
 
 @torch.no_grad()
 def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
-                loras: Optional[List[LoRABranch]] = None, workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """The patched forward of longcat_video_dit.py:234-249 for a bf16 Linear."""
+                loras: Optional[List[LoRABranch]] = None, workspace: Optional[torch.Tensor] = None,
+                residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The patched forward of longcat_video_dit.py:234-249 for a bf16 Linear; with a gate, residual + gate * that, as gated_residual."""
     active = [b for b in (loras or []) if b.use_lora]
+    if gate is not None and not (len(active) == 1 and _one_pass(active[0])):
+        return gated_residual(residual, gate, lora_linear(x, weight, bias, loras, workspace))
     if not active:
         return linear_bf16(x, weight, bias, workspace=workspace)                    # `org_output + 0`
     if len(active) > MAX_BRANCHES:
@@ -112,7 +117,7 @@ def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     # alpha_scale lives in a bf16 buffer in the reference
     alphas = [float(torch.tensor(b.alpha_scale, dtype=torch.bfloat16)) for b in active]
     if len(active) == 1 and _one_pass(active[0]):
-        return _with_one_branch(x, x2, weight, bias, active[0], alphas[0], workspace)
+        return _with_one_branch(x, x2, weight, bias, active[0], alphas[0], workspace, residual, gate)
     org = linear_bf16(x, weight, bias, workspace=workspace)
     ups = []
     for b, a in zip(active, alphas):

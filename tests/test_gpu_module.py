@@ -392,6 +392,48 @@ def test_layer_with_lora_branch_in_one_product(M, K, r, n_sep, per, scale):
     assert torch.equal(L().lora_linear(x, w, None, [br]), (x.float() @ w.float().T + scale * up).bfloat16())
 
 
+@pytest.mark.parametrize("lora", [False, True])
+@pytest.mark.parametrize("frames,per,K,N,one_rounding", [
+    ((2, 3), 750, 576, 3072, True),           # frames and prompts that end within a tile and within a wavefront's tokens
+    ((1, 4481), 1, 576, 3072, True), ((1, 1), 4481, 1024, 3072, True),
+    ((1, 5), 1, 128, 256, True),              # a short K is served whatever the tiles
+    ((1, 5), 3, 1088, 256, False), ((3, 4), 100, 1088, 512, False),
+])
+def test_layer_behind_a_gate(frames, per, K, N, one_rounding, lora):
+    """residual + gate * layer in one product: small integers and gates of quarters, exact up to the last rounding, and where the GEMM
+    does not serve it up to that of the layer's output."""
+    g = torch.Generator(device="cuda").manual_seed(K + per)
+    ints = lambda lo, hi, *s: torch.randint(lo, hi, s, generator=g, device="cuda").bfloat16()      # noqa: E731
+    (B, T), r = frames, 128
+    x, w, b, res = ints(-2, 3, B, T * per, K), ints(-2, 3, N, K), ints(-2, 3, N), ints(-99, 100, B, T * per, N)
+    gate = torch.randint(-9, 10, (B, T, 1, N), generator=g, device="cuda").float() / 4
+    y = x.float() @ w.float().T + b.float()
+    if lora:
+        br = L().LoRABranch(ints(-1, 2, r, K), [ints(-1, 2, N, r)], 0.5, r)
+        up = 0.5 * ((x.float() @ br.lora_down.float().T).bfloat16().float() @ br.lora_up[0].float().T)
+        y = y + up if one_rounding else y.bfloat16().float() + (up * 2).bfloat16().float() / 2
+    if not one_rounding:
+        y = y.bfloat16().float()
+    want = (res.float().view(B, T, per, N) + gate * y.view(B, T, per, N)).view(B, T * per, N).bfloat16()
+    got = L().lora_linear(x, w, b, [br], residual=res, gate=gate) if lora else M().linear_gated(x, w, b, res, gate)
+    assert torch.equal(got, want)
+
+
+def test_a_hook_sees_the_attention_without_its_gate():
+    m = make_module(sparsity=0.5, seed=15).cuda()
+    g = torch.Generator(device="cuda").manual_seed(16)
+    x = torch.randn(1, 256, 512, generator=g, device="cuda").bfloat16()
+    shift, scale, gate = torch.randn(3, 1, 4, 1, 512, generator=g, device="cuda").unbind(0)
+    plain = M().dit_self_attention_branch(x, shift, scale, gate, m, (4, 8, 8))
+    seen = []
+    hook = m.register_forward_hook(lambda mod, args, out: seen.append(out))
+    hooked = M().dit_self_attention_branch(x, shift, scale, gate, m, (4, 8, 8))
+    hook.remove()
+    assert len(seen) == 1 and torch.equal(hooked, M().gated_residual(x, gate, seen[0]))
+    bound = 2 * BF16_ULP * (hooked.float().abs() + (gate * seen[0].float().view(1, 4, 64, 512)).abs().view(1, 256, 512))      # two roundings for one
+    assert torch.all((plain.float() - hooked.float()).abs() <= bound)
+
+
 def test_module_forward_with_lora_branches():
     """longcat_video_dit.py:211-249: LoRA branches on attn.qkv (up-projection split in three) and attn.proj."""
     shape = (4, 8, 8)
