@@ -17,7 +17,59 @@ namespace bsa {
 namespace {
 
 // ------------------------------------------------------------- row RMSNorm
-// out = bf16(x * rsqrt(mean(x^2) + eps)) * w, one wavefront per row.
+constexpr int kRmsRows = 2;                      // rows of a wavefront
+// out = bf16(x * rsqrt(mean(x^2) + eps)) * w.  HBM-bound: a wavefront holds a row and the weights in registers, and its next row
+// is on its way.  For long rows and enough of them to fill the chip eight to a workgroup, us, the kernel below / this one: 86 400 x 4 096 304 / 269
+// (5.3 TB/s), 24 960 x 4 096 99 / 85, 8 000 x 8 192 75 / 61, 40 000 x 2 048 73 / 64; 4 000 x 4 096 15.3 / 16.5, 86 400 x 1 024 63 / 64.  One row
+// a wavefront 308, four 271, eight 280 of the first.
+template <typename T, int kPieces>        // 16-byte pieces of a row per lane: dim <= 512 kPieces
+__global__ __launch_bounds__(256) void rmsnorm_held_kernel(const T* __restrict__ x, const T* __restrict__ w,
+                                                           T* __restrict__ out, int64_t rows, int dim, float eps) {
+    const int lane = threadIdx.x & 63;
+    int64_t row = (int64_t)blockIdx.x * (4 * kRmsRows) + (threadIdx.x >> 6);
+    const int64_t end = min(rows, ((int64_t)blockIdx.x + 1) * (4 * kRmsRows));
+    uint4 raw[kPieces], ahead[kPieces], wraw[kPieces];
+    auto request = [&](int64_t r) {
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            if (j * 512 + lane * 8 < dim) ahead[j] = *reinterpret_cast<const uint4*>(x + r * dim + j * 512 + lane * 8);
+    };
+    if (row < end) request(row);
+#pragma unroll
+    for (int j = 0; j < kPieces; ++j)
+        if (j * 512 + lane * 8 < dim) wraw[j] = *reinterpret_cast<const uint4*>(w + j * 512 + lane * 8);
+    for (; row < end; row += 4) {
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j) raw[j] = ahead[j];
+        if (row + 4 < end) request(row + 4);
+        float ss = 0.f;
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            if (j * 512 + lane * 8 < dim) {
+                const T* e = reinterpret_cast<const T*>(&raw[j]);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) { const float f = (float)e[i]; ss = fmaf(f, f, ss); }
+            }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+        const float r = rsqrtf(ss / (float)dim + eps);
+        // widened again: kept in fp32 over the sum, a row of 4 096 would take 64 registers more
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j) asm volatile("" : "+v"(raw[j].x), "+v"(raw[j].y), "+v"(raw[j].z), "+v"(raw[j].w));
+#pragma unroll
+        for (int j = 0; j < kPieces; ++j)
+            if (j * 512 + lane * 8 < dim) {
+                const T* e = reinterpret_cast<const T*>(&raw[j]);
+                const T* we = reinterpret_cast<const T*>(&wraw[j]);
+                T res[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) res[i] = (T)((float)(T)((float)e[i] * r) * (float)we[i]);
+                *reinterpret_cast<uint4*>(out + row * dim + j * 512 + lane * 8) = *reinterpret_cast<const uint4*>(res);
+            }
+    }
+}
+
+// The same for few rows, and rows of any length: one wavefront per row, which it asks for twice.
 template <typename T>
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                            T* __restrict__ out, int64_t rows, int dim, float eps) {
@@ -379,12 +431,24 @@ int bsa_rmsnorm(const void* x, const void* weight, void* out, int64_t rows, int 
     if (!(eps >= 0.f)) return set_error(BSA_ERR_BAD_ARG, "rmsnorm: eps must be non-negative");
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(out)) & 15u)
         return set_error(BSA_ERR_BAD_ARG, "rmsnorm: pointers must be 16-byte aligned");
-    const dim3 grid((unsigned)((rows + 3) / 4)), block(256);
-    if (dtype == BSA_BF16)
-        hipLaunchKernelGGL((rmsnorm_rows_kernel<__bf16>), grid, block, 0, (hipStream_t)stream, (const __bf16*)x, (const __bf16*)weight, (__bf16*)out, rows, dim, eps);
-    else if (dtype == BSA_F16)
-        hipLaunchKernelGGL((rmsnorm_rows_kernel<_Float16>), grid, block, 0, (hipStream_t)stream, (const _Float16*)x, (const _Float16*)weight, (_Float16*)out, rows, dim, eps);
+    const bool held = dim > 1024 && dim <= 8192 && rows >= 8000;
+    const int64_t per_wg = held ? 4 * kRmsRows : 4;
+    const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg)), block(256);
+#define BSA_RMS_(T, KERNEL) hipLaunchKernelGGL((KERNEL), grid, block, 0, (hipStream_t)stream, (const T*)x, (const T*)weight, (T*)out, rows, dim, eps)
+#define BSA_HELD(T, N) rmsnorm_held_kernel<T, N>
+#define BSA_RMS(T)                                                 \
+    do {                                                           \
+        if (!held) BSA_RMS_(T, rmsnorm_rows_kernel<T>);            \
+        else if (dim <= 2048) BSA_RMS_(T, BSA_HELD(T, 4));         \
+        else if (dim <= 4096) BSA_RMS_(T, BSA_HELD(T, 8));         \
+        else BSA_RMS_(T, BSA_HELD(T, 16));                         \
+    } while (0)
+    if (dtype == BSA_BF16) BSA_RMS(__bf16);
+    else if (dtype == BSA_F16) BSA_RMS(_Float16);
     else
+#undef BSA_RMS
+#undef BSA_HELD
+#undef BSA_RMS_
         return set_error(BSA_ERR_UNSUPPORTED, "rmsnorm: dtype %d is not built (bf16, fp16)", dtype);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? BSA_OK : set_error(BSA_ERR_HIP, "rmsnorm launch: %s", hipGetErrorString(e));

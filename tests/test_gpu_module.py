@@ -50,6 +50,20 @@ def test_row_rmsnorm():
     assert (got.float() - want.float()).abs().mean() < 1e-3
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,dim", [(8000, 1032), (8001, 2048), (8007, 2056), (8004, 4096), (8003, 4104), (8001, 8192), (8000, 8200)])
+def test_row_rmsnorm_of_many_rows(rows, dim, dtype):
+    """Many long rows go to a kernel that holds them; the sums run in the same order as for few rows: the same bits, last rows included."""
+    g = torch.Generator(device="cuda").manual_seed(rows + dim)
+    x = (torch.randn(rows, dim, generator=g, device="cuda") * 3).to(dtype)
+    w = (1 + 0.2 * torch.randn(dim, generator=g, device="cuda")).to(dtype)
+    got, few = M().rms_norm(x, w, 1e-6), M().rms_norm(x[-3000:].contiguous(), w, 1e-6)
+    assert torch.equal(got[-3000:], few)
+    want = (x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6)).to(dtype).double() * w.double()
+    ulp = BF16_ULP if dtype is torch.bfloat16 else 2.0 ** -10
+    assert torch.all((got.double() - want).abs() <= want.abs() * 2 * ulp + 1e-6)
+
+
 def test_linear_with_bias_and_residual():
     g = torch.Generator().manual_seed(2)
     x = torch.randn(2, 100, 512, generator=g).bfloat16()
