@@ -37,8 +37,9 @@
 //
 // A LoRA side branch is more of the same sum: a tile's first k blocks are those of the rank axis (t . up^T, scaled where they end), for a pass
 // that reads and writes the layer's output at 4 TB/s.  Its two blocks of 66 cost 3 % of the product (128 multiplications a lane included).
-// A gated residual is added in the epilogue, for the same reason: 24 960 x 4 096 x 4 096 as the library's product and gated_residual_kernel
-// 741 us, with the sum in this epilogue 673, 32 760 rows 836 / 823; with a side branch of rank 128 in front of it as well 0.04 ms of a segment's 5.5.
+// A gated residual is added in the epilogue, for the same reason and by the rule of a residual: the library's product and gated_residual_kernel /
+// this, us, 28 618 x 4 096 x 4 096 (rounds full) 734 / 734, 44 969 x 2 304 x 2 304 (0.88) 505 / 432, 25 128 x 1 280 (0.97) 112 / 81, 0.72
+// full 5 795 x 3 968 168 / 172, K = 256 13.6 / 16.4 (506 rows, a launch less) to 26 / 21 (45 731).
 //
 // What bounds it: power, and the reading half of a phase.  Per k block and group 610 clocks to request 32 KB (the address unit of a
 // CU takes 16 a load of 1 KB, and a wavefront issues in order) and 500 to read 96 KB of fragments, against 1 009 of MFMAs, so the
@@ -452,8 +453,9 @@ bool gemm_serves_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, 
 // lora_up_add_kernel / this kernel.  Rank 128, tiles that fill their rounds: 32 760 x 12 288 x 4 096 2 471 / 2 386 (the library alone 2 115), x 4 096 x 4 096
 // 834 / 809, 86 400 x 4 096 x 4 096 2 276 / 2 192, 20 000 x 3 072 x 1 024 170 / 127.  Three quarters full 2 000 x 12 288 x 4 096 187 / 173, 0.73
 // 12 000 x 2 048 x 2 048 105 / 94, two thirds 1 560 x 12 288 x 4 096 152 / 169, 0.56 9 000 x 2 048 x 2 048 89 / 90.  A short K has less to lose: K = 1 024
-// 0.54 full 17 500 x 1 024 67 / 56, 3 000 x 3 072 45 / 29, a quarter full 4 000 x 1 024 24 / 27; K = 512 0.16 full 20.2 / 19.0, 0.09 level, K = 256 400 x 768
-// 16.5 / 12.9, 30 000 x 256 32 / 17.  Pointers and rows as above.
+// 0.54 full 17 500 x 1 024 67 / 56, 3 000 x 3 072 45 / 29, a quarter full 4 000 x 1 024 24 / 27; K = 768 a third full 28 / 24, 0.07 12.9 / 22.5; K = 256
+// 17.3 / 14.3 (506 x 256) to 33 / 17 (39 401).  With a gated residual as well, K = 256 19.4 / 19.1 to 41 / 23, 0.34 full 33 / 30, 0.84 27 580 x 2 048
+// 287 / 235, 1.00 28 618 x 4 096 856 / 765.  Pointers and rows as above.
 static bool lora_serves(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
                         const void* out, int64_t M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || n_sep <= 0 || n_sep > kMaxSlices || rank <= 0 || rank % kBK || rank > 128) return false;
@@ -466,7 +468,7 @@ static bool lora_serves(const void* x, const void* w, const void* bias, const vo
     for (int i = 0; i < n_sep; ++i)
         if (!up[i] || (at(up[i]) & 15u) || meets(up[i], (uintptr_t)(N / n_sep) * rank * 2u)) return false;
     const int64_t tiles = (M + kTileM - 1) / kTileM * (N / kTileN), round = (tiles + kCus - 1) / kCus * kCus;
-    return K <= 512 || 4 * tiles >= (K <= 1024 ? 2 : 3) * round;
+    return K <= 256 || (K <= 1024 ? 5 * tiles >= 2 * round : 4 * tiles >= 3 * round);
 }
 
 static GemmArgs layer_args(const void* x, const void* w, const void* bias, void* out, int64_t M, int N, int K) {

@@ -347,18 +347,18 @@ class Attention(nn.Module):
         # epilogue) and bsa_gemm_bf16.  Both round at the same points.
         self.projection_backend = "hipblaslt"
 
-    def _linear(self, x, layer, loras, residual=None, gate=None):
+    def _linear(self, x, layer, loras, residual=None, gate=None, one_rounding=True):
         engine = self.projection_backend == "engine" and layer.weight.shape[0] % 128 == 0 and layer.weight.shape[1] % 64 == 0
         if gate is not None:                              # residual + gate * the layer
             if any(b.use_lora for b in loras):
                 from .lora import lora_linear
-                return lora_linear(x, layer.weight, layer.bias, loras, residual=residual, gate=gate)
+                return lora_linear(x, layer.weight, layer.bias, loras, None, one_rounding, residual, gate)
             if engine:
                 return gated_residual(residual, gate, gemm_bf16(x, layer.weight, layer.bias))
             return linear_gated(x, layer.weight, layer.bias, residual, gate)
         if any(b.use_lora for b in loras):
             from .lora import lora_linear
-            y = lora_linear(x, layer.weight, layer.bias, loras)
+            y = lora_linear(x, layer.weight, layer.bias, loras, None, one_rounding)
             return y if residual is None else y + residual
         if engine:
             return gemm_bf16(x, layer.weight, layer.bias, residual=residual)
@@ -412,7 +412,8 @@ class Attention(nn.Module):
 
     def _project_qkv(self, x):
         B, N, C = x.shape
-        qkv = self._linear(x, self.qkv, self.qkv_loras)                           # [B, N, 3C]
+        # q and k choose the blocks: rounded once, with a side branch inside the product, near ties would fall differently than eager
+        qkv = self._linear(x, self.qkv, self.qkv_loras, one_rounding=False)       # [B, N, 3C]
         return qkv.view(B, N, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4).unbind(0)   # strided [B,H,N,D] views
 
     @torch.no_grad()

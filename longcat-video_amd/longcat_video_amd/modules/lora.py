@@ -3,9 +3,9 @@
 The reference patches the forward of every Linear a LoRA file names (longcat_video_dit.py:211-249):
 ``org_forward(x) + sum_i lora_up_i(lora_down_i(x)) * multiplier_i * alpha_scale_i``.  ``lora_up`` is either one
 Linear or, for fused projections such as qkv, one Linear per equal slice of the output features, each fed its own
-slice of the rank axis (lora_utils.py:12-21, 47-53).  Here the down projection goes to hipBLASLt through the C ABI; the layer with
-a single branch is one call (bsa_linear_lora_bf16): one product of the engine's GEMM, in fp32 up to its one rounding, or the layer by
-hipBLASLt and one pass over its output with the eager expression's roundings.  Several branches, whose scaled terms are summed before the
+slice of the rank axis (lora_utils.py:12-21, 47-53).  Here the layer and the down projection go to hipBLASLt through the C ABI; the
+up-projection of a single branch, its scaling and the sum are one pass over the layer's output (bsa_lora_up_add), or, where the caller
+takes one rounding for the eager expression's, a part of the layer's product (bsa_linear_lora_bf16, bsa_linear_gated_bf16).  Several branches, whose scaled terms are summed before the
 layer's output is added, take their up-projections from hipBLASLt too (the sliced one with row strides, in place) and one
 elementwise pass, with the eager roundings.
 """
@@ -68,14 +68,14 @@ def _up_projection(lx: torch.Tensor, branch: LoRABranch, workspace: torch.Tensor
 
 
 def _one_pass(b: LoRABranch) -> bool:
-    """What bsa_linear_lora_bf16 is built for, and faster at from 1 to 32 760 tokens, rank 16 to 128 and 64 to 12 288 columns (figures at the
-    kernels); other branches, and sums over several, take the up-projection as a tensor."""
+    """What bsa_lora_up_add is built for, and faster at from 1 to 32 760 tokens, rank 16 to 128 and 64 to 12 288 columns (figures at the
+    kernel); other branches, and sums over several, take the up-projection as a tensor."""
     per = b.lora_up[0].shape[0]
     return (b.rank % 16 == 0 and b.rank <= 128 and len(b.lora_up) <= 8 and per % 64 == 0
             and all(u.dtype == torch.bfloat16 and (not u.is_contiguous() or u.data_ptr() % 16 == 0) for u in b.lora_up))
 
 
-def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace, residual, gate) -> torch.Tensor:
+def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace, one_rounding, residual, gate) -> torch.Tensor:
     """The down projection, then the layer with its side branch, and with a gate residual + gate * that."""
     M, K, N = x2.shape[0], x2.shape[1], weight.shape[0]
     assert weight.shape[1] == K and b.out_features == N and b.lora_down.shape[1] == K
@@ -89,6 +89,11 @@ def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace
     side = (_ptr(lx), lx.shape[1], ptrs, len(ups), b.rank, float(b.multiplier), alpha)
     if gate is not None:
         return linear_gated(x2, w, bw, residual, gate, workspace, side)
+    if not one_rounding:
+        out = linear_bf16(x, weight, bias, workspace=workspace)
+        with _on_device(x):
+            _capi.check(_capi.load().bsa_lora_up_add(_ptr(out), *side, _ptr(out), M, N, _stream(x)), "lora_up_add")
+        return out
     out = torch.empty(*x.shape[:-1], N, dtype=torch.bfloat16, device=x.device)
     with _on_device(x):
         _capi.check(_capi.load().bsa_linear_lora_bf16(_ptr(x2), _ptr(w), _ptr(bw), *side, _ptr(out), M, N, K, _ptr(workspace),
@@ -99,11 +104,12 @@ def _with_one_branch(x, x2, weight, bias, b: LoRABranch, alpha: float, workspace
 @torch.no_grad()
 def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor],
                 loras: Optional[List[LoRABranch]] = None, workspace: Optional[torch.Tensor] = None,
-                residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """The patched forward of longcat_video_dit.py:234-249 for a bf16 Linear; with a gate, residual + gate * that, as gated_residual."""
+                one_rounding: bool = False, residual: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The patched forward of longcat_video_dit.py:234-249 for a bf16 Linear, with the eager expression's roundings; one_rounding: a
+    single branch may go into the layer's sum instead.  With a gate, residual + gate * that, as gated_residual."""
     active = [b for b in (loras or []) if b.use_lora]
-    if gate is not None and not (len(active) == 1 and _one_pass(active[0])):
-        return gated_residual(residual, gate, lora_linear(x, weight, bias, loras, workspace))
+    if gate is not None and not (one_rounding and len(active) == 1 and _one_pass(active[0])):
+        return gated_residual(residual, gate, lora_linear(x, weight, bias, loras, workspace, one_rounding))
     if not active:
         return linear_bf16(x, weight, bias, workspace=workspace)                    # `org_output + 0`
     if len(active) > MAX_BRANCHES:
@@ -117,7 +123,7 @@ def lora_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     # alpha_scale lives in a bf16 buffer in the reference
     alphas = [float(torch.tensor(b.alpha_scale, dtype=torch.bfloat16)) for b in active]
     if len(active) == 1 and _one_pass(active[0]):
-        return _with_one_branch(x, x2, weight, bias, active[0], alphas[0], workspace, residual, gate)
+        return _with_one_branch(x, x2, weight, bias, active[0], alphas[0], workspace, one_rounding, residual, gate)
     org = linear_bf16(x, weight, bias, workspace=workspace)
     ups = []
     for b, a in zip(active, alphas):
