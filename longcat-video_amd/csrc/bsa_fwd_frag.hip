@@ -483,11 +483,8 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
     // rounding of the pair to the storage type, 16 pairs - is cut into pieces that go between the MFMAs so that
     // no gap holds more than two MFMAs last: the first 14 pairs behind slots 0 .. 23 (the eight pairs of queries 0 .. 31
     // first: they are complete well before slot 24), the last two behind slots 24 .. 31 together with the row
-    // maximum of S(u+1), which is complete by then.  Fragment registers are reloaded in bursts behind the last
-    // MFMA that reads them: V(u+1) behind slot 7, a step and a half before it is used, K(u+3) behind slot 23, two steps.
-    // Within a burst the fragment that is used first is
-    // requested last: loads return in order, so the wait in front of its first use covers the whole burst and
-    // the fragments behind it need none of their own.
+    // maximum of S(u+1), which is complete by then.  A fragment register is reloaded behind the last MFMA that reads it: V(u+1)
+    // behind slots 0 .. 7, a step and a half before it is used, K(u+3) behind slots 9 .. 23, two steps.
     // `between` puts scalar work of the walk behind the slots.
     auto step = [&](auto jj, auto between) __attribute__((always_inline)) {
         constexpr int j = decltype(jj)::value;
@@ -568,8 +565,7 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                 __builtin_amdgcn_sched_barrier(0);
                 mfma_acc16(oacc[t][1], vb[vcur][t], pb[1]);
             }
-            // ---- reloads, in bursts behind the last MFMA that reads the fragments (single loads between the
-            // arithmetic cost more issue time than they take): V(u+1), K(u+3)
+            // ---- reloads, one by one behind the last MFMA that reads a fragment: V(u+1), K(u+3)
             if constexpr (slot < 8) vb[vprev][slot] = v_frag(offset_of(w[j]), slot);
             if constexpr (slot >= 8 && slot < 24 && slot % 2 == 1) kb[kslot][(slot - 9) / 2] = k_frag(offset_of(w[j + 2]), (slot - 9) / 2);
             if constexpr (slot == 7) {

@@ -40,6 +40,8 @@
 // A gated residual is added in the epilogue, for the same reason and by the rule of a residual: the library's product and gated_residual_kernel /
 // this, us, 28 618 x 4 096 x 4 096 (rounds full) 734 / 734, 44 969 x 2 304 x 2 304 (0.88) 505 / 432, 25 128 x 1 280 (0.97) 112 / 81, 0.72
 // full 5 795 x 3 968 168 / 172, K = 256 13.6 / 16.4 (506 rows, a launch less) to 26 / 21 (45 731).
+// A token's gate is asked for before its sums (32 760 x 4 096 x 4 096 845 -> 840).  The residual's lines brought into the L2 three k blocks ahead of
+// the epilogue (two loads a lane, whose wait falls into a phase) cost more than they save: 823 -> 842 with a residual.
 //
 // What bounds it: power, and the reading half of a phase.  Per k block and group 610 clocks to request 32 KB (the address unit of a
 // CU takes 16 a load of 1 KB, and a wavefront issues in order) and 500 to read 96 KB of fragments, against 1 009 of MFMAs, so the
@@ -348,8 +350,12 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
                 } else {
                     to = a.out + (int64_t)tok * a.ldo + f0;
                 }
-                const float* gate = nullptr;
-                if constexpr (kEpi == kGated) gate = a.gate + (int64_t)((uint32_t)min(tok, a.M - 1) / (uint32_t)a.gate_rows) * a.N + f0 + 4 * lg;
+                f32x4_ gate[8];
+                if constexpr (kEpi == kGated) {
+                    const float* row = a.gate + (int64_t)((uint32_t)min(tok, a.M - 1) / (uint32_t)a.gate_rows) * a.N + f0 + 4 * lg;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) gate[i] = *reinterpret_cast<const f32x4_*>(row + 16 * i);
+                }
                 uint4 o[4];
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
@@ -366,10 +372,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_nt_kernel(const GemmArgs a) 
 #pragma unroll
                         for (int h = 0; h < 2; ++h) {
                             const uint32_t raw[2] = {lo[h], hi[h]};
-                            f32x4_ g = {1.f, 1.f, 1.f, 1.f};
-                            if constexpr (kEpi == kGated) g = *reinterpret_cast<const f32x4_*>(gate + 32 * p + 16 * h);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) v[h][e] = (float)reinterpret_cast<const __bf16*>(raw)[e] + (kEpi == kGated ? g[e] * v[h][e] : v[h][e]);
+                            for (int e = 0; e < 4; ++e) v[h][e] = (float)reinterpret_cast<const __bf16*>(raw)[e] + (kEpi == kGated ? gate[2 * p + h][e] * v[h][e] : v[h][e]);
                         }
                     }
                     uint32_t w[2][2];
