@@ -172,6 +172,24 @@ def test_which_linear_layers_work_without_a_product():
     assert not alone(out=0x100000000 + (65536 * 1024 * 2 - 16)) and alone(out=0x100000000 + 65536 * 1024 * 2)
 
 
+def test_layers_behind_a_gate_or_with_a_branch_reject_bad_arguments():
+    lib = _capi.load()
+    p = [C.c_void_p(0x100000000 * i) for i in range(1, 9)]
+    ups = (C.c_void_p * 1)(0x900000000)
+
+    def gated(x=p[0], w=p[1], t=p[2], up=ups, res=p[3], gate=p[4], rows=4, out=p[5], M=8, N=256, K=128):
+        return lib.bsa_linear_gated_bf16(x, w, None, t, 64, up, 1, 64, 1.0, 1.0, res, gate, rows, out, M, N, K, p[6], 64 << 20, None)
+
+    for bad in ("x", "w", "up", "res", "gate", "out"):
+        assert gated(**{bad: None}) == _capi.BSA_ERR_BAD_ARG
+    assert gated(out=p[3]) == _capi.BSA_ERR_BAD_ARG                   # over the residual
+    assert gated(M=0) == gated(N=0) == gated(K=0) == _capi.BSA_ERR_BAD_ARG
+    assert gated(rows=3) == gated(rows=0) == _capi.BSA_ERR_SHAPE
+    args = [p[0], p[1], None, p[2], 64, ups, 1, 64, 1.0, 1.0, p[5], 8, 256, 128, p[6], 64 << 20, None]
+    for i in (0, 1, 3, 5, 10):
+        assert lib.bsa_linear_lora_bf16(*args[:i], None, *args[i + 1:]) == _capi.BSA_ERR_BAD_ARG
+
+
 def test_gemm_and_qkv_projection_reject_bad_arguments():
     lib = _capi.load()
 
