@@ -104,7 +104,7 @@ constexpr int kPipeList = 256;
 //   * the next item's Q rows go from global memory straight into an LDS staging tile (LDS DMA) and from there into
 //     the Q registers once the current item's last S^T product has been issued;
 //   * the positions of the tile walk behind the end of the list name the next item's first tile, so the fragment
-//     rings hold K(0), K(1), V(0), V_A(1) of the next item when the loop ends - what its prologue would load.
+//     rings hold K(0), K(1), V(0) of the next item when the loop ends - what its prologue would load.
 // K and V fragments are read through buffer resources (an SGPR base, a 32-bit scalar tile offset, the lane's
 // 16 bytes): no 64-bit vector address arithmetic in the loop, and an offset outside the buffer reads zeros.
 // kBounded: the kernel for items whose logits are bounded below the level at which the running maximum would move
