@@ -442,7 +442,8 @@ int make_plan(const bsa_3d_params* p, Plan* pl, bool compact = false) {
     pl->off_kp = take(bh * kv_rows * p->D * pl->es);
     pl->off_vp = take(bh * kv_rows * p->D * pl->es);
     pl->off_qc = take(bh * pl->nbq * p->D * pl->es);
-    pl->off_kc = take(bh * ((pl->nbk + 31) / 32 * 32) * p->D * pl->es);      // in operand order groups of 32 are filled up
+    // in operand order, which only the fragment-order kernel has them in, groups of 32 are filled up
+    pl->off_kc = take(bh * (pl->frag ? (pl->nbk + 31) / 32 * 32 : pl->nbk) * p->D * pl->es);
     pl->off_score = take(bh * pl->nbq * (size_t)pl->nbk * pl->es);
     pl->off_idx = take(bh * pl->nbq * (size_t)(pl->sel_width > 0 ? pl->sel_width : 1) * sizeof(int32_t));
     pl->off_idx_sorted = take(bh * pl->nbq * (size_t)(pl->sel_width > 0 ? pl->sel_width : 1) * sizeof(int32_t));

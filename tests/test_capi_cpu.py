@@ -148,6 +148,19 @@ def test_fwd_3d_plan_and_workspace():
     assert lib.bsa_fwd_3d(None, *args, ws, need, None, None, None, None) == _capi.BSA_ERR_BAD_ARG
 
 
+@pytest.mark.parametrize("heads,T,H,W", [(23, 28, 28, 80), (25, 24, 48, 52), (25, 32, 36, 52), (25, 36, 32, 52)])
+def test_fwd_3d_static_takes_what_its_buffer_holds(heads, T, H, W):
+    """The largest problems of its 64 MiB at density 1/16: no room for an order of k's chunk means that this route does not use."""
+    lib = _capi.load()
+    n = T // 4 * (H // 4) * (W // 4)
+    prm = _capi.Bsa3dParams(1, heads, 128, _capi.BSA_BF16, T, H, W, T, H, W, 4, 4, 4, 4, 4, 4, n // 16, 0.0883883)
+    st = _capi.strides3([heads * T * H * W * 128, T * H * W * 128, 128])
+    call = lambda: lib.bsa_fwd_3d_static(C.byref(prm), None, st, FAKE, st, FAKE, st, FAKE, st, None, None, None, None)      # noqa: E731
+    assert call() in (_capi.BSA_ERR_HIP, _capi.BSA_ERR_BAD_ARG)      # no GPU, or the tensor that is missing: behind the test of the size
+    prm.Hn = heads + 1
+    assert call() == _capi.BSA_ERR_WORKSPACE
+
+
 def test_which_linear_layers_work_without_a_product():
     """With a residual, a layer that the engine's GEMM serves needs the 64 MiB that every call brings; any other an fp32 product too."""
     lib = _capi.load()
