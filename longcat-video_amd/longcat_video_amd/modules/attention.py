@@ -347,22 +347,29 @@ class Attention(nn.Module):
         # epilogue) and bsa_gemm_bf16.  Both round at the same points.
         self.projection_backend = "hipblaslt"
 
-    def _linear(self, x, layer, loras, residual=None, gate=None, one_rounding=True):
-        engine = self.projection_backend == "engine" and layer.weight.shape[0] % 128 == 0 and layer.weight.shape[1] % 64 == 0
-        if gate is not None:                              # residual + gate * the layer
-            if any(b.use_lora for b in loras):
-                from .lora import lora_linear
-                return lora_linear(x, layer.weight, layer.bias, loras, None, one_rounding, residual, gate)
-            if engine:
-                return gated_residual(residual, gate, gemm_bf16(x, layer.weight, layer.bias))
-            return linear_gated(x, layer.weight, layer.bias, residual, gate)
+    def _engine_gemm(self, layer):
+        return self.projection_backend == "engine" and layer.weight.shape[0] % 128 == 0 and layer.weight.shape[1] % 64 == 0
+
+    def _linear(self, x, layer, loras, residual=None):
         if any(b.use_lora for b in loras):
             from .lora import lora_linear
-            y = lora_linear(x, layer.weight, layer.bias, loras, None, one_rounding)
+            # q and k choose the blocks: rounded once, with a side branch inside the product, near ties would fall differently than eager
+            y = lora_linear(x, layer.weight, layer.bias, loras, None, one_rounding=layer is not self.qkv)
             return y if residual is None else y + residual
-        if engine:
+        if self._engine_gemm(layer):
             return gemm_bf16(x, layer.weight, layer.bias, residual=residual)
         return linear_bf16(x, layer.weight, layer.bias, residual=residual)
+
+    def _output(self, x, residual, gate):
+        """The output projection, plus a residual, or residual + gate * the projection."""
+        if gate is None:
+            return self._linear(x, self.proj, self.proj_loras, residual=residual)
+        if any(b.use_lora for b in self.proj_loras):
+            from .lora import lora_linear
+            return lora_linear(x, self.proj.weight, self.proj.bias, self.proj_loras, None, True, residual, gate)
+        if self._engine_gemm(self.proj):
+            return gated_residual(residual, gate, gemm_bf16(x, self.proj.weight, self.proj.bias))
+        return linear_gated(x, self.proj.weight, self.proj.bias, residual, gate)
 
     def _fused_projection(self, x, shape, return_kv):
         """True when the QKV GEMM with the fused epilogue applies: engine backend, no LoRA branch on qkv, no
@@ -412,8 +419,7 @@ class Attention(nn.Module):
 
     def _project_qkv(self, x):
         B, N, C = x.shape
-        # q and k choose the blocks: rounded once, with a side branch inside the product, near ties would fall differently than eager
-        qkv = self._linear(x, self.qkv, self.qkv_loras, one_rounding=False)       # [B, N, 3C]
+        qkv = self._linear(x, self.qkv, self.qkv_loras)                           # [B, N, 3C]
         return qkv.view(B, N, 3, self.num_heads, self.head_dim).permute(2, 0, 3, 1, 4).unbind(0)   # strided [B,H,N,D] views
 
     @torch.no_grad()
@@ -445,7 +451,7 @@ class Attention(nn.Module):
                 self._process_attn(qs[:, :, n:], ks, vs, shape, out=ov[:, :, n:], qk_norm=norm(num_cond_latents), kv_out=kv_out)   # attention.py:132-133
             else:
                 self._process_attn(qs, ks, vs, shape, out=ov, qk_norm=norm(0), kv_out=kv_out)
-            y = self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
+            y = self._output(o.view(B, N, C), residual, gate)
             return (y, kv_out) if return_kv else y
         else:
             # q moves into a per-head tensor on the way (the attention kernel fetches its rows tile by tile); k is
@@ -467,7 +473,7 @@ class Attention(nn.Module):
             self._process_attn(q[:, :, n:], k, v, shape, out=ov[:, :, n:])                       # attention.py:132-133
         else:
             self._process_attn(q, k, v, shape, out=ov)
-        y = self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
+        y = self._output(o.view(B, N, C), residual, gate)
         if return_kv:
             return y, (k_cache, v.contiguous())
         return y
@@ -500,7 +506,7 @@ class Attention(nn.Module):
             tab = rope_table(grid_full, D, x.device)
             self._process_attn(qs, ks, vs, shape, out=o.permute(0, 2, 1, 3), kv_cache=(kc, vc, int(num_cond_latents)),
                                qk_norm=(self.q_norm.weight, self.k_norm.weight, tab, T + num_cond_latents, num_cond_latents, 0, eps))
-            return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
+            return self._output(o.view(B, N, C), residual, gate)
         k_full = torch.empty(B, Hn, n_c + N, D, dtype=x.dtype, device=x.device)
         v_full = torch.empty_like(k_full)
         kc = k_cache.to(x.device).expand(B, -1, -1, -1)                            # attention.py:162-164
@@ -514,7 +520,19 @@ class Attention(nn.Module):
                       t_offset=num_cond_latents, table_grid=grid_full)
         o = torch.empty(B, N, Hn, D, dtype=x.dtype, device=x.device)
         self._process_attn(q, k_full, v_full, shape, out=o.permute(0, 2, 1, 3))
-        return self._linear(o.view(B, N, C), self.proj, self.proj_loras, residual, gate)
+        return self._output(o.view(B, N, C), residual, gate)
+
+
+# What runs between the branch of a DiT block and its output projection, as defined here.
+_OWN = {name: getattr(Attention, name) for name in ("__call__", "forward", "forward_with_kv_cache", "_linear")}
+
+
+def _takes_the_gate(attn, x) -> bool:
+    """True where nothing between the branch and the output projection can look at what the projection gives, or has another signature:
+    no subclass, no hook, and none of these methods replaced, on the object or on the class."""
+    return (type(attn) is Attention and x.dtype == torch.bfloat16 and not attn._forward_hooks and not attn._forward_pre_hooks
+            and not torch.nn.modules.module._has_any_global_hook() and not _OWN.keys() & attn.__dict__.keys()
+            and all(getattr(Attention, name) is own for name, own in _OWN.items()))
 
 
 @torch.no_grad()
@@ -583,9 +601,7 @@ def dit_self_attention_branch(x: torch.Tensor, shift_msa: torch.Tensor, scale_ms
     small fp32 linear layer outside this path)."""
     x_m = layernorm_modulate(x, shift_msa, scale_msa)
     new_cache = None
-    # the gate and the sum inside the output projection, where nothing between the two can look at what it gives
-    if (type(attn) is Attention and x.dtype == torch.bfloat16 and not attn._forward_hooks and not attn._forward_pre_hooks
-            and not torch.nn.modules.module._has_any_global_hook() and not {"forward", "forward_with_kv_cache", "_linear"} & attn.__dict__.keys()):
+    if _takes_the_gate(attn, x):                          # the gate and the sum inside the output projection
         inside = dict(shape=latent_shape, num_cond_latents=num_cond_latents, residual=x, gate=gate_msa)
         if kv_cache is not None:
             out = attn.forward_with_kv_cache(x_m, kv_cache=kv_cache, **inside)

@@ -140,6 +140,55 @@ def test_tokens_that_do_not_fill_the_grid_are_refused(monkeypatch, kw):
         attn(torch.zeros(1, 256, 256, dtype=torch.bfloat16), shape=(4, 8, 8), **kw)
 
 
+@pytest.mark.parametrize("name", ["forward", "forward_with_kv_cache", "__call__", "_linear"])
+@pytest.mark.parametrize("where", ["class", "object"])
+def test_a_replaced_attention_is_called_with_the_signature_it_had(monkeypatch, name, where):
+    """The adaLN branch, with a method of Attention replaced on the class or on the object by one that knows no gate."""
+    from longcat_video_amd.modules import attention as A
+    if (name, where) == ("__call__", "object"):
+        pytest.skip("looked up on the class alone")
+    attn = A.Attention(256, 2, enable_bsa=True, bsa_params=dict(sparsity=0.5, chunk_3d_shape_q=[4, 4, 4], chunk_3d_shape_k=[4, 4, 4])).to(torch.bfloat16)
+    calls = []
+
+    def replaced(self, x, shape=None, num_cond_latents=None, return_kv=False):
+        calls.append(name)
+        return (x + 1, "cache") if return_kv else x + 1
+
+    def replaced_cached(self, x, shape=None, num_cond_latents=None, kv_cache=None):
+        calls.append(name)
+        return x + 1
+
+    def replaced_linear(self, x, layer, loras, residual=None):
+        calls.append(layer)
+        y = torch.nn.functional.linear(x, layer.weight, layer.bias)
+        return y if residual is None else y + residual
+
+    new = {"forward_with_kv_cache": replaced_cached, "_linear": replaced_linear}.get(name, replaced)
+    if where == "class":
+        monkeypatch.setattr(A.Attention, name, new)
+    else:
+        monkeypatch.setattr(attn, name, new.__get__(attn))
+    monkeypatch.setattr(A, "layernorm_modulate", lambda x, shift, scale: x)
+    monkeypatch.setattr(A, "gated_residual", lambda x, gate, y: ("gated", y))
+    monkeypatch.setattr(A, "rope_table", lambda *a: None)
+    monkeypatch.setattr(A.Attention, "_process_attn", lambda self, q, k, v, shape, out=None, **kw: out.zero_())
+    x, mod = torch.zeros(1, 256, 256, dtype=torch.bfloat16), torch.zeros(1, 4, 1, 256)
+    cache = [torch.zeros(1, 2, 128, 128, dtype=torch.bfloat16) for _ in range(2)]
+    run = lambda **kw: A.dit_self_attention_branch(x, mod, mod, mod, attn, (4, 8, 8), **kw)      # noqa: E731
+    with torch.no_grad():
+        after = x + 1 if name != "_linear" else torch.nn.functional.linear(x, attn.proj.weight, attn.proj.bias)
+    if name != "forward_with_kv_cache":
+        for kw in (dict(), dict(num_cond_latents=1)):
+            out = run(**kw)
+            assert out[0] == "gated" and torch.equal(out[1], after)
+        out, kept = run(return_kv=True)
+        assert out[0] == "gated" and torch.equal(out[1], after) and (kept == "cache" or len(kept) == 2)
+    if name in ("forward_with_kv_cache", "_linear"):
+        out = run(num_cond_latents=2, kv_cache=cache)
+        assert out[0] == "gated" and torch.equal(out[1], after)
+    assert len(calls) > 0
+
+
 def test_plans_are_kept_by_value():
     """Grids as tensor elements (what an int() of them would have read at each call), rules as tensors."""
     I._capi.load()
