@@ -360,6 +360,15 @@ class Attention(nn.Module):
             return gemm_bf16(x, layer.weight, layer.bias, residual=residual)
         return linear_bf16(x, layer.weight, layer.bias, residual=residual)
 
+    @staticmethod
+    def _check_gate(residual, gate):
+        """At the door, not behind the attention."""
+        if gate is None:
+            return
+        if residual is None:
+            raise ValueError("a gate comes with the residual that the gated projection is added to")
+        _check_frames(residual, gate, "gate")
+
     def _output(self, x, residual, gate):
         """The output projection, plus a residual, or residual + gate * the projection."""
         if gate is None:
@@ -429,6 +438,7 @@ class Attention(nn.Module):
         residual + gate * the projection."""
         B, N, C = x.shape
         Hn, D = self.num_heads, self.head_dim
+        self._check_gate(residual, gate)
         eps = self.q_norm.eps
         new = lambda: torch.empty(B, Hn, N, D, dtype=x.dtype, device=x.device)
         if self._fused_projection(x, shape, return_kv):
@@ -487,6 +497,7 @@ class Attention(nn.Module):
         B, N, C = x.shape
         Hn, D = self.num_heads, self.head_dim
         T, Hg, Wg = (int(g) for g in shape)
+        self._check_gate(residual, gate)
         k_cache, v_cache = kv_cache
         assert k_cache.shape[0] == v_cache.shape[0] and k_cache.shape[0] in [1, B]
         if not (num_cond_latents is not None and num_cond_latents > 0):
@@ -547,14 +558,19 @@ def attention_block_forward(x: torch.Tensor, pre_norm_weight: torch.Tensor, attn
 # ---------------------------------------------------------------------------
 # adaLN wrapper of the self-attention branch of a DiT block
 # ---------------------------------------------------------------------------
-def _frames(x: torch.Tensor, mod: torch.Tensor, name: str):
+def _check_frames(x: torch.Tensor, mod: torch.Tensor, name: str) -> int:
     B, N, C = x.shape
     assert mod.dtype == torch.float32, "%s must be fp32 (blocks.py:129)" % name
     assert mod.dim() == 4 and mod.shape[0] == B and mod.shape[2] == 1 and mod.shape[3] == C, \
         "%s must be [B, T, 1, C]" % name
     T = mod.shape[1]
-    assert N % T == 0
-    return mod.contiguous(), N // T
+    assert N % T == 0, "%s: %d tokens are not whole frames of %d" % (name, N, T)
+    return N // T
+
+
+def _frames(x: torch.Tensor, mod: torch.Tensor, name: str):
+    per = _check_frames(x, mod, name)
+    return mod.contiguous(), per
 
 
 def layernorm_modulate(x: torch.Tensor, shift: torch.Tensor, scale: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:

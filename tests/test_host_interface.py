@@ -189,6 +189,20 @@ def test_a_replaced_attention_is_called_with_the_signature_it_had(monkeypatch, n
     assert len(calls) > 0
 
 
+def test_a_gate_without_its_residual_is_refused_before_any_launch(monkeypatch):
+    attn = _small_module(monkeypatch)
+    x, gate = torch.zeros(1, 256, 256, dtype=torch.bfloat16), torch.zeros(1, 4, 1, 256)
+    cache = [torch.zeros(1, 2, 128, 128, dtype=torch.bfloat16) for _ in range(2)]
+    with pytest.raises(ValueError, match="residual"):
+        attn(x, shape=(4, 8, 8), gate=gate)
+    with pytest.raises(ValueError, match="residual"):
+        attn.forward_with_kv_cache(x, shape=(4, 8, 8), num_cond_latents=2, kv_cache=cache, gate=gate)
+    with pytest.raises(AssertionError, match="gate"):
+        attn(x, shape=(4, 8, 8), residual=x, gate=gate[..., :128])
+    with pytest.raises(AssertionError, match="gate"):
+        attn.forward_with_kv_cache(x, shape=(4, 8, 8), num_cond_latents=2, kv_cache=cache, residual=x, gate=gate.bfloat16())
+
+
 def test_plans_are_kept_by_value():
     """Grids as tensor elements (what an int() of them would have read at each call), rules as tensors."""
     I._capi.load()
