@@ -443,11 +443,12 @@ size_t bsa_linear_bf16_ld_workspace_bytes(const void* x, int64_t ldx, const void
 /* One-time tuning of a linear shape (no counterpart in the reference, whose nn.Linear leaves the choice to the
  * BLAS library): runs every algorithm hipBLASLt proposes for this call (up to 32, each four times on the given
  * buffers; `out` is overwritten), and remembers the fastest for later bsa_linear_bf16 / _ld calls with the same
- * M, N, K, row strides, bias / residual presence (and, with a residual, a workspace of the same size) in this process,
- * as far as these go to the library.  Unlike every other entry point it WAITS for
+ * M, N, K, row strides, bias / residual presence (and, with a residual, a workspace of the same size) in this process.
+ * A call that the engine's own GEMM serves leaves nothing to choose: that kernel alone is timed, in a workspace as the call
+ * needs it, 1 is returned and both times are its own.  Unlike every other entry point it WAITS for
  * the stream, so call it at set-up, outside graph capture.  Returns the number of algorithms timed (> 0) or a
  * negative status; default_ms / best_ms (optional) receive the time of the algorithm an untuned call uses and
- * of the one chosen.  Algorithms differ in summation order, so results can differ in the last bit. */
+ * of the one chosen (the library's with a residual: without the pass that adds it).  Algorithms differ in summation order, so results can differ in the last bit. */
 int bsa_linear_bf16_tune(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
                          void* out, int64_t ldo, int64_t M, int N, int K, void* workspace, size_t workspace_bytes,
                          void* stream, float* default_ms, float* best_ms);

@@ -727,6 +727,26 @@ size_t bsa_linear_bf16_ld_workspace_bytes(const void* x, int64_t ldx, const void
     return bsa_linear_bf16_workspace_bytes(M, N, residual != nullptr && !gemm_serves_linear(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K));
 }
 
+// bsa_linear_bf16_tune where the engine's GEMM serves the call: nothing to choose, the time is that of what runs.
+static int time_own_gemm(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual, void* out, int64_t ldo,
+                         int64_t M, int N, int K, void* stream, float* default_ms, float* best_ms) {
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    int rc = hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess ? BSA_OK : set_error(BSA_ERR_HIP, "linear tune: hipEventCreate failed");
+    for (int r = 0; r < 4 && rc == BSA_OK; ++r) {
+        if (r == 1 && hipEventRecord(e0, (hipStream_t)stream) != hipSuccess) rc = set_error(BSA_ERR_HIP, "linear tune: hipEventRecord failed");
+        if (rc == BSA_OK) rc = bsa_gemm_bf16(x, ldx, w, ldw, bias, residual, ldo, out, ldo, M, N, K, stream);
+    }
+    float ms = 0.f;
+    if (rc == BSA_OK && (hipEventRecord(e1, (hipStream_t)stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))
+        rc = set_error(BSA_ERR_HIP, "linear tune: the timed runs failed");
+    if (e0) (void)hipEventDestroy(e0);
+    if (e1) (void)hipEventDestroy(e1);
+    if (rc != BSA_OK) return rc;
+    if (default_ms) *default_ms = ms / 3.f;
+    if (best_ms) *best_ms = ms / 3.f;
+    return 1;
+}
+
 static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias, const void* residual,
                        void* out, int64_t ldo, int64_t M, int N, int K, void* workspace, size_t workspace_bytes,
                        void* stream, bool tune, float* default_ms, float* best_ms) {
@@ -738,8 +758,9 @@ static int linear_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, c
     // want just under 64 MiB (1.52 PFLOP/s instead of 1.24 with 32 MiB); more brings nothing.
     if (!workspace || workspace_bytes < kLtWorkspace)
         return set_error(BSA_ERR_WORKSPACE, "linear: a workspace of at least 64 MiB is required (got %zu bytes)", workspace_bytes);
-    if (!tune && gemm_serves_linear(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K))
-        return bsa_gemm_bf16(x, ldx, w, ldw, bias, residual, ldo, out, ldo, M, N, K, stream);
+    if (gemm_serves_linear(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K))
+        return tune ? time_own_gemm(x, ldx, w, ldw, bias, residual, out, ldo, M, N, K, stream, default_ms, best_ms)
+                    : bsa_gemm_bf16(x, ldx, w, ldw, bias, residual, ldo, out, ldo, M, N, K, stream);
     if (!residual) return lt_product(x, ldx, w, ldw, bias, out, ldo, false, M, N, K, workspace, workspace_bytes, stream, tune, default_ms, best_ms);
 
     // With a residual the product goes to fp32 behind the library's share of the workspace, as many rows (and columns) at a time

@@ -161,7 +161,8 @@ def tune_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
                 workspace: Optional[torch.Tensor] = None):
     """One-time choice of the GEMM algorithm for ``linear_bf16`` calls of this shape (rows of x, weight shape, bias and
     residual presence): times what hipBLASLt proposes and keeps the fastest for the rest of the process.  Waits for
-    the stream; call at set-up.  Returns (algorithms timed, ms of the default choice, ms of the chosen one)."""
+    the stream; call at set-up.  Returns (algorithms timed, ms of the default choice, ms of the chosen one); where the engine's own
+    GEMM serves such calls there is no choice: 1 and its time twice."""
     if not x.is_cuda:
         raise RuntimeError("the engine runs on the GPU only")
     K, N = x.shape[-1], weight.shape[0]
@@ -171,7 +172,8 @@ def tune_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     out = torch.empty(x2.shape[0], N, dtype=torch.bfloat16, device=x.device)
     r = torch.zeros_like(out) if residual else None
     if workspace is None:
-        need = None if not residual else lambda: _capi.load().bsa_linear_bf16_workspace_bytes(x2.shape[0], N, 1)
+        need = None if not residual else lambda: _capi.load().bsa_linear_bf16_ld_workspace_bytes(
+            _ptr(x2), K, _ptr(w), K, _ptr(b), _ptr(r), _ptr(out), N, x2.shape[0], N, K)
         workspace = _linear_workspace(x2.shape[0], N, need, x.device)
     d, best = C.c_float(0), C.c_float(0)
     with _on_device(x):

@@ -500,6 +500,28 @@ def test_linear_tuning_keeps_results_and_is_remembered():
     assert torch.equal(after, M().linear_bf16(x, w, b).cpu())          # the remembered choice is deterministic
 
 
+@pytest.mark.parametrize("rows,n,k,residual,own", [
+    (8192, 2048, 2048, True, True), (1000, 256, 128, False, True),          # full rounds with a residual, short rows
+    (2048, 1024, 1024, True, False),                                        # 32 tiles: the library's product
+])
+def test_linear_tuning_times_what_runs(rows, n, k, residual, own):
+    """Where the engine's GEMM serves a layer, that kernel's time, in no more workspace than the call has use for."""
+    g = torch.Generator(device="cuda").manual_seed(34)
+    x, w = (torch.randn(*s, generator=g, device="cuda").bfloat16() for s in ((1, rows, k), (n, k)))
+    M().linear_bf16(x, w, None)                              # the kept workspace
+    torch.cuda.synchronize()
+    held = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    timed, default_ms, best_ms = M().tune_linear(x, w, None, residual=residual)
+    used = torch.cuda.max_memory_allocated() - held
+    assert timed >= 1 and best_ms > 0
+    if own:
+        assert timed == 1 and default_ms == best_ms
+        assert used <= (2 if residual else 1) * rows * n * 2 + (1 << 20)      # out and the residual
+    else:
+        assert timed > 1
+
+
 @pytest.mark.parametrize("grid,dtype", [((4, 8, 8), torch.bfloat16), ((3, 6, 10), torch.bfloat16), ((2, 9, 8), torch.float16)])
 def test_operator_with_the_norm_inside_equals_the_separate_passes(grid, dtype):
     """bsa_fwd_3d_qknorm (q and k normalised and rotated inside the operator's own passes) against bsa_norm_rope
