@@ -474,13 +474,13 @@ int bsa_lora_up_add(const void* org, const void* t, int64_t ldt, const void* con
 /* A Linear with one side branch from its down projection on: out = T(x . w^T + bias + s), s = multiplier * alpha_scale * up(t), bf16 in and
  * out.  Operands as in bsa_linear_bf16 (rows of x, w and out next to each other, the workspace too) and bsa_lora_up_add.  Where the engine's
  * GEMM serves it, all of it is accumulated in fp32 and rounded once; otherwise bsa_linear_bf16 and bsa_lora_up_add with
- * their roundings, and what these are not built for is refused as there.  out must be memory of its own. */
+ * their roundings, and what these are not built for is refused as there.  out must be memory of its own (BSA_ERR_BAD_ARG otherwise). */
 int bsa_linear_lora_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
                          float multiplier, float alpha_scale, void* out, int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream);
 
 /* The same behind a gate, as a DiT block adds its attention (longcat_video_dit.py:101-103): out = T(residual + gate * y), y the layer's output
  * with its side branch, or, with t NULL, without one.  gate: fp32 [M / rows_per_group, N].  One rounding where the engine's GEMM serves
- * it, otherwise that of y and that of bsa_gated_residual.  out must be memory of its own. */
+ * it, otherwise that of y and that of bsa_gated_residual.  out must be memory of its own (BSA_ERR_BAD_ARG otherwise). */
 int bsa_linear_gated_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
                           float multiplier, float alpha_scale, const void* residual, const float* gate, int rows_per_group, void* out,
                           int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream);

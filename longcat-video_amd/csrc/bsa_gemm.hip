@@ -459,20 +459,33 @@ bool gemm_serves_linear(const void* x, int64_t ldx, const void* w, int64_t ldw, 
 // 12 000 x 2 048 x 2 048 105 / 94, two thirds 1 560 x 12 288 x 4 096 152 / 169, 0.56 9 000 x 2 048 x 2 048 89 / 90.  A short K has less to lose: K = 1 024
 // 0.54 full 17 500 x 1 024 67 / 56, 3 000 x 3 072 45 / 29, a quarter full 4 000 x 1 024 24 / 27; K = 768 a third full 28 / 24, 0.07 12.9 / 22.5; K = 256
 // 17.3 / 14.3 (506 x 256) to 33 / 17 (39 401).  With a gated residual as well, K = 256 19.4 / 19.1 to 41 / 23, 0.34 full 33 / 30, 0.84 27 580 x 2 048
-// 287 / 235, 1.00 28 618 x 4 096 856 / 765.  Pointers and rows as above.
+// 287 / 235, 1.00 28 618 x 4 096 856 / 765.  Pointers and rows as above; out is memory of its own (check_own_memory).
 static bool lora_serves(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
                         const void* out, int64_t M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || M > 0x7fffffffLL || n_sep <= 0 || n_sep > kMaxSlices || rank <= 0 || rank % kBK || rank > 128) return false;
     if (K % kBK || K >= (1 << 22) || N % n_sep || N / n_sep % kTileN || ldt < (int64_t)n_sep * rank || ldt % 8 || ldt >= (1 << 22)) return false;
     const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
     if (((at(x) | at(w) | at(t) | at(out)) & 15u) || (at(bias) & 7u)) return false;
-    const uintptr_t o = at(out), o_end = o + (uintptr_t)M * N * 2u;
-    const auto meets = [&](const void* p, uintptr_t bytes) { return p != nullptr && at(p) < o_end && o < at(p) + bytes; };
-    if (meets(x, (uintptr_t)M * K * 2u) || meets(w, (uintptr_t)N * K * 2u) || meets(bias, (uintptr_t)N * 2u) || meets(t, (uintptr_t)((M - 1) * ldt + n_sep * rank) * 2u)) return false;
     for (int i = 0; i < n_sep; ++i)
-        if (!up[i] || (at(up[i]) & 15u) || meets(up[i], (uintptr_t)(N / n_sep) * rank * 2u)) return false;
+        if (!up[i] || (at(up[i]) & 15u)) return false;
     const int64_t tiles = (M + kTileM - 1) / kTileM * (N / kTileN), round = (tiles + kCus - 1) / kCus * kCus;
     return K <= 256 || (K <= 1024 ? 5 * tiles >= 2 * round : 4 * tiles >= 3 * round);
+}
+
+// What a layer with a side branch or behind a gate reads: neither route has read all of it before its first result is stored.
+static int check_own_memory(const char* what, const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
+                            const void* residual, const float* gate, int64_t groups, const void* out, int64_t M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0) return set_error(BSA_ERR_BAD_ARG, "%s: sizes must be positive", what);
+    const auto at = [](const void* p) { return reinterpret_cast<uintptr_t>(p); };
+    const uintptr_t o = at(out), o_end = o + (uintptr_t)M * N * 2u;
+    const auto meets = [&](const void* p, uintptr_t bytes) { return p != nullptr && at(p) < o_end && o < at(p) + bytes; };
+    bool over = meets(x, (uintptr_t)M * K * 2u) || meets(w, (uintptr_t)N * K * 2u) || meets(bias, (uintptr_t)N * 2u) || meets(residual, (uintptr_t)M * N * 2u) ||
+                meets(gate, (uintptr_t)groups * N * sizeof(float));
+    if (t != nullptr && n_sep > 0 && n_sep <= kMaxSlices && rank > 0 && ldt > 0) {      // refused otherwise
+        over = over || meets(t, (uintptr_t)((M - 1) * ldt + (int64_t)n_sep * rank) * 2u);
+        for (int i = 0; i < n_sep; ++i) over = over || meets(up[i], (uintptr_t)(N / n_sep) * rank * 2u);
+    }
+    return over ? set_error(BSA_ERR_BAD_ARG, "%s: out must be memory of its own", what) : BSA_OK;
 }
 
 static GemmArgs layer_args(const void* x, const void* w, const void* bias, void* out, int64_t M, int N, int K) {
@@ -512,9 +525,11 @@ int bsa_gemm_bf16(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
 int bsa_linear_lora_bf16(const void* x, const void* w, const void* bias, const void* t, int64_t ldt, const void* const* up, int n_sep, int rank,
                          float multiplier, float alpha_scale, void* out, int64_t M, int N, int K, void* workspace, size_t workspace_bytes, void* stream) {
     if (!x || !w || !t || !up || !out) return set_error(BSA_ERR_BAD_ARG, "linear_lora: null pointer");
+    const int rc = check_own_memory("linear_lora", x, w, bias, t, ldt, up, n_sep, rank, nullptr, nullptr, 0, out, M, N, K);
+    if (rc != BSA_OK) return rc;
     if (!lora_serves(x, w, bias, t, ldt, up, n_sep, rank, out, M, N, K)) {
-        const int rc = bsa_linear_bf16(x, w, bias, nullptr, out, M, N, K, workspace, workspace_bytes, stream);
-        return rc != BSA_OK ? rc : bsa_lora_up_add(out, t, ldt, up, n_sep, rank, multiplier, alpha_scale, out, M, N, stream);
+        const int lrc = bsa_linear_bf16(x, w, bias, nullptr, out, M, N, K, workspace, workspace_bytes, stream);
+        return lrc != BSA_OK ? lrc : bsa_lora_up_add(out, t, ldt, up, n_sep, rank, multiplier, alpha_scale, out, M, N, stream);
     }
     GemmArgs a = layer_args(x, w, bias, out, M, N, K);
     add_side(a, t, ldt, up, n_sep, rank, multiplier * alpha_scale);
@@ -528,10 +543,9 @@ int bsa_linear_gated_bf16(const void* x, const void* w, const void* bias, const 
     if (M <= 0 || N <= 0 || K <= 0) return set_error(BSA_ERR_BAD_ARG, "linear_gated: sizes must be positive");
     if (rows_per_group <= 0 || M % rows_per_group != 0)
         return set_error(BSA_ERR_SHAPE, "linear_gated: %lld rows do not split into groups of %d", (long long)M, rows_per_group);
-    if (out == residual) return set_error(BSA_ERR_BAD_ARG, "linear_gated: out must be memory of its own");
-    const uintptr_t o = reinterpret_cast<uintptr_t>(out), g = reinterpret_cast<uintptr_t>(gate);
-    const bool over_gate = g < o + (uintptr_t)M * N * 2u && o < g + (uintptr_t)(M / rows_per_group) * N * sizeof(float);
-    if (!(g & 15u) && !over_gate && gemm_takes(x, K, w, K, bias, residual, out, N, M, N, K) &&
+    const int own = check_own_memory("linear_gated", x, w, bias, t, ldt, up, n_sep, rank, residual, gate, M / rows_per_group, out, M, N, K);
+    if (own != BSA_OK) return own;
+    if (!(reinterpret_cast<uintptr_t>(gate) & 15u) && gemm_takes(x, K, w, K, bias, residual, out, N, M, N, K) &&
         (t ? lora_serves(x, w, bias, t, ldt, up, n_sep, rank, out, M, N, K) : residual_serves(M, N, K))) {
         GemmArgs a = layer_args(x, w, bias, out, M, N, K);
         a.residual = (const __bf16*)residual; a.ldr = N; a.gate = gate; a.gate_rows = rows_per_group;

@@ -203,6 +203,32 @@ def test_layers_behind_a_gate_or_with_a_branch_reject_bad_arguments():
         assert lib.bsa_linear_lora_bf16(*args[:i], None, *args[i + 1:]) == _capi.BSA_ERR_BAD_ARG
 
 
+@pytest.mark.parametrize("K,M", [(128, 8), (1000, 8), (4096, 4608)])      # served whatever the tiles; not served; served without a branch alone
+def test_layers_behind_a_gate_or_with_a_branch_refuse_results_over_their_operands(K, M):
+    """`out` is written while they are still read, or before: also where a few bytes meet; refused in front of any launch."""
+    lib = _capi.load()
+    N, r, rows = 512, 64, 4
+    size = dict(x=M * K * 2, w=N * K * 2, bias=N * 2, t=((M - 1) * 72 + r) * 2, up=N * r * 2, res=M * N * 2, gate=M // rows * N * 4)
+    at = {name: 0x100000000 * (i + 1) for i, name in enumerate(size)}
+    ws = C.c_void_p(0xb00000000)
+    p = {name: C.c_void_p(a) for name, a in at.items()}
+    ups = (C.c_void_p * 1)(at["up"])
+
+    def gated(out, t=p["t"]):
+        return lib.bsa_linear_gated_bf16(p["x"], p["w"], p["bias"], t, 72, ups, 1, r, 1.0, 0.5, p["res"], p["gate"], rows, C.c_void_p(out), M, N, K, ws, 64 << 20, None)
+
+    def lora(out):
+        return lib.bsa_linear_lora_bf16(p["x"], p["w"], p["bias"], p["t"], 72, ups, 1, r, 1.0, 0.5, C.c_void_p(out), M, N, K, ws, 64 << 20, None)
+
+    for name, a in at.items():
+        for out in (a, a + size[name] // 16 * 16 - 16, a - M * N * 2 + 16):
+            assert gated(out) == _capi.BSA_ERR_BAD_ARG and "own" in _capi.last_error(), name
+            if name not in ("t", "up"):
+                assert gated(out, None) == _capi.BSA_ERR_BAD_ARG
+            if name not in ("res", "gate"):
+                assert lora(out) == _capi.BSA_ERR_BAD_ARG and "own" in _capi.last_error(), name
+
+
 def test_gemm_and_qkv_projection_reject_bad_arguments():
     lib = _capi.load()
 
