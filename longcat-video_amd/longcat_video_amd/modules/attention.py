@@ -346,7 +346,9 @@ class Attention(nn.Module):
         self.proj_loras = []
         # "hipblaslt": the projections through bsa_linear_bf16, norm and rotation as separate passes (the faster
         # route at the 720p shapes); "engine": bsa_qkv_projection (GEMM with norm, rotation and head split in its
-        # epilogue) and bsa_gemm_bf16.  Both round at the same points.
+        # epilogue) and bsa_gemm_bf16.  Both round at the same points, but for the output projection behind a gate: the default
+        # route rounds all of it once where the GEMM serves it (bsa_linear_gated_bf16), this one the projection first.
+        # A LoRA branch takes the default route on either.
         self.projection_backend = "hipblaslt"
 
     def _engine_gemm(self, layer):

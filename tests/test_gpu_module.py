@@ -448,6 +448,25 @@ def test_a_hook_sees_the_attention_without_its_gate():
     assert torch.all((plain.float() - hooked.float()).abs() <= bound)
 
 
+def test_roundings_of_a_gated_block_on_both_backends():
+    """The default route adds the gate in the product (dim 256: short rows), rounded once; the engine's projections leave the layer's own
+    rounding in between, as separate passes do."""
+    shape = (4, 8, 8)
+    m = make_module(dim=256, heads=2, sparsity=0.5, seed=17).cuda()
+    g = torch.Generator(device="cuda").manual_seed(18)
+    x = torch.randn(1, 256, 256, generator=g, device="cuda").bfloat16()
+    shift, scale, gate = torch.randn(3, 1, 4, 1, 256, generator=g, device="cuda").unbind(0)
+    x_m = M().layernorm_modulate(x, shift, scale)
+    for backend in ("hipblaslt", "engine"):
+        m.projection_backend = backend
+        y = m(x_m, shape=shape)
+        apart, got = M().gated_residual(x, gate, y), M().dit_self_attention_branch(x, shift, scale, gate, m, shape)
+        if backend == "engine":
+            assert torch.equal(got, apart)
+        bound = BF16_ULP * (apart.float().abs() + (gate * y.float().view(1, 4, 64, 256)).abs().view(1, 256, 256))      # y's rounding and the last, half an ulp each, twice
+        assert torch.all((got.float() - apart.float()).abs() <= bound)
+
+
 def test_module_forward_with_lora_branches():
     """longcat_video_dit.py:211-249: LoRA branches on attn.qkv (up-projection split in three) and attn.proj."""
     shape = (4, 8, 8)
