@@ -1,4 +1,5 @@
-"""bf16 linear layers with a residual: bf16(x w^T + bias + residual), an fp32 product and a pass that adds the rest."""
+"""bf16 linear layers with a residual: bf16(x w^T + bias + residual), by the engine's GEMM where it serves them, otherwise an fp32
+product of the library and a pass that adds the rest."""
 import pytest
 import torch
 
@@ -20,8 +21,8 @@ def _integers(g, *shape):
     (257, 384, 512, False),
     (300, 100, 60, False),            # columns that 16-byte pieces do not divide
     (33, 4100, 128, True),
-    (3000, 4096, 64, True),           # the least workspace takes 2 048 rows at a time
-    (3, 8388616, 8, False),           # ... and not all columns of a row
+    (3000, 4096, 64, True),           # by the engine's GEMM
+    (3, 8388616, 8, False),           # the least workspace does not take all columns of a row
 ])
 def test_sums_are_rounded_once(rows, cols, k, with_bias, in_place):
     """Small integers: every sum is exact in fp32, so the result is the exact one, rounded, whatever the workspace and the groups of
@@ -37,6 +38,33 @@ def test_sums_are_rounded_once(rows, cols, k, with_bias, in_place):
         res = r.clone()
         got = M().linear_bf16(x, w, b, residual=res, workspace=workspace, out=res if in_place else None)
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("in_place", [False, True])
+@pytest.mark.parametrize("with_bias", [True, False])
+@pytest.mark.parametrize("rows,cols,k", [
+    (4500, 4096, 320),                # 288 tiles in two rounds of 256: 2 048 rows at a time, the last group of 404
+    (3000, 4100, 64),                 # columns that the engine's GEMM does not take: 1 792 (of 2 046) and 1 208
+])
+def test_groups_of_rows_of_the_library_route(rows, cols, k, with_bias, in_place):
+    from longcat_video_amd import _capi
+    lib = _capi.load()
+    g = torch.Generator(device="cuda").manual_seed(44)
+    x, w, r = _integers(g, rows, k), _integers(g, cols, k), _integers(g, rows, cols) * 37
+    b = _integers(g, cols) * 5 if with_bias else None
+    want = x.float() @ w.float().t() + r.float()
+    if with_bias:
+        want += b.float()
+    out = r.clone() if in_place else torch.empty_like(r)
+    res = out if in_place else r
+    p = lambda t: None if t is None else t.data_ptr()      # noqa: E731
+    need = lib.bsa_linear_bf16_ld_workspace_bytes(p(x), k, p(w), k, p(b), p(res), p(out), cols, rows, cols, k)
+    assert need > (64 << 20) + rows * cols * 4      # the library's: room for the whole product
+    edge, room = 1 << 20, 64 << 20
+    around = torch.full((room + 2 * edge,), 0x5a, dtype=torch.uint8, device="cuda")
+    got = M().linear_bf16(x, w, b, residual=res, workspace=around[edge:edge + room], out=out)
+    assert torch.equal(got, want.bfloat16())
+    assert (around[:edge] == 0x5a).all() and (around[edge + room:] == 0x5a).all()
 
 
 def test_strided_rows():
@@ -56,7 +84,7 @@ def test_strided_rows():
 
 
 def test_equal_calls_are_equal_at_720p_size():
-    """The output projection of a 720p block, 2 000 times.  With the residual added by the library's product (beta = 1) one call in 550 to
+    """The output projection of a 720p block, 2 000 times (by the engine's GEMM, which serves it).  With the residual added by the library's product (beta = 1) one call in 550 to
     830 came out with wrong rows."""
     g = torch.Generator(device="cuda").manual_seed(43)
     rows, dim = 86400, 4096
