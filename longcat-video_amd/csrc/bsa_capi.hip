@@ -306,6 +306,7 @@ int bsa_fwd_fragment(const void* q, const void* k, const void* v, const int32_t*
     a.k.tile_norm = knorm + tile_norm_offset(B, Hn);
     a.v = prep_rows(v, kv_st);
     a.v.frag = vf;
+    a.k.few = a.v.few = frag_few((int64_t)B * Hn, Sq, Sk, nullptr);
     a.k.valid_in = a.v.valid_in = tile_valid;
     a.zero = reinterpret_cast<uint32_t*>(fallback);
     hipError_t e = launch_prepare(a, B, dtype, st);
@@ -555,6 +556,7 @@ hipError_t prepare_thw(const Plan& pl, const bsa_3d_params* p, const Ws& w, cons
         a.k.valid = padded_k ? w.valid : nullptr;
         a.v = prep_rows(v, v_strides);
         a.v.frag = static_cast<char*>(w.vp);
+        a.k.few = a.v.few = frag_few((int64_t)p->B * p->Hn, pl.Sqp, pl.Skp, &pl.gq);
         if (pool) {
             a.k.pooled = static_cast<uint16_t*>(w.kc);
             a.k.pooled_operand = operand_means;

@@ -285,9 +285,10 @@ struct PrepRows {
     int64_t cB, cH, cS;
     int split;
     int heads;                       // set by launch_prepare: heads of a chunk that a workgroup takes
-    char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order, the real slots of a tile first, zeros behind
+    char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order (bsa_fwd_frag.hip, bsa_fwd_round.hip), the real slots of a tile first, zeros behind
     uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
     int pooled_operand;              // k: ... in operand order instead (operand_mean_at)
+    int few;                         // k, v: the order is that of 32x32x16 products (frag_few)
     int32_t* rows;                   // q: row_table_ints() entries; the real slots of a chunk come first
     uint64_t* valid;                 // k, optional: bit s of word i = slot 64 i + s holds a real token
     const uint64_t* valid_in;        // k, v, optional: the real slots of every tile as the caller has them (instead of the grid's)
@@ -339,6 +340,8 @@ constexpr int kFragQueueWords = 16;
 size_t frag_part_floats(const Grid3& q_grid, int64_t heads);
 // Work items of a call, those of its last, partial round, and how these are shared: `parts` parts of an item, `team` wavefronts a part.
 struct LastRound { int total, items, team, parts; };
+// The fragment order of K and V that launch_fwd_frag reads: for a call of few items that of 32x32x16 products, otherwise of 16x16x32.
+bool frag_few(int64_t heads, int64_t Sq, int64_t Sk, const Grid3* q_grid);
 // Whether the attention kernel makes the lists of a call itself; then the chunk means of k are in operand order.
 bool frag_selects(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length, int nbk, int width);
 LastRound frag_last_round(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int idx_stride, const Grid3* halves_of, const Grid3* q_grid, bool one_length);

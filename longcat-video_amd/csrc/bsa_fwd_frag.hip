@@ -22,10 +22,11 @@
 //        order in which the accumulator registers of S^T hold them, so that P^T needs no shuffle.
 //
 // 16x16x32 and not 32x32x16: the board's power is what bounds this kernel, and the small form moves half as many
-// accumulators per multiplication (MFMAs alone on random data: 2 080 TFLOP/s against 1 820).
+// accumulators per multiplication (MFMAs alone on random data: 2 080 TFLOP/s against 1 820).  Calls that leave much of the chip
+// idle are not bound by it and go to bsa_fwd_round.hip (frag_few).
 //
-// Work decomposition.  One wavefront (a workgroup of 64 threads, one per SIMD; of small calls two or four,
-// see kTeam) = one work item =
+// Work decomposition.  One wavefront (a workgroup of 64 threads, one per SIMD; two or four where
+// they would be idle, see kTeam) = one work item =
 // 64 query rows against its list of KV blocks, walked in steps of 32 keys (half a tile).  Per
 // step: 32 MFMAs for S^T of the next step interleaved with the exp2 / row sum / rounding of the
 // current one, then 32 MFMAs for O^T += V^T P^T interleaved with the row maximum of the next.
@@ -37,20 +38,10 @@
 // bf16 a form that takes no maxima where the norms bound the logits (kBounded); numerics
 // follow flash_attn_bsa_varlen_mask.py:242-285: fp32 logits, scale * log2(e) applied after the
 // dot, exp2, P rounded to the storage type for the P V product, fp32 row sum, one final rounding.
-#include "bsa_gate.h"
-#include "bsa_mfma.h"
-
-#include <type_traits>
-#include <utility>
+#include "bsa_frag.h"
 
 namespace bsa {
 namespace {
-
-using namespace mfma;
-
-constexpr int kHalfBytes = 8192;      // 32 keys of a fragment-order K (or V) tile
-constexpr int kListEntries = 4096;    // longest list a work item can walk (its staging area in LDS: 17 KB)
-constexpr int kHalfEntries = 4096;    // ... of halves
 
 // ------------------------------------------------------------------ attention
 // acc + x[2e]^2 + x[2e+1]^2 for a fragment of eight 16-bit values
@@ -65,36 +56,9 @@ __device__ __forceinline__ float dot2_self(f16x8 x, int e, float acc) {
     return __builtin_amdgcn_fdot2(p, p, acc, false);
 }
 
-struct FragLayout {
-    const int32_t* q_rows;        // token row of every blocked-order query slot, -1 = padding; null: q, o in blocked order
-    int64_t q_st[3], o_st[3];     // element strides: batch, head, row
-    // The query tiles of one (batch, head) that hold real rows, n_live numbers (null: every tile): work item u is then tile
-    // tiles[u % n_live] of (batch, head) u / n_live.
-    const int32_t* tiles;
-    int n_live;
-    Divisor by_live, by_tiles, by_block, by_heads, by_sub;       // n_live; query tiles of a (batch, head), of a block; heads; tiles of a KV block
-};
-// The tile number (over all heads) of work item u.  The table was written by an earlier kernel and is read through the scalar
-// cache: the wait for it is its own, not one for every load of the wavefront, and all that is derived from it stays scalar.
-// (Asked for an item ahead with vector loads, at every turn of every call, it cost grids without such a table 70 of 8 500 us
-// at 32 heads of 720p.)
-__device__ __forceinline__ int item_at(const FragLayout& L, int u, int nqt) {
-    if (L.tiles == nullptr) return u;
-    const int bh = u / L.by_live;
-    return bh * nqt + *(const __attribute__((address_space(4))) int32_t*)(L.tiles + (u - bh * L.n_live));
-}
-
 // Lists of at most this many entries are staged in LDS for the next work item while the current one runs.
 constexpr int kPipeList = 256;
 
-// How an item's keys are listed (kWalk).  The walk goes in pairs of 32-key halves:
-//   kTiles:  idx holds KV blocks of one 64-key tile (bs_k == 64; no division in the walk), a pair is a tile;
-//   kBlocks: KV blocks of several tiles;
-//   kHalves: idx holds the halves themselves, empty ones left out: half of the (batch, head) | real keys << 20, an even
-//            number of entries (the last may repeat a half with no key), lens counts them without such a repeat.
-// The real keys of a tile come first (prepare_kernel), so its validity is a count.  Leaving out a half whose
-// probabilities would all be 0 changes no bit of the result: the sums run over the same numbers in the same order.
-//
 // A workgroup (one wavefront) runs the work items b, b + round, b + 2 round, ... of its launch one after the other
 // (or draws them from its XCD's queue).  What an item needs before its first MFMA - its list, its Q rows, its first K and
 // V fragments - is requested while the item before it still runs, so that an item costs its tile walk and an
@@ -111,20 +75,6 @@ constexpr int kPipeList = 256;
 // (see where the bound is tested): its steps take no row maxima.  An item that fails the test is not computed but
 // appended to `fallback` (its count in fallback_count), and the other instantiation, which takes its items from that
 // list, runs behind it.
-enum { kTiles, kBlocks, kHalves };
-constexpr uint32_t kHalfId = 0xfffff;     // of a kHalves entry: the half; above it: its number of real keys
-constexpr int kHalfCountShift = 20;
-
-// An item in parts: `count` wavefronts walk a share of its pairs each and leave the sums of their share (unnormalised
-// accumulators in register order, running maximum and row sum per query) in `buf`, kPartFloats per part; merge_parts_kernel
-// puts them together.  Part p of the launch's item i is its work item p * items + i.  count 1: whole items.
-constexpr int kPartFloats = kTile * kD + 2 * kTile;
-struct Parts {
-    float* buf;
-    int count, items;
-    Divisor by_count, by_items;
-};
-
 // The schedule for lists of unequal length: a queue per XCD.  Section x holds the items [section_begin(x), section_begin(x + 1))
 // of the call, a contiguous run of query tiles, and workgroup b draws from section b % 8, the XCD it runs on.
 constexpr int kQueues = 8, kQueueChoice = kQueues, kQueueWords = kQueues + 1;      // a counter per section, the choice of schedule
@@ -133,35 +83,13 @@ __device__ __forceinline__ int section_begin(int n, int x) { return (int)(((int6
 
 // kTeam: 0, one wavefront a workgroup, which runs one item after another as above; otherwise a workgroup runs one item, with
 // nothing prepared ahead and none of the code for it, as wavefronts that have a SIMD of a compute unit each.  1: a call of one
-// round (two prompts of 8 heads, 7x15x26: 40.0 -> 38.0 us).  2, 4: a team.  Each of its wavefronts walks a share of the item's pairs (of a part's
+// round.  2, 4: a team.  Each of its wavefronts walks a share of the item's pairs (of a part's
 // share, where the item is in parts as well) from the list that they stage together; then their sums are put together in LDS, in the
-// order of the shares, wavefront w those of its 4 / kTeam tiles of d, and the rows leave from all of them.  For calls of so few
-// items that most SIMDs would have none: see choose_split.
-template <int kTeam>
-constexpr int kTeamBytes = kTeam * (kTile * kD + 2 * kTile) * 4;      // the sums, maxima and row sums of every wavefront
-static_assert(kTeamBytes<4> <= 160 * 1024 && 2 * (kTeamBytes<2> + 512) <= 160 * 1024, "LDS of a compute unit with four wavefronts");
-
-// kGate: the item's list does not exist yet.  The workgroup makes it from the chunk means, as gate_kernel does (the same products and
-// roundings, the same lists), in front of its walk: the scores of its block against every key block, a share of 32 of them to a
-// wavefront at a time, then the first wavefront selects and orders.  Instead of another launch, its start and its end.
-// Whole operator, us, with gate_kernel in front / like this: 2 heads of 16x22x12 23.0 / 19.9, 4 of 9x13x10 30.2 / 26.3, two prompts of
-// 13 heads of 7x8x8 24.2 / 21.6, of 8 heads of 7x15x26 40.3 / 38.2.  `fallback` and `fallback_count` are then where the lists
-// ([BH][nbq][width]) and their lengths go, null: nowhere.  (As arguments of their own they would be 392 bytes, beyond what is asked for
-// together, and two arguments that the kernel can do without in their place cost the layers 0.3 to 0.7 %, by where the loop then lies.)
-struct FragGate {
-    const uint16_t *qc, *kc;         // chunk means, 16-bit storage; k's in operand order (operand_mean_at)
-    int nbk, width;                  // entries of a list: the top-k rule's count, the most of the CDF rule's
-    float threshold, scale;          // of the CDF rule, as cdf_count_kernel's; threshold 0: top-k
-    int k_min;
-    Divisor by_span;
-};
-constexpr int kGateWaveBlocks = 256, kGateMostBlocks = 512;      // key blocks that one wavefront scores, that a team does
-// LDS of the selection: the list of halves; scores; keys of every tile; where the first wavefront works; the list's length
-__host__ __device__ inline int gate_list_words(int width, int nsub, bool halves) { return halves ? (2 * width * nsub + 3) / 4 * 4 : 0; }
-__host__ __device__ inline int gate_here_bytes(int nbk, int width, int nsub, bool halves) {
-    return (gate_list_words(width, nsub, halves) + gate_wave_words(width) + 4) * 4 + (nbk + 31) / 32 * 64 + (halves ? (nbk * nsub + 15) / 16 * 16 : 0);
-}
-
+// order of the shares, wavefront w those of its 8 / kTeam tiles of d, and the rows leave from all of them.  For the items behind whole
+// rounds, and calls that teams of two fill the chip with: see choose_split.
+// kGate: the item's list does not exist yet (FragGate).  `fallback` and `fallback_count` are then where the lists ([BH][nbq][width]) and their
+// lengths go, null: nowhere.  (As arguments of their own they would be 392 bytes, beyond what is asked for together, and two arguments that
+// the kernel can do without in their place cost the layers 0.3 to 0.7 %, by where the loop then lies.)
 // The first of a step's 96 pieces (six a pair, nine instructions' time) that stands behind MFMA g or a later one, in the kernel with maxima.
 constexpr int first_piece(int g) {
     for (int p = 0; p < 96; ++p) {
@@ -173,7 +101,9 @@ constexpr int first_piece(int g) {
 }
 
 template <typename T, int kWalk, bool kBounded, int kTeam, bool kGate>
-__global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kernel(
+// At a page: the queues' kernel, the same instructions, took 1 252 us of a call (16 heads of 20x30x52 by the CDF rule) at 0x500 of one and 1 245 at
+// its start, where the linker had put it until other kernels left this file.  Level elsewhere.
+__attribute__((aligned(4096))) __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
     const int32_t* __restrict__ idx, const int32_t* __restrict__ lens, const uint64_t* __restrict__ tile_valid,
     T* __restrict__ o, float* __restrict__ lse, int64_t Sq, int64_t Sk, int bs_q, int bs_k, int idx_stride,
@@ -696,96 +626,8 @@ __global__ __launch_bounds__(kTeam > 1 ? 64 * kTeam : 64, 1) void fwd_frag_kerne
                     if (lane_now + 64 * e < nent) big[lane_now + 64 * e] = (uint32_t)entry[e];
                 for (int e = lane_now + 64 * kAhead; e < nent; e += 64) big[e] = (uint32_t)list[e];
             } else if constexpr (kGate) {
-                char* const work = ost_bytes;
-                const int words = gate_list_words(G.width, nsub_of_block, kWalk == kHalves);
-                int32_t* const halves_list = reinterpret_cast<int32_t*>(work);
-                uint32_t* const mine = reinterpret_cast<uint32_t*>(work) + words;
-                int* const total_at = reinterpret_cast<int*>(mine + gate_wave_words(G.width));
-                T* const scores = reinterpret_cast<T*>(total_at + 4);
-                uint8_t* const counts = reinterpret_cast<uint8_t*>(scores + (G.nbk + 31) / 32 * 32);
-                const int64_t brow = cur.item / L.by_block;
-                if (kWalk == kHalves)
-                    for (int i = threadIdx.x; i < G.nbk * nsub_of_block; i += 64 * kTeam) counts[i] = (uint8_t)__popcll(tile_valid[i]);
-                const int lr = lane & 31, lh = lane >> 5;
-                const T* const qm = reinterpret_cast<const T*>(G.qc) + brow * kD + lh * 8;      // its mean as every row of the product
-                // k's means in whole kilobytes; as rows of 256 bytes a load took 32 bytes of each of 32
-                const T* const km = reinterpret_cast<const T*>(G.kc) + operand_mean_at(bh, G.nbk, 0, 0) + lane * 8;
-                V8 qa[8];
-#pragma unroll
-                for (int c = 0; c < 8; ++c) qa[c] = *reinterpret_cast<const V8*>(qm + 16 * c);
-                // four of this wavefront's blocks of 32 are on their way at a time
-                for (int n_first = 32 * wave; n_first < G.nbk; n_first += 4 * 32 * kTeam) {
-                    V8 kr[4][8];
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const int n0 = n_first + 32 * kTeam * t;
-                        if (n0 < G.nbk) {
-                            const T* const kt = km + n0 / 32 * 4096;
-#pragma unroll
-                            for (int c = 0; c < 8; ++c) kr[t][c] = *reinterpret_cast<const V8*>(kt + 512 * c);
-                        }
-                    }
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const int n0 = n_first + 32 * kTeam * t;
-                        if (n0 < G.nbk) {
-                            f32x16 acc;
-#pragma unroll
-                            for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-                            for (int c = 0; c < 8; ++c) acc = mfma32(qa[c], kr[t][c], acc);
-                            if (lh == 0) scores[n0 + lr] = (T)acc[0];
-                        }
-                    }
-                }
-                __syncthreads();
-                if (wave == 0) {
-                    const uint16_t* const raw = reinterpret_cast<const uint16_t*>(scores);
-                    int32_t* const list = reinterpret_cast<int32_t*>(mine);
-                    auto select = [&](auto n_c) -> int {                 // by columns to a lane
-                        constexpr int kPerLane = decltype(n_c)::value;
-                        uint32_t val[kPerLane];
-#pragma unroll
-                        for (int j = 0; j < kPerLane; ++j) {
-                            const int i = j * 64 + lane;
-                            const uint16_t x = raw[min(i, G.nbk - 1)];
-                            val[j] = i < G.nbk ? ord_of(x) : 0u;
-                        }
-                        int n = G.width;
-                        if (G.threshold > 0.f) {
-                            float e[kPerLane];
-#pragma unroll
-                            for (int j = 0; j < kPerLane; ++j) e[j] = j * 64 + lane < G.nbk ? (float)scores[min(j * 64 + lane, G.nbk - 1)] : -INFINITY;
-                            n = cdf_row<16>(val, e, lane, G.nbk, G.threshold, G.scale, G.k_min, G.width);
-                        }
-                        if (n > 0) select_row<uint16_t, kPerLane, false>(val, [&](int i) { return raw[i]; }, lane, G.nbk, n, nullptr, list, nullptr, mine);
-                        return n;
-                    };
-                    int k_sel;
-                    if (G.nbk <= 64) k_sel = select(std::integral_constant<int, 1>{});
-                    else if (G.nbk <= 128) k_sel = select(std::integral_constant<int, 2>{});
-                    else if (kTeam == 1 || G.nbk <= 256) k_sel = select(std::integral_constant<int, 4>{});
-                    else k_sel = select(std::integral_constant<int, 8>{});
-                    int32_t* const dst = fallback != nullptr ? fallback + brow * G.width : nullptr;
-                    wave_sync();
-                    const int32_t* order_here = list;
-                    if (k_sel > kPaceWidth) order_here = pace_row(list, k_sel, k_sel, G.nbk, lane, dst, G.by_span);
-                    else if (dst != nullptr)
-                        for (int e = lane; e < k_sel; e += 64) dst[e] = list[e];
-                    if (dst != nullptr)
-                        for (int e = k_sel + lane; e < G.width; e += 64) dst[e] = -1;
-                    if (fallback_count != nullptr && lane == 0) fallback_count[brow] = (uint32_t)k_sel;
-                    int total = k_sel;
-                    if constexpr (kWalk == kHalves) total = expand_list(order_here, k_sel, nsub_of_block, halves_list, lane, [&](int tile) { return (int)counts[tile]; });
-                    if (lane == 0) {
-                        total_at[0] = total;
-                        total_at[1] = (int)(order_here - list);
-                    }
-                }
-                __syncthreads();
-                cur.nent = total_at[0];
+                ents = make_list<T, kTeam, kWalk == kHalves>(G, ost_bytes, cur.item / L.by_block, bh, nsub_of_block, tile_valid, fallback, fallback_count, lane, wave, cur.nent);
                 nent = list_length(cur);
-                ents = kWalk == kHalves ? reinterpret_cast<const uint32_t*>(halves_list) : mine + uni(total_at[1]);
                 if (kTeam == 1) npairs = uni(kWalk == kHalves ? nent >> 1 : nent * nsub);
             } else {
                 if ((int)threadIdx.x < nent) big[threadIdx.x] = (uint32_t)team_entry;
@@ -1434,9 +1276,21 @@ static Split choose_split(int items, int list_tiles, int resident, bool is_tail,
         }
     return best;
 }
+// Calls of so few items that SIMDs are left over run fwd_round_kernel, whose 32x32x16 products leave a wavefront more of its issue; where nearly
+// all are busy the board's power is the bound again.  Whole operator in us, this file's kernel / that one, items x tiles: with a wavefront an item
+// 640 x 20 53.7 / 50.3, x 80 140.6 / 130.0, 768 x 64 118.0 / 116.4, 800 x 20 56.9 / 56.9, x 80 145.5 / 145.2, 832 x 104 183.3 / 185.6, 896 x 64
+// 126.2 / 128.9, 1 024 x 128 246.8 / 255.9; teams of two 384 x 64 70.6 / 69.0, 416 x 104 101.5 / 101.3, 448 x 112 111.4 / 113.0, 512 x 128
+// 133.9 / 137.8; teams of four 128 x 64 43.6 / 39.6, 176 x 88 54.8 / 50.6, 208 x 104 61.0 / 60.0, 256 x 128 77.8 / 78.2.  So the line lies at
+// 800 wavefronts, counted in full teams of two (of four it is level up to the most), and by the items alone, because K and V are prepared
+// before the length of the lists, and with it the team, need be known (bsa_thw_prepare).
+constexpr int kBusyWide = 800;
+bool frag_few(int64_t heads, int64_t Sq, int64_t Sk, const Grid3* q_grid) {
+    const int64_t items = heads * (q_grid != nullptr ? live_query_tiles(*q_grid) : Sq / kTile);
+    return heads * (Sk / kTile) * (int64_t)kTileBytes < ((int64_t)1 << 32) && (items <= kBusyWide / 2 || (items > kMostResident / 2 && items <= kBusyWide));
+}
 struct Rounds {
     int heads_per_span;              // (batch, head)s that one buffer of K reaches
-    bool one_span;
+    bool one_span, few;
     int n_live, total, resident, list_tiles, tail;
     Split split;
 };
@@ -1458,7 +1312,9 @@ static Rounds plan_rounds(int64_t heads, int64_t Sq, int64_t Sk, int bs_k, int i
     // kernel reaches every head from one buffer); behind whole rounds and into parts only for lists of one length.
     r.tail = r.total % r.resident;
     r.split = {1, 1};
-    if (r.one_span && r.tail > 0 && (one_length || r.total < r.resident))
+    // (frag_few goes by the whole chip: on a part of it such a call may have more than one round, which is not cut)
+    r.few = frag_few(heads, Sq, Sk, q_grid);
+    if (r.one_span && r.tail > 0 && (r.total < r.resident || (one_length && !r.few)))
         r.split = choose_split(r.tail, r.list_tiles, r.resident, r.total > r.resident, one_length, halves_of);
     return r;
 }
@@ -1504,7 +1360,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     const int64_t kv_bh_bytes = (Sk / kTile) * (int64_t)kTileBytes;
     if (kv_bh_bytes > ((int64_t)1 << 32) - 1) return hipErrorInvalidValue;
     // a buffer for parts comes with lists of one length
-    const auto [heads_per_span, one_span, n_live, total, resident, list_tiles, tail, split] =
+    const auto [heads_per_span, one_span, few, n_live, total, resident, list_tiles, tail, split] =
         plan_rounds((int64_t)B * Hn, Sq, Sk, bs_k, idx_stride, halves_of, q_grid, part_buf != nullptr);
     L.tiles = n_live < per_head ? q_rows + Sq : nullptr;
     L.n_live = n_live;
@@ -1521,7 +1377,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     // the items it has to leave to the other kernel is given, and that kernel can reach every head from one buffer.
     // A short call runs the exact kernel alone: its steps are 3 % longer, but a last launch that finds nothing to do costs 4.7 us.
     Parts parts = {nullptr, 1, 0, divisor(1), divisor(1)};
-    const bool bounded = dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident &&
+    const bool bounded = !few && dtype == BSA_BF16 && key_norm != nullptr && fallback != nullptr && one_span && total > resident &&
                          (int64_t)total * list_tiles > (int64_t)kExactRoundTiles * resident;
     uint32_t* fb_count = bounded ? reinterpret_cast<uint32_t*>(fallback) : nullptr;
     int32_t* fb_list = bounded ? fallback + 64 : nullptr;
@@ -1543,17 +1399,21 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, BD, 0, false, __VA_ARGS__);                                   \
         else BSA_FRAG_LAUNCH_W(_Float16, false, 0, false, __VA_ARGS__);                                                \
     } while (0)
+#define BSA_FRAG_LAUNCH_LISTED(TEAM, ...)                                                                              \
+    do {                                                                                                               \
+        if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, false, __VA_ARGS__);                             \
+        else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, false, __VA_ARGS__);                                             \
+    } while (0)
 #define BSA_FRAG_LAUNCH_ONCE(TEAM, ...)                                                                                \
     do {                                                                                                               \
         if (here.qc != nullptr) {                                                                                      \
             if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, true, __VA_ARGS__);                          \
             else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, true, __VA_ARGS__);                                          \
         } else {                                                                                                       \
-            if (dtype == BSA_BF16) BSA_FRAG_LAUNCH_W(__bf16, false, TEAM, false, __VA_ARGS__);                         \
-            else BSA_FRAG_LAUNCH_W(_Float16, false, TEAM, false, __VA_ARGS__);                                         \
+            BSA_FRAG_LAUNCH_LISTED(TEAM, __VA_ARGS__);                                                                 \
         }                                                                                                              \
     } while (0)
-    const bool once = one_span && total <= resident && (split.team > 1 || split.parts == 1);
+    const bool once = few || (one_span && total <= resident && (split.team > 1 || split.parts == 1));
     if (gate_call != nullptr) {
         const GateCall& c = *gate_call;
         if (c.inside) {
@@ -1570,7 +1430,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     }
     if (bounded && !fallback_cleared) hipLaunchKernelGGL(frag_zero_kernel, dim3(1), dim3(64), 0, st, fb_count, 1);
     // Lists of unequal length of one round need no plan: every item has a wavefront of its own from the start.
-    if (queue != nullptr && one_span && total > resident) {
+    if (queue != nullptr && one_span && total > resident && !few) {
         hipLaunchKernelGGL(queue_plan_kernel, dim3(kQueues + 1), dim3(kPlanThreads), 0, st, lens, per_head, L, total, resident, idx_stride,
                            order, queue);
         gate = queue + kQueueChoice;
@@ -1601,7 +1461,11 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
         const int n = (total - whole) * split.parts;
         const dim3 grid((unsigned)(split.team == 1 && n > resident ? resident : n));
 #define BSA_FRAG_TAIL grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, gate_lists, gate_lens
-        if (split.team == 4) BSA_FRAG_LAUNCH_ONCE(4, BSA_FRAG_TAIL);
+        if (few) {
+            const FragCall c = {q, kf, vf, idx, lens, tile_valid, o, lse, Sq, Sk, lse_rows, bs_k, idx_stride, Hn, dtype, qk_scale, halves, st};
+            const hipError_t e = launch_fwd_round(c, L, parts, total, split.team, here.qc != nullptr ? &here : nullptr, gate_lists, gate_lens, whole_span);
+            if (e != hipSuccess) return e;
+        } else if (split.team == 4) BSA_FRAG_LAUNCH_LISTED(4, BSA_FRAG_TAIL);      // 4 x more than kBusyWide / 2 items are not one round: no selection inside
         else if (split.team == 2) BSA_FRAG_LAUNCH_ONCE(2, BSA_FRAG_TAIL);
         else if (once) BSA_FRAG_LAUNCH_ONCE(1, BSA_FRAG_TAIL);
         else BSA_FRAG_LAUNCH(false, BSA_FRAG_TAIL);
@@ -1623,6 +1487,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
     }
 #undef BSA_FRAG_LAUNCH
 #undef BSA_FRAG_LAUNCH_ONCE
+#undef BSA_FRAG_LAUNCH_LISTED
 #undef BSA_FRAG_LAUNCH_W
 #undef BSA_FRAG_LAUNCH_T
     return hipGetLastError();

@@ -12,6 +12,8 @@
 #include "bsa_rope.h"
 #include "bsa_slots.h"
 
+#include <type_traits>
+
 namespace bsa {
 namespace {
 
@@ -285,9 +287,10 @@ __device__ __forceinline__ void row_part(const PrepRows& x, const Grid3& g, int 
         if (x.frag != nullptr) {
             __syncthreads();
             char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
-            // 16-byte piece tid + 256 i of the output: lane l of fragment w + 4 i, which is key half i / 2, d chunk w / 2 + 2 (i % 2), its 16 keys w % 2
+            // 16-byte piece tid + 256 i of the output: lane l of fragment w + 4 i, which is key half i / 2 and, of 16 keys x 32 d, d chunk
+            // w / 2 + 2 (i % 2), its keys w % 2; of 32 keys x 16 d (few) d chunk w + 4 (i % 2)
             const int l = tid & 63, w = tid >> 6;
-            const uint16_t* p = tile + (16 * (w & 1) + (l & 15)) * kPitchK + 32 * (w >> 1) + 8 * (l >> 4);
+            const uint16_t* p = tile + (x.few ? (l & 31) * kPitchK + 16 * w + 8 * (l >> 5) : (16 * (w & 1) + (l & 15)) * kPitchK + 32 * (w >> 1) + 8 * (l >> 4));
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const uint16_t* at = p + 32 * (i >> 1) * kPitchK + 64 * (i & 1);
@@ -349,16 +352,21 @@ __device__ __forceinline__ void value_part(const PrepRows& x, const Grid3& g, in
     __syncthreads();
     char* out = x.frag + ((int64_t)bh * tiles + tile_id) * kTileBytes;
     // ds_read_b64_tr_b16: the 16 lanes of a group point at a 4-key x 16-d patch (lane s at key s / 4,
-    // d 4 (s % 4) .. + 4) and each receives the 4 keys of one d.  Piece threadIdx.x + 256 i: lane l of fragment w + 4 i, key half i / 2, d tile w + 4 (i % 2)
+    // d 4 (s % 4) .. + 4) and each receives the 4 keys of one d.  Piece threadIdx.x + 256 i: lane l of fragment w + 4 i, key half i / 2,
+    // d tile w + 4 (i % 2) of 16, or (few) key step i % 2, d tile w of 32
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const uint16_t* from = tile + (4 * (l >> 4) + ((l & 15) >> 2)) * kPitchV + 16 * w + 4 * (l & 3);
+    auto write = [&](const uint16_t* from, auto odd, auto upper) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint16_t* at = from + 32 * (i >> 1) * kPitchV + 64 * (i & 1);
-        const s16x4 lo = lds_read_tr16(at), hi = lds_read_tr16(at + 16 * kPitchV);
-        typedef short s16x8_ __attribute__((ext_vector_type(8)));
-        *reinterpret_cast<s16x8_*>(out + (int64_t)(threadIdx.x + 256 * i) * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-    }
+        for (int i = 0; i < 4; ++i) {
+            const uint16_t* at = from + 32 * (i >> 1) * kPitchV + (i & 1) * odd;
+            const s16x4 lo = lds_read_tr16(at), hi = lds_read_tr16(at + upper);
+            typedef short s16x8_ __attribute__((ext_vector_type(8)));
+            *reinterpret_cast<s16x8_*>(out + (int64_t)(threadIdx.x + 256 * i) * 16) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    };
+    const int key = (l & 15) >> 2, d = 4 * (l & 3);
+    if (x.few) write(tile + (4 * (l >> 5) + key) * kPitchV + 32 * w + 16 * (l >> 4 & 1) + d, std::integral_constant<int, 16 * kPitchV>{}, std::integral_constant<int, 8 * kPitchV>{});
+    else write(tile + (4 * (l >> 4) + key) * kPitchV + 16 * w + d, std::integral_constant<int, 64>{}, std::integral_constant<int, 16 * kPitchV>{});
 }
 
 // Chunk means and row table of q, nothing else of it: a wavefront per chunk, no LDS, all of a lane's sixteen 16-byte loads
