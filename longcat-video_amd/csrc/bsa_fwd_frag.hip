@@ -30,7 +30,7 @@
 // 64 query rows against its list of KV blocks, walked in steps of 32 keys (half a tile).  Per
 // step: 32 MFMAs for S^T of the next step interleaved with the exp2 / row sum / rounding of the
 // current one, then 32 MFMAs for O^T += V^T P^T interleaved with the row maximum of the next.
-// K and V fragments of the following steps are in flight in register rings (kRing steps each).
+// K and V fragments of the following steps are in flight in register rings (two steps each).
 // The output accumulators (128 registers) and the rings live in the 512-register file that a
 // single wavefront per SIMD has to itself.
 //
@@ -259,8 +259,8 @@ __attribute__((aligned(4096))) __global__ __launch_bounds__(kTeam > 1 ? 64 * kTe
     float alpha_p[4];
     bool rescale_pending = false;
 
-    // Q fragments of 16 queries into their registers, and the lane's part of the rows' squared norms.  The queries 32 .. 63 are
-    // read by the assembly MFMAs from accumulation registers.  Their values pass through an assembly statement that
+    // Q fragments of 16 queries into their registers, and the lane's part of the rows' squared norms.  All of Q is
+    // read by the assembly MFMAs from accumulation registers.  The values pass through an assembly statement that
     // ties them to that register class: a value that C++ code also reads (the squares) the compiler would keep in
     // ordinary registers and copy in front of every MFMA that names it, without the wait states such a copy needs.
     float q_sq[4] = {0.f, 0.f, 0.f, 0.f};
@@ -482,11 +482,11 @@ __attribute__((aligned(4096))) __global__ __launch_bounds__(kTeam > 1 ? 64 * kTe
                 mfma_acc16(oacc[slot][3], vb[vprev][slot], pb[3]);
             } else if constexpr (slot < 24) {
                 constexpr int f = (slot - 8) >> 1, c = f >> 1, kk = f & 1, qb = 2 * (slot & 1);      // d step, key block
-                mfma_s16<c == 0, true>(s[sn][kk][qb], kb[kslot][f], qreg[qb][c]);
+                mfma_s16<c == 0>(s[sn][kk][qb], kb[kslot][f], qreg[qb][c]);
                 __builtin_amdgcn_sched_barrier(0);
                 gap(std::integral_constant<int, 2 * slot>{});
                 __builtin_amdgcn_sched_barrier(0);
-                mfma_s16<c == 0, true>(s[sn][kk][qb + 1], kb[kslot][f], qreg[qb + 1][c]);
+                mfma_s16<c == 0>(s[sn][kk][qb + 1], kb[kslot][f], qreg[qb + 1][c]);
             } else {
                 constexpr int t = slot - 24;
                 mfma_acc16(oacc[t][0], vb[vcur][t], pb[0]);
@@ -741,8 +741,8 @@ __attribute__((aligned(4096))) __global__ __launch_bounds__(kTeam > 1 ? 64 * kTe
             for (int f = 0; f < 8; ++f)
 #pragma unroll
                 for (int qb = 0; qb < 4; ++qb) {
-                    if (f < 2) mfma_s16<true, true>(s[0][f & 1][qb], kb[0][f], qreg[qb][f >> 1]);
-                    else mfma_s16<false, true>(s[0][f & 1][qb], kb[0][f], qreg[qb][f >> 1]);
+                    if (f < 2) mfma_s16<true>(s[0][f & 1][qb], kb[0][f], qreg[qb][f >> 1]);
+                    else mfma_s16<false>(s[0][f & 1][qb], kb[0][f], qreg[qb][f >> 1]);
                 }
 #pragma unroll
             for (int c = 0; c < 8; ++c) kb[0][c] = k_frag(offset_of(w[1]), c);              // K(2), behind the last reader of K(0)

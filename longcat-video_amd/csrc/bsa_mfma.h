@@ -25,9 +25,6 @@ __device__ inline f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
 __device__ inline f32x4_ mfma16(bf16x8 a, bf16x8 b, f32x4_ c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-__device__ inline f32x4_ mfma16(f16x8 a, f16x8 b, f32x4_ c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-}
 template <typename T> struct Vec8;
 template <> struct Vec8<__bf16> { typedef bf16x8 type; };
 template <> struct Vec8<_Float16> { typedef f16x8 type; };
@@ -95,17 +92,17 @@ __device__ __forceinline__ s16x4 lds_read_tr16_at(uint32_t address) {
 // output accumulators belong in AGPRs.  For a kernel that may use more than 256 registers the compiler puts
 // the result of every builtin MFMA into AGPRs, so the S^T MFMAs are written as inline assembly with VGPR
 // operands.  The compiler does not see that such a statement is an MFMA and adds no wait states behind it:
-// the code keeps every VALU access to these accumulators at least eight MFMAs (256 clocks) behind the MFMA
-// that writes them, or puts explicit s_nop there.
+// the code keeps every VALU access to these accumulators at least 64 clocks of MFMAs - two of 32x32x16, four of 16x16x32 -
+// behind the MFMA that writes them, or puts explicit s_nop there.  (A result of eight passes, 32x32x16, may be read after 12 wait
+// states of four clocks, one of four passes, 16x16x32, after 8.)
 // The register allocator sees such a statement as an ordinary instruction that is complete when issued.  If the
 // result were dead behind the last statement of a chain (a timing build that compiles the consumer out, say), the
 // allocator could hand the registers to something else - an address, a loaded value - while the MFMA, whose
 // passes run for another 32 clocks and more, still writes them: the new value is overwritten, and an overwritten
 // address is a memory fault.  mfma_chain_end() (below) costs no instruction and ties the accumulators as live up
 // to the place where it stands; every chain is closed with one, placed where the distance rule above holds.
-// kAgprB: the B operand (the Q fragment) lives in an AGPR.  The queries 32 .. 63 of a work item are kept there,
-// the queries 0 .. 31 in VGPRs, which balances the two register files (VGPR: S^T, P^T, the K ring, half of Q;
-// AGPR: the output accumulators, the V ring, the other half of Q).
+// kAgprB: the B operand lives in an AGPR (fwd_round_kernel: the Q fragments of the queries 32 .. 63 of a work item; those of the queries
+// 0 .. 31 are in VGPRs, which balances the two register files).
 template <bool kFirst, bool kAgprB>
 __device__ inline void mfma_s(f32x16& acc, bf16x8 a, bf16x8 b) {
     if (kFirst) {
@@ -127,26 +124,16 @@ __device__ inline void mfma_s(f32x16& acc, f16x8 a, f16x8 b) {
     }
 }
 
-// The same for 16x16x32 products.
-template <bool kFirst, bool kAgprB>
+// The same for 16x16x32 products, B in AGPRs (fwd_frag_kernel: all of Q).
+template <bool kFirst>
 __device__ inline void mfma_s16(f32x4_& acc, bf16x8 a, bf16x8 b) {
-    if (kFirst) {
-        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
-        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
-    } else {
-        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
-        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
-    }
+    if (kFirst) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
+    else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
 }
-template <bool kFirst, bool kAgprB>
+template <bool kFirst>
 __device__ inline void mfma_s16(f32x4_& acc, f16x8 a, f16x8 b) {
-    if (kFirst) {
-        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
-        else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "v"(b));
-    } else {
-        if (kAgprB) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
-        else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
-    }
+    if (kFirst) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, 0" : "=&v"(acc) : "v"(a), "a"(b));
+    else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "a"(b));
 }
 
 // An accumulation into AGPRs, in place: with the builtin, whose result may lie elsewhere than what it adds to, the compiler put 32
@@ -173,7 +160,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 
 // Marks the end of a chain of assembly MFMAs into `acc`: from here on the accumulators may be read, written or
 // reused.  Emits nothing; it only keeps `acc` allocated, and unchanged, between the chain's last MFMA and this
-// point, which the caller places at least eight MFMAs (or the equivalent s_nop) behind that MFMA.
+// point, which the caller places 64 clocks of MFMAs (two of 32x32x16, four of 16x16x32) or the equivalent s_nop behind that MFMA.
 __device__ __forceinline__ void mfma_chain_end(f32x16& acc) { asm volatile("" : "+v"(acc)); }
 __device__ __forceinline__ void mfma_chain_end(f32x4_& acc) { asm volatile("" : "+v"(acc)); }
 
