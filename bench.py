@@ -38,7 +38,7 @@ ATTENTION_KERNEL = "fwd_frag_kernel<bf16> (all launches of one layer)"
 # what the attention kernel's traffic depends on: the kernel and its helpers, the visiting order of the lists it walks,
 # and the layer that decides rounds per launch and whether the visiting order runs
 ATTENTION_SOURCES = [os.path.join(ROOT, "longcat-video_amd", "csrc", f)
-                     for f in ("bsa_fwd_frag.hip", "bsa_select.hip", "bsa_mfma.h", "bsa_common.h", "bsa_capi.hip")]
+                     for f in ("bsa_fwd_frag.hip", "bsa_frag.h", "bsa_select.hip", "bsa_mfma.h", "bsa_common.h", "bsa_capi.hip")]
 
 
 def source_sha16(paths=ATTENTION_SOURCES):

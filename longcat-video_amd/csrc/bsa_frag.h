@@ -1,5 +1,5 @@
-// What the two attention kernels on fragment-order K and V (bsa_fwd_frag.hip: calls of whole rounds; bsa_fwd_round.hip: calls of less
-// than one) have in common: their items, how the keys of an item are listed, items in parts, and a list made in front of its walk.
+// What the two attention kernels on fragment-order K and V (bsa_fwd_frag.hip; bsa_fwd_round.hip: calls that leave SIMDs
+// idle) have in common: their items, how the keys of an item are listed, items in parts, and a list made in front of its walk.
 #pragma once
 #include "bsa_gate.h"
 #include "bsa_mfma.h"
@@ -33,7 +33,8 @@ struct Parts {
 // roundings, the same lists), in front of its walk: the scores of its block against every key block, a share of 32 of them to a
 // wavefront at a time, then the first wavefront selects and orders.  Instead of another launch, its start and its end.
 // Whole operator, us, with gate_kernel in front / like this: 2 heads of 16x22x12 23.0 / 19.9, 4 of 9x13x10 30.2 / 26.3, two prompts of
-// 13 heads of 7x8x8 24.2 / 21.6, of 8 heads of 7x15x26 40.3 / 38.2.  The lists ([BH][nbq][width]) and their lengths also go to memory where they are wanted.
+// 13 heads of 7x8x8 24.2 / 21.6, of 8 heads of 7x15x26 40.3 / 38.2.  The lists ([BH][nbq][width]) and
+// their lengths also go to memory where they are wanted.
 struct FragGate {
     const uint16_t *qc, *kc;         // chunk means, 16-bit storage; k's in operand order (operand_mean_at)
     int nbk, width;                  // entries of a list: the top-k rule's count, the most of the CDF rule's
@@ -99,7 +100,7 @@ __host__ __device__ inline int gate_here_bytes(int nbk, int width, int nsub, boo
     return (gate_list_words(width, nsub, halves) + gate_wave_words(width) + 4) * 4 + (nbk + 31) / 32 * 64 + (halves ? (nbk * nsub + 15) / 16 * 16 : 0);
 }
 
-// The list of `item`, of block row `row`, in LDS (`work`, gate_here_bytes), its length in `length`.  By all threads of the workgroup, with a
+// The list of an item, of block row `row`, in LDS (`work`, gate_here_bytes), its length in `length`.  By all threads of the workgroup, with a
 // barrier at the end.
 template <typename T, int kTeam, bool kHalfLists>
 __device__ __forceinline__ const uint32_t* make_list(const FragGate& G, char* work, int64_t row, int bh, int nsub, const uint64_t* tile_valid, int32_t* lists,

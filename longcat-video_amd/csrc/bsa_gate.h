@@ -1,5 +1,5 @@
 // One score row's selection and visiting order by a wavefront: what the gating kernels (bsa_select.hip) and the attention kernel
-// of small calls, which selects for itself (bsa_fwd_frag.hip), have in common.
+// of small calls, which selects for itself (bsa_frag.h), have in common.
 #pragma once
 #include "bsa_common.h"
 

@@ -44,11 +44,12 @@
 // the epilogue (two loads a lane, whose wait falls into a phase) cost more than they save: 823 -> 842 with a residual.
 //
 // What bounds it: power, and the reading half of a phase.  Per k block and group 610 clocks to request 32 KB (the address unit of a
-// CU takes 16 a load of 1 KB, and a wavefront issues in order) and 500 to read 96 KB of fragments, against 1 009 of MFMAs, so the
-// MFMAs run 0.76 of the clocks at 1.87 GHz.  Measured and not kept: the requests between the fragment reads (R 1 170 clocks)
+// CU takes 16 a load of 1 KB, and a wavefront issues in order) and 500 to read 96 KB of fragments, against 1 009 of MFMAs (an
+// instrumented build).  By counters the MFMAs run 0.74 of the clocks at 1.72 GHz with a residual, 86 400 x 4 096 x 4 096, and 0.73 at 1.67 with the
+// QKV epilogue, without a bank conflict.  Measured and not kept: the requests between the fragment reads (R 1 170 clocks)
 // or between the MFMAs (both wait for the address unit: 0.66-0.70), MFMAs behind the barrier of a phase, with and without priority (0.75),
 // an L2 prefetch three to eight blocks ahead (1-2 % slower), one barrier a k block with the groups half a block apart (0.54-0.74).
-// hipBLASLt's kernel for the QKV shape reaches 0.80 at 1.80 GHz.
+// hipBLASLt's kernel for the QKV shape runs 0.87 of its clocks at 1.53 GHz in the same runs.
 #include "bsa_mfma.h"
 
 #include <algorithm>

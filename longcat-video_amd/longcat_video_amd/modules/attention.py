@@ -358,6 +358,7 @@ class Attention(nn.Module):
         if any(b.use_lora for b in loras):
             from .lora import lora_linear
             # q and k choose the blocks: rounded once, with a side branch inside the product, near ties would fall differently than eager
+            # (v chooses none, but is a third of the same product)
             y = lora_linear(x, layer.weight, layer.bias, loras, None, one_rounding=layer is not self.qkv)
             return y if residual is None else y + residual
         if self._engine_gemm(layer):
