@@ -21,7 +21,7 @@ OUT_DIR = os.path.join(HERE, "longcat_video_amd", "lib")
 LIB = os.path.join(OUT_DIR, "libbsa_mi355x.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
-SOURCES = ["bsa_capi.hip", "bsa_permute.hip", "bsa_prepare.hip", "bsa_select.hip", "bsa_fwd.hip", "bsa_fwd_frag.hip", "bsa_fwd_round.hip", "bsa_f32.hip", "bsa_bwd.hip", "bsa_glue.hip", "bsa_lora.hip", "bsa_gemm.hip"]
+SOURCES = ["bsa_capi.hip", "bsa_permute.hip", "bsa_prepare.hip", "bsa_select.hip", "bsa_fwd.hip", "bsa_fwd_frag.hip", "bsa_fwd_few.hip", "bsa_f32.hip", "bsa_bwd.hip", "bsa_glue.hip", "bsa_lora.hip", "bsa_gemm.hip"]
 # The attention kernel never produces a NaN by construction (the -inf cases are guarded), so its
 # maxima need no NaN-quieting extra instructions.  Infinities keep their IEEE meaning.
 # The glue and LoRA kernels restate eager fp32 expressions (x * cos + rot * sin, x * (scale + 1) + shift, x + gate * y)
@@ -29,7 +29,7 @@ SOURCES = ["bsa_capi.hip", "bsa_permute.hip", "bsa_prepare.hip", "bsa_select.hip
 # The fragment pass and the GEMM epilogue share those expressions (bsa_rope.h) beside code that wants its FMAs:
 # contraction stays on for the file and the shared functions switch it off with a pragma, which the compiler only
 # honours under fast-honor-pragmas.
-EXTRA_FLAGS = {"bsa_fwd.hip": ["-fno-honor-nans"], "bsa_fwd_frag.hip": ["-fno-honor-nans"], "bsa_fwd_round.hip": ["-fno-honor-nans"], "bsa_prepare.hip": ["-ffp-contract=fast-honor-pragmas"],
+EXTRA_FLAGS = {"bsa_fwd.hip": ["-fno-honor-nans"], "bsa_fwd_frag.hip": ["-fno-honor-nans"], "bsa_fwd_few.hip": ["-fno-honor-nans"], "bsa_prepare.hip": ["-ffp-contract=fast-honor-pragmas"],
                "bsa_bwd.hip": ["-fno-honor-nans"], "bsa_glue.hip": ["-ffp-contract=off"], "bsa_lora.hip": ["-ffp-contract=off"],
                "bsa_gemm.hip": ["-ffp-contract=fast-honor-pragmas"]}
 

@@ -285,7 +285,7 @@ struct PrepRows {
     int64_t cB, cH, cS;
     int split;
     int heads;                       // set by launch_prepare: heads of a chunk that a workgroup takes
-    char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order (bsa_fwd_frag.hip, bsa_fwd_round.hip), the real slots of a tile first, zeros behind
+    char* frag;                      // k, v: [B*Hn][padded slots / 64][16 KB] in fragment order (bsa_fwd_frag.hip, bsa_fwd_few.hip), the real slots of a tile first, zeros behind
     uint16_t* pooled;                // q, k: chunk means [B*Hn][blocks][128], the bits launch_permute's pooling gives; optional for k
     int pooled_operand;              // k: ... in operand order instead (operand_mean_at)
     int few;                         // k, v: the order is that of 32x32x16 products (frag_few)

@@ -1,4 +1,4 @@
-// What the two attention kernels on fragment-order K and V (bsa_fwd_frag.hip; bsa_fwd_round.hip: calls that leave SIMDs
+// What the two attention kernels on fragment-order K and V (bsa_fwd_frag.hip; bsa_fwd_few.hip: calls that leave SIMDs
 // idle) have in common: their items, how the keys of an item are listed, items in parts, and a list made in front of its walk.
 #pragma once
 #include "bsa_gate.h"
@@ -56,8 +56,8 @@ struct FragCall {
     bool halves;
     hipStream_t st;
 };
-// `items` work items at once, `team` wavefronts each (bsa_fwd_round.hip); gate: their lists are made in front of the walk.
-hipError_t launch_fwd_round(const FragCall& c, const FragLayout& L, const Parts& parts, int items, int team, const FragGate* gate, int32_t* lists, uint32_t* list_lens,
+// `items` work items at once, `team` wavefronts each (bsa_fwd_few.hip); gate: their lists are made in front of the walk.
+hipError_t launch_fwd_few(const FragCall& c, const FragLayout& L, const Parts& parts, int items, int team, const FragGate* gate, int32_t* lists, uint32_t* list_lens,
                             uint32_t kv_bytes);
 
 namespace {

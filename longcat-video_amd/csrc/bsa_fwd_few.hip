@@ -23,7 +23,7 @@ namespace {
 // of the item's pairs (of a part's share, where the item is in parts as well) and put their sums together in LDS, in the order of the
 // shares, wavefront w those of its 4 / kTeam tiles of d (choose_split).
 template <typename T, int kWalk, int kTeam, bool kGate>
-__global__ __launch_bounds__(64 * kTeam, 1) void fwd_round_kernel(
+__global__ __launch_bounds__(64 * kTeam, 1) void fwd_few_kernel(
     const T* __restrict__ q, const char* __restrict__ kf, const char* __restrict__ vf,
     const int32_t* __restrict__ idx, const int32_t* __restrict__ lens, const uint64_t* __restrict__ tile_valid,
     T* __restrict__ o, float* __restrict__ lse, int64_t Sq, int64_t Sk, int bs_k, int idx_stride,
@@ -34,7 +34,7 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_round_kernel(
     // log2 headroom before the running maximum is raised: probabilities reach 2^kTau, which the storage type of P
     // must hold (fp16 ends at 65 504) and the fp32 sums must hold times the number of keys
     constexpr float kTau = std::is_same<T, _Float16>::value ? 14.0f : 30.0f;
-    touch_arguments<decltype(fwd_round_kernel<T, kWalk, kTeam, kGate>)>();
+    touch_arguments<decltype(fwd_few_kernel<T, kWalk, kTeam, kGate>)>();
     // the item's list; then a team's sums; then 64 rows of the output of 256 B, 272 B apart
     constexpr int kOutPitch = kD + 8;
     constexpr int kOutBytes = kTile * kOutPitch * (int)sizeof(T);
@@ -684,37 +684,37 @@ __global__ __launch_bounds__(64 * kTeam, 1) void fwd_round_kernel(
 
 }  // namespace
 
-hipError_t launch_fwd_round(const FragCall& c, const FragLayout& L, const Parts& parts, int items, int team, const FragGate* gate, int32_t* lists, uint32_t* list_lens,
+hipError_t launch_fwd_few(const FragCall& c, const FragLayout& L, const Parts& parts, int items, int team, const FragGate* gate, int32_t* lists, uint32_t* list_lens,
                             uint32_t kv_bytes) {
     const dim3 grid((unsigned)(items * parts.count));
     const FragGate none = {};
-#define BSA_ROUND_W(T, WALK, TEAM, GATE)                                                                                                     \
-    hipLaunchKernelGGL((fwd_round_kernel<T, WALK, TEAM, GATE>), grid, dim3(64 * TEAM), 0, c.st, (const T*)c.q, (const char*)c.kf, (const char*)c.vf, \
+#define BSA_FEW_W(T, WALK, TEAM, GATE)                                                                                                     \
+    hipLaunchKernelGGL((fwd_few_kernel<T, WALK, TEAM, GATE>), grid, dim3(64 * TEAM), 0, c.st, (const T*)c.q, (const char*)c.kf, (const char*)c.vf, \
                        c.idx, c.lens, c.tile_valid, (T*)c.o, c.lse, c.Sq, c.Sk, c.bs_k, c.idx_stride, c.qk_scale, items, c.Hn, c.lse_rows, L, kv_bytes,  \
                        lists, list_lens, parts, gate != nullptr ? *gate : none)
-#define BSA_ROUND_G(T, TEAM, GATE)                                              \
+#define BSA_FEW_G(T, TEAM, GATE)                                              \
     do {                                                                        \
-        if (c.halves) BSA_ROUND_W(T, kHalves, TEAM, GATE);                      \
-        else if (c.bs_k == kTile) BSA_ROUND_W(T, kTiles, TEAM, GATE);           \
-        else BSA_ROUND_W(T, kBlocks, TEAM, GATE);                               \
+        if (c.halves) BSA_FEW_W(T, kHalves, TEAM, GATE);                      \
+        else if (c.bs_k == kTile) BSA_FEW_W(T, kTiles, TEAM, GATE);           \
+        else BSA_FEW_W(T, kBlocks, TEAM, GATE);                               \
     } while (0)
-#define BSA_ROUND_T(T, TEAM)                                                    \
+#define BSA_FEW_T(T, TEAM)                                                    \
     do {                                                                        \
-        if (gate != nullptr) BSA_ROUND_G(T, TEAM, true);                        \
-        else BSA_ROUND_G(T, TEAM, false);                                       \
+        if (gate != nullptr) BSA_FEW_G(T, TEAM, true);                        \
+        else BSA_FEW_G(T, TEAM, false);                                       \
     } while (0)
-#define BSA_ROUND(TEAM)                                                         \
+#define BSA_FEW(TEAM)                                                         \
     do {                                                                        \
-        if (c.dtype == BSA_BF16) BSA_ROUND_T(__bf16, TEAM);                     \
-        else BSA_ROUND_T(_Float16, TEAM);                                       \
+        if (c.dtype == BSA_BF16) BSA_FEW_T(__bf16, TEAM);                     \
+        else BSA_FEW_T(_Float16, TEAM);                                       \
     } while (0)
-    if (team == 4) BSA_ROUND(4);
-    else if (team == 2) BSA_ROUND(2);
-    else BSA_ROUND(1);
-#undef BSA_ROUND
-#undef BSA_ROUND_T
-#undef BSA_ROUND_G
-#undef BSA_ROUND_W
+    if (team == 4) BSA_FEW(4);
+    else if (team == 2) BSA_FEW(2);
+    else BSA_FEW(1);
+#undef BSA_FEW
+#undef BSA_FEW_T
+#undef BSA_FEW_G
+#undef BSA_FEW_W
     return hipGetLastError();
 }
 

@@ -23,7 +23,7 @@
 //
 // 16x16x32 and not 32x32x16: the board's power is what bounds this kernel, and the small form moves half as many
 // accumulators per multiplication (MFMAs alone on random data: 2 080 TFLOP/s against 1 820).  Calls that leave much of the chip
-// idle are not bound by it and go to bsa_fwd_round.hip (frag_few).
+// idle are not bound by it and go to bsa_fwd_few.hip (frag_few).
 //
 // Work decomposition.  One wavefront (a workgroup of 64 threads, one per SIMD; two or four where
 // they would be idle, see kTeam) = one work item =
@@ -1276,7 +1276,7 @@ static Split choose_split(int items, int list_tiles, int resident, bool is_tail,
         }
     return best;
 }
-// Calls of so few items that SIMDs are left over run fwd_round_kernel, whose 32x32x16 products leave a wavefront more of its issue; where nearly
+// Calls of so few items that SIMDs are left over run fwd_few_kernel, whose 32x32x16 products leave a wavefront more of its issue; where nearly
 // all are busy the board's power is the bound again.  Whole operator in us, this file's kernel / that one, items x tiles: with a wavefront an item
 // 640 x 20 53.7 / 50.3, x 80 140.6 / 130.0, 768 x 64 118.0 / 116.4, 800 x 20 56.9 / 56.9, x 80 145.5 / 145.2, 832 x 104 183.3 / 185.6, 896 x 64
 // 126.2 / 128.9, 1 024 x 128 246.8 / 255.9; teams of two 384 x 64 70.6 / 69.0, 416 x 104 101.5 / 101.3, 448 x 112 111.4 / 113.0, 512 x 128
@@ -1463,7 +1463,7 @@ hipError_t launch_fwd_frag(const void* q, const void* kf, const void* vf, const 
 #define BSA_FRAG_TAIL grid, whole, total, (const int32_t*)nullptr, (uint32_t*)nullptr, 0u, 0, whole_span, gate_lists, gate_lens
         if (few) {
             const FragCall c = {q, kf, vf, idx, lens, tile_valid, o, lse, Sq, Sk, lse_rows, bs_k, idx_stride, Hn, dtype, qk_scale, halves, st};
-            const hipError_t e = launch_fwd_round(c, L, parts, total, split.team, here.qc != nullptr ? &here : nullptr, gate_lists, gate_lens, whole_span);
+            const hipError_t e = launch_fwd_few(c, L, parts, total, split.team, here.qc != nullptr ? &here : nullptr, gate_lists, gate_lens, whole_span);
             if (e != hipSuccess) return e;
         } else if (split.team == 4) BSA_FRAG_LAUNCH_LISTED(4, BSA_FRAG_TAIL);      // 4 x more than kBusyWide / 2 items are not one round: no selection inside
         else if (split.team == 2) BSA_FRAG_LAUNCH_ONCE(2, BSA_FRAG_TAIL);

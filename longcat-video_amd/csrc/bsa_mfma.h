@@ -101,7 +101,7 @@ __device__ __forceinline__ s16x4 lds_read_tr16_at(uint32_t address) {
 // passes run for another 32 clocks and more, still writes them: the new value is overwritten, and an overwritten
 // address is a memory fault.  mfma_chain_end() (below) costs no instruction and ties the accumulators as live up
 // to the place where it stands; every chain is closed with one, placed where the distance rule above holds.
-// kAgprB: the B operand lives in an AGPR (fwd_round_kernel: the Q fragments of the queries 32 .. 63 of a work item; those of the queries
+// kAgprB: the B operand lives in an AGPR (fwd_few_kernel: the Q fragments of the queries 32 .. 63 of a work item; those of the queries
 // 0 .. 31 are in VGPRs, which balances the two register files).
 template <bool kFirst, bool kAgprB>
 __device__ inline void mfma_s(f32x16& acc, bf16x8 a, bf16x8 b) {

@@ -1,5 +1,5 @@
 // What the fragment-order attention kernel needs besides the selection, in one launch (HBM-bound): k and v in fragment
-// order (the layouts are described in bsa_fwd_frag.hip and bsa_fwd_round.hip), the chunk means of q and k, the row table of q, the validity
+// order (the layouts are described in bsa_fwd_frag.hip and bsa_fwd_few.hip), the chunk means of q and k, the row table of q, the validity
 // words of the KV tiles, the largest key norm per tile; with a row transform also the per-head RMSNorm and the 3-D RoPE of
 // q and k on their way through.
 //

@@ -56,7 +56,7 @@ def asked_for_together(code_objects, symbol):
     return []
 
 
-@pytest.mark.parametrize("name", ["15fwd_frag_kernel", "16fwd_round_kernel", "15bwd_dkdv_kernel"])
+@pytest.mark.parametrize("name", ["15fwd_frag_kernel", "14fwd_few_kernel", "15bwd_dkdv_kernel"])
 def test_every_line_of_the_arguments_is_asked_for(code_objects, name):
     """A 64-byte line of them that is left out is a wait for memory of its own; a load behind them may read past their segment."""
     for symbol, entry in metadata(code_objects, name).items():
