@@ -22,7 +22,7 @@
 //        order in which the accumulator registers of S^T hold them, so that P^T needs no shuffle.
 //
 // 16x16x32 and not 32x32x16: the board's power is what bounds this kernel, and the small form moves half as many
-// accumulators per multiplication (MFMAs alone on random data: 2 080 TFLOP/s against 1 820).  Calls that leave much of the chip
+// accumulators per multiplication (MFMAs alone on random data: 2 070 TFLOP/s against 1 850).  Calls that leave much of the chip
 // idle are not bound by it and go to bsa_fwd_few.hip (frag_few).
 //
 // Work decomposition.  One wavefront (a workgroup of 64 threads, one per SIMD; two or four where

@@ -12,7 +12,7 @@
 // therefore owns whole rotation pairs (features 2i, 2i + 1) and a quarter of the features of its tokens: the per-head
 // sum of squares is an in-lane sum plus two exchanges.  16x16x32 and not 32x32x16: what bounds a large product is the
 // board's power, and the small form moves half as many accumulators per multiplication.  Registers alone, random data, nothing but
-// MFMAs: 2 080 TFLOP/s against 1 820; this kernel (then one tile a workgroup), 86 400 x 4 096 x 4 096: 2 149 us against 2 282, the
+// MFMAs: 2 070 TFLOP/s against 1 850; this kernel (then one tile a workgroup), 86 400 x 4 096 x 4 096: 2 149 us against 2 282, the
 // clock under it 1.78 GHz against 1.65.
 //
 // A workgroup of eight wavefronts computes tiles of 256 tokens x 256 features, a wavefront 64 x 128 of a tile: for the
